@@ -74,6 +74,26 @@ def load() -> C.CDLL:
     return _lib
 
 
+_call = None
+
+
+def call():
+    """The extension module ``mojo_amd._call`` (``csrc/py_call.cpp``); like the library, it has no fallback."""
+    global _call
+    if _call is None:
+        load()
+        try:
+            from . import _call as native
+        except ImportError as e:
+            raise RuntimeError(f"mojo_amd/_call.so is not built or does not load ({e}); run `python -m mojo_amd.build`") from e
+        from .quantization import _BLOCKS, _CODES
+
+        native.setup([(enc, code, *((_BLOCKS[enc].elements_per_block, _BLOCKS[enc].block_size) if enc in _BLOCKS else (0, 0)))
+                      for enc, code in _CODES.items()])
+        _call = native
+    return _call
+
+
 class QmmError(RuntimeError):
     pass
 

@@ -15,6 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libqmm.so")
+CALL = os.path.join(HERE, "_call.so")  # the extension module in front of libqmm.so
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -85,7 +86,30 @@ def build(verbose: bool = False, force: bool = True, jobs: int | None = None) ->
     if proc.returncode != 0:
         sys.stderr.write(proc.stdout + proc.stderr)
         raise RuntimeError("hipcc failed linking libqmm.so")
+    _build_call(force, verbose)
     return LIB
+
+
+def _build_call(force: bool, verbose: bool) -> None:
+    """The extension module ``_call`` (host code only) against the headers of the installed torch and ``libqmm.so``."""
+    src = os.path.join(CSRC, "py_call.cpp")
+    if not force and os.path.exists(CALL) and os.path.getmtime(CALL) > max(os.path.getmtime(src), _headers_mtime()):
+        return
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    cmd = [HIPCC, "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "c++", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
+           f"-I{os.path.join(os.path.dirname(os.path.dirname(HIPCC)), 'include')}", src,
+           "-o", CALL, f"-L{HERE}", "-l:libqmm.so", f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        sys.stderr.write(proc.stdout + proc.stderr)
+        raise RuntimeError("hipcc failed on py_call.cpp")
 
 
 if __name__ == "__main__":
