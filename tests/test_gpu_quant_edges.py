@@ -1,0 +1,55 @@
+"""Quantisers and dequantisers at the edges of their tiles, byte for byte against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, dequantize, quantize, quantize_gptq
+
+pytestmark = pytest.mark.gpu
+ORACLE = {QE.Q4_0: O.Q4_0, QE.Q4_K: O.Q4_K, QE.Q5_K: O.Q5_K, QE.Q6_K: O.Q6_K}
+
+
+def weights(seed, n, k):
+    """Normal values with zero blocks, and runs of equal magnitude and either sign (the first extreme of a block decides its scale)."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    w = (0.02 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32)
+    flat = w.reshape(-1)
+    flat[: flat.size // 4 // 256 * 256] = 0.0 if seed % 2 else flat[: flat.size // 4 // 256 * 256]
+    tied = flat[flat.size // 2 :]
+    tied[:] = np.round(tied * 50) * np.float32(0.02)
+    return w
+
+
+def bits(t):
+    return t.cpu().view(torch.int32 if t.dtype == torch.float32 else torch.int16).numpy()
+
+
+@pytest.mark.parametrize("enc", list(ORACLE))
+@pytest.mark.parametrize("n,blocks", [(1, 1), (1, 3), (3, 5), (17, 4), (33, 9), (515, 37)])
+def test_gguf_edges(enc, n, blocks):
+    k = blocks * enc.block_parameters.elements_per_block  # (Q4_0: pieces of eight blocks with a remainder)
+    w = weights(n + blocks, n, k)
+    packed = O.quantize(ORACLE[enc], w)
+    assert np.array_equal(quantize(enc, torch.from_numpy(w).cuda()).cpu().numpy(), packed)
+    want = O.dequantize(ORACLE[enc], packed, k)
+    assert np.array_equal(bits(dequantize(enc, torch.from_numpy(packed).cuda())), want.view(np.int32))
+    assert np.array_equal(bits(dequantize(enc, torch.from_numpy(packed).cuda(), dtype=torch.bfloat16)), O.f32_to_bf16(want).view(np.int16))
+
+
+@pytest.mark.parametrize("n,k,group", [(8, 32, 32), (72, 96, 96), (64, 512, 128), (56, 640, 160), (200, 1024, 1024), (8, 416, 32)])
+def test_gptq_edges(n, k, group):
+    w = weights(n + k, n, k)
+    got = [t.cpu().numpy() for t in quantize_gptq(torch.from_numpy(w).cuda(), QuantizationConfig("gptq", 4, group, False, True))]
+    want = O.quantize_gptq(w, group)
+    for a, b in zip(got, want):
+        assert np.array_equal(a.view(np.uint16) if a.dtype == np.float16 else a, b)
+    qw, sc, qz, _ = want
+    order = np.random.Generator(np.random.PCG64(k)).integers(0, k // group, k).astype(np.int32)
+    tensors = [torch.from_numpy(qw).cuda(), torch.from_numpy(sc.view(np.float16)).cuda(), torch.from_numpy(qz).cuda()]
+    for g_idx in (None, order):
+        config = QuantizationConfig("gptq", 4, group, g_idx is not None, True)
+        rhs = tensors + ([torch.from_numpy(g_idx).cuda()] if g_idx is not None else [])
+        plain = O.dequantize_gptq(qw, sc, qz, group, g_idx)
+        assert np.array_equal(bits(dequantize(QE.GPTQ, *rhs, config=config)), plain.view(np.int32))
+        assert np.array_equal(bits(dequantize(QE.GPTQ, *rhs, config=config, dtype=torch.bfloat16)), O.f32_to_bf16(plain).view(np.int16))
