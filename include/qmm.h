@@ -123,9 +123,19 @@ int qmm_quantize_gptq(const qmm_gptq_config* cfg, const float* w, int64_t n, int
 /* Bytes of device scratch qmm_matmul needs for this problem (may be 0); the second form for a call with `flags`
  * (QMM_FLAG_OUT_BF16 adds room for an fp32 result wherever the kernel does not store bf16 itself).  For large
  * Q4_K / GPTQ prefill problems (more than 512 lhs rows) the figure includes fp16 planes of the weights (2 bytes per
- * weight) for the faster of two kernels; qmm_matmul given less than that, but enough for the lhs planes, runs the other one. */
+ * weight) for the faster of two kernels; qmm_matmul given less than that, but enough for the lhs planes, runs the other one.
+ * A call that needs none (0) may still run faster with some: qmm_preferred_workspace_bytes. */
 int64_t qmm_matmul_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k);
 int64_t qmm_matmul_workspace_bytes_flags(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags);
+
+/*
+ * The workspace with which a call runs fastest, never less than the figure that the call requires (qmm_matmul_workspace_bytes and its
+ * like): from a few lhs rows on, some kernels keep the narrowed lhs there that others do without.  A call given less than this but
+ * enough is served by those others, with results of the same precision.  cfg: GPTQ, else null.  A grouped call: the largest QMM_OP_MATMUL
+ * figure of its matrices.
+ */
+enum qmm_op { QMM_OP_MATMUL = 0, QMM_OP_RMSNORM = 1, QMM_OP_SWIGLU = 2, QMM_OP_REPACKED = 3 };
+int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags);
 
 /*
  * ops.qmatmul: out fp32[m, n] = lhs[m, k] . dequant(rhs)^T.

@@ -11,6 +11,7 @@ QMM_F32, QMM_BF16, QMM_F16 = 0, 1, 2
 QMM_FLAG_W_BF16 = 1
 QMM_FLAG_ACT_Q8K = 2
 QMM_FLAG_OUT_BF16 = 4
+QMM_OP_MATMUL, QMM_OP_RMSNORM, QMM_OP_SWIGLU, QMM_OP_REPACKED = 0, 1, 2, 3
 QMM_STATIC_SCRATCH_BYTES = 64 * 1024 * 1024
 
 
@@ -34,6 +35,7 @@ SIGNATURES = {
     "qmm_quantize_gptq": (_int, [C.POINTER(GptqConfig), _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp]),
     "qmm_matmul_workspace_bytes": (_i64, [_int, _int, _i64, _i64, _i64]),
     "qmm_matmul_workspace_bytes_flags": (_i64, [_int, _int, _i64, _i64, _i64, _int]),
+    "qmm_preferred_workspace_bytes": (_i64, [_int, _int, C.POINTER(GptqConfig), _int, _i64, _i64, _i64, _int]),
     "qmm_matmul": (_int, [_int, C.POINTER(GptqConfig), _vp, _int, _i64, _i64, C.POINTER(_vp), _int, _i64, _vp, _vp,
                           _i64, _int, _vp]),
     "qmm_matmul_static": (_int, [_int, C.POINTER(GptqConfig), _vp, _int, _i64, _i64, C.POINTER(_vp), _int, _i64, _vp, _int,

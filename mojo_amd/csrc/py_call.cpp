@@ -194,7 +194,7 @@ PyObject* py_matmul(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (out_type < 0) return none();
     const int flags = (int)PyLong_AsLong(a[4]) | (out_type == QMM_BF16 ? QMM_FLAG_OUT_BF16 : 0);
     at::Tensor out = c.result(w.n, out_type == QMM_BF16 ? at::kBFloat16 : at::kFloat);
-    const int64_t need = qmm_matmul_workspace_bytes_flags(e->code, c.dtype, c.m, w.n, c.k, flags);
+    const int64_t need = qmm_preferred_workspace_bytes(QMM_OP_MATMUL, e->code, w.cfg_p, c.dtype, c.m, w.n, c.k, flags);
     c10::DataPtr ws = c.workspace(need);
     int rc;
     {
@@ -222,7 +222,7 @@ PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (!(eps >= 0.0)) return none();
     const int flags = out_type == QMM_BF16 ? QMM_FLAG_OUT_BF16 : 0;
     at::Tensor out = c.result(w.n, out_type == QMM_BF16 ? at::kBFloat16 : at::kFloat);
-    const int64_t need = qmm_matmul_rmsnorm_workspace_bytes(e->code, c.dtype, c.m, w.n, c.k, flags);
+    const int64_t need = qmm_preferred_workspace_bytes(QMM_OP_RMSNORM, e->code, w.cfg_p, c.dtype, c.m, w.n, c.k, flags);
     c10::DataPtr ws = c.workspace(need);
     int rc;
     {
@@ -253,7 +253,7 @@ PyObject* py_grouped(PyObject*, PyObject* const* a, Py_ssize_t count) {
         if (!packed_matrix(e, t, c.k)) return none();
         rhs[i] = t->data_ptr();
         n[i] = t->size(0);
-        need = std::max(need, qmm_matmul_workspace_bytes(e->code, c.dtype, c.m, n[i], c.k));
+        need = std::max(need, qmm_preferred_workspace_bytes(QMM_OP_MATMUL, e->code, nullptr, c.dtype, c.m, n[i], c.k, 0));
     }
     for (Py_ssize_t i = 0; i < mats; i++) {
         out[i] = c.result(n[i], at::kFloat);
@@ -284,7 +284,7 @@ PyObject* py_swiglu(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (!packed_matrix(e, gate, c.k) || !packed_matrix(e, up, c.k) || gate->size(0) != up->size(0)) return none();
     const int64_t n = gate->size(0);
     at::Tensor out = c.result(n, at::kFloat);
-    const int64_t need = qmm_matmul_swiglu_workspace_bytes(e->code, c.dtype, c.m, n, c.k);
+    const int64_t need = qmm_preferred_workspace_bytes(QMM_OP_SWIGLU, e->code, nullptr, c.dtype, c.m, n, c.k, 0);
     c10::DataPtr ws = c.workspace(need);
     int rc;
     {
@@ -315,7 +315,7 @@ PyObject* py_repacked(PyObject*, PyObject* const* a, Py_ssize_t count) {
         w.cfg_p = &w.cfg;
     }
     at::Tensor out = c.result(n, at::kFloat);
-    const int64_t need = qmm_matmul_repacked_workspace_bytes(e->code, c.dtype, c.m, n, c.k);
+    const int64_t need = qmm_preferred_workspace_bytes(QMM_OP_REPACKED, e->code, w.cfg_p, c.dtype, c.m, n, c.k, 0);
     c10::DataPtr ws = c.workspace(need);
     int rc;
     {

@@ -324,7 +324,8 @@ static bool gptq_planes(int64_t m, int64_t n, int64_t k, int group) {
     return !g_skip_optional_planes && qmm::gemm_gptq_planes_wanted(m, n, k, group);
 }
 
-int64_t qmm_matmul_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+// what a call cannot do without
+static int64_t required_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || k <= 0) return 0;
     if (kquant_planes(encoding, lhs_dtype, m, n, k)) return qmm::gemm_planes_workspace_bytes(encoding, lhs_dtype, m, n, k);
     if (encoding == QMM_Q4_0) {
@@ -351,6 +352,15 @@ int64_t qmm_matmul_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64
 
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
+// The direct GEMM serves a problem when the caller's workspace holds its operands (qmm_preferred_workspace_bytes); with the smaller one
+// the other kernels do.
+static int direct_group(const qmm_gptq_config* cfg) { return cfg ? cfg->group_size : 0; }
+static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* workspace, int64_t workspace_bytes) {
+    if (encoding == QMM_GPTQ && (!cfg || cfg->desc_act)) return false;
+    return workspace && aligned(workspace, 256) && m > 0 && n > 0 && k > 0 && qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg)) &&
+           workspace_bytes >= qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k);
+}
+
 // Does the kernel that serves this problem store bf16 itself?  (The Q4_K decode kernel does; everything else goes
 // through an fp32 result in the workspace and a narrowing pass.)
 static bool stores_bf16_itself(int encoding, int64_t m, int64_t k, int flags) {
@@ -368,18 +378,47 @@ static bool q8k_integer_kernel(int encoding, int64_t m, int64_t k) {
 }
 static int64_t q8k_integer_workspace(int encoding, int64_t m, int64_t k) { return encoding == QMM_Q4_K ? 0 : qmm::q8k_planes_bytes(m, k); }
 
-int64_t qmm_matmul_workspace_bytes_flags(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
-    int64_t base = qmm_matmul_workspace_bytes(encoding, lhs_dtype, m, n, k);
+static int64_t required_bytes_flags(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
+    int64_t base = required_bytes(encoding, lhs_dtype, m, n, k);
     if ((flags & QMM_FLAG_ACT_Q8K) && m > 0 && k > 0)
         base = q8k_integer_kernel(encoding, m, k) ? q8k_integer_workspace(encoding, m, k)
-                                                  : up256(m * k * 4) + qmm_matmul_workspace_bytes(encoding, QMM_F32, m, n, k);
+                                                  : up256(m * k * 4) + required_bytes(encoding, QMM_F32, m, n, k);
     if (!(flags & QMM_FLAG_OUT_BF16) || m <= 0 || n <= 0 || stores_bf16_itself(encoding, m, k, flags)) return base;
     return up256(base) + up256(m * n * 4);
 }
 
+static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
+    const int64_t need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+    if (m <= 0 || n <= 0 || k <= 0 || (encoding == QMM_GPTQ && (!cfg || cfg->desc_act || cfg->group_size <= 0))) return need;
+    int64_t ahead = 0;
+    if (flags & QMM_FLAG_ACT_Q8K) {  // (the lhs as fp32 rows in front, where the integer kernels do not serve the call)
+        if (q8k_integer_kernel(encoding, m, k) || (flags & QMM_FLAG_OUT_BF16)) return need;
+        ahead = up256(m * k * 4);
+        lhs_dtype = QMM_F32;
+    }
+    if (!qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg))) return need;
+    return std::max(need, ahead + qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k));
+}
+
+// Where a call takes a workspace at all, the figure holds what the direct GEMM needs too (up to a size that the static buffer also has).
+int64_t qmm_matmul_workspace_bytes_flags(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
+    const int64_t need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+    if (need <= 0) return need;
+    qmm_gptq_config cfg{4, 128, 0, 1};
+    int64_t more = preferred_matmul(encoding, &cfg, lhs_dtype, m, n, k, flags);
+    if (encoding == QMM_GPTQ) {  // (the group size is not known here)
+        cfg.group_size = 32;
+        more = std::max(more, preferred_matmul(encoding, &cfg, lhs_dtype, m, n, k, flags));
+    }
+    return more <= (int64_t)QMM_STATIC_SCRATCH_BYTES ? more : need;
+}
+int64_t qmm_matmul_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    return qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, 0);
+}
+
 static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lhs_dtype, int64_t m, int64_t k,
                       const void* const* rhs, int n_rhs, int64_t n, float* out, void* workspace, int64_t workspace_bytes,
-                      int flags, void* stream);
+                      int flags, void* stream, uint16_t* out16 = nullptr);
 
 int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lhs_dtype, int64_t m, int64_t k,
                const void* const* rhs, int n_rhs, int64_t n, float* out, void* workspace, int64_t workspace_bytes,
@@ -387,7 +426,7 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
     // the plane GEMM for Q4_K / GPTQ only with a workspace that holds the planes
     const bool optional = (encoding == QMM_Q4_K || encoding == QMM_GPTQ) && m > 0 && n > 0 && k > 0 && !g_skip_optional_planes;
     const OptionalPlanesScope scope(g_skip_optional_planes ||
-                                    (optional && (!workspace || workspace_bytes < qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, flags))));
+                                    (optional && (!workspace || workspace_bytes < required_bytes_flags(encoding, lhs_dtype, m, n, k, flags))));
     if (!(flags & QMM_FLAG_OUT_BF16) || (flags & ~(QMM_FLAG_W_BF16 | QMM_FLAG_ACT_Q8K | QMM_FLAG_OUT_BF16)))
         return matmul_f32(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, flags, stream);
     // bf16 output
@@ -403,8 +442,10 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
         if (handled) return QMM_OK;
     }
     if (m <= 0 || n <= 0) return fail(QMM_ERR_INVALID, "qmm_matmul: M=%lld N=%lld must be positive", (long long)m, (long long)n);
+    if (!(inner & QMM_FLAG_ACT_Q8K) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
+        return matmul_f32(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, inner, stream, (uint16_t*)out);
     // (the fp32 result sits behind everything the inner call needs, the Q8_K round trip of the lhs included)
-    const int64_t base = up256(qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, inner)), need = base + up256(m * n * 4);
+    const int64_t base = up256(required_bytes_flags(encoding, lhs_dtype, m, n, k, inner)), need = base + up256(m * n * 4);
     if (!workspace || workspace_bytes < need)
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul: bf16 output of this problem goes through an fp32 result in the workspace: %lld bytes required "
                                        "(qmm_matmul_workspace_bytes_flags), %lld given", (long long)need, (long long)workspace_bytes);
@@ -416,7 +457,8 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
 
 static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lhs_dtype, int64_t m, int64_t k,
                       const void* const* rhs, int n_rhs, int64_t n, float* out, void* workspace, int64_t workspace_bytes,
-                      int flags, void* stream) {
+                      int flags, void* stream, uint16_t* out16) {
+    // (out16 != null: a call that the direct GEMM serves, with the bf16 form of the result stored there instead of `out`)
     hipStream_t s = (hipStream_t)stream;
     if (!lhs || !rhs || !out) return fail(QMM_ERR_INVALID, "qmm_matmul: null pointer");
     if (flags & ~(QMM_FLAG_W_BF16 | QMM_FLAG_ACT_Q8K)) return fail(QMM_ERR_INVALID, "qmm_matmul: unknown flag bits 0x%x", flags);
@@ -428,9 +470,9 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
     if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return fail(QMM_ERR_INVALID, "qmm_matmul: dimension too large");
     if (lhs_dtype != QMM_F32 && lhs_dtype != QMM_BF16)
         return fail(QMM_ERR_INVALID, "qmm_matmul: lhs dtype must be f32 or bf16");
-    if (!aligned(lhs, 16) || !aligned(out, 4)) return fail(QMM_ERR_INVALID, "qmm_matmul: lhs must be 16-byte aligned");
+    if (!aligned(lhs, 16) || !aligned(out, (void*)out == (void*)out16 ? 2 : 4)) return fail(QMM_ERR_INVALID, "qmm_matmul: lhs must be 16-byte aligned");
     int64_t esz = lhs_dtype == QMM_F32 ? 4 : 2;
-    int64_t need = qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, flags & QMM_FLAG_ACT_Q8K);
+    int64_t need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags & QMM_FLAG_ACT_Q8K);
     if (need > 0 && (!workspace || workspace_bytes < need))
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul: workspace of %lld bytes required, %lld given", (long long)need,
                     (long long)workspace_bytes);
@@ -455,6 +497,10 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
             }
             return QMM_OK;
         }
+        if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
+            return hip_status(qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],
+                                                      cfg->group_size, m, k, out16, workspace, s),
+                              "qmm_matmul(direct GEMM)");
         // GEMM (128 x 256 tiles) or passes of the small-batch kernel (16 rows each)?
         if (gptq_planes(m, n, k, cfg->group_size))
             return hip_status(qmm::launch_gemm_gptq_planes(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],
@@ -537,6 +583,9 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
         if (e != hipSuccess) return hip_status(e, "qmm_matmul(Q8_K round trip)");
         return matmul_f32(encoding, cfg, y, QMM_F32, m, k, rhs, n_rhs, n, out, (char*)workspace + ybytes, workspace_bytes - ybytes, 0, stream);
     }
+    // from a few to a few hundred lhs rows
+    if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
+        return hip_status(qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, nullptr, nullptr, 0, m, k, out16, workspace, s), "qmm_matmul(direct GEMM)");
     // Q5_K and Q6_K with many lhs rows, Q4_K with more than 512 on large matrices: weights to fp16 integer planes in the workspace,
     // then the matrix cores
     if (kquant_planes(encoding, lhs_dtype, m, n, k))
@@ -633,7 +682,7 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
 
 int64_t qmm_matmul_rmsnorm_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
     if (m <= 0 || k <= 0) return 0;
-    return up256(m * k * (lhs_dtype == QMM_F32 ? 4 : 2)) + qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+    return up256(m * k * (lhs_dtype == QMM_F32 ? 4 : 2)) + required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
 }
 
 int qmm_matmul_rmsnorm(int encoding, const qmm_gptq_config* cfg, const void* x, int x_dtype, const float* gamma, float eps, int64_t m,
@@ -655,7 +704,7 @@ int qmm_matmul_rmsnorm(int encoding, const qmm_gptq_config* cfg, const void* x, 
     }
     // Otherwise: normalised rows into the workspace, then the matmul on them.
     const int64_t ybytes = up256(m * k * (x_dtype == QMM_F32 ? 4 : 2));
-    const int64_t need = ybytes + qmm_matmul_workspace_bytes_flags(encoding, x_dtype, m, n, k, flags);
+    const int64_t need = ybytes + required_bytes_flags(encoding, x_dtype, m, n, k, flags);
     if (!workspace || workspace_bytes < need)
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul_rmsnorm: workspace of %lld bytes required (qmm_matmul_rmsnorm_workspace_bytes), %lld given",
                     (long long)need, (long long)workspace_bytes);
@@ -667,12 +716,12 @@ int qmm_matmul_rmsnorm(int encoding, const qmm_gptq_config* cfg, const void* x, 
 
 int qmm_matmul_static(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lhs_dtype, int64_t m, int64_t k,
                       const void* const* rhs, int n_rhs, int64_t n, float* out, int flags, void* stream) {
-    int64_t need = qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+    int64_t need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
     const TwinRowsScope twin(need > (int64_t)QMM_STATIC_SCRATCH_BYTES);  // (the two-pass treatment of an fp32 lhs needs less)
-    if (need > (int64_t)QMM_STATIC_SCRATCH_BYTES) need = qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+    if (need > (int64_t)QMM_STATIC_SCRATCH_BYTES) need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
     if (need > (int64_t)QMM_STATIC_SCRATCH_BYTES && (encoding == QMM_Q4_K || encoding == QMM_GPTQ)) {
         const OptionalPlanesScope no_planes(true);  // the kernels that need no weight planes
-        need = qmm_matmul_workspace_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+        need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
     }
     if (need > (int64_t)QMM_STATIC_SCRATCH_BYTES)
         return fail(QMM_ERR_WORKSPACE,
@@ -797,6 +846,14 @@ int qmm_repack(int encoding, const qmm_gptq_config* cfg, const void* const* rhs,
 // Q4_0: passes of the 16-row int8 kernel against the kept planes.  4096 x 4096: 28 us against 35 at 64 rows, 41 against 37 at 96;
 // 4096 x 14336: 57 against 83 at 64 rows, 84 against 84 at 96.
 static int64_t q4_0_repacked_min_rows(int64_t k) { return k > 4096 ? 96 : 80; }
+// With the planes at hand the direct GEMM on the packed tensors still wins while the weights are most of the traffic (the planes are 2 or 4
+// bytes a weight against 0.6 .. 0.8): us, planes / direct: Q5_K 4096 x 4096 128 bf16 rows 33 / 20, 300 rows 46 / 35; 14336 x 4096 200 rows
+// 69 / 60, 300 rows 81 / 93; 300 fp32 rows 167 / 117, 450 rows 178 / 186; Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.
+static bool direct_over_planes(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    const bool narrow = m * n <= (int64_t)1300 << 10;
+    return (narrow || m <= (lhs_dtype == QMM_F32 && encoding != QMM_Q4_0 ? 400 : 150)) && !(encoding == QMM_GPTQ && cfg->desc_act) &&
+           qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg));
+}
 static bool repacked_path(int encoding, int64_t m, int64_t n, int64_t k, bool have_rhs) {
     if (!have_rhs) return true;
     if (encoding == QMM_Q4_0) return m > q4_0_repacked_min_rows(k);
@@ -810,7 +867,7 @@ int64_t qmm_matmul_repacked_workspace_bytes(int encoding, int lhs_dtype, int64_t
                                                   : qmm::repacked_planes_workspace_bytes(encoding, lhs_dtype, m, n, k);
     if (repacked_path(encoding, m, n, k, true)) return planes;
     const OptionalPlanesScope no_planes(true);  // the other route: qmm_matmul's kernels on the packed tensors (or, without those, the planes)
-    return std::max(planes, qmm_matmul_workspace_bytes(encoding, lhs_dtype, m, n, k));
+    return std::max(planes, required_bytes(encoding, lhs_dtype, m, n, k));
 }
 
 int qmm_matmul_repacked(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lhs_dtype, int64_t m, int64_t k,
@@ -824,7 +881,8 @@ int qmm_matmul_repacked(int encoding, const qmm_gptq_config* cfg, const void* lh
     if (packed_bytes < qmm_repack_bytes(encoding, cfg, n, k) || !aligned(packed, 256))
         return fail(QMM_ERR_INVALID, "qmm_matmul_repacked: the packed buffer must be 256-byte aligned and hold qmm_repack_bytes = %lld bytes (%lld given)",
                     (long long)qmm_repack_bytes(encoding, cfg, n, k), (long long)packed_bytes);
-    if (!repacked_path(encoding, m, n, k, rhs != nullptr)) {
+    if (!repacked_path(encoding, m, n, k, rhs != nullptr) ||
+        (rhs && direct_over_planes(encoding, cfg, lhs_dtype, m, n, k) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))) {
         const OptionalPlanesScope no_planes(true);
         return qmm_matmul(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, 0, stream);
     }
@@ -859,6 +917,26 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
         return fail(QMM_ERR_INVALID, "qmm_matmul_grouped: encoding %d is not a GGUF weight encoding", encoding);
     for (int j = 0; j < count; j++)
         if (!rhs[j] || !out[j] || n[j] <= 0) return fail(QMM_ERR_INVALID, "qmm_matmul_grouped: matrix %d: null pointer or N <= 0", j);
+    // Matrices that a call of their own would give to the direct GEMM go there together; the others, if any, then form their own group.
+    if (m > 0 && m <= INT32_MAX && k > 0 && k <= INT32_MAX && (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && aligned(lhs, 16)) {
+        const void *direct_w[64], *rest_w[64];
+        int64_t direct_n[64], rest_n[64];
+        float *direct_out[64], *rest_out[64];
+        int directs = 0, rest = 0;
+        for (int j = 0; j < count; j++) {
+            if (aligned(rhs[j], 16) && aligned(out[j], 4) && n[j] <= INT32_MAX && direct_serves(encoding, nullptr, lhs_dtype, m, n[j], k, workspace, workspace_bytes))
+                direct_w[directs] = rhs[j], direct_n[directs] = n[j], direct_out[directs++] = out[j];
+            else rest_w[rest] = rhs[j], rest_n[rest] = n[j], rest_out[rest++] = out[j];
+        }
+        for (int j = 0; j < directs; j += qmm::kDirectMaxMats) {
+            const hipError_t e = qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, std::min(qmm::kDirectMaxMats, directs - j), direct_w + j, direct_n + j,
+                                                         direct_out + j, nullptr, nullptr, 0, m, k, nullptr, workspace, (hipStream_t)stream);
+            if (e != hipSuccess) return hip_status(e, "qmm_matmul_grouped(direct GEMM)");
+        }
+        if (directs > 0)
+            return rest == 0 ? QMM_OK
+                             : qmm_matmul_grouped(encoding, lhs, lhs_dtype, m, k, rest, rest_w, rest_n, rest_out, workspace, workspace_bytes, stream);
+    }
     if (encoding == QMM_Q4_K && m >= 1 && m <= 16 && k > 0 && k % 256 == 0 && count <= qmm::kLanesMaxMats &&
         (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && aligned(lhs, 16)) {
         bool ok = true;
@@ -923,7 +1001,7 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
 int64_t qmm_matmul_swiglu_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     // one lhs row of Q4_K goes through the decode kernel with the combination as its epilogue: nothing to keep
     if (encoding == QMM_Q4_K && m == 1 && k % 256 == 0 && k <= 16384) return 0;
-    return align_up(qmm_matmul_workspace_bytes(encoding, lhs_dtype, m, n, k), 256) + 2 * align_up(m * n * 4, 256);
+    return align_up(required_bytes(encoding, lhs_dtype, m, n, k), 256) + 2 * align_up(m * n * 4, 256);
 }
 
 int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, int64_t k, const void* gate, const void* up,
@@ -946,8 +1024,10 @@ int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, i
         if (e != hipSuccess) return hip_status(e, "qmm_matmul_swiglu(Q4_K decode)");
         if (handled) return QMM_OK;
     }
-    // two products into the workspace, then the combination
-    const int64_t mm_ws = align_up(qmm_matmul_workspace_bytes(encoding, lhs_dtype, m, n, k), 256), plane = align_up(m * n * 4, 256);
+    // two products into the workspace, then the combination (all that the caller gave beyond the products is the matmuls' workspace)
+    int64_t mm_ws = align_up(required_bytes(encoding, lhs_dtype, m, n, k), 256);
+    const int64_t plane = align_up(m * n * 4, 256);
+    if (workspace_bytes > mm_ws + 2 * plane) mm_ws = (workspace_bytes - 2 * plane) / 256 * 256;
     if (!workspace || workspace_bytes < mm_ws + 2 * plane)
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul_swiglu: workspace of %lld bytes required, %lld given", (long long)(mm_ws + 2 * plane),
                     (long long)workspace_bytes);
@@ -969,6 +1049,23 @@ int qmm_block_dots_q4_0(const void* lhs_q8_0, const void* rhs_q4_0, int64_t m, i
     return hip_status(qmm::launch_block_dots_q4_0((const uint8_t*)lhs_q8_0, (const uint8_t*)rhs_q4_0, m, n, k, out,
                                                   (hipStream_t)stream),
                       "qmm_block_dots_q4_0");
+}
+
+int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
+    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    switch (op) {
+        case QMM_OP_MATMUL: return preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, flags);
+        case QMM_OP_RMSNORM: return up256(m * k * (lhs_dtype == QMM_F32 ? 4 : 2)) + preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, flags);
+        case QMM_OP_SWIGLU: {
+            const int64_t need = qmm_matmul_swiglu_workspace_bytes(encoding, lhs_dtype, m, n, k);
+            return need ? std::max(need, up256(preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, 0)) + 2 * up256(m * n * 4)) : 0;
+        }
+        case QMM_OP_REPACKED: {
+            const int64_t need = qmm_matmul_repacked_workspace_bytes(encoding, lhs_dtype, m, n, k);
+            return repacked_path(encoding, m, n, k, true) && !direct_over_planes(encoding, cfg, lhs_dtype, m, n, k) ? need : std::max(need, preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, 0));
+        }
+        default: return 0;
+    }
 }
 
 }  // extern "C"

@@ -148,7 +148,7 @@ def qmatmul(encoding: QuantizationEncoding, config: Optional[QuantizationConfig]
         rc = lib.qmm_matmul_static(encoding.code, cfg_p, _ptr(lhs), lhs_dt, m, k, ptrs, len(rhs), n, _ptr(out), flags,
                                    _stream(lhs))
     else:
-        need = lib.qmm_matmul_workspace_bytes_flags(encoding.code, lhs_dt, m, n, k, flags)
+        need = lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, encoding.code, cfg_p, lhs_dt, m, n, k, flags)
         ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
         rc = lib.qmm_matmul(encoding.code, cfg_p, _ptr(lhs), lhs_dt, m, k, ptrs, len(rhs), n, _ptr(out), _ptr(ws),
                             need, flags, _stream(lhs))
@@ -232,7 +232,7 @@ def qmatmul_repacked(lhs: torch.Tensor, weights: RepackedWeights, out: Optional[
     lib = _lib.load()
     cfg_p = C.byref(_gptq_cfg(weights.config)) if enc == QuantizationEncoding.GPTQ else None
     lhs_dt = _DTYPES[lhs.dtype]
-    need = lib.qmm_matmul_repacked_workspace_bytes(enc.code, lhs_dt, m, n, k)
+    need = lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_REPACKED, enc.code, cfg_p, lhs_dt, m, n, k, 0)
     ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
     ptrs = (C.c_void_p * len(weights.rhs))(*[t.data_ptr() for t in weights.rhs]) if weights.rhs else None
     rc = lib.qmm_matmul_repacked(enc.code, cfg_p, _ptr(lhs), lhs_dt, m, k, ptrs, len(weights.rhs), _ptr(weights.packed),
@@ -276,7 +276,7 @@ def qmatmul_rmsnorm(encoding: QuantizationEncoding, config: Optional[Quantizatio
     x_dt = _DTYPES[x.dtype]
     flags = _lib.QMM_FLAG_OUT_BF16 if out_dtype == torch.bfloat16 else 0
     out = torch.empty((m, n), dtype=out_dtype, device=x.device)
-    need = lib.qmm_matmul_rmsnorm_workspace_bytes(encoding.code, x_dt, m, n, k, flags)
+    need = lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_RMSNORM, encoding.code, cfg_p, x_dt, m, n, k, flags)
     ws = torch.empty((need,), dtype=torch.uint8, device=x.device) if need > 0 else None
     ptrs = (C.c_void_p * len(rhs))(*[t.data_ptr() for t in rhs])
     rc = lib.qmm_matmul_rmsnorm(encoding.code, cfg_p, _ptr(x), x_dt, _ptr(gamma), C.c_float(eps), m, k, ptrs, len(rhs), n,
@@ -319,7 +319,7 @@ def qmatmul_grouped(encoding: QuantizationEncoding, lhs: torch.Tensor, rhs: Sequ
     lib = _lib.load()
     lhs_dt = _DTYPES[lhs.dtype]
     outs = [torch.empty((m, w.shape[0]), dtype=torch.float32, device=lhs.device) for w in rhs]
-    need = max(lib.qmm_matmul_workspace_bytes(encoding.code, lhs_dt, m, w.shape[0], k) for w in rhs)
+    need = max(lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, encoding.code, None, lhs_dt, m, w.shape[0], k, 0) for w in rhs)
     ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
     count = len(rhs)
     rhs_p = (C.c_void_p * count)(*[w.data_ptr() for w in rhs])
@@ -365,7 +365,7 @@ def qmatmul_swiglu(encoding: QuantizationEncoding, lhs: torch.Tensor, gate: torc
     lib = _lib.load()
     lhs_dt = _DTYPES[lhs.dtype]
     out = torch.empty((m, n), dtype=torch.float32, device=lhs.device)
-    need = lib.qmm_matmul_swiglu_workspace_bytes(encoding.code, lhs_dt, m, n, k)
+    need = lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_SWIGLU, encoding.code, None, lhs_dt, m, n, k, 0)
     ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
     rc = lib.qmm_matmul_swiglu(encoding.code, _ptr(lhs), lhs_dt, m, k, _ptr(gate), _ptr(up), n, _ptr(out), _ptr(ws), need,
                                _stream(lhs))

@@ -1,0 +1,72 @@
+"""The GEMM that reads packed weights straight into the matrix cores, at the edges of its tiles (32 or 64 rows and columns), of its units
+of 256 values of K and of the ways it cuts K (4 or 8 wavefronts, one or two workgroups a tile), against float64 products of the same
+integers."""
+import ctypes as C
+
+import pytest
+import torch
+
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, _lib, dequantize, qmatmul, qmatmul_grouped, quantize, quantize_gptq
+
+pytestmark = pytest.mark.gpu
+
+
+def weights(enc, group, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    w = torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen)
+    if enc != QE.GPTQ:
+        return None, (quantize(enc, w),)
+    config = QuantizationConfig("gptq", 4, group, False, True)
+    qweight, scales, qzeros, _ = quantize_gptq(w, config)
+    qzeros = torch.randint(-2**31, 2**31 - 1, qzeros.shape, device="cuda", dtype=torch.int64, generator=gen).int()  # every zero point
+    return config, (qweight, scales, qzeros)
+
+
+def check(got, enc, config, rhs, a):
+    w = dequantize(enc, *rhs, config=config).double()
+    x = a.double()
+    if enc == QE.Q4_0:  # (multiplies with the lhs quantised to Q8_0)
+        blocks = quantize(QE.Q8_0, a.float()).view(a.shape[0], -1, 34)
+        scale = blocks[:, :, :2].contiguous().view(torch.float16)
+        x = (scale.double() * blocks[:, :, 2:].contiguous().view(torch.int8).double()).view(a.shape)
+    want, size = x @ w.T, x.abs() @ w.abs().T
+    # A lhs value is two fp16 terms (2^-22) or exact (bf16); K / 16 products enter a sum one after the other, and 32 for the parts of K.
+    # A GPTQ or Q4_K product may be the difference of two terms sixteen times as large (code and zero point or minimum apart).
+    bound = (a.shape[1] / 16 + 32) * 2.0**-24 * 16 * size + 1e-30
+    if got.dtype == torch.bfloat16:
+        bound = bound + 2.0**-8 * want.abs()
+    worst = ((got.double() - want).abs() / bound).max().item()
+    assert worst <= 1.0, (enc, got.shape, a.shape, worst)
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("enc,group,odd", [(QE.Q4_0, 0, 32), (QE.Q4_K, 0, 0), (QE.Q5_K, 0, 0), (QE.Q6_K, 0, 0), (QE.GPTQ, 128, 128), (QE.GPTQ, 32, 32)])
+def test_edges(enc, group, odd, lhs):
+    for m, n, k in ((17, 40, 256), (32, 264, 512 + odd), (17, 40, 2304 + odd), (33, 2056, 2304), (33, 4104, 4352 - odd), (65, 4104, 4352), (100, 4104, 256 + odd),
+                    (200, 4104, 256), (450, 264, 1024)):
+        config, rhs = weights(enc, group, n, k)
+        a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(lhs)
+        a[m // 2] *= 1e-6
+        a[m - 1] = 0.0
+        cfg = C.byref(_lib.GptqConfig(4, group, 0, 1)) if config else None
+        lib, dtype = _lib.load(), _lib.QMM_F32 if lhs == torch.float32 else _lib.QMM_BF16
+        assert lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, enc.code, cfg, dtype, m, n, k, 0) > 0
+        check(qmatmul(enc, config, a, *rhs), enc, config, rhs, a)
+        check(qmatmul(enc, config, a, *rhs, out_dtype=torch.bfloat16), enc, config, rhs, a)
+        # with the workspace that a caller of the C interface gives (none for some: other kernels)
+        need = lib.qmm_matmul_workspace_bytes(enc.code, dtype, m, n, k)
+        ws, out = torch.empty(max(need, 1), dtype=torch.uint8, device="cuda"), torch.full((m, n), float("nan"), device="cuda")
+        ptrs = (C.c_void_p * len(rhs))(*[t.data_ptr() for t in rhs])
+        assert lib.qmm_matmul(enc.code, cfg, a.data_ptr(), dtype, m, k, ptrs, len(rhs), n, out.data_ptr(), ws.data_ptr(), need, 0,
+                              torch.cuda.current_stream().cuda_stream) == 0
+        check(out, enc, config, rhs, a)
+
+
+@pytest.mark.parametrize("enc", [QE.Q4_0, QE.Q4_K, QE.Q5_K, QE.Q6_K])
+@pytest.mark.parametrize("m,k,ns", [(17, 768, (40, 264, 1000)), (33, 2304, (4104, 2056, 40, 1, 31)), (3, 1024, (6400, 40, 6400))])
+def test_group_equals_separate_calls(enc, m, k, ns):
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m))
+    rhs = [weights(enc, 0, n, k)[1] for n in ns]
+    for got, w in zip(qmatmul_grouped(enc, a, [w[0] for w in rhs]), rhs):
+        assert torch.equal(got, qmatmul(enc, None, a, *w))
+        check(got, enc, None, w, a)
