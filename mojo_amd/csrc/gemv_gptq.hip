@@ -318,7 +318,8 @@ template <int MT, bool TABLE, typename AT>
 __global__ __launch_bounds__(64 * kWaves) void gemv_gptq_act_order_kernel(
     const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     const int32_t* __restrict__ g_idx, const AT* __restrict__ a, float* __restrict__ out, int m, int n, int k, int group,
-    int64_t ldo) {
+    int64_t ldo, const int32_t* __restrict__ only_if) {
+    if (only_if && *only_if == 0) return;
     extern __shared__ __attribute__((aligned(16))) float gsm[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -337,69 +338,77 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_gptq_act_order_kernel(
         for (int g = wave; g < ngroups; g += kWaves) table[g * 64 + lane] = pair_of(g);
         __syncthreads();
     }
-    float acc[MT];
+    for (int m0 = 0; m0 < m; m0 += MT) {  // passes of MT rows
+        const int left = m - m0;
+        float acc[MT];
 #pragma unroll
-    for (int mi = 0; mi < MT; mi++) acc[mi] = 0.0f;
-    // wavefront w walks the k8 rows [w * per, (w + 1) * per), four rows of loads at a time (K / 8 is a multiple of 4)
-    constexpr int U = 4;
-    const int rows = k >> 3;
-    const int per = ((rows + kWaves - 1) / kWaves + U - 1) / U * U;
-    const int r_end = min(rows, (wave + 1) * per);
-    for (int r = wave * per; r < r_end; r += U) {
-        uint32_t x[U];
+        for (int mi = 0; mi < MT; mi++) acc[mi] = 0.0f;
+        // wavefront w walks the k8 rows [w * per, (w + 1) * per), four rows of loads at a time (K / 8 is a multiple of 4)
+        constexpr int U = 4;
+        const int rows = k >> 3;
+        const int per = ((rows + kWaves - 1) / kWaves + U - 1) / U * U;
+        const int r_end = min(rows, (wave + 1) * per);
+        for (int r = wave * per; r < r_end; r += U) {
+            uint32_t x[U];
 #pragma unroll
-        for (int j = 0; j < U; j++) x[j] = (qweight + (int64_t)(r + j) * n)[ccol];
+            for (int j = 0; j < U; j++) x[j] = (qweight + (int64_t)(r + j) * n)[ccol];
 #pragma unroll
-        for (int j = 0; j < U; j++) {
-            const int k0 = (r + j) * 8;
-            const uint32_t qe = x[j] & 0x0F0F0F0Fu, qo = (x[j] >> 4) & 0x0F0F0F0Fu;  // k 0,2,4,6 / k 1,3,5,7
-            const float q[8] = {gub0(qe), gub0(qo), gub1(qe), gub1(qo), gub2(qe), gub2(qo), gub3(qe), gub3(qo)};
+            for (int j = 0; j < U; j++) {
+                const int k0 = (r + j) * 8;
+                const uint32_t qe = x[j] & 0x0F0F0F0Fu, qo = (x[j] >> 4) & 0x0F0F0F0Fu;  // k 0,2,4,6 / k 1,3,5,7
+                const float q[8] = {gub0(qe), gub0(qo), gub1(qe), gub1(qo), gub2(qe), gub2(qo), gub3(qe), gub3(qo)};
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int g = min(max(g_idx[k0 + i], 0), ngroups - 1);  // wave-uniform
-                const float2 sz = TABLE ? table[g * 64 + lane] : pair_of(g);
-                const float w = fmaf(sz.x, q[i], sz.y);
+                for (int i = 0; i < 8; i++) {
+                    const int g = min(max(g_idx[k0 + i], 0), ngroups - 1);  // wave-uniform
+                    const float2 sz = TABLE ? table[g * 64 + lane] : pair_of(g);
+                    const float w = fmaf(sz.x, q[i], sz.y);
 #pragma unroll
-                for (int mi = 0; mi < MT; mi++)
-                    acc[mi] = fmaf(w, act(a + (int64_t)(mi < m ? mi : 0) * k, k0 + i), acc[mi]);
+                    for (int mi = 0; mi < MT; mi++)
+                        acc[mi] = fmaf(w, act(a + (int64_t)m0 * k + (int64_t)(mi < left ? mi : 0) * k, k0 + i), acc[mi]);
+                }
             }
         }
-    }
 #pragma unroll
-    for (int mi = 0; mi < MT; mi++) red[(wave * MT + mi) * 64 + lane] = acc[mi];
-    __syncthreads();
-    if (wave == 0 && col < n) {
+        for (int mi = 0; mi < MT; mi++) red[(wave * MT + mi) * 64 + lane] = acc[mi];
+        __syncthreads();
+        if (wave == 0 && col < n) {
 #pragma unroll
-        for (int mi = 0; mi < MT; mi++) {
-            if (mi < m) {
-                float v = 0.0f;
+            for (int mi = 0; mi < MT; mi++) {
+                if (mi < left) {
+                    float v = 0.0f;
 #pragma unroll
-                for (int w = 0; w < kWaves; w++) v += red[(w * MT + mi) * 64 + lane];
-                out[(int64_t)mi * ldo + col] = v;
+                    for (int w = 0; w < kWaves; w++) v += red[(w * MT + mi) * 64 + lane];
+                    out[(int64_t)(m0 + mi) * ldo + col] = v;
+                }
             }
         }
+        __syncthreads();  // (the next pass writes `red` again)
     }
 }
 
-// m <= 4 lhs rows; K % 32 == 0 and N % 8 == 0 are the caller's checks.
+// K % 32 == 0 and N % 8 == 0 are the caller's checks.  only_if != null: the launch does nothing where that word is zero.
 hipError_t launch_gemv_gptq_act_order(const void* a, int a_dtype, const uint32_t* qweight, const uint16_t* scales,
                                       const uint32_t* qzeros, const int32_t* g_idx, int m, int64_t n, int64_t k, int group,
-                                      float* out, int64_t ldo, hipStream_t s) {
-    if (m < 1 || m > 4 || (k & 31)) return hipErrorInvalidValue;
+                                      float* out, int64_t ldo, hipStream_t s, const int32_t* only_if) {
+    if (m < 1 || (k & 31)) return hipErrorInvalidValue;
     const int mt = m <= 1 ? 1 : m <= 2 ? 2 : 4;
     const size_t red_bytes = (size_t)kWaves * mt * 64 * 4;
     const size_t table_bytes = (size_t)(k / group) * 64 * 8;
-    const bool table = table_bytes + red_bytes <= 64 * 1024;
+    // (past half of the LDS one workgroup fills a compute unit, and that is still better than a scale and a zero point from memory per weight)
+    const bool table = table_bytes + red_bytes <= (size_t)kLdsPerCu;
     const size_t lds = red_bytes + (table ? table_bytes : 0);
     dim3 grid((unsigned)((n + 63) / 64)), block(64 * kWaves);
 #define QMM_GPTQ_AO(MT_, TB_)                                                                                          \
     do {                                                                                                              \
+        const hipError_t e = a_dtype == QMM_F32 ? allow_full_lds<gemv_gptq_act_order_kernel<MT_, TB_, float>>()       \
+                                                : allow_full_lds<gemv_gptq_act_order_kernel<MT_, TB_, uint16_t>>();   \
+        if (e != hipSuccess) return e;                                                                                \
         if (a_dtype == QMM_F32)                                                                                       \
             gemv_gptq_act_order_kernel<MT_, TB_, float><<<grid, block, lds, s>>>(                                     \
-                qweight, scales, qzeros, g_idx, (const float*)a, out, m, (int)n, (int)k, group, ldo);                 \
+                qweight, scales, qzeros, g_idx, (const float*)a, out, m, (int)n, (int)k, group, ldo, only_if);        \
         else                                                                                                          \
             gemv_gptq_act_order_kernel<MT_, TB_, uint16_t><<<grid, block, lds, s>>>(                                  \
-                qweight, scales, qzeros, g_idx, (const uint16_t*)a, out, m, (int)n, (int)k, group, ldo);              \
+                qweight, scales, qzeros, g_idx, (const uint16_t*)a, out, m, (int)n, (int)k, group, ldo, only_if);     \
     } while (0)
 #define QMM_GPTQ_AO_MT(TB_)                        \
     do {                                           \

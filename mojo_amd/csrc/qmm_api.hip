@@ -387,9 +387,30 @@ static int64_t required_bytes_flags(int encoding, int lhs_dtype, int64_t m, int6
     return up256(base) + up256(m * n * 4);
 }
 
+static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags);
+
+// Act-order GPTQ by sorted columns: the sorted tensors, then what the plain product on them needs.  0: not this way.
+static qmm_gptq_config plain_groups(qmm_gptq_config cfg) {
+    cfg.desc_act = 0;
+    return cfg;
+}
+static int64_t order_bytes(const qmm_gptq_config& cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
+    if (!cfg.desc_act || cfg.group_size <= 0 || k % cfg.group_size || (flags & ~QMM_FLAG_OUT_BF16) || !qmm::gptq_order_wanted(m, n, k)) return 0;
+    const qmm_gptq_config plain = plain_groups(cfg);
+    return qmm::gptq_order_space(nullptr, lhs_dtype, m, n, k).bytes + up256(preferred_matmul(QMM_GPTQ, &plain, lhs_dtype, m, n, k, 0));
+}
+static bool order_serves(const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags, const void* workspace, int64_t workspace_bytes) {
+    const int64_t need = order_bytes(*cfg, lhs_dtype, m, n, k, flags);
+    return need > 0 && workspace && aligned(workspace, 256) && workspace_bytes >= need;
+}
+
 static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
     const int64_t need = required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
-    if (m <= 0 || n <= 0 || k <= 0 || (encoding == QMM_GPTQ && (!cfg || cfg->desc_act || cfg->group_size <= 0))) return need;
+    if (m <= 0 || n <= 0 || k <= 0 || (encoding == QMM_GPTQ && (!cfg || cfg->group_size <= 0))) return need;
+    if (encoding == QMM_GPTQ && cfg->desc_act) {
+        const int64_t order = order_bytes(*cfg, lhs_dtype, m, n, k, flags);
+        return order ? std::max(need, order + ((flags & QMM_FLAG_OUT_BF16) ? up256(m * n * 4) : 0)) : need;
+    }
     int64_t ahead = 0;
     if (flags & QMM_FLAG_ACT_Q8K) {  // (the lhs as fp32 rows in front, where the integer kernels do not serve the call)
         if (q8k_integer_kernel(encoding, m, k) || (flags & QMM_FLAG_OUT_BF16)) return need;
@@ -445,7 +466,12 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
     if (!(inner & QMM_FLAG_ACT_Q8K) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
         return matmul_f32(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, inner, stream, (uint16_t*)out);
     // (the fp32 result sits behind everything the inner call needs, the Q8_K round trip of the lhs included)
-    const int64_t base = up256(required_bytes_flags(encoding, lhs_dtype, m, n, k, inner)), need = base + up256(m * n * 4);
+    int64_t base = up256(required_bytes_flags(encoding, lhs_dtype, m, n, k, inner));
+    if (encoding == QMM_GPTQ && cfg) {
+        const int64_t order = std::max(base, order_bytes(*cfg, lhs_dtype, m, n, k, inner));
+        if (workspace_bytes >= order + up256(m * n * 4)) base = order;
+    }
+    const int64_t need = base + up256(m * n * 4);
     if (!workspace || workspace_bytes < need)
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul: bf16 output of this problem goes through an fp32 result in the workspace: %lld bytes required "
                                        "(qmm_matmul_workspace_bytes_flags), %lld given", (long long)need, (long long)workspace_bytes);
@@ -485,16 +511,24 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
         for (int i = 0; i < 3; i++)
             if (!rhs[i] || !aligned(rhs[i], 4)) return fail(QMM_ERR_INVALID, "qmm_matmul: GPTQ rhs[%d] null or misaligned", i);
         if (cfg->desc_act) {
-            // act-order checkpoints: the decode kernel that looks the group of every k up, four lhs rows per pass
+            // act-order checkpoints: the columns sorted by group, then the kernels for plain groups; the decode kernel that looks the group of
+            // every k up, four lhs rows per pass, for few rows and with a workspace too small for the sorted matrix
             if (n_rhs != 4 || !rhs[3] || !aligned(rhs[3], 4))
                 return fail(QMM_ERR_INVALID, "qmm_matmul: GPTQ desc_act=True needs rhs[3] = g_idx int32[K]");
-            for (int64_t m0 = 0; m0 < m; m0 += 4) {
-                hipError_t e = qmm::launch_gemv_gptq_act_order((const char*)lhs + m0 * k * esz, lhs_dtype, (const uint32_t*)rhs[0],
-                                                               (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],
-                                                               (const int32_t*)rhs[3], (int)std::min<int64_t>(4, m - m0), n, k,
-                                                               cfg->group_size, out + m0 * n, n, s);
-                if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order)");
+            const int32_t* only_if = nullptr;
+            if (order_serves(cfg, lhs_dtype, m, n, k, flags, workspace, workspace_bytes)) {
+                const qmm::GptqOrderSpace p = qmm::gptq_order_space(workspace, lhs_dtype, m, n, k);
+                hipError_t e = qmm::launch_gptq_order(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const int32_t*)rhs[3], m, n, k, cfg->group_size, p, s);
+                if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, sort)");
+                const qmm_gptq_config plain = plain_groups(*cfg);
+                const void* sorted[3] = {p.qweight, rhs[1], rhs[2]};
+                if (int rc = matmul_f32(encoding, &plain, p.lhs, lhs_dtype, m, k, sorted, 3, n, out, (char*)workspace + p.bytes, workspace_bytes - p.bytes, flags, stream))
+                    return rc;
+                only_if = p.uneven;
             }
+            hipError_t e = qmm::launch_gemv_gptq_act_order(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],
+                                                           (const int32_t*)rhs[3], (int)m, n, k, cfg->group_size, out, n, s, only_if);
+            if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order)");
             return QMM_OK;
         }
         if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))

@@ -12,7 +12,7 @@ namespace qmm {
 // Kernel families switched off by the environment variable QMM_DISABLE (a comma-separated list of names, read once
 // per process), for tests and triage: a disabled family reports that it does not take a shape, and the next kernel
 // in the dispatch order serves it.  Names: direct, q4k_lanes, q4k_lanes_rows, q4k_stream, q4k_mm, q4k_kc, q4k_tile, q4k_gemm64, q4k_twin_rows, q4k_rows_v2,
-// q4_0_stream, q4_0_mfma, q4_0_small, q4_0_small_passes, q4_0_wide, q4_0_planes, q6k_lanes, q6k_slab, q6k_staged, kquant_planes, planes_wide, planes_192, planes_quarters, planes_twin_rows, gptq_twin_rows, gptq_k_shares, gptq_long_k_mm, kquant_mm_rounds_grid, q4k_mm_k_parts, q4k_planes, gptq_planes, gptq_mm, gptq_cols, gptq_cols16.
+// q4_0_stream, q4_0_mfma, q4_0_small, q4_0_small_passes, q4_0_wide, q4_0_planes, q6k_lanes, q6k_slab, q6k_staged, kquant_planes, planes_wide, planes_192, planes_quarters, planes_twin_rows, gptq_twin_rows, gptq_k_shares, gptq_long_k_mm, kquant_mm_rounds_grid, q4k_mm_k_parts, q4k_planes, gptq_planes, gptq_mm, gptq_cols, gptq_cols16, gptq_order.
 // Nothing is disabled by default.
 bool kernel_disabled(const char* family);
 // False while qmm_matmul_static serves a problem whose one-pass treatment of an fp32 lhs (the lhs as twice the rows, the
@@ -156,7 +156,21 @@ hipError_t launch_gemv_gptq_mm(const void* a, int a_dtype, const uint32_t* qweig
                                void* workspace, hipStream_t s, bool* handled);
 hipError_t launch_gemv_gptq_act_order(const void* a, int a_dtype, const uint32_t* qweight, const uint16_t* scales,
                                       const uint32_t* qzeros, const int32_t* g_idx, int m, int64_t n, int64_t k, int group,
-                                      float* out, int64_t ldo, hipStream_t s);
+                                      float* out, int64_t ldo, hipStream_t s, const int32_t* only_if = nullptr);
+
+// gptq_order.hip: the columns of an act-order matrix and of the lhs sorted by group into the workspace.  `uneven` is set where the groups are not of
+// group_size columns each: the sorted forms are then of no use, and the look-up kernel above (only_if = uneven) has to follow the product.
+struct GptqOrderSpace {
+    int32_t* uneven;
+    int32_t* source;
+    uint32_t* qweight;
+    void* lhs;
+    int64_t bytes;
+};
+GptqOrderSpace gptq_order_space(void* workspace, int lhs_dtype, int64_t m, int64_t n, int64_t k);
+bool gptq_order_wanted(int64_t m, int64_t n, int64_t k);
+hipError_t launch_gptq_order(const void* lhs, int lhs_dtype, const uint32_t* qweight, const int32_t* g_idx, int64_t m, int64_t n, int64_t k, int group,
+                             const GptqOrderSpace& p, hipStream_t s);
 bool gemv_q4_k_kc_supported(const void* w, int64_t k);
 int64_t gemv_q4_k_kc_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemv_q4_k_kc(const void* a, int a_dtype, const uint8_t* w, int m, int64_t n, int64_t k, float* out,

@@ -1,0 +1,92 @@
+"""Act-order GPTQ with several lhs rows (columns sorted by group, then the kernels for plain groups): edges of the sort (K / 16 columns per
+wavefront, groups of 32 .. K), of the column slabs (8, 16, 32), of the row counts at which the plain kernels change, groups of uneven
+size (served by the look-up kernel), workspaces with and without room for the sorted matrix; against float64 products."""
+import ctypes as C
+
+import pytest
+import torch
+
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, _lib, dequantize, qmatmul, quantize_gptq
+
+pytestmark = pytest.mark.gpu
+
+
+def act_order(n, k, group, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen)
+    qweight, scales, qzeros, g_idx = quantize_gptq(w, QuantizationConfig("gptq", 4, group, False, True))
+    qweight = torch.randint(-2**31, 2**31 - 1, qweight.shape, device="cuda", dtype=torch.int64, generator=gen).int()
+    qzeros = torch.randint(-2**31, 2**31 - 1, qzeros.shape, device="cuda", dtype=torch.int64, generator=gen).int()
+    return QuantizationConfig("gptq", 4, group, True, True), (qweight, scales, qzeros, g_idx[torch.randperm(k, device="cuda", generator=gen)].contiguous())
+
+
+def check(got, config, rhs, a):
+    w = dequantize(QE.GPTQ, *rhs, config=config).double()
+    x = a.double()
+    want, size = x @ w.T, x.abs() @ w.abs().T
+    # A weight is exact (code and zero point apart: a product of up to sixteen times its size), a lhs value two fp16 terms (2^-22) or exact; the
+    # look-up kernel adds K / 16 products one after the other and sixteen sums, the others K / 16 products and 32 sums.
+    bound = (a.shape[1] / 16 + 32) * 2.0**-24 * 16 * size + 1e-30
+    if got.dtype == torch.bfloat16:
+        bound = bound + 2.0**-8 * want.abs()
+    worst = ((got.double() - want).abs() / bound).max().item()
+    assert worst <= 1.0, (got.shape, a.shape, worst)
+
+
+def c_call(config, rhs, a, need):
+    """The C entry point with a workspace of `need` bytes."""
+    m, (k, n) = a.shape[0], (a.shape[1], rhs[0].shape[1])
+    ws, out = torch.empty(max(need, 1), dtype=torch.uint8, device="cuda"), torch.full((m, n), float("nan"), device="cuda")
+    ptrs = (C.c_void_p * 4)(*[t.data_ptr() for t in rhs])
+    cfg = C.byref(_lib.GptqConfig(4, config.group_size, 1, 1))
+    assert _lib.load().qmm_matmul(QE.GPTQ.code, cfg, a.data_ptr(), _lib.QMM_F32 if a.dtype == torch.float32 else _lib.QMM_BF16, m, k, ptrs, 4, n, out.data_ptr(),
+                                  ws.data_ptr(), need, 0, torch.cuda.current_stream().cuda_stream) == 0
+    return out
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,group", [(3, 72, 256, 32), (5, 8, 32, 32), (6, 40, 1056, 32), (17, 264, 1024, 1024), (16, 136, 5120, 128), (33, 136, 5376, 256),
+                                         (9, 72, 10240, 128), (20, 40, 10496, 64), (20, 24, 32768, 32), (130, 1032, 2304, 128), (600, 4104, 512, 128)])
+def test_edges(m, n, k, group, lhs):
+    config, rhs = act_order(n, k, group, m)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(lhs)
+    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a)
+    check(qmatmul(QE.GPTQ, config, a, *rhs, out_dtype=torch.bfloat16), config, rhs, a)
+    cfg, dtype = C.byref(_lib.GptqConfig(4, group, 1, 1)), _lib.QMM_F32 if lhs == torch.float32 else _lib.QMM_BF16
+    room = _lib.load().qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, dtype, m, n, k, 0)
+    least = _lib.load().qmm_matmul_workspace_bytes(QE.GPTQ.code, dtype, m, n, k)
+    for need in (room, max(room - 1, least), least):
+        check(c_call(config, rhs, a, need), config, rhs, a)
+
+
+@pytest.mark.parametrize("change", ["one column", "one group empty", "out of range"])
+def test_uneven_groups(change):
+    m, n, k, group = 37, 264, 2048, 128
+    config, (qweight, scales, qzeros, g_idx) = act_order(n, k, group, 5)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(2))
+    if change == "one column":
+        g_idx[7] = (g_idx[7] + 1) % (k // group)
+    elif change == "one group empty":
+        g_idx[g_idx == 3] = 4
+    else:  # (clamped to the last group)
+        g_idx[g_idx == k // group - 1] = 10**6
+        rhs = (qweight, scales, qzeros, g_idx.clamp(max=k // group - 1))
+        check(qmatmul(QE.GPTQ, config, a, qweight, scales, qzeros, g_idx), config, rhs, a)
+        return
+    check(qmatmul(QE.GPTQ, config, a, qweight, scales, qzeros, g_idx), config, (qweight, scales, qzeros, g_idx), a)
+
+
+def test_replayed_from_a_graph():
+    config, rhs = act_order(264, 1024, 128, 9)
+    a = torch.randn((40, 1024), device="cuda")
+    want = qmatmul(QE.GPTQ, config, a, *rhs)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = qmatmul(QE.GPTQ, config, a, *rhs)
+    for i in range(3):
+        a.copy_(torch.randn((40, 1024), device="cuda"))
+        rhs[3].copy_(rhs[3][torch.randperm(1024, device="cuda")])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, qmatmul(QE.GPTQ, config, a, *rhs))
+        assert not torch.equal(got, want)
