@@ -14,40 +14,18 @@
 //   acc += d * sum(u * a16) [+ -dmin * sum(mn * s)],  u: integer weights (sc * q, or q - zero), a16: the row scaled by a power of two and
 //   narrowed to fp16 (fp32 rows: hi + residual, both products into one accumulator), s: sub-block sums of the scaled row as hi + lo.
 //   Q6_K: sc * q may need 13 bits, so sc = 16 hi + lo gives two integer operands per weight (see gemm_planes.hip).
+#include <math.h>
 #include <stdlib.h>
 
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm_lhs.h"
-#include "qmm_internal.h"
+#include "gemm_direct.h"
 
 namespace qmm {
 
 namespace {
 
-typedef uint32_t gd_u4 __attribute__((ext_vector_type(4)));
-typedef uint32_t gd_u2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ half2v as_h2(uint32_t x) { return __builtin_bit_cast(half2v, x); }
-__device__ __forceinline__ uint32_t as_u32(half2v x) { return __builtin_bit_cast(uint32_t, x); }
-__device__ __forceinline__ uint32_t pk_add(uint32_t x, uint32_t y) { return as_u32(as_h2(x) + as_h2(y)); }
-// byte j of v under the byte `top` in both halves: with top 0x64 the fp16 pair 1024 + byte, with 0x68 2048 + 2 byte, with 0x78 32768 + 32 byte
-template <int J>
-__device__ __forceinline__ uint32_t byte_pair(uint32_t top4, uint32_t v) { return __builtin_amdgcn_perm(top4, v, 0x04000400u | (J << 16) | J); }
-
-// The operand order of the lhs: step t = 2 blk + a of 16 columns holds, for half wavefront g, the columns
-//   32 blk + 16 g + 8 a + slot order   (kOrderK: slots 0,2,1,3,4,6,5,7; kOrderGptq: 0,4,1,5,2,6,3,7)
-constexpr int kOrderK = 0, kOrderGptq = 1;  // (Q4_0: 32 blk + 16 a + 8 g + the slots of kOrderK)
-
-// Sizes of what the preparation launch leaves behind.  Every row tile of 32 rows: k / 16 operands of 1 KB, rounded up to whole units of 16 (fp32 lhs: pairs of
-// them, hi then residual), and room for one more unit behind the last (the loop reads ahead); sums: one operand per 256 columns; inverse row scales.
-struct DirectSpace {
-    _Float16* a16;
-    _Float16* sums;
-    float* inv;
-    int64_t bytes;
-};
 DirectSpace direct_space(void* ws, bool f32, bool with_sums, int64_t m, int64_t k) {
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     const int64_t tiles = (m + 31) / 32;
@@ -63,14 +41,6 @@ DirectSpace direct_space(void* ws, bool f32, bool with_sums, int64_t m, int64_t 
     p.bytes = off;
     return p;
 }
-
-// The matrices of one launch (they share the lhs): their results, and where each ends in the grid, in eights of column tiles.
-struct DirectMats {
-    const uint8_t* w[kDirectMaxMats];
-    float* out[kDirectMaxMats];
-    int n[kDirectMaxMats], end[kDirectMaxMats];
-    int count;
-};
 
 // ---------------------------------------------------------------------------------------------------------------------------
 // preparation: one workgroup per lhs row (the first m workgroups), then zeroing of `out` for two workgroups per tile
@@ -240,406 +210,6 @@ __global__ __launch_bounds__(256) void direct_prep_q8_kernel(const AT* __restric
     }
 }
 
-// ---------------------------------------------------------------------------------------------------------------------------
-// the weights of one wavefront: what it holds of a unit of K, how a step's operands come out of it
-// ---------------------------------------------------------------------------------------------------------------------------
-struct WeightTensors {
-    const uint8_t* w;        // K-quant blocks, or GPTQ qweight
-    const uint16_t* scales;  // GPTQ
-    const uint32_t* qzeros;
-    int n, k, group;
-};
-
-// The packed rows of a K-quant: 32 FN columns x one block.  A lane that loaded its own column's codes would touch a cache line of its
-// own with every load (64 lines an instruction, which took longer than everything else here), so the wavefront loads the blocks as they
-// lie in memory, 16 bytes per lane, a whole unit ahead, and hands them out through a part of LDS that is its own (no barrier).
-template <int BPB, int FN>
-struct StagedRows {
-    static constexpr int kPieces = (BPB + 15) / 16, kRow = kPieces * 16;  // the last piece ends with the block (Q6_K: bytes 194 .. 209)
-    static constexpr int kTotal = 32 * FN * kPieces, kLoads = (kTotal + 63) / 64, kBytes = 32 * FN * kRow;
-    const uint8_t* w;
-    uint8_t* lds;
-    uint32_t off[kLoads];
-    gd_u4 raw[kLoads];
-    struct __attribute__((packed, aligned(2))) Bytes16 {
-        gd_u4 v;
-    };
-    __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* stage) {
-        w = t.w;
-        lds = stage;
-#pragma unroll
-        for (int j = 0; j < kLoads; j++) {
-            const int i = min(j * 64 + lane, kTotal - 1), row = i / kPieces, piece = i - row * kPieces;
-            off[j] = (uint32_t)min(n0 + row, t.n - 1) * (uint32_t)(t.k / 256 * BPB) + min(16 * piece, BPB - 16);
-        }
-    }
-    __device__ __forceinline__ void load(int unit) {
-        const uint8_t* b = w + (int64_t)unit * BPB;
-#pragma unroll
-        for (int j = 0; j < kLoads; j++) {
-            if constexpr (BPB % 16 == 0) raw[j] = *(const gd_u4*)(b + off[j]);
-            else raw[j] = ((const Bytes16*)(b + off[j]))->v;
-        }
-    }
-    __device__ __forceinline__ void to_lds(int lane) {
-#pragma unroll
-        for (int j = 0; j < kLoads; j++)
-            if (j * 64 + 63 < kTotal || j * 64 + lane < kTotal) *(gd_u4*)(lds + j * 1024 + lane * 16) = raw[j];
-    }
-};
-
-// Q4_K, Q5_K.  Lane (column nl of a group, half g) takes bytes 16 g .. 16 g + 15 of each of the four 32-byte code runs of a block: run c is
-// sub-block 2 c in its low nibbles and 2 c + 1 in its high ones.  A nibble masked in place reads as the fp16 subnormal q 2^-24 (low) or
-// q 2^-20 (high); times 32 sc or 2 sc it is sc q 2^-19, exact (sc q at most 1953), and a normal number from sc q = 32 on: the matrix cores
-// keep fewer bits of a sum whose operands are subnormal (fp32 rows, 2.5e-7 relative error against 6e-7 with sc q 2^-24).
-template <int ENC, int FN>
-struct KQuantWeights {
-    static constexpr int kSteps = 16, kFlush = 16, kPlanes = 1;
-    static constexpr bool kMin = true, kPairs = false;
-    static constexpr int kCodes = ENC == QMM_Q5_K ? 48 : 16;
-    using Rows = StagedRows<ENC == QMM_Q5_K ? Q5_K_BPB : Q4_K_BPB, FN>;
-    static constexpr int kStage = Rows::kBytes;
-    Rows rows;
-    const uint8_t* mine;  // the lane's column in LDS
-    int goff, lane_;
-    gd_u4 q[FN][2], fifth[ENC == QMM_Q5_K ? FN : 1];
-    uint32_t scs[FN][2], mns[FN][2], dm[FN];
-
-    __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* stage) {
-        rows.init(t, n0, lane, stage);
-        goff = 16 * (lane >> 5);
-        lane_ = lane;
-        mine = stage + (lane & 31) * Rows::kRow;
-    }
-    __device__ __forceinline__ void load(int unit) { rows.load(unit); }
-    __device__ __forceinline__ void read_codes(int c) {
-#pragma unroll
-        for (int f = 0; f < FN; f++) q[f][c & 1] = *(const gd_u4*)(mine + f * 32 * Rows::kRow + goff + (kCodes + 32 * c));
-    }
-    // the loaded unit becomes the current one
-    __device__ __forceinline__ void open() {
-        rows.to_lds(lane_);
-        read_codes(0);
-#pragma unroll
-        for (int f = 0; f < FN; f++) {
-            if constexpr (ENC == QMM_Q5_K) fifth[f] = *(const gd_u4*)(mine + f * 32 * Rows::kRow + goff + 16);
-            const gd_u4 hdr = *(const gd_u4*)(mine + f * 32 * Rows::kRow);
-            const uint32_t s0 = hdr.y, s1 = hdr.z, s2 = hdr.w;
-            dm[f] = hdr.x;
-            scs[f][0] = s0 & 0x3f3f3f3fu;
-            scs[f][1] = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
-            mns[f][0] = s1 & 0x3f3f3f3fu;
-            mns[f][1] = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
-        }
-    }
-    // operands of step T (plane 0 only)
-    template <int T>
-    __device__ __forceinline__ void step(int f, half8 (&b)[1]) const {
-        constexpr int c = T >> 2, h = (T >> 1) & 1, a = T & 1, blk = 2 * c + h;
-        uint32_t sp;
-        if constexpr (h == 0) sp = pk_add(byte_pair<(blk & 3)>(0x78787878u, scs[f][blk >> 2]), 0xF800F800u);  // 32768 + 32 sc - 32768
-        else sp = pk_add(byte_pair<(blk & 3)>(0x68686868u, scs[f][blk >> 2]), 0xE800E800u);                   // 2048 + 2 sc - 2048
-        constexpr uint32_t mask = h == 0 ? 0x000F000Fu : 0x00F000F0u;
-        uint32_t v[4];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const uint32_t x = q[f][c & 1][2 * a + i], y = x >> 8;
-            v[2 * i] = x & mask;
-            v[2 * i + 1] = y & mask;
-            if constexpr (ENC == QMM_Q5_K) {
-                constexpr int bit = h == 0 ? 4 : 8;  // where the fifth bit goes, from bit blk of its byte
-                constexpr uint32_t fm = h == 0 ? 0x00100010u : 0x01000100u;
-                const uint32_t e = fifth[f][2 * a + i];
-                v[2 * i] |= (bit >= blk ? e << (bit - blk) : e >> (blk - bit)) & fm;
-                v[2 * i + 1] |= (bit >= blk + 8 ? e << (bit - blk - 8) : e >> (blk + 8 - bit)) & fm;
-            }
-        }
-        b[0] = pack4(pk_mul(v[0], sp), pk_mul(v[1], sp), pk_mul(v[2], sp), pk_mul(v[3], sp));
-    }
-    template <int T>
-    __device__ __forceinline__ void before_step() {
-        if constexpr ((T & 3) == 0 && T < 12) read_codes((T >> 2) + 1);
-    }
-    template <int T>
-    __device__ __forceinline__ void after_step(int) {}
-    __device__ __forceinline__ float scale(int f) const { return h2f((uint16_t)(dm[f] & 0xffffu)) * 524288.0f; }
-    __device__ __forceinline__ float min_scale(int f) const { return -h2f((uint16_t)(dm[f] >> 16)); }
-    __device__ __forceinline__ half8 min_operand(int f) const {  // the eight mins, for the hi sums (g = 0) and the lo sums (g = 1)
-        uint32_t v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            v[i] = pk_add(__builtin_amdgcn_perm(0x64646464u, mns[f][i >> 1], (i & 1) ? 0x04030402u : 0x04010400u), 0xE400E400u);
-        return pack4(v[0], v[1], v[2], v[3]);
-    }
-};
-
-// Q6_K.  Half block h: code bytes ql[0..31] (quarters 0 low, 2 high nibbles) and ql[32..63] (quarters 1, 3), two more bits of all four
-// quarters in qh[0..31]; a lane takes bytes 16 g .. 16 g + 15 of each.  (u - 32) 2^-24 or 2^-20 as above, then the two integer operands
-// 16 (sc >> 4) q and (sc & 15) q, times 2^-19.
-template <int FN>
-struct Q6Weights {
-    static constexpr int kSteps = 16, kFlush = 16, kPlanes = 2;
-    static constexpr bool kMin = false, kPairs = false;
-    using Rows = StagedRows<Q6_K_BPB, FN>;
-    static constexpr int kStage = Rows::kBytes;
-    Rows rows;
-    const uint8_t* mine;
-    int g, lane_;
-    gd_u4 ql[FN][2], qh[FN];
-    uint32_t sc[FN][2], d[FN];
-
-    __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* stage) {
-        rows.init(t, n0, lane, stage);
-        g = lane >> 5;
-        lane_ = lane;
-        mine = stage + (lane & 31) * Rows::kRow;
-    }
-    __device__ __forceinline__ void load(int unit) { rows.load(unit); }
-    __device__ __forceinline__ void read_half(int h) {
-#pragma unroll
-        for (int f = 0; f < FN; f++) {
-            const uint8_t* p = mine + f * 32 * Rows::kRow + 16 * g;
-            ql[f][0] = *(const gd_u4*)(p + 64 * h);
-            ql[f][1] = *(const gd_u4*)(p + (64 * h + 32));
-            qh[f] = *(const gd_u4*)(p + (128 + 32 * h));
-        }
-    }
-    __device__ __forceinline__ void open() {
-        rows.to_lds(lane_);
-        read_half(0);
-#pragma unroll
-        for (int f = 0; f < FN; f++) {
-            // the lane's scales: index 2 (4 h + quarter) + g, as bytes 4 h + quarter of two dwords
-            const gd_u4 s = *(const gd_u4*)(mine + f * 32 * Rows::kRow + 192);
-            const uint32_t sel = g ? 0x07050301u : 0x06040200u;
-            sc[f][0] = __builtin_amdgcn_perm(s.y, s.x, sel);
-            sc[f][1] = __builtin_amdgcn_perm(s.w, s.z, sel);
-            d[f] = *(const uint16_t*)(mine + f * 32 * Rows::kRow + 222);
-        }
-    }
-    template <int T>
-    __device__ __forceinline__ void step(int f, half8 (&b)[2]) const {
-        constexpr int h = T >> 3, quarter = (T >> 1) & 3, a = T & 1;
-        constexpr bool high = quarter >= 2;
-        const uint32_t sb = (uint32_t)((int32_t)(sc[f][h] << (24 - 8 * quarter)) >> 24);  // sign-extended
-        // sc = 16 hi + lo; low nibbles: 32 times 16 hi and lo, high nibbles (codes 16-fold): twice
-        const _Float16 s1 = (_Float16)(float)((int)sb >> 4), s0 = (_Float16)(float)(sb & 15u);
-        const _Float16 m1 = s1 * (_Float16)(high ? 32.0f : 512.0f), m0 = s0 * (_Float16)(high ? 2.0f : 32.0f);
-        const uint32_t p1 = as_u32(half2v{m1, m1}), p0 = as_u32(half2v{m0, m0});
-        constexpr uint32_t mask = high ? 0x00F000F0u : 0x000F000Fu, hm = high ? 0x03000300u : 0x00300030u;
-        constexpr int bit = high ? 8 : 4;
-        constexpr uint32_t minus32 = high ? 0x82008200u : 0x80208020u;  // -32 in the unit of the codes
-        uint32_t v[4];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const uint32_t x = ql[f][quarter & 1][2 * a + i], e = qh[f][2 * a + i];
-            constexpr int from = 2 * quarter;
-            const uint32_t e0 = bit >= from ? e << (bit - from) : e >> (from - bit);
-            const uint32_t e1 = bit >= from + 8 ? e << (bit - from - 8) : e >> (from + 8 - bit);
-            v[2 * i] = pk_add((x & mask) | (e0 & hm), minus32);
-            v[2 * i + 1] = pk_add(((x >> 8) & mask) | (e1 & hm), minus32);
-        }
-        b[0] = pack4(pk_mul(v[0], p1), pk_mul(v[1], p1), pk_mul(v[2], p1), pk_mul(v[3], p1));
-        b[1] = pack4(pk_mul(v[0], p0), pk_mul(v[1], p0), pk_mul(v[2], p0), pk_mul(v[3], p0));
-    }
-    template <int T>
-    __device__ __forceinline__ void before_step() {
-        if constexpr (T == 7) read_half(1);  // (step 7 is unpacked)
-    }
-    template <int T>
-    __device__ __forceinline__ void after_step(int) {}
-    __device__ __forceinline__ float scale(int f) const { return h2f((uint16_t)d[f]) * 524288.0f; }
-    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
-    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
-};
-
-// GPTQ, plain groups.  Word row 32 unit + 4 blk + 2 g + a is a lane's share of step 2 blk + a.  With FN = 2 a lane owns two neighbouring columns
-// (8-byte loads).  FLUSH: steps per scale block, 8 (groups that are multiples of 128) or 2 (any group: blocks of 32).  A K that is no multiple of
-// 256 ends in a partial unit: its lhs columns beyond K are zeros, its words and scales the last ones of the tensors.
-template <int FN, int FLUSH>
-struct GptqWeights {
-    static constexpr int kSteps = 16, kFlush = FLUSH, kPlanes = 1;
-    static constexpr bool kMin = false, kPairs = FN == 2;
-    static constexpr int kBlocks = 16 / FLUSH, kStage = 0;
-    const uint32_t* qw;
-    const uint16_t* scales;
-    const uint32_t* qzeros;
-    int n, group, col, g, rows, groups;
-    uint32_t q[16][FN], s_next[kBlocks], z_next[kBlocks], s_raw[kBlocks], z_raw[kBlocks];
-
-    __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t*) {
-        qw = (const uint32_t*)t.w;
-        scales = t.scales;
-        qzeros = t.qzeros;
-        n = t.n;
-        group = t.group;
-        rows = t.k >> 3;
-        groups = t.k / group;
-        g = lane >> 5;
-        col = min(n0 + FN * (lane & 31), n - FN);
-    }
-    __device__ __forceinline__ void load_words(int unit, int t) {
-        const int row = min(32 * unit + 4 * (t >> 1), rows - 4) + (t & 1);  // (K / 8 is a multiple of 4)
-        const uint32_t* p = qw + (int64_t)row * n + (uint32_t)(2 * g * n + col);
-#pragma unroll
-        for (int f = 0; f < FN; f++) q[t][f] = p[f];
-    }
-    __device__ __forceinline__ void load_head(int unit) {
-#pragma unroll
-        for (int i = 0; i < kBlocks; i++) {
-            const int64_t gi = min((unit * 256 + i * 16 * FLUSH) / group, groups - 1);
-            const uint16_t* sp = scales + gi * n + col;
-            s_next[i] = sp[0];
-            if constexpr (FN == 2) s_next[i] |= (uint32_t)sp[1] << 16;
-            z_next[i] = qzeros[gi * (n >> 3) + (col >> 3)];
-        }
-    }
-    __device__ __forceinline__ void load(int unit) {  // (the words of later units step by step, as those of this one are used up)
-        load_head(unit);
-    }
-    __device__ __forceinline__ void load_first(int unit) {
-        load_head(unit);
-#pragma unroll
-        for (int t = 0; t < 16; t++) load_words(unit, t);
-    }
-    __device__ __forceinline__ void open() {
-#pragma unroll
-        for (int i = 0; i < kBlocks; i++) {
-            s_raw[i] = s_next[i];
-            z_raw[i] = z_next[i];
-        }
-    }
-    template <int T>
-    __device__ __forceinline__ void before_step() {}
-    template <int T>
-    __device__ __forceinline__ void step(int f, half8 (&b)[1]) const {
-        const uint32_t z = ((z_raw[T / FLUSH] >> (4 * ((col + f) & 7))) & 0xFu) + 1u;
-        // nibbles under 0x6400 read as 1024 + q, in their place one nibble up under 0x5400 as 64 + q; the difference to 1024 (64) + zero is
-        // exact.  (As fp16 subnormals, codes this small lost bits in the matrix-core sums: 3e-5 relative, against 3e-7.)
-        const uint32_t m0 = 0xE400E400u | (z * 0x00010001u), m1 = 0xD400D400u | (z * 0x00100010u);
-        const uint32_t x = q[T][f], y = x >> 8;
-        b[0] = pack4(pk_add((x & 0x000F000Fu) | 0x64006400u, m0), pk_add((x & 0x00F000F0u) | 0x54005400u, m1),
-                     pk_add((y & 0x000F000Fu) | 0x64006400u, m0), pk_add((y & 0x00F000F0u) | 0x54005400u, m1));
-    }
-    template <int T>
-    __device__ __forceinline__ void after_step(int next_unit) { load_words(next_unit, T); }
-    template <int I>
-    __device__ __forceinline__ float scale_at(int f) const { return h2f((uint16_t)(f ? s_raw[I] >> 16 : s_raw[I] & 0xffffu)); }
-    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
-    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
-};
-
-// Q4_0: the exact integer block dots of the Q8_0 lhs (codes as fp16) with q - 8, block by block.  Lane half g takes bytes 8 g .. 8 g + 7 of a
-// block: its low nibbles are columns 8 g + 0..7 of the block (step a = 0), the high ones 16 + 8 g + 0..7 (a = 1).  Rows
-// whose K is no multiple of 256 end in a partial unit: what lies behind the row's end is read as zeros.
-template <int FN>
-struct Q40Weights {
-    static constexpr int kSteps = 16, kFlush = 2, kPlanes = 1;
-    static constexpr bool kMin = false, kPairs = false;
-    static constexpr int kUnit = 8 * Q4_0_BPB, kPieces = kUnit / 16;
-    static constexpr int kTotal = 32 * FN * kPieces, kLoads = (kTotal + 63) / 64, kStage = 32 * FN * kUnit;
-    const uint8_t* w;
-    uint8_t* lds;
-    const uint8_t* mine;
-    int row_bytes, g, lane_;
-    uint32_t off[kLoads];
-    gd_u4 raw[kLoads];
-    uint32_t x[FN][2][3];  // block b in x[f][b & 1]: its eight code bytes in dwords 0, 1 (odd b) or from byte 2 of dword 0 on (even b)
-    uint32_t d[FN][8];     // (of lanes g = 0; zero in the others)
-    struct __attribute__((packed, aligned(2))) Bytes16 {
-        gd_u4 v;
-    };
-
-    __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* stage) {
-        w = t.w;
-        lds = stage;
-        g = lane >> 5;
-        lane_ = lane;
-        mine = stage + (lane & 31) * kUnit;
-        row_bytes = t.k / 32 * Q4_0_BPB;
-#pragma unroll
-        for (int j = 0; j < kLoads; j++) {
-            const int i = min(j * 64 + lane, kTotal - 1), row = i / kPieces, piece = i - row * kPieces;
-            off[j] = (uint32_t)min(n0 + row, t.n - 1) * (uint32_t)row_bytes + 16 * piece;
-        }
-    }
-    __device__ __forceinline__ void load(int unit) {
-        const uint8_t* b = w + (int64_t)unit * kUnit;
-        const int left = row_bytes - unit * kUnit;  // bytes of the rows from here on
-        if (left >= kUnit) {
-#pragma unroll
-            for (int j = 0; j < kLoads; j++) raw[j] = ((const Bytes16*)(b + off[j]))->v;
-        } else {
-#pragma unroll
-            for (int j = 0; j < kLoads; j++) {
-                const int i = min(j * 64 + lane_, kTotal - 1), at = (i % kPieces) * 16;
-                // the last 16 bytes of the row, moved down to the place the piece would have (rows are at least 18 bytes long)
-                const int over = max(at + 16 - left, 0);
-                const gd_u4 v = ((const Bytes16*)(b + off[j] - over))->v;
-                uint64_t lo = v.x | (uint64_t)v.y << 32, hi = v.z | (uint64_t)v.w << 32;
-                if (over >= 16) lo = hi = 0;
-                else if (over >= 8) { lo = hi >> (8 * over - 64); hi = 0; }
-                else if (over > 0) { lo = (lo >> (8 * over)) | (hi << (64 - 8 * over)); hi >>= 8 * over; }
-                raw[j] = gd_u4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
-            }
-        }
-    }
-    __device__ __forceinline__ void read_block(int b) {
-#pragma unroll
-        for (int f = 0; f < FN; f++) {
-            const uint32_t* p = (const uint32_t*)(mine + f * 32 * kUnit + 8 * g + (b & 1 ? 18 * b + 2 : 18 * b));
-            x[f][b & 1][0] = p[0];
-            x[f][b & 1][1] = p[1];
-            if (!(b & 1)) x[f][b & 1][2] = p[2];
-        }
-    }
-    __device__ __forceinline__ void open() {
-#pragma unroll
-        for (int j = 0; j < kLoads; j++)
-            if (j * 64 + 63 < kTotal || j * 64 + lane_ < kTotal) *(gd_u4*)(lds + j * 1024 + lane_ * 16) = raw[j];
-        read_block(0);
-#pragma unroll
-        for (int f = 0; f < FN; f++)
-#pragma unroll
-            for (int b = 0; b < 8; b++) d[f][b] = g ? 0u : (uint32_t)*(const uint16_t*)(mine + f * 32 * kUnit + 18 * b);
-    }
-    template <int T>
-    __device__ __forceinline__ void step(int f, half8 (&b)[1]) const {
-        constexpr int blk = T >> 1, a = T & 1;
-        uint32_t v[4];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const uint32_t q = blk & 1 ? x[f][1][i] : __builtin_amdgcn_alignbyte(x[f][0][i + 1], x[f][0][i], 2), y = q >> 8;
-            if constexpr (a == 0) {
-                v[2 * i] = pk_add((q & 0x000F000Fu) | 0x64006400u, 0xE408E408u);  // 1024 + q - 1032
-                v[2 * i + 1] = pk_add((y & 0x000F000Fu) | 0x64006400u, 0xE408E408u);
-            } else {
-                v[2 * i] = pk_add((q & 0x00F000F0u) | 0x54005400u, 0xD480D480u);  // 64 + q - 72
-                v[2 * i + 1] = pk_add((y & 0x00F000F0u) | 0x54005400u, 0xD480D480u);
-            }
-        }
-        b[0] = pack4(v[0], v[1], v[2], v[3]);
-    }
-    template <int T>
-    __device__ __forceinline__ void before_step() {
-        if constexpr ((T & 1) == 0 && T < 14) read_block((T >> 1) + 1);
-    }
-    template <int T>
-    __device__ __forceinline__ void after_step(int) {}
-    template <int B>
-    __device__ __forceinline__ half8 scale_operand(int f) const {
-        const uint32_t v = d[f][B] << (16 * (B & 1));
-        return pack4(B >> 1 == 0 ? v : 0u, B >> 1 == 1 ? v : 0u, B >> 1 == 2 ? v : 0u, B >> 1 == 3 ? v : 0u);
-    }
-    __device__ __forceinline__ float scale(int) const { return 0.0f; }
-    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
-    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
-};
-
-template <int ENC, int FN, int FLUSH>
-using WeightsOf = std::conditional_t<ENC == QMM_GPTQ, GptqWeights<FN, FLUSH>, std::conditional_t<ENC == QMM_Q6_K, Q6Weights<FN>,
-                  std::conditional_t<ENC == QMM_Q4_0, Q40Weights<FN>, KQuantWeights<ENC == QMM_Q5_K ? QMM_Q5_K : QMM_Q4_K, FN>>>>;
-
 constexpr int direct_ahead(int flush, int fm, int fn, bool hilo) {
     if (fm * fn == 2) return hilo ? 4 : 8;
     return flush == 2 && hilo ? 8 : 16;
@@ -647,15 +217,6 @@ constexpr int direct_ahead(int flush, int fm, int fn, bool hilo) {
 
 template <typename W>
 constexpr int direct_slot(int frags) { return W::kStage > frags * 4096 ? W::kStage : frags * 4096; }
-
-// compile-time loop: f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>)
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void unrolled(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        unrolled<N, I + 1>(f);
-    }
-}
 
 }  // namespace
 
@@ -858,10 +419,6 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
 
 namespace {
 
-struct DirectPlan {
-    int fm, fn, wk, shares;
-};
-
 int64_t direct_units(int64_t k) { return (k + 255) / 256; }
 
 // What a call takes, in microseconds: launches and the preparation of the lhs, a fixed part per round of workgroups (eight wavefronts fill
@@ -872,7 +429,7 @@ struct DirectCost {
     float base, round, weights, lhs, out;  // us, us, us per MB of packed weights, us per million lhs values, us per million results and share
     float unit[6];                         // us per unit of K: the plans of kDirectPlans
 };
-constexpr DirectPlan kDirectPlans[6] = {{1, 1, 8, 0}, {2, 1, 8, 0}, {1, 2, 8, 0}, {1, 1, 4, 0}, {2, 1, 4, 0}, {1, 2, 4, 0}};
+constexpr DirectPlan kDirectPlans[6] = {{1, 1, 8, 0, 1}, {2, 1, 8, 0, 1}, {1, 2, 8, 0, 1}, {1, 1, 4, 0, 1}, {2, 1, 4, 0, 1}, {1, 2, 4, 0, 1}};
 constexpr DirectCost kDirectCost[6][2] = {
     // bf16 lhs; fp32 lhs
     {{3.98f, 1.61f, 0.18f, 3.99f, 2.25f, {2.43f, 3.65f, 4.78f, 1.86f, 2.70f, 3.76f}}, {3.99f, 1.60f, 0.18f, 3.98f, 2.32f, {2.43f, 3.63f, 4.77f, 1.86f, 2.70f, 3.75f}}},  // Q4_0
@@ -889,23 +446,54 @@ double direct_us(const DirectCost& c, int plan, int shares, int encoding, int64_
     const double bytes = encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56;
     return c.base + rounds * (c.round + walk * c.unit[plan]) + c.weights * (bytes * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
 }
+// The same for the kernel whose wavefronts share the lhs, fitted to 67 problems per encoding and lhs type (33 .. 1300 rows) in every plan: 3 .. 4 %
+// mean error.  It wins where its tiles of 64 x 256 (64 x 128) fill the part with most of K in a workgroup.  us, direct plans / shared: Q4_K, bf16 rows:
+// 14336 x 4096 100 rows 36 / 30, 200 rows 59 / 49, 4096 x 4096 500 rows 42 / 35; fp32 rows: 14336 x 4096 500 rows 183 / 150; Q6_K 4096 x 14336 500
+// bf16 rows 153 / 134; but 4096 x 4096 200 bf16 rows 23.5 / 24.4, 64 rows 12 / 18.
+struct SharedCost {
+    float base, round, weights, lhs, out;
+    float unit[3], unit_alone;  // the plans of kSharedPlans; four wavefronts with a compute unit to themselves
+    float direct, direct_slope; // what the direct plans took in that measurement (weights from the last-level cache) over direct_us, and per factor e beyond 30 us
+};
+constexpr DirectPlan kSharedPlans[3] = {{2, 1, 1, 0, 8}, {2, 1, 2, 0, 4}, {2, 1, 1, 0, 4}};
+constexpr SharedCost kSharedCost[6][2] = {
+    // bf16 lhs; fp32 lhs
+    {{5.92f, 0.42f, 0.106f, 2.20f, 2.84f, {3.49f, 3.63f, 2.86f}, 2.59f, 1.11f, 0.04f}, {6.05f, 0.25f, 0.090f, 2.08f, 2.89f, {3.51f, 3.66f, 2.89f}, 2.60f, 1.10f, 0.05f}},  // Q4_0
+    {{3.82f, 2.47f, 0.071f, 2.18f, 2.93f, {1.97f, 2.26f, 1.95f}, 1.63f, 1.11f, 0.01f}, {4.28f, 1.58f, 0.068f, 3.53f, 3.96f, {3.24f, 3.78f, 3.24f}, 2.38f, 1.15f, 0.05f}},  // Q4_K
+    {{4.75f, 1.94f, 0.076f, 2.26f, 2.94f, {2.45f, 2.65f, 2.29f}, 1.83f, 1.11f, -0.01f}, {4.72f, 1.40f, 0.080f, 3.55f, 3.94f, {3.48f, 4.19f, 3.46f}, 2.57f, 1.16f, 0.04f}},  // Q5_K
+    {{4.41f, 1.99f, 0.064f, 2.55f, 3.16f, {3.51f, 3.88f, 3.24f}, 2.26f, 1.13f, 0.05f}, {3.95f, 1.33f, 0.075f, 4.11f, 4.77f, {5.27f, 6.04f, 5.26f}, 3.40f, 1.20f, 0.15f}},  // Q6_K
+    {{6.52f, 0.30f, 0.052f, 2.16f, 2.66f, {2.30f, 2.48f, 1.78f}, 1.67f, 1.08f, -0.06f}, {6.42f, 0.00f, 0.037f, 3.25f, 3.38f, {3.46f, 4.02f, 3.09f}, 2.62f, 1.11f, 0.01f}},  // GPTQ, groups of 128
+    {{7.46f, 0.00f, 0.070f, 2.30f, 2.59f, {3.40f, 3.57f, 2.55f}, 2.38f, 1.10f, 0.04f}, {6.94f, 0.11f, 0.022f, 3.00f, 3.27f, {4.54f, 5.01f, 4.11f}, 3.21f, 1.14f, 0.05f}},  // GPTQ, other groups
+};
+double shared_us(const SharedCost& c, int plan, int shares, int encoding, int64_t m, int64_t n, int64_t k) {
+    const DirectPlan& p = kSharedPlans[plan];
+    const int64_t wgs = ((m + 63) / 64) * ((n + 32 * p.wn - 1) / (32 * p.wn)) * shares, slots = p.wn * p.wk == 8 ? 256 : 512;
+    const int64_t rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
+    const double unit = slots == 512 && wgs <= 256 ? c.unit_alone : c.unit[plan];
+    return c.base + rounds * (c.round + walk * unit) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
+}
 // whole_tiles: one workgroup per tile (bf16 results are stored, not added up); like: with that plan's cut of K
 DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, const DirectPlan* like = nullptr) {
     const int row = encoding == QMM_Q4_0 ? 0 : encoding == QMM_Q4_K ? 1 : encoding == QMM_Q5_K ? 2 : encoding == QMM_Q6_K ? 3 : group % 128 == 0 ? 4 : 5;
-    const DirectCost& c = kDirectCost[row][lhs_dtype == QMM_F32 ? 1 : 0];
-    DirectPlan best{1, 1, 8, 1};
-    double best_us = 1e30;
-    for (int i = 0; i < 6; i++)
-        for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
-            if (like && (kDirectPlans[i].wk != like->wk || shares != like->shares)) continue;
-            const double t = direct_us(c, i, shares, encoding, m, n, k);
-            if (t < best_us) {
-                best_us = t;
-                best = kDirectPlans[i];
-                best.shares = shares;
-            }
-        }
-    return best;
+    const int type = lhs_dtype == QMM_F32 ? 1 : 0;
+    DirectPlan best[2] = {{1, 1, 8, 1, 1}, {}};
+    double us[2] = {1e30, 1e30};  // of the best direct and the best shared plan
+    auto consider = [&](const DirectPlan& p, int shares, double t) {
+        const int kind = p.wn > 1 ? 1 : 0;
+        if (t >= us[kind] || (like && (p.wk != like->wk || shares != like->shares || kind != (like->wn > 1 ? 1 : 0)))) return;
+        us[kind] = t;
+        best[kind] = p;
+        best[kind].shares = shares;
+    };
+    const SharedCost& c = kSharedCost[row][type];
+    for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
+        for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, m, n, k));
+        if (m > 32 && !kernel_disabled("shared"))
+            for (int i = 0; i < 3; i++) consider(kSharedPlans[i], shares, shared_us(c, i, shares, encoding, m, n, k));
+    }
+    if (us[0] >= 1e30) return best[us[1] < 1e30 ? 1 : 0];
+    // (the margin: with it next to no problem of that measurement lost more than 5 % to a wrong choice)
+    return us[1] * (encoding == QMM_GPTQ ? 1.14 : 1.08) < us[0] * (c.direct + c.direct_slope * log(us[0] / 30)) ? best[1] : best[0];
 }
 
 template <int ENC, int FLUSH, int FM, int FN, int WK, bool HILO>
@@ -981,8 +569,17 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     }
     if (m < from) return false;
     if (r <= (f32 && encoding != QMM_Q4_0 ? 1.6 : 1)) return true;
-    // fp32 rows are split in two fp16 terms here and in the other kernels, so both multiply twice
-    if (f32) return m <= (w <= 24 || (encoding != QMM_Q4_0 && encoding != QMM_GPTQ) ? 720 : 450) || (k <= 1024 ? r <= 6 : m < 1100 && r <= 3.5);
+    // fp32 rows are split in two fp16 terms here and in the other kernels, so both multiply twice; the others take K in two passes.  us, others / here:
+    // Q4_K 14336 x 4096 800 rows 327 / 232, 5120 x 5120 1300 rows 239 / 198; Q6_K 14336 x 4096 800 rows 514 / 380.
+    const bool shared = !kernel_disabled("shared");
+    if (f32) {
+        if (shared && encoding != QMM_Q4_0 && (m <= 1100 || (m <= 1400 && r <= 5.5))) return true;
+        return m <= (w <= 24 || (encoding != QMM_Q4_0 && encoding != QMM_GPTQ) ? 720 : 450) || (k <= 1024 ? r <= 6 : m < 1100 && r <= 3.5);
+    }
+    // (one round of 64 x 256 tiles that fills the part by four fifths or more: 11008 x 4096 320 bf16 rows Q4_K 78 / 55, GPTQ 71 / 53, Q5_K 85 / 63;
+    // 8192 x 8192 500 rows Q6_K 205 / 162, Q5_K 145 / 119, but Q4_K 106 / 105 and GPTQ 92 / 101)
+    const int64_t tiles = (m + 63) / 64 * ((n + 255) / 256);
+    if (shared && tiles >= 205 && tiles <= 256 && k <= (encoding == QMM_Q4_K || encoding == QMM_GPTQ ? 4096 : 8192)) return true;
     return m <= anyway || (m <= 1100 && r <= most);
 }
 
@@ -1026,12 +623,16 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
         DirectMats mats{};
         int64_t n = 0;
         for (int i = j; i < count; i++) {
-            if (done[i] || plans[i].wk != pl.wk || plans[i].shares != pl.shares) continue;
+            if (done[i] || plans[i].wk != pl.wk || plans[i].shares != pl.shares || (plans[i].wn > 1) != (pl.wn > 1)) continue;
             mats.w[mats.count] = (const uint8_t*)ws[i], mats.out[mats.count] = outs[i], mats.n[mats.count++] = (int)ns[i];
             n += ns[i];
             done[i] = true;
         }
         if (mats.count > 1) pl = direct_plan(encoding, lhs_dtype, m, n, k, group, false, &pl);
+        if (pl.wn > 1) {
+            e = launch_gemm_shared(encoding, f32 && !q40, pl, wt, mats, p, out16, m, units, s);
+            continue;
+        }
 #define QMM_GD_ENC(ENC, FLUSH) \
     e = f32 ? run_direct_plan<ENC, FLUSH, true>(pl, wt, mats, p, out16, m, units, s) : run_direct_plan<ENC, FLUSH, false>(pl, wt, mats, p, out16, m, units, s)
         if (q40) e = run_direct_plan<QMM_Q4_0, 2, false>(pl, wt, mats, p, out16, m, units, s);

@@ -62,8 +62,23 @@ def test_edges(enc, group, odd, lhs):
         check(out, enc, config, rhs, a)
 
 
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("enc,group,odd", [(QE.Q4_0, 0, 32), (QE.Q4_K, 0, 0), (QE.Q5_K, 0, 0), (QE.Q6_K, 0, 0), (QE.GPTQ, 128, 128), (QE.GPTQ, 32, 32)])
+def test_shared_lhs_edges(enc, group, odd, lhs):
+    """Sizes at which the wavefronts of a workgroup share the lhs: ragged last tiles of 64 rows and of 128 and 256 columns, one and two parts of K
+    (of one unit, of unequal lengths), one and two workgroups a tile."""
+    for m, n, k in ((200, 14344, 2048), (200, 14344, 2304 + odd), (65, 14600, 1280), (97, 11016, 2048 + odd), (449, 4104, 2304), (500, 4104, 4352 + odd),
+                    (321, 11008, 256), (130, 14344, 256 + odd)):
+        config, rhs = weights(enc, group, n, k)
+        a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(lhs)
+        a[m // 2] *= 1e-6
+        a[m - 1] = 0.0
+        check(qmatmul(enc, config, a, *rhs), enc, config, rhs, a)
+        check(qmatmul(enc, config, a, *rhs, out_dtype=torch.bfloat16), enc, config, rhs, a)
+
+
 @pytest.mark.parametrize("enc", [QE.Q4_0, QE.Q4_K, QE.Q5_K, QE.Q6_K])
-@pytest.mark.parametrize("m,k,ns", [(17, 768, (40, 264, 1000)), (33, 2304, (4104, 2056, 40, 1, 31)), (3, 1024, (6400, 40, 6400))])
+@pytest.mark.parametrize("m,k,ns", [(17, 768, (40, 264, 1000)), (33, 2304, (4104, 2056, 40, 1, 31)), (3, 1024, (6400, 40, 6400)), (200, 2048, (14344, 14344, 264))])
 def test_group_equals_separate_calls(enc, m, k, ns):
     a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m))
     rhs = [weights(enc, 0, n, k)[1] for n in ns]
