@@ -6,7 +6,7 @@
 // (hi, plus a residual plane) after an exact power-of-two scaling, the fp32 super-block scale is
 // applied in the lanes and the min term is one extra matrix product per super-block.
 //
-// Shape of the work: a workgroup of 8 wavefronts walks a list of up to 4 weight tiles of 16 rows.
+// Shape of the work: a workgroup of 8 wavefronts walks a list of up to 4 weight tiles of 16 rows (8 with up to four lhs rows).
 // The super-blocks of a row are dealt to the wavefronts in groups of 16, two per wavefront; a
 // wavefront's lhs fragments for its two super-blocks of a group are held in registers and reused
 // for every tile of the workgroup.  The weights of a (group, tile) item, 288 contiguous bytes of
@@ -49,6 +49,7 @@ constexpr int kSlots = 3;                       // ring: one item being decoded,
 constexpr float kTwo18f = 262144.0f;
 constexpr int kWaves = 8;                       // wavefronts per workgroup
 constexpr int kMaxTiles = 4;                    // tiles per workgroup (private LDS accumulators per wavefront)
+constexpr int kMaxTilesFew = 8;                 // with up to four lhs rows, whose results are in half of the lanes
 constexpr int kPlaneStride = 528;               // staged lhs plane of one super-block: 512 bytes + 16 (bank spread)
 constexpr int kStageBytes = 2 * kPlaneStride + 32;  // hi plane, residual plane, 8 sub-block sums (hi, lo)
 constexpr int kRingBytes = kWaves * kSlots * kSlotBytes;
@@ -83,7 +84,11 @@ __device__ __forceinline__ void mm_body(const MmMats& mats, const AT* __restrict
     const int nn = lane & 15, kg = lane >> 4;
     uint8_t* ring = smem + wave * (kSlots * kSlotBytes);
     const uint32_t ring_lds = lds_address(ring);
-    float* accs = (float*)(smem + kRingBytes);  // [kWaves][kMaxTiles][4][64]
+    // Up to four lhs rows: the results (rows 0 .. 3, and 8 .. 11 for the residual) are in the lanes with even kg, and only those are kept.
+    constexpr bool kFew = INLINE && MROWS <= 4;
+    constexpr int kTiles = kFew ? kMaxTilesFew : kMaxTiles, kAccLanes = kFew ? 32 : 64;
+    static_assert(kWaves * kTiles * 4 * kAccLanes * 4 <= kAccBytes, "the accumulators fit");
+    float* accs = (float*)(smem + kRingBytes);  // [kWaves][kTiles][4][kAccLanes]
     const int ntiles = mats.tile_end[kLanesMaxMats - 1];  // 16-row tiles, numbered through the matrices (entries past count repeat the last)
     // One matrix (the plain call) needs nothing from the argument block per item; with several, the tile's matrix is
     // looked up there (dependent scalar loads per item).
@@ -91,7 +96,7 @@ __device__ __forceinline__ void mm_body(const MmMats& mats, const AT* __restrict
     const uint8_t* const w_first = mats.w[0];
     float* const out_first = mats.out[0];
     const int n_first = mats.n[0];
-    const int my_tiles = min(kMaxTiles, (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
+    const int my_tiles = min(kTiles, (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
     // group g is super-blocks [16 g, 16 g + 16): two per wavefront, or, when 8 or fewer are left, one
     const int ngrp_all = (nblk + kRunBlk * kWaves - 1) / (kRunBlk * kWaves);
     const int grp0 = KPART ? (int)blockIdx.y : 0;          // first group of this workgroup
@@ -417,9 +422,11 @@ __device__ __forceinline__ void mm_body(const MmMats& mats, const AT* __restrict
             }
         }
         // this wavefront's running sum of the tile over its groups
-        float* mine = accs + ((wave * kMaxTiles + ti) * 4) * 64 + lane;
+        if (!kFew || (kg & 1) == 0) {
+            float* mine = accs + ((wave * kTiles + ti) * 4) * kAccLanes + (kFew ? 16 * (kg >> 1) + nn : lane);
 #pragma unroll
-        for (int r = 0; r < 4; r++) mine[r * 64] = grp == grp0 ? acc[r] : mine[r * 64] + acc[r];
+            for (int r = 0; r < 4; r++) mine[r * kAccLanes] = grp == grp0 ? acc[r] : mine[r * kAccLanes] + acc[r];
+        }
 
         slot = slot == kSlots - 1 ? 0 : slot + 1;
         if (++ti == my_tiles) { ti = 0; grp++; }
@@ -442,8 +449,8 @@ __device__ __forceinline__ void mm_body(const MmMats& mats, const AT* __restrict
         float v = 0.0f;
 #pragma unroll
         for (int ww = 0; ww < kWaves; ww++) {
-            const float* slot_r = accs + ((ww * kMaxTiles + t) * 4 + r) * 64;
-            v += INLINE ? slot_r[lane & 31] + slot_r[(lane & 31) + 32] : slot_r[lane];
+            const float* slot_r = accs + ((ww * kTiles + t) * 4 + r) * kAccLanes;
+            v += kFew ? slot_r[nn] + slot_r[nn + 16] : INLINE ? slot_r[lane & 31] + slot_r[(lane & 31) + 32] : slot_r[lane];
         }
         if (row < m && col < n) out[(int64_t)row * n + col] = INLINE ? v : v * inv[row];
     }
@@ -567,7 +574,9 @@ hipError_t launch_gemv_q4_k_mm_grouped(const void* lhs, int lhs_dtype, int count
     }
     // every workgroup gets the same number of tiles (at most kMaxTiles), one workgroup per compute unit when that fits
     // (more tiles on fewer workgroups is slower at every size: 4096 x 14336, 4 rows: 18.1 / 23.8 / 36.0 us with 1 / 2 / 4 tiles)
-    const int64_t per_wg = std::min<int64_t>(kMaxTiles, (ntiles + cus - 1) / cus);
+    // (a second round of workgroups starts over, 6 us before its second tile: gate and up of 14336 x 4096 with 4 rows, 1792 tiles, as 448
+    // workgroups of 4 25.8 us, as 256 of 7 20.8)
+    const int64_t per_wg = std::min<int64_t>(m <= 4 ? kMaxTilesFew : kMaxTiles, (ntiles + cus - 1) / cus);
     const int64_t wgs = (ntiles + per_wg - 1) / per_wg;
     dim3 grid((unsigned)wgs), block(64 * kWaves);
     if (m <= 8) {
