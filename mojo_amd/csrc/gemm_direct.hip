@@ -570,10 +570,11 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     if (m < from) return false;
     if (r <= (f32 && encoding != QMM_Q4_0 ? 1.6 : 1)) return true;
     // fp32 rows are split in two fp16 terms here and in the other kernels, so both multiply twice; the others take K in two passes.  us, others / here:
-    // Q4_K 14336 x 4096 800 rows 327 / 232, 5120 x 5120 1300 rows 239 / 198; Q6_K 14336 x 4096 800 rows 514 / 380.
+    // Q4_K 14336 x 4096 800 rows 327 / 232, 5120 x 5120 1300 rows 239 / 198; Q6_K 14336 x 4096 800 rows 514 / 380;
+    // but GPTQ 4096 x 14336 1050 rows 470 / 560.
     const bool shared = !kernel_disabled("shared");
     if (f32) {
-        if (shared && encoding != QMM_Q4_0 && (m <= 1100 || (m <= 1400 && r <= 5.5))) return true;
+        if (shared && encoding != QMM_Q4_0 && (m <= 1100 || (m <= 1400 && r <= 5.5)) && (encoding != QMM_GPTQ || k <= 8192)) return true;
         return m <= (w <= 24 || (encoding != QMM_Q4_0 && encoding != QMM_GPTQ) ? 720 : 450) || (k <= 1024 ? r <= 6 : m < 1100 && r <= 3.5);
     }
     // (one round of 64 x 256 tiles that fills the part by four fifths or more: 11008 x 4096 320 bf16 rows Q4_K 78 / 55, GPTQ 71 / 53, Q5_K 85 / 63;

@@ -882,10 +882,12 @@ int qmm_repack(int encoding, const qmm_gptq_config* cfg, const void* const* rhs,
 static int64_t q4_0_repacked_min_rows(int64_t k) { return k > 4096 ? 96 : 80; }
 // With the planes at hand the direct GEMM on the packed tensors still wins while the weights are most of the traffic (the planes are 2 or 4
 // bytes a weight against 0.6 .. 0.8): us, planes / direct: Q5_K 4096 x 4096 128 bf16 rows 33 / 20, 300 rows 46 / 35; 14336 x 4096 200 rows
-// 69 / 60, 300 rows 81 / 93; 300 fp32 rows 167 / 117, 450 rows 178 / 186; Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.
+// 69 / 60, 300 rows 81 / 93; Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.  fp32 rows
+// walk the planes twice: 450 / 1050 rows, Q5_K 14336 x 4096 177 / 160, 470 / 329, 4096 x 14336 326 / 157, 459 / 388; Q6_K 4096 x 4096 152 / 70, 203 / 203;
+// Q4_K 14336 x 4096 199 / 178, 468 / 297 (700 rows 274 / 286); but GPTQ 14336 x 4096 148 / 159, 4096 x 14336 700 rows 247 / 291.
 static bool direct_over_planes(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const bool narrow = m * n <= (int64_t)1300 << 10;
-    return (narrow || m <= (lhs_dtype == QMM_F32 && encoding != QMM_Q4_0 ? 400 : 150)) && !(encoding == QMM_GPTQ && cfg->desc_act) &&
+    return (narrow || m <= (lhs_dtype != QMM_F32 || encoding == QMM_Q4_0 ? 150 : encoding == QMM_GPTQ ? 400 : 1400)) && !(encoding == QMM_GPTQ && cfg->desc_act) &&
            qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg));
 }
 static bool repacked_path(int encoding, int64_t m, int64_t n, int64_t k, bool have_rhs) {
