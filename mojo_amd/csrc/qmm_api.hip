@@ -1068,6 +1068,11 @@ int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, i
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul_swiglu: workspace of %lld bytes required, %lld given", (long long)(mm_ws + 2 * plane),
                     (long long)workspace_bytes);
     if (!aligned(workspace, 256)) return fail(QMM_ERR_INVALID, "qmm_matmul_swiglu: workspace must be 256-byte aligned");
+    // Q4_K with 2 .. 8 rows, where the small-batch kernel would serve both products
+    if (encoding == QMM_Q4_K && m >= 2 && m <= 8 && k % 256 == 0 && aligned(gate, 16) && aligned(up, 16) && !(m <= 4 && q4k_lanes_rows_wins(n, k)) &&
+        !qmm::kernel_disabled("q4k_mm") && !qmm::kernel_disabled("q4k_mm_gated") && !direct_serves(encoding, nullptr, lhs_dtype, m, n, k, workspace, mm_ws))
+        return hip_status(qmm::launch_gemv_q4_k_mm_gated(lhs, lhs_dtype, (const uint8_t*)gate, (const uint8_t*)up, m, n, k, out, (hipStream_t)stream),
+                          "qmm_matmul_swiglu(Q4_K small batch)");
     float* g = (float*)((char*)workspace + mm_ws);
     float* u = (float*)((char*)workspace + mm_ws + plane);
     // (one launch for both products where a kernel takes matrices that share their lhs: Q4_K with 2..16 rows)

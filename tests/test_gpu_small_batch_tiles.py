@@ -41,3 +41,16 @@ def test_group_and_gated_pair():
     gated = qmatmul_swiglu(QE.Q4_K, a, ws[0], ws[1]).double()
     want = torch.nn.functional.silu(outs[0].double()) * outs[1].double()
     assert torch.allclose(gated, want, rtol=1e-5, atol=1e-6)  # (exp and the quotient in fp32: some units of 2^-24 each)
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(2, 4104, 4096), (3, 1032, 8448), (4, 14344, 256), (4, 32776, 2304), (5, 4104, 4352), (8, 20488, 512)])
+def test_gated_pair_is_the_two_products_combined(m, n, k, lhs):
+    gate, up = packed(n, k), packed(n + 8, k)[:n].contiguous()
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(lhs)
+    products = qmatmul_grouped(QE.Q4_K, a, [gate, up])
+    check(products[0], gate, a)
+    check(products[1], up, a)
+    g, u = (p.double() for p in products)
+    # the same sums in the same order; exp, the quotient and two products in fp32 (8 units of 2^-24)
+    assert torch.allclose(qmatmul_swiglu(QE.Q4_K, a, gate, up).double(), g / (1 + torch.exp(-g)) * u, rtol=2.0**-21, atol=1e-30)
