@@ -63,10 +63,11 @@ __device__ __forceinline__ void load8(const AT* p, float (&v)[8]) {
 }
 // the e-th of `count` workgroups zeroes its part of the results (m rows)
 __device__ __forceinline__ void zero_out(const DirectMats& z, int m, int e, int count) {
+    const int threads = (int)blockDim.x;
     for (int j = 0; j < z.count; j++) {
         float* __restrict__ const out = z.out[j];
         const int64_t values = (int64_t)m * z.n[j];
-        for (int64_t i = ((int64_t)e * 256 + threadIdx.x) * 4; i < values; i += (int64_t)count * 1024) {
+        for (int64_t i = ((int64_t)e * threads + threadIdx.x) * 4; i < values; i += (int64_t)count * threads * 4) {
             if (i + 3 < values) *(float4*)(out + i) = make_float4(0.f, 0.f, 0.f, 0.f);
             else
                 for (int64_t q = i; q < values; q++) out[q] = 0.0f;
@@ -74,12 +75,15 @@ __device__ __forceinline__ void zero_out(const DirectMats& z, int m, int e, int 
     }
 }
 
+// With few rows the latency of a row's passes (load, maximum, narrow, store) bounds it: as many threads as leave each one or two pieces of eight
+// columns (200 x 14336 bf16 rows with 256 threads a row 10.1 us, with 1024 7.2); with many, that a row writes 16 bytes of a 128-byte line, the rest
+// of which other workgroups of the XCD fill (500 x 14336: 11.5 us for 28 MB, whatever the number of threads).
 // Rows of one group of eight go to workgroups of one XCD (ids congruent mod 8): a 128-byte line of an operand holds eight rows.
 template <typename AT, int ORDER>
-__global__ __launch_bounds__(256) void direct_prep_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, int with_sums, DirectMats zero) {
+__global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, int with_sums, DirectMats zero) {
     constexpr bool kF32 = sizeof(AT) == 4;
-    __shared__ uint32_t wmax[4];
-    const int tid = threadIdx.x, rows = (m + 63) / 64 * 64;
+    __shared__ uint32_t wmax[16];
+    const int tid = threadIdx.x, threads = (int)blockDim.x, rows = (m + 63) / 64 * 64;
     if ((int)blockIdx.x >= rows) {
         zero_out(zero, m, (int)blockIdx.x - rows, (int)gridDim.x - rows);
         return;
@@ -89,9 +93,9 @@ __global__ __launch_bounds__(256) void direct_prep_kernel(const AT* __restrict__
     const AT* ar = a + (int64_t)row * k;
     const int pieces = k >> 3;  // of eight columns, one per thread and turn
     const int steps = (k + 255) / 256 * 16;
-    constexpr int kHeld = 4;    // rows of up to 8192 columns stay in registers between the search for the maximum and the narrowing
+    constexpr int kHeld = 4;    // rows of up to 32768 columns (1024 threads) stay in registers between the search for the maximum and the narrowing
     float held[kHeld][8];
-    const bool hold = pieces <= kHeld * 256;
+    const bool hold = pieces <= kHeld * threads;
     auto load = [&](int pc, float (&v)[8]) __attribute__((always_inline)) { load8(ar + pc * 8, v); };
     float mx = 0.0f;
     auto top = [&](const float (&v)[8]) __attribute__((always_inline)) {
@@ -101,12 +105,12 @@ __global__ __launch_bounds__(256) void direct_prep_kernel(const AT* __restrict__
     if (hold) {
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * 256 < pieces) load(tid + i * 256, held[i]);
+            if (tid + i * threads < pieces) load(tid + i * threads, held[i]);
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * 256 < pieces) top(held[i]);
+            if (tid + i * threads < pieces) top(held[i]);
     } else {
-        for (int pc = tid; pc < pieces; pc += 256) {
+        for (int pc = tid; pc < pieces; pc += threads) {
             float v[8];
             load(pc, v);
             top(v);
@@ -115,7 +119,8 @@ __global__ __launch_bounds__(256) void direct_prep_kernel(const AT* __restrict__
     const uint32_t mb = wave_max_nonneg_bits(mx);
     if ((tid & 63) == 0) wmax[tid >> 6] = mb;
     __syncthreads();
-    const uint32_t mxb = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+    uint32_t mxb = 0;
+    for (int i = 0; i < threads >> 6; i++) mxb = max(mxb, wmax[i]);
     int e = (int)((mxb >> 23) & 0xffu) - 127;
     if (e < -100 || e > 127) e = 9;  // zero, denormal or non-finite row: leave unscaled
     const float s = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
@@ -154,16 +159,16 @@ __global__ __launch_bounds__(256) void direct_prep_kernel(const AT* __restrict__
             }
         }
     };
-    for (int pc = pieces + tid; pc < 2 * steps; pc += 256) {  // zeros up to a whole unit
+    for (int pc = pieces + tid; pc < 2 * steps; pc += threads) {  // zeros up to a whole unit
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         emit(pc, v);
     }
     if (hold) {
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * 256 < pieces) emit(tid + i * 256, held[i]);
+            if (tid + i * threads < pieces) emit(tid + i * threads, held[i]);
     } else {
-        for (int pc = tid; pc < pieces; pc += 256) {
+        for (int pc = tid; pc < pieces; pc += threads) {
             float v[8];
             load(pc, v);
             emit(pc, v);
@@ -174,8 +179,8 @@ __global__ __launch_bounds__(256) void direct_prep_kernel(const AT* __restrict__
 // The same for Q4_0: rows quantised to Q8_0, codes as fp16, no row scale; the fp16 block scales of a row as the first eight slots of the
 // unit's operand in `sums` (lanes g = 0; zeros in g = 1).  Four neighbouring threads hold a block.
 template <typename AT>
-__global__ __launch_bounds__(256) void direct_prep_q8_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, DirectMats zero) {
-    const int tid = threadIdx.x, rows = (m + 63) / 64 * 64;
+__global__ __launch_bounds__(1024) void direct_prep_q8_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, DirectMats zero) {
+    const int tid = threadIdx.x, threads = (int)blockDim.x, rows = (m + 63) / 64 * 64;
     if ((int)blockIdx.x >= rows) {
         zero_out(zero, m, (int)blockIdx.x - rows, (int)gridDim.x - rows);
         return;
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(256) void direct_prep_q8_kernel(const AT* __restric
     const int pieces = k >> 3, units = (k + 255) / 256;
     const int tile = row >> 5, lane = row & 31;
     if (tid == 0) p.inv[row] = 1.0f;
-    for (int pc = tid; pc < units * 32; pc += 256) {
+    for (int pc = tid; pc < units * 32; pc += threads) {
         const int blk = pc >> 2, sub = pc & 3, g = sub & 1, step = 2 * blk + (sub >> 1);
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         if (pc < pieces) load8(ar + pc * 8, v);
@@ -209,6 +214,8 @@ __global__ __launch_bounds__(256) void direct_prep_q8_kernel(const AT* __restric
         }
     }
 }
+
+int prep_threads(int64_t k) { return k <= 2048 ? 256 : k <= 4096 ? 512 : 1024; }
 
 constexpr int direct_ahead(int flush, int fm, int fn, bool hilo) {
     if (fm * fn == 2) return hilo ? 4 : 8;
@@ -604,15 +611,16 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
         if (plans[j].shares > 1) zero.out[zero.count] = outs[j], zero.n[zero.count++] = (int)ns[j], zeros = std::max(zeros, m * ns[j]);
     }
     const unsigned grid = (unsigned)((m + 63) / 64 * 64 + std::min<int64_t>(1024, (zeros + 4095) / 4096));
+    const int threads = prep_threads(k);
     if (q40) {
-        if (f32) direct_prep_q8_kernel<float><<<dim3(grid), dim3(256), 0, s>>>((const float*)lhs, (int)m, (int)k, p, zero);
-        else direct_prep_q8_kernel<uint16_t><<<dim3(grid), dim3(256), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, zero);
+        if (f32) direct_prep_q8_kernel<float><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, zero);
+        else direct_prep_q8_kernel<uint16_t><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, zero);
     } else if (encoding == QMM_GPTQ) {
-        if (f32) direct_prep_kernel<float, kOrderGptq><<<dim3(grid), dim3(256), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero);
-        else direct_prep_kernel<uint16_t, kOrderGptq><<<dim3(grid), dim3(256), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero);
+        if (f32) direct_prep_kernel<float, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero);
+        else direct_prep_kernel<uint16_t, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero);
     } else {
-        if (f32) direct_prep_kernel<float, kOrderK><<<dim3(grid), dim3(256), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero);
-        else direct_prep_kernel<uint16_t, kOrderK><<<dim3(grid), dim3(256), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero);
+        if (f32) direct_prep_kernel<float, kOrderK><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero);
+        else direct_prep_kernel<uint16_t, kOrderK><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero);
     }
     hipError_t e = hipGetLastError();
     const WeightTensors wt{nullptr, scales, qzeros, 0, (int)k, group};
