@@ -496,7 +496,8 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
         for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, m, n, k));
         if (m > 32 && !kernel_disabled("shared"))
-            for (int i = 0; i < 3; i++) consider(kSharedPlans[i], shares, shared_us(c, i, shares, encoding, m, n, k));
+            for (int i = 0; i < 3; i++)  // (between predictions that close, workgroups of four wavefronts took 5 .. 7 % longer)
+                consider(kSharedPlans[i], shares, shared_us(c, i, shares, encoding, m, n, k) * (i == 2 ? 1.03 : 1.0));
     }
     if (us[0] >= 1e30) return best[us[1] < 1e30 ? 1 : 0];
     // (the margin: with it next to no problem of that measurement lost more than 5 % to a wrong choice)
