@@ -217,7 +217,8 @@ __global__ __launch_bounds__(1024) void direct_prep_q8_kernel(const AT* __restri
 
 int prep_threads(int64_t k) { return k <= 2048 ? 256 : k <= 4096 ? 512 : 1024; }
 
-constexpr int direct_ahead(int flush, int fm, int fn, bool hilo) {
+constexpr int direct_ahead(int flush, int fm, int fn, bool hilo, bool split) {
+    if (split && fm * fn == 1) return 8;  // (registers)
     if (fm * fn == 2) return hilo ? 4 : 8;
     return flush == 2 && hilo ? 8 : 16;
 }
@@ -259,6 +260,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             const int part_e = min(e * WK + wave, kParts - 1), row = m0 + 32 * ((part_e >> 2) / FN) + 8 * (part_e & 3) + 4 * (lane >> 5) + r;
             inv[e][r] = p.inv[min(row, m - 1)];
         }
+    constexpr bool kSplit = HILO && W::kMin;  // the residual's products in sums of their own (see gemm_direct.h)
     float16v T[FM][FN];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
     if (u0 < u1) {
         // Lhs operands are loaded kAhead steps ahead.  Loads return in the order they were issued, so an lhs operand (from L2) waits for
         // the weights (from memory) requested before it: a whole unit ahead where the registers allow it.
-        constexpr int kPer = HILO ? 2 : 1, kAhead = direct_ahead(FLUSH, FM, FN, HILO);
+        constexpr int kPer = HILO ? 2 : 1, kAhead = direct_ahead(FLUSH, FM, FN, HILO, kSplit);
         const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         W w;
         w.init(wt, n0, lane, (uint8_t*)red + wave * kSlot);
@@ -297,7 +299,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             const bool more = u + 1 < u1;
             w.open();
             if (more) w.load(u + 1);
-            float16v P[FM][FN];
+            float16v P[FM][FN], L[kSplit ? FM : 1][kSplit ? FN : 1];
             half8 sf[FM];
             if constexpr (W::kMin || ENC == QMM_Q4_0) {
 #pragma unroll
@@ -323,7 +325,8 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                         for (int a = 0; a < FM; a++)
 #pragma unroll
                             for (int f = 0; f < FN; f++) {
-                                if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], zero16, 0, 0, 0);
+                                if (kSplit && q == 1) L[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], t % W::kFlush == 0 ? zero16 : L[a][f], 0, 0, 0);
+                                else if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], zero16, 0, 0, 0);
                                 else P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], P[a][f], 0, 0, 0);
                             }
                 if constexpr (t + 1 < W::kSteps) {
@@ -362,7 +365,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
 #pragma unroll
                         for (int a = 0; a < FM; a++) {
 #pragma unroll
-                            for (int r = 0; r < 16; r++) T[a][f][r] = fmaf(d, P[a][f][r], T[a][f][r]);
+                            for (int r = 0; r < 16; r++) T[a][f][r] = fmaf(d, kSplit ? P[a][f][r] + L[a][f][r] : P[a][f][r], T[a][f][r]);
                             // (left to itself the compiler puts these off and keeps the P of every scale block)
                             asm volatile("" : "+v"(T[a][f]));
                         }

@@ -44,6 +44,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
     const int u0 = (int)((unsigned)units * (unsigned)part / (unsigned)parts), u1 = (int)((unsigned)units * (unsigned)(part + 1) / (unsigned)parts);
     if (threadIdx.x < 32 * FM) inv[threadIdx.x] = p.inv[min(m0 + (int)threadIdx.x, m - 1)];
 
+    constexpr bool kSplit = HILO && W::kMin;  // the residual's products in sums of their own (see gemm_direct.h)
     float16v T[FM];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
                 sf[a] = *(const half8*)((const uint8_t*)p.sums + ((int64_t)min(tile_m * FM + a, last_tile) * units + u) * 1024 + l16);
         };
         if constexpr (ENC == QMM_Q4_0) load_sums();
-        float16v P[FM];
+        float16v P[FM], L[kSplit ? FM : 1];
         half8 b[2][W::kPlanes];
         w.template step<0>(0, b[0]);
         __builtin_amdgcn_sched_barrier(0);
@@ -130,7 +131,8 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
                 for (int q = 0; q < kPer; q++)
 #pragma unroll
                     for (int a = 0; a < FM; a++) {
-                        if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], zero16, 0, 0, 0);
+                        if (kSplit && q == 1) L[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], t % W::kFlush == 0 ? zero16 : L[a], 0, 0, 0);
+                        else if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], zero16, 0, 0, 0);
                         else P[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], P[a], 0, 0, 0);
                     }
             if constexpr (t + 1 < W::kSteps) {
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
 #pragma unroll
                     for (int a = 0; a < FM; a++) {
 #pragma unroll
-                        for (int r = 0; r < 16; r++) T[a][r] = fmaf(d, P[a][r], T[a][r]);
+                        for (int r = 0; r < 16; r++) T[a][r] = fmaf(d, kSplit ? P[a][r] + L[a][r] : P[a][r], T[a][r]);
                         asm volatile("" : "+v"(T[a]));
                     }
                     if constexpr (W::kMin) {
