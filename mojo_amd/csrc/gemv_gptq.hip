@@ -314,7 +314,13 @@ hipError_t launch_gemv_gptq_cols(const void* a, int a_dtype, const uint32_t* qwe
 // Group indices outside [0, K / group) are clamped (the result is then meaningless, nothing is read
 // out of bounds).
 // ---------------------------------------------------------------------------
-template <int MT, bool TABLE, typename AT>
+//
+// The table reads of a weight's group are a chain of their own (g_idx, table, product), so the time of a call is how many of them the
+// compiler keeps in flight.  A loop over passes of rows around the body leaves it 23 .. 27 registers and one weight at a time; without
+// the loop it takes 62 (fp32) and 75 (bf16): 14336 x 4096, g128, one bf16 row 19.1 us with the loop, 13.6 without; one fp32 row 16.8 and
+// 13.7, two 18.6 and 14.8; 4096 x 4096 with one bf16 row 15.8 and 12.8.  PASSES (all m rows in one launch) is only for the launch behind a sorted
+// product, which returns at once unless the groups are of uneven size.
+template <int MT, bool TABLE, bool PASSES, typename AT>
 __global__ __launch_bounds__(64 * kWaves) void gemv_gptq_act_order_kernel(
     const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     const int32_t* __restrict__ g_idx, const AT* __restrict__ a, float* __restrict__ out, int m, int n, int k, int group,
@@ -338,7 +344,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_gptq_act_order_kernel(
         for (int g = wave; g < ngroups; g += kWaves) table[g * 64 + lane] = pair_of(g);
         __syncthreads();
     }
-    for (int m0 = 0; m0 < m; m0 += MT) {  // passes of MT rows
+    for (int m0 = 0; m0 < (PASSES ? m : 1); m0 += MT) {  // passes of MT rows
         const int left = m - m0;
         float acc[MT];
 #pragma unroll
@@ -382,45 +388,54 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_gptq_act_order_kernel(
                 }
             }
         }
-        __syncthreads();  // (the next pass writes `red` again)
+        if constexpr (PASSES) __syncthreads();  // (the next pass writes `red` again)
     }
 }
 
-// K % 32 == 0 and N % 8 == 0 are the caller's checks.  only_if != null: the launch does nothing where that word is zero.
+// K % 32 == 0 and N % 8 == 0 are the caller's checks.  only_if == null: a launch per four rows; otherwise one launch for all rows, which does
+// nothing where that word is zero.
 hipError_t launch_gemv_gptq_act_order(const void* a, int a_dtype, const uint32_t* qweight, const uint16_t* scales,
                                       const uint32_t* qzeros, const int32_t* g_idx, int m, int64_t n, int64_t k, int group,
                                       float* out, int64_t ldo, hipStream_t s, const int32_t* only_if) {
     if (m < 1 || (k & 31)) return hipErrorInvalidValue;
-    const int mt = m <= 1 ? 1 : m <= 2 ? 2 : 4;
-    const size_t red_bytes = (size_t)kWaves * mt * 64 * 4;
-    const size_t table_bytes = (size_t)(k / group) * 64 * 8;
-    // (past half of the LDS one workgroup fills a compute unit, and that is still better than a scale and a zero point from memory per weight)
-    const bool table = table_bytes + red_bytes <= (size_t)kLdsPerCu;
-    const size_t lds = red_bytes + (table ? table_bytes : 0);
     dim3 grid((unsigned)((n + 63) / 64)), block(64 * kWaves);
-#define QMM_GPTQ_AO(MT_, TB_)                                                                                          \
-    do {                                                                                                              \
-        const hipError_t e = a_dtype == QMM_F32 ? allow_full_lds<gemv_gptq_act_order_kernel<MT_, TB_, float>>()       \
-                                                : allow_full_lds<gemv_gptq_act_order_kernel<MT_, TB_, uint16_t>>();   \
-        if (e != hipSuccess) return e;                                                                                \
-        if (a_dtype == QMM_F32)                                                                                       \
-            gemv_gptq_act_order_kernel<MT_, TB_, float><<<grid, block, lds, s>>>(                                     \
-                qweight, scales, qzeros, g_idx, (const float*)a, out, m, (int)n, (int)k, group, ldo, only_if);        \
-        else                                                                                                          \
-            gemv_gptq_act_order_kernel<MT_, TB_, uint16_t><<<grid, block, lds, s>>>(                                  \
-                qweight, scales, qzeros, g_idx, (const uint16_t*)a, out, m, (int)n, (int)k, group, ldo, only_if);     \
+    const int64_t esz = a_dtype == QMM_F32 ? 4 : 2;
+    const bool passes = only_if && m > 4;
+    for (int m0 = 0; m0 < (passes ? 1 : m); m0 += 4) {
+        const int left = m - m0, rows = passes ? m : left < 4 ? left : 4, mt = rows <= 1 ? 1 : rows <= 2 ? 2 : 4;
+        const size_t red_bytes = (size_t)kWaves * mt * 64 * 4;
+        const size_t table_bytes = (size_t)(k / group) * 64 * 8;
+        // (past half of the LDS one workgroup fills a compute unit, and that is still better than a scale and a zero point from memory per weight)
+        const bool table = table_bytes + red_bytes <= (size_t)kLdsPerCu;
+        const size_t lds = red_bytes + (table ? table_bytes : 0);
+        const char* const am = (const char*)a + m0 * k * esz;
+        float* const om = out + m0 * ldo;
+#define QMM_GPTQ_AO(MT_, TB_, PS_)                                                                                         \
+    do {                                                                                                                  \
+        const hipError_t e = a_dtype == QMM_F32 ? allow_full_lds<gemv_gptq_act_order_kernel<MT_, TB_, PS_, float>>()      \
+                                                : allow_full_lds<gemv_gptq_act_order_kernel<MT_, TB_, PS_, uint16_t>>();  \
+        if (e != hipSuccess) return e;                                                                                    \
+        if (a_dtype == QMM_F32)                                                                                           \
+            gemv_gptq_act_order_kernel<MT_, TB_, PS_, float><<<grid, block, lds, s>>>(                                    \
+                qweight, scales, qzeros, g_idx, (const float*)am, om, rows, (int)n, (int)k, group, ldo, only_if);         \
+        else                                                                                                              \
+            gemv_gptq_act_order_kernel<MT_, TB_, PS_, uint16_t><<<grid, block, lds, s>>>(                                 \
+                qweight, scales, qzeros, g_idx, (const uint16_t*)am, om, rows, (int)n, (int)k, group, ldo, only_if);      \
     } while (0)
-#define QMM_GPTQ_AO_MT(TB_)                        \
-    do {                                           \
-        if (mt == 1) QMM_GPTQ_AO(1, TB_);          \
-        else if (mt == 2) QMM_GPTQ_AO(2, TB_);     \
-        else QMM_GPTQ_AO(4, TB_);                  \
+#define QMM_GPTQ_AO_MT(TB_)                               \
+    do {                                                  \
+        if (passes) QMM_GPTQ_AO(4, TB_, true);            \
+        else if (mt == 1) QMM_GPTQ_AO(1, TB_, false);     \
+        else if (mt == 2) QMM_GPTQ_AO(2, TB_, false);     \
+        else QMM_GPTQ_AO(4, TB_, false);                  \
     } while (0)
-    if (table) QMM_GPTQ_AO_MT(true);
-    else QMM_GPTQ_AO_MT(false);
+        if (table) QMM_GPTQ_AO_MT(true);
+        else QMM_GPTQ_AO_MT(false);
 #undef QMM_GPTQ_AO_MT
 #undef QMM_GPTQ_AO
-    return hipGetLastError();
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace qmm

@@ -1,0 +1,51 @@
+"""What the compiler made of kernels whose speed hangs on it: the register counts in the code objects of the built library."""
+import os
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+from mojo_amd import _lib
+from mojo_amd.build import HIPCC
+
+LLVM = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "llvm", "bin")
+READELF, OBJCOPY = os.path.join(LLVM, "llvm-readelf"), os.path.join(LLVM, "llvm-objcopy")
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{demangled kernel name: (vector registers, spilled vector registers)}"""
+    if not (os.path.exists(_lib.LIB_PATH) and os.path.exists(READELF) and os.path.exists(OBJCOPY) and shutil.which("c++filt")):
+        pytest.skip("needs the built library, llvm-readelf, llvm-objcopy and c++filt")
+    tmp = tmp_path_factory.mktemp("code")
+    fat = tmp / "fat.bin"
+    subprocess.run([OBJCOPY, "--dump-section", f".hip_fatbin={fat}", _lib.LIB_PATH, str(tmp / "rest")], check=True)
+    data = fat.read_bytes()
+    names, counts = [], []
+    for at in (m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)):  # one bundle per source file
+        (entries,), p = struct.unpack_from("<Q", data, at + 24), at + 32
+        for _ in range(entries):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            target = data[p + 24:p + 24 + length].decode()
+            p += 24 + length
+            if "gfx950" not in target or not size:
+                continue
+            obj = tmp / "kernel.o"
+            obj.write_bytes(data[at + offset:at + offset + size])
+            notes = subprocess.run([READELF, "--notes", str(obj)], check=True, capture_output=True, text=True).stdout
+            for block in re.split(r"\n\s*- \.agpr_count", notes)[1:]:
+                names.append(re.search(r"\n    \.name:\s+(\S+)", block).group(1))
+                counts.append(tuple(int(re.search(rf"\.{key}:\s+(\d+)", block).group(1)) for key in ("vgpr_count", "vgpr_spill_count")))
+    plain = subprocess.run(["c++filt"], input="\n".join(names), capture_output=True, text=True, check=True).stdout.split("\n")
+    assert len(names) > 100
+    return {re.sub(r"\(anonymous namespace\)::|qmm::|^void ", "", n).split("(")[0]: c for n, c in zip(plain, counts)}
+
+
+@pytest.mark.parametrize("rows,lhs", [(1, "float"), (1, "unsigned short"), (2, "float")])
+def test_act_order_look_up_keeps_its_table_reads_in_flight(kernels, rows, lhs):
+    """Each weight waits for a chain of its own (group, table, product).  With 62 .. 75 registers the reads of eight weights overlap; a body that
+    the compiler schedules one weight at a time takes 23 .. 27 and 14336 x 4096 with one bf16 row 19.1 us instead of 13.6."""
+    found = [c for name, c in kernels.items() if re.match(rf"gemv_gptq_act_order_kernel<{rows}, true, .*{lhs}>$", name)]
+    assert found and all(registers >= 56 and spilled == 0 for registers, spilled in found), found
