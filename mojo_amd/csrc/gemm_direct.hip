@@ -122,7 +122,8 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     uint32_t mxb = 0;
     for (int i = 0; i < threads >> 6; i++) mxb = max(mxb, wmax[i]);
     int e = (int)((mxb >> 23) & 0xffu) - 127;
-    if (e < -100 || e > 127) e = 9;  // zero, denormal or non-finite row: leave unscaled
+    if (e > 127) e = 9;  // non-finite row: leave unscaled
+    e = max(e, -117);    // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
     const float s = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
     if (tid == 0) p.inv[row] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
     const int tile = row >> 5, lane = row & 31;

@@ -85,3 +85,23 @@ def test_group_equals_separate_calls(enc, m, k, ns):
     for got, w in zip(qmatmul_grouped(enc, a, [w[0] for w in rhs]), rhs):
         assert torch.equal(got, qmatmul(enc, None, a, *w))
         check(got, enc, None, w, a)
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("enc,group,order", [(QE.Q4_K, 0, False), (QE.Q5_K, 0, False), (QE.Q6_K, 0, False), (QE.GPTQ, 128, False), (QE.GPTQ, 32, False),
+                                             (QE.GPTQ, 128, True)])
+def test_rows_of_any_magnitude(enc, group, order, lhs):
+    """A row is narrowed behind a power of two of its own: rows from denormal numbers (2^-140) up to 2^120, next to each other."""
+    m, n, k = 33, 264, 512
+    config, rhs = weights(enc, group, n, k)
+    if order:
+        config, rhs = QuantizationConfig("gptq", 4, group, True, True), (*rhs, torch.arange(k, device="cuda", dtype=torch.int32) // group)
+    exponents = torch.tensor([(-140, -133, -126, -125, -118, -117, -110, -101, -100, -60, 0, 60, 120)[i % 13] for i in range(m)], device="cuda")
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    a = torch.ldexp(a.double(), exponents[:, None]).to(lhs)  # (rounded to the type's denormal grid where that is coarser)
+    w, x = dequantize(enc, *rhs, config=config).double(), a.double()
+    want, size = x @ w.T, x.abs() @ w.abs().T
+    # as in check(), and the grid of denormal results
+    bound = (k / 16 + 32) * 2.0**-24 * 16 * size + 2.0**-149
+    worst = ((qmatmul(enc, config, a, *rhs).double() - want).abs() / bound).amax(1)
+    assert worst.max().item() <= 1.0, (enc, [(int(e), round(v, 2)) for e, v in zip(exponents, worst.tolist()) if v > 1.0])
