@@ -100,7 +100,7 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     float mx = 0.0f;
     auto top = [&](const float (&v)[8]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]));
+        for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]) <= 3.402823466e38f ? fabsf(v[i]) : 0.0f);  // (of the finite values)
     };
     if (hold) {
 #pragma unroll
@@ -122,8 +122,7 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     uint32_t mxb = 0;
     for (int i = 0; i < threads >> 6; i++) mxb = max(mxb, wmax[i]);
     int e = (int)((mxb >> 23) & 0xffu) - 127;
-    if (e > 127) e = 9;  // non-finite row: leave unscaled
-    e = max(e, -117);    // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
+    e = max(e, -117);  // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
     const float s = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
     if (tid == 0) p.inv[row] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
     const int tile = row >> 5, lane = row & 31;
@@ -142,9 +141,11 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
         *(gd_u4*)at = hi;
         if constexpr (kF32) {
             gd_u4 lo;
+            float residual[8];
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                lo[i] = pack_half2(v[perm[ORDER][2 * i]] - h[perm[ORDER][2 * i]], v[perm[ORDER][2 * i + 1]] - h[perm[ORDER][2 * i + 1]]);
+            for (int i = 0; i < 8; i++) residual[i] = fabsf(h[i]) <= 65504.0f ? v[i] - h[i] : 0.0f;  // (an infinity has no residual: inf - inf)
+#pragma unroll
+            for (int i = 0; i < 4; i++) lo[i] = pack_half2(residual[perm[ORDER][2 * i]], residual[perm[ORDER][2 * i + 1]]);
             *(gd_u4*)(at + 512) = lo;
         }
         if (with_sums) {

@@ -105,3 +105,23 @@ def test_rows_of_any_magnitude(enc, group, order, lhs):
     bound = (k / 16 + 32) * 2.0**-24 * 16 * size + 2.0**-149
     worst = ((qmatmul(enc, config, a, *rhs).double() - want).abs() / bound).amax(1)
     assert worst.max().item() <= 1.0, (enc, [(int(e), round(v, 2)) for e, v in zip(exponents, worst.tolist()) if v > 1.0])
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(17, 264, 512), (33, 2056, 1024), (200, 4104, 512)])
+@pytest.mark.parametrize("group,order", [(128, False), (32, False), (128, True)])
+def test_gptq_infinities_and_nans_keep_their_kind(group, order, m, n, k, lhs):
+    """code - zero is one integer, so an infinity meets no difference of sums: +-inf where the weight is not zero, NaN where it is, as in the
+    product of the dequantised weights; a NaN makes its row NaN; finite neighbours in such a row (1e30) and other rows are what they are."""
+    config, rhs = weights(QE.GPTQ, group, n, k)
+    if order:
+        config, rhs = QuantizationConfig("gptq", 4, group, True, True), (*rhs, torch.arange(k, device="cuda", dtype=torch.int32) // group)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(4)).to(lhs)
+    a[1, 7], a[3, k - 1], a[4, 5], a[5, 100], a[5, 101] = float("inf"), -float("inf"), float("nan"), float("inf"), 1e30
+    got = qmatmul(QE.GPTQ, config, a, *rhs)
+    w, special = dequantize(QE.GPTQ, *rhs, config=config).double().cpu(), [1, 3, 4, 5]
+    want, have = a[special].double().cpu() @ w.T, got[special].double().cpu()
+    assert not want.isfinite().any()
+    assert torch.equal(have.isnan(), want.isnan()) and torch.equal(have.isposinf(), want.isposinf())
+    rest = [i for i in range(m) if i not in special]
+    check(got[rest], QE.GPTQ, config, rhs, a[rest])
