@@ -54,6 +54,11 @@ __device__ __forceinline__ uint32_t pk_add(uint32_t x, uint32_t y) { return as_u
 template <int J>
 __device__ __forceinline__ uint32_t byte_pair(uint32_t top4, uint32_t v) { return __builtin_amdgcn_perm(top4, v, 0x04000400u | (J << 16) | J); }
 
+// A row is scaled by a power of two so that its largest value lies in [2^kRowTop, 2^(kRowTop + 1)), as high as fp16 goes: an fp32 value is then
+// held to 22 bits down to 2^-17 of the row's largest and to 2^-39 of that below (2^-12 and 2^-34 with a top of 9).  Where sums of 32 values
+// are held in fp16 too (Q4_K, Q5_K), 2^9 leaves them room.
+constexpr int kRowTop = 14, kRowTopWithSums = 9;
+
 // The operand order of the lhs: step t = 2 blk + a of 16 columns holds, for half wavefront g, the columns
 //   32 blk + 16 g + 8 a + slot order   (kOrderK: slots 0,2,1,3,4,6,5,7; kOrderGptq: 0,4,1,5,2,6,3,7)
 constexpr int kOrderK = 0, kOrderGptq = 1;  // (Q4_0: 32 blk + 16 a + 8 g + the slots of kOrderK)

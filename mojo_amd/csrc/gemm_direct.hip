@@ -122,9 +122,10 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     uint32_t mxb = 0;
     for (int i = 0; i < threads >> 6; i++) mxb = max(mxb, wmax[i]);
     int e = (int)((mxb >> 23) & 0xffu) - 127;
-    e = max(e, -117);  // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
-    const float s = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
-    if (tid == 0) p.inv[row] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
+    const int row_top = with_sums ? kRowTopWithSums : kRowTop;
+    e = max(e, row_top - 126);  // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
+    const float s = __uint_as_float((uint32_t)(127 + row_top - e) << 23);
+    if (tid == 0) p.inv[row] = __uint_as_float((uint32_t)(127 - row_top + e) << 23);
     const int tile = row >> 5, lane = row & 31;
     auto emit = [&](int pc, float (&v)[8]) __attribute__((always_inline)) {
         constexpr int perm[2][8] = {{0, 2, 1, 3, 4, 6, 5, 7}, {0, 4, 1, 5, 2, 6, 3, 7}};

@@ -125,3 +125,30 @@ def test_gptq_infinities_and_nans_keep_their_kind(group, order, m, n, k, lhs):
     assert torch.equal(have.isnan(), want.isnan()) and torch.equal(have.isposinf(), want.isposinf())
     rest = [i for i in range(m) if i not in special]
     check(got[rest], QE.GPTQ, config, rhs, a[rest])
+
+
+@pytest.mark.parametrize("lhs,spike", [(torch.float32, 2.0**20), (torch.bfloat16, 2.0**28)])
+@pytest.mark.parametrize("group", [128, 32])
+def test_values_far_below_the_largest_of_their_row(group, lhs, spike):
+    """Columns with values 2^20 (2^28) times the others' that no weight multiplies (code = zero): the rest of the row has to come through."""
+    m, n, k = 33, 264, 1024
+    config, (qweight, scales, qzeros) = weights(QE.GPTQ, group, n, k)
+    columns = torch.tensor([3, 300, 801], device="cuda")
+    zero = (qzeros[columns // group].repeat_interleave(8, 1) >> (4 * (torch.arange(n, device="cuda") & 7))) & 15  # stored zero; the code is one more
+    scales, qzeros = scales.clone(), qzeros.clone()
+    for c, z in zip(columns.tolist(), zero):
+        z = (z + 1).clamp(max=15)  # (a zero point of 16 has no code: those columns of the output are left out below)
+        word = qweight[c // 8] & ~(15 << (4 * (c % 8)))
+        qweight[c // 8] = word | (z << (4 * (c % 8)))
+    keep = ((zero + 1) <= 15).all(0)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(6))
+    a[:, columns] = spike
+    a = a.to(lhs)
+    rhs = (qweight, scales, qzeros)
+    w, x = dequantize(QE.GPTQ, *rhs, config=config).double()[keep], a.double()
+    assert keep.sum() > 100 and not w[:, columns].any()
+    want, size = x @ w.T, x.abs() @ w.abs().T
+    # as in check(), but code - zero is one operand: no terms sixteen times as large; a value is held to 2^-39 of its row's largest
+    bound = (k / 16 + 32) * 2.0**-24 * size + 2.0**-39 * spike * w.abs().sum(1)
+    worst = ((qmatmul(QE.GPTQ, config, a, *rhs)[:, keep].double() - want).abs() / bound).max().item()
+    assert worst <= 1.0, worst
