@@ -210,3 +210,13 @@ def test_product_never_imports_the_oracle():
             if f.endswith((".py", ".hip", ".h", ".cpp")):
                 text = open(os.path.join(base, f), errors="ignore").read()
                 assert "import oracle" not in text and "qmm_oracle" not in text and "oracle/" not in text, f
+
+
+def test_act_order_beyond_the_direct_gemm_stays_with_the_look_up_kernel():
+    """The sorted columns are for the direct GEMM, which takes up to 2^32 weights; no room is asked for them where it does not serve the call (the GEMM
+    that unpacks tiles, the next in line, has ten times the error of the look-up kernel)."""
+    lib, cfg = _lib.load(), C.byref(_lib.GptqConfig(4, 128, 1, 1))
+    for m in (9, 17, 200):
+        least = lib.qmm_matmul_workspace_bytes(QE.GPTQ.code, _lib.QMM_BF16, m, 1 << 17, 1 << 15)
+        assert lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, _lib.QMM_BF16, m, (1 << 17) - 8, 1 << 15, 0) > (1 << 31)
+        assert lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, _lib.QMM_BF16, m, 1 << 17, 1 << 15, 0) <= least
