@@ -394,15 +394,16 @@ static qmm_gptq_config plain_groups(qmm_gptq_config cfg) {
     cfg.desc_act = 0;
     return cfg;
 }
-// More than 16 rows take the direct GEMM whatever their number: the GEMM that unpacks tiles drops low bits of its products (3e-6 relative error
-// against 2e-7 of the look-up kernel and 7e-8 of the direct GEMM, 14336 x 4096 with 400 bf16 rows; the call takes 93 us with it and 103 with the direct one).
-// Matrices beyond what that takes (2^32 weights) stay with the look-up kernel.
-static bool order_direct(int64_t m) { return m > 16 && !qmm::kernel_disabled("direct"); }
+// The sorted columns go to the direct GEMM whatever the number of rows: the small-batch kernel and the GEMM that unpacks tiles drop low bits of their
+// products.  Relative errors, look-up / small batch / tile GEMM / direct: 6400 x 1024 with 5 fp32 rows 1.6e-7 / 4.0e-7 / - / 1.1e-7, 14336 x 4096 with
+// 400 bf16 rows 2e-7 / - / 3e-6 / 7e-8 (the call takes 93 us with the tile GEMM, 103 with the direct one).  Matrices beyond what that
+// takes (2^32 weights) stay with the look-up kernel.
+static bool order_direct() { return !qmm::kernel_disabled("direct"); }
 static int64_t order_bytes(const qmm_gptq_config& cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
     if (!cfg.desc_act || cfg.group_size <= 0 || k % cfg.group_size || (flags & ~QMM_FLAG_OUT_BF16) || !qmm::gptq_order_wanted(m, n, k) || n * k >= ((int64_t)1 << 32)) return 0;
     const qmm_gptq_config plain = plain_groups(cfg);
     return qmm::gptq_order_space(nullptr, lhs_dtype, m, n, k).bytes +
-           up256(order_direct(m) ? qmm::gemm_direct_workspace_bytes(QMM_GPTQ, lhs_dtype, m, k) : preferred_matmul(QMM_GPTQ, &plain, lhs_dtype, m, n, k, 0));
+           up256(order_direct() ? qmm::gemm_direct_workspace_bytes(QMM_GPTQ, lhs_dtype, m, k) : preferred_matmul(QMM_GPTQ, &plain, lhs_dtype, m, n, k, 0));
 }
 static bool order_serves(const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags, const void* workspace, int64_t workspace_bytes) {
     const int64_t need = order_bytes(*cfg, lhs_dtype, m, n, k, flags);
@@ -527,7 +528,7 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
                 if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, sort)");
                 const qmm_gptq_config plain = plain_groups(*cfg);
                 const void* sorted[3] = {p.qweight, rhs[1], rhs[2]};
-                if (order_direct(m)) {
+                if (order_direct()) {
                     e = qmm::launch_gemm_direct(encoding, p.lhs, lhs_dtype, 1, sorted, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], cfg->group_size, m, k,
                                                 nullptr, (char*)workspace + p.bytes, s);
                     if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, direct GEMM)");

@@ -108,8 +108,8 @@ def test_rows_of_any_magnitude(enc, group, order, lhs):
 
 
 @pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("m,n,k", [(17, 264, 512), (33, 2056, 1024), (200, 4104, 512)])
-@pytest.mark.parametrize("group,order", [(128, False), (32, False), (128, True)])
+@pytest.mark.parametrize("group,order,m,n,k", [(g, o, *s) for g, o in ((128, False), (32, False), (128, True)) for s in ((17, 264, 512), (33, 2056, 1024),
+                                                                                                                       (200, 4104, 512))] + [(128, True, 6, 264, 512)])
 def test_gptq_infinities_and_nans_keep_their_kind(group, order, m, n, k, lhs):
     """code - zero is one integer, so an infinity meets no difference of sums: +-inf where the weight is not zero, NaN where it is, as in the
     product of the dequantised weights; a NaN makes its row NaN; finite neighbours in such a row (1e30) and other rows are what they are."""
