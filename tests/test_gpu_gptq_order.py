@@ -11,12 +11,13 @@ from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, _lib, dequa
 pytestmark = pytest.mark.gpu
 
 
-def act_order(n, k, group, seed):
+def act_order(n, k, group, seed, any_codes=True):
     gen = torch.Generator(device="cuda").manual_seed(seed)
     w = torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen)
     qweight, scales, qzeros, g_idx = quantize_gptq(w, QuantizationConfig("gptq", 4, group, False, True))
-    qweight = torch.randint(-2**31, 2**31 - 1, qweight.shape, device="cuda", dtype=torch.int64, generator=gen).int()
-    qzeros = torch.randint(-2**31, 2**31 - 1, qzeros.shape, device="cuda", dtype=torch.int64, generator=gen).int()
+    if any_codes:
+        qweight = torch.randint(-2**31, 2**31 - 1, qweight.shape, device="cuda", dtype=torch.int64, generator=gen).int()
+        qzeros = torch.randint(-2**31, 2**31 - 1, qzeros.shape, device="cuda", dtype=torch.int64, generator=gen).int()
     return QuantizationConfig("gptq", 4, group, True, True), (qweight, scales, qzeros, g_idx[torch.randperm(k, device="cuda", generator=gen)].contiguous())
 
 
@@ -52,17 +53,28 @@ def c_call(config, rhs, a, need):
 
 @pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k,group", [(3, 72, 256, 32), (5, 8, 32, 32), (6, 40, 1056, 32), (17, 264, 1024, 1024), (16, 136, 5120, 128), (33, 136, 5376, 256),
-                                         (9, 72, 10240, 128), (20, 40, 10496, 64), (20, 24, 32768, 32), (130, 1032, 2304, 128), (600, 4104, 512, 128)])
+                                         (9, 72, 10240, 128), (20, 40, 10496, 64), (20, 24, 32768, 32), (130, 1032, 2304, 128), (600, 4104, 512, 128),
+                                         (40, 72, 256, 32), (40, 8, 32, 32), (40, 40, 1056, 32), (1, 40, 14336, 32), (2, 72, 10240, 128), (4, 72, 10240, 128)])
 def test_edges(m, n, k, group, lhs):
     config, rhs = act_order(n, k, group, m)
     a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(lhs)
-    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, m >= 5)
-    check(qmatmul(QE.GPTQ, config, a, *rhs, out_dtype=torch.bfloat16), config, rhs, a)
     cfg, dtype = C.byref(_lib.GptqConfig(4, group, 1, 1)), _lib.QMM_F32 if lhs == torch.float32 else _lib.QMM_BF16
     room = _lib.load().qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, dtype, m, n, k, 0)
+    sorted_columns = room > n * k // 2  # (room for the sorted matrix)
+    assert sorted_columns or m < 20
+    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns)
+    check(qmatmul(QE.GPTQ, config, a, *rhs, out_dtype=torch.bfloat16), config, rhs, a)
     least = _lib.load().qmm_matmul_workspace_bytes(QE.GPTQ.code, dtype, m, n, k)
     for need in (room, max(room - 1, least), least):
         check(c_call(config, rhs, a, need), config, rhs, a)
+
+
+@pytest.mark.parametrize("m,n,k", [(9, 6400, 1024), (16, 512, 512), (8, 1024, 4096), (12, 2056, 1280)])
+def test_few_rows_keep_their_fp32_precision(m, n, k):
+    """Codes around a zero point of 8, as quantised weights have them: a kernel that sums codes and zero points apart loses two bits to the difference."""
+    config, rhs = act_order(n, k, 128, m, any_codes=False)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m))
+    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns=True)
 
 
 @pytest.mark.parametrize("change", ["one column", "one group empty", "out of range"])
