@@ -392,6 +392,10 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_gptq_act_order_kernel(
     }
 }
 
+static size_t act_order_red_bytes(int64_t m) { return (size_t)kWaves * (m <= 1 ? 1 : m <= 2 ? 2 : 4) * 64 * 4; }
+// (past half of the LDS one workgroup fills a compute unit, and that is still better than a scale and a zero point from memory per weight)
+bool gptq_act_order_table_fits(int64_t m, int64_t k, int group) { return (size_t)(k / group) * 64 * 8 + act_order_red_bytes(m) <= (size_t)kLdsPerCu; }
+
 // K % 32 == 0 and N % 8 == 0 are the caller's checks.  only_if == null: a launch per four rows; otherwise one launch for all rows, which does
 // nothing where that word is zero.
 hipError_t launch_gemv_gptq_act_order(const void* a, int a_dtype, const uint32_t* qweight, const uint16_t* scales,
@@ -403,11 +407,8 @@ hipError_t launch_gemv_gptq_act_order(const void* a, int a_dtype, const uint32_t
     const bool passes = only_if && m > 4;
     for (int m0 = 0; m0 < (passes ? 1 : m); m0 += 4) {
         const int left = m - m0, rows = passes ? m : left < 4 ? left : 4, mt = rows <= 1 ? 1 : rows <= 2 ? 2 : 4;
-        const size_t red_bytes = (size_t)kWaves * mt * 64 * 4;
-        const size_t table_bytes = (size_t)(k / group) * 64 * 8;
-        // (past half of the LDS one workgroup fills a compute unit, and that is still better than a scale and a zero point from memory per weight)
-        const bool table = table_bytes + red_bytes <= (size_t)kLdsPerCu;
-        const size_t lds = red_bytes + (table ? table_bytes : 0);
+        const bool table = gptq_act_order_table_fits(rows, k, group);
+        const size_t lds = act_order_red_bytes(rows) + (table ? (size_t)(k / group) * 64 * 8 : 0);
         const char* const am = (const char*)a + m0 * k * esz;
         float* const om = out + m0 * ldo;
 #define QMM_GPTQ_AO(MT_, TB_, PS_)                                                                                         \

@@ -10,6 +10,8 @@
 // A sorted column list is a plain-group matrix only if every group has exactly group_size columns, which is so in any checkpoint that was
 // quantised group by group.  The device finds out: where it is not so, the sort leaves a mark, the order as it was (the products are then
 // meaningless) and the look-up kernel, launched behind them, replaces the whole result; otherwise that launch returns at once.
+#include <algorithm>
+
 #include "qmm_internal.h"
 
 namespace qmm {
@@ -149,11 +151,21 @@ GptqOrderSpace gptq_order_space(void* workspace, int lhs_dtype, int64_t m, int64
     return p;
 }
 
-// The look-up kernel serves four rows at the cost of little more than one, and sorting costs 20 us and more (us, look-up / sorted: 14336 x 4096
-// 4 bf16 rows 29 / 34, 5 rows 47 / 35, 16 rows 87 / 36; 4096 x 4096 5 rows 41 / 27; 1024 x 4096 5 rows 41 / 22).  It walks K with one workgroup
-// per 64 columns, though, so that on few columns and a long K sorting wins from the first row: 4096 x 14336 with 1 / 4 rows 62 / 89, sorted 49.
-bool gptq_order_wanted(int64_t m, int64_t n, int64_t k) {
-    return (m >= 5 || (k > 8192 && n <= 4096)) && k <= 32768 && n % 8 == 0 && k % 32 == 0 && !kernel_disabled("gptq_order");
+// The look-up kernel or the sort and the direct GEMM: the predicted time of both in microseconds.  The look-up kernel walks K with one workgroup per 64
+// columns, in passes of up to four rows; where its table of scales does not fit LDS (small groups on a long K), every weight reads its
+// scale from memory.  The sorted way is five launches and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
+// 20 matrices (512 x 512 .. 8192 x 28672, groups of 32 and 128) with 1 .. 16 rows: 9 .. 12 % off, and what it picks takes 0.4 % longer on average than
+// the faster of the two.  us, look-up / sorted: 14336 x 4096 4 bf16 rows 25 / 38, 6 rows 45 / 38, fp32 8 rows 41 / 40; 4096 x 4096 4 / 5 rows
+// 23 / 25, 35 / 25; 512 x 512 8 / 16 rows 11 / 14, 21 / 13; 4096 x 14336 one row 39 / 51, two 66 / 51; group 32 one row 182 / 57.
+bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
+    if (k > 32768 || n % 8 || k % 32 || kernel_disabled("gptq_order")) return false;
+    const bool f32 = lhs_dtype == QMM_F32;
+    const double kk = k / 1024.0, w = (double)n * k / (1 << 20);
+    const double rows[4] = {0.0, 1.0, f32 ? 1.06 : 1.45, f32 ? 1.42 : 1.7};  // a pass of that many, over a pass of one
+    double one = 1.9 + 2.75 * kk * std::max(1.0, n / 16384.0) + 0.06 * w;
+    if (!gptq_act_order_table_fits(m, k, group)) one *= f32 ? 1.9 : 3.0;
+    const double look_up = one * ((m / 4) * rows[3] + rows[std::min<int64_t>(m % 4, 3)]);
+    return look_up > 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0);
 }
 
 hipError_t launch_gptq_order(const void* lhs, int lhs_dtype, const uint32_t* qweight, const int32_t* g_idx, int64_t m, int64_t n, int64_t k, int group,

@@ -400,7 +400,7 @@ static qmm_gptq_config plain_groups(qmm_gptq_config cfg) {
 // takes (2^32 weights) stay with the look-up kernel.
 static bool order_direct() { return !qmm::kernel_disabled("direct"); }
 static int64_t order_bytes(const qmm_gptq_config& cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
-    if (!cfg.desc_act || cfg.group_size <= 0 || k % cfg.group_size || (flags & ~QMM_FLAG_OUT_BF16) || !qmm::gptq_order_wanted(m, n, k) || n * k >= ((int64_t)1 << 32)) return 0;
+    if (!cfg.desc_act || cfg.group_size <= 0 || k % cfg.group_size || (flags & ~QMM_FLAG_OUT_BF16) || !qmm::gptq_order_wanted(lhs_dtype, m, n, k, cfg.group_size) || n * k >= ((int64_t)1 << 32)) return 0;
     const qmm_gptq_config plain = plain_groups(cfg);
     return qmm::gptq_order_space(nullptr, lhs_dtype, m, n, k).bytes +
            up256(order_direct() ? qmm::gemm_direct_workspace_bytes(QMM_GPTQ, lhs_dtype, m, k) : preferred_matmul(QMM_GPTQ, &plain, lhs_dtype, m, n, k, 0));

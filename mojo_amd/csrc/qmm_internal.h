@@ -170,7 +170,8 @@ struct GptqOrderSpace {
     int64_t bytes;
 };
 GptqOrderSpace gptq_order_space(void* workspace, int lhs_dtype, int64_t m, int64_t n, int64_t k);
-bool gptq_order_wanted(int64_t m, int64_t n, int64_t k);
+bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
+bool gptq_act_order_table_fits(int64_t m, int64_t k, int group);  // the look-up kernel's scales in LDS
 hipError_t launch_gptq_order(const void* lhs, int lhs_dtype, const uint32_t* qweight, const int32_t* g_idx, int64_t m, int64_t n, int64_t k, int group,
                              const GptqOrderSpace& p, hipStream_t s);
 bool gemv_q4_k_kc_supported(const void* w, int64_t k);
