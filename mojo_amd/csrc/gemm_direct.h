@@ -105,7 +105,7 @@ struct StagedRows {
 };
 
 // fp32 rows: the products of the residual are summed apart from those of the hi part until the end of the block.  Added to the same sum they
-// double its roundings, and the difference of codes and minima magnifies them (4096 x 4096, 100 rows: relative error 4.0e-7, apart 3.2e-7; 0 to
+// double its roundings, and the difference of codes and minima magnifies them (4096 x 4096, 100 rows, one flush a block: relative error 4.0e-7, apart 3.2e-7; 0 to
 // 10 % of the time of these kernels).
 //
 // Q4_K, Q5_K.  Lane (column nl of a group, half g) takes bytes 16 g .. 16 g + 15 of each of the four 32-byte code runs of a block: run c is

@@ -12,7 +12,7 @@
 //
 // Arithmetic (exact products, fp32 sums), per scale block of a column:
 //   acc += d * sum(u * a16) [+ -dmin * sum(mn * s)],  u: integer weights (sc * q, or q - zero), a16: the row scaled by a power of two and
-//   narrowed to fp16 (fp32 rows: hi + residual, both products into one accumulator), s: sub-block sums of the scaled row as hi + lo.
+//   narrowed to fp16 (fp32 rows: hi + residual; Q4_K and Q5_K sum their products apart), s: sub-block sums of the scaled row as hi + lo.
 //   Q6_K: sc * q may need 13 bits, so sc = 16 hi + lo gives two integer operands per weight (see gemm_planes.hip).
 #include <math.h>
 #include <stdlib.h>
@@ -226,6 +226,13 @@ constexpr int direct_ahead(int flush, int fm, int fn, bool hilo, bool split) {
     return flush == 2 && hilo ? 8 : 16;
 }
 
+// Steps after which the sums in the matrix cores go to the running ones.  A scale block of the K-quants is 16 steps, but every matrix-core
+// instruction rounds its sum, and with codes that are all positive the sums are large against what is left of them.  Relative error with one
+// flush a block / two / four (the small-batch kernels): Q5_K bf16 rows 2.2e-7 / 1.7e-7 / 1.6e-7 (1.6e-7); Q6_K bf16 rows 1.2e-7 / 0.95e-7 (0.95e-7), fp32
+// rows, twice the products, 2.1e-7 / 1.6e-7 / 1.3e-7 (1.6e-7); Q4_K and Q5_K fp32 rows 3.2e-7 / 2.5e-7.  Time: two 0 .. 1 % (Q6_K bf16 rows up to 6 %), four
+// 0 .. 4 % (Q6_K fp32 rows on two fragments 22 %, in spilled registers).  The same on every tile: a call of its own and one in a group sum alike.
+constexpr int direct_flush(int enc, int flush, bool hilo) { return flush < 16 ? flush : enc == QMM_Q5_K && !hilo ? 4 : 8; }
+
 template <typename W>
 constexpr int direct_slot(int frags) { return W::kStage > frags * 4096 ? W::kStage : frags * 4096; }
 
@@ -237,7 +244,7 @@ template <int ENC, int FLUSH, int FM, int FN, int WK, bool HILO>
 __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
                                                                 int tiles_m, int shares) {
     using W = WeightsOf<ENC, FN, FLUSH>;
-    constexpr int kSlot = direct_slot<W>(FM * FN);
+    constexpr int kSlot = direct_slot<W>(FM * FN), kFlush = direct_flush(ENC, W::kFlush, HILO);
     extern __shared__ __attribute__((aligned(16))) float red[];  // a slot per wavefront: its packed rows, at the end its results [FM * FN][4][64] float4
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int i = (int)(blockIdx.x >> 3), tile_m = i % tiles_m, rest = i / tiles_m, share = rest % shares;
@@ -328,8 +335,8 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                         for (int a = 0; a < FM; a++)
 #pragma unroll
                             for (int f = 0; f < FN; f++) {
-                                if (kSplit && q == 1) L[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], t % W::kFlush == 0 ? zero16 : L[a][f], 0, 0, 0);
-                                else if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], zero16, 0, 0, 0);
+                                if (kSplit && q == 1) L[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], t % kFlush == 0 ? zero16 : L[a][f], 0, 0, 0);
+                                else if (t % kFlush == 0 && pl == 0 && q == 0) P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], zero16, 0, 0, 0);
                                 else P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], P[a][f], 0, 0, 0);
                             }
                 if constexpr (t + 1 < W::kSteps) {
@@ -347,7 +354,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                     __builtin_amdgcn_sched_group_barrier(0x2, (W::kPlanes == 2 ? 28 : 11) * FN / kMfma + 1, 0);
                 });
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (t % W::kFlush == W::kFlush - 1) {
+                if constexpr (t % kFlush == kFlush - 1) {
 #pragma unroll
                     for (int f = 0; f < FN; f++) {
                         if constexpr (ENC == QMM_Q4_0) {
@@ -363,7 +370,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                             continue;
                         }
                         float d = 0.0f;
-                        if constexpr (ENC == QMM_GPTQ) d = w.template scale_at<t / W::kFlush>(f);
+                        if constexpr (ENC == QMM_GPTQ) d = w.template scale_at<t / kFlush>(f);
                         else d = w.scale(f);
 #pragma unroll
                         for (int a = 0; a < FM; a++) {
@@ -372,7 +379,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                             // (left to itself the compiler puts these off and keeps the P of every scale block)
                             asm volatile("" : "+v"(T[a][f]));
                         }
-                        if constexpr (W::kMin) {
+                        if constexpr (W::kMin && t + 1 == W::kSteps) {
                             const half8 mo = w.min_operand(f);
                             const float dmin = w.min_scale(f);
 #pragma unroll
@@ -501,7 +508,9 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
     const SharedCost& c = kSharedCost[row][type];
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
         for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, m, n, k));
-        if (m > 32 && !kernel_disabled("shared"))
+        // (Q6_K up to 64 rows: the shared kernel sums 16 steps of two planes in one go, 1.1e-7 relative error with bf16 rows and 2.0e-7 with fp32 rows
+        // where the direct one has 0.95e-7 and 1.6e-7; 14336 x 4096 with 33 rows: bf16 27.4 us in either, fp32 36.3 and 39.0)
+        if (m > (encoding == QMM_Q6_K ? 64 : 32) && !kernel_disabled("shared"))
             for (int i = 0; i < 3; i++)  // (between predictions that close, workgroups of four wavefronts took 5 .. 7 % longer)
                 consider(kSharedPlans[i], shares, shared_us(c, i, shares, encoding, m, n, k) * (i == 2 ? 1.03 : 1.0));
     }
