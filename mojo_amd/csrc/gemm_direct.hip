@@ -271,6 +271,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             inv[e][r] = p.inv[min(row, m - 1)];
         }
     constexpr bool kSplit = HILO && W::kMin;  // the residual's products in sums of their own (see gemm_direct.h)
+    constexpr bool kUnit = unit_sums(ENC, kFlush, HILO) && ENC != QMM_Q4_0;  // (Q4_0 on two fragments has no registers for them)
     float16v T[FM][FN];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             const bool more = u + 1 < u1;
             w.open();
             if (more) w.load(u + 1);
-            float16v P[FM][FN], L[kSplit ? FM : 1][kSplit ? FN : 1];
+            float16v P[FM][FN], U[kUnit ? FM : 1][kUnit ? FN : 1], L[kSplit ? FM : 1][kSplit ? FN : 1];
             half8 sf[FM];
             if constexpr (W::kMin || ENC == QMM_Q4_0) {
 #pragma unroll
@@ -375,9 +376,14 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
 #pragma unroll
                         for (int a = 0; a < FM; a++) {
 #pragma unroll
-                            for (int r = 0; r < 16; r++) T[a][f][r] = fmaf(d, kSplit ? P[a][f][r] + L[a][f][r] : P[a][f][r], T[a][f][r]);
+                            for (int r = 0; r < 16; r++) {
+                                if constexpr (kUnit) U[a][f][r] = t < kFlush ? d * P[a][f][r] : fmaf(d, P[a][f][r], U[a][f][r]);
+                                else T[a][f][r] = fmaf(d, kSplit ? P[a][f][r] + L[a][f][r] : P[a][f][r], T[a][f][r]);
+                                if constexpr (kUnit && t + 1 == W::kSteps) T[a][f][r] += U[a][f][r];
+                            }
                             // (left to itself the compiler puts these off and keeps the P of every scale block)
-                            asm volatile("" : "+v"(T[a][f]));
+                            if constexpr (kUnit) asm volatile("" : "+v"(U[a][f]));
+                            else asm volatile("" : "+v"(T[a][f]));
                         }
                         if constexpr (W::kMin && t + 1 == W::kSteps) {
                             const half8 mo = w.min_operand(f);

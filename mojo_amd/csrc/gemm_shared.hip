@@ -45,6 +45,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
     if (threadIdx.x < 32 * FM) inv[threadIdx.x] = p.inv[min(m0 + (int)threadIdx.x, m - 1)];
 
     constexpr bool kSplit = HILO && W::kMin;  // the residual's products in sums of their own (see gemm_direct.h)
+    constexpr bool kUnit = unit_sums(ENC, W::kFlush, HILO);
     float16v T[FM];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
                 sf[a] = *(const half8*)((const uint8_t*)p.sums + ((int64_t)min(tile_m * FM + a, last_tile) * units + u) * 1024 + l16);
         };
         if constexpr (ENC == QMM_Q4_0) load_sums();
-        float16v P[FM], L[kSplit ? FM : 1];
+        float16v P[FM], U[kUnit ? FM : 1], L[kSplit ? FM : 1];
         half8 b[2][W::kPlanes];
         w.template step<0>(0, b[0]);
         __builtin_amdgcn_sched_barrier(0);
@@ -156,8 +157,11 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
                     for (int a = 0; a < FM; a++) {
                         const float16v S = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf[a], dw, zero16, 0, 0, 0);
 #pragma unroll
-                        for (int r = 0; r < 16; r++) T[a][r] = fmaf(P[a][r], S[r], T[a][r]);
-                        asm volatile("" : "+v"(T[a]));
+                        for (int r = 0; r < 16; r++) {
+                            U[a][r] = t < W::kFlush ? P[a][r] * S[r] : fmaf(P[a][r], S[r], U[a][r]);
+                            if constexpr (t + 1 == W::kSteps) T[a][r] += U[a][r];
+                        }
+                        asm volatile("" : "+v"(U[a]));
                     }
                 } else {
                     float d = 0.0f;
@@ -166,8 +170,13 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
 #pragma unroll
                     for (int a = 0; a < FM; a++) {
 #pragma unroll
-                        for (int r = 0; r < 16; r++) T[a][r] = fmaf(d, kSplit ? P[a][r] + L[a][r] : P[a][r], T[a][r]);
-                        asm volatile("" : "+v"(T[a]));
+                        for (int r = 0; r < 16; r++) {
+                            if constexpr (kUnit) U[a][r] = t < W::kFlush ? d * P[a][r] : fmaf(d, P[a][r], U[a][r]);
+                            else T[a][r] = fmaf(d, kSplit ? P[a][r] + L[a][r] : P[a][r], T[a][r]);
+                            if constexpr (kUnit && t + 1 == W::kSteps) T[a][r] += U[a][r];
+                        }
+                        if constexpr (kUnit) asm volatile("" : "+v"(U[a]));
+                        else asm volatile("" : "+v"(T[a]));
                     }
                     if constexpr (W::kMin) {
                         const half8 mo = w.min_operand(0);

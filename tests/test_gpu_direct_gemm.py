@@ -168,6 +168,9 @@ PRECISION = [
     ("Q6_K", 0, "f32", 33, 11008, 4096, 1.8e-7),   # 1.6e-7 (2.05e-7)
     ("GPTQ", 128, "bf16", 33, 4096, 4096, 0.72e-7),  # 0.64e-7
     ("GPTQ", 128, "f32", 33, 4096, 4096, 1.35e-7),   # 1.22e-7
+    ("GPTQ", 32, "bf16", 300, 11008, 4096, 1.0e-7),  # 0.9e-7 (one chain over K: 2.0e-7)
+    ("GPTQ", 32, "bf16", 100, 5120, 5120, 1.1e-7),   # 1.0e-7 (1.2e-7)
+    ("Q4_0", 0, "bf16", 700, 5120, 5120, 1.4e-7),    # 1.2e-7 (2.3e-7)
 ]
 
 
