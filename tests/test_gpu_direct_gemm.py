@@ -166,6 +166,10 @@ PRECISION = [
     ("Q6_K", 0, "bf16", 33, 11008, 4096, 1.07e-7),  # 0.96e-7 (1.12e-7)
     ("Q6_K", 0, "f32", 9, 4096, 4096, 1.8e-7),     # 1.6e-7 (2.1e-7)
     ("Q6_K", 0, "f32", 33, 11008, 4096, 1.8e-7),   # 1.6e-7 (2.05e-7)
+    ("Q4_K", 0, "bf16", 3, 6400, 1024, 1.0e-7),    # 0.9e-7: the decode kernel (the direct GEMM: 1.5e-7)
+    ("Q5_K", 0, "bf16", 4, 6400, 1024, 1.15e-7),   # 1.0e-7: likewise (1.45e-7)
+    ("Q6_K", 0, "f32", 5, 6400, 1024, 1.15e-7),    # 1.0e-7: likewise (1.55e-7)
+    ("Q5_K", 0, "bf16", 3, 2056, 1280, 1.15e-7),   # 1.0e-7: likewise (1.45e-7)
     ("GPTQ", 128, "bf16", 33, 4096, 4096, 0.72e-7),  # 0.64e-7
     ("GPTQ", 128, "f32", 33, 4096, 4096, 1.35e-7),   # 1.22e-7
     ("GPTQ", 32, "bf16", 300, 11008, 4096, 1.0e-7),  # 0.9e-7 (one chain over K: 2.0e-7)
