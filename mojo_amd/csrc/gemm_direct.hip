@@ -468,7 +468,7 @@ constexpr DirectCost kDirectCost[6][2] = {
 double direct_us(const DirectCost& c, int plan, int shares, int encoding, int64_t m, int64_t n, int64_t k) {
     const DirectPlan& p = kDirectPlans[plan];
     const int64_t wgs = ((m + 32 * p.fm - 1) / (32 * p.fm)) * ((n + 32 * p.fn - 1) / (32 * p.fn)) * shares;
-    const int64_t slots = p.wk == 8 ? 256 : 512, rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
+    const int64_t slots = compute_units() * (p.wk == 8 ? 1 : 2), rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
     const double bytes = encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56;
     return c.base + rounds * (c.round + walk * c.unit[plan]) + c.weights * (bytes * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
 }
@@ -493,9 +493,9 @@ constexpr SharedCost kSharedCost[6][2] = {
 };
 double shared_us(const SharedCost& c, int plan, int shares, int encoding, int64_t m, int64_t n, int64_t k) {
     const DirectPlan& p = kSharedPlans[plan];
-    const int64_t wgs = ((m + 63) / 64) * ((n + 32 * p.wn - 1) / (32 * p.wn)) * shares, slots = p.wn * p.wk == 8 ? 256 : 512;
+    const int64_t wgs = ((m + 63) / 64) * ((n + 32 * p.wn - 1) / (32 * p.wn)) * shares, cus = compute_units(), slots = cus * (p.wn * p.wk == 8 ? 1 : 2);
     const int64_t rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
-    const double unit = slots == 512 && wgs <= 256 ? c.unit_alone : c.unit[plan];
+    const double unit = slots > cus && wgs <= cus ? c.unit_alone : c.unit[plan];
     return c.base + rounds * (c.round + walk * unit) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
 }
 // whole_tiles: one workgroup per tile (bf16 results are stored, not added up); like: with that plan's cut of K
@@ -606,10 +606,10 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
         if (shared && encoding != QMM_Q4_0 && (m <= 1100 || (m <= 1400 && r <= 5.5)) && (encoding != QMM_GPTQ || k <= 8192)) return true;
         return m <= (w <= 24 || (encoding != QMM_Q4_0 && encoding != QMM_GPTQ) ? 720 : 450) || (k <= 1024 ? r <= 6 : m < 1100 && r <= 3.5);
     }
-    // (one round of 64 x 256 tiles that fills the part by four fifths or more: 11008 x 4096 320 bf16 rows Q4_K 78 / 55, GPTQ 71 / 53, Q5_K 85 / 63;
+    // (one round of 64 x 256 tiles that fills the compute units by four fifths or more: 11008 x 4096 320 bf16 rows Q4_K 78 / 55, GPTQ 71 / 53, Q5_K 85 / 63;
     // 8192 x 8192 500 rows Q6_K 205 / 162, Q5_K 145 / 119, but Q4_K 106 / 105 and GPTQ 92 / 101)
     const int64_t tiles = (m + 63) / 64 * ((n + 255) / 256);
-    if (shared && tiles >= 205 && tiles <= 256 && k <= (encoding == QMM_Q4_K || encoding == QMM_GPTQ ? 4096 : 8192)) return true;
+    if (shared && 5 * tiles >= 4 * compute_units() && tiles <= compute_units() && k <= (encoding == QMM_Q4_K || encoding == QMM_GPTQ ? 4096 : 8192)) return true;
     return m <= anyway || (m <= 1100 && r <= most);
 }
 

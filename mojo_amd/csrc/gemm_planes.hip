@@ -1029,12 +1029,10 @@ WidePlan wide_plan(int64_t m, int64_t n, int cus) {
 }
 
 int compute_units() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-    }
+    static const int cus = [] {
+        int dev = 0, count = 0;
+        return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && count > 0 ? count : 256;
+    }();
     return cus;
 }
 

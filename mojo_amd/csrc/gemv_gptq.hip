@@ -240,12 +240,6 @@ hipError_t launch_gemv_gptq_cols(const void* a, int a_dtype, const uint32_t* qwe
     if (m > 4 || group % 32) return hipSuccess;
     const int mt = m <= 1 ? 1 : m <= 2 ? 2 : 4;
     // few columns: the kernel with 16 columns per workgroup
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-    }
     if (gemv_gptq_cols16_wanted(n, group)) {
         const size_t lds16 = ((size_t)kWaves * mt * group + (size_t)kWaves * mt * 64) * 4;
         const int per_xcd = (int)(((n + 15) / 16 + 7) / 8);

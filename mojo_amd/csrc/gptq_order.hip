@@ -162,7 +162,7 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     const bool f32 = lhs_dtype == QMM_F32;
     const double kk = k / 1024.0, w = (double)n * k / (1 << 20);
     const double rows[4] = {0.0, 1.0, f32 ? 1.06 : 1.45, f32 ? 1.42 : 1.7};  // a pass of that many, over a pass of one
-    double one = 1.9 + 2.75 * kk * std::max(1.0, n / 16384.0) + 0.06 * w;
+    double one = 1.9 + 2.75 * kk * std::max(1.0, n / (64.0 * compute_units())) + 0.06 * w;
     if (!gptq_act_order_table_fits(m, k, group)) one *= f32 ? 1.9 : 3.0;
     const double look_up = one * ((m / 4) * rows[3] + rows[std::min<int64_t>(m % 4, 3)]);
     return look_up > 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0);

@@ -19,6 +19,9 @@ bool kernel_disabled(const char* family);
 // result in the workspace) does not fit its scratch: the GEMMs then take their two passes.  Per thread.
 bool twin_rows_allowed();
 
+// compute units of the current device (asked for once; 256 where there is none)
+int compute_units();
+
 // gemm_direct.hip: a few to a few hundred lhs rows, every encoding; out16 != null: bf16 results (out is then unused)
 bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k);
