@@ -13,7 +13,8 @@ namespace qmm {
 // them, hi then residual), and room for one more unit behind the last (the loop reads ahead); sums: one operand per 256 columns; inverse row scales.
 struct DirectSpace {
     _Float16* a16;
-    _Float16* sums;
+    _Float16* sums;  // of 32 columns, hi and lo parts (Q4_0: the block scales)
+    float* sums32;   // the same in fp32: four per lane and 256 columns (Q4_K, Q5_K)
     float* inv;
     int64_t bytes;
 };
@@ -104,16 +105,23 @@ struct StagedRows {
     }
 };
 
-// fp32 rows: the products of the residual are summed apart from those of the hi part until the end of the block.  Added to the same sum they
-// double its roundings, and the difference of codes and minima magnifies them (4096 x 4096, 100 rows, one flush a block: relative error 4.0e-7, apart 3.2e-7; 0 to
-// 10 % of the time of these kernels).
-//
 // Q4_K, Q5_K.  Lane (column nl of a group, half g) takes bytes 16 g .. 16 g + 15 of each of the four 32-byte code runs of a block: run c is
 // sub-block 2 c in its low nibbles and 2 c + 1 in its high ones.  A nibble masked in place reads as the fp16 subnormal q 2^-24 (low) or
 // q 2^-20 (high); times 32 sc or 2 sc it is sc q 2^-19, exact (sc q at most 1953), and a normal number from sc q = 32 on: the matrix cores
 // keep fewer bits of a sum whose operands are subnormal (fp32 rows, 2.5e-7 relative error against 6e-7 with sc q 2^-24).
-template <int ENC, int FN>
+//
+// CENTER (the direct kernel): the operand is sc (q - kMid), exact as well (one fused multiply-add), and what that leaves out, kMid d sc - dmin mn per
+// sub-block, multiplies the sums of the lhs in fp32 (four matrix-core instructions of their own, onto the running sums).  Codes that are all positive
+// make sums 2.4 times as large as what the minima leave of them, and the error of a sum of the lhs counts fifteenfold.  Relative error without and with
+// it (decode kernel): Q4_K 4096 x 4096 17 bf16 rows 1.9e-7, 0.9e-7 (0.9e-7), fp32 3.1e-7, 1.7e-7 (2.6e-7); Q5_K 2.2e-7, 1.0e-7 (1.0e-7), 3.2e-7, 1.7e-7
+// (2.4e-7); the time is the same with bf16 rows and 2 .. 6 % less with fp32 rows, whose residual needs no sums of its own any more.
+//
+// Without CENTER (the shared kernel, whose matrix cores are busier) the minima multiply sums held as hi and lo parts in fp16, and with fp32 rows the products
+// of the residual are summed apart from those of the hi part: added to the same sum they double its roundings, and the difference of codes and minima
+// magnifies them (4096 x 4096, 100 rows: relative error 4.0e-7, apart 3.2e-7; 0 to 10 % of the time).
+template <int ENC, int FN, bool CENTER>
 struct KQuantWeights {
+    static constexpr int kMid = ENC == QMM_Q5_K ? 16 : 8;
     static constexpr int kSteps = 16, kFlush = 16, kPlanes = 1;
     static constexpr bool kMin = true, kPairs = false;
     static constexpr int kCodes = ENC == QMM_Q5_K ? 48 : 16;
@@ -174,7 +182,12 @@ struct KQuantWeights {
                 v[2 * i + 1] |= (bit >= blk + 8 ? e << (bit - blk - 8) : e >> (blk + 8 - bit)) & fm;
             }
         }
-        b[0] = pack4(pk_mul(v[0], sp), pk_mul(v[1], sp), pk_mul(v[2], sp), pk_mul(v[3], sp));
+        if constexpr (CENTER) {
+            const uint32_t mid = pk_mul(sp, 0x80008000u | (uint32_t)kMid * (h == 0 ? 0x00010001u : 0x00100010u));  // -kMid 2^-24 or 2^-20
+            b[0] = pack4(pk_fma(v[0], sp, mid), pk_fma(v[1], sp, mid), pk_fma(v[2], sp, mid), pk_fma(v[3], sp, mid));
+        } else {
+            b[0] = pack4(pk_mul(v[0], sp), pk_mul(v[1], sp), pk_mul(v[2], sp), pk_mul(v[3], sp));
+        }
     }
     template <int T>
     __device__ __forceinline__ void before_step() {
@@ -184,6 +197,13 @@ struct KQuantWeights {
     __device__ __forceinline__ void after_step(int) {}
     __device__ __forceinline__ float scale(int f) const { return h2f((uint16_t)(dm[f] & 0xffffu)) * 524288.0f; }
     __device__ __forceinline__ float min_scale(int f) const { return -h2f((uint16_t)(dm[f] >> 16)); }
+    __device__ __forceinline__ float4 offsets(int f) const {  // kMid d sc - dmin mn of sub-blocks g, 2 + g, 4 + g, 6 + g
+        const float d = (float)kMid * h2f((uint16_t)(dm[f] & 0xffffu)), dmin = min_scale(f);
+        const uint32_t by = goff >> 1;  // 8 g
+        const uint32_t s0 = scs[f][0] >> by, s1 = scs[f][1] >> by, m0 = mns[f][0] >> by, m1 = mns[f][1] >> by;
+        auto of = [&](uint32_t s, uint32_t mn) __attribute__((always_inline)) { return fmaf(d, (float)(s & 0xffu), dmin * (float)(mn & 0xffu)); };
+        return make_float4(of(s0, m0), of(s0 >> 16, m0 >> 16), of(s1, m1), of(s1 >> 16, m1 >> 16));
+    }
     __device__ __forceinline__ half8 min_operand(int f) const {  // the eight mins, for the hi sums (g = 0) and the lo sums (g = 1)
         uint32_t v[4];
 #pragma unroll
@@ -195,10 +215,12 @@ struct KQuantWeights {
 
 // Q6_K.  Half block h: code bytes ql[0..31] (quarters 0 low, 2 high nibbles) and ql[32..63] (quarters 1, 3), two more bits of all four
 // quarters in qh[0..31]; a lane takes bytes 16 g .. 16 g + 15 of each.  (u - 32) 2^-24 or 2^-20 as above, then the two integer operands
-// 16 (sc >> 4) q and (sc & 15) q, times 2^-19.
-template <int FN>
+// 16 (sc >> 4) q and (sc & 15) q, times 2^-19.  FLUSH: steps after which the matrix cores' sums go to the running ones.  Every instruction rounds its
+// sum; with 8, which the direct kernel takes, the relative error of bf16 rows is 0.95e-7 and not 1.2e-7 (small-batch kernel: 0.95e-7), of fp32 rows 1.6e-7
+// and not 2.1e-7 (1.6e-7), for up to 6 % of the time; the shared kernel serves more rows than the small-batch one did and takes 16.
+template <int FN, int FLUSH>
 struct Q6Weights {
-    static constexpr int kSteps = 16, kFlush = 16, kPlanes = 2;
+    static constexpr int kSteps = 16, kFlush = FLUSH, kPlanes = 2;
     static constexpr bool kMin = false, kPairs = false;
     using Rows = StagedRows<Q6_K_BPB, FN>;
     static constexpr int kStage = Rows::kBytes;
@@ -271,6 +293,7 @@ struct Q6Weights {
     __device__ __forceinline__ float scale(int f) const { return h2f((uint16_t)d[f]) * 524288.0f; }
     __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
     __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
+    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
 };
 
 // GPTQ, plain groups.  Word row 32 unit + 4 blk + 2 g + a is a lane's share of step 2 blk + a.  With FN = 2 a lane owns two neighbouring columns
@@ -347,6 +370,7 @@ struct GptqWeights {
     __device__ __forceinline__ float scale_at(int f) const { return h2f((uint16_t)(f ? s_raw[I] >> 16 : s_raw[I] & 0xffffu)); }
     __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
     __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
+    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
 };
 
 // Q4_0: the exact integer block dots of the Q8_0 lhs (codes as fp16) with q - 8, block by block.  Lane half g takes bytes 8 g .. 8 g + 7 of a
@@ -454,6 +478,7 @@ struct Q40Weights {
     __device__ __forceinline__ float scale(int) const { return 0.0f; }
     __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
     __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
+    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
 };
 
 // Scale blocks of 32 columns: the sums of a unit of K (eight blocks) are kept apart from the running ones, which otherwise are a chain of K / 32 rounded
@@ -462,9 +487,9 @@ struct Q40Weights {
 // (fp32 rows: two products a value, no more than 2.2e-7 where the column kernel had 3.3e-7.)
 constexpr bool unit_sums(int enc, int flush, bool hilo) { return (enc == QMM_GPTQ || enc == QMM_Q4_0) && flush == 2 && !hilo; }
 
-template <int ENC, int FN, int FLUSH>
-using WeightsOf = std::conditional_t<ENC == QMM_GPTQ, GptqWeights<FN, FLUSH>, std::conditional_t<ENC == QMM_Q6_K, Q6Weights<FN>,
-                  std::conditional_t<ENC == QMM_Q4_0, Q40Weights<FN>, KQuantWeights<ENC == QMM_Q5_K ? QMM_Q5_K : QMM_Q4_K, FN>>>>;
+template <int ENC, int FN, int FLUSH, bool CENTER>
+using WeightsOf = std::conditional_t<ENC == QMM_GPTQ, GptqWeights<FN, FLUSH>, std::conditional_t<ENC == QMM_Q6_K, Q6Weights<FN, FLUSH>,
+                  std::conditional_t<ENC == QMM_Q4_0, Q40Weights<FN>, KQuantWeights<ENC == QMM_Q5_K ? QMM_Q5_K : QMM_Q4_K, FN, CENTER>>>>;
 
 // compile-time loop: f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>)
 template <int N, int I = 0, typename F>

@@ -11,8 +11,8 @@
 // 1.1 PFLOP/s with FN = 2 (35 TB/s of L2 reads measured, 60 bytes per clock and compute unit).
 //
 // Arithmetic (exact products, fp32 sums), per scale block of a column:
-//   acc += d * sum(u * a16) [+ -dmin * sum(mn * s)],  u: integer weights (sc * q, or q - zero), a16: the row scaled by a power of two and
-//   narrowed to fp16 (fp32 rows: hi + residual; Q4_K and Q5_K sum their products apart), s: sub-block sums of the scaled row as hi + lo.
+//   acc += d * sum(u * a16) [+ sum((mid * d * sc - dmin * mn) * s)],  u: integer weights (sc * (q - mid), or q - zero), a16: the row scaled by a power of
+//   two and narrowed to fp16 (fp32 rows: hi + residual, both products into one accumulator), s: sub-block sums of the scaled row in fp32.
 //   Q6_K: sc * q may need 13 bits, so sc = 16 hi + lo gives two integer operands per weight (see gemm_planes.hip).
 #include <math.h>
 #include <stdlib.h>
@@ -26,7 +26,7 @@ namespace qmm {
 
 namespace {
 
-DirectSpace direct_space(void* ws, bool f32, bool with_sums, int64_t m, int64_t k) {
+DirectSpace direct_space(void* ws, bool f32, bool with_sums, bool with_sums32, int64_t m, int64_t k) {
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     const int64_t tiles = (m + 31) / 32;
     DirectSpace p;
@@ -36,6 +36,8 @@ DirectSpace direct_space(void* ws, bool f32, bool with_sums, int64_t m, int64_t 
     off += tiles * ((k + 255) / 256) * 16384 * (f32 ? 2 : 1) + 32768;
     p.sums = (_Float16*)(base + off);
     off += with_sums ? tiles * ((k + 255) / 256) * 1024 : 0;
+    p.sums32 = (float*)(base + off);
+    off += with_sums32 ? tiles * ((k + 255) / 256) * 1024 : 0;
     p.inv = (float*)(base + off);
     off += up(tiles * 32 * 4);
     p.bytes = off;
@@ -159,6 +161,7 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
                 _Float16* sp = p.sums + ((int64_t)tile * (k >> 8) + (blk >> 3)) * 512 + lane * 8 + (blk & 7);
                 sp[0] = (_Float16)sh;
                 sp[256] = (_Float16)(sum - sh);
+                p.sums32[((int64_t)tile * (k >> 8) + (blk >> 3)) * 256 + (lane + 32 * (blk & 1)) * 4 + ((blk & 7) >> 1)] = sum;
             }
         }
     };
@@ -220,18 +223,11 @@ __global__ __launch_bounds__(1024) void direct_prep_q8_kernel(const AT* __restri
 
 int prep_threads(int64_t k) { return k <= 2048 ? 256 : k <= 4096 ? 512 : 1024; }
 
-constexpr int direct_ahead(int flush, int fm, int fn, bool hilo, bool split) {
-    if (split && fm * fn == 1) return 8;  // (registers)
+constexpr int direct_ahead(int enc, int fm, int fn, bool hilo, int flush) {
     if (fm * fn == 2) return hilo ? 4 : 8;
-    return flush == 2 && hilo ? 8 : 16;
+    // (one fragment of the K-quants with fp32 rows: 16 ahead takes 5 % longer)
+    return hilo && (enc != QMM_GPTQ || flush == 2) ? 8 : 16;
 }
-
-// Steps after which the sums in the matrix cores go to the running ones.  A scale block of the K-quants is 16 steps, but every matrix-core
-// instruction rounds its sum, and with codes that are all positive the sums are large against what is left of them.  Relative error with one
-// flush a block / two / four (the small-batch kernels): Q5_K bf16 rows 2.2e-7 / 1.7e-7 / 1.6e-7 (1.6e-7); Q6_K bf16 rows 1.2e-7 / 0.95e-7 (0.95e-7), fp32
-// rows, twice the products, 2.1e-7 / 1.6e-7 / 1.3e-7 (1.6e-7); Q4_K and Q5_K fp32 rows 3.2e-7 / 2.5e-7.  Time: two 0 .. 1 % (Q6_K bf16 rows up to 6 %), four
-// 0 .. 4 % (Q6_K fp32 rows on two fragments 22 %, in spilled registers).  The same on every tile: a call of its own and one in a group sum alike.
-constexpr int direct_flush(int enc, int flush, bool hilo) { return flush < 16 ? flush : enc == QMM_Q5_K && !hilo ? 4 : 8; }
 
 template <typename W>
 constexpr int direct_slot(int frags) { return W::kStage > frags * 4096 ? W::kStage : frags * 4096; }
@@ -243,8 +239,8 @@ constexpr int direct_slot(int frags) { return W::kStage > frags * 4096 ? W::kSta
 template <int ENC, int FLUSH, int FM, int FN, int WK, bool HILO>
 __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
                                                                 int tiles_m, int shares) {
-    using W = WeightsOf<ENC, FN, FLUSH>;
-    constexpr int kSlot = direct_slot<W>(FM * FN), kFlush = direct_flush(ENC, W::kFlush, HILO);
+    using W = WeightsOf<ENC, FN, FLUSH, true>;
+    constexpr int kSlot = direct_slot<W>(FM * FN);
     extern __shared__ __attribute__((aligned(16))) float red[];  // a slot per wavefront: its packed rows, at the end its results [FM * FN][4][64] float4
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int i = (int)(blockIdx.x >> 3), tile_m = i % tiles_m, rest = i / tiles_m, share = rest % shares;
@@ -270,8 +266,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             const int part_e = min(e * WK + wave, kParts - 1), row = m0 + 32 * ((part_e >> 2) / FN) + 8 * (part_e & 3) + 4 * (lane >> 5) + r;
             inv[e][r] = p.inv[min(row, m - 1)];
         }
-    constexpr bool kSplit = HILO && W::kMin;  // the residual's products in sums of their own (see gemm_direct.h)
-    constexpr bool kUnit = unit_sums(ENC, kFlush, HILO) && ENC != QMM_Q4_0;  // (Q4_0 on two fragments has no registers for them)
+    constexpr bool kUnit = unit_sums(ENC, W::kFlush, HILO) && ENC != QMM_Q4_0;  // (Q4_0 on two fragments has no registers for them)
     float16v T[FM][FN];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -283,7 +278,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
     if (u0 < u1) {
         // Lhs operands are loaded kAhead steps ahead.  Loads return in the order they were issued, so an lhs operand (from L2) waits for
         // the weights (from memory) requested before it: a whole unit ahead where the registers allow it.
-        constexpr int kPer = HILO ? 2 : 1, kAhead = direct_ahead(FLUSH, FM, FN, HILO, kSplit);
+        constexpr int kPer = HILO ? 2 : 1, kOffsetsAt = 12, kAhead = direct_ahead(ENC, FM, FN, HILO, FLUSH);
         const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         W w;
         w.init(wt, n0, lane, (uint8_t*)red + wave * kSlot);
@@ -310,13 +305,13 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             const bool more = u + 1 < u1;
             w.open();
             if (more) w.load(u + 1);
-            float16v P[FM][FN], U[kUnit ? FM : 1][kUnit ? FN : 1], L[kSplit ? FM : 1][kSplit ? FN : 1];
-            half8 sf[FM];
+            float16v P[FM][FN], U[kUnit ? FM : 1][kUnit ? FN : 1];
+            half8 sf[FM];  // (Q4_K, Q5_K: four fp32 sums)
             if constexpr (W::kMin || ENC == QMM_Q4_0) {
 #pragma unroll
                 for (int a = 0; a < FM; a++) {
                     const int tile = min(tile_m * FM + a, (m - 1) >> 5);
-                    sf[a] = *(const half8*)((const uint8_t*)p.sums + ((int64_t)tile * units + u) * 1024 + l16);
+                    sf[a] = *(const half8*)((const uint8_t*)(W::kMin ? (const void*)p.sums32 : (const void*)p.sums) + ((int64_t)tile * units + u) * 1024 + l16);
                 }
             }
             half8 b[2][FN][W::kPlanes];
@@ -336,8 +331,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                         for (int a = 0; a < FM; a++)
 #pragma unroll
                             for (int f = 0; f < FN; f++) {
-                                if (kSplit && q == 1) L[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], t % kFlush == 0 ? zero16 : L[a][f], 0, 0, 0);
-                                else if (t % kFlush == 0 && pl == 0 && q == 0) P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], zero16, 0, 0, 0);
+                                if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], zero16, 0, 0, 0);
                                 else P[a][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a][slot][q], b[cur][f][pl], P[a][f], 0, 0, 0);
                             }
                 if constexpr (t + 1 < W::kSteps) {
@@ -355,7 +349,22 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                     __builtin_amdgcn_sched_group_barrier(0x2, (W::kPlanes == 2 ? 28 : 11) * FN / kMfma + 1, 0);
                 });
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (t % kFlush == kFlush - 1) {
+                if constexpr (W::kMin && t == kOffsetsAt) {  // (the running sums are idle until the flush)
+#pragma unroll
+                    for (int f = 0; f < FN; f++) {
+                        const float4 o = w.offsets(f);
+#pragma unroll
+                        for (int a = 0; a < FM; a++) {
+                            const float4 s = __builtin_bit_cast(float4, sf[a]);
+                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.x, o.x, T[a][f], 0, 0, 0);
+                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.y, o.y, T[a][f], 0, 0, 0);
+                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.z, o.z, T[a][f], 0, 0, 0);
+                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.w, o.w, T[a][f], 0, 0, 0);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (t % W::kFlush == W::kFlush - 1) {
 #pragma unroll
                     for (int f = 0; f < FN; f++) {
                         if constexpr (ENC == QMM_Q4_0) {
@@ -371,29 +380,19 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                             continue;
                         }
                         float d = 0.0f;
-                        if constexpr (ENC == QMM_GPTQ) d = w.template scale_at<t / kFlush>(f);
+                        if constexpr (ENC == QMM_GPTQ) d = w.template scale_at<t / W::kFlush>(f);
                         else d = w.scale(f);
 #pragma unroll
                         for (int a = 0; a < FM; a++) {
 #pragma unroll
                             for (int r = 0; r < 16; r++) {
-                                if constexpr (kUnit) U[a][f][r] = t < kFlush ? d * P[a][f][r] : fmaf(d, P[a][f][r], U[a][f][r]);
-                                else T[a][f][r] = fmaf(d, kSplit ? P[a][f][r] + L[a][f][r] : P[a][f][r], T[a][f][r]);
+                                if constexpr (kUnit) U[a][f][r] = t < W::kFlush ? d * P[a][f][r] : fmaf(d, P[a][f][r], U[a][f][r]);
+                                else T[a][f][r] = fmaf(d, P[a][f][r], T[a][f][r]);
                                 if constexpr (kUnit && t + 1 == W::kSteps) T[a][f][r] += U[a][f][r];
                             }
                             // (left to itself the compiler puts these off and keeps the P of every scale block)
                             if constexpr (kUnit) asm volatile("" : "+v"(U[a][f]));
                             else asm volatile("" : "+v"(T[a][f]));
-                        }
-                        if constexpr (W::kMin && t + 1 == W::kSteps) {
-                            const half8 mo = w.min_operand(f);
-                            const float dmin = w.min_scale(f);
-#pragma unroll
-                            for (int a = 0; a < FM; a++) {
-                                const float16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf[a], mo, zero16, 0, 0, 0);
-#pragma unroll
-                                for (int r = 0; r < 16; r++) T[a][f][r] = fmaf(dmin, M[r], T[a][f][r]);
-                            }
                         }
                     }
                 }
@@ -514,9 +513,9 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
     const SharedCost& c = kSharedCost[row][type];
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
         for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, m, n, k));
-        // (Q6_K up to 64 rows: the shared kernel sums 16 steps of two planes in one go, 1.1e-7 relative error with bf16 rows and 2.0e-7 with fp32 rows
-        // where the direct one has 0.95e-7 and 1.6e-7; 14336 x 4096 with 33 rows: bf16 27.4 us in either, fp32 36.3 and 39.0)
-        if (m > (encoding == QMM_Q6_K ? 64 : 32) && !kernel_disabled("shared"))
+        // (Q5_K and Q6_K up to 64 rows: the shared kernel sums 16 steps in one go, Q6_K those of two planes, 2.2e-7 and 1.1e-7 relative error with bf16
+        // rows where the direct one has 1.0e-7 and 0.95e-7; 14336 x 4096 Q6_K with 33 rows: bf16 27.4 us in either, fp32 36.3 and 39.0)
+        if (m > (encoding == QMM_Q5_K || encoding == QMM_Q6_K ? 64 : 32) && !kernel_disabled("shared"))
             for (int i = 0; i < 3; i++)  // (between predictions that close, workgroups of four wavefronts took 5 .. 7 % longer)
                 consider(kSharedPlans[i], shares, shared_us(c, i, shares, encoding, m, n, k) * (i == 2 ? 1.03 : 1.0));
     }
@@ -530,7 +529,7 @@ hipError_t run_direct(const WeightTensors& wt, DirectMats mats, const DirectSpac
     const int tiles_m = (int)((m + 32 * FM - 1) / (32 * FM));
     int eights = 0;
     for (int j = 0; j < mats.count; j++) mats.end[j] = eights += (mats.n[j] + 256 * FN - 1) / (256 * FN);
-    constexpr int lds = WK * direct_slot<WeightsOf<ENC, FN, FLUSH>>(FM * FN);
+    constexpr int lds = WK * direct_slot<WeightsOf<ENC, FN, FLUSH, true>>(FM * FN);
     hipError_t e = allow_full_lds<gemm_direct_kernel<ENC, FLUSH, FM, FN, WK, HILO>>();
     if (e != hipSuccess) return e;
     gemm_direct_kernel<ENC, FLUSH, FM, FN, WK, HILO><<<dim3((unsigned)(8 * eights * tiles_m * shares)), dim3(64 * WK), lds, s>>>(wt, mats, p, out16, (int)m,
@@ -614,7 +613,8 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
 }
 
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k) {
-    return direct_space(nullptr, lhs_dtype == QMM_F32 && encoding != QMM_Q4_0, encoding == QMM_Q4_K || encoding == QMM_Q5_K || encoding == QMM_Q4_0, m, k).bytes;
+    return direct_space(nullptr, lhs_dtype == QMM_F32 && encoding != QMM_Q4_0, encoding == QMM_Q4_K || encoding == QMM_Q5_K || encoding == QMM_Q4_0,
+                        encoding == QMM_Q4_K || encoding == QMM_Q5_K, m, k).bytes;
 }
 
 // Several matrices: one preparation, and one launch for all those whose own plans cut K the same way (the order of the sums is that of a
@@ -624,7 +624,7 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
                               hipStream_t s) {
     const bool q40 = encoding == QMM_Q4_0, f32 = lhs_dtype == QMM_F32, sums = encoding == QMM_Q4_K || encoding == QMM_Q5_K || q40;
     if (count < 1 || count > kDirectMaxMats) return hipErrorInvalidValue;
-    const DirectSpace p = direct_space(workspace, f32 && !q40, sums, m, k);
+    const DirectSpace p = direct_space(workspace, f32 && !q40, sums, sums && !q40, m, k);
     DirectPlan plans[kDirectMaxMats];
     DirectMats zero{};
     int64_t zeros = 0;
@@ -669,7 +669,7 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
         if (q40) e = run_direct_plan<QMM_Q4_0, 2, false>(pl, wt, mats, p, out16, m, units, s);
         else if (encoding == QMM_Q4_K) QMM_GD_ENC(QMM_Q4_K, 16);
         else if (encoding == QMM_Q5_K) QMM_GD_ENC(QMM_Q5_K, 16);
-        else if (encoding == QMM_Q6_K) QMM_GD_ENC(QMM_Q6_K, 16);
+        else if (encoding == QMM_Q6_K) QMM_GD_ENC(QMM_Q6_K, 8);
         else if (group % 128 == 0) QMM_GD_ENC(QMM_GPTQ, 8);
         else QMM_GD_ENC(QMM_GPTQ, 2);
 #undef QMM_GD_ENC

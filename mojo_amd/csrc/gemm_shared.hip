@@ -22,7 +22,7 @@ constexpr int kLhsBuffers = 2;
 template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO>
 __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
                                                             int tiles_m, int shares) {
-    using W = WeightsOf<ENC, 1, FLUSH>;
+    using W = WeightsOf<ENC, 1, FLUSH, false>;
     constexpr int kPer = HILO ? 2 : 1, kChunk = 8 / kPer, kChunks = W::kSteps / kChunk;
     constexpr int kBuf = FM * kChunk * kPer * 1024, kLoads = FM * kChunk * kPer / WN;
     static_assert(kChunks % kLhsBuffers == 0 && kLoads * WN == FM * kChunk * kPer, "buffers alternate within a unit; whole loads per wavefront");
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
 
 template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO>
 hipError_t run_shared(const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units, int shares, hipStream_t s) {
-    using W = WeightsOf<ENC, 1, FLUSH>;
+    using W = WeightsOf<ENC, 1, FLUSH, false>;
     constexpr int kBuf = FM * 8 * 1024;
     constexpr int lds = WK * kLhsBuffers * kBuf + WN * WK * W::kStage + 32 * FM * 4;
     static_assert(WK == 1 || WN * FM * 4096 <= lds - 32 * FM * 4, "the partial results fit in front of the row scales");

@@ -352,23 +352,18 @@ static int64_t required_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n,
 
 static int64_t up256(int64_t v) { return (v + 255) / 256 * 256; }
 
-// Up to four rows, the decode kernels of Q4_K and Q5_K sum weight by weight in fp32; the matrix cores' sums of codes that are all positive, less
-// the sums of the minima, lose a bit more.  Where those decode kernels are the alternative, they keep the call.  Relative error / us, decode kernel
-// against direct GEMM, 6400 x 1024: Q4_K 4 bf16 rows 0.9e-7 / 12.4 and 1.5e-7 / 7.4; Q5_K 3 bf16 rows 1.0e-7 / 14.8 and 1.4e-7 / 7.5,
-// 3 fp32 rows 2.4e-7 / 15.0 and 3.4e-7 / 7.8; 2056 x 1280 Q5_K 3 bf16 rows 1.0e-7 / 10.2 and 1.45e-7 / 7.4.  Likewise Q6_K with five and six fp32
-// rows on a short K that is no multiple of 2048 (6400 x 1024: 1.0e-7 / 10.9, 12.0 and 1.55e-7 / 9.7; with four rows its decode kernel has 2.5e-7).
-static bool decode_sums_more_exactly(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    if (encoding == QMM_Q6_K) return lhs_dtype == QMM_F32 && (m == 5 || m == 6) && k % 2048 != 0 && k < 4096;
-    if (m > 4) return false;
-    if (encoding == QMM_Q4_K) return q4k_lanes_rows_wins(n, k) && !qmm::kernel_disabled("q4k_lanes_rows");
-    return encoding == QMM_Q5_K && !(q5k_mm_wanted(lhs_dtype, m, n, k) && k % 512 == 0);
+// Q6_K with five and six fp32 rows on a short K that is no multiple of 2048: the kernel behind sums weight by weight in fp32, the matrix cores, with four
+// products a value, a bit less exactly.  Relative error / us against the direct GEMM, 6400 x 1024: 1.0e-7 / 10.9, 12.0 and 1.55e-7 / 9.7 (with four
+// rows the decode kernel has 2.5e-7, from seven on the next one 1.9e-7).
+static bool decode_sums_more_exactly(int encoding, int lhs_dtype, int64_t m, int64_t k) {
+    return encoding == QMM_Q6_K && lhs_dtype == QMM_F32 && (m == 5 || m == 6) && k % 2048 != 0 && k < 4096;
 }
 
 // The direct GEMM serves a problem when the caller's workspace holds its operands (qmm_preferred_workspace_bytes); with the smaller one
 // the other kernels do.
 static int direct_group(const qmm_gptq_config* cfg) { return cfg ? cfg->group_size : 0; }
 static bool direct_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    return qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg)) && !decode_sums_more_exactly(encoding, lhs_dtype, m, n, k);
+    return qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg)) && !decode_sums_more_exactly(encoding, lhs_dtype, m, k);
 }
 static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* workspace, int64_t workspace_bytes) {
     if (encoding == QMM_GPTQ && (!cfg || cfg->desc_act)) return false;
