@@ -14,7 +14,6 @@
 //   acc += d * sum(u * a16) [+ sum((mid * d * sc - dmin * mn) * s)],  u: integer weights (sc * (q - mid), or q - zero), a16: the row scaled by a power of
 //   two and narrowed to fp16 (fp32 rows: hi + residual, both products into one accumulator), s: sub-block sums of the scaled row in fp32.
 //   Q6_K: sc * q may need 13 bits, so sc = 16 hi + lo gives two integer operands per weight (see gemm_planes.hip).
-#include <math.h>
 #include <stdlib.h>
 
 #include <algorithm>
@@ -278,7 +277,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
     if (u0 < u1) {
         // Lhs operands are loaded kAhead steps ahead.  Loads return in the order they were issued, so an lhs operand (from L2) waits for
         // the weights (from memory) requested before it: a whole unit ahead where the registers allow it.
-        constexpr int kPer = HILO ? 2 : 1, kOffsetsAt = 12, kAhead = direct_ahead(ENC, FM, FN, HILO, FLUSH);
+        constexpr int kPer = HILO ? 2 : 1, kAhead = direct_ahead(ENC, FM, FN, HILO, FLUSH);
         const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         W w;
         w.init(wt, n0, lane, (uint8_t*)red + wave * kSlot);
@@ -314,6 +313,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                     sf[a] = *(const half8*)((const uint8_t*)(W::kMin ? (const void*)p.sums32 : (const void*)p.sums) + ((int64_t)tile * units + u) * 1024 + l16);
                 }
             }
+            float of[FN][4];  // Q4_K, Q5_K: offsets of the lane's four sub-blocks
             half8 b[2][FN][W::kPlanes];
 #pragma unroll
             for (int f = 0; f < FN; f++) w.template step<0>(f, b[0][f]);
@@ -349,17 +349,18 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
                     __builtin_amdgcn_sched_group_barrier(0x2, (W::kPlanes == 2 ? 28 : 11) * FN / kMfma + 1, 0);
                 });
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (W::kMin && t == kOffsetsAt) {  // (the running sums are idle until the flush)
+                if constexpr (W::kMin && (t & 3) == 3) {  // the offsets, one instruction behind every fourth step (the running sums are idle until the flush)
+                    constexpr int c = t >> 2;
 #pragma unroll
                     for (int f = 0; f < FN; f++) {
-                        const float4 o = w.offsets(f);
+                        if constexpr (c == 0) {
+                            const float4 o = w.offsets(f);
+                            of[f][0] = o.x, of[f][1] = o.y, of[f][2] = o.z, of[f][3] = o.w;
+                        }
 #pragma unroll
                         for (int a = 0; a < FM; a++) {
                             const float4 s = __builtin_bit_cast(float4, sf[a]);
-                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.x, o.x, T[a][f], 0, 0, 0);
-                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.y, o.y, T[a][f], 0, 0, 0);
-                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.z, o.z, T[a][f], 0, 0, 0);
-                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.w, o.w, T[a][f], 0, 0, 0);
+                            T[a][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(c == 0 ? s.x : c == 1 ? s.y : c == 2 ? s.z : s.w, of[f][c], T[a][f], 0, 0, 0);
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -447,52 +448,66 @@ namespace {
 int64_t direct_units(int64_t k) { return (k + 255) / 256; }
 
 // What a call takes, in microseconds: launches and the preparation of the lhs, a fixed part per round of workgroups (eight wavefronts fill
-// a compute unit, four half of it), the units of K that a wavefront walks, and terms for the weights, the lhs and the results.  Fitted to 143
-// problems per encoding and lhs type (N 512 .. 28672, K 1024 .. 14336, 4 .. 512 rows) in every plan: 4 .. 8 % mean error, and the plan
-// it picks is within 1 % of the best one on average (3 % for GPTQ with a bf16 lhs).
+// a compute unit, four half of it; counted on the XCD with the most, column tiles go to XCDs in eights), the units of K that a wavefront walks, terms for the weights, the lhs and the results, and one for lhs operands
+// beyond 8 MB, which an XCD's L2 does not keep for the next column tile.  Fitted to the problems among 186 per encoding and lhs type (512 x 512 ..
+// 28672 x 4096, K up to 14336, 4 .. 1300 rows, weights from memory; profiles/direct_and_shared_gemm__plans.txt) that these kernels serve, in every plan:
+// 8 .. 13 % off; what it picks takes 1 .. 3 % longer on average than the best plan.
+// unit = 0: a plan that is not built (two fragments side by side spill registers and never win with Q4_0 and Q6_K).
 struct DirectCost {
     float base, round, weights, lhs, out;  // us, us, us per MB of packed weights, us per million lhs values, us per million results and share
     float unit[6];                         // us per unit of K: the plans of kDirectPlans
+    float far;                             // us per 10^9 lhs operands read, where they are more than 8 MB
 };
 constexpr DirectPlan kDirectPlans[6] = {{1, 1, 8, 0, 1}, {2, 1, 8, 0, 1}, {1, 2, 8, 0, 1}, {1, 1, 4, 0, 1}, {2, 1, 4, 0, 1}, {1, 2, 4, 0, 1}};
+constexpr bool direct_built(int encoding, int fn) { return !(fn == 2 && (encoding == QMM_Q4_0 || encoding == QMM_Q6_K)); }
 constexpr DirectCost kDirectCost[6][2] = {
     // bf16 lhs; fp32 lhs
-    {{3.98f, 1.61f, 0.18f, 3.99f, 2.25f, {2.43f, 3.65f, 4.78f, 1.86f, 2.70f, 3.76f}}, {3.99f, 1.60f, 0.18f, 3.98f, 2.32f, {2.43f, 3.63f, 4.77f, 1.86f, 2.70f, 3.75f}}},  // Q4_0
-    {{3.94f, 1.39f, 0.15f, 4.32f, 2.03f, {2.08f, 2.81f, 3.01f, 1.43f, 1.99f, 2.13f}}, {3.42f, 1.40f, 0.18f, 7.65f, 3.27f, {3.19f, 4.39f, 3.95f, 2.13f, 3.06f, 2.62f}}},  // Q4_K
-    {{3.90f, 1.46f, 0.14f, 4.31f, 2.37f, {2.38f, 3.02f, 3.76f, 1.66f, 2.14f, 2.59f}}, {3.36f, 1.52f, 0.16f, 7.53f, 3.65f, {3.46f, 4.46f, 4.43f, 2.29f, 3.08f, 2.91f}}},  // Q5_K
-    {{3.71f, 1.15f, 0.18f, 4.46f, 3.39f, {3.08f, 3.97f, 7.05f, 2.19f, 2.75f, 5.49f}}, {3.00f, 1.77f, 0.22f, 7.86f, 4.87f, {4.39f, 5.70f, 7.66f, 3.01f, 3.67f, 5.98f}}},  // Q6_K
-    {{4.74f, 0.70f, 0.14f, 3.76f, 2.23f, {1.98f, 3.12f, 3.22f, 1.48f, 2.43f, 2.28f}}, {3.48f, 1.55f, 0.16f, 6.98f, 3.33f, {3.20f, 4.42f, 4.00f, 2.35f, 3.20f, 2.87f}}},  // GPTQ, groups of 128
-    {{4.99f, 0.29f, 0.14f, 3.82f, 3.07f, {2.87f, 4.18f, 4.52f, 2.05f, 3.04f, 3.16f}}, {3.78f, 1.19f, 0.14f, 6.67f, 3.76f, {3.83f, 5.23f, 5.14f, 2.79f, 3.72f, 3.56f}}},  // GPTQ, other groups
+    {{3.57f, 1.17f, 0.202f, 2.86f, 3.35f, {2.81f, 3.96f, 0.0f, 2.19f, 3.06f, 0.0f}, 9.94f}, {3.56f, 1.19f, 0.206f, 3.01f, 3.1f, {2.8f, 3.96f, 0.0f, 2.19f, 3.04f, 0.0f}, 9.73f}},  // Q4_0
+    {{4.26f, 0.777f, 0.219f, 3.03f, 3.12f, {2.54f, 3.39f, 3.79f, 1.84f, 2.34f, 2.58f}, 0.0f}, {4.03f, 0.554f, 0.237f, 4.49f, 4.56f, {3.3f, 4.81f, 4.7f, 2.42f, 3.44f, 3.22f}, 31.7f}},  // Q4_K
+    {{4.23f, 0.756f, 0.193f, 2.76f, 3.42f, {3.01f, 3.81f, 4.67f, 2.18f, 2.65f, 3.23f}, 11.5f}, {3.9f, 0.701f, 0.227f, 4.3f, 4.66f, {3.62f, 5.03f, 5.32f, 2.62f, 3.54f, 3.62f}, 33.4f}},  // Q5_K
+    {{3.54f, 1.19f, 0.191f, 2.62f, 3.77f, {3.66f, 4.44f, 0.0f, 2.58f, 3.21f, 0.0f}, 30.9f}, {3.32f, 0.869f, 0.248f, 3.87f, 5.83f, {4.57f, 6.02f, 0.0f, 3.22f, 4.3f, 0.0f}, 50.3f}},  // Q6_K
+    {{4.89f, 0.0f, 0.192f, 2.73f, 3.26f, {2.45f, 3.52f, 3.5f, 1.81f, 2.82f, 2.72f}, 0.0f}, {3.84f, 0.662f, 0.233f, 4.38f, 4.6f, {3.65f, 4.74f, 4.33f, 2.73f, 3.76f, 3.44f}, 23.0f}},  // GPTQ, groups of 128
+    {{4.12f, 0.832f, 0.179f, 2.44f, 3.4f, {3.31f, 4.33f, 4.55f, 2.55f, 3.43f, 3.63f}, 12.7f}, {4.05f, 0.483f, 0.221f, 4.17f, 4.64f, {4.22f, 5.57f, 5.39f, 3.17f, 4.22f, 4.03f}, 23.5f}},  // GPTQ, other groups
 };
-double direct_us(const DirectCost& c, int plan, int shares, int encoding, int64_t m, int64_t n, int64_t k) {
-    const DirectPlan& p = kDirectPlans[plan];
-    const int64_t wgs = ((m + 32 * p.fm - 1) / (32 * p.fm)) * ((n + 32 * p.fn - 1) / (32 * p.fn)) * shares;
-    const int64_t slots = compute_units() * (p.wk == 8 ? 1 : 2), rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
-    const double bytes = encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56;
-    return c.base + rounds * (c.round + walk * c.unit[plan]) + c.weights * (bytes * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
+constexpr bool direct_costs_match_what_is_built() {
+    for (int row = 0; row < 6; row++)
+        for (int type = 0; type < 2; type++)
+            for (int i = 0; i < 6; i++)
+                if ((kDirectCost[row][type].unit[i] != 0.0f) !=
+                    direct_built(row == 0 ? QMM_Q4_0 : row == 1 ? QMM_Q4_K : row == 2 ? QMM_Q5_K : row == 3 ? QMM_Q6_K : QMM_GPTQ, kDirectPlans[i].fn))
+                    return false;
+    return true;
 }
-// The same for the kernel whose wavefronts share the lhs, fitted to 67 problems per encoding and lhs type (33 .. 1300 rows) in every plan: 3 .. 4 %
-// mean error.  It wins where its tiles of 64 x 256 (64 x 128) fill the part with most of K in a workgroup.  us, direct plans / shared: Q4_K, bf16 rows:
-// 14336 x 4096 100 rows 36 / 30, 200 rows 59 / 49, 4096 x 4096 500 rows 42 / 35; fp32 rows: 14336 x 4096 500 rows 183 / 150; Q6_K 4096 x 14336 500
-// bf16 rows 153 / 134; but 4096 x 4096 200 bf16 rows 23.5 / 24.4, 64 rows 12 / 18.
+static_assert(direct_costs_match_what_is_built());
+double direct_us(const DirectCost& c, int plan, int shares, int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    const DirectPlan& p = kDirectPlans[plan];
+    if (c.unit[plan] == 0.0f) return 1e30;
+    const int64_t wgs = ((m + 32 * p.fm - 1) / (32 * p.fm)) * ((n + 256 * p.fn - 1) / (256 * p.fn)) * shares;
+    const int64_t slots = compute_units() / 8 * (p.wk == 8 ? 1 : 2), rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
+    const double bytes = encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56, per = lhs_dtype == QMM_F32 && encoding != QMM_Q4_0 ? 2 : 1;
+    const double far = 2 * m * k * per > 8e6 ? c.far * (m * k * per * 1e-9) * n / (32 * p.fn) : 0.0;
+    return c.base + rounds * (c.round + walk * c.unit[plan]) + c.weights * (bytes * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares + far;
+}
+// The same for the kernel whose wavefronts share the lhs, fitted to the same problems from 33 rows on: 5 .. 8 % off.  It wins where its tiles of 64 x 256
+// (64 x 128) fill the part with most of K in a workgroup.  us, direct plans / shared: Q4_K, bf16 rows: 14336 x 4096 200 rows 59 / 49; fp32 rows:
+// 14336 x 4096 500 rows 183 / 150; Q6_K 4096 x 14336 500 bf16 rows 153 / 134; but 4096 x 4096 Q4_K 64 bf16 rows 12 / 18.
 struct SharedCost {
     float base, round, weights, lhs, out;
     float unit[3], unit_alone;  // the plans of kSharedPlans; four wavefronts with a compute unit to themselves
-    float direct, direct_slope; // what the direct plans took in that measurement (weights from the last-level cache) over direct_us, and per factor e beyond 30 us
 };
 constexpr DirectPlan kSharedPlans[3] = {{2, 1, 1, 0, 8}, {2, 1, 2, 0, 4}, {2, 1, 1, 0, 4}};
 constexpr SharedCost kSharedCost[6][2] = {
     // bf16 lhs; fp32 lhs
-    {{5.92f, 0.42f, 0.106f, 2.20f, 2.84f, {3.49f, 3.63f, 2.86f}, 2.59f, 1.11f, 0.04f}, {6.05f, 0.25f, 0.090f, 2.08f, 2.89f, {3.51f, 3.66f, 2.89f}, 2.60f, 1.10f, 0.05f}},  // Q4_0
-    {{3.82f, 2.47f, 0.071f, 2.18f, 2.93f, {1.97f, 2.26f, 1.95f}, 1.63f, 1.11f, 0.01f}, {4.28f, 1.58f, 0.068f, 3.53f, 3.96f, {3.24f, 3.78f, 3.24f}, 2.38f, 1.15f, 0.05f}},  // Q4_K
-    {{4.75f, 1.94f, 0.076f, 2.26f, 2.94f, {2.45f, 2.65f, 2.29f}, 1.83f, 1.11f, -0.01f}, {4.72f, 1.40f, 0.080f, 3.55f, 3.94f, {3.48f, 4.19f, 3.46f}, 2.57f, 1.16f, 0.04f}},  // Q5_K
-    {{4.41f, 1.99f, 0.064f, 2.55f, 3.16f, {3.51f, 3.88f, 3.24f}, 2.26f, 1.13f, 0.05f}, {3.95f, 1.33f, 0.075f, 4.11f, 4.77f, {5.27f, 6.04f, 5.26f}, 3.40f, 1.20f, 0.15f}},  // Q6_K
-    {{6.52f, 0.30f, 0.052f, 2.16f, 2.66f, {2.30f, 2.48f, 1.78f}, 1.67f, 1.08f, -0.06f}, {6.42f, 0.00f, 0.037f, 3.25f, 3.38f, {3.46f, 4.02f, 3.09f}, 2.62f, 1.11f, 0.01f}},  // GPTQ, groups of 128
-    {{7.46f, 0.00f, 0.070f, 2.30f, 2.59f, {3.40f, 3.57f, 2.55f}, 2.38f, 1.10f, 0.04f}, {6.94f, 0.11f, 0.022f, 3.00f, 3.27f, {4.54f, 5.01f, 4.11f}, 3.21f, 1.14f, 0.05f}},  // GPTQ, other groups
+    {{5.04f, 0.664f, 0.1f, 1.55f, 2.64f, {3.75f, 4.03f, 3.26f}, 2.91f}, {5.17f, 0.534f, 0.105f, 1.67f, 2.58f, {3.74f, 4.02f, 3.24f}, 2.9f}},  // Q4_0
+    {{4.84f, 1.74f, 0.0796f, 1.43f, 2.58f, {2.28f, 2.52f, 2.19f}, 1.85f}, {4.98f, 1.46f, 0.0729f, 2.32f, 3.17f, {3.54f, 4.09f, 3.55f}, 2.62f}},  // Q4_K
+    {{4.95f, 1.59f, 0.08f, 1.47f, 2.61f, {2.7f, 3.02f, 2.76f}, 2.12f}, {4.82f, 1.59f, 0.134f, 2.34f, 3.13f, {3.87f, 4.45f, 3.83f}, 2.81f}},  // Q5_K
+    {{4.91f, 1.37f, 0.109f, 1.73f, 2.69f, {3.85f, 4.21f, 3.64f}, 2.46f}, {3.76f, 1.92f, 0.123f, 2.17f, 3.47f, {5.85f, 6.55f, 5.9f}, 3.71f}},  // Q6_K
+    {{5.33f, 1.07f, 0.0461f, 1.6f, 2.63f, {2.41f, 2.58f, 2.1f}, 1.89f}, {5.98f, 0.298f, 0.0814f, 2.44f, 3.09f, {3.58f, 4.03f, 3.23f}, 2.92f}},  // GPTQ, groups of 128
+    {{6.09f, 0.507f, 0.078f, 1.6f, 2.66f, {3.47f, 3.79f, 3.1f}, 2.65f}, {6.03f, 0.46f, 0.073f, 2.37f, 3.06f, {4.52f, 5.0f, 4.27f}, 3.51f}},  // GPTQ, other groups
 };
-double shared_us(const SharedCost& c, int plan, int shares, int encoding, int64_t m, int64_t n, int64_t k) {
+double shared_us(const SharedCost& c, int plan, int shares, int64_t m, int64_t n, int64_t k) {
     const DirectPlan& p = kSharedPlans[plan];
-    const int64_t wgs = ((m + 63) / 64) * ((n + 32 * p.wn - 1) / (32 * p.wn)) * shares, cus = compute_units(), slots = cus * (p.wn * p.wk == 8 ? 1 : 2);
+    const int64_t wgs = ((m + 63) / 64) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, cus = compute_units() / 8, slots = cus * (p.wn * p.wk == 8 ? 1 : 2);
     const int64_t rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
     const double unit = slots > cus && wgs <= cus ? c.unit_alone : c.unit[plan];
     return c.base + rounds * (c.round + walk * unit) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
@@ -501,27 +516,23 @@ double shared_us(const SharedCost& c, int plan, int shares, int encoding, int64_
 DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, const DirectPlan* like = nullptr) {
     const int row = encoding == QMM_Q4_0 ? 0 : encoding == QMM_Q4_K ? 1 : encoding == QMM_Q5_K ? 2 : encoding == QMM_Q6_K ? 3 : group % 128 == 0 ? 4 : 5;
     const int type = lhs_dtype == QMM_F32 ? 1 : 0;
-    DirectPlan best[2] = {{1, 1, 8, 1, 1}, {}};
-    double us[2] = {1e30, 1e30};  // of the best direct and the best shared plan
+    DirectPlan best{1, 1, 8, 1, 1};
+    double us = 1e29;
     auto consider = [&](const DirectPlan& p, int shares, double t) {
-        const int kind = p.wn > 1 ? 1 : 0;
-        if (t >= us[kind] || (like && (p.wk != like->wk || shares != like->shares || kind != (like->wn > 1 ? 1 : 0)))) return;
-        us[kind] = t;
-        best[kind] = p;
-        best[kind].shares = shares;
+        if (t >= us || (like && (p.wk != like->wk || shares != like->shares || (p.wn > 1) != (like->wn > 1)))) return;
+        us = t;
+        best = p;
+        best.shares = shares;
     };
-    const SharedCost& c = kSharedCost[row][type];
+    // (Q5_K and Q6_K up to 64 rows: the shared kernel sums 16 steps in one go, Q6_K those of two planes, 2.2e-7 and 1.1e-7 relative error with bf16
+    // rows where the direct one has 1.0e-7 and 0.95e-7; 14336 x 4096 Q6_K with 33 rows: bf16 27.4 us in either, fp32 36.3 and 39.0)
+    const bool shared = m > (encoding == QMM_Q5_K || encoding == QMM_Q6_K ? 64 : 32) && !kernel_disabled("shared");
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
-        for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, m, n, k));
-        // (Q5_K and Q6_K up to 64 rows: the shared kernel sums 16 steps in one go, Q6_K those of two planes, 2.2e-7 and 1.1e-7 relative error with bf16
-        // rows where the direct one has 1.0e-7 and 0.95e-7; 14336 x 4096 Q6_K with 33 rows: bf16 27.4 us in either, fp32 36.3 and 39.0)
-        if (m > (encoding == QMM_Q5_K || encoding == QMM_Q6_K ? 64 : 32) && !kernel_disabled("shared"))
-            for (int i = 0; i < 3; i++)  // (between predictions that close, workgroups of four wavefronts took 5 .. 7 % longer)
-                consider(kSharedPlans[i], shares, shared_us(c, i, shares, encoding, m, n, k) * (i == 2 ? 1.03 : 1.0));
+        for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, lhs_dtype, m, n, k));
+        if (shared)  // (between predictions this close these took 3 % less, except GPTQ, and workgroups of four wavefronts 3 % longer)
+            for (int i = 0; i < 3; i++) consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (encoding == QMM_GPTQ ? 1.0 : 0.97) * (i == 2 ? 1.03 : 1.0));
     }
-    if (us[0] >= 1e30) return best[us[1] < 1e30 ? 1 : 0];
-    // (the margin: with it next to no problem of that measurement lost more than 5 % to a wrong choice)
-    return us[1] * (encoding == QMM_GPTQ ? 1.14 : 1.08) < us[0] * (c.direct + c.direct_slope * log(us[0] / 30)) ? best[1] : best[0];
+    return best;
 }
 
 template <int ENC, int FLUSH, int FM, int FN, int WK, bool HILO>
@@ -540,8 +551,9 @@ hipError_t run_direct(const WeightTensors& wt, DirectMats mats, const DirectSpac
 template <int ENC, int FLUSH, bool HILO>
 hipError_t run_direct_plan(const DirectPlan& pl, const WeightTensors& wt, const DirectMats& mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units,
                            hipStream_t s) {
-#define QMM_GD(FM, FN, WK) \
-    if (pl.fm == FM && pl.fn == FN && pl.wk == WK) return run_direct<ENC, FLUSH, FM, FN, WK, HILO>(wt, mats, p, out16, m, units, pl.shares, s)
+#define QMM_GD(FM, FN, WK)                           \
+    if constexpr (direct_built(ENC, FN))             \
+        if (pl.fm == FM && pl.fn == FN && pl.wk == WK) return run_direct<ENC, FLUSH, FM, FN, WK, HILO>(wt, mats, p, out16, m, units, pl.shares, s)
     QMM_GD(1, 1, 8);
     QMM_GD(2, 1, 8);
     QMM_GD(1, 2, 8);
