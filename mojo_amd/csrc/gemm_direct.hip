@@ -592,11 +592,12 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
             if (k > 4096) most = 1.3;
             break;
         case QMM_Q5_K:
-            from = wide && k <= 2048 ? 2 : n >= 2048 && (k % 512 || w <= (f32 ? 16 : 24)) ? 3 : w <= 32 ? 5 : f32 ? 9 : 17;
+            // (5 .. 16 bf16 rows on a long K: the small-batch kernel cuts it into rounds side by side; 1024 x 14336 9 rows 22.2 / 12.5 us)
+            from = wide && k <= 2048 ? 2 : n >= 2048 && (k % 512 || w <= (f32 ? 16 : 24)) ? 3 : w <= 32 && (f32 || k <= 8192 || k % 512) ? 5 : f32 ? 9 : 17;
             break;
         case QMM_Q6_K:
             if (f32) from = k % 2048 == 0 ? 9 : wide ? 3 : n >= 2048 ? 4 : 6;
-            else from = k % 2048 == 0 && !(wide && k <= 2048) ? (w <= 30 ? 5 : 17) : wide ? 2 : n >= 2048 ? 3 : 6;
+            else from = k % 2048 == 0 && !(wide && k <= 2048) ? (w <= 30 && k <= 8192 ? 5 : 17) : wide ? 2 : n >= 2048 ? 3 : 6;
             most = 3.5, anyway = 450;
             break;
         case QMM_GPTQ:
