@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libqmm.so")
@@ -79,15 +80,29 @@ def load() -> C.CDLL:
 _call = None
 
 
+class _Declines:
+    """In place of ``mojo_amd._call`` where that does not load: every function declines every call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def call():
-    """The extension module ``mojo_amd._call`` (``csrc/py_call.cpp``); like the library, it has no fallback."""
+    """The extension module ``mojo_amd._call`` (``csrc/py_call.cpp``).
+
+    It is only the quicker way to ``libqmm.so``: where it is missing or does not load (a Python without its headers, another
+    torch), a warning says so once and every call takes the Python code in ``ops.py``, which reaches the same kernels
+    through ctypes.  Without ``libqmm.so`` this raises as :func:`load` does."""
     global _call
     if _call is None:
         load()
         try:
             from . import _call as native
         except ImportError as e:
-            raise RuntimeError(f"mojo_amd/_call.so is not built or does not load ({e}); run `python -m mojo_amd.build`") from e
+            warnings.warn(f"mojo_amd/_call.so is not built or does not load ({e}): calls go through ctypes, some 8 us slower each; "
+                          "`python -m mojo_amd.build` builds it", RuntimeWarning, stacklevel=3)
+            _call = _Declines()
+            return _call
         from .quantization import _BLOCKS, _CODES
 
         native.setup([(enc, code, *((_BLOCKS[enc].elements_per_block, _BLOCKS[enc].block_size) if enc in _BLOCKS else (0, 0)))

@@ -2,13 +2,15 @@
 import ctypes as C
 import os
 import re
+import sys
+import warnings
 
 import numpy as np
 import pytest
 import torch
 
 import mojo_amd
-from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, _lib
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, _lib, build
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -220,3 +222,37 @@ def test_act_order_beyond_the_direct_gemm_stays_with_the_look_up_kernel():
         least = lib.qmm_matmul_workspace_bytes(QE.GPTQ.code, _lib.QMM_BF16, m, 1 << 17, 1 << 15)
         assert lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, _lib.QMM_BF16, m, (1 << 17) - 8, 1 << 15, 0) > (1 << 31)
         assert lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, _lib.QMM_BF16, m, 1 << 17, 1 << 15, 0) <= least
+
+
+def without_call_module(monkeypatch):
+    """As on an installation where ``_call.so`` is missing: ``from . import _call`` raises ImportError."""
+    monkeypatch.setattr(_lib, "_call", None)
+    monkeypatch.delattr(mojo_amd, "_call", raising=False)
+    monkeypatch.setitem(sys.modules, "mojo_amd._call", None)
+
+
+def test_calls_are_served_without_the_call_module(monkeypatch):
+    without_call_module(monkeypatch)
+    lhs, w = torch.zeros(1, 256), torch.zeros((8, 144), dtype=torch.uint8)
+    with pytest.warns(RuntimeWarning, match="_call.so"):
+        with pytest.raises(ValueError, match="must live on the GPU"):  # the Python code behind the module looked at the call
+            mojo_amd.qmatmul(QE.Q4_K, None, lhs, w)
+    with warnings.catch_warnings():  # the warning comes once
+        warnings.simplefilter("error")
+        gamma = torch.ones(256)
+        for call in (lambda: mojo_amd.qmatmul(QE.Q4_K, None, lhs, w), lambda: mojo_amd.qmatmul_grouped(QE.Q4_K, lhs, [w]),
+                     lambda: mojo_amd.qmatmul_swiglu(QE.Q4_K, lhs, w, w), lambda: mojo_amd.qmatmul_rmsnorm(QE.Q4_K, None, lhs, gamma, 1e-5, w),
+                     lambda: mojo_amd.dequantize(QE.Q4_K, w), lambda: mojo_amd.quantize(QE.Q4_K, lhs),
+                     lambda: mojo_amd.quantize_gptq(torch.zeros(8, 256))):
+            with pytest.raises(ValueError, match="must live on the GPU"):
+                call()
+
+
+def test_a_call_module_that_does_not_compile_is_no_build_error(monkeypatch, tmp_path):
+    call = tmp_path / "_call.so"
+    call.write_bytes(b"an older module")
+    monkeypatch.setattr(build, "CALL", str(call))
+    monkeypatch.setattr(build, "HIPCC", "/bin/false")
+    with pytest.warns(RuntimeWarning, match="ctypes"):
+        build._build_call(force=True, verbose=False)
+    assert not call.exists()
