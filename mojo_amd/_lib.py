@@ -3,10 +3,14 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import sys
 import warnings
+
+import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libqmm.so")
+CALL_PATH = os.path.join(HERE, "_call.so")
 
 QMM_F32, QMM_BF16, QMM_F16 = 0, 1, 2
 QMM_FLAG_W_BF16 = 1
@@ -87,16 +91,32 @@ class _Declines:
         return lambda *args: None
 
 
+def call_stamp() -> str:
+    """What ``_call.so`` is bound to: it reads torch's C++ objects, whose layout another torch (or Python) may change."""
+    return f"qmm_call for torch {torch.__version__} {torch.version.git_version} {sys.implementation.cache_tag};"
+
+
+def call_is_current(path: str) -> bool:
+    """Whether the module file at ``path`` was compiled for this torch and Python (its bytes hold their stamp); nothing is loaded."""
+    try:
+        with open(path, "rb") as f:
+            return call_stamp().encode() in f.read()
+    except OSError:
+        return False
+
+
 def call():
     """The extension module ``mojo_amd._call`` (``csrc/py_call.cpp``).
 
-    It is only the quicker way to ``libqmm.so``: where it is missing or does not load (a Python without its headers, another
-    torch), a warning says so once and every call takes the Python code in ``ops.py``, which reaches the same kernels
-    through ctypes.  Without ``libqmm.so`` this raises as :func:`load` does."""
+    It is only the quicker way to ``libqmm.so``: where it is missing (a Python without its headers), does not
+    load or was compiled for another torch, a warning says so once and every call takes the Python code in ``ops.py``, which
+    reaches the same kernels through ctypes.  Without ``libqmm.so`` this raises as :func:`load` does."""
     global _call
     if _call is None:
         load()
         try:
+            if os.path.exists(CALL_PATH) and not call_is_current(CALL_PATH):
+                raise ImportError("it was compiled for another torch or Python")
             from . import _call as native
         except ImportError as e:
             warnings.warn(f"mojo_amd/_call.so is not built or does not load ({e}): calls go through ctypes, some 8 us slower each; "

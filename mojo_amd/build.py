@@ -95,8 +95,10 @@ def _build_call(force: bool, verbose: bool) -> None:
     """The extension module ``_call`` (host code only) against the headers of the installed torch and ``libqmm.so``.
 
     The package works without it (through ctypes), so where it cannot be compiled that is a warning, and no older module stays."""
+    from . import _lib
+
     src = os.path.join(CSRC, "py_call.cpp")
-    if not force and os.path.exists(CALL) and os.path.getmtime(CALL) > max(os.path.getmtime(src), _headers_mtime()):
+    if not force and _lib.call_is_current(CALL) and os.path.getmtime(CALL) > max(os.path.getmtime(src), _headers_mtime()):
         return
     import sysconfig
 
@@ -104,7 +106,7 @@ def _build_call(force: bool, verbose: bool) -> None:
 
     root = os.path.dirname(torch.__file__)
     cmd = [HIPCC, "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "c++", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
+           f'-DQMM_CALL_STAMP="{_lib.call_stamp()}"', f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
            f"-I{os.path.join(os.path.dirname(os.path.dirname(HIPCC)), 'include')}", src,
            "-o", CALL, f"-L{HERE}", "-l:libqmm.so", f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
     if verbose:

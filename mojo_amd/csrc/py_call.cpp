@@ -447,5 +447,11 @@ PyMODINIT_FUNC PyInit__call(void) {
     s_sym = PyUnicode_InternFromString("sym");
     s_gptq = PyUnicode_InternFromString("gptq");
     if (!s_quant_method || !s_bits || !s_group_size || !s_desc_act || !s_sym || !s_gptq) return nullptr;
-    return PyModule_Create(&g_module);
+    PyObject* const module = PyModule_Create(&g_module);
+    // the build's torch and Python: the loader looks for these bytes in the file before it loads it
+    if (module && PyModule_AddStringConstant(module, "compiled_for", QMM_CALL_STAMP) < 0) {
+        Py_DECREF(module);
+        return nullptr;
+    }
+    return module;
 }

@@ -2,6 +2,7 @@
 import ctypes as C
 import os
 import re
+import subprocess
 import sys
 import warnings
 
@@ -256,3 +257,23 @@ def test_a_call_module_that_does_not_compile_is_no_build_error(monkeypatch, tmp_
     with pytest.warns(RuntimeWarning, match="ctypes"):
         build._build_call(force=True, verbose=False)
     assert not call.exists()
+
+
+def test_a_call_module_of_another_torch_is_rebuilt_and_not_loaded(monkeypatch, tmp_path):
+    assert _lib.call_is_current(_lib.CALL_PATH) and _lib.call().compiled_for == _lib.call_stamp()
+    old = _lib.call_stamp().encode()
+    monkeypatch.setattr(torch, "__version__", torch.__version__ + "x")  # as after an update of torch
+    assert old != _lib.call_stamp().encode() and not _lib.call_is_current(_lib.CALL_PATH)
+    monkeypatch.setattr(_lib, "_call", None)
+    with pytest.warns(RuntimeWarning, match="another torch"):
+        assert _lib.call().matmul() is None
+    call = tmp_path / "_call.so"  # newer than every source
+    call.write_bytes(old)
+    compiled = []
+    monkeypatch.setattr(build, "CALL", str(call))
+    monkeypatch.setattr(build.subprocess, "run", lambda cmd, **kw: compiled.append(cmd) or subprocess.CompletedProcess(cmd, 0, "", ""))
+    build._build_call(force=False, verbose=False)
+    assert len(compiled) == 1
+    call.write_bytes(_lib.call_stamp().encode())
+    build._build_call(force=False, verbose=False)
+    assert len(compiled) == 1  # current: nothing to do
