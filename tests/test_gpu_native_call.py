@@ -36,3 +36,11 @@ def test_native_call_declines_what_is_not_plain():
     with pytest.raises(ValueError, match="K=128"):
         qmatmul(QE.Q4_K, None, a[:, :128].contiguous(), w)
     assert dequantize(QE.Q4_K, w, k=256).shape == (8, 256)
+
+
+def test_without_the_module_the_kernels_are_the_same(monkeypatch):
+    w = quantize(QE.Q4_K, torch.randn(264, 512, device="cuda"))
+    a = torch.randn(3, 512, device="cuda")
+    want = qmatmul(QE.Q4_K, None, a, w), dequantize(QE.Q4_K, w)
+    monkeypatch.setattr(_lib, "_call", _lib._Declines())
+    assert torch.equal(want[0], qmatmul(QE.Q4_K, None, a, w)) and torch.equal(want[1], dequantize(QE.Q4_K, w))

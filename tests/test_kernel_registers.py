@@ -49,3 +49,11 @@ def test_act_order_look_up_keeps_its_table_reads_in_flight(kernels, rows, lhs):
     the compiler schedules one weight at a time takes 23 .. 27 and 14336 x 4096 with one bf16 row 19.1 us instead of 13.6."""
     found = [c for name, c in kernels.items() if re.match(rf"gemv_gptq_act_order_kernel<{rows}, true, .*{lhs}>$", name)]
     assert found and all(registers >= 56 and spilled == 0 for registers, spilled in found), found
+
+
+def test_direct_and_shared_gemms_keep_their_sums_in_registers(kernels):
+    """Their accumulators, operands and read-ahead are sized to the 256 registers of a wavefront.  Two plans (Q4_0 and Q6_K with fp32 rows) give up
+    to seven registers to scratch outside the loop; an fp32 Q6_K body with a flush every four units spilled 30 and was 22 % slower."""
+    found = {name: spilled for name, (_, spilled) in kernels.items() if re.match(r"gemm_(direct|shared)_kernel<", name)}
+    assert len(found) > 60
+    assert {name: spilled for name, spilled in found.items() if spilled > 8} == {}
