@@ -110,15 +110,15 @@ struct StagedRows {
 // q 2^-20 (high); times 32 sc or 2 sc it is sc q 2^-19, exact (sc q at most 1953), and a normal number from sc q = 32 on: the matrix cores
 // keep fewer bits of a sum whose operands are subnormal (fp32 rows, 2.5e-7 relative error against 6e-7 with sc q 2^-24).
 //
-// CENTER (the direct kernel): the operand is sc (q - kMid), exact as well (one fused multiply-add), and what that leaves out, kMid d sc - dmin mn per
-// sub-block, multiplies the sums of the lhs in fp32 (four matrix-core instructions of their own, onto the running sums).  Codes that are all positive
-// make sums 2.4 times as large as what the minima leave of them, and the error of a sum of the lhs counts fifteenfold.  Relative error without and with
-// it (decode kernel): Q4_K 4096 x 4096 17 bf16 rows 1.9e-7, 0.9e-7 (0.9e-7), fp32 3.1e-7, 1.7e-7 (2.6e-7); Q5_K 2.2e-7, 1.0e-7 (1.0e-7), 3.2e-7, 1.7e-7
-// (2.4e-7); the time is the same with bf16 rows and 2 .. 6 % less with fp32 rows, whose residual needs no sums of its own any more.
-//
-// Without CENTER (the shared kernel, whose matrix cores are busier) the minima multiply sums held as hi and lo parts in fp16, and with fp32 rows the products
-// of the residual are summed apart from those of the hi part: added to the same sum they double its roundings, and the difference of codes and minima
-// magnifies them (4096 x 4096, 100 rows: relative error 4.0e-7, apart 3.2e-7; 0 to 10 % of the time).
+// CENTER: the operand is sc (q - kMid), exact as well (one fused multiply-add), and what that leaves out, kMid d sc - dmin mn per sub-block, multiplies the
+// sums of the lhs.  Codes that are all positive make sums 2.4 times as large as what the minima leave of them, and the error of a sum of the lhs counts
+// fifteenfold.  Relative error without and with it, direct kernel (decode kernel): Q4_K 4096 x 4096 17 bf16 rows 1.9e-7, 0.9e-7 (0.9e-7), fp32 3.1e-7,
+// 1.7e-7 (2.6e-7); Q5_K 2.2e-7, 1.0e-7 (1.0e-7), 3.2e-7, 1.7e-7 (2.4e-7).
+// - direct kernel: always, the sums in fp32 (four matrix-core instructions of their own, onto the running sums); the time is the same with bf16 rows and 2 .. 6 %
+//   less with fp32 rows, whose residual would need sums of its own otherwise.
+// - shared kernel, whose matrix cores are busier: both the offsets and the sums as two fp16 terms (two instructions a unit; the offsets exact to 22 bits of the
+//   larger product).  fp32 rows 3.4e-7 -> 1.85e-7 in the same time.  bf16 rows 2.3e-7 -> 1.1e-7, but 3 .. 4 % slower, its vector units being the limit: only Q5_K up
+//   to 64 rows, where the small-batch kernel has 1.6e-7; beyond, the GEMMs that it replaces have 2.6e-7 and more.
 template <int ENC, int FN, bool CENTER>
 struct KQuantWeights {
     static constexpr int kMid = ENC == QMM_Q5_K ? 16 : 8;
@@ -204,6 +204,40 @@ struct KQuantWeights {
         auto of = [&](uint32_t s, uint32_t mn) __attribute__((always_inline)) { return fmaf(d, (float)(s & 0xffu), dmin * (float)(mn & 0xffu)); };
         return make_float4(of(s0, m0), of(s0 >> 16, m0 >> 16), of(s1, m1), of(s1 >> 16, m1 >> 16));
     }
+    // The same as two fp16 terms each, in units of the returned power of two, of all eight sub-blocks (the shared kernel): open them, add sub-block by
+    // sub-block, and they multiply sums that are held as hi (g = 0) and lo parts (g = 1).
+    float od, om;
+    uint32_t ohi[4], olo[4];
+    __device__ __forceinline__ float open_offsets() {
+        const float d = (float)kMid * h2f((uint16_t)(dm[0] & 0xffffu)), dmin = min_scale(0);
+        const int e = __builtin_amdgcn_frexp_expf(64.0f * fmaxf(fabsf(d), fabsf(dmin)));  // both products below 2^e
+        od = ldexpf(d, 14 - e);
+        om = ldexpf(dmin, 14 - e);
+        return ldexpf(1.0f, e - 14);
+    }
+    __device__ __forceinline__ float scale_per_unit() const { return od * (524288.0f / (float)kMid); }
+    // (each half wavefront works out four sub-blocks)
+    template <int PAIR>
+    __device__ __forceinline__ void add_offsets() {
+        if constexpr (PAIR < 2) {
+            const uint32_t sc = goff ? scs[0][1] : scs[0][0], mn = goff ? mns[0][1] : mns[0][0];
+            float v[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) v[i] = fmaf(od, (float)((sc >> (16 * PAIR + 8 * i)) & 0xffu), om * (float)((mn >> (16 * PAIR + 8 * i)) & 0xffu));
+            const half2v hi = {(_Float16)v[0], (_Float16)v[1]};
+            const half2v lo = {(_Float16)(v[0] - (float)hi.x), (_Float16)(v[1] - (float)hi.y)};
+            ohi[PAIR] = as_u32(hi);
+            olo[PAIR] = as_u32(lo);
+        } else {
+            // (both operands the same register: the result's first half is the low lanes' value in every lane, the second that of the high lanes)
+            const auto h = __builtin_amdgcn_permlane32_swap(ohi[PAIR - 2], ohi[PAIR - 2], false, false);
+            const auto l = __builtin_amdgcn_permlane32_swap(olo[PAIR - 2], olo[PAIR - 2], false, false);
+            ohi[PAIR - 2] = h[0], ohi[PAIR] = h[1];
+            olo[PAIR - 2] = l[0], olo[PAIR] = l[1];
+        }
+    }
+    __device__ __forceinline__ half8 offsets_hi() const { return pack4(ohi[0], ohi[1], ohi[2], ohi[3]); }
+    __device__ __forceinline__ half8 offsets_lo() const { return pack4(olo[0], olo[1], olo[2], olo[3]); }
     __device__ __forceinline__ half8 min_operand(int f) const {  // the eight mins, for the hi sums (g = 0) and the lo sums (g = 1)
         uint32_t v[4];
 #pragma unroll
@@ -213,13 +247,26 @@ struct KQuantWeights {
     }
 };
 
+struct NoOffsets {  // the encodings without minima
+    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
+    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
+    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
+    __device__ __forceinline__ float open_offsets() { return 0.0f; }
+    __device__ __forceinline__ float scale_per_unit() const { return 0.0f; }
+    template <int PAIR>
+    __device__ __forceinline__ void add_offsets() {}
+    __device__ __forceinline__ half8 offsets_hi() const { return half8{}; }
+    __device__ __forceinline__ half8 offsets_lo() const { return half8{}; }
+};
+
 // Q6_K.  Half block h: code bytes ql[0..31] (quarters 0 low, 2 high nibbles) and ql[32..63] (quarters 1, 3), two more bits of all four
 // quarters in qh[0..31]; a lane takes bytes 16 g .. 16 g + 15 of each.  (u - 32) 2^-24 or 2^-20 as above, then the two integer operands
 // 16 (sc >> 4) q and (sc & 15) q, times 2^-19.  FLUSH: steps after which the matrix cores' sums go to the running ones.  Every instruction rounds its
 // sum; with 8, which the direct kernel takes, the relative error of bf16 rows is 0.95e-7 and not 1.2e-7 (small-batch kernel: 0.95e-7), of fp32 rows 1.6e-7
-// and not 2.1e-7 (1.6e-7), for up to 6 % of the time; the shared kernel serves more rows than the small-batch one did and takes 16.
+// and not 2.1e-7 (1.6e-7), for up to 6 % of the time.  The shared kernel takes 8 up to 64 rows, with sums of a unit of their own (1.1e-7, 1.7e-7; 2 .. 3 % of the
+// time), and 16 beyond (1.26e-7, 2.1e-7), where the plane GEMM that it replaces has 4e-7 and more.
 template <int FN, int FLUSH>
-struct Q6Weights {
+struct Q6Weights : NoOffsets {
     static constexpr int kSteps = 16, kFlush = FLUSH, kPlanes = 2;
     static constexpr bool kMin = false, kPairs = false;
     using Rows = StagedRows<Q6_K_BPB, FN>;
@@ -291,16 +338,13 @@ struct Q6Weights {
     template <int T>
     __device__ __forceinline__ void after_step(int) {}
     __device__ __forceinline__ float scale(int f) const { return h2f((uint16_t)d[f]) * 524288.0f; }
-    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
-    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
-    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
 };
 
 // GPTQ, plain groups.  Word row 32 unit + 4 blk + 2 g + a is a lane's share of step 2 blk + a.  With FN = 2 a lane owns two neighbouring columns
 // (8-byte loads).  FLUSH: steps per scale block, 8 (groups that are multiples of 128) or 2 (any group: blocks of 32).  A K that is no multiple of
 // 256 ends in a partial unit: its lhs columns beyond K are zeros, its words and scales the last ones of the tensors.
 template <int FN, int FLUSH>
-struct GptqWeights {
+struct GptqWeights : NoOffsets {
     static constexpr int kSteps = 16, kFlush = FLUSH, kPlanes = 1;
     static constexpr bool kMin = false, kPairs = FN == 2;
     static constexpr int kBlocks = 16 / FLUSH, kStage = 0;
@@ -368,16 +412,13 @@ struct GptqWeights {
     __device__ __forceinline__ void after_step(int next_unit) { load_words(next_unit, T); }
     template <int I>
     __device__ __forceinline__ float scale_at(int f) const { return h2f((uint16_t)(f ? s_raw[I] >> 16 : s_raw[I] & 0xffffu)); }
-    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
-    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
-    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
 };
 
 // Q4_0: the exact integer block dots of the Q8_0 lhs (codes as fp16) with q - 8, block by block.  Lane half g takes bytes 8 g .. 8 g + 7 of a
 // block: its low nibbles are columns 8 g + 0..7 of the block (step a = 0), the high ones 16 + 8 g + 0..7 (a = 1).  Rows
 // whose K is no multiple of 256 end in a partial unit: what lies behind the row's end is read as zeros.
 template <int FN>
-struct Q40Weights {
+struct Q40Weights : NoOffsets {
     static constexpr int kSteps = 16, kFlush = 2, kPlanes = 1;
     static constexpr bool kMin = false, kPairs = false;
     static constexpr int kUnit = 8 * Q4_0_BPB, kPieces = kUnit / 16;
@@ -476,16 +517,13 @@ struct Q40Weights {
         return pack4(B >> 1 == 0 ? v : 0u, B >> 1 == 1 ? v : 0u, B >> 1 == 2 ? v : 0u, B >> 1 == 3 ? v : 0u);
     }
     __device__ __forceinline__ float scale(int) const { return 0.0f; }
-    __device__ __forceinline__ float min_scale(int) const { return 0.0f; }
-    __device__ __forceinline__ half8 min_operand(int) const { return half8{}; }
-    __device__ __forceinline__ float4 offsets(int) const { return float4{}; }
 };
 
 // Scale blocks of 32 columns: the sums of a unit of K (eight blocks) are kept apart from the running ones, which otherwise are a chain of K / 32 rounded
 // sums.  Relative error of GPTQ in groups of 32, bf16 rows: 11008 x 4096 with 300 rows 2.0e-7 -> 0.9e-7 (column kernel: 0.95e-7), 5120 x 5120
 // with 700 rows 2.3e-7 -> 1.0e-7; Q4_0, where the wavefronts share the lhs, 5120 x 5120 with 700 rows 2.3e-7 -> 1.1e-7; for less than 1 % of the time.
 // (fp32 rows: two products a value, no more than 2.2e-7 where the column kernel had 3.3e-7.)
-constexpr bool unit_sums(int enc, int flush, bool hilo) { return (enc == QMM_GPTQ || enc == QMM_Q4_0) && flush == 2 && !hilo; }
+constexpr bool unit_sums(int enc, int flush, bool hilo) { return (enc == QMM_Q6_K && flush == 8) || ((enc == QMM_GPTQ || enc == QMM_Q4_0) && flush == 2 && !hilo); }
 
 template <int ENC, int FN, int FLUSH, bool CENTER>
 using WeightsOf = std::conditional_t<ENC == QMM_GPTQ, GptqWeights<FN, FLUSH>, std::conditional_t<ENC == QMM_Q6_K, Q6Weights<FN, FLUSH>,

@@ -265,7 +265,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
             const int part_e = min(e * WK + wave, kParts - 1), row = m0 + 32 * ((part_e >> 2) / FN) + 8 * (part_e & 3) + 4 * (lane >> 5) + r;
             inv[e][r] = p.inv[min(row, m - 1)];
         }
-    constexpr bool kUnit = unit_sums(ENC, W::kFlush, HILO) && ENC != QMM_Q4_0;  // (Q4_0 on two fragments has no registers for them)
+    constexpr bool kUnit = ENC == QMM_GPTQ && unit_sums(ENC, W::kFlush, HILO);  // (Q4_0 and Q6_K on two fragments have no registers for them)
     float16v T[FM][FN];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -524,13 +524,17 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
         best = p;
         best.shares = shares;
     };
-    // (Q5_K and Q6_K up to 64 rows: the shared kernel sums 16 steps in one go, Q6_K those of two planes, 2.2e-7 and 1.1e-7 relative error with bf16
-    // rows where the direct one has 1.0e-7 and 0.95e-7; 14336 x 4096 Q6_K with 33 rows: bf16 27.4 us in either, fp32 36.3 and 39.0)
-    const bool shared = m > (encoding == QMM_Q5_K || encoding == QMM_Q6_K ? 64 : 32) && !kernel_disabled("shared");
+    // Q6_K up to 64 rows, which the small-batch kernel would take in passes of 16: only plans with parts of K of up to 2048, as exact as that kernel
+    // (28672 x 8192 with 64 bf16 rows, shared: parts of 2048 1.0e-7 relative error, of 4096 1.1e-7, small-batch kernel 0.98e-7; 101, 93 and 224 us).
+    const int64_t longest = encoding == QMM_Q6_K && m <= 64 ? 8 : 1 << 20;  // units of K in a part
+    const bool shared = m > 32 && !kernel_disabled("shared");
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++) {
-        for (int i = 0; i < 6; i++) consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, lhs_dtype, m, n, k));
-        if (shared)  // (between predictions this close these took 3 % less, except GPTQ, and workgroups of four wavefronts 3 % longer)
-            for (int i = 0; i < 3; i++) consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (encoding == QMM_GPTQ ? 1.0 : 0.97) * (i == 2 ? 1.03 : 1.0));
+        for (int i = 0; i < 6; i++)
+            if (direct_units(k) <= longest * kDirectPlans[i].wk * shares)
+                consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, lhs_dtype, m, n, k));
+        for (int i = 0; shared && i < 3; i++)  // (between predictions this close these took 3 % less, except GPTQ, and workgroups of four wavefronts 3 % longer)
+            if (direct_units(k) <= longest * kSharedPlans[i].wk * shares)
+                consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (encoding == QMM_GPTQ ? 1.0 : 0.97) * (i == 2 ? 1.03 : 1.0));
     }
     return best;
 }

@@ -17,12 +17,13 @@ namespace qmm {
 namespace {
 
 constexpr int kLhsBuffers = 2;
+constexpr int64_t kFewSharedRows = 64;  // up to which Q5_K and Q6_K take their most exact sums (KQuantWeights, Q6Weights)
 
 // Workgroup id -> tile as in gemm_direct_kernel, with column tiles of 32 WN.
-template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO>
+template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER>
 __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
                                                             int tiles_m, int shares) {
-    using W = WeightsOf<ENC, 1, FLUSH, false>;
+    using W = WeightsOf<ENC, 1, FLUSH, CENTER>;
     constexpr int kPer = HILO ? 2 : 1, kChunk = 8 / kPer, kChunks = W::kSteps / kChunk;
     constexpr int kBuf = FM * kChunk * kPer * 1024, kLoads = FM * kChunk * kPer / WN;
     static_assert(kChunks % kLhsBuffers == 0 && kLoads * WN == FM * kChunk * kPer, "buffers alternate within a unit; whole loads per wavefront");
@@ -44,7 +45,6 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
     const int u0 = (int)((unsigned)units * (unsigned)part / (unsigned)parts), u1 = (int)((unsigned)units * (unsigned)(part + 1) / (unsigned)parts);
     if (threadIdx.x < 32 * FM) inv[threadIdx.x] = p.inv[min(m0 + (int)threadIdx.x, m - 1)];
 
-    constexpr bool kSplit = HILO && W::kMin;  // the residual's products in sums of their own (see gemm_direct.h)
     constexpr bool kUnit = unit_sums(ENC, W::kFlush, HILO);
     float16v T[FM];
 #pragma unroll
@@ -53,7 +53,8 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
         for (int r = 0; r < 16; r++) T[a][r] = 0.0f;
 
     const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    constexpr int kSumsAt = W::kSteps - 4;
+    // Q4_K, Q5_K: the steps at which the sums of the lhs are asked for and multiplied (asked for at step 12 and waited for behind the last one they cost 8 .. 13 % with CENTER)
+    constexpr int kSumsAt = 2, kOffsetsAt = 13;
     const uint32_t l16 = lane * 16;
     uint8_t* const bufs = smem + wk * kLhsBuffers * kBuf;
     W w;
@@ -110,13 +111,14 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
                 sf[a] = *(const half8*)((const uint8_t*)p.sums + ((int64_t)min(tile_m * FM + a, last_tile) * units + u) * 1024 + l16);
         };
         if constexpr (ENC == QMM_Q4_0) load_sums();
-        float16v P[FM], U[kUnit ? FM : 1], L[kSplit ? FM : 1];
+        float16v P[FM], U[kUnit ? FM : 1], M[W::kMin ? FM : 1];
         half8 b[2][W::kPlanes];
+        float offset_unit = 0.0f;
         w.template step<0>(0, b[0]);
         __builtin_amdgcn_sched_barrier(0);
         unrolled<W::kSteps>([&](auto tt) __attribute__((always_inline)) {
             constexpr int t = decltype(tt)::value, chunk = t / kChunk, in = t % kChunk, cur = t & 1;
-            constexpr int kMfma = FM * kPer * W::kPlanes;
+            constexpr int kMfma = FM * kPer * W::kPlanes + (W::kMin && t == kOffsetsAt ? (CENTER ? 2 : 1) * FM : 0);
             if constexpr (in == 0) {
                 __syncthreads();  // this chunk has arrived, the one before it is used up
                 store_lhs((chunk + 1) % kLhsBuffers);
@@ -126,16 +128,27 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
             }
             if constexpr (in + 1 < kChunk) read_lhs(chunk, in + 1, cur ^ 1);
             if constexpr (W::kMin && t == kSumsAt) load_sums();
+            if constexpr (W::kMin && t == kOffsetsAt) {
+                const half8 first = CENTER ? w.offsets_lo() : w.min_operand(0);
+#pragma unroll
+                for (int a = 0; a < FM; a++) M[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf[a], first, zero16, 0, 0, 0);
+                if constexpr (CENTER)
+#pragma unroll
+                    for (int a = 0; a < FM; a++) M[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf[a], w.offsets_hi(), M[a], 0, 0, 0);
+            }
 #pragma unroll
             for (int pl = 0; pl < W::kPlanes; pl++)
 #pragma unroll
                 for (int q = 0; q < kPer; q++)
 #pragma unroll
                     for (int a = 0; a < FM; a++) {
-                        if (kSplit && q == 1) L[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], t % W::kFlush == 0 ? zero16 : L[a], 0, 0, 0);
-                        else if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], zero16, 0, 0, 0);
+                        if (t % W::kFlush == 0 && pl == 0 && q == 0) P[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], zero16, 0, 0, 0);
                         else P[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[cur][a][q], b[cur][pl], P[a], 0, 0, 0);
                     }
+            if constexpr (W::kMin && CENTER && t >= kOffsetsAt - 5 && t < kOffsetsAt) {
+                if constexpr (t == kOffsetsAt - 5) offset_unit = w.open_offsets();
+                else w.template add_offsets<t - (kOffsetsAt - 4)>();
+            }
             if constexpr (t + 1 < W::kSteps) {
                 w.template before_step<t>();
                 w.template step<t + 1>(0, b[cur ^ 1]);
@@ -147,7 +160,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
             if constexpr (in + 1 < kChunk) __builtin_amdgcn_sched_group_barrier(0x100, FM * kPer, 0);  // the next operands first, then the weights in between
             unrolled<kMfma>([&](auto) __attribute__((always_inline)) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, (W::kPlanes == 2 ? 28 : 11) / kMfma + 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, (W::kPlanes == 2 ? 28 : W::kMin ? 17 : 11) / kMfma + 1, 0);
             });
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (t % W::kFlush == W::kFlush - 1) {
@@ -167,27 +180,19 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
                     float d = 0.0f;
                     if constexpr (ENC == QMM_GPTQ) d = w.template scale_at<t / W::kFlush>(0);
                     else d = w.scale(0);
+                    const float per_unit = CENTER ? w.scale_per_unit() : 0.0f, dmin = w.min_scale(0);
 #pragma unroll
                     for (int a = 0; a < FM; a++) {
 #pragma unroll
                         for (int r = 0; r < 16; r++) {
                             if constexpr (kUnit) U[a][r] = t < W::kFlush ? d * P[a][r] : fmaf(d, P[a][r], U[a][r]);
-                            else T[a][r] = fmaf(d, kSplit ? P[a][r] + L[a][r] : P[a][r], T[a][r]);
+                            else if constexpr (W::kMin && CENTER) T[a][r] = fmaf(offset_unit, fmaf(per_unit, P[a][r], M[a][r]), T[a][r]);
+                            else if constexpr (W::kMin) T[a][r] = fmaf(dmin, M[a][r], fmaf(d, P[a][r], T[a][r]));
+                            else T[a][r] = fmaf(d, P[a][r], T[a][r]);
                             if constexpr (kUnit && t + 1 == W::kSteps) T[a][r] += U[a][r];
                         }
                         if constexpr (kUnit) asm volatile("" : "+v"(U[a]));
                         else asm volatile("" : "+v"(T[a]));
-                    }
-                    if constexpr (W::kMin) {
-                        const half8 mo = w.min_operand(0);
-                        const float dmin = w.min_scale(0);
-#pragma unroll
-                        for (int a = 0; a < FM; a++) {
-                            const float16v M = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf[a], mo, zero16, 0, 0, 0);
-#pragma unroll
-                            for (int r = 0; r < 16; r++) T[a][r] = fmaf(dmin, M[r], T[a][r]);
-                            asm volatile("" : "+v"(T[a]));
-                        }
                     }
                 }
             }
@@ -238,9 +243,9 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
     }
 }
 
-template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO>
+template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER>
 hipError_t run_shared(const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units, int shares, hipStream_t s) {
-    using W = WeightsOf<ENC, 1, FLUSH, false>;
+    using W = WeightsOf<ENC, 1, FLUSH, CENTER>;
     constexpr int kBuf = FM * 8 * 1024;
     constexpr int lds = WK * kLhsBuffers * kBuf + WN * WK * W::kStage + 32 * FM * 4;
     static_assert(WK == 1 || WN * FM * 4096 <= lds - 32 * FM * 4, "the partial results fit in front of the row scales");
@@ -248,18 +253,18 @@ hipError_t run_shared(const WeightTensors& wt, DirectMats mats, const DirectSpac
     const int tiles_m = (int)((m + 32 * FM - 1) / (32 * FM));
     int eights = 0;
     for (int j = 0; j < mats.count; j++) mats.end[j] = eights += (mats.n[j] + 256 * WN - 1) / (256 * WN);
-    hipError_t e = allow_full_lds<gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO>>();
+    hipError_t e = allow_full_lds<gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER>>();
     if (e != hipSuccess) return e;
-    gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO><<<dim3((unsigned)(8 * eights * tiles_m * shares)), dim3(64 * WN * WK), lds, s>>>(wt, mats, p, out16, (int)m, units,
+    gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER><<<dim3((unsigned)(8 * eights * tiles_m * shares)), dim3(64 * WN * WK), lds, s>>>(wt, mats, p, out16, (int)m, units,
                                                                                                                        tiles_m, shares);
     return hipGetLastError();
 }
 
-template <int ENC, int FLUSH, bool HILO>
+template <int ENC, int FLUSH, bool HILO, bool CENTER = false>
 hipError_t run_shared_plan(const DirectPlan& pl, const WeightTensors& wt, const DirectMats& mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units,
                            hipStream_t s) {
 #define QMM_GS(FM, WN, WK) \
-    if (pl.fm == FM && pl.wn == WN && pl.wk == WK) return run_shared<ENC, FLUSH, FM, WN, WK, HILO>(wt, mats, p, out16, m, units, pl.shares, s)
+    if (pl.fm == FM && pl.wn == WN && pl.wk == WK) return run_shared<ENC, FLUSH, FM, WN, WK, HILO, CENTER>(wt, mats, p, out16, m, units, pl.shares, s)
     QMM_GS(2, 8, 1);
     QMM_GS(2, 4, 2);
     QMM_GS(2, 4, 1);
@@ -271,18 +276,31 @@ hipError_t run_shared_plan(const DirectPlan& pl, const WeightTensors& wt, const 
 
 hipError_t launch_gemm_shared(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
                               int64_t m, int units, hipStream_t s) {
-#define QMM_GS_ENC(ENC, FLUSH) \
-    return hilo ? run_shared_plan<ENC, FLUSH, true>(pl, wt, mats, p, out16, m, units, s) : run_shared_plan<ENC, FLUSH, false>(pl, wt, mats, p, out16, m, units, s)
+    const bool few = m <= kFewSharedRows;
+#define QMM_GS_RUN(...) return run_shared_plan<__VA_ARGS__>(pl, wt, mats, p, out16, m, units, s)
+#define QMM_GS_ENC(ENC, FLUSH)                \
+    do {                                      \
+        if (hilo) QMM_GS_RUN(ENC, FLUSH, true); \
+        QMM_GS_RUN(ENC, FLUSH, false);        \
+    } while (0)
     switch (encoding) {
-        case QMM_Q4_0: return run_shared_plan<QMM_Q4_0, 2, false>(pl, wt, mats, p, out16, m, units, s);
-        case QMM_Q4_K: QMM_GS_ENC(QMM_Q4_K, 16);
-        case QMM_Q5_K: QMM_GS_ENC(QMM_Q5_K, 16);
-        case QMM_Q6_K: QMM_GS_ENC(QMM_Q6_K, 16);
+        case QMM_Q4_0: QMM_GS_RUN(QMM_Q4_0, 2, false);
+        case QMM_Q4_K:
+            if (hilo) QMM_GS_RUN(QMM_Q4_K, 16, true, true);
+            QMM_GS_RUN(QMM_Q4_K, 16, false);
+        case QMM_Q5_K:
+            if (hilo) QMM_GS_RUN(QMM_Q5_K, 16, true, true);
+            if (few) QMM_GS_RUN(QMM_Q5_K, 16, false, true);
+            QMM_GS_RUN(QMM_Q5_K, 16, false);
+        case QMM_Q6_K:
+            if (few) QMM_GS_ENC(QMM_Q6_K, 8);
+            QMM_GS_ENC(QMM_Q6_K, 16);
         case QMM_GPTQ:
             if (wt.group % 128 == 0) QMM_GS_ENC(QMM_GPTQ, 8);
             QMM_GS_ENC(QMM_GPTQ, 2);
         default: return hipErrorInvalidValue;
     }
+#undef QMM_GS_RUN
 #undef QMM_GS_ENC
 }
 

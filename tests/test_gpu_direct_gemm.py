@@ -165,6 +165,12 @@ PRECISION = [
     ("Q5_K", 0, "f32", 33, 4096, 4096, 1.95e-7),   # 1.75e-7 (3.3e-7)
     ("Q5_K", 0, "bf16", 4, 6400, 1024, 1.0e-7),    # 0.9e-7 (2.2e-7)
     ("Q5_K", 0, "f32", 3, 2056, 1280, 1.9e-7),     # 1.65e-7 (2.8e-7)
+    ("Q4_K", 0, "f32", 200, 11008, 4096, 2.05e-7),  # 1.85e-7 (3.3e-7)
+    ("Q5_K", 0, "f32", 100, 14336, 4096, 2.1e-7),   # 1.9e-7 (3.4e-7)
+    ("Q5_K", 0, "bf16", 64, 20000, 4096, 1.1e-7),   # 1.0e-7 (2.35e-7)
+    ("Q5_K", 0, "f32", 64, 20000, 4096, 1.95e-7),   # 1.77e-7 (3.4e-7)
+    ("Q6_K", 0, "bf16", 64, 20000, 4096, 1.07e-7),  # 0.95e-7 (1.2e-7)
+    ("Q6_K", 0, "f32", 64, 8192, 8192, 1.82e-7),    # 1.65e-7 (2.1e-7)
     ("Q6_K", 0, "bf16", 17, 4096, 4096, 1.07e-7),  # 0.97e-7 (1.17e-7)
     ("Q6_K", 0, "bf16", 33, 11008, 4096, 1.07e-7),  # 0.96e-7 (1.12e-7)
     ("Q6_K", 0, "f32", 9, 4096, 4096, 1.8e-7),     # 1.6e-7 (2.1e-7)
@@ -192,3 +198,28 @@ def test_precision(enc, group, lhs, m, n, k, limit):
     want = x @ dequantize(enc, *rhs, config=config).double().T
     error = ((qmatmul(enc, config, a, *rhs).double() - want).norm() / want.norm()).item()
     assert error <= limit, (enc, lhs, m, n, k, error)
+
+
+@pytest.mark.parametrize("enc", ["Q4_K", "Q5_K"])
+@pytest.mark.parametrize("lhs", ["bf16", "f32"])
+@pytest.mark.parametrize("m,n", [(40, 6200), (64, 20000), (200, 6200)])
+def test_scales_of_any_size(enc, lhs, m, n):
+    """The offsets of the sub-blocks are two fp16 terms in units of a power of two that suits the larger of the block's two scales: any pair of them, zeros
+    and negative ones among them."""
+    enc, k = QE[enc], 512
+    gen = torch.Generator(device="cuda").manual_seed(n + m)
+    w = quantize(enc, torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen))
+    scales = w.view(n, k // 256, -1)[:, :, :4].contiguous().view(torch.float16)
+    kinds = torch.tensor([0.0, 2.0**-24, -3 * 2.0**-20, 0.02, -1.0, 700.0, -1000.0], device="cuda").half()
+    scales.copy_(kinds[torch.randint(len(kinds), scales.shape, device="cuda", generator=gen)])
+    w.view(n, k // 256, -1)[:, :, :4] = scales.view(torch.uint8).view(n, k // 256, 4)
+    a = torch.randn((m, k), device="cuda", generator=gen).to(torch.float32 if lhs == "f32" else torch.bfloat16)
+    out, x = qmatmul(enc, None, a, w).double(), a.double()
+    # d sc q and dmin mn apart: with the other scale zero
+    no_min, no_d = w.clone(), w.clone()
+    no_min.view(n, k // 256, -1)[:, :, 2:4] = 0
+    no_d.view(n, k // 256, -1)[:, :, :2] = 0
+    parts = [dequantize(enc, t).double() for t in (no_min, no_d)]
+    size = x.abs() @ (parts[0].abs() + parts[1].abs()).T
+    # 32 roundings of a chain and 22 bits of an operand, all in one direction; the mean of the codes (half their range) doubles what the sums hold
+    assert ((out - x @ (parts[0] + parts[1]).T).abs() <= 2.0**-24 * 2 * (32 + 4) * size).all()
