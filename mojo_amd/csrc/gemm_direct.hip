@@ -447,27 +447,34 @@ namespace {
 
 int64_t direct_units(int64_t k) { return (k + 255) / 256; }
 
-// What a call takes, in microseconds: launches and the preparation of the lhs, a fixed part per round of workgroups (eight wavefronts fill
-// a compute unit, four half of it; counted on the XCD with the most, column tiles go to XCDs in eights), the units of K that a wavefront walks, terms for the weights, the lhs and the results, and one for lhs operands
-// beyond 8 MB, which an XCD's L2 does not keep for the next column tile.  Fitted to the problems among 186 per encoding and lhs type (512 x 512 ..
-// 28672 x 4096, K up to 14336, 4 .. 1300 rows, weights from memory; profiles/direct_and_shared_gemm__plans.txt) that these kernels serve, in every plan:
-// 8 .. 13 % off; what it picks takes 1 .. 3 % longer on average than the best plan.
+// What a call takes, in microseconds: launches and the preparation of the lhs, a fixed part per round of workgroups (Rounds), the units of K that a wavefront
+// walks, terms for the weights, the lhs and the results, and one for lhs operands beyond 8 MB, which an XCD's L2 does not keep for the next column tile.
+// Fitted to the problems among 205 per encoding and lhs type (512 x 512 .. 28672 x 8192, K up to 14336, 4 .. 1300 rows, weights from memory;
+// profiles/direct_and_shared_gemm__plans.txt) that these kernels serve, in every plan: 7 .. 10 % off; what it picks takes 0.6 .. 1.8 % longer on average than
+// the best plan (3 % for GPTQ with bf16 rows).
 // unit = 0: a plan that is not built (two fragments side by side spill registers and never win with Q4_0 and Q6_K).
 struct DirectCost {
     float base, round, weights, lhs, out;  // us, us, us per MB of packed weights, us per million lhs values, us per million results and share
     float unit[6];                         // us per unit of K: the plans of kDirectPlans
+    float alone[3];                        // the same of the last three with a compute unit to themselves
     float far;                             // us per 10^9 lhs operands read, where they are more than 8 MB
 };
 constexpr DirectPlan kDirectPlans[6] = {{1, 1, 8, 0, 1}, {2, 1, 8, 0, 1}, {1, 2, 8, 0, 1}, {1, 1, 4, 0, 1}, {2, 1, 4, 0, 1}, {1, 2, 4, 0, 1}};
 constexpr bool direct_built(int encoding, int fn) { return !(fn == 2 && (encoding == QMM_Q4_0 || encoding == QMM_Q6_K)); }
 constexpr DirectCost kDirectCost[6][2] = {
     // bf16 lhs; fp32 lhs
-    {{3.57f, 1.17f, 0.202f, 2.86f, 3.35f, {2.81f, 3.96f, 0.0f, 2.19f, 3.06f, 0.0f}, 9.94f}, {3.56f, 1.19f, 0.206f, 3.01f, 3.1f, {2.8f, 3.96f, 0.0f, 2.19f, 3.04f, 0.0f}, 9.73f}},  // Q4_0
-    {{4.26f, 0.777f, 0.219f, 3.03f, 3.12f, {2.54f, 3.39f, 3.79f, 1.84f, 2.34f, 2.58f}, 0.0f}, {4.03f, 0.554f, 0.237f, 4.49f, 4.56f, {3.3f, 4.81f, 4.7f, 2.42f, 3.44f, 3.22f}, 31.7f}},  // Q4_K
-    {{4.23f, 0.756f, 0.193f, 2.76f, 3.42f, {3.01f, 3.81f, 4.67f, 2.18f, 2.65f, 3.23f}, 11.5f}, {3.9f, 0.701f, 0.227f, 4.3f, 4.66f, {3.62f, 5.03f, 5.32f, 2.62f, 3.54f, 3.62f}, 33.4f}},  // Q5_K
-    {{3.54f, 1.19f, 0.191f, 2.62f, 3.77f, {3.66f, 4.44f, 0.0f, 2.58f, 3.21f, 0.0f}, 30.9f}, {3.32f, 0.869f, 0.248f, 3.87f, 5.83f, {4.57f, 6.02f, 0.0f, 3.22f, 4.3f, 0.0f}, 50.3f}},  // Q6_K
-    {{4.89f, 0.0f, 0.192f, 2.73f, 3.26f, {2.45f, 3.52f, 3.5f, 1.81f, 2.82f, 2.72f}, 0.0f}, {3.84f, 0.662f, 0.233f, 4.38f, 4.6f, {3.65f, 4.74f, 4.33f, 2.73f, 3.76f, 3.44f}, 23.0f}},  // GPTQ, groups of 128
-    {{4.12f, 0.832f, 0.179f, 2.44f, 3.4f, {3.31f, 4.33f, 4.55f, 2.55f, 3.43f, 3.63f}, 12.7f}, {4.05f, 0.483f, 0.221f, 4.17f, 4.64f, {4.22f, 5.57f, 5.39f, 3.17f, 4.22f, 4.03f}, 23.5f}},  // GPTQ, other groups
+    {{3.56f, 1.4f, 0.179f, 2.88f, 2.57f, {2.79f, 4.04f, 0.0f, 2.31f, 3.43f, 0.0f}, {2.12f, 2.91f, 0.0f}, 7.01f},
+     {3.51f, 1.45f, 0.182f, 3.09f, 2.33f, {2.76f, 4.02f, 0.0f, 2.3f, 3.45f, 0.0f}, {2.1f, 2.89f, 0.0f}, 5.8f}},  // Q4_0
+    {{4.18f, 1.15f, 0.185f, 2.87f, 2.04f, {2.51f, 3.44f, 3.82f, 2.07f, 3.02f, 3.09f}, {1.72f, 2.19f, 2.57f}, 0.0f},
+     {3.74f, 1.12f, 0.184f, 4.61f, 2.31f, {3.39f, 5.19f, 5.03f, 3.09f, 5.05f, 4.46f}, {2.27f, 3.03f, 3.07f}, 20.1f}},  // Q4_K
+    {{4.18f, 1.18f, 0.159f, 2.82f, 1.94f, {2.96f, 3.89f, 4.73f, 2.42f, 3.37f, 3.99f}, {1.94f, 2.42f, 3.07f}, 0.0f},
+     {3.59f, 1.37f, 0.165f, 4.42f, 2.03f, {3.74f, 5.54f, 5.74f, 3.36f, 5.45f, 5.27f}, {2.44f, 3.12f, 3.47f}, 18.7f}},  // Q5_K
+    {{3.49f, 1.75f, 0.158f, 2.66f, 1.36f, {3.69f, 4.77f, 0.0f, 3.14f, 4.4f, 0.0f}, {2.27f, 2.89f, 0.0f}, 11.0f},
+     {2.94f, 1.78f, 0.172f, 4.48f, 1.46f, {4.9f, 7.0f, 0.0f, 4.4f, 7.37f, 0.0f}, {2.97f, 3.91f, 0.0f}, 20.8f}},  // Q6_K
+    {{4.94f, 0.0025f, 0.169f, 2.65f, 3.11f, {2.5f, 3.62f, 3.56f, 1.87f, 3.17f, 2.71f}, {1.82f, 2.7f, 2.81f}, 0.0f},
+     {3.74f, 1.04f, 0.178f, 4.44f, 2.88f, {3.78f, 5.21f, 4.6f, 3.27f, 5.09f, 4.22f}, {2.55f, 3.41f, 3.4f}, 15.2f}},  // GPTQ, groups of 128
+    {{4.02f, 1.17f, 0.157f, 2.49f, 2.39f, {3.3f, 4.46f, 4.6f, 2.77f, 3.92f, 4.02f}, {2.36f, 3.22f, 3.52f}, 6.54f},
+     {3.77f, 1.05f, 0.175f, 4.28f, 2.75f, {4.3f, 5.96f, 5.6f, 3.67f, 5.65f, 4.97f}, {3.01f, 3.8f, 3.92f}, 15.3f}},  // GPTQ, other groups
 };
 constexpr bool direct_costs_match_what_is_built() {
     for (int row = 0; row < 6; row++)
@@ -479,16 +486,26 @@ constexpr bool direct_costs_match_what_is_built() {
     return true;
 }
 static_assert(direct_costs_match_what_is_built());
+// The rounds of a grid of wgs workgroups per XCD (column tiles go to XCDs in eights).  Two workgroups of four wavefronts fit a compute unit; an odd
+// last one has it to itself and is done sooner.
+struct Rounds {
+    int64_t all, full, alone;
+};
+Rounds rounds_of(int64_t wgs, bool pairs) {
+    const int64_t cus = compute_units() / 8, deep = (wgs + cus - 1) / cus;
+    return pairs ? Rounds{(deep + 1) / 2, deep / 2, deep % 2} : Rounds{deep, deep, 0};
+}
 double direct_us(const DirectCost& c, int plan, int shares, int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const DirectPlan& p = kDirectPlans[plan];
     if (c.unit[plan] == 0.0f) return 1e30;
-    const int64_t wgs = ((m + 32 * p.fm - 1) / (32 * p.fm)) * ((n + 256 * p.fn - 1) / (256 * p.fn)) * shares;
-    const int64_t slots = compute_units() / 8 * (p.wk == 8 ? 1 : 2), rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
+    const int64_t wgs = ((m + 32 * p.fm - 1) / (32 * p.fm)) * ((n + 256 * p.fn - 1) / (256 * p.fn)) * shares, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
+    const Rounds r = rounds_of(wgs, p.wk == 4);
     const double bytes = encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56, per = lhs_dtype == QMM_F32 && encoding != QMM_Q4_0 ? 2 : 1;
     const double far = 2 * m * k * per > 8e6 ? c.far * (m * k * per * 1e-9) * n / (32 * p.fn) : 0.0;
-    return c.base + rounds * (c.round + walk * c.unit[plan]) + c.weights * (bytes * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares + far;
+    return c.base + r.all * c.round + walk * (r.full * c.unit[plan] + r.alone * c.alone[plan % 3]) + c.weights * (bytes * n * k * 1e-6) + c.lhs * (m * k * 1e-6) +
+           c.out * (m * n * 1e-6) * shares + far;
 }
-// The same for the kernel whose wavefronts share the lhs, fitted to the same problems from 33 rows on: 5 .. 8 % off.  It wins where its tiles of 64 x 256
+// The same for the kernel whose wavefronts share the lhs, fitted to the same problems from 33 rows on: 5 .. 6 % off.  It wins where its tiles of 64 x 256
 // (64 x 128) fill the part with most of K in a workgroup.  us, direct plans / shared: Q4_K, bf16 rows: 14336 x 4096 200 rows 59 / 49; fp32 rows:
 // 14336 x 4096 500 rows 183 / 150; Q6_K 4096 x 14336 500 bf16 rows 153 / 134; but 4096 x 4096 Q4_K 64 bf16 rows 12 / 18.
 struct SharedCost {
@@ -498,19 +515,19 @@ struct SharedCost {
 constexpr DirectPlan kSharedPlans[3] = {{2, 1, 1, 0, 8}, {2, 1, 2, 0, 4}, {2, 1, 1, 0, 4}};
 constexpr SharedCost kSharedCost[6][2] = {
     // bf16 lhs; fp32 lhs
-    {{5.04f, 0.664f, 0.1f, 1.55f, 2.64f, {3.75f, 4.03f, 3.26f}, 2.91f}, {5.17f, 0.534f, 0.105f, 1.67f, 2.58f, {3.74f, 4.02f, 3.24f}, 2.9f}},  // Q4_0
-    {{4.84f, 1.74f, 0.0796f, 1.43f, 2.58f, {2.28f, 2.52f, 2.19f}, 1.85f}, {4.98f, 1.46f, 0.0729f, 2.32f, 3.17f, {3.54f, 4.09f, 3.55f}, 2.62f}},  // Q4_K
-    {{4.95f, 1.59f, 0.08f, 1.47f, 2.61f, {2.7f, 3.02f, 2.76f}, 2.12f}, {4.82f, 1.59f, 0.134f, 2.34f, 3.13f, {3.87f, 4.45f, 3.83f}, 2.81f}},  // Q5_K
-    {{4.91f, 1.37f, 0.109f, 1.73f, 2.69f, {3.85f, 4.21f, 3.64f}, 2.46f}, {3.76f, 1.92f, 0.123f, 2.17f, 3.47f, {5.85f, 6.55f, 5.9f}, 3.71f}},  // Q6_K
-    {{5.33f, 1.07f, 0.0461f, 1.6f, 2.63f, {2.41f, 2.58f, 2.1f}, 1.89f}, {5.98f, 0.298f, 0.0814f, 2.44f, 3.09f, {3.58f, 4.03f, 3.23f}, 2.92f}},  // GPTQ, groups of 128
-    {{6.09f, 0.507f, 0.078f, 1.6f, 2.66f, {3.47f, 3.79f, 3.1f}, 2.65f}, {6.03f, 0.46f, 0.073f, 2.37f, 3.06f, {4.52f, 5.0f, 4.27f}, 3.51f}},  // GPTQ, other groups
+    {{4.93f, 0.853f, 0.094f, 1.55f, 2.62f, {3.79f, 3.93f, 3.35f}, 2.85f}, {5.01f, 0.774f, 0.1f, 1.71f, 2.52f, {3.78f, 3.92f, 3.34f}, 2.84f}},  // Q4_0
+    {{4.58f, 1.97f, 0.0798f, 1.42f, 2.57f, {2.31f, 2.56f, 2.27f}, 1.78f}, {4.49f, 1.95f, 0.0749f, 2.15f, 3.19f, {3.62f, 4.15f, 3.81f}, 2.61f}},  // Q4_K
+    {{4.57f, 2.11f, 0.106f, 1.38f, 2.41f, {2.72f, 3.02f, 2.78f}, 2.08f}, {3.94f, 2.46f, 0.114f, 2.06f, 3.12f, {3.97f, 4.53f, 4.17f}, 2.83f}},  // Q5_K
+    {{3.74f, 2.76f, 0.132f, 1.48f, 2.48f, {3.83f, 4.16f, 3.83f}, 2.45f}, {2.61f, 3.28f, 0.124f, 1.55f, 3.33f, {5.87f, 6.55f, 6.39f}, 3.72f}},  // Q6_K
+    {{5.18f, 1.29f, 0.0415f, 1.6f, 2.58f, {2.41f, 2.58f, 2.22f}, 1.87f}, {5.93f, 0.433f, 0.0638f, 2.43f, 2.93f, {3.62f, 4.06f, 3.5f}, 2.85f}},  // GPTQ, groups of 128
+    {{5.89f, 0.703f, 0.0642f, 1.57f, 2.6f, {3.54f, 3.82f, 3.28f}, 2.64f}, {5.71f, 0.809f, 0.0638f, 2.23f, 2.96f, {4.56f, 5.04f, 4.56f}, 3.49f}},  // GPTQ, other groups
 };
 double shared_us(const SharedCost& c, int plan, int shares, int64_t m, int64_t n, int64_t k) {
     const DirectPlan& p = kSharedPlans[plan];
-    const int64_t wgs = ((m + 63) / 64) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, cus = compute_units() / 8, slots = cus * (p.wn * p.wk == 8 ? 1 : 2);
-    const int64_t rounds = (wgs + slots - 1) / slots, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
-    const double unit = slots > cus && wgs <= cus ? c.unit_alone : c.unit[plan];
-    return c.base + rounds * (c.round + walk * unit) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) + c.out * (m * n * 1e-6) * shares;
+    const int64_t wgs = (m + 63) / 64 * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, walk = (direct_units(k) + p.wk * shares - 1) / (p.wk * shares);
+    const Rounds r = rounds_of(wgs, p.wn * p.wk == 4);
+    return c.base + r.all * c.round + walk * (r.full * c.unit[plan] + r.alone * c.unit_alone) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) +
+           c.out * (m * n * 1e-6) * shares;
 }
 // whole_tiles: one workgroup per tile (bf16 results are stored, not added up); like: with that plan's cut of K
 DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, const DirectPlan* like = nullptr) {
@@ -532,9 +549,9 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
         for (int i = 0; i < 6; i++)
             if (direct_units(k) <= longest * kDirectPlans[i].wk * shares)
                 consider(kDirectPlans[i], shares, direct_us(kDirectCost[row][type], i, shares, encoding, lhs_dtype, m, n, k));
-        for (int i = 0; shared && i < 3; i++)  // (between predictions this close these took 3 % less, except GPTQ, and workgroups of four wavefronts 3 % longer)
+        for (int i = 0; shared && i < 3; i++)  // (between predictions this close workgroups of four wavefronts took 3 % longer)
             if (direct_units(k) <= longest * kSharedPlans[i].wk * shares)
-                consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (encoding == QMM_GPTQ ? 1.0 : 0.97) * (i == 2 ? 1.03 : 1.0));
+                consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (i == 2 ? 1.03 : 1.0));
     }
     return best;
 }
