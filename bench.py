@@ -57,7 +57,7 @@ class Gemv:
         self.n = w.shape[0]
         self.out = torch.empty((self.m, self.n), dtype=torch.float32, device=a.device)
         dt = _lib.QMM_F32 if a.dtype == torch.float32 else _lib.QMM_BF16
-        need = self.lib.qmm_matmul_workspace_bytes(enc.code, dt, self.m, self.n, self.k)
+        need = self.lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, enc.code, None, dt, self.m, self.n, self.k, flags)  # (as qmatmul)
         self.ws = torch.empty((max(need, 1),), dtype=torch.uint8, device=a.device)
         self.need = need
         self.dt = dt
@@ -141,9 +141,9 @@ class GptqMatmul:
         self.n = tensors[0].shape[1]
         self.out = torch.empty((self.m, self.n), dtype=torch.float32, device=a.device)
         self.dt = _lib.QMM_F32 if a.dtype == torch.float32 else _lib.QMM_BF16
-        self.need = self.lib.qmm_matmul_workspace_bytes(QE.GPTQ.code, self.dt, self.m, self.n, self.k)
-        self.ws = torch.empty((max(self.need, 1),), dtype=torch.uint8, device=a.device)
         self.cfg = _lib.GptqConfig(4, group, 0 if g_idx is None else 1, 1)  # g_idx given: an act-order checkpoint
+        self.need = self.lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, C.byref(self.cfg), self.dt, self.m, self.n, self.k, 0)
+        self.ws = torch.empty((max(self.need, 1),), dtype=torch.uint8, device=a.device)
         ptrs = [t.data_ptr() for t in tensors[:3]] + ([] if g_idx is None else [g_idx.data_ptr()])
         self.ptrs = (C.c_void_p * len(ptrs))(*ptrs)
 

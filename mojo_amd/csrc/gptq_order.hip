@@ -2,10 +2,10 @@
 // groups serve the call.
 //
 // The kernel that looks the group of every k up (gemv_gptq.hip) passes over the weights once per four rows and multiplies on the vector
-// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, now 103 us.  Sorting costs one small launch and one pass over the packed weights: the words of
+// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 103 us.  Sorting costs one small launch and one pass over the packed weights: the words of
 // some columns of the output lie in LDS (all of K), from which every word of the sorted matrix takes its eight nibbles; other workgroups
-// of that launch sort the columns of the lhs.  What bounds the pass is reading and writing the packed weights (2 x 29 MB at 14336 x 4096: 16.4 us with 400 rows of
-// lhs, 4.0 TB/s; the sort, one workgroup, 5.6).
+// of that launch sort the columns of the lhs.  What bounds the pass is reading and writing the packed weights (2 x 29 MB at 14336 x 4096: 17 us with 400 rows of
+// lhs, 3.8 TB/s; the sort, one workgroup, 6; profiles/direct_gemm_act_order_quantisers__kernel_trace.txt).
 //
 // A sorted column list is a plain-group matrix only if every group has exactly group_size columns, which is so in any checkpoint that was
 // quantised group by group.  The device finds out: where it is not so, the sort leaves a mark, the order as it was (the products are then
