@@ -617,7 +617,9 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
             from = wide && k <= 2048 ? 2 : n >= 2048 && (k % 512 || w <= (f32 ? 16 : 24)) ? 3 : w <= 32 && (f32 || k <= 8192 || k % 512) ? 5 : f32 ? 9 : 17;
             break;
         case QMM_Q6_K:
-            if (f32) from = k % 2048 == 0 ? 9 : wide ? 3 : n >= 2048 ? 4 : 6;
+            // (fp32 rows with K = 4096, one round of the small-batch kernel, on a vocabulary's columns: 9 .. 16 rows on 128256 x 4096 216 / 151 us, 40960 x 4096
+            // 71 / 66, but 32000 x 4096 58 / 60, 128256 x 2048 110 / 165, 65536 x 8192 209 / 238)
+            if (f32) from = k % 2048 == 0 ? (k == 4096 && n > 36000 ? 17 : 9) : wide ? 3 : n >= 2048 ? 4 : 6;
             else from = k % 2048 == 0 && !(wide && k <= 2048) ? (w <= 30 && k <= 8192 ? 5 : 17) : wide ? 2 : n >= 2048 ? 3 : 6;
             most = 3.5, anyway = 450;
             break;
