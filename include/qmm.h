@@ -142,8 +142,9 @@ int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_confi
  *   encoding Q4_0/Q4_K/Q6_K: n_rhs = 1, rhs[0] = uint8[n, k/epb*bpb];
  *   encoding GPTQ: cfg required, n_rhs = 3 or 4,
  *     rhs = {qweight i32[k/8, n], scales f16[k/g, n], qzeros i32[k/g, n/8], g_idx i32[k]}.
- *     cfg->desc_act = 1 (n_rhs = 4) goes through a decode-shaped kernel for every m, four lhs rows per
- *     pass over the weights; the matrix-core kernel takes plain groups only.
+ *     cfg->desc_act = 1 (n_rhs = 4): a few rows go through a decode-shaped kernel, four lhs rows per pass over
+ *     the weights; more, with a workspace of qmm_preferred_workspace_bytes, through the plain-group kernels on
+ *     columns that the call sorts by group.
  *   lhs_dtype QMM_F32 or QMM_BF16.  Q4_0 quantises lhs rows to Q8_0 and takes
  *   integer block dots (the reference CPU path); the others keep lhs as given.
  *   flags: bit 0 (QMM_FLAG_W_BF16) is reserved for a mode that rounds the dequantised
