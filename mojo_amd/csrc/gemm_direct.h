@@ -114,8 +114,8 @@ struct StagedRows {
 // sums of the lhs.  Codes that are all positive make sums 2.4 times as large as what the minima leave of them, and the error of a sum of the lhs counts
 // fifteenfold.  Relative error without and with it, direct kernel (decode kernel): Q4_K 4096 x 4096 17 bf16 rows 1.9e-7, 0.9e-7 (0.9e-7), fp32 3.1e-7,
 // 1.7e-7 (2.6e-7); Q5_K 2.2e-7, 1.0e-7 (1.0e-7), 3.2e-7, 1.7e-7 (2.4e-7).
-// - direct kernel: always, the sums in fp32 (four matrix-core instructions of their own, onto the running sums); the time is the same with bf16 rows and 2 .. 6 %
-//   less with fp32 rows, whose residual would need sums of its own otherwise.
+// - direct kernel: always, the sums in fp32 (four matrix-core instructions of their own, onto the running sums); bf16 rows take 0 .. 5 % longer
+//   (weights from memory; 14336 x 4096 17 rows 19.1 -> 19.9 us), fp32 rows, whose residual would need sums of its own otherwise, 2 .. 6 % less.
 // - shared kernel, whose matrix cores are busier: both the offsets and the sums as two fp16 terms (two instructions a unit; the offsets exact to 22 bits of the
 //   larger product).  fp32 rows 3.4e-7 -> 1.85e-7 in the same time.  bf16 rows 2.3e-7 -> 1.1e-7, but 3 .. 4 % slower, its vector units being the limit: only Q5_K up
 //   to 64 rows, where the small-batch kernel has 1.6e-7; beyond, the GEMMs that it replaces have 2.6e-7 and more.
