@@ -35,13 +35,19 @@ struct WeightTensors {
 };
 
 // How a call is cut: every wavefront takes 32 fm rows x 32 fn columns.  wn = 1: the wk wavefronts of a workgroup take wk parts of K of one tile
-// (gemm_direct.hip).  wn > 1: wn wavefronts side by side share the lhs, wk parts of K (gemm_shared.hip).  shares: workgroups per tile (1, or 2 that
-// add onto zeros).
+// (gemm_direct.hip).  wn > 1: wn wavefronts side by side share the lhs, wk parts of K (gemm_shared.hip, and with fn = 0, which means one, gemm_staged.hip).  shares:
+// workgroups per tile (1, or 2 that add onto zeros).  centred: gemm_staged.hip, codes of Q4_K and Q5_K around their middle.
 struct DirectPlan {
     int fm, fn, wk, shares, wn;
+    bool centred = false;
 };
 hipError_t launch_gemm_shared(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
                               int64_t m, int units, hipStream_t s);
+hipError_t launch_gemm_staged(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
+                              int64_t m, int units, hipStream_t s);
+
+// What gemm_staged.hip has: fp32 rows and small groups leave no registers for 128 rows a wavefront.
+constexpr bool staged_built(int encoding, int flush, int fm, bool hilo) { return fm <= 3 || !(hilo || (encoding == QMM_GPTQ && flush == 2)); }
 
 namespace {
 
@@ -147,6 +153,9 @@ struct KQuantWeights {
     // the loaded unit becomes the current one
     __device__ __forceinline__ void open() {
         rows.to_lds(lane_);
+        read_head();
+    }
+    __device__ __forceinline__ void read_head() {
         read_codes(0);
 #pragma unroll
         for (int f = 0; f < FN; f++) {

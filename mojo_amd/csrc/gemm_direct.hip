@@ -529,8 +529,77 @@ double shared_us(const SharedCost& c, int plan, int shares, int64_t m, int64_t n
     return c.base + r.all * c.round + walk * (r.full * c.unit[plan] + r.alone * c.unit_alone) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) +
            c.out * (m * n * 1e-6) * shares;
 }
-// whole_tiles: one workgroup per tile (bf16 results are stored, not added up); like: with that plan's cut of K
-DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, const DirectPlan* like = nullptr) {
+// The same for the kernel whose lhs and weights go to LDS by themselves (gemm_staged.hip), fitted to 326 problems per encoding and lhs type (512 x 512 .. 28672 x
+// 8192, K up to 18944, 24 .. 4096 rows, weights from memory): 3 .. 4 % off, what it picks takes 0.2 % longer on average than its best plan.
+// other: what the GEMMs behind this file (planes, tiles) take, from 200 rows on, in us: a fixed part, per MB of weights, per million lhs values, per million
+// results, per 10^9 products with the rows in 256s (6 .. 10 % off; none for groups that are no multiple of 128, which have no such GEMM).
+struct StagedCost {
+    float base, round, weights, lhs, out, share;
+    float unit[7];  // the plans of kStagedPlans; 0: not built
+    float other[5];
+};
+constexpr DirectPlan kStagedPlans[7] = {{2, 0, 4, 0, 2}, {2, 0, 2, 0, 4}, {2, 0, 1, 0, 8}, {3, 0, 2, 0, 4}, {3, 0, 1, 0, 8}, {4, 0, 2, 0, 4}, {4, 0, 1, 0, 8}};
+constexpr StagedCost kStagedCost[5][2] = {
+    // bf16 lhs; fp32 lhs
+    {{4.97f, 2.08f, 0.0626f, 1.61f, 1.88f, 4.7f, {2.78f, 2.04f, 1.83f, 2.75f, 2.31f, 3.41f, 2.88f}, {16.1f, 0.147f, 1.61f, 0.0f, 2.11f}},
+     {3.99f, 2.7f, 0.088f, 2.97f, 2.61f, 4.77f, {4.74f, 3.32f, 2.98f, 4.73f, 3.94f, 0.0f, 0.0f}, {16.3f, 4.73f, 3.8f, 4.79f, 2.69f}}},  // Q4_K
+    {{5.06f, 2.12f, 0.0665f, 1.39f, 1.74f, 4.71f, {3.27f, 2.61f, 2.23f, 3.12f, 2.69f, 4.08f, 3.4f}, {14.7f, 1.05f, 2.44f, 0.107f, 1.61f}},
+     {3.65f, 3.15f, 0.0849f, 2.75f, 2.55f, 4.65f, {4.94f, 3.96f, 3.3f, 5.02f, 4.28f, 0.0f, 0.0f}, {25.6f, 3.16f, 4.81f, 3.69f, 2.82f}}},  // Q5_K
+    {{3.93f, 3.1f, 0.0983f, 1.55f, 2.23f, 4.61f, {4.2f, 3.56f, 3.19f, 4.28f, 3.82f, 5.69f, 5.04f}, {13.2f, 1.45f, 2.3f, 0.0f, 2.77f}},
+     {2.13f, 4.38f, 0.141f, 3.05f, 3.48f, 4.43f, {6.53f, 5.51f, 4.88f, 7.3f, 6.59f, 0.0f, 0.0f}, {23.6f, 2.72f, 5.61f, 3.47f, 5.44f}}},  // Q6_K
+    {{5.21f, 2.55f, 0.0331f, 1.43f, 1.55f, 4.57f, {2.45f, 1.9f, 1.77f, 2.53f, 2.21f, 3.15f, 2.72f}, {14.9f, 0.0609f, 1.56f, 0.0f, 1.88f}},
+     {4.51f, 2.82f, 0.0544f, 2.78f, 2.26f, 4.62f, {4.37f, 2.93f, 2.66f, 4.4f, 3.7f, 0.0f, 0.0f}, {9.65f, 1.9f, 3.89f, 4.38f, 3.13f}}},  // GPTQ, groups of 128
+    {{5.25f, 2.87f, 0.0408f, 1.41f, 1.22f, 4.49f, {3.16f, 2.72f, 2.65f, 3.77f, 3.43f, 0.0f, 0.0f}, {}},
+     {4.16f, 3.4f, 0.0772f, 2.7f, 2.3f, 4.44f, {4.61f, 3.56f, 3.39f, 4.98f, 4.46f, 0.0f, 0.0f}, {}}},  // GPTQ, other groups
+};
+int staged_row(int encoding, int group) {
+    return encoding == QMM_Q4_K ? 0 : encoding == QMM_Q5_K ? 1 : encoding == QMM_Q6_K ? 2 : encoding == QMM_GPTQ ? (group % 128 == 0 ? 3 : 4) : -1;
+}
+double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56) * n * k * 1e-6; }
+// The best of its plans whose parts of K are at most `longest` units; returns its time (1e30: there is none).
+double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, int64_t longest, DirectPlan& best) {
+    const int row = staged_row(encoding, group);
+    if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
+    const StagedCost& c = kStagedCost[row][lhs_dtype == QMM_F32 ? 1 : 0];
+    double us = 1e30;
+    for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++)
+        for (int i = 0; i < 7; i++) {
+            const DirectPlan& p = kStagedPlans[i];
+            const int64_t parts = p.wk * shares, walk = (direct_units(k) + parts - 1) / parts;
+            if (c.unit[i] == 0.0f || walk > longest) continue;
+            const int64_t rounds = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, false).all;
+            const double t = c.base + rounds * (c.round + walk * c.unit[i]) + c.weights * packed_mb(encoding, n, k) + c.lhs * (m * k * 1e-6) +
+                             (c.out + c.share * (shares - 1)) * (m * n * 1e-6);
+            if (t < us) us = t, best = p, best.shares = shares;
+        }
+    return us;
+}
+// Calls that go to this file for the sake of the direct and the shared kernel: up to where the GEMMs that unpack a tile or all weights once and then share
+// them take over (r = outputs, w = weights, in Mi; beyond about 1100 rows the lhs no longer stays in an L2).
+bool direct_range(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
+    if (encoding == QMM_GPTQ && group % 128) return true;  // (the alternative is the decode kernel, eight rows a pass)
+    const bool f32 = lhs_dtype == QMM_F32, few_products = encoding == QMM_Q4_0 || encoding == QMM_Q6_K;
+    const double w = (double)n * k / (1 << 20), r = (double)m * n / (1 << 20);
+    const double most = few_products ? 3.5 : k > 4096 && (encoding == QMM_Q4_K || encoding == QMM_GPTQ) ? 1.3 : 2.75;  // bf16 outputs
+    const int64_t anyway = few_products ? 450 : 0;  // rows up to which the number of outputs does not matter
+    if (r <= (f32 && encoding != QMM_Q4_0 ? 1.6 : 1)) return true;
+    // fp32 rows are split in two fp16 terms here and in the other kernels, so both multiply twice; the others take K in two passes.  us, others / here:
+    // Q4_K 14336 x 4096 800 rows 327 / 232, 5120 x 5120 1300 rows 239 / 198; Q6_K 14336 x 4096 800 rows 514 / 380;
+    // but GPTQ 4096 x 14336 1050 rows 470 / 560.
+    const bool shared = !kernel_disabled("shared");
+    if (f32) {
+        if (shared && encoding != QMM_Q4_0 && (m <= 1100 || (m <= 1400 && r <= 5.5)) && (encoding != QMM_GPTQ || k <= 8192)) return true;
+        return m <= (w <= 24 || (encoding != QMM_Q4_0 && encoding != QMM_GPTQ) ? 720 : 450) || (k <= 1024 ? r <= 6 : m < 1100 && r <= 3.5);
+    }
+    // (one round of 64 x 256 tiles that fills the compute units by four fifths or more: 11008 x 4096 320 bf16 rows Q4_K 78 / 55, GPTQ 71 / 53, Q5_K 85 / 63;
+    // 8192 x 8192 500 rows Q6_K 205 / 162, Q5_K 145 / 119, but Q4_K 106 / 105 and GPTQ 92 / 101)
+    const int64_t tiles = (m + 63) / 64 * ((n + 255) / 256);
+    if (shared && 5 * tiles >= 4 * compute_units() && tiles <= compute_units() && k <= (encoding == QMM_Q4_K || encoding == QMM_GPTQ ? 4096 : 8192)) return true;
+    return m <= anyway || (m <= 1100 && r <= most);
+}
+// whole_tiles: one workgroup per tile (bf16 results are stored, not added up); staged: the weights lie as the staged kernel wants them; beyond: the call
+// would not be this file's without that kernel (direct_range); like: with that plan's cut of K and kind of sums
+DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, bool staged, bool beyond, const DirectPlan* like = nullptr) {
     const int row = encoding == QMM_Q4_0 ? 0 : encoding == QMM_Q4_K ? 1 : encoding == QMM_Q5_K ? 2 : encoding == QMM_Q6_K ? 3 : group % 128 == 0 ? 4 : 5;
     const int type = lhs_dtype == QMM_F32 ? 1 : 0;
     DirectPlan best{1, 1, 8, 1, 1};
@@ -541,6 +610,17 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
         best = p;
         best.shares = shares;
     };
+    if (like && like->fn == 0) {  // (several matrices that all go to the staged kernel with this cut: the tile that suits them together)
+        for (const DirectPlan& p : kStagedPlans) {
+            const StagedCost& c = kStagedCost[staged_row(encoding, group)][type];
+            const int i = (int)(&p - kStagedPlans);
+            if (c.unit[i] == 0.0f || p.wk != like->wk) continue;
+            const int64_t walk = (direct_units(k) + p.wk * like->shares - 1) / (p.wk * like->shares);
+            const double t = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * like->shares, false).all * (c.round + walk * c.unit[i]);
+            if (t < us) us = t, best = p, best.shares = like->shares, best.centred = like->centred;
+        }
+        return best;
+    }
     // Q6_K up to 64 rows, which the small-batch kernel would take in passes of 16: only plans with parts of K of up to 2048, as exact as that kernel
     // (28672 x 8192 with 64 bf16 rows, shared: parts of 2048 1.0e-7 relative error, of 4096 1.1e-7, small-batch kernel 0.98e-7; 101, 93 and 224 us).
     const int64_t longest = encoding == QMM_Q6_K && m <= 64 ? 8 : 1 << 20;  // units of K in a part
@@ -552,6 +632,20 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
         for (int i = 0; shared && i < 3; i++)  // (between predictions this close workgroups of four wavefronts took 3 % longer)
             if (direct_units(k) <= longest * kSharedPlans[i].wk * shares)
                 consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (i == 2 ? 1.03 : 1.0));
+    }
+    if (like || !staged || (encoding == QMM_Q6_K && !beyond && (m <= 64 || best.wn == 1))) return best;
+    // The staged kernel, held to the error of what it replaces: sums no longer than those of that plan (a part of K is one chain of fp32 sums), and where that is
+    // the direct kernel the codes of Q4_K and Q5_K around their middle (KQuantWeights), as there; Q6_K, whose sums leave the matrix cores half as often as in the direct
+    // kernel, only for the shared one.  Beyond the range of those two anything is more exact than the GEMMs that share unpacked weights (2.2e-7 .. 3.5e-6).
+    const bool k_quant = encoding == QMM_Q4_K || encoding == QMM_Q5_K;
+    const bool centred = k_quant && (type == 1 || (!beyond && best.wn == 1) || (encoding == QMM_Q5_K && m <= 64));
+    const int64_t parts = best.wk * best.shares, chain = beyond ? 1 << 20 : std::max<int64_t>(4, (direct_units(k) + parts - 1) / parts);
+    DirectPlan p;
+    // (4 %: as far as the predictions are off; within it the staged kernel was slower as often as faster, GPTQ 4552 x 3072 472 fp32 rows 55.7 and 56.4 us predicted,
+    // 61 and 56 taken; codes around the middle are not in its figures)
+    if (staged_plan(encoding, lhs_dtype, m, n, k, group, whole_tiles, chain, p) * (centred && type == 0 ? 1.08 : 1.04) < us) {
+        best = p;
+        best.centred = centred;
     }
     return best;
 }
@@ -592,25 +686,20 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     if (encoding == QMM_GPTQ && (n % 8 || group % 32)) return false;
     // Served from `from` rows on, where this kernel's time crosses that of the small-batch kernels (passes of four to sixteen rows over
     // the weights; at their best on long weight matrices and on the row lengths their wavefronts divide evenly, 512, 2048 or 4096 values;
-    // this kernel has no such preference), and up to where it crosses that of the GEMMs that unpack a tile or all weights once and then
-    // share them (r = outputs, w = weights, in Mi; beyond about 1100 rows the lhs no longer stays in an L2).  Both lines were fitted to
+    // this kernel has no such preference), and up to where it crosses that of the GEMMs behind it (direct_range).  Both lines were fitted to
     // timings of 4700 calls, 512 x 512 .. 28672 x 4096 with K of 512 .. 14336 and 1 .. 2048 rows: within 2 % on average of always taking
     // the faster of the two.  E.g. 5120 x 5120, 17 bf16 rows: Q4_0 22 -> 16 us, Q4_K 19.6 -> 14.4, Q5_K 34 -> 15.7, Q6_K 54 -> 17.9.
     const bool f32 = lhs_dtype == QMM_F32, wide = n >= 6000;
-    const double w = (double)n * k / (1 << 20), r = (double)m * n / (1 << 20);
+    const double w = (double)n * k / (1 << 20);
     int64_t from = 17;
-    double most = 2.75;      // bf16 outputs at which the other kernels' matrix products, which convert once for all rows, take over
-    int64_t anyway = 0;      // rows up to which the number of outputs does not matter
     switch (encoding) {
         case QMM_Q4_0:
             from = wide && k <= 1024 ? 3 : k <= 2048 ? 5 : 17;
-            most = 3.5, anyway = 450;
             break;
         case QMM_Q4_K:
             // (with few long rows the small-batch kernel cuts K to fill the part)
             from = n >= 2048 && (k <= 1024 || (k < 1536 && w <= 8)) ? 2
                    : !f32 && k > 4096 && n <= 4096 && gemv_q4_k_mm_plain_workspace_bytes(lhs_dtype, m, n, k) == 0 ? 5 : 9;
-            if (k > 4096) most = 1.3;
             break;
         case QMM_Q5_K:
             // (5 .. 16 bf16 rows on a long K: the small-batch kernel cuts it into rounds side by side; 1024 x 14336 9 rows 22.2 / 12.5 us)
@@ -621,31 +710,28 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
             // 71 / 66, but 32000 x 4096 58 / 60, 128256 x 2048 110 / 165, 65536 x 8192 209 / 238)
             if (f32) from = k % 2048 == 0 ? (k == 4096 && n > 36000 ? 17 : 9) : wide ? 3 : n >= 2048 ? 4 : 6;
             else from = k % 2048 == 0 && !(wide && k <= 2048) ? (w <= 30 && k <= 8192 ? 5 : 17) : wide ? 2 : n >= 2048 ? 3 : 6;
-            most = 3.5, anyway = 450;
             break;
         case QMM_GPTQ:
             // Groups that are no multiple of 128: the alternative is the decode kernel, eight rows a pass.
             if (group % 128) return m >= (k >= 7936 && n <= 4096 ? 1 : k >= 2048 ? 2 : w >= 1 ? 3 : 5);
             from = !f32 || k < 2048 ? 17 : k <= 8192 ? 8 : 9;
-            if (k > 4096) most = 1.3;
             break;
         default: return false;
     }
     if (m < from) return false;
-    if (r <= (f32 && encoding != QMM_Q4_0 ? 1.6 : 1)) return true;
-    // fp32 rows are split in two fp16 terms here and in the other kernels, so both multiply twice; the others take K in two passes.  us, others / here:
-    // Q4_K 14336 x 4096 800 rows 327 / 232, 5120 x 5120 1300 rows 239 / 198; Q6_K 14336 x 4096 800 rows 514 / 380;
-    // but GPTQ 4096 x 14336 1050 rows 470 / 560.
-    const bool shared = !kernel_disabled("shared");
-    if (f32) {
-        if (shared && encoding != QMM_Q4_0 && (m <= 1100 || (m <= 1400 && r <= 5.5)) && (encoding != QMM_GPTQ || k <= 8192)) return true;
-        return m <= (w <= 24 || (encoding != QMM_Q4_0 && encoding != QMM_GPTQ) ? 720 : 450) || (k <= 1024 ? r <= 6 : m < 1100 && r <= 3.5);
-    }
-    // (one round of 64 x 256 tiles that fills the compute units by four fifths or more: 11008 x 4096 320 bf16 rows Q4_K 78 / 55, GPTQ 71 / 53, Q5_K 85 / 63;
-    // 8192 x 8192 500 rows Q6_K 205 / 162, Q5_K 145 / 119, but Q4_K 106 / 105 and GPTQ 92 / 101)
-    const int64_t tiles = (m + 63) / 64 * ((n + 255) / 256);
-    if (shared && 5 * tiles >= 4 * compute_units() && tiles <= compute_units() && k <= (encoding == QMM_Q4_K || encoding == QMM_GPTQ ? 4096 : 8192)) return true;
-    return m <= anyway || (m <= 1100 && r <= most);
+    if (direct_range(encoding, lhs_dtype, m, n, k, group)) return true;
+    // Beyond, the staged kernel against the GEMMs that unpack the weights once.  us, those / here: Q4_K 14336 x 4096 400 bf16 rows 80 / 70, 1000 149 / 136, 4096 x 14336 2048 rows
+    // 294 / 258; Q5_K 32000 x 4096 200 rows 165 / 82; Q4_K 14336 x 4096 1300 fp32 rows 506 / 347.  With many bf16 rows on many columns those run at their best,
+    // 256 x 256 results at a time, which the figures of `other` do not know (14336 x 4096 2048 rows 260 / 281, 5120 x 5120 2500 rows 163 / 191, 4096 x 4096 3000 rows 126 / 135).
+    const int row = staged_row(encoding, group);
+    if (row < 0 || (!f32 && m > 1600 && (n > 4096 || (m > 2048 && k <= 8192)))) return false;
+    // On a short K those are the more exact ones for fp32 rows (relative error, those / here: GPTQ K = 256 7.6e-8 / 1.0e-7, 512 9.7e-8 / 1.1e-7, 768 1.1e-7 / 1.1e-7; Q6_K
+    // 1.4e-7 / 2.0e-7, 1.8e-7 / 2.0e-7, 2.3e-7 / 2.0e-7).
+    if (f32 && k < 768 && (encoding == QMM_GPTQ || encoding == QMM_Q6_K)) return false;
+    const float(&o)[5] = kStagedCost[row][f32 ? 1 : 0].other;
+    DirectPlan p;
+    return staged_plan(encoding, lhs_dtype, m, n, k, group, false, 1 << 20, p) <
+           (f32 || m <= 1024 ? 0.95 : 0.9) * (o[0] + o[1] * packed_mb(encoding, n, k) + o[2] * (m * k * 1e-6) + o[3] * (m * n * 1e-6) + o[4] * (1e-9 * ((m + 255) / 256 * 256) * n * k));
 }
 
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k) {
@@ -657,15 +743,18 @@ int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int6
 // call of its own; the tile is the one that suits them together).  q | k | v of 4096 | 1024 | 1024 x 4096 with 16 rows: one launch for three.
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
                               const uint16_t* scales, const uint32_t* qzeros, int group, int64_t m, int64_t k, uint16_t* out16, void* workspace,
-                              hipStream_t s) {
+                              hipStream_t s, bool any_rows) {
     const bool q40 = encoding == QMM_Q4_0, f32 = lhs_dtype == QMM_F32, sums = encoding == QMM_Q4_K || encoding == QMM_Q5_K || q40;
     if (count < 1 || count > kDirectMaxMats) return hipErrorInvalidValue;
     const DirectSpace p = direct_space(workspace, f32 && !q40, sums, sums && !q40, m, k);
+    // (loads of 16 bytes straight to LDS, of 4 for the scales and zeros of GPTQ)
+    bool staged = (((uintptr_t)scales | (uintptr_t)qzeros) & 3) == 0;
+    for (int j = 0; j < count; j++) staged = staged && ((uintptr_t)ws[j] & 15) == 0;
     DirectPlan plans[kDirectMaxMats];
     DirectMats zero{};
     int64_t zeros = 0;
     for (int j = 0; j < count; j++) {
-        plans[j] = direct_plan(encoding, lhs_dtype, m, ns[j], k, group, out16 != nullptr);
+        plans[j] = direct_plan(encoding, lhs_dtype, m, ns[j], k, group, out16 != nullptr, staged, !any_rows && !direct_range(encoding, lhs_dtype, m, ns[j], k, group));
         if (plans[j].shares > 1) zero.out[zero.count] = outs[j], zero.n[zero.count++] = (int)ns[j], zeros = std::max(zeros, m * ns[j]);
     }
     const unsigned grid = (unsigned)((m + 63) / 64 * 64 + std::min<int64_t>(1024, (zeros + 4095) / 4096));
@@ -690,12 +779,18 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
         DirectMats mats{};
         int64_t n = 0;
         for (int i = j; i < count; i++) {
-            if (done[i] || plans[i].wk != pl.wk || plans[i].shares != pl.shares || (plans[i].wn > 1) != (pl.wn > 1)) continue;
+            if (done[i] || plans[i].wk != pl.wk || plans[i].shares != pl.shares || (plans[i].wn > 1) != (pl.wn > 1) || (plans[i].fn == 0) != (pl.fn == 0) ||
+                plans[i].centred != pl.centred)
+                continue;
             mats.w[mats.count] = (const uint8_t*)ws[i], mats.out[mats.count] = outs[i], mats.n[mats.count++] = (int)ns[i];
             n += ns[i];
             done[i] = true;
         }
-        if (mats.count > 1) pl = direct_plan(encoding, lhs_dtype, m, n, k, group, false, &pl);
+        if (mats.count > 1) pl = direct_plan(encoding, lhs_dtype, m, n, k, group, false, staged, false, &pl);
+        if (pl.fn == 0) {
+            e = launch_gemm_staged(encoding, f32 && !q40, pl, wt, mats, p, out16, m, units, s);
+            continue;
+        }
         if (pl.wn > 1) {
             e = launch_gemm_shared(encoding, f32 && !q40, pl, wt, mats, p, out16, m, units, s);
             continue;

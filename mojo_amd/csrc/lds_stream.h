@@ -55,6 +55,15 @@ __device__ __forceinline__ void load16_to_lds(uint32_t lane_offset, const void* 
                  : "memory");
 }
 
+// 4 bytes per lane, to LDS at lds_base + 4 * lane.
+__device__ __forceinline__ void load4_to_lds(const void* g, uint32_t lds_base) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(g), "s"(lds_base)
+                 : "memory");
+}
+
 // Plain global loads into registers, hidden the same way.  The destination may only be used after
 // wait_vmcnt and tie() on it.
 __device__ __forceinline__ void hidden_load(u32x4& d, const void* g) {

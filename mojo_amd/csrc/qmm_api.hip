@@ -540,7 +540,7 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
                 const void* sorted[3] = {p.qweight, rhs[1], rhs[2]};
                 if (order_direct()) {
                     e = qmm::launch_gemm_direct(encoding, p.lhs, lhs_dtype, 1, sorted, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], cfg->group_size, m, k,
-                                                nullptr, (char*)workspace + p.bytes, s);
+                                                nullptr, (char*)workspace + p.bytes, s, true);
                     if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, direct GEMM)");
                 } else if (int rc = matmul_f32(encoding, &plain, p.lhs, lhs_dtype, m, k, sorted, 3, n, out, (char*)workspace + p.bytes, workspace_bytes - p.bytes, flags, stream))
                     return rc;
@@ -901,14 +901,12 @@ int qmm_repack(int encoding, const qmm_gptq_config* cfg, const void* const* rhs,
 // 4096 x 14336: 57 against 83 at 64 rows, 84 against 84 at 96.
 static int64_t q4_0_repacked_min_rows(int64_t k) { return k > 4096 ? 96 : 80; }
 // With the planes at hand the direct GEMM on the packed tensors still wins while the weights are most of the traffic (the planes are 2 or 4
-// bytes a weight against 0.6 .. 0.8): us, planes / direct: Q5_K 4096 x 4096 128 bf16 rows 33 / 20, 300 rows 46 / 35; 14336 x 4096 200 rows
-// 69 / 60, 300 rows 81 / 93; Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.  fp32 rows
-// walk the planes twice: 450 / 1050 rows, Q5_K 14336 x 4096 177 / 160, 470 / 329, 4096 x 14336 326 / 157, 459 / 388; Q6_K 4096 x 4096 152 / 70, 203 / 203;
-// Q4_K 14336 x 4096 199 / 178, 468 / 297 (700 rows 274 / 286); but GPTQ 14336 x 4096 148 / 159, 4096 x 14336 700 rows 247 / 291.
+// bytes a weight against 0.6 .. 0.8): us, planes / direct: Q5_K 4096 x 4096 512 bf16 rows 54 / 37, 14336 x 4096 200 rows 75 / 49, 700 121 / 119, 1000 130 / 149; Q4_K 14336 x 4096
+// 700 rows 121 / 108, 1000 128 / 134; Q6_K 14336 x 4096 700 rows 172 / 168 (1000 219 / 214); Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.  fp32 rows
+// walk the planes twice: GPTQ 14336 x 4096 700 rows 260 / 173, 1400 466 / 315; Q5_K 14336 x 4096 1050 rows 470 / 329; Q6_K 4096 x 4096 450 rows 152 / 70.
 static bool direct_over_planes(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    const bool narrow = m * n <= (int64_t)1300 << 10;
-    return (narrow || m <= (lhs_dtype != QMM_F32 || encoding == QMM_Q4_0 ? 150 : encoding == QMM_GPTQ ? 400 : 1400)) && !(encoding == QMM_GPTQ && cfg->desc_act) &&
-           direct_wanted(encoding, cfg, lhs_dtype, m, n, k);
+    const bool narrow = m * n <= (int64_t)1300 << 10, q40 = encoding == QMM_Q4_0;
+    return (narrow || m <= (q40 ? 150 : 768) || (lhs_dtype == QMM_F32 && !q40)) && !(encoding == QMM_GPTQ && cfg->desc_act) && direct_wanted(encoding, cfg, lhs_dtype, m, n, k);
 }
 static bool repacked_path(int encoding, int64_t m, int64_t n, int64_t k, bool have_rhs) {
     if (!have_rhs) return true;

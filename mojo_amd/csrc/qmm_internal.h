@@ -11,7 +11,7 @@ namespace qmm {
 
 // Kernel families switched off by the environment variable QMM_DISABLE (a comma-separated list of names, read once
 // per process), for tests and triage: a disabled family reports that it does not take a shape, and the next kernel
-// in the dispatch order serves it.  Names: direct, shared, q4k_lanes, q4k_lanes_rows, q4k_stream, q4k_mm, q4k_kc, q4k_tile, q4k_gemm64, q4k_twin_rows, q4k_rows_v2,
+// in the dispatch order serves it.  Names: direct, shared, staged, q4k_lanes, q4k_lanes_rows, q4k_stream, q4k_mm, q4k_kc, q4k_tile, q4k_gemm64, q4k_twin_rows, q4k_rows_v2,
 // q4_0_stream, q4_0_mfma, q4_0_small, q4_0_small_passes, q4_0_wide, q4_0_planes, q6k_lanes, q6k_slab, q6k_staged, kquant_planes, planes_wide, planes_192, planes_quarters, planes_twin_rows, gptq_twin_rows, gptq_k_shares, gptq_long_k_mm, kquant_mm_rounds_grid, q4k_mm_k_parts, q4k_planes, gptq_planes, gptq_mm, gptq_cols, gptq_cols16, gptq_order, q4k_mm_gated.
 // Nothing is disabled by default.
 bool kernel_disabled(const char* family);
@@ -22,13 +22,14 @@ bool twin_rows_allowed();
 // compute units of the current device (asked for once; 256 where there is none)
 int compute_units();
 
-// gemm_direct.hip: a few to a few hundred lhs rows, every encoding; out16 != null: bf16 results (out is then unused)
+// gemm_direct.hip: a few to a few hundred lhs rows, more where the staged kernel pays, every encoding; out16 != null: bf16 results (out is then unused).
+// any_rows: called with more rows than gemm_direct_wanted says, held to the error of the direct and shared kernels all the same.
 bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k);
 constexpr int kDirectMaxMats = 4;  // count: matrices that share the lhs (out16: one)
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
                               const uint16_t* scales, const uint32_t* qzeros, int group, int64_t m, int64_t k, uint16_t* out16, void* workspace,
-                              hipStream_t s);
+                              hipStream_t s, bool any_rows = false);
 
 hipError_t launch_read_probe(const void* buf, int64_t bytes, hipStream_t s);
 // register-resident matrix-core loop (probes.hip): `workgroups` workgroups of 8 wavefronts, out fp32 [workgroups * 512]

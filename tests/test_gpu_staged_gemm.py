@@ -1,0 +1,80 @@
+"""The GEMM whose lhs and packed weights go to LDS by themselves, at the edges of its tiles (64, 96 or 128 rows, 64, 128 or 256 columns), of its units of 256
+values of K and of the ways it cuts K (one to four parts a workgroup, one or two workgroups a tile), against float64 products of the same integers."""
+import ctypes as C
+
+import pytest
+import torch
+
+from mojo_amd import QuantizationEncoding as QE, _lib, qmatmul, qmatmul_grouped
+from test_gpu_direct_gemm import check, weights
+
+pytestmark = pytest.mark.gpu
+
+# (rows, columns, K): one unit and several, parts of unequal lengths; a row and a column short of a tile and beyond one
+SIZES = ((79, 5128, 4352), (97, 4104, 4352), (100, 14344, 256), (129, 11016, 2304), (161, 14344, 1280), (200, 4104, 4352), (255, 14336, 512), (257, 6152, 2304), (330, 8200, 768),
+         (385, 14328, 1024), (641, 4104, 2304), (700, 9000, 512), (1300, 4104, 768))
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("enc,group", [(QE.Q4_K, 0), (QE.Q5_K, 0), (QE.Q6_K, 0), (QE.GPTQ, 128), (QE.GPTQ, 256), (QE.GPTQ, 32)])
+def test_edges(enc, group, lhs):
+    for m, n, k in SIZES:
+        config, rhs = weights(enc, group, n, k)
+        a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(lhs)
+        a[m // 2] *= 1e-6
+        a[m - 1] = 0.0
+        check(qmatmul(enc, config, a, *rhs), enc, config, rhs, a)
+        check(qmatmul(enc, config, a, *rhs, out_dtype=torch.bfloat16), enc, config, rhs, a)
+
+
+@pytest.mark.parametrize("n", [2048 + 1, 14336 - 3])
+def test_odd_columns(n):
+    """K-quants take any number of columns: rows of the result that begin at any multiple of four bytes."""
+    for enc in (QE.Q4_K, QE.Q6_K):
+        _, rhs = weights(enc, 0, n, 1024)
+        a = torch.randn((190, 1024), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n)).bfloat16()
+        check(qmatmul(enc, None, a, *rhs), enc, None, rhs, a)
+
+
+def test_misaligned_gptq_words():
+    """qweight may lie at any multiple of four bytes; loads of 16 bytes to LDS want sixteen, so those calls stay with the kernels before."""
+    config, rhs = weights(QE.GPTQ, 128, 14336, 1024)
+    a = torch.randn((200, 1024), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)).bfloat16()
+    words = torch.empty(rhs[0].numel() + 1, dtype=torch.int32, device="cuda")
+    words[1:] = rhs[0].flatten()
+    moved = (words[1:].view(rhs[0].shape), *rhs[1:])
+    lib = _lib.load()
+    cfg = C.byref(_lib.GptqConfig(4, 128, 0, 1))
+    need = lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, cfg, _lib.QMM_BF16, 200, 14336, 1024, 0)
+    ws, out = torch.empty(need, dtype=torch.uint8, device="cuda"), torch.full((200, 14336), float("nan"), device="cuda")
+    ptrs = (C.c_void_p * 3)(*[t.data_ptr() for t in moved])
+    assert lib.qmm_matmul(QE.GPTQ.code, cfg, a.data_ptr(), _lib.QMM_BF16, 200, 1024, ptrs, 3, 14336, out.data_ptr(), ws.data_ptr(), need, 0,
+                          torch.cuda.current_stream().cuda_stream) == 0
+    check(out, QE.GPTQ, config, moved, a)
+
+
+def test_matrices_together_sum_as_alone():
+    """q | k | v in one launch: the bits of three calls of their own."""
+    for enc in (QE.Q4_K, QE.Q5_K, QE.Q6_K):
+        for m, ns, k in ((200, (4096, 1024, 1024), 4096), (300, (4104, 4104), 2304)):
+            mats = [weights(enc, 0, n, k)[1][0] for n in ns]
+            a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).bfloat16()
+            for got, w in zip(qmatmul_grouped(enc, a, mats), mats):
+                assert torch.equal(got, qmatmul(enc, None, a, w))
+
+
+# Relative error of (enc, group, rows, n, k, lhs): the float32 sums of the kernel that served the call before, by 1.08
+@pytest.mark.parametrize("enc,group,m,n,k,lhs,most", [
+    (QE.Q4_K, 0, 96, 4096, 4096, torch.bfloat16, 1.06e-7), (QE.Q4_K, 0, 200, 14336, 4096, torch.bfloat16, 2.2e-7), (QE.Q4_K, 0, 200, 4096, 4096, torch.float32, 2.04e-7),
+    (QE.Q5_K, 0, 64, 14336, 4096, torch.bfloat16, 1.35e-7), (QE.Q6_K, 0, 500, 4096, 14336, torch.bfloat16, 1.5e-7), (QE.GPTQ, 128, 400, 4096, 4096, torch.bfloat16, 0.86e-7),
+    (QE.GPTQ, 32, 300, 4096, 4096, torch.bfloat16, 0.85e-7), (QE.GPTQ, 128, 800, 14336, 4096, torch.float32, 1.7e-7)])
+def test_precision(enc, group, m, n, k, lhs, most):
+    from mojo_amd import QuantizationConfig, dequantize, quantize, quantize_gptq
+
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    w = torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen)
+    config = QuantizationConfig("gptq", 4, group, False, True) if enc == QE.GPTQ else None
+    rhs = quantize_gptq(w, config)[:3] if config else (quantize(enc, w),)
+    a = torch.randn((m, k), device="cuda", generator=gen).to(lhs)
+    want = a.double() @ dequantize(enc, *rhs, config=config).double().T
+    assert ((qmatmul(enc, config, a, *rhs).double() - want).norm() / want.norm()).item() < most

@@ -57,3 +57,10 @@ def test_direct_and_shared_gemms_keep_their_sums_in_registers(kernels):
     found = {name: spilled for name, (_, spilled) in kernels.items() if re.match(r"gemm_(direct|shared)_kernel<", name)}
     assert len(found) > 60
     assert {name: spilled for name, spilled in found.items() if spilled > 8} == {}
+
+
+def test_staged_gemm_keeps_its_sums_in_registers(kernels):
+    """Up to 128 rows a wavefront fit 256 registers only because its loads hold none; a body that spilled 12 took twice the time."""
+    found = {name: spilled for name, (_, spilled) in kernels.items() if name.startswith("gemm_staged_kernel<")}
+    assert len(found) > 50
+    assert {name: spilled for name, spilled in found.items() if spilled} == {}
