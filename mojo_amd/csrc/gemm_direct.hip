@@ -639,7 +639,10 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
     // kernel, only for the shared one.  Beyond the range of those two anything is more exact than the GEMMs that share unpacked weights (2.2e-7 .. 3.5e-6).
     const bool k_quant = encoding == QMM_Q4_K || encoding == QMM_Q5_K;
     const bool centred = k_quant && (type == 1 || (!beyond && best.wn == 1) || (encoding == QMM_Q5_K && m <= 64));
-    const int64_t parts = best.wk * best.shares, chain = beyond ? 1 << 20 : std::max<int64_t>(4, (direct_units(k) + parts - 1) / parts);
+    // K-quants with fp32 rows grow less with it here and in the shared kernel (relative error after 1, 3, 4 units in the direct kernel 1.63e-7, 1.80e-7, 1.89e-7; here
+    // after 4, 16, 24, 40 1.64e-7, 1.78e-7, 1.87e-7, 2.04e-7).
+    const int64_t parts = best.wk * best.shares, part = (direct_units(k) + parts - 1) / parts;
+    const int64_t chain = beyond ? 1 << 20 : std::max<int64_t>(4, k_quant && type == 1 && best.wn == 1 && part > 1 ? 5 * part : part);
     DirectPlan p;
     // (4 %: as far as the predictions are off; within it the staged kernel was slower as often as faster, GPTQ 4552 x 3072 472 fp32 rows 55.7 and 56.4 us predicted,
     // 61 and 56 taken; codes around the middle are not in its figures)
