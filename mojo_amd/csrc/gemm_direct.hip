@@ -80,9 +80,12 @@ __device__ __forceinline__ void zero_out(const DirectMats& z, int m, int e, int 
 // columns (200 x 14336 bf16 rows with 256 threads a row 10.1 us, with 1024 7.2); with many, that a row writes 16 bytes of a 128-byte line, the rest
 // of which other workgroups of the XCD fill (500 x 14336: 11.5 us for 28 MB, whatever the number of threads).
 // Rows of one group of eight go to workgroups of one XCD (ids congruent mod 8): a 128-byte line of an operand holds eight rows.
-template <typename AT, int ORDER>
-__global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, int with_sums, DirectMats zero) {
+// SORTED: column p of the operands is column source[p] of the row, which lies in LDS (k values) meanwhile.
+template <typename AT, int ORDER, bool SORTED = false>
+__global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, int with_sums, DirectMats zero,
+                                                           const int32_t* __restrict__ source) {
     constexpr bool kF32 = sizeof(AT) == 4;
+    extern __shared__ __attribute__((aligned(16))) uint8_t row_lds[];
     __shared__ uint32_t wmax[16];
     const int tid = threadIdx.x, threads = (int)blockDim.x, rows = (m + 63) / 64 * 64;
     if ((int)blockIdx.x >= rows) {
@@ -97,7 +100,24 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     constexpr int kHeld = 4;    // rows of up to 32768 columns (1024 threads) stay in registers between the search for the maximum and the narrowing
     float held[kHeld][8];
     const bool hold = pieces <= kHeld * threads;
-    auto load = [&](int pc, float (&v)[8]) __attribute__((always_inline)) { load8(ar + pc * 8, v); };
+    if constexpr (SORTED) {
+        constexpr int kPer = 16 / sizeof(AT);
+        for (int i = tid * kPer; i < k; i += threads * kPer) *(gd_u4*)((AT*)row_lds + i) = *(const gd_u4*)(ar + i);
+        __syncthreads();
+    }
+    auto load = [&](int pc, float (&v)[8]) __attribute__((always_inline)) {
+        if constexpr (SORTED) {
+            const int4 s0 = *(const int4*)(source + 8 * pc), s1 = *(const int4*)(source + 8 * pc + 4);
+            const int from[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                if constexpr (kF32) v[i] = ((const float*)row_lds)[from[i]];
+                else v[i] = __uint_as_float((uint32_t)((const uint16_t*)row_lds)[from[i]] << 16);
+            }
+        } else {
+            load8(ar + pc * 8, v);
+        }
+    };
     float mx = 0.0f;
     auto top = [&](const float (&v)[8]) __attribute__((always_inline)) {
 #pragma unroll
@@ -746,7 +766,7 @@ int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int6
 // call of its own; the tile is the one that suits them together).  q | k | v of 4096 | 1024 | 1024 x 4096 with 16 rows: one launch for three.
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
                               const uint16_t* scales, const uint32_t* qzeros, int group, int64_t m, int64_t k, uint16_t* out16, void* workspace,
-                              hipStream_t s, bool any_rows) {
+                              hipStream_t s, bool any_rows, const int32_t* source) {
     const bool q40 = encoding == QMM_Q4_0, f32 = lhs_dtype == QMM_F32, sums = encoding == QMM_Q4_K || encoding == QMM_Q5_K || q40;
     if (count < 1 || count > kDirectMaxMats) return hipErrorInvalidValue;
     const DirectSpace p = direct_space(workspace, f32 && !q40, sums, sums && !q40, m, k);
@@ -765,12 +785,19 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
     if (q40) {
         if (f32) direct_prep_q8_kernel<float><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, zero);
         else direct_prep_q8_kernel<uint16_t><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, zero);
+    } else if (source) {  // (the rest of the path takes it up to K = 32768, fp32 rows of 128 KB)
+        if (encoding != QMM_GPTQ || k % 32 || k > 32768) return hipErrorInvalidValue;
+        hipError_t e = f32 ? allow_full_lds<direct_prep_kernel<float, kOrderGptq, true>, 64>() : allow_full_lds<direct_prep_kernel<uint16_t, kOrderGptq, true>, 64>();
+        if (e != hipSuccess) return e;
+        const size_t row = (size_t)k * (f32 ? 4 : 2);
+        if (f32) direct_prep_kernel<float, kOrderGptq, true><<<dim3(grid), dim3(threads), row, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero, source);
+        else direct_prep_kernel<uint16_t, kOrderGptq, true><<<dim3(grid), dim3(threads), row, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero, source);
     } else if (encoding == QMM_GPTQ) {
-        if (f32) direct_prep_kernel<float, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero);
-        else direct_prep_kernel<uint16_t, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero);
+        if (f32) direct_prep_kernel<float, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero, nullptr);
+        else direct_prep_kernel<uint16_t, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero, nullptr);
     } else {
-        if (f32) direct_prep_kernel<float, kOrderK><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero);
-        else direct_prep_kernel<uint16_t, kOrderK><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero);
+        if (f32) direct_prep_kernel<float, kOrderK><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero, nullptr);
+        else direct_prep_kernel<uint16_t, kOrderK><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero, nullptr);
     }
     hipError_t e = hipGetLastError();
     const WeightTensors wt{nullptr, scales, qzeros, 0, (int)k, group};

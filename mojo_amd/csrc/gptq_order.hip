@@ -2,16 +2,21 @@
 // groups serve the call.
 //
 // The kernel that looks the group of every k up (gemv_gptq.hip) passes over the weights once per four rows and multiplies on the vector
-// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 103 us.  Sorting costs one small launch and one pass over the packed weights: the words of
-// some columns of the output lie in LDS (all of K), from which every word of the sorted matrix takes its eight nibbles; other workgroups
-// of that launch sort the columns of the lhs.  What bounds the pass is reading and writing the packed weights (2 x 29 MB at 14336 x 4096: 17 us with 400 rows of
-// lhs, 3.8 TB/s; the sort, one workgroup, 6; profiles/direct_gemm_act_order_quantisers__kernel_trace.txt).
+// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 99 us.  Sorting costs one launch and one pass over the packed weights: a workgroup holds some
+// columns of the output in LDS (all of K), sorts the columns of K by group while those are on their way, and takes the eight nibbles of every word of the sorted
+// matrix from there.  The preparation of the lhs in the direct GEMM reads its rows in the same order.
+// What bounds the pass, at 14336 x 4096 (2 x 29 MB, 22 us with nothing in the caches, 2.6 TB/s): loads, sort (hidden behind them but for its start),
+// nibbles (two vector instructions each, about 6 us) and stores one after the other, since all workgroups run at once.
+// us of the whole call with the sort as a launch of its own and a sorted copy of the lhs / this way, nothing in the caches: 14336 x 4096 400 rows 127 / 122, 8 rows 50 / 44;
+// 4096 x 14336 64 rows 76 / 63; 4096 x 4096 64 rows 37 / 30; 8192 x 8192 300 rows 130 / 123; 1024 x 4096 20 rows 29 / 22; 8192 x 28672 20 rows 184 / 174;
+// 3584 x 18944 33 rows 90 / 90.
 //
 // A sorted column list is a plain-group matrix only if every group has exactly group_size columns, which is so in any checkpoint that was
 // quantised group by group.  The device finds out: where it is not so, the sort leaves a mark, the order as it was (the products are then
 // meaningless) and the look-up kernel, launched behind them, replaces the whole result; otherwise that launch returns at once.
 #include <algorithm>
 
+#include "lds_stream.h"
 #include "qmm_internal.h"
 
 namespace qmm {
@@ -19,123 +24,138 @@ namespace qmm {
 namespace {
 
 typedef uint32_t go_u4 __attribute__((ext_vector_type(4)));
-struct __attribute__((packed, aligned(4))) GoWords4 {  // (qweight is 4-byte aligned)
-    go_u4 v;
-};
 
-constexpr int kSortWaves = 16;
+constexpr int kWaves = 16, kThreads = 64 * kWaves;
 
-// source[p]: the column of K at sorted position p.  Stable (within a group the columns keep their order).  One workgroup; wavefront w
-// takes a sixteenth of K.  Group indices outside [0, groups) are clamped, as in the look-up kernel.
-__global__ __launch_bounds__(64 * kSortWaves) void gptq_order_sort_kernel(const int32_t* __restrict__ g_idx, int k, int group, int bits,
-                                                                          int32_t* __restrict__ source, int32_t* __restrict__ uneven) {
-    extern __shared__ uint32_t counts[];  // [kSortWaves][groups], then whether any group has another size
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int groups = k / group;
-    uint32_t* const bad = counts + kSortWaves * groups;
-    for (int i = tid; i <= kSortWaves * groups; i += 64 * kSortWaves) counts[i] = 0;
-    __syncthreads();
-    const int per = ((k + kSortWaves - 1) / kSortWaves + 63) / 64 * 64, lo = min(k, wave * per), hi = min(k, lo + per);
-    uint32_t* const mine = counts + wave * groups;
-    auto group_of = [&](int i) __attribute__((always_inline)) { return min(max(g_idx[i], 0), groups - 1); };
-    for (int i = lo + lane; i < hi; i += 64) atomicAdd(mine + group_of(i), 1u);
-    __syncthreads();
-    for (int g = tid; g < groups; g += 64 * kSortWaves) {  // where each wavefront's columns of the group begin
-        uint32_t at = 0;
-        for (int w = 0; w < kSortWaves; w++) {
-            const uint32_t c = counts[w * groups + g];
-            counts[w * groups + g] = at;
-            at += c;
-        }
-        if (at != (uint32_t)group) *bad = 1;
-    }
-    __syncthreads();
-    const bool as_is = *bad != 0;
-    if (tid == 0) *uneven = as_is;
-    if (as_is) {
-        for (int i = tid; i < k; i += 64 * kSortWaves) source[i] = i;
-        return;
-    }
-    for (int i0 = lo; i0 < hi; i0 += 64) {
-        const int i = i0 + lane;
-        const bool live = i < hi;
-        const int g = live ? group_of(i) : 0;
-        uint64_t same = __ballot(live);  // the lanes with this lane's group
-        for (int b = 0; b < bits; b++) {
-            const bool set = (g >> b) & 1;
-            const uint64_t with = __ballot(set);
-            same &= set ? with : ~with;
-        }
-        const int rank = __popcll(same & ((1ull << lane) - 1)), count = __popcll(same);
-        if (live) {
-            const uint32_t at = mine[g];
-            source[g * group + (int)at + rank] = i;
-            if (rank == count - 1) mine[g] = at + (uint32_t)count;
-        }
-        // (the next turn of this wavefront reads what its lanes wrote: LDS operations of a wavefront are performed in order)
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
-// The first 8 * per_xcd workgroups: COLS columns of the weights each, neighbours on one XCD (they share cache lines).  Then one per lhs row.
-template <typename AT, int COLS>
-__global__ __launch_bounds__(512) void gptq_order_permute_kernel(const uint32_t* __restrict__ qweight, const AT* __restrict__ a, int n, int k, int per_xcd,
-                                                                 const int32_t* __restrict__ source, uint32_t* __restrict__ sorted_w,
-                                                                 AT* __restrict__ sorted_a) {
+// Workgroup: COLS columns of the weights, neighbours on one XCD (they share cache lines).  It sorts for itself while its words are on their way to LDS: where the
+// sort was a launch of one workgroup it took 6.6 us at K = 4096 and 18 at 14336.
+// Stable sort (within a group the columns keep their order), wavefront w takes a sixteenth of K, TURNS times 64 columns; group indices outside [0, groups) are
+// clamped, as in the look-up kernel.  The first workgroup leaves the order (source[p]: the column of K at sorted position p) and the mark in memory.
+// LDS: [k / 8][COLS] words, uint16 [k] order, uint16 [kWaves][groups] counts.
+// Where that is more than a compute unit has (K beyond 26208, less with groups of 32 or 64): a launch of one workgroup without words (qweight null) that only sorts, then TURNS = 0, which
+// takes the order from memory.
+template <int COLS, int TURNS>
+__global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_permute_kernel(const uint32_t* __restrict__ qweight, const int32_t* __restrict__ g_idx, int n,
+                                                                                          int k, int group, int bits, int per_xcd, int32_t* __restrict__ source,
+                                                                                          int32_t* __restrict__ uneven, uint32_t* __restrict__ sorted_w) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int tid = threadIdx.x, b = (int)blockIdx.x;
-    if (b < 8 * per_xcd) {
-        constexpr int kPieces = COLS / 4;
-        const int col = ((b & 7) * per_xcd + (b >> 3)) * COLS + 4 * (tid & (kPieces - 1));
-        const int rows = k >> 3, r0 = tid / kPieces;
-        constexpr int kRows = 512 / kPieces;  // rows per turn
-        const bool in_n = col < n;            // (N is a multiple of 8)
-        const uint32_t* from = qweight + (in_n ? col : 0);
-        uint32_t* const words = (uint32_t*)smem + 4 * (tid & (kPieces - 1));
-#pragma unroll 8
-        for (int r = r0; r < rows; r += kRows) *(go_u4*)(words + r * COLS) = ((const GoWords4*)(from + (int64_t)r * n))->v;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = (int)blockIdx.x;
+    constexpr int kPieces = COLS / 4, kRows = kThreads / kPieces;  // rows of words per turn
+    const int slab = ((b & 7) * per_xcd + (b >> 3)) * COLS;
+    if (slab >= n) return;
+    const int col = slab + 4 * (tid & (kPieces - 1)), rows = qweight ? k >> 3 : 0, r0 = tid / kPieces, groups = k / group;
+    const bool in_n = col < n;  // (N is a multiple of 8)
+    uint16_t* const order = (uint16_t*)(smem + (size_t)rows * COLS * 4);
+    uint16_t* const counts = order + k;
+    uint32_t* const pairs = (uint32_t*)counts;  // (k is even)
+    uint32_t* const bad = (uint32_t*)order;     // until the order is written
+
+    auto load_words = [&]() __attribute__((always_inline)) {
+        const uint32_t to = lds_address(smem) + wave * 1024;
+        const uint32_t* const from = qweight + (in_n ? col : 0);
+        for (int i = 0; i * kRows < rows; i++)
+            if (i * kRows + r0 < rows) load16_to_lds(from + (int64_t)(i * kRows + r0) * n, to + i * (kThreads * 16));
+    };
+    if constexpr (TURNS == 0) {
+        load_words();
+        wait_vmcnt<0>();
         __syncthreads();
-        if (!in_n) return;
-#pragma unroll 2
-        for (int r = r0; r < rows; r += kRows) {
-            const int4 s0 = *(const int4*)(source + 8 * r), s1 = *(const int4*)(source + 8 * r + 4);
-            const int src[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-            go_u4 o = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const go_u4 x = *(const go_u4*)(words + (src[j] >> 3) * COLS);
-                const int at = 4 * (src[j] & 7);
-#pragma unroll
-                for (int c = 0; c < 4; c++) o[c] |= ((x[c] >> at) & 0xFu) << (4 * j);
+    } else {
+        // (asked for before the words: a wait for these would be one for everything asked for earlier)
+        const int per = (k + 64 * kWaves - 1) / (64 * kWaves) * 64, lo = wave * per;
+        int g[TURNS];
+    #pragma unroll
+        for (int t = 0; t < TURNS; t++) g[t] = g_idx[min(lo + 64 * t + lane, k - 1)];
+        for (int i = tid; i < (kWaves * groups + 1) / 2; i += kThreads) pairs[i] = 0;
+        if (tid == 0) *bad = 0;
+    #pragma unroll
+        for (int t = 0; t < TURNS; t++) {
+            g[t] = min(max(g[t], 0), groups - 1);
+            tie(g[t]);
+        }
+        load_words();
+
+        const int turns = min(per, max(0, k - lo));  // columns of this wavefront
+        __syncthreads();
+    #pragma unroll
+        for (int t = 0; t < TURNS; t++)
+            if (64 * t + lane < turns) {
+                const int at = wave * groups + g[t];
+                atomicAdd(pairs + (at >> 1), 1u << (16 * (at & 1)));
             }
-            *(go_u4*)(sorted_w + (int64_t)r * n + col) = o;
+        __syncthreads();
+        for (int i = tid; i < groups; i += kThreads) {  // where each wavefront's columns of the group begin
+            uint32_t c[kWaves], at = 0;
+    #pragma unroll
+            for (int w = 0; w < kWaves; w++) c[w] = counts[w * groups + i];
+    #pragma unroll
+            for (int w = 0; w < kWaves; w++) {
+                counts[w * groups + i] = (uint16_t)at;
+                at += c[w];
+            }
+            if (at != (uint32_t)group) *bad = 1;
         }
-        return;
+        __syncthreads();
+        const bool as_is = *bad != 0;
+        __syncthreads();
+        if (as_is) {
+            for (int i = tid; i < k; i += kThreads) order[i] = (uint16_t)i;
+        } else {
+            uint16_t* const mine = counts + wave * groups;
+    #pragma unroll
+            for (int t = 0; t < TURNS; t++) {
+                if (64 * t >= turns) break;
+                const bool live = 64 * t + lane < turns;
+                uint64_t same = __ballot(live);  // the lanes with this lane's group
+                for (int bit = 0; bit < bits; bit++) {
+                    const bool set = (g[t] >> bit) & 1;
+                    const uint64_t with = __ballot(set);
+                    same &= set ? with : ~with;
+                }
+                const int rank = __popcll(same & ((1ull << lane) - 1)), count = __popcll(same);
+                if (live) {
+                    const uint32_t at = mine[g[t]];
+                    order[g[t] * group + (int)at + rank] = (uint16_t)(lo + 64 * t + lane);
+                    if (rank == count - 1) mine[g[t]] = (uint16_t)(at + (uint32_t)count);
+                }
+                // (the next turn of this wavefront reads what its lanes wrote: LDS operations of a wavefront are performed in order)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        wait_vmcnt<0>();
+        __syncthreads();
+        if (b == 0) {
+            if (tid == 0) *uneven = as_is;
+            for (int i = tid; i < k; i += kThreads) source[i] = order[i];
+        }
     }
-    const int64_t row = b - 8 * per_xcd;
-    AT* const held = (AT*)smem;
-    const AT* ar = a + row * k;
-    constexpr int kPer = 16 / sizeof(AT);
-    for (int i = tid * kPer; i < k; i += 512 * kPer) *(go_u4*)(held + i) = *(const go_u4*)(ar + i);
-    __syncthreads();
-    for (int i = tid * kPer; i < k; i += 512 * kPer) {
-        AT v[kPer] __attribute__((aligned(16)));
-#pragma unroll
-        for (int j = 0; j < kPer; j += 4) {
-            const int4 s = *(const int4*)(source + i + j);
-            v[j] = held[s.x];
-            v[j + 1] = held[s.y];
-            v[j + 2] = held[s.z];
-            v[j + 3] = held[s.w];
+    if (!in_n) return;
+    const uint8_t* const words = smem + 16 * (tid & (kPieces - 1));
+#pragma unroll 2
+    for (int r = r0; r < rows; r += kRows) {
+        go_u4 s;
+        if constexpr (TURNS == 0) {
+            const go_u4 s0 = *(const go_u4*)(source + 8 * r), s1 = *(const go_u4*)(source + 8 * r + 4);
+            s = go_u4{s0.x | s0.y << 16, s0.z | s0.w << 16, s1.x | s1.y << 16, s1.z | s1.w << 16};
+        } else {
+            s = *(const go_u4*)(order + 8 * r);
         }
-        *(go_u4*)(sorted_a + row * k + i) = *(const go_u4*)v;
+        go_u4 o = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t src = (j & 1) ? s[j >> 1] >> 16 : s[j >> 1] & 0xffffu;
+            const go_u4 x = *(const go_u4*)(words + (src >> 3) * (COLS * 4));
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_alignbit(x[c] >> ((src << 2) & 31u), o[c], 4);
+        }
+        *(go_u4*)(sorted_w + (int64_t)r * n + col) = o;
     }
 }
 
 }  // namespace
 
-GptqOrderSpace gptq_order_space(void* workspace, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+GptqOrderSpace gptq_order_space(void* workspace, int64_t n, int64_t k) {
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     GptqOrderSpace p;
     char* base = (char*)workspace;
@@ -145,15 +165,13 @@ GptqOrderSpace gptq_order_space(void* workspace, int lhs_dtype, int64_t m, int64
     off += up(k * 4);
     p.qweight = (uint32_t*)(base + off);
     off += up(n * k / 2);
-    p.lhs = base + off;
-    off += up(m * k * (lhs_dtype == QMM_F32 ? 4 : 2));
     p.bytes = off;
     return p;
 }
 
 // The look-up kernel or the sort and the direct GEMM: the predicted time of both in microseconds.  The look-up kernel walks K with one workgroup per 64
 // columns, in passes of up to four rows; where its table of scales does not fit LDS (small groups on a long K), every weight reads its
-// scale from memory.  The sorted way is five launches and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
+// scale from memory.  The sorted way is four launches and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
 // 20 matrices (512 x 512 .. 8192 x 28672, groups of 32 and 128) with 1 .. 16 rows: 9 .. 12 % off, and what it picks takes 0.4 % longer on average than
 // the faster of the two.  us, look-up / sorted: 14336 x 4096 4 bf16 rows 25 / 38, 6 rows 45 / 38, fp32 8 rows 41 / 40; 4096 x 4096 4 / 5 rows
 // 23 / 25, 35 / 25; 512 x 512 8 / 16 rows 11 / 14, 21 / 13; 4096 x 14336 one row 39 / 51, two 66 / 51; group 32 one row 182 / 57.
@@ -168,32 +186,44 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     return look_up > 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0);
 }
 
-hipError_t launch_gptq_order(const void* lhs, int lhs_dtype, const uint32_t* qweight, const int32_t* g_idx, int64_t m, int64_t n, int64_t k, int group,
-                             const GptqOrderSpace& p, hipStream_t s) {
+hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int64_t n, int64_t k, int group, const GptqOrderSpace& p, hipStream_t s) {
     const int groups = (int)(k / group);
     int bits = 0;
     while ((1 << bits) < groups) bits++;
-    hipError_t e = allow_full_lds<gptq_order_sort_kernel>();
-    if (e != hipSuccess) return e;
-    gptq_order_sort_kernel<<<dim3(1), dim3(64 * kSortWaves), (size_t)(kSortWaves * groups + 1) * 4, s>>>(g_idx, (int)k, group, bits, p.source, p.uneven);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    // columns per workgroup: the most (whole cache lines with 32) with which two workgroups fit a compute unit
-#define QMM_GO(AT, COLS)                                                                                                                                  \
-    do {                                                                                                                                                  \
-        const int per_xcd = (int)((n + 8 * COLS - 1) / (8 * COLS));                                                                                       \
-        if ((e = allow_full_lds<gptq_order_permute_kernel<AT, COLS>>()) != hipSuccess) return e;                                                          \
-        gptq_order_permute_kernel<AT, COLS><<<dim3((unsigned)(8 * per_xcd + m)), dim3(512), (size_t)k * COLS / 2, s>>>(                                    \
-            qweight, (const AT*)lhs, (int)n, (int)k, per_xcd, p.source, p.qweight, (AT*)p.lhs);                                                           \
+    const size_t sort_lds = 2 * k + (2 * kWaves * groups + 3) / 4 * 4;
+    auto words = [&](int cols) { return (size_t)(k / 2 * cols); };
+    // The widest slab that fits a compute unit (a row of 32 words is a whole cache line), narrower ones where those would not give every compute unit one.  us of the
+    // whole call, 32 / 16 / 8 / 4 columns: 14336 x 4096 400 rows 123 / 126 / 133 / 152, 8192 x 8192 300 rows 125 / 131 / 133 / 151, 4096 x 14336 64 rows - / 64 / 75 / 99,
+    // 4096 x 4096 64 rows 32.5 / 29.9 / 32.3 / 37.2, 1024 x 4096 20 rows 24.3 / 22.3 / 21.4 / 21.4.
+    int cols = 32;
+    while (cols > 8 && (words(cols) + sort_lds > kLdsPerCu || n < (int64_t)cols * compute_units())) cols /= 2;
+    const unsigned per_xcd = (unsigned)((n + 8 * cols - 1) / (8 * cols));
+    hipError_t e;
+#define QMM_GO(COLS, TURNS, WORDS, GRID, LDS)                                                                                                       \
+    do {                                                                                                                                            \
+        if ((e = allow_full_lds<gptq_order_permute_kernel<COLS, TURNS>>()) != hipSuccess) return e;                                                 \
+        gptq_order_permute_kernel<COLS, TURNS><<<dim3(GRID), dim3(kThreads), LDS, s>>>(WORDS, g_idx, (int)n, (int)k, group, bits, (int)per_xcd,     \
+                                                                                       p.source, p.uneven, p.qweight);                              \
     } while (0)
-#define QMM_GO_COLS(AT)                              \
-    do {                                             \
-        if (k <= kLdsPerCu / 32) QMM_GO(AT, 32);     \
-        else if (k <= kLdsPerCu / 16) QMM_GO(AT, 16); \
-        else QMM_GO(AT, 8);                          \
-    } while (0)
-    if (lhs_dtype == QMM_F32) QMM_GO_COLS(float);
-    else QMM_GO_COLS(uint16_t);
-#undef QMM_GO_COLS
+#define QMM_GO_WORDS(COLS, TURNS) QMM_GO(COLS, TURNS, qweight, 8 * per_xcd, words(COLS) + sort_lds)
+    if (words(cols) + sort_lds > kLdsPerCu) {
+        QMM_GO(8, 32, nullptr, 1, sort_lds);
+        QMM_GO(8, 0, qweight, 8 * per_xcd, words(8));
+    } else if (cols == 32) {  // (fits up to K = 9100)
+        if (k <= 4096) QMM_GO_WORDS(32, 4);
+        else if (k <= 8192) QMM_GO_WORDS(32, 8);
+        else QMM_GO_WORDS(32, 16);
+    } else if (cols == 16) {  // (up to K = 16380)
+        if (k <= 4096) QMM_GO_WORDS(16, 4);
+        else if (k <= 8192) QMM_GO_WORDS(16, 8);
+        else QMM_GO_WORDS(16, 16);
+    } else {
+        if (k <= 4096) QMM_GO_WORDS(8, 4);
+        else if (k <= 8192) QMM_GO_WORDS(8, 8);
+        else if (k <= 16384) QMM_GO_WORDS(8, 16);
+        else QMM_GO_WORDS(8, 32);
+    }
+#undef QMM_GO_WORDS
 #undef QMM_GO
     return hipGetLastError();
 }

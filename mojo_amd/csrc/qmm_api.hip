@@ -400,20 +400,15 @@ static int64_t required_bytes_flags(int encoding, int lhs_dtype, int64_t m, int6
 static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags);
 
 // Act-order GPTQ by sorted columns: the sorted tensors, then what the plain product on them needs.  0: not this way.
-static qmm_gptq_config plain_groups(qmm_gptq_config cfg) {
-    cfg.desc_act = 0;
-    return cfg;
-}
 // The sorted columns go to the direct GEMM whatever the number of rows: the small-batch kernel and the GEMM that unpacks tiles drop low bits of their
 // products.  Relative errors, look-up / small batch / tile GEMM / direct: 6400 x 1024 with 5 fp32 rows 1.6e-7 / 4.0e-7 / - / 1.1e-7, 14336 x 4096 with
-// 400 bf16 rows 2e-7 / - / 3e-6 / 7e-8 (the call takes 93 us with the tile GEMM, 103 with the direct one).  Matrices beyond what that
+// 400 bf16 rows 2e-7 / - / 3e-6 / 7e-8 (the call takes 10 us less with the tile GEMM).  Matrices beyond what that
 // takes (2^32 weights) stay with the look-up kernel.
-static bool order_direct() { return !qmm::kernel_disabled("direct"); }
 static int64_t order_bytes(const qmm_gptq_config& cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags) {
-    if (!cfg.desc_act || cfg.group_size <= 0 || k % cfg.group_size || (flags & ~QMM_FLAG_OUT_BF16) || !qmm::gptq_order_wanted(lhs_dtype, m, n, k, cfg.group_size) || n * k >= ((int64_t)1 << 32)) return 0;
-    const qmm_gptq_config plain = plain_groups(cfg);
-    return qmm::gptq_order_space(nullptr, lhs_dtype, m, n, k).bytes +
-           up256(order_direct() ? qmm::gemm_direct_workspace_bytes(QMM_GPTQ, lhs_dtype, m, k) : preferred_matmul(QMM_GPTQ, &plain, lhs_dtype, m, n, k, 0));
+    if (!cfg.desc_act || cfg.group_size <= 0 || k % cfg.group_size || (flags & ~QMM_FLAG_OUT_BF16) || qmm::kernel_disabled("direct") ||
+        !qmm::gptq_order_wanted(lhs_dtype, m, n, k, cfg.group_size) || n * k >= ((int64_t)1 << 32))
+        return 0;
+    return qmm::gptq_order_space(nullptr, n, k).bytes + up256(qmm::gemm_direct_workspace_bytes(QMM_GPTQ, lhs_dtype, m, k));
 }
 static bool order_serves(const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags, const void* workspace, int64_t workspace_bytes) {
     const int64_t need = order_bytes(*cfg, lhs_dtype, m, n, k, flags);
@@ -533,17 +528,13 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
                 return fail(QMM_ERR_INVALID, "qmm_matmul: GPTQ desc_act=True needs rhs[3] = g_idx int32[K]");
             const int32_t* only_if = nullptr;
             if (order_serves(cfg, lhs_dtype, m, n, k, flags, workspace, workspace_bytes)) {
-                const qmm::GptqOrderSpace p = qmm::gptq_order_space(workspace, lhs_dtype, m, n, k);
-                hipError_t e = qmm::launch_gptq_order(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const int32_t*)rhs[3], m, n, k, cfg->group_size, p, s);
+                const qmm::GptqOrderSpace p = qmm::gptq_order_space(workspace, n, k);
+                hipError_t e = qmm::launch_gptq_order((const uint32_t*)rhs[0], (const int32_t*)rhs[3], n, k, cfg->group_size, p, s);
                 if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, sort)");
-                const qmm_gptq_config plain = plain_groups(*cfg);
-                const void* sorted[3] = {p.qweight, rhs[1], rhs[2]};
-                if (order_direct()) {
-                    e = qmm::launch_gemm_direct(encoding, p.lhs, lhs_dtype, 1, sorted, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], cfg->group_size, m, k,
-                                                nullptr, (char*)workspace + p.bytes, s, true);
-                    if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, direct GEMM)");
-                } else if (int rc = matmul_f32(encoding, &plain, p.lhs, lhs_dtype, m, k, sorted, 3, n, out, (char*)workspace + p.bytes, workspace_bytes - p.bytes, flags, stream))
-                    return rc;
+                const void* sorted[1] = {p.qweight};
+                e = qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, sorted, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], cfg->group_size, m, k,
+                                            nullptr, (char*)workspace + p.bytes, s, true, p.source);
+                if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, direct GEMM)");
                 only_if = p.uneven;
             }
             hipError_t e = qmm::launch_gemv_gptq_act_order(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],

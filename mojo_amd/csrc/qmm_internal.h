@@ -24,12 +24,13 @@ int compute_units();
 
 // gemm_direct.hip: a few to a few hundred lhs rows, more where the staged kernel pays, every encoding; out16 != null: bf16 results (out is then unused).
 // any_rows: called with more rows than gemm_direct_wanted says, held to the error of the direct and shared kernels all the same.
+// source (GPTQ, K a multiple of 32): column p of the weights is column source[p] of the lhs.
 bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k);
 constexpr int kDirectMaxMats = 4;  // count: matrices that share the lhs (out16: one)
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
                               const uint16_t* scales, const uint32_t* qzeros, int group, int64_t m, int64_t k, uint16_t* out16, void* workspace,
-                              hipStream_t s, bool any_rows = false);
+                              hipStream_t s, bool any_rows = false, const int32_t* source = nullptr);
 
 hipError_t launch_read_probe(const void* buf, int64_t bytes, hipStream_t s);
 // register-resident matrix-core loop (probes.hip): `workgroups` workgroups of 8 wavefronts, out fp32 [workgroups * 512]
@@ -73,10 +74,11 @@ hipError_t launch_gemv_q4_k(const void* a, int a_dtype, const uint8_t* w, int m,
                             float* out, int64_t ldo, hipStream_t s);
 // Kernels that use more than 64 KB of dynamic LDS must say so once before their first launch: this raises the
 // kernel's limit to the 160 KB of a gfx950 compute unit, the first time it is called for the kernel.
+// STATIC: what the kernel has of it under names of its own.
 constexpr int kLdsPerCu = 160 * 1024;
-template <auto Kernel>
+template <auto Kernel, int STATIC = 0>
 inline hipError_t allow_full_lds() {
-    static const hipError_t st = hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
+    static const hipError_t st = hipFuncSetAttribute((const void*)Kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu - STATIC);
     return st;
 }
 
@@ -170,14 +172,12 @@ struct GptqOrderSpace {
     int32_t* uneven;
     int32_t* source;
     uint32_t* qweight;
-    void* lhs;
     int64_t bytes;
 };
-GptqOrderSpace gptq_order_space(void* workspace, int lhs_dtype, int64_t m, int64_t n, int64_t k);
+GptqOrderSpace gptq_order_space(void* workspace, int64_t n, int64_t k);
 bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
 bool gptq_act_order_table_fits(int64_t m, int64_t k, int group);  // the look-up kernel's scales in LDS
-hipError_t launch_gptq_order(const void* lhs, int lhs_dtype, const uint32_t* qweight, const int32_t* g_idx, int64_t m, int64_t n, int64_t k, int group,
-                             const GptqOrderSpace& p, hipStream_t s);
+hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int64_t n, int64_t k, int group, const GptqOrderSpace& p, hipStream_t s);
 bool gemv_q4_k_kc_supported(const void* w, int64_t k);
 int64_t gemv_q4_k_kc_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemv_q4_k_kc(const void* a, int a_dtype, const uint8_t* w, int m, int64_t n, int64_t k, float* out,

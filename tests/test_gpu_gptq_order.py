@@ -108,3 +108,17 @@ def test_replayed_from_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(got, qmatmul(QE.GPTQ, config, a, *rhs))
         assert not torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,k,group", [(8200, 4096, 128), (8200, 4128, 32), (8200, 8704, 128),  # slabs of 32 columns: 4, 8, 16 columns of K a lane
+                                       (4104, 4096, 512), (4104, 8192, 128), (4104, 14336, 128),  # of 16
+                                       (40, 16384, 128), (40, 18944, 128), (40, 26112, 128),  # of 8, up to where words and order fill a compute unit
+                                       (40, 26240, 128), (40, 28672, 32)])  # beyond: the sort as a launch of its own
+def test_slabs(n, k, group):
+    config, rhs = act_order(n, k, group, 3)
+    a = torch.randn((20, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(4)).bfloat16()
+    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns=True)
+    uneven = rhs[3].clone()
+    uneven[k - 1] = (uneven[k - 1] + 1) % (k // group)
+    rhs = (*rhs[:3], uneven)
+    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a)
