@@ -172,18 +172,18 @@ GptqOrderSpace gptq_order_space(void* workspace, int64_t n, int64_t k) {
 // The look-up kernel or the sort and the direct GEMM: the predicted time of both in microseconds.  The look-up kernel walks K with one workgroup per 64
 // columns, in passes of up to four rows; where its table of scales does not fit LDS (small groups on a long K), every weight reads its
 // scale from memory.  The sorted way is four launches and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
-// 20 matrices (512 x 512 .. 8192 x 28672, groups of 32 and 128) with 1 .. 16 rows: 9 .. 12 % off, and what it picks takes 0.4 % longer on average than
-// the faster of the two.  us, look-up / sorted: 14336 x 4096 4 bf16 rows 25 / 38, 6 rows 45 / 38, fp32 8 rows 41 / 40; 4096 x 4096 4 / 5 rows
-// 23 / 25, 35 / 25; 512 x 512 8 / 16 rows 11 / 14, 21 / 13; 4096 x 14336 one row 39 / 51, two 66 / 51; group 32 one row 182 / 57.
+// 15 matrices (512 x 512 .. 28672 x 8192, groups of 32 and 128, weights from memory) with 1 .. 12 rows; what it picks takes 0.2 % longer on average than the faster of
+// the two.  us, look-up / sorted: 14336 x 4096 4 bf16 rows 34 / 38, 5 rows 47 / 37, fp32 6 rows 39.6 / 40.1; 4096 x 4096 2 / 3 bf16 rows 27 / 22,
+// 32.5 / 21.6; 8192 x 8192 4 rows 62 / 42; 512 x 512 8 / 12 fp32 rows 9 / 12, 13.6 / 12.4; 1024 x 14336 one bf16 row 44 / 39, one fp32 row 43 / 45.
 bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
     if (k > 32768 || n % 8 || k % 32 || kernel_disabled("gptq_order")) return false;
     const bool f32 = lhs_dtype == QMM_F32;
     const double kk = k / 1024.0, w = (double)n * k / (1 << 20);
-    const double rows[4] = {0.0, 1.0, f32 ? 1.06 : 1.45, f32 ? 1.42 : 1.7};  // a pass of that many, over a pass of one
+    const double rows[4] = {0.0, 1.0, f32 ? 1.06 : 1.7, f32 ? 1.42 : 1.7};  // a pass of that many, over a pass of one
     double one = 1.9 + 2.75 * kk * std::max(1.0, n / (64.0 * compute_units())) + 0.06 * w;
     if (!gptq_act_order_table_fits(m, k, group)) one *= f32 ? 1.9 : 3.0;
     const double look_up = one * ((m / 4) * rows[3] + rows[std::min<int64_t>(m % 4, 3)]);
-    return look_up > 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0);
+    return look_up > 11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w;
 }
 
 hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int64_t n, int64_t k, int group, const GptqOrderSpace& p, hipStream_t s) {
