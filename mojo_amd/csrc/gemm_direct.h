@@ -46,8 +46,8 @@ hipError_t launch_gemm_shared(int encoding, bool hilo, const DirectPlan& pl, con
 hipError_t launch_gemm_staged(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
                               int64_t m, int units, hipStream_t s);
 
-// What gemm_staged.hip has: fp32 rows and small groups leave no registers for 128 rows a wavefront.
-constexpr bool staged_built(int encoding, int flush, int fm, bool hilo) { return fm <= 3 || !(hilo || (encoding == QMM_GPTQ && flush == 2)); }
+// What gemm_staged.hip has: fp32 rows, small groups and codes around their middle, which all sum a unit of K by itself, leave no registers for 128 rows a wavefront.
+constexpr bool staged_built(int encoding, int flush, int fm, bool hilo, bool centred) { return fm <= 3 || !(hilo || centred || (encoding == QMM_GPTQ && flush == 2)); }
 
 namespace {
 

@@ -576,8 +576,10 @@ int staged_row(int encoding, int group) {
     return encoding == QMM_Q4_K ? 0 : encoding == QMM_Q5_K ? 1 : encoding == QMM_Q6_K ? 2 : encoding == QMM_GPTQ ? (group % 128 == 0 ? 3 : 4) : -1;
 }
 double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56) * n * k * 1e-6; }
+// Codes around their middle: unit sums, and no plan with 128 rows a wavefront, which has no registers for them.
+bool staged_has(const StagedCost& c, int plan, bool centred) { return c.unit[plan] != 0.0f && !(centred && kStagedPlans[plan].fm == 4); }
 // The best of its plans whose parts of K are at most `longest` units; returns its time (1e30: there is none).
-double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, int64_t longest, DirectPlan& best) {
+double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, bool centred, int64_t longest, DirectPlan& best) {
     const int row = staged_row(encoding, group);
     if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
     const StagedCost& c = kStagedCost[row][lhs_dtype == QMM_F32 ? 1 : 0];
@@ -586,7 +588,7 @@ double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k,
         for (int i = 0; i < 7; i++) {
             const DirectPlan& p = kStagedPlans[i];
             const int64_t parts = p.wk * shares, walk = (direct_units(k) + parts - 1) / parts;
-            if (c.unit[i] == 0.0f || walk > longest) continue;
+            if (!staged_has(c, i, centred) || walk > longest) continue;
             const int64_t rounds = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, false).all;
             const double t = c.base + rounds * (c.round + walk * c.unit[i]) + c.weights * packed_mb(encoding, n, k) + c.lhs * (m * k * 1e-6) +
                              (c.out + c.share * (shares - 1)) * (m * n * 1e-6);
@@ -634,7 +636,7 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
         for (const DirectPlan& p : kStagedPlans) {
             const StagedCost& c = kStagedCost[staged_row(encoding, group)][type];
             const int i = (int)(&p - kStagedPlans);
-            if (c.unit[i] == 0.0f || p.wk != like->wk) continue;
+            if (!staged_has(c, i, like->centred) || p.wk != like->wk) continue;
             const int64_t walk = (direct_units(k) + p.wk * like->shares - 1) / (p.wk * like->shares);
             const double t = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * like->shares, false).all * (c.round + walk * c.unit[i]);
             if (t < us) us = t, best = p, best.shares = like->shares, best.centred = like->centred;
@@ -666,7 +668,7 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
     DirectPlan p;
     // (4 %: as far as the predictions are off; within it the staged kernel was slower as often as faster, GPTQ 4552 x 3072 472 fp32 rows 55.7 and 56.4 us predicted,
     // 61 and 56 taken; codes around the middle are not in its figures)
-    if (staged_plan(encoding, lhs_dtype, m, n, k, group, whole_tiles, chain, p) * (centred && type == 0 ? 1.08 : 1.04) < us) {
+    if (staged_plan(encoding, lhs_dtype, m, n, k, group, whole_tiles, centred, chain, p) * (centred && type == 0 ? 1.08 : 1.04) < us) {
         best = p;
         best.centred = centred;
     }
@@ -753,7 +755,7 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     if (f32 && k < 768 && (encoding == QMM_GPTQ || encoding == QMM_Q6_K)) return false;
     const float(&o)[5] = kStagedCost[row][f32 ? 1 : 0].other;
     DirectPlan p;
-    return staged_plan(encoding, lhs_dtype, m, n, k, group, false, 1 << 20, p) <
+    return staged_plan(encoding, lhs_dtype, m, n, k, group, false, false, 1 << 20, p) <
            (f32 || m <= 1024 ? 0.95 : 0.9) * (o[0] + o[1] * packed_mb(encoding, n, k) + o[2] * (m * k * 1e-6) + o[3] * (m * n * 1e-6) + o[4] * (1e-9 * ((m + 255) / 256 * 256) * n * k));
 }
 

@@ -284,9 +284,9 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTens
     const int u0 = (units * part) >> log_parts, u1 = (units * (part + 1)) >> log_parts;
 
     // (the offsets of a unit first join its products, as in the direct and shared kernels: with two additions to T a unit instead of one, Q4_K with fp32 rows was
-    // off by 2.30e-7 instead of 2.04e-7 after sums of 40 units, Q5_K with bf16 rows by 1.06e-7 instead of 0.99e-7; for codes from 0, and for 128 rows, which have
-    // no registers for it, the error is that of larger terms)
-    constexpr bool kUnit = unit_sums(ENC, FLUSH, HILO) || (W::kMin && (HILO || (CENTER && FM < 4)));
+    // off by 2.30e-7 instead of 2.04e-7 after sums of 40 units, Q5_K with bf16 rows by 1.06e-7 instead of 0.99e-7; for codes from 0 the error is that of larger
+    // terms.  Never a question of FM: matrices that share a launch share its tile, and keep the bits that calls of their own give.)
+    constexpr bool kUnit = unit_sums(ENC, FLUSH, HILO) || (W::kMin && (HILO || CENTER));
     float16v T[FM], P[FM], M, U[kUnit ? FM : 1];
 #pragma unroll
     for (int a = 0; a < FM; a++)
@@ -477,7 +477,7 @@ hipError_t run_staged(const WeightTensors& wt, DirectMats mats, const DirectSpac
 template <int ENC, int FLUSH, bool HILO, bool CENTER = false>
 hipError_t run_staged_plan(const DirectPlan& pl, const WeightTensors& wt, const DirectMats& mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units, hipStream_t s) {
 #define QMM_GS(FM, WN, WK)                       \
-    if constexpr (staged_built(ENC, FLUSH, FM, HILO)) \
+    if constexpr (staged_built(ENC, FLUSH, FM, HILO, CENTER)) \
         if (pl.fm == FM && pl.wn == WN && pl.wk == WK) return run_staged<ENC, FLUSH, FM, WN, WK, HILO, CENTER>(wt, mats, p, out16, m, units, pl.shares, s)
     QMM_GS(2, 2, 4);
     QMM_GS(2, 4, 2);

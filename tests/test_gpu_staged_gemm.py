@@ -63,6 +63,16 @@ def test_matrices_together_sum_as_alone():
                 assert torch.equal(got, qmatmul(enc, None, a, w))
 
 
+@pytest.mark.parametrize("enc,m,n,count,k", [(QE.Q4_K, 385, 5120, 3, 4096), (QE.Q5_K, 193, 5120, 3, 4096), (QE.Q4_K, 228, 5632, 2, 1024), (QE.Q4_K, 540, 4096, 3, 1024)])
+def test_a_tile_for_several_matrices_keeps_their_sums(enc, m, n, count, k):
+    """Sizes at which matrices together would take 128 rows a wavefront where each alone takes 64 or 96, with codes around their middle."""
+    w = weights(enc, 0, n, k)[1][0]
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).bfloat16()
+    alone = qmatmul(enc, None, a, w)
+    for got in qmatmul_grouped(enc, a, [w] * count):
+        assert torch.equal(got, alone)
+
+
 # Relative error of (enc, group, rows, n, k, lhs): the float32 sums of the kernel that served the call before, by 1.08
 @pytest.mark.parametrize("enc,group,m,n,k,lhs,most", [
     (QE.Q4_K, 0, 96, 4096, 4096, torch.bfloat16, 1.06e-7), (QE.Q4_K, 0, 200, 14336, 4096, torch.bfloat16, 2.2e-7), (QE.Q4_K, 0, 200, 4096, 4096, torch.float32, 2.04e-7),
