@@ -576,23 +576,58 @@ int staged_row(int encoding, int group) {
     return encoding == QMM_Q4_K ? 0 : encoding == QMM_Q5_K ? 1 : encoding == QMM_Q6_K ? 2 : encoding == QMM_GPTQ ? (group % 128 == 0 ? 3 : 4) : -1;
 }
 double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56) * n * k * 1e-6; }
+// What a plan's fp32 sums cost: the square of the relative error of the results (2-norm, against 64 bits) in units of 2^-48 / 6, the mean square of a rounding
+// halved.  An addition counts by the share of K that its sum holds by then: `unit` times half the squares of the parts' lengths, `join` for adding the parts up
+// in order; `first`: additions to zero, which are exact.  Fitted to every plan on 22 K of 256 .. 28672 (profiles/relative_error_by_plan.txt): mean of 0.05 .. 0.8 %
+// off by encoding, lhs type and kind of sums; beyond K = 14336 up to 4 % with the K-quants.
+struct SumsError {
+    float base, unit, join, first;
+};
+constexpr SumsError kSumsError[5][2][3] = {
+    // the direct kernel; the shared and the staged one, codes from 0 (fp32 rows: around their middle); bf16 rows, codes around their middle
+    {{{2.1f, 9.85f, 1.2f, 0.3f}, {53.67f, 2.18f, 0.95f, 0.39f}, {7.9f, 1.21f, 1.37f, -1.64f}}, {{37.3f, 10.02f, 1.27f, -0.1f}, {43.27f, 1.41f, 1.99f, -2.5f}, {43.27f, 1.41f, 1.99f, -2.5f}}},  // Q4_K
+    {{{4.81f, 9.83f, 1.19f, 0.24f}, {72.94f, 2.19f, 0.92f, 0.46f}, {10.55f, 1.2f, 1.36f, -1.65f}}, {{38.99f, 10.04f, 1.28f, -0.1f}, {44.98f, 1.4f, 1.97f, -2.47f}, {44.98f, 1.4f, 1.97f, -2.47f}}},  // Q5_K
+    {{{8.17f, 2.21f, 1.19f, 0.14f}, {16.13f, 1.08f, 1.25f, 0.03f}, {}}, {{36.44f, 2.19f, 1.18f, 0.06f}, {65.72f, 1.08f, 1.21f, 0.15f}, {}}},  // Q6_K
+    {{{0.65f, 2.17f, 1.23f, 0.01f}, {0.65f, 2.17f, 1.23f, 0.01f}, {}}, {{17.37f, 2.19f, 1.25f, -0.08f}, {17.37f, 2.19f, 1.25f, -0.08f}, {}}},  // GPTQ, groups of 128
+    {{{5.93f, 1.14f, 1.21f, -1.48f}, {5.93f, 1.14f, 1.21f, -1.48f}, {}}, {{8.43f, 8.68f, 1.24f, -0.01f}, {8.43f, 8.68f, 1.24f, -0.01f}, {}}},  // GPTQ, other groups
+};
+double sums_error(const SumsError& e, const DirectPlan& p, int64_t units) {
+    const int log_parts = __builtin_ctz((unsigned)(p.wk * p.shares));
+    double squares = 0.0, join = 0.0;
+    int held_parts = 0;
+    for (int s = 0; s < p.shares; s++) {
+        int64_t held = 0;  // units in the sum of this workgroup
+        for (int i = s * p.wk; i < (s + 1) * p.wk; i++) {
+            const int64_t q = (units * (i + 1) >> log_parts) - (units * i >> log_parts);
+            if (q == 0) continue;
+            squares += (double)(q * q), held_parts++;
+            if (held > 0) join += (double)(held + q);
+            held += q;
+        }
+        if (s == 1 && held < units) join += (double)units;
+    }
+    return e.base + (e.unit * 0.5 * squares + e.join * join + e.first * held_parts) / (double)units;
+}
 // Codes around their middle: unit sums, and no plan with 128 rows a wavefront, which has no registers for them.
 bool staged_has(const StagedCost& c, int plan, bool centred) { return c.unit[plan] != 0.0f && !(centred && kStagedPlans[plan].fm == 4); }
-// The best of its plans whose parts of K are at most `longest` units; returns its time (1e30: there is none).
-double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, bool centred, int64_t longest, DirectPlan& best) {
+// The best of its plans whose parts of K are at most `longest` units and whose sums are off by no more than `most` (sums_error); returns its time (1e30: there is none).
+double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, bool centred, int64_t longest, double most, DirectPlan& best) {
     const int row = staged_row(encoding, group);
     if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
-    const StagedCost& c = kStagedCost[row][lhs_dtype == QMM_F32 ? 1 : 0];
+    const int type = lhs_dtype == QMM_F32 ? 1 : 0;
+    const StagedCost& c = kStagedCost[row][type];
+    const SumsError& e = kSumsError[row][type][centred ? 2 : 1];
     double us = 1e30;
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++)
         for (int i = 0; i < 7; i++) {
-            const DirectPlan& p = kStagedPlans[i];
+            DirectPlan p = kStagedPlans[i];
+            p.shares = shares;
             const int64_t parts = p.wk * shares, walk = (direct_units(k) + parts - 1) / parts;
             if (!staged_has(c, i, centred) || walk > longest) continue;
             const int64_t rounds = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, false).all;
             const double t = c.base + rounds * (c.round + walk * c.unit[i]) + c.weights * packed_mb(encoding, n, k) + c.lhs * (m * k * 1e-6) +
                              (c.out + c.share * (shares - 1)) * (m * n * 1e-6);
-            if (t < us) us = t, best = p, best.shares = shares;
+            if (t < us && sums_error(e, p, direct_units(k)) <= most) us = t, best = p;
         }
     return us;
 }
@@ -656,19 +691,20 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
                 consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (i == 2 ? 1.03 : 1.0));
     }
     if (like || !staged || (encoding == QMM_Q6_K && !beyond && (m <= 64 || best.wn == 1))) return best;
-    // The staged kernel, held to the error of what it replaces: sums no longer than those of that plan (a part of K is one chain of fp32 sums), and where that is
-    // the direct kernel the codes of Q4_K and Q5_K around their middle (KQuantWeights), as there; Q6_K, whose sums leave the matrix cores half as often as in the direct
-    // kernel, only for the shared one.  Beyond the range of those two anything is more exact than the GEMMs that share unpacked weights (2.2e-7 .. 3.5e-6).
+    // The staged kernel, held to the error of what it replaces (sums_error), and where that is the direct kernel with the codes of Q4_K and Q5_K around their
+    // middle (KQuantWeights), as there; Q6_K, whose sums leave the matrix cores half as often as in the direct kernel, only for the shared one.
+    // Beyond the range of those two anything is more exact than the GEMMs that share unpacked weights (2.2e-7 .. 3.5e-6).
     const bool k_quant = encoding == QMM_Q4_K || encoding == QMM_Q5_K;
     const bool centred = k_quant && (type == 1 || (!beyond && best.wn == 1) || (encoding == QMM_Q5_K && m <= 64));
-    // K-quants with fp32 rows grow less with it here and in the shared kernel (relative error after 1, 3, 4 units in the direct kernel 1.63e-7, 1.80e-7, 1.89e-7; here
-    // after 4, 16, 24, 40 1.64e-7, 1.78e-7, 1.87e-7, 2.04e-7).
+    // As far as parts of K longer than those of that plan have been tried.
     const int64_t parts = best.wk * best.shares, part = (direct_units(k) + parts - 1) / parts;
     const int64_t chain = beyond ? 1 << 20 : std::max<int64_t>(4, k_quant && type == 1 && best.wn == 1 && part > 1 ? 5 * part : part);
+    const int errors = staged_row(encoding, group);
+    const double most = beyond || errors < 0 ? 1e30 : sums_error(kSumsError[errors][type][best.wn == 1 ? 0 : centred ? 2 : 1], best, direct_units(k));
     DirectPlan p;
     // (4 %: as far as the predictions are off; within it the staged kernel was slower as often as faster, GPTQ 4552 x 3072 472 fp32 rows 55.7 and 56.4 us predicted,
     // 61 and 56 taken; codes around the middle are not in its figures)
-    if (staged_plan(encoding, lhs_dtype, m, n, k, group, whole_tiles, centred, chain, p) * (centred && type == 0 ? 1.08 : 1.04) < us) {
+    if (staged_plan(encoding, lhs_dtype, m, n, k, group, whole_tiles, centred, chain, most, p) * (centred && type == 0 ? 1.08 : 1.04) < us) {
         best = p;
         best.centred = centred;
     }
@@ -755,7 +791,7 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     if (f32 && k < 768 && (encoding == QMM_GPTQ || encoding == QMM_Q6_K)) return false;
     const float(&o)[5] = kStagedCost[row][f32 ? 1 : 0].other;
     DirectPlan p;
-    return staged_plan(encoding, lhs_dtype, m, n, k, group, false, false, 1 << 20, p) <
+    return staged_plan(encoding, lhs_dtype, m, n, k, group, false, false, 1 << 20, 1e30, p) <
            (f32 || m <= 1024 ? 0.95 : 0.9) * (o[0] + o[1] * packed_mb(encoding, n, k) + o[2] * (m * k * 1e-6) + o[3] * (m * n * 1e-6) + o[4] * (1e-9 * ((m + 255) / 256 * 256) * n * k));
 }
 
