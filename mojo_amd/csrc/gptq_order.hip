@@ -32,8 +32,8 @@ constexpr int kWaves = 16, kThreads = 64 * kWaves;
 // Stable sort (within a group the columns keep their order), wavefront w takes a sixteenth of K, TURNS times 64 columns; group indices outside [0, groups) are
 // clamped, as in the look-up kernel.  The first workgroup leaves the order (source[p]: the column of K at sorted position p) and the mark in memory.
 // LDS: [k / 8][COLS] words, uint16 [k] order, uint16 [kWaves][groups] counts.
-// Where that is more than a compute unit has (K beyond 26208, less with groups of 32 or 64): a launch of one workgroup without words (qweight null) that only sorts, then TURNS = 0, which
-// takes the order from memory.
+// Where that is more than a compute unit has (K beyond 26208, less with groups of 32 or 64), or leaves room for one workgroup and there are several for each compute unit: a launch of
+// one workgroup without words (qweight null) that only sorts, then TURNS = 0, which takes the order from memory.
 template <int COLS, int TURNS>
 __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_permute_kernel(const uint32_t* __restrict__ qweight, const int32_t* __restrict__ g_idx, int n,
                                                                                           int k, int group, int bits, int per_xcd, int32_t* __restrict__ source,
@@ -192,11 +192,17 @@ hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int6
     while ((1 << bits) < groups) bits++;
     const size_t sort_lds = 2 * k + (2 * kWaves * groups + 3) / 4 * 4;
     auto words = [&](int cols) { return (size_t)(k / 2 * cols); };
-    // The widest slab that fits a compute unit (a row of 32 words is a whole cache line), narrower ones where those would not give every compute unit one.  us of the
+    // The widest slab that fits a compute unit (a row of 32 words is a whole cache line), narrower ones where those still are no more than one for each.  us of the
     // whole call, 32 / 16 / 8 / 4 columns: 14336 x 4096 400 rows 123 / 126 / 133 / 152, 8192 x 8192 300 rows 125 / 131 / 133 / 151, 4096 x 14336 64 rows - / 64 / 75 / 99,
-    // 4096 x 4096 64 rows 32.5 / 29.9 / 32.3 / 37.2, 1024 x 4096 20 rows 24.3 / 22.3 / 21.4 / 21.4.
+    // 4096 x 4096 64 rows 32.5 / 29.9 / 32.3 / 37.2, 1024 x 4096 20 rows 24.3 / 22.3 / 21.4 / 21.4; 12 rows 6144 x 8192 42.6 / 49.2 / 48.2, 2560 x 9088 - / 41.3 / 48.4.
     int cols = 32;
-    while (cols > 8 && (words(cols) + sort_lds > kLdsPerCu || n < (int64_t)cols * compute_units())) cols /= 2;
+    while (cols > 8 && (words(cols) + sort_lds > kLdsPerCu || n <= (int64_t)cols / 2 * compute_units())) cols /= 2;
+    // Several slabs for each compute unit, of which it holds one with the order: nothing is asked for while one is being sorted and permuted.  Without the order two
+    // fit.  us, 12 rows, one launch / two: 28672 x 16384 393 / 261, 11008 x 18944 205 / 139, 14336 x 9088 97 / 81, 28672 x 8192 127 / 117, 14336 x 8192 72.5 / 73.4;
+    // with one slab for each the other way round: 4096 x 14336 54 / 60 (and up to one and a half of 32 columns: 11008 x 5120 49.4 / 51.3).
+    const bool sort_apart = words(cols) + sort_lds > kLdsPerCu ||
+                            (2 * (words(cols) + sort_lds) > kLdsPerCu && n > (int64_t)(cols == 32 ? 48 : cols) * compute_units());
+    if (sort_apart) cols = k <= 5120 ? 32 : k <= 20480 ? 16 : 8;  // (32 up to where two fit, 28672 x 5120 32 / 16 columns 78.5 / 80.4; 16 up to where one does, 14336 x 20480 16 / 8 165 / 175)
     const unsigned per_xcd = (unsigned)((n + 8 * cols - 1) / (8 * cols));
     hipError_t e;
 #define QMM_GO(COLS, TURNS, WORDS, GRID, LDS)                                                                                                       \
@@ -206,9 +212,11 @@ hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int6
                                                                                        p.source, p.uneven, p.qweight);                              \
     } while (0)
 #define QMM_GO_WORDS(COLS, TURNS) QMM_GO(COLS, TURNS, qweight, 8 * per_xcd, words(COLS) + sort_lds)
-    if (words(cols) + sort_lds > kLdsPerCu) {
+    if (sort_apart) {
         QMM_GO(8, 32, nullptr, 1, sort_lds);
-        QMM_GO(8, 0, qweight, 8 * per_xcd, words(8));
+        if (cols == 32) QMM_GO(32, 0, qweight, 8 * per_xcd, words(32));
+        else if (cols == 16) QMM_GO(16, 0, qweight, 8 * per_xcd, words(16));
+        else QMM_GO(8, 0, qweight, 8 * per_xcd, words(8));
     } else if (cols == 32) {  // (fits up to K = 9100)
         if (k <= 4096) QMM_GO_WORDS(32, 4);
         else if (k <= 8192) QMM_GO_WORDS(32, 8);

@@ -122,3 +122,16 @@ def test_slabs(n, k, group):
     uneven[k - 1] = (uneven[k - 1] + 1) % (k // group)
     rhs = (*rhs[:3], uneven)
     check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a)
+
+
+@pytest.mark.parametrize("n,k,group", [(12296, 5120, 128), (12296, 4608, 32),  # slabs of 32 columns
+                                       (12296, 8704, 128), (4104, 9120, 32), (4104, 16384, 128), (2056, 20480, 64),  # of 16
+                                       (2056, 20608, 128), (2056, 28672, 32)])  # of 8
+def test_slabs_with_the_sort_apart(n, k, group):
+    """More slabs than compute units, each with its order too large for two to a compute unit."""
+    test_slabs(n, k, group)
+
+
+@pytest.mark.parametrize("n,k,group", [(4104, 8704, 128), (4104, 4096, 128), (2056, 9088, 128)])  # the widest slabs of which there is one for each compute unit
+def test_one_slab_a_compute_unit(n, k, group):
+    test_slabs(n, k, group)
