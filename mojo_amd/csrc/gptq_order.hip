@@ -183,7 +183,10 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     double one = 1.9 + 2.75 * kk * std::max(1.0, n / (64.0 * compute_units())) + 0.06 * w;
     if (!gptq_act_order_table_fits(m, k, group)) one *= f32 ? 1.9 : 3.0;
     const double look_up = one * ((m / 4) * rows[3] + rows[std::min<int64_t>(m % 4, 3)]);
-    return look_up > 11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w;
+    // Beyond some 60 M weights that line finds the look-up kernel ahead with one row more or two, but there it is two to four times further off: the second line, from when
+    // the sort was a launch of its own.  Relative error, us, look-up / sorted: 5504 x 18944 4 fp32 rows 5.7e-7 / 1.3e-7, 100 / 92; 18944 x 4096 6 rows 2.8e-7 / 1.2e-7,
+    // 71 / 56; groups of 32, 11648 x 12032 2 rows 4.7e-7 / 1.5e-7, 84 / 100; 32000 x 28672 4 bf16 rows 6.1e-7 / 1.4e-7, 420 / 483.
+    return look_up > std::min(11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w, 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0));
 }
 
 hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int64_t n, int64_t k, int group, const GptqOrderSpace& p, hipStream_t s) {

@@ -77,6 +77,14 @@ def test_few_rows_keep_their_fp32_precision(m, n, k):
     check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns=True)
 
 
+@pytest.mark.parametrize("m,n,k,group", [(6, 18944, 4096, 128), (4, 5504, 18944, 128), (2, 11648, 12032, 32), (5, 16472, 7936, 32)])
+def test_few_rows_of_large_matrices_keep_their_precision(m, n, k, group):
+    """The look-up kernel, which walks K in one chain a wavefront, is up to four times further off there."""
+    config, rhs = act_order(n, k, group, m, any_codes=False)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m))
+    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns=True)
+
+
 @pytest.mark.parametrize("change", ["one column", "one group empty", "out of range"])
 def test_uneven_groups(change):
     m, n, k, group = 37, 264, 2048, 128
