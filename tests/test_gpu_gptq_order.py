@@ -77,12 +77,17 @@ def test_few_rows_keep_their_fp32_precision(m, n, k):
     check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns=True)
 
 
-@pytest.mark.parametrize("m,n,k,group", [(6, 18944, 4096, 128), (4, 5504, 18944, 128), (2, 11648, 12032, 32), (5, 16472, 7936, 32)])
-def test_few_rows_of_large_matrices_keep_their_precision(m, n, k, group):
-    """The look-up kernel, which walks K in one chain a wavefront, is up to four times further off there."""
+# Relative error (2-norm, against float64) of the sorted columns, a tenth above what they have; the look-up kernel's in the comment
+@pytest.mark.parametrize("m,n,k,group,most", [(6, 18944, 4096, 128, 1.34e-7),  # 2.75e-7
+                                              (4, 5504, 18944, 128, 1.46e-7),  # 5.7e-7
+                                              (2, 11648, 12032, 32, 1.67e-7),  # 4.7e-7
+                                              (5, 16472, 7936, 32, 1.3e-7)])   # 3.8e-7
+def test_few_rows_of_large_matrices_keep_their_precision(m, n, k, group, most):
     config, rhs = act_order(n, k, group, m, any_codes=False)
     a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m))
-    check(qmatmul(QE.GPTQ, config, a, *rhs), config, rhs, a, sorted_columns=True)
+    want = a.double() @ dequantize(QE.GPTQ, *rhs, config=config).double().T
+    error = ((qmatmul(QE.GPTQ, config, a, *rhs).double() - want).norm() / want.norm()).item()
+    assert error <= most, error
 
 
 @pytest.mark.parametrize("change", ["one column", "one group empty", "out of range"])
