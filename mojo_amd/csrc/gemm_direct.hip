@@ -808,13 +808,11 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
     const bool q40 = encoding == QMM_Q4_0, f32 = lhs_dtype == QMM_F32, sums = encoding == QMM_Q4_K || encoding == QMM_Q5_K || q40;
     if (count < 1 || count > kDirectMaxMats) return hipErrorInvalidValue;
     const DirectSpace p = direct_space(workspace, f32 && !q40, sums, sums && !q40, m, k);
-    // (loads of 16 bytes straight to LDS, of 4 for the scales and zeros of GPTQ)
-    bool staged = (((uintptr_t)scales | (uintptr_t)qzeros) & 3) == 0;
-    for (int j = 0; j < count; j++) staged = staged && ((uintptr_t)ws[j] & 15) == 0;
     DirectPlan plans[kDirectMaxMats];
     DirectMats zero{};
     int64_t zeros = 0;
     for (int j = 0; j < count; j++) {
+        const bool staged = ((uintptr_t)ws[j] & 3) == 0;  // (what loads to LDS want; scales and zeros of GPTQ lie so, Q6_K may not)
         plans[j] = direct_plan(encoding, lhs_dtype, m, ns[j], k, group, out16 != nullptr, staged, !any_rows && !direct_range(encoding, lhs_dtype, m, ns[j], k, group));
         if (plans[j].shares > 1) zero.out[zero.count] = outs[j], zero.n[zero.count++] = (int)ns[j], zeros = std::max(zeros, m * ns[j]);
     }
@@ -854,7 +852,7 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
             n += ns[i];
             done[i] = true;
         }
-        if (mats.count > 1) pl = direct_plan(encoding, lhs_dtype, m, n, k, group, false, staged, false, &pl);
+        if (mats.count > 1) pl = direct_plan(encoding, lhs_dtype, m, n, k, group, false, true, false, &pl);
         if (pl.fn == 0) {
             e = launch_gemm_staged(encoding, f32 && !q40, pl, wt, mats, p, out16, m, units, s);
             continue;

@@ -48,7 +48,7 @@ struct StagedK : KQuantWeights<ENC, 1, CENTER> {
     }
 };
 
-// GPTQ, plain groups, K a multiple of 256 (the packed words of a unit: 32 rows), 16-byte aligned qweight.  FLUSH as for GptqWeights.
+// GPTQ, plain groups, K a multiple of 256 (the packed words of a unit: 32 rows).  FLUSH as for GptqWeights.
 template <int FLUSH>
 struct StagedGptq : NoOffsets {
     static constexpr int kSteps = 16, kFlush = FLUSH, kPlanes = 1;
@@ -126,7 +126,7 @@ struct StagedGptq : NoOffsets {
     __device__ __forceinline__ float scale_at() const { return h2f((uint16_t)s_raw[I]); }
 };
 
-// Q6_K: blocks of 210 bytes lie at even addresses, loads to LDS want multiples of four: a row's 212 bytes from the last such address on, 208 of them in pieces
+// Q6_K in a tensor that begins at a multiple of four: blocks of 210 bytes lie at even addresses, loads to LDS want multiples of four: a row's 212 bytes from the last such address on, 208 of them in pieces
 // of 16, the last four apart.  The fields begin `skew` (0 or 2) bytes later, other in every row and unit.
 template <int FLUSH>
 struct StagedQ6 : Q6Weights<1, FLUSH> {

@@ -21,8 +21,9 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_space_ptr)p);
 }
 
-// 16 bytes per lane from global memory to LDS at lds_base + 16 * lane (lds_base uniform).  m0 is put
-// back; the s_nop is the wait state the hardware wants between a write of m0 and an LDS-direct load.
+// 16 bytes per lane from global memory to LDS at lds_base + 16 * lane (lds_base uniform, a multiple of
+// 16).  The global address may be any multiple of four: GPTQ words (gptq_order.hip, gemm_staged.hip) and
+// Q6_K blocks (gemm_staged.hip) begin at every one of them.  m0 is put back; the s_nop is the wait state the hardware wants between a write of m0 and an LDS-direct load.
 __device__ __forceinline__ void load16_to_lds(const void* g, uint32_t lds_base) {
     uint32_t keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"

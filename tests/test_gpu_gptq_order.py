@@ -148,3 +148,16 @@ def test_slabs_with_the_sort_apart(n, k, group):
 @pytest.mark.parametrize("n,k,group", [(4104, 8704, 128), (4104, 4096, 128), (2056, 9088, 128)])  # the widest slabs of which there is one for each compute unit
 def test_one_slab_a_compute_unit(n, k, group):
     test_slabs(n, k, group)
+
+
+@pytest.mark.parametrize("n,k", [(8200, 4096), (4104, 4096), (40, 16384), (2056, 20608)])  # slabs of 32, 16, 8 columns, the sort apart
+@pytest.mark.parametrize("words", [1, 2, 3])
+def test_qweight_at_any_multiple_of_four(n, k, words):
+    config, rhs = act_order(n, k, 128, 3)
+    a = torch.randn((20, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(4)).bfloat16()
+    moved = torch.empty(rhs[0].numel() + words, dtype=torch.int32, device="cuda")[words:].view(rhs[0].shape)
+    moved.copy_(rhs[0])
+    assert moved.data_ptr() % 16 == 4 * words
+    got = qmatmul(QE.GPTQ, config, a, moved, *rhs[1:])
+    check(got, config, rhs, a, sorted_columns=True)
+    assert torch.equal(got, qmatmul(QE.GPTQ, config, a, *rhs))

@@ -37,7 +37,7 @@ def test_odd_columns(n):
 
 
 def test_misaligned_gptq_words():
-    """qweight may lie at any multiple of four bytes; loads of 16 bytes to LDS want sixteen, so those calls stay with the kernels before."""
+    """qweight may lie at any multiple of four bytes, which is what loads of 16 bytes to LDS want."""
     config, rhs = weights(QE.GPTQ, 128, 14336, 1024)
     a = torch.randn((200, 1024), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)).bfloat16()
     words = torch.empty(rhs[0].numel() + 1, dtype=torch.int32, device="cuda")
@@ -51,6 +51,17 @@ def test_misaligned_gptq_words():
     assert lib.qmm_matmul(QE.GPTQ.code, cfg, a.data_ptr(), _lib.QMM_BF16, 200, 1024, ptrs, 3, 14336, out.data_ptr(), ws.data_ptr(), need, 0,
                           torch.cuda.current_stream().cuda_stream) == 0
     check(out, QE.GPTQ, config, moved, a)
+
+
+@pytest.mark.parametrize("group,m,n,k", [(128, 200, 14336, 1024), (32, 200, 14336, 1024), (128, 1000, 14336, 4096), (128, 161, 14344, 1280)])
+@pytest.mark.parametrize("words", [1, 2, 3])
+def test_misaligned_gptq_words_give_the_same_bits(group, m, n, k, words):
+    config, rhs = weights(QE.GPTQ, group, n, k)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).bfloat16()
+    moved = torch.empty(rhs[0].numel() + words, dtype=torch.int32, device="cuda")[words:].view(rhs[0].shape)
+    moved.copy_(rhs[0])
+    assert moved.data_ptr() % 16 == 4 * words
+    assert torch.equal(qmatmul(QE.GPTQ, config, a, moved, *rhs[1:]), qmatmul(QE.GPTQ, config, a, *rhs))
 
 
 def test_matrices_together_sum_as_alone():
