@@ -610,6 +610,8 @@ double sums_error(const SumsError& e, const DirectPlan& p, int64_t units) {
 }
 // Codes around their middle: unit sums, and no plan with 128 rows a wavefront, which has no registers for them.
 bool staged_has(const StagedCost& c, int plan, bool centred) { return c.unit[plan] != 0.0f && !(centred && kStagedPlans[plan].fm == 4); }
+// What loads to LDS want.  Scales and zeros of GPTQ lie so; only a Q6_K tensor may begin elsewhere.
+bool staged_takes(const void* w) { return ((uintptr_t)w & 3) == 0; }
 // The best of its plans whose parts of K are at most `longest` units and whose sums are off by no more than `most` (sums_error); returns its time (1e30: there is none).
 double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, bool centred, int64_t longest, double most, DirectPlan& best) {
     const int row = staged_row(encoding, group);
@@ -742,7 +744,7 @@ hipError_t run_direct_plan(const DirectPlan& pl, const WeightTensors& wt, const 
 
 }  // namespace
 
-bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
+bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, const void* w_at) {
     if (kernel_disabled("direct") || k % (encoding == QMM_GPTQ || encoding == QMM_Q4_0 ? 32 : 256) || n * k >= ((int64_t)1 << 32)) return false;
     if (encoding == QMM_GPTQ && (n % 8 || group % 32)) return false;
     // Served from `from` rows on, where this kernel's time crosses that of the small-batch kernels (passes of four to sixteen rows over
@@ -785,7 +787,7 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     // 294 / 258; Q5_K 32000 x 4096 200 rows 165 / 82; Q4_K 14336 x 4096 1300 fp32 rows 506 / 347.  With many bf16 rows on many columns those run at their best,
     // 256 x 256 results at a time, which the figures of `other` do not know (14336 x 4096 2048 rows 260 / 281, 5120 x 5120 2500 rows 163 / 191, 4096 x 4096 3000 rows 126 / 135).
     const int row = staged_row(encoding, group);
-    if (row < 0 || (!f32 && m > 1600 && (n > 4096 || (m > 2048 && k <= 8192)))) return false;
+    if (row < 0 || !staged_takes(w_at) || (!f32 && m > 1600 && (n > 4096 || (m > 2048 && k <= 8192)))) return false;
     // On a short K those are the more exact ones for fp32 rows (relative error, those / here: GPTQ K = 256 7.6e-8 / 1.0e-7, 512 9.7e-8 / 1.1e-7, 768 1.1e-7 / 1.1e-7; Q6_K
     // 1.4e-7 / 2.0e-7, 1.8e-7 / 2.0e-7, 2.3e-7 / 2.0e-7).
     if (f32 && k < 768 && (encoding == QMM_GPTQ || encoding == QMM_Q6_K)) return false;
@@ -812,8 +814,7 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
     DirectMats zero{};
     int64_t zeros = 0;
     for (int j = 0; j < count; j++) {
-        const bool staged = ((uintptr_t)ws[j] & 3) == 0;  // (what loads to LDS want; scales and zeros of GPTQ lie so, Q6_K may not)
-        plans[j] = direct_plan(encoding, lhs_dtype, m, ns[j], k, group, out16 != nullptr, staged, !any_rows && !direct_range(encoding, lhs_dtype, m, ns[j], k, group));
+        plans[j] = direct_plan(encoding, lhs_dtype, m, ns[j], k, group, out16 != nullptr, staged_takes(ws[j]), !any_rows && !direct_range(encoding, lhs_dtype, m, ns[j], k, group));
         if (plans[j].shares > 1) zero.out[zero.count] = outs[j], zero.n[zero.count++] = (int)ns[j], zeros = std::max(zeros, m * ns[j]);
     }
     const unsigned grid = (unsigned)((m + 63) / 64 * 64 + std::min<int64_t>(1024, (zeros + 4095) / 4096));

@@ -362,12 +362,13 @@ static bool decode_sums_more_exactly(int encoding, int lhs_dtype, int64_t m, int
 // The direct GEMM serves a problem when the caller's workspace holds its operands (qmm_preferred_workspace_bytes); with the smaller one
 // the other kernels do.
 static int direct_group(const qmm_gptq_config* cfg) { return cfg ? cfg->group_size : 0; }
-static bool direct_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    return qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg)) && !decode_sums_more_exactly(encoding, lhs_dtype, m, k);
+static bool direct_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w = nullptr) {
+    return qmm::gemm_direct_wanted(encoding, lhs_dtype, m, n, k, direct_group(cfg), w) && !decode_sums_more_exactly(encoding, lhs_dtype, m, k);
 }
-static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* workspace, int64_t workspace_bytes) {
+static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w, const void* workspace,
+                          int64_t workspace_bytes) {
     if (encoding == QMM_GPTQ && (!cfg || cfg->desc_act)) return false;
-    return workspace && aligned(workspace, 256) && m > 0 && n > 0 && k > 0 && direct_wanted(encoding, cfg, lhs_dtype, m, n, k) &&
+    return workspace && aligned(workspace, 256) && m > 0 && n > 0 && k > 0 && direct_wanted(encoding, cfg, lhs_dtype, m, n, k, w) &&
            workspace_bytes >= qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k);
 }
 
@@ -474,7 +475,7 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
         if (handled) return QMM_OK;
     }
     if (m <= 0 || n <= 0) return fail(QMM_ERR_INVALID, "qmm_matmul: M=%lld N=%lld must be positive", (long long)m, (long long)n);
-    if (!(inner & QMM_FLAG_ACT_Q8K) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
+    if (!(inner & QMM_FLAG_ACT_Q8K) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, n_rhs > 0 ? rhs[0] : nullptr, workspace, workspace_bytes))
         return matmul_f32(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, inner, stream, (uint16_t*)out);
     // (the fp32 result sits behind everything the inner call needs, the Q8_K round trip of the lhs included)
     int64_t base = up256(required_bytes_flags(encoding, lhs_dtype, m, n, k, inner));
@@ -542,7 +543,7 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
             if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order)");
             return QMM_OK;
         }
-        if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
+        if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, rhs[0], workspace, workspace_bytes))
             return hip_status(qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],
                                                       cfg->group_size, m, k, out16, workspace, s),
                               "qmm_matmul(direct GEMM)");
@@ -629,7 +630,7 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
         return matmul_f32(encoding, cfg, y, QMM_F32, m, k, rhs, n_rhs, n, out, (char*)workspace + ybytes, workspace_bytes - ybytes, 0, stream);
     }
     // from a few to a few hundred lhs rows
-    if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))
+    if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, w, workspace, workspace_bytes))
         return hip_status(qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, nullptr, nullptr, 0, m, k, out16, workspace, s), "qmm_matmul(direct GEMM)");
     // Q5_K and Q6_K with many lhs rows, Q4_K with more than 512 on large matrices: weights to fp16 integer planes in the workspace,
     // then the matrix cores
@@ -927,7 +928,7 @@ int qmm_matmul_repacked(int encoding, const qmm_gptq_config* cfg, const void* lh
         return fail(QMM_ERR_INVALID, "qmm_matmul_repacked: the packed buffer must be 256-byte aligned and hold qmm_repack_bytes = %lld bytes (%lld given)",
                     (long long)qmm_repack_bytes(encoding, cfg, n, k), (long long)packed_bytes);
     if (!repacked_path(encoding, m, n, k, rhs != nullptr) ||
-        (rhs && direct_over_planes(encoding, cfg, lhs_dtype, m, n, k) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, workspace, workspace_bytes))) {
+        (rhs && direct_over_planes(encoding, cfg, lhs_dtype, m, n, k) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, rhs[0], workspace, workspace_bytes))) {
         const OptionalPlanesScope no_planes(true);
         return qmm_matmul(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, 0, stream);
     }
@@ -969,7 +970,7 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
         float *direct_out[64], *rest_out[64];
         int directs = 0, rest = 0;
         for (int j = 0; j < count; j++) {
-            if (aligned(rhs[j], 16) && aligned(out[j], 4) && n[j] <= INT32_MAX && direct_serves(encoding, nullptr, lhs_dtype, m, n[j], k, workspace, workspace_bytes))
+            if (aligned(rhs[j], 16) && aligned(out[j], 4) && n[j] <= INT32_MAX && direct_serves(encoding, nullptr, lhs_dtype, m, n[j], k, rhs[j], workspace, workspace_bytes))
                 direct_w[directs] = rhs[j], direct_n[directs] = n[j], direct_out[directs++] = out[j];
             else rest_w[rest] = rhs[j], rest_n[rest] = n[j], rest_out[rest++] = out[j];
         }
@@ -1079,7 +1080,7 @@ int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, i
     if (!aligned(workspace, 256)) return fail(QMM_ERR_INVALID, "qmm_matmul_swiglu: workspace must be 256-byte aligned");
     // Q4_K with 2 .. 8 rows, where the small-batch kernel would serve both products
     if (encoding == QMM_Q4_K && m >= 2 && m <= 8 && k % 256 == 0 && aligned(gate, 16) && aligned(up, 16) && !(m <= 4 && q4k_lanes_rows_wins(n, k)) &&
-        !qmm::kernel_disabled("q4k_mm") && !qmm::kernel_disabled("q4k_mm_gated") && !direct_serves(encoding, nullptr, lhs_dtype, m, n, k, workspace, mm_ws))
+        !qmm::kernel_disabled("q4k_mm") && !qmm::kernel_disabled("q4k_mm_gated") && !direct_serves(encoding, nullptr, lhs_dtype, m, n, k, gate, workspace, mm_ws))
         return hip_status(qmm::launch_gemv_q4_k_mm_gated(lhs, lhs_dtype, (const uint8_t*)gate, (const uint8_t*)up, m, n, k, out, (hipStream_t)stream),
                           "qmm_matmul_swiglu(Q4_K small batch)");
     float* g = (float*)((char*)workspace + mm_ws);

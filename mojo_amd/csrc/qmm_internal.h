@@ -23,9 +23,10 @@ bool twin_rows_allowed();
 int compute_units();
 
 // gemm_direct.hip: a few to a few hundred lhs rows, more where the staged kernel pays, every encoding; out16 != null: bf16 results (out is then unused).
+// w: the weights, where they are known: beyond some rows the answer rests on the staged kernel, which does not take every alignment (null: any).
 // any_rows: called with more rows than gemm_direct_wanted says, held to the error of the direct and shared kernels all the same.
 // source (GPTQ, K a multiple of 32): column p of the weights is column source[p] of the lhs.
-bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
+bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, const void* w);
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k);
 constexpr int kDirectMaxMats = 4;  // count: matrices that share the lhs (out16: one)
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,

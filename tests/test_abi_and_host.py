@@ -277,3 +277,19 @@ def test_a_call_module_of_another_torch_is_rebuilt_and_not_loaded(monkeypatch, t
     call.write_bytes(_lib.call_stamp().encode())
     build._build_call(force=False, verbose=False)
     assert len(compiled) == 1  # current: nothing to do
+
+
+def wanted(enc, m, n, k, at, lhs=_lib.QMM_BF16, group=0):
+    """gemm_direct.hip's answer to: does the direct GEMM, or a kernel behind it there, serve weights at that address?"""
+    call = getattr(C.CDLL(_lib.LIB_PATH), "_ZN3qmm18gemm_direct_wantedEiillliPKv")
+    call.argtypes, call.restype = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_void_p], C.c_bool
+    return call(enc.code, lhs, m, n, k, group, at)
+
+
+def test_q6_k_between_multiples_of_four_is_not_served_beyond_the_direct_range():
+    """The staged GEMM, on which the range beyond rests, does not take such tensors; the direct and the shared one would be up to half as slow again there as the
+    GEMM that unpacks the weights once."""
+    for m, n, k in ((700, 14336, 4096), (1000, 11008, 4096), (1500, 4096, 4096)):
+        assert wanted(QE.Q6_K, m, n, k, 0x10000) and wanted(QE.Q6_K, m, n, k, 0x10004)
+        assert not wanted(QE.Q6_K, m, n, k, 0x10002)
+    assert wanted(QE.Q6_K, 400, 4096, 4096, 0x10002)  # (within it they serve it)

@@ -64,6 +64,16 @@ def test_misaligned_gptq_words_give_the_same_bits(group, m, n, k, words):
     assert torch.equal(qmatmul(QE.GPTQ, config, a, moved, *rhs[1:]), qmatmul(QE.GPTQ, config, a, *rhs))
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 8192, 512), (700, 14336, 1024), (1500, 4096, 768)])
+def test_q6_k_between_multiples_of_four(m, n, k):
+    _, (w,) = weights(QE.Q6_K, 0, n, k)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).bfloat16()
+    moved = torch.empty(w.numel() + 2, dtype=torch.uint8, device="cuda")[2:].view(w.shape)
+    moved.copy_(w)
+    check(qmatmul(QE.Q6_K, None, a, moved), QE.Q6_K, None, (w,), a)
+    check(qmatmul(QE.Q6_K, None, a, moved, out_dtype=torch.bfloat16), QE.Q6_K, None, (w,), a)
+
+
 def test_matrices_together_sum_as_alone():
     """q | k | v in one launch: the bits of three calls of their own."""
     for enc in (QE.Q4_K, QE.Q5_K, QE.Q6_K):
