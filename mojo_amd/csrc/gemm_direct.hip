@@ -615,6 +615,8 @@ bool staged_takes(const void* w) { return ((uintptr_t)w & 3) == 0; }
 // The best of its plans whose parts of K are at most `longest` units and whose sums are off by no more than `most` (sums_error); returns its time (1e30: there is none).
 double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool whole_tiles, bool centred, int64_t longest, double most, DirectPlan& best) {
     const int row = staged_row(encoding, group);
+    // (Q6_K: the last block would be read two bytes beyond its end where it begins at a multiple of four, which it does if the blocks before it are even in number)
+    if (encoding == QMM_Q6_K && (n * direct_units(k)) % 2 != 0) return 1e30;
     if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
     const int type = lhs_dtype == QMM_F32 ? 1 : 0;
     const StagedCost& c = kStagedCost[row][type];

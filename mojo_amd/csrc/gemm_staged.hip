@@ -127,7 +127,8 @@ struct StagedGptq : NoOffsets {
 };
 
 // Q6_K in a tensor that begins at a multiple of four: blocks of 210 bytes lie at even addresses, loads to LDS want multiples of four: a row's 212 bytes from the last such address on, 208 of them in pieces
-// of 16, the last four apart.  The fields begin `skew` (0 or 2) bytes later, other in every row and unit.
+// of 16, the last four apart.  The fields begin `skew` (0 or 2) bytes later, other in every row and unit.  With an even number of blocks the last one of the matrix
+// begins at 2 mod 4 and ends with those four bytes; an odd number of them, whose last would be read two bytes beyond its end, is not this kernel's (staged_plan).
 template <int FLUSH>
 struct StagedQ6 : Q6Weights<1, FLUSH> {
     using Base = Q6Weights<1, FLUSH>;

@@ -293,3 +293,10 @@ def test_q6_k_between_multiples_of_four_is_not_served_beyond_the_direct_range():
         assert wanted(QE.Q6_K, m, n, k, 0x10000) and wanted(QE.Q6_K, m, n, k, 0x10004)
         assert not wanted(QE.Q6_K, m, n, k, 0x10002)
     assert wanted(QE.Q6_K, 400, 4096, 4096, 0x10002)  # (within it they serve it)
+
+
+def test_q6_k_that_ends_between_multiples_of_four_is_not_served_beyond_the_direct_range():
+    """An odd number of blocks: the staged GEMM reads whole multiples of four and would read beyond the last one."""
+    for m, n, k in ((700, 14337, 2304), (800, 14337, 2304), (1500, 4095, 3840)):
+        assert not wanted(QE.Q6_K, m, n, k, 0x10000) and wanted(QE.Q6_K, m, n - 1, k, 0x10000)
+        assert wanted(QE.Q6_K, m, n, k + 256, 0x10000)

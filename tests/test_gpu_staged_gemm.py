@@ -74,6 +74,18 @@ def test_q6_k_between_multiples_of_four(m, n, k):
     check(qmatmul(QE.Q6_K, None, a, moved, out_dtype=torch.bfloat16), QE.Q6_K, None, (w,), a)
 
 
+@pytest.mark.parametrize("m,n,k", [(190, 8193, 256), (190, 8193, 768), (300, 4097, 2304), (700, 14337, 1280), (200, 8194, 768)])
+def test_q6_k_with_an_odd_number_of_blocks(m, n, k):
+    """In the last bytes of a buffer: no kernel may look beyond them for what it multiplies."""
+    _, (w,) = weights(QE.Q6_K, 0, n, k)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).bfloat16()
+    whole = torch.full(((w.numel() + 2047) // 1024 * 1024,), 255, dtype=torch.uint8, device="cuda")
+    start = (whole.numel() - w.numel()) // 4 * 4
+    moved = whole[start:start + w.numel()].view(w.shape)
+    moved.copy_(w)
+    check(qmatmul(QE.Q6_K, None, a, moved), QE.Q6_K, None, (w,), a)
+
+
 def test_matrices_together_sum_as_alone():
     """q | k | v in one launch: the bits of three calls of their own."""
     for enc in (QE.Q4_K, QE.Q5_K, QE.Q6_K):
