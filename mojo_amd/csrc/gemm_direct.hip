@@ -694,7 +694,8 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
             if (direct_units(k) <= longest * kSharedPlans[i].wk * shares)
                 consider(kSharedPlans[i], shares, shared_us(kSharedCost[row][type], i, shares, m, n, k) * (i == 2 ? 1.03 : 1.0));
     }
-    if (like || !staged || (encoding == QMM_Q6_K && !beyond && (m <= 64 || best.wn == 1))) return best;
+    // (up to 32 rows half of the staged kernel's smallest tile is empty: GPTQ 28672 x 8192 17 bf16 rows 46 .. 48 us direct, 50 .. 52 staged)
+    if (like || !staged || (m <= 32 && !beyond) || (encoding == QMM_Q6_K && !beyond && (m <= 64 || best.wn == 1))) return best;
     // The staged kernel, held to the error of what it replaces (sums_error), and where that is the direct kernel with the codes of Q4_K and Q5_K around their
     // middle (KQuantWeights), as there; Q6_K, whose sums leave the matrix cores half as often as in the direct kernel, only for the shared one.
     // Beyond the range of those two anything is more exact than the GEMMs that share unpacked weights (2.2e-7 .. 3.5e-6).
