@@ -898,6 +898,10 @@ static int64_t q4_0_repacked_min_rows(int64_t k) { return k > 4096 ? 96 : 80; }
 // walk the planes twice: GPTQ 14336 x 4096 700 rows 260 / 173, 1400 466 / 315; Q5_K 14336 x 4096 1050 rows 470 / 329; Q6_K 4096 x 4096 450 rows 152 / 70.
 static bool direct_over_planes(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const bool narrow = m * n <= (int64_t)1300 << 10, q40 = encoding == QMM_Q4_0;
+    // Where planes served before the staged kernel and are the more exact ones: relative error, planes / direct, GPTQ 30424 x 512 700 rows 0.92e-7 / 1.07e-7, Q6_K 2056 x 256
+    // 2048 rows 1.38e-7 / 1.98e-7, 1536 x 1024 2048 rows 1.92e-7 / 2.00e-7 (but 14336 x 1024 2.6e-7 / 2.0e-7, K = 4096 5.5e-7 / 2.1e-7).
+    if (lhs_dtype == QMM_F32 && !narrow && ((encoding == QMM_GPTQ && m > 400 && k < 768) || (encoding == QMM_Q6_K && m > 1400 && k < 768))) return false;
+    if (lhs_dtype == QMM_F32 && encoding == QMM_Q6_K && m > 1400 && k <= 1024 && m * n <= (int64_t)4 << 20 && !narrow) return false;
     return (narrow || m <= (q40 ? 150 : 768) || (lhs_dtype == QMM_F32 && !q40)) && !(encoding == QMM_GPTQ && cfg->desc_act) && direct_wanted(encoding, cfg, lhs_dtype, m, n, k);
 }
 static bool repacked_path(int encoding, int64_t m, int64_t n, int64_t k, bool have_rhs) {

@@ -11,7 +11,7 @@ import torch
 import oracle as O
 from conftest import synth
 from mojo_amd import QuantizationConfig, QuantizationEncoding as QE
-from mojo_amd import qmatmul, qmatmul_repacked, repack_weights
+from mojo_amd import dequantize, qmatmul, qmatmul_repacked, quantize, quantize_gptq, repack_weights
 from test_gpu_parity import ENC, assert_close, gpu
 
 pytestmark = pytest.mark.gpu
@@ -217,3 +217,18 @@ def test_a_buffer_made_for_something_else_is_caught():
         assert lib.qmm_repack_check(QE.GPTQ.code, C.byref(cfg128), n, k, C.c_void_p(gp.data_ptr()), gsize, C.c_void_p(s)) == 0
         assert lib.qmm_repack_check(QE.GPTQ.code, C.byref(cfg256), n, k, C.c_void_p(gp.data_ptr()), gsize, C.c_void_p(s)) == -1
         assert b"group 128" in lib.qmm_last_error() and b"group 256" in lib.qmm_last_error()
+
+
+# Relative error (2-norm, against float64) of the planes, by 1.02; of the kernels on the packed tensors in the comment
+@pytest.mark.parametrize("enc,m,n,k,most", [("GPTQ", 700, 30424, 512, 0.93e-7),  # 1.07e-7
+                                            ("Q6_K", 2048, 2056, 256, 1.39e-7),  # 1.98e-7
+                                            ("Q6_K", 2048, 1536, 1024, 1.93e-7)])  # 2.00e-7
+def test_fp32_rows_on_a_short_k_keep_the_precision_of_the_planes(enc, m, n, k, most):
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    w = torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen)
+    a = torch.randn((m, k), device="cuda", generator=gen)
+    config = QuantizationConfig("gptq", 4, 128, False, True) if enc == "GPTQ" else None
+    rhs = quantize_gptq(w, config)[:3] if config else (quantize(QE[enc], w),)
+    want = a.double() @ dequantize(QE[enc], *rhs, config=config).double().T
+    error = ((qmatmul_repacked(a, repack_weights(QE[enc], config, *rhs)).double() - want).norm() / want.norm()).item()
+    assert error <= 1.02 * most, error
