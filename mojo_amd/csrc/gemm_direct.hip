@@ -800,6 +800,10 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
            (f32 || m <= 1024 ? 0.95 : 0.9) * (o[0] + o[1] * packed_mb(encoding, n, k) + o[2] * (m * k * 1e-6) + o[3] * (m * n * 1e-6) + o[4] * (1e-9 * ((m + 255) / 256 * 256) * n * k));
 }
 
+bool gemm_direct_takes_staged(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
+    return direct_plan(encoding, lhs_dtype, m, n, k, group, false, true, !direct_range(encoding, lhs_dtype, m, n, k, group)).fn == 0;
+}
+
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k) {
     return direct_space(nullptr, lhs_dtype == QMM_F32 && encoding != QMM_Q4_0, encoding == QMM_Q4_K || encoding == QMM_Q5_K || encoding == QMM_Q4_0,
                         encoding == QMM_Q4_K || encoding == QMM_Q5_K, m, k).bytes;

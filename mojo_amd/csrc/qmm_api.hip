@@ -893,16 +893,27 @@ int qmm_repack(int encoding, const qmm_gptq_config* cfg, const void* const* rhs,
 // 4096 x 14336: 57 against 83 at 64 rows, 84 against 84 at 96.
 static int64_t q4_0_repacked_min_rows(int64_t k) { return k > 4096 ? 96 : 80; }
 // With the planes at hand the direct GEMM on the packed tensors still wins while the weights are most of the traffic (the planes are 2 or 4
-// bytes a weight against 0.6 .. 0.8): us, planes / direct: Q5_K 4096 x 4096 512 bf16 rows 54 / 37, 14336 x 4096 200 rows 75 / 49, 700 121 / 119, 1000 130 / 149; Q4_K 14336 x 4096
-// 700 rows 121 / 108, 1000 128 / 134; Q6_K 14336 x 4096 700 rows 172 / 168 (1000 219 / 214); Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.  fp32 rows
-// walk the planes twice: GPTQ 14336 x 4096 700 rows 260 / 173, 1400 466 / 315; Q5_K 14336 x 4096 1050 rows 470 / 329; Q6_K 4096 x 4096 450 rows 152 / 70.
+// bytes a weight against 0.6 .. 0.8), and with fp32 rows, for which the planes are walked twice.  us, planes / direct:
+// - up to 150 bf16 rows, or few results: Q5_K 4096 x 4096 128 rows 33 / 20; Q4_0 14336 x 4096 128 rows 60 / 42, 450 rows 94 / 138.
+// - bf16 rows beyond: Q5_K 4096 x 4096 512 rows 54 / 37, 14336 x 4096 200 rows 75 / 49, 700 121 / 119, 1000 130 / 149; Q4_K 14336 x 4096 700 rows 121 / 108, 1000 128 / 134.
+//   From some 256 rows on only for the staged kernel (Q6_K 14336 x 4096 400 rows 119 / 154 in the direct one, Q5_K 2560 x 14336 700 rows 105 / 196), and but for Q4_K
+//   not on 100 M weights and more (Q5_K 28672 x 4096 512 rows 143 / 167, Q6_K 400 rows 224 / 298, GPTQ 28672 x 8192 512 rows 233 / 245).
+// - fp32 rows: GPTQ 14336 x 4096 700 rows 260 / 173, 3000 rows 0.78 times as long; Q5_K 14336 x 4096 1400 rows 0.78, 3000 rows 0.87; on a longer K not
+//   beyond 2048 rows (Q4_K 4096 x 14336 2048 rows 0.94, 2560 x 14336 3000 rows 1.13, 5120 x 8192 3000 rows 1.09).  Where planes served before the staged kernel and
+//   are the more exact ones they still do: relative error, planes / direct, GPTQ 30424 x 512 700 rows 0.92e-7 / 1.07e-7, Q6_K 2056 x 256 2048 rows 1.38e-7 / 1.98e-7,
+//   1536 x 1024 2048 rows 1.92e-7 / 2.00e-7 (but 14336 x 1024 2.6e-7 / 2.0e-7, K = 4096 5.5e-7 / 2.1e-7).
 static bool direct_over_planes(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    const bool narrow = m * n <= (int64_t)1300 << 10, q40 = encoding == QMM_Q4_0;
-    // Where planes served before the staged kernel and are the more exact ones: relative error, planes / direct, GPTQ 30424 x 512 700 rows 0.92e-7 / 1.07e-7, Q6_K 2056 x 256
-    // 2048 rows 1.38e-7 / 1.98e-7, 1536 x 1024 2048 rows 1.92e-7 / 2.00e-7 (but 14336 x 1024 2.6e-7 / 2.0e-7, K = 4096 5.5e-7 / 2.1e-7).
-    if (lhs_dtype == QMM_F32 && !narrow && ((encoding == QMM_GPTQ && m > 400 && k < 768) || (encoding == QMM_Q6_K && m > 1400 && k < 768))) return false;
-    if (lhs_dtype == QMM_F32 && encoding == QMM_Q6_K && m > 1400 && k <= 1024 && m * n <= (int64_t)4 << 20 && !narrow) return false;
-    return (narrow || m <= (q40 ? 150 : 768) || (lhs_dtype == QMM_F32 && !q40)) && !(encoding == QMM_GPTQ && cfg->desc_act) && direct_wanted(encoding, cfg, lhs_dtype, m, n, k);
+    const bool narrow = m * n <= (int64_t)1300 << 10, q40 = encoding == QMM_Q4_0, f32 = lhs_dtype == QMM_F32 && !q40;
+    if ((encoding == QMM_GPTQ && cfg->desc_act) || !direct_wanted(encoding, cfg, lhs_dtype, m, n, k)) return false;
+    if (narrow || m <= (!f32 ? 150 : encoding == QMM_GPTQ ? 400 : 1400)) return true;
+    if (q40) return false;
+    if (f32) {
+        if (encoding == QMM_GPTQ && k < 768) return false;
+        if (encoding == QMM_Q6_K && (k < 768 || (k <= 1024 && m * n <= (int64_t)4 << 20))) return false;
+        return k <= 4096 || m <= 2048;
+    }
+    if (m <= 256) return true;
+    return m <= 768 && (encoding == QMM_Q4_K || n * k <= (int64_t)100 << 20) && qmm::gemm_direct_takes_staged(encoding, lhs_dtype, m, n, k, direct_group(cfg));
 }
 static bool repacked_path(int encoding, int64_t m, int64_t n, int64_t k, bool have_rhs) {
     if (!have_rhs) return true;

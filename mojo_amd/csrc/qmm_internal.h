@@ -27,6 +27,7 @@ int compute_units();
 // any_rows: called with more rows than gemm_direct_wanted says, held to the error of the direct and shared kernels all the same.
 // source (GPTQ, K a multiple of 32): column p of the weights is column source[p] of the lhs.
 bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, const void* w);
+bool gemm_direct_takes_staged(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);  // which of its kernels a call that it serves goes to
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k);
 constexpr int kDirectMaxMats = 4;  // count: matrices that share the lhs (out16: one)
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
