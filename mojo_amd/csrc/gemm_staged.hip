@@ -375,10 +375,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTens
                 buffer(buf);
             }
             read_lhs((t + 1) % kCS, cur ^ 1);
-            if constexpr (t + 1 == W::kSteps) {
-                if constexpr (ENC == QMM_GPTQ) dnext = w.template scale_at<W::kBlocks - 1>();
-                w.open(u + 1 < u1 ? u + 1 : u, (it + 1) & 1);
-            }
+            if constexpr (t + 1 == W::kSteps) w.open(u + 1 < u1 ? u + 1 : u, (it + 1) & 1);
             w.template before_step<t>();
             // one row tile every three steps, the last at steps 14 and 15
             constexpr int min_a = (t - 14 + 3 * (FM - 1)) / 3, min_at = 14 - 3 * (FM - 1);
