@@ -583,13 +583,18 @@ double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q
 struct SumsError {
     float base, unit, join, first;
 };
-constexpr SumsError kSumsError[5][2][3] = {
-    // the direct kernel; the shared and the staged one, codes from 0 (fp32 rows: around their middle); bf16 rows, codes around their middle
-    {{{2.1f, 9.85f, 1.2f, 0.3f}, {53.67f, 2.18f, 0.95f, 0.39f}, {7.9f, 1.21f, 1.37f, -1.64f}}, {{37.3f, 10.02f, 1.27f, -0.1f}, {43.27f, 1.41f, 1.99f, -2.5f}, {43.27f, 1.41f, 1.99f, -2.5f}}},  // Q4_K
-    {{{4.81f, 9.83f, 1.19f, 0.24f}, {72.94f, 2.19f, 0.92f, 0.46f}, {10.55f, 1.2f, 1.36f, -1.65f}}, {{38.99f, 10.04f, 1.28f, -0.1f}, {44.98f, 1.4f, 1.97f, -2.47f}, {44.98f, 1.4f, 1.97f, -2.47f}}},  // Q5_K
-    {{{8.17f, 2.21f, 1.19f, 0.14f}, {16.13f, 1.08f, 1.25f, 0.03f}, {}}, {{36.44f, 2.19f, 1.18f, 0.06f}, {65.72f, 1.08f, 1.21f, 0.15f}, {}}},  // Q6_K
-    {{{0.65f, 2.17f, 1.23f, 0.01f}, {0.65f, 2.17f, 1.23f, 0.01f}, {}}, {{17.37f, 2.19f, 1.25f, -0.08f}, {17.37f, 2.19f, 1.25f, -0.08f}, {}}},  // GPTQ, groups of 128
-    {{{5.93f, 1.14f, 1.21f, -1.48f}, {5.93f, 1.14f, 1.21f, -1.48f}, {}}, {{8.43f, 8.68f, 1.24f, -0.01f}, {8.43f, 8.68f, 1.24f, -0.01f}, {}}},  // GPTQ, other groups
+constexpr SumsError kSumsError[5][2][4] = {
+    // the direct kernel; the shared one, codes from 0 (fp32 rows: around their middle); the staged one, likewise; both with bf16 rows, codes around their middle
+    {{{2.1f, 9.85f, 1.2f, 0.3f}, {54.32f, 2.17f, 1.0f, 0.53f}, {53.32f, 2.18f, 1.08f, 0.38f}, {7.9f, 1.21f, 1.37f, -1.64f}},
+     {{37.3f, 10.02f, 1.27f, -0.1f}, {43.27f, 1.41f, 1.99f, -2.5f}, {43.27f, 1.41f, 1.99f, -2.5f}, {43.27f, 1.41f, 1.99f, -2.5f}}},  // Q4_K
+    {{{4.81f, 9.83f, 1.19f, 0.24f}, {73.53f, 2.19f, 0.94f, 0.76f}, {72.65f, 2.18f, 1.06f, 0.35f}, {10.55f, 1.2f, 1.36f, -1.65f}},
+     {{38.99f, 10.04f, 1.28f, -0.1f}, {44.98f, 1.4f, 1.97f, -2.47f}, {44.98f, 1.4f, 1.97f, -2.47f}, {44.98f, 1.4f, 1.97f, -2.47f}}},  // Q5_K
+    {{{8.17f, 2.21f, 1.19f, 0.14f}, {16.13f, 1.08f, 1.25f, 0.03f}, {16.13f, 1.08f, 1.25f, 0.03f}, {}},
+     {{36.44f, 2.19f, 1.18f, 0.06f}, {65.72f, 1.08f, 1.21f, 0.15f}, {65.72f, 1.08f, 1.21f, 0.15f}, {}}},  // Q6_K
+    {{{0.65f, 2.17f, 1.23f, 0.01f}, {0.65f, 2.17f, 1.23f, 0.01f}, {0.65f, 2.17f, 1.23f, 0.01f}, {}},
+     {{17.37f, 2.19f, 1.25f, -0.08f}, {17.37f, 2.19f, 1.25f, -0.08f}, {17.37f, 2.19f, 1.25f, -0.08f}, {}}},  // GPTQ, groups of 128
+    {{{5.93f, 1.14f, 1.21f, -1.48f}, {5.93f, 1.14f, 1.21f, -1.48f}, {5.93f, 1.14f, 1.21f, -1.48f}, {}},
+     {{8.43f, 8.68f, 1.24f, -0.01f}, {8.43f, 8.68f, 1.24f, -0.01f}, {8.43f, 8.68f, 1.24f, -0.01f}, {}}},  // GPTQ, other groups
 };
 double sums_error(const SumsError& e, const DirectPlan& p, int64_t units) {
     const int log_parts = __builtin_ctz((unsigned)(p.wk * p.shares));
@@ -620,7 +625,7 @@ double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k,
     if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
     const int type = lhs_dtype == QMM_F32 ? 1 : 0;
     const StagedCost& c = kStagedCost[row][type];
-    const SumsError& e = kSumsError[row][type][centred ? 2 : 1];
+    const SumsError& e = kSumsError[row][type][centred ? 3 : 2];
     double us = 1e30;
     for (int shares = 1; shares <= (whole_tiles ? 1 : 2); shares++)
         for (int i = 0; i < 7; i++) {
@@ -705,7 +710,7 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
     const int64_t parts = best.wk * best.shares, part = (direct_units(k) + parts - 1) / parts;
     const int64_t chain = beyond ? 1 << 20 : std::max<int64_t>(4, k_quant && type == 1 && best.wn == 1 && part > 1 ? 5 * part : part);
     const int errors = staged_row(encoding, group);
-    const double most = beyond || errors < 0 ? 1e30 : sums_error(kSumsError[errors][type][best.wn == 1 ? 0 : centred ? 2 : 1], best, direct_units(k));
+    const double most = beyond || errors < 0 ? 1e30 : sums_error(kSumsError[errors][type][best.wn == 1 ? 0 : centred ? 3 : 1], best, direct_units(k));
     DirectPlan p;
     // (4 %: as far as the predictions are off; within it the staged kernel was slower as often as faster, GPTQ 4552 x 3072 472 fp32 rows 55.7 and 56.4 us predicted,
     // 61 and 56 taken; codes around the middle are not in its figures)

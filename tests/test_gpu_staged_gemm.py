@@ -129,6 +129,6 @@ def test_precision(enc, group, m, n, k, lhs, most):
     (QE.GPTQ, 32, 202, 12192, 1024, torch.float32, 0.9592e-7), (QE.GPTQ, 32, 360, 13248, 1792, torch.float32, 1.0652e-7), (QE.GPTQ, 32, 66, 14336, 4096, torch.float32, 1.1225e-7),
     (QE.GPTQ, 128, 786, 2248, 512, torch.bfloat16, 0.4073e-7), (QE.GPTQ, 128, 60, 14336, 4096, torch.bfloat16, 0.6657e-7), (QE.GPTQ, 128, 1330, 728, 2048, torch.float32, 1.1498e-7),
     (QE.Q6_K, 0, 252, 15480, 512, torch.bfloat16, 1.0096e-7), (QE.Q4_K, 0, 481, 6144, 1024, torch.float32, 1.6326e-7), (QE.Q4_K, 0, 385, 5120, 4096, torch.bfloat16, 1.2078e-7),
-    (QE.Q5_K, 0, 193, 5120, 4096, torch.bfloat16, 1.0544e-7)])
+    (QE.Q5_K, 0, 193, 5120, 4096, torch.bfloat16, 1.0544e-7), (QE.Q4_K, 0, 200, 4096, 4096, torch.bfloat16, 1.9066e-7), (QE.Q5_K, 0, 481, 7104, 512, torch.bfloat16, 2.0712e-7)])
 def test_no_less_exact_than_the_kernel_before(enc, group, m, n, k, lhs, most):
     test_precision(enc, group, m, n, k, lhs, 1.003 * most)
