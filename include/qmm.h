@@ -143,7 +143,7 @@ int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_confi
  *   encoding GPTQ: cfg required, n_rhs = 3 or 4,
  *     rhs = {qweight i32[k/8, n], scales f16[k/g, n], qzeros i32[k/g, n/8], g_idx i32[k]}.
  *     cfg->desc_act = 1 (n_rhs = 4): a few rows go through a decode-shaped kernel, four lhs rows per pass over
- *     the weights; more, with a workspace of qmm_preferred_workspace_bytes, through the plain-group kernels on
+ *     the weights; more, with a workspace of qmm_preferred_workspace_bytes, through the plain-group GEMM on
  *     columns that the call sorts by group.
  *   lhs_dtype QMM_F32 or QMM_BF16.  Q4_0 quantises lhs rows to Q8_0 and takes
  *   integer block dots (the reference CPU path); the others keep lhs as given.
@@ -196,7 +196,8 @@ int qmm_matmul_static(int encoding, const qmm_gptq_config* cfg, const void* lhs,
  * block do (q | k | v, and gate | up, take the same activations):
  *   out[j] fp32[m, n[j]] = lhs[m, k] . dequant(rhs[j])^T,  j < count, all rhs of `encoding` and of row length k.
  * Where a kernel takes the whole group (Q4_K, count <= 4: m = 1 with k <= 16384, or 2 <= m <= 16) this is one
- * launch that numbers the rows of the matrices through (the lhs is staged or narrowed once for all of them); otherwise it is one qmm_matmul per matrix, in order
+ * launch that numbers the rows of the matrices through (the lhs is staged or narrowed once for all of them), as it is for up to four matrices that the GEMM on packed weights
+ * (a few to some hundreds of rows) takes with the same cut of k; otherwise it is one qmm_matmul per matrix, in order.  The results are those of separate calls
  * (workspace: the largest any of them needs).  The reference exposes the per-matrix op only; fusing
  * its calls is its graph compiler's job, for which this is the kernel-side counterpart.
  * rhs, n and out are host arrays.

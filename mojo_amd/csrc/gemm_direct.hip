@@ -549,10 +549,12 @@ double shared_us(const SharedCost& c, int plan, int shares, int64_t m, int64_t n
     return c.base + r.all * c.round + walk * (r.full * c.unit[plan] + r.alone * c.unit_alone) + c.weights * (0.6 * n * k * 1e-6) + c.lhs * (m * k * 1e-6) +
            c.out * (m * n * 1e-6) * shares;
 }
-// The same for the kernel whose lhs and weights go to LDS by themselves (gemm_staged.hip), fitted to 326 problems per encoding and lhs type (512 x 512 .. 28672 x
-// 8192, K up to 18944, 24 .. 4096 rows, weights from memory): 3 .. 4 % off, what it picks takes 0.2 % longer on average than its best plan.
+// The same for the kernel whose lhs and weights go to LDS by themselves (gemm_staged.hip).  On 1215 problems that it was not fitted to (512 x 512 .. 28672 x 8192, K up to
+// 18944, 33 .. 4096 rows, weights from memory; profiles/staged_gemm__plans.txt): 4 .. 6 % off on average by encoding and lhs type, what it has first takes 1 .. 2 % longer than
+// the best plan.
 // other: what the GEMMs behind this file (planes, tiles) take, from 200 rows on, in us: a fixed part, per MB of weights, per million lhs values, per million
-// results, per 10^9 products with the rows in 256s (6 .. 10 % off; none for groups that are no multiple of 128, which have no such GEMM).
+// results, per 10^9 products with the rows in 256s (8 .. 12 % off beyond direct_range, where it is asked for, and what is picked there by it takes 0.9 % longer on average than the
+// faster of both; none for groups that are no multiple of 128, which have no such GEMM).
 struct StagedCost {
     float base, round, weights, lhs, out, share;
     float unit[7];  // the plans of kStagedPlans; 0: not built
@@ -578,8 +580,9 @@ int staged_row(int encoding, int group) {
 double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56) * n * k * 1e-6; }
 // What a plan's fp32 sums cost: the square of the relative error of the results (2-norm, against 64 bits) in units of 2^-48 / 6, the mean square of a rounding
 // halved.  An addition counts by the share of K that its sum holds by then: `unit` times half the squares of the parts' lengths, `join` for adding the parts up
-// in order; `first`: additions to zero, which are exact.  Fitted to every plan on 22 K of 256 .. 28672 (profiles/relative_error_by_plan.txt): mean of 0.05 .. 0.8 %
-// off by encoding, lhs type and kind of sums; beyond K = 14336 up to 4 % with the K-quants.
+// in order; `first`: additions to zero, which are exact.  Fitted to every plan on K of 256 .. 14336 (profiles/relative_error_by_plan.txt): mean of 0.05 .. 0.8 %
+// off by encoding, lhs type and kind of sums; beyond up to 4 % with the K-quants.  The shared and the staged kernel apart for codes from 0: with one set for both, 0.7 .. 0.9 % off,
+// 52 of the 480 pairs of plans were refused that are no further off (Q4_K 4096 x 4096, 200 bf16 rows: 1.894e-7 staged, 1.907e-7 shared), with their own 4.
 struct SumsError {
     float base, unit, join, first;
 };
@@ -791,8 +794,8 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     }
     if (m < from) return false;
     if (direct_range(encoding, lhs_dtype, m, n, k, group)) return true;
-    // Beyond, the staged kernel against the GEMMs that unpack the weights once.  us, those / here: Q4_K 14336 x 4096 400 bf16 rows 80 / 70, 1000 149 / 136, 4096 x 14336 2048 rows
-    // 294 / 258; Q5_K 32000 x 4096 200 rows 165 / 82; Q4_K 14336 x 4096 1300 fp32 rows 506 / 347.  With many bf16 rows on many columns those run at their best,
+    // Beyond, the staged kernel against the GEMMs that unpack the weights once.  us, those / here: Q4_K 14336 x 4096 320 bf16 rows 85 / 60, 800 152 / 120, 4096 x 14336 2048 rows
+    // 299 / 261; Q5_K 32000 x 4096 200 rows 167 / 82; Q4_K 14336 x 4096 1300 fp32 rows 522 / 347.  With many bf16 rows on many columns those run at their best,
     // 256 x 256 results at a time, which the figures of `other` do not know (14336 x 4096 2048 rows 260 / 281, 5120 x 5120 2500 rows 163 / 191, 4096 x 4096 3000 rows 126 / 135).
     const int row = staged_row(encoding, group);
     if (row < 0 || !staged_takes(w_at) || (!f32 && m > 1600 && (n > 4096 || (m > 2048 && k <= 8192)))) return false;

@@ -4,14 +4,15 @@
 // instructions), but brings everything through registers, which leaves room for 64 rows a wavefront: 8.5 vector instructions a matrix-core instruction, where
 // a wavefront of those hides four (32 cycles against 12 + 4 each), and 2.3 us a unit of 256 columns for 64 x 256 results.  Here loads go from
 // memory to LDS directly (load16_to_lds) and hold no registers while they are on their way, so that a wavefront takes up to 128 rows: 5 vector instructions
-// a matrix-core instruction, 2.5 .. 3.0 us a unit for 128 x 256 results.  What bounds a unit now: the matrix cores (2.2 us of it), then LDS (1 KB of lhs a
-// matrix-core instruction, 80 % of what a compute unit reads), a barrier every four or eight steps.  What bounds a call of a few units: 14 us around them (the
-// preparation 2.6, the boundary between the launches 2.4, the way to the first unit 3, the results 3 .. 4).
+// a matrix-core instruction, 2.5 .. 3.0 us a unit for 128 x 256 results.  What bounds a unit now: the matrix cores (2.2 us of it), then a
+// barrier every four or eight steps.  By the counters (profiles/staged_gemm__counters.txt) the matrix cores of the compute units in use are busy 0.42 .. 0.59 of a launch of
+// 45 us and more (0.27 of one of 20), a wavefront waits 0.27 .. 0.39 of its time, 0.02 .. 0.04 for LDS, which is active 0.19 .. 0.32 of it.  What bounds a call of a few units: 14 us
+// around them (the preparation 2.6, the boundary between the launches 2.4, the way to the first unit 3, the results 3 .. 4).
 //
-// us, kernels before / here, weights from memory: Q4_K 14336 x 4096 200 bf16 rows 51 / 43, 400 80 / 70, 4096 x 14336 320 rows 84 / 67; Q5_K 32000 x 4096 200 rows
-// 165 / 82; GPTQ 14336 x 4096 160 rows 51 / 33; Q6_K 4096 x 14336 430 rows 142 / 127; Q4_K 14336 x 4096 1300 fp32 rows 506 / 347.  Over 326 problems per
-// encoding and lhs type from 33 rows on, the faster of both: 0.90 bf16 rows, 0.93 fp32 rows of what it was, 0.87 .. 0.90 and 0.75 .. 0.81 beyond the rows that
-// the direct and shared kernels served.
+// us, without this kernel / with it, weights from memory (profiles/staged_gemm__plans.txt): Q4_K 14336 x 4096 200 bf16 rows 53 / 44, 320 85 / 60, 4096 x 4096 200 rows 25 / 22,
+// 4096 x 14336 2048 rows 301 / 261; Q5_K 32000 x 4096 200 rows 167 / 82; GPTQ 14336 x 4096 160 rows 52 / 33; Q6_K 4096 x 14336 500 rows 143 / 121; Q4_K 14336 x 4096 1300 fp32 rows
+// 525 / 347.  Over 1215 problems from 33 rows on, geometric means by encoding: 0.87 .. 0.95 (bf16 rows) and 0.90 .. 0.96 (fp32 rows) of what it was within the rows that the direct and
+// shared kernels served, 0.80 .. 0.85 and 0.65 .. 0.71 beyond.
 //
 // Tried without gain: 64 x 64 results a wavefront with one wavefront a SIMD (nothing hides its waits: 2.1 us for 64 x 256); wavefronts that load only weights or
 // only lhs, with the weights two units ahead; the loads spread over the steps; chunks of the lhs half as long and twice as many.

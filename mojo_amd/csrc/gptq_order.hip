@@ -172,9 +172,9 @@ GptqOrderSpace gptq_order_space(void* workspace, int64_t n, int64_t k) {
 // The look-up kernel or the sort and the direct GEMM: the predicted time of both in microseconds.  The look-up kernel walks K with one workgroup per 64
 // columns, in passes of up to four rows; where its table of scales does not fit LDS (small groups on a long K), every weight reads its
 // scale from memory.  The sorted way is four launches and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
-// 15 matrices (512 x 512 .. 28672 x 8192, groups of 32 and 128, weights from memory) with 1 .. 12 rows; what it picks takes 0.2 % longer on average than the faster of
-// the two.  us, look-up / sorted: 14336 x 4096 4 bf16 rows 34 / 38, 5 rows 47 / 37, fp32 6 rows 39.6 / 40.1; 4096 x 4096 2 / 3 bf16 rows 27 / 22,
-// 32.5 / 21.6; 8192 x 8192 4 rows 62 / 42; 512 x 512 8 / 12 fp32 rows 9 / 12, 13.6 / 12.4; 1024 x 14336 one bf16 row 44 / 39, one fp32 row 43 / 45.
+// 15 matrices (512 x 512 .. 28672 x 8192, groups of 32 and 128, weights from memory) with 1 .. 12 rows; what is taken, the second line included, takes 0.14 % longer on
+// average than the faster of the two (profiles/gptq_act_order__look_up_against_sorted.txt, 576 calls).  us, look-up / sorted: 14336 x 4096 4 bf16 rows 34 / 38, 5 rows 47 / 38, fp32 6 rows
+// 40.2 / 40.2; 4096 x 4096 2 / 3 bf16 rows 27 / 22, 32 / 22; 8192 x 8192 4 rows 62 / 42; 512 x 512 8 / 12 fp32 rows 9 / 12, 13.6 / 12.4; 1024 x 14336 one bf16 row 43 / 41, one fp32 row 42 / 46.
 bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
     if (k > 32768 || n % 8 || k % 32 || kernel_disabled("gptq_order")) return false;
     const bool f32 = lhs_dtype == QMM_F32;
