@@ -943,7 +943,7 @@ int qmm_matmul_repacked(int encoding, const qmm_gptq_config* cfg, const void* lh
         return fail(QMM_ERR_INVALID, "qmm_matmul_repacked: the packed buffer must be 256-byte aligned and hold qmm_repack_bytes = %lld bytes (%lld given)",
                     (long long)qmm_repack_bytes(encoding, cfg, n, k), (long long)packed_bytes);
     if (!repacked_path(encoding, m, n, k, rhs != nullptr) ||
-        (rhs && direct_over_planes(encoding, cfg, lhs_dtype, m, n, k) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, rhs[0], workspace, workspace_bytes))) {
+        (rhs && direct_over_planes(encoding, cfg, lhs_dtype, m, n, k) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, n_rhs > 0 ? rhs[0] : nullptr, workspace, workspace_bytes))) {
         const OptionalPlanesScope no_planes(true);
         return qmm_matmul(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, 0, stream);
     }

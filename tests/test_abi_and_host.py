@@ -300,3 +300,21 @@ def test_q6_k_that_ends_between_multiples_of_four_is_not_served_beyond_the_direc
     for m, n, k in ((700, 14337, 2304), (800, 14337, 2304), (1500, 4095, 3840)):
         assert not wanted(QE.Q6_K, m, n, k, 0x10000) and wanted(QE.Q6_K, m, n - 1, k, 0x10000)
         assert wanted(QE.Q6_K, m, n, k + 256, 0x10000)
+
+
+def test_no_tensors_means_none_is_looked_at():
+    """n_rhs = 0 with an array all the same (here one that ends where memory does): an error, not a read of its first entry."""
+    import mmap
+
+    lib, libc, page = _lib.load(), C.CDLL(None, use_errno=True), mmap.PAGESIZE
+    pages = mmap.mmap(-1, 2 * page)
+    base = C.addressof(C.c_char.from_buffer(pages))
+    libc.mprotect.argtypes = [C.c_void_p, C.c_size_t, C.c_int]
+    assert libc.mprotect(base + page, page, 0) == 0
+    end, m, n, k = C.cast(base + page, C.POINTER(C.c_void_p)), 64, 4096, 4096
+    at, packed = 1 << 20, lib.qmm_repack_bytes(QE.Q5_K.code, None, n, k)
+    need = lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_REPACKED, QE.Q5_K.code, None, _lib.QMM_BF16, m, n, k, 0)
+    assert need > 0 and packed > 0
+    assert lib.qmm_matmul_repacked(QE.Q5_K.code, None, at, _lib.QMM_BF16, m, k, end, 0, at, packed, n, at, at, need, 0, None) == -1
+    assert lib.qmm_matmul(QE.Q5_K.code, None, at, _lib.QMM_BF16, m, k, end, 0, n, at, at, need, _lib.QMM_FLAG_OUT_BF16, None) == -1
+    libc.mprotect(base + page, page, 3)
