@@ -580,24 +580,25 @@ int staged_row(int encoding, int group) {
 double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56) * n * k * 1e-6; }
 // What a plan's fp32 sums cost: the square of the relative error of the results (2-norm, against 64 bits) in units of 2^-48 / 6, the mean square of a rounding
 // halved.  An addition counts by the share of K that its sum holds by then: `unit` times half the squares of the parts' lengths, `join` for adding the parts up
-// in order; `first`: additions to zero, which are exact.  Fitted to every plan on K of 256 .. 14336 (profiles/relative_error_by_plan.txt): mean of 0.05 .. 0.8 %
-// off by encoding, lhs type and kind of sums; beyond up to 4 % with the K-quants.  The shared and the staged kernel apart for codes from 0: with one set for both, 0.7 .. 0.9 % off,
-// 52 of the 480 pairs of plans were refused that are no further off (Q4_K 4096 x 4096, 200 bf16 rows: 1.894e-7 staged, 1.907e-7 shared), with their own 4.
+// in order; `first`: additions to zero, which are exact; `length`: what grows with K however it is cut.  Fitted to every plan on 22 K of 256 .. 28672
+// (profiles/relative_error_by_plan.txt): 0.07 .. 0.4 % off on average by encoding, lhs type and kind of sums, 1.3 % at most, most of which is common to the plans of a K.
+// Kinds that sum alike share a row; the shared and the staged kernel with codes from 0 do not (Q4_K 4096 x 4096, 200 bf16 rows: 1.907e-7 shared, 1.894e-7 staged).
+// Of 9504 pairs of a plan and a staged one it takes the staged one in 35 where that is more than 0.05 % further off (0.4 % at most), and refuses 125 that are no further off.
 struct SumsError {
-    float base, unit, join, first;
+    float base, unit, join, first, length;
 };
 constexpr SumsError kSumsError[5][2][4] = {
     // the direct kernel; the shared one, codes from 0 (fp32 rows: around their middle); the staged one, likewise; both with bf16 rows, codes around their middle
-    {{{2.1f, 9.85f, 1.2f, 0.3f}, {54.32f, 2.17f, 1.0f, 0.53f}, {53.32f, 2.18f, 1.08f, 0.38f}, {7.9f, 1.21f, 1.37f, -1.64f}},
-     {{37.3f, 10.02f, 1.27f, -0.1f}, {43.27f, 1.41f, 1.99f, -2.5f}, {43.27f, 1.41f, 1.99f, -2.5f}, {43.27f, 1.41f, 1.99f, -2.5f}}},  // Q4_K
-    {{{4.81f, 9.83f, 1.19f, 0.24f}, {73.53f, 2.19f, 0.94f, 0.76f}, {72.65f, 2.18f, 1.06f, 0.35f}, {10.55f, 1.2f, 1.36f, -1.65f}},
-     {{38.99f, 10.04f, 1.28f, -0.1f}, {44.98f, 1.4f, 1.97f, -2.47f}, {44.98f, 1.4f, 1.97f, -2.47f}, {44.98f, 1.4f, 1.97f, -2.47f}}},  // Q5_K
-    {{{8.17f, 2.21f, 1.19f, 0.14f}, {16.13f, 1.08f, 1.25f, 0.03f}, {16.13f, 1.08f, 1.25f, 0.03f}, {}},
-     {{36.44f, 2.19f, 1.18f, 0.06f}, {65.72f, 1.08f, 1.21f, 0.15f}, {65.72f, 1.08f, 1.21f, 0.15f}, {}}},  // Q6_K
-    {{{0.65f, 2.17f, 1.23f, 0.01f}, {0.65f, 2.17f, 1.23f, 0.01f}, {0.65f, 2.17f, 1.23f, 0.01f}, {}},
-     {{17.37f, 2.19f, 1.25f, -0.08f}, {17.37f, 2.19f, 1.25f, -0.08f}, {17.37f, 2.19f, 1.25f, -0.08f}, {}}},  // GPTQ, groups of 128
-    {{{5.93f, 1.14f, 1.21f, -1.48f}, {5.93f, 1.14f, 1.21f, -1.48f}, {5.93f, 1.14f, 1.21f, -1.48f}, {}},
-     {{8.43f, 8.68f, 1.24f, -0.01f}, {8.43f, 8.68f, 1.24f, -0.01f}, {8.43f, 8.68f, 1.24f, -0.01f}, {}}},  // GPTQ, other groups
+    {{{2.29f, 9.77f, 1.24f, 0.084f, -0.002f}, {54.12f, 2.12f, 0.838f, 0.922f, 0.021f}, {53.18f, 2.12f, 0.936f, 0.746f, 0.018f}, {7.92f, 1.11f, 1.25f, -1.56f, 0.03f}},
+     {{37.22f, 9.76f, 1.24f, 0.054f, 0.027f}, {43.18f, 1.1f, 1.25f, -1.65f, 0.117f}, {43.18f, 1.1f, 1.25f, -1.65f, 0.117f}, {43.18f, 1.1f, 1.25f, -1.65f, 0.117f}}},  // Q4_K
+    {{{4.97f, 9.75f, 1.23f, 0.018f, -0.001f}, {73.39f, 2.12f, 0.843f, 0.955f, 0.021f}, {72.41f, 2.12f, 0.932f, 0.831f, 0.018f}, {10.56f, 1.11f, 1.24f, -1.57f, 0.027f}},
+     {{38.88f, 9.76f, 1.23f, 0.107f, 0.031f}, {44.89f, 1.1f, 1.23f, -1.64f, 0.116f}, {44.89f, 1.1f, 1.23f, -1.64f, 0.116f}, {44.89f, 1.1f, 1.23f, -1.64f, 0.116f}}},  // Q5_K
+    {{{8.29f, 2.17f, 1.22f, -0.008f, 0.0f}, {16.1f, 1.08f, 1.28f, -0.05f, 0.0f}, {16.1f, 1.08f, 1.28f, -0.05f, 0.0f}, {}},
+     {{36.48f, 2.17f, 1.23f, -0.058f, -0.001f}, {65.7f, 1.08f, 1.28f, -0.064f, 0.002f}, {65.7f, 1.08f, 1.28f, -0.064f, 0.002f}, {}}},  // Q6_K
+    {{{0.66f, 2.17f, 1.26f, -0.03f, -0.001f}, {0.66f, 2.17f, 1.26f, -0.03f, -0.001f}, {0.66f, 2.17f, 1.26f, -0.03f, -0.001f}, {}},
+     {{17.3f, 2.17f, 1.24f, -0.001f, 0.009f}, {17.3f, 2.17f, 1.24f, -0.001f, 0.009f}, {17.3f, 2.17f, 1.24f, -0.001f, 0.009f}, {}}},  // GPTQ, groups of 128
+    {{{5.95f, 1.13f, 1.24f, -1.55f, 0.001f}, {5.95f, 1.13f, 1.24f, -1.55f, 0.001f}, {5.95f, 1.13f, 1.24f, -1.55f, 0.001f}, {}},
+     {{8.41f, 8.66f, 1.25f, 0.003f, 0.007f}, {8.41f, 8.66f, 1.25f, 0.003f, 0.007f}, {8.41f, 8.66f, 1.25f, 0.003f, 0.007f}, {}}},  // GPTQ, other groups
 };
 double sums_error(const SumsError& e, const DirectPlan& p, int64_t units) {
     const int log_parts = __builtin_ctz((unsigned)(p.wk * p.shares));
@@ -614,7 +615,7 @@ double sums_error(const SumsError& e, const DirectPlan& p, int64_t units) {
         }
         if (s == 1 && held < units) join += (double)units;
     }
-    return e.base + (e.unit * 0.5 * squares + e.join * join + e.first * held_parts) / (double)units;
+    return e.base + e.length * (double)units + (e.unit * 0.5 * squares + e.join * join + e.first * held_parts) / (double)units;
 }
 // Codes around their middle: unit sums, and no plan with 128 rows a wavefront, which has no registers for them.
 bool staged_has(const StagedCost& c, int plan, bool centred) { return c.unit[plan] != 0.0f && !(centred && kStagedPlans[plan].fm == 4); }
