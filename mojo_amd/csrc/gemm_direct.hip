@@ -772,9 +772,7 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
             from = wide && k <= 1024 ? 3 : k <= 2048 ? 5 : 17;
             break;
         case QMM_Q4_K:
-            // (with few long rows the small-batch kernel cuts K to fill the part)
-            from = n >= 2048 && (k <= 1024 || (k < 1536 && w <= 8)) ? 2
-                   : !f32 && k > 4096 && n <= 4096 && gemv_q4_k_mm_plain_workspace_bytes(lhs_dtype, m, n, k) == 0 ? 5 : 9;
+            from = n >= 2048 && (k <= 1024 || (k < 1536 && w <= 8)) ? 2 : 9;
             break;
         case QMM_Q5_K:
             // (5 .. 16 bf16 rows on a long K: the small-batch kernel cuts it into rounds side by side; 1024 x 14336 9 rows 22.2 / 12.5 us)

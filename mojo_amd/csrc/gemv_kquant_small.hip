@@ -1,0 +1,601 @@
+// Q4_K, Q5_K and Q6_K with a few lhs rows (2 .. 16 bf16, 2 .. 8 fp32) on the matrix cores, K any multiple of 256: one launch, no workspace.
+//
+// Shape of the work.  A workgroup has as many wavefronts, up to 16, as divide the super-blocks of a row evenly into groups: wavefront w owns super-block
+// w + waves g of group g (K = 4096: one group of 16; 14336: four of 14).  It converts the lhs columns of its super-block into matrix-core operands once a
+// group, keeps them in 32 registers, and walks the workgroup's tiles of 16 weight rows with them.  The super-block of a tile's 16 rows (2.3 .. 3.8 KB) goes global -> LDS
+// directly into a private ring of two slots, one item ahead of the one being multiplied: no wavefront waits for another before the end.  Partial results
+// stay in LDS and are added in wavefront order, so they depend on K and the number of lhs rows only, not on N or on timing.
+//
+// Why 16 wavefronts with one super-block each (two before, eight wavefronts): an item is a chain LDS reads -> unpacking -> matrix cores of some 150 vector instructions, and with two
+// wavefronts a SIMD most of it was waiting.  Why the rows of the lhs go where they go (row j to operand row 4 j mod 16, fp32 residuals in the rows between): a
+// lane of the result holds operand rows 4 (lane / 16) + 0 .. 3, so with up to four rows every lane has one wanted result (two with fp32 residuals), and
+// what is done to results (scales, sums, LDS) shrinks to a quarter.
+//
+// What bounds it: the way to the first product (launch, lhs from L2, conversion: some 4 us with four rows, 6 with sixteen), then memory (14336 x 4096, 4 bf16 rows: a tile of 16 rows, 37 .. 54 KB
+// a compute unit, every 1.4 / 1.75 / 2.1 us).  us, the kernels before / this one, 14336 x 4096 4 bf16 rows, weights from memory: Q4_K 11.2 / 9.4, Q5_K 17.8 / 10.8, Q6_K 20.3 / 12.6; 16 bf16 rows
+// 18.6 / 12.7, 17.5 / 13.9, 22.6 / 17.5; 4096 x 14336 4 fp32 rows 13.9 / 12.2, 22.7 / 13.9, 23.1 / 15.7; 2048 x 1024 4 bf16 rows 9.2 / 3.9.  Relative error, K = 4096, before / now: fp32 rows Q4_K
+// 4.0e-7 / 1.1e-7, Q5_K 1.7e-7 / 1.2e-7, Q6_K 1.6e-7 / 1.0e-7; bf16 rows 2.5e-7 / 0.8e-7, 1.0e-7 / 0.85e-7, 0.97e-7 / 0.84e-7 (codes around their middle, residuals to nearest, super-blocks added in
+// four chains).
+//
+// Arithmetic.  lhs: a power of two per (row, super-block) where its values are not of ordinary size, then fp16 (bf16 rows: exact down to 2^-26 of the largest; fp32 rows: hi part and residual, 22
+// bits).  Weights: integers sc * (q - mid) (Q4_K, Q5_K) or q (Q6_K) as fp16, so every product is exact and the sums are fp32.
+//   Q4_K: a masked nibble is the subnormal q * 2^-24 (or 16 q * 2^-24), one packed multiply-add leaves sc * (q - 8) * 2^-18.
+//   Q5_K: a byte permute puts nibble and fifth bit under 0x54: 64 + q; one packed multiply-add, (64 + q) * sc - 80 * sc, leaves sc * (q - 16) (exact: below 2^11).
+//   Q6_K: the same with 96 taken off; sc * q may need 13 bits, so the scale multiplies the results of its 16 weights instead.
+//   What codes around their middle leave out (Q4_K, Q5_K): mid * d * sc - dmin * mn times the sum of 32 lhs values, both as two fp16 terms, one more matrix product a super-block.
+#include <stdlib.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "gemm_lhs.h"
+#include "lds_stream.h"
+#include "qmm_internal.h"
+
+namespace qmm {
+
+namespace {
+
+typedef _Float16 ks_half4 __attribute__((ext_vector_type(4)));
+typedef float ks_float4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+
+constexpr int kSmallWaves = 16;
+constexpr int kSmallPlane = 528;  // an lhs row of a super-block on its way between lanes: 512 bytes + 16 (bank spread)
+
+// The item of a wavefront: 16 rows of one super-block.  kRow: bytes of a row in LDS; Q6_K blocks lie at even addresses, loads to LDS want multiples of
+// four: 212 bytes from the last such address on, the last 16 of them as a piece of their own (which overlaps the one before), and one piece of padding that
+// spreads the rows over the banks.
+template <int ENC>
+struct SmallItem {
+    static constexpr int kBpb = ENC == QMM_Q4_K ? Q4_K_BPB : ENC == QMM_Q5_K ? Q5_K_BPB : Q6_K_BPB;
+    static constexpr int kRow = ENC == QMM_Q6_K ? 240 : kBpb, kRowPieces = kRow / 16, kPieces = 16 * kRowPieces, kLoads = (kPieces + 63) / 64, kSlot = 16 * kRow;
+    static_assert(4 * kSmallPlane + 16 <= kSlot, "four planes of lhs rows and their scales fit a ring slot");
+};
+
+// 16 bytes per lane, non-temporal, global (uniform base + lane offset) -> LDS at lds_base + 16 * lane
+__device__ __forceinline__ void small_stream16(uint32_t lane_offset, const void* uniform_base, uint32_t lds_base) {
+    uint32_t keep;
+    const uint64_t b = (uint64_t)(uintptr_t)uniform_base;
+    const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(lane_offset), "s"(sb), "s"(lds_base)
+                 : "memory");
+}
+__device__ __forceinline__ half2v to_half2(float a, float b) { return __builtin_convertvector((float2v{a, b}), half2v); }  // to nearest, one instruction
+__device__ __forceinline__ uint32_t to_half2_bits(float a, float b) { return __builtin_bit_cast(uint32_t, to_half2(a, b)); }
+
+enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
+
+}  // namespace
+
+// MROWS: lhs rows, 2, 4, 8 or 16 (>= m; rows past m repeat the last one and their results are dropped).
+// MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up).
+struct SmallCut {
+    int per, stride;  // tiles (gated: pairs) of a workgroup at most, workgroups across the tiles
+    uint32_t packed;  // wavefronts; << 8: items (tile, matrix) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups
+};
+template <int ENC, int MROWS, typename AT, int MODE>
+__device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restrict__ a, int m, int k, const SmallCut& cut) {
+    using I = SmallItem<ENC>;
+    constexpr int PL = sizeof(AT) == 4 ? 2 : 1;             // operand rows of an lhs row
+    constexpr int LR = MROWS <= 4 ? 1 : MROWS / 4;          // lhs rows of a lane's results: lane / 16 + 4 j
+    constexpr int RN = LR * PL;
+    constexpr int kPass = std::min(MROWS, 4 / PL);          // lhs rows that change lanes together
+    static_assert(RN <= 4, "operand rows");
+    constexpr bool kMin = ENC != QMM_Q6_K;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    // (what follows from the launch comes as arguments: the compiler fetches blockDim and gridDim with a vector load and waits for it)
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = (int)(cut.packed & 0xffu), chunk = (int)(cut.packed >> 8) & 0xff, per = cut.per, stride = cut.stride;
+    const bool out_bf16 = (cut.packed >> 16) & 1, apart = (cut.packed >> 17) & 1;
+    const int nn = lane & 15, kg = lane >> 4;
+    const int nblk = k >> 8, groups = (int)(cut.packed >> 18);
+    const int g_first = apart ? (int)blockIdx.y : 0, g_end = apart ? g_first + 1 : groups;  // (one group per workgroup, or all of them)
+    const uint32_t row_bytes = (uint32_t)(nblk * I::kBpb);
+    uint8_t* const ring = smem + wave * (2 * I::kSlot);
+    const uint32_t ring_lds = lds_address(ring);
+    float* const accs = (float*)(smem + waves * (2 * I::kSlot));  // [chunk][waves][LR][64]
+    float* const totals = accs + chunk * waves * LR * 64;  // [chunk][LR][64], with more than one group
+    const int ntiles = MODE == kSmallMats ? mats.tile_end[kLanesMaxMats - 1] : (mats.n[0] + 15) >> 4;
+    const int my_items = (MODE == kSmallGated ? 2 : 1) * ((int)blockIdx.x + (per - 1) * stride < ntiles ? per : per - 1);  // (the grid has no workgroup without a tile)
+
+    // item i of the workgroup: its matrix, and the first row there
+    auto matrix_of = [&](int i, int& n0, int& n) __attribute__((always_inline)) {
+        const int tile = (int)blockIdx.x + (MODE == kSmallGated ? i >> 1 : i) * stride;
+        int j = 0;
+        if constexpr (MODE == kSmallMats) {  // (entries past the last repeat it)
+#pragma unroll
+            for (int i = 0; i + 1 < kLanesMaxMats; i++) j += tile >= mats.tile_end[i] ? 1 : 0;
+        }
+        n0 = (MODE == kSmallMats && j ? tile - mats.tile_end[j - 1] : tile) * 16;
+        if constexpr (MODE == kSmallGated) j = i & 1;
+        n = mats.n[j];
+        return j;
+    };
+    // piece p = lane + 64 i of an item: row p / kRowPieces
+    uint32_t full[I::kLoads];  // byte offset of the piece (Q6_K: of its row) in a tile that lies inside the matrix
+    uint32_t at_row = 0;       // Q6_K: where it begins in the row, eight bits each
+#pragma unroll
+    for (int i = 0; i < I::kLoads; i++) {
+        const int p = min(lane + 64 * i, I::kPieces - 1), pr = p / I::kRowPieces, pc = p - pr * I::kRowPieces;
+        full[i] = (uint32_t)pr * row_bytes + (ENC == QMM_Q6_K ? 0u : 16u * (uint32_t)pc);
+        if constexpr (ENC == QMM_Q6_K) at_row |= (pc < 13 ? 16u * (uint32_t)pc : 196u) << (8 * i);
+    }
+    auto issue = [&](int sb, int item, int slot) {
+        int n0, n;
+        const int j = matrix_of(item, n0, n);
+        const uint8_t* const base = mats.w[j] + (int64_t)n0 * row_bytes + (ENC == QMM_Q6_K ? 0 : sb * I::kBpb);
+        const int last = n - 1 - n0;  // rows past the matrix repeat its last row (their results are dropped)
+#pragma unroll
+        for (int i = 0; i < I::kLoads; i++) {
+            uint32_t off = full[i];
+            if (last < 15) {  // (the last tile of a ragged matrix only)
+                const int pr = min(lane + 64 * i, I::kPieces - 1) / I::kRowPieces;
+                off -= (uint32_t)(pr - min(pr, last)) * row_bytes;
+            }
+            if constexpr (ENC == QMM_Q6_K) off = ((off + (uint32_t)(sb * Q6_K_BPB)) & ~3u) + ((at_row >> (8 * i)) & 0xffu);
+            if (i < I::kLoads - 1 || I::kPieces % 64 == 0 || lane < I::kPieces - 64 * (I::kLoads - 1))
+                small_stream16(off, base, ring_lds + slot * I::kSlot + i * 1024);
+        }
+    };
+
+    // ---- lhs operands of the wavefront's super-block.  Operand row nn: lhs row nn / 4 + 4 j, hi part or (fp32) residual, j and part by nn % 4.
+    // Q4_K, Q5_K: fragment (p, h) of lane quarter kg holds columns 64 kg + 32 h + 8 p + (0 .. 7; Q4_K in the order 0,2,1,3,4,6,5,7); Q6_K: fragment g holds 16 g + 4 kg + 0 .. 3.
+    half8 fa[ENC == QMM_Q6_K ? 1 : 4][2], fs;
+    ks_half4 fq[ENC == QMM_Q6_K ? 16 : 1];
+    float bs[LR];  // inverse lhs scales of this lane's results
+#pragma unroll
+    for (int p = 0; p < (ENC == QMM_Q6_K ? 1 : 4); p++) fa[p][0] = fa[p][1] = pack4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int g = 0; g < (ENC == QMM_Q6_K ? 16 : 1); g++) fq[g] = ks_half4{0, 0, 0, 0};
+    fs = pack4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int j = 0; j < LR; j++) bs[j] = 0.0f;
+    typedef typename std::conditional<sizeof(AT) == 4, u32x4, u32x2>::type xraw_t;
+    // xr: columns 4 lane .. 4 lane + 3 of every lhs row; area: a free ring slot
+    auto narrow = [&](const xraw_t (&xr)[MROWS], uint8_t* area) __attribute__((always_inline)) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));  // (what is computed from it here is not kept in registers between the groups)
+        const int nn = lane & 15, kg = lane >> 4, my_row = (nn >> 2) + 4 * ((nn & 3) / PL), my_part = (nn & 3) % PL;
+        float* const scales = (float*)(area + 4 * kSmallPlane);
+#pragma unroll
+        for (int r0 = 0; r0 < MROWS; r0 += kPass) {
+            float x[kPass][4], mx[kPass], top = 0.0f;
+            bool floor_ok = true;
+#pragma unroll
+            for (int j = 0; j < kPass; j++) {
+                const xraw_t raw = xr[r0 + j];
+                if constexpr (sizeof(AT) == 4) {
+                    x[j][0] = __uint_as_float(raw.x), x[j][1] = __uint_as_float(raw.y), x[j][2] = __uint_as_float(raw.z), x[j][3] = __uint_as_float(raw.w);
+                } else {
+                    x[j][0] = __uint_as_float(raw.x << 16), x[j][1] = __uint_as_float(raw.x & 0xffff0000u);
+                    x[j][2] = __uint_as_float(raw.y << 16), x[j][3] = __uint_as_float(raw.y & 0xffff0000u);
+                }
+                mx[j] = fmaxf(fmaxf(fmaxf(fabsf(x[j][0]), fabsf(x[j][1])), fabsf(x[j][2])), fabsf(x[j][3]));
+                top = fmaxf(top, mx[j]);
+                floor_ok = floor_ok & (__builtin_amdgcn_ballot_w64(mx[j] >= 0.125f) != 0);
+            }
+            // Every row's largest value between 2^-3 and 2^10 (activations of ordinary size): the values go to fp16 as they are, what is below fp16's
+            // normal range (2^-14) is small against the largest, and a sum of 32 is an fp16 number.  Otherwise a power of two per row brings its largest value to [2^9, 2^10) first.
+            const bool scaled = !floor_ok || __builtin_amdgcn_ballot_w64(top >= 1024.0f) != 0;
+            __builtin_amdgcn_wave_barrier();
+            if (scaled) {
+#pragma unroll
+                for (int j = 0; j < kPass; j++) {
+                    // (2^-117: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly; a row with an infinity stays unscaled)
+                    int e = max((int)(wave_max_nonneg_bits(mx[j]) >> 23) - 127, -117);
+                    if (e > 127) e = 9;
+                    const float sc = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
+                    if (lane == 0) scales[j] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) x[j][i] *= sc;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kPass; j++) {
+                constexpr int i1 = ENC == QMM_Q4_K ? 2 : 1, i2 = ENC == QMM_Q4_K ? 1 : 2;
+                const float xs[4] = {x[j][0], x[j][i1], x[j][i2], x[j][3]};
+                const half2v ha = to_half2(xs[0], xs[1]), hb = to_half2(xs[2], xs[3]);
+                uint8_t* const at = area + (j * PL) * kSmallPlane + 8 * lane;
+                *(uint2*)at = make_uint2(__builtin_bit_cast(uint32_t, ha), __builtin_bit_cast(uint32_t, hb));
+                if constexpr (PL == 2) {  // residual x - hi: exact in fp32
+                    const half2v ra = to_half2(fmaf((float)ha.x, -1.0f, xs[0]), fmaf((float)ha.y, -1.0f, xs[1]));
+                    const half2v rb = to_half2(fmaf((float)hb.x, -1.0f, xs[2]), fmaf((float)hb.y, -1.0f, xs[3]));
+                    *(uint2*)(at + kSmallPlane) = make_uint2(__builtin_bit_cast(uint32_t, ra), __builtin_bit_cast(uint32_t, rb));
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
+                const uint8_t* const pl = area + ((my_row - r0) * PL + my_part) * kSmallPlane;
+                if constexpr (ENC == QMM_Q6_K) {
+#pragma unroll
+                    for (int g = 0; g < 16; g++) fq[g] = *(const ks_half4*)(pl + 32 * g + 8 * kg);
+                } else {
+#pragma unroll
+                    for (int p = 0; p < 4; p++) {
+                        fa[p][0] = *(const half8*)(pl + 128 * kg + 16 * p);
+                        fa[p][1] = *(const half8*)(pl + 128 * kg + 64 + 16 * p);
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < LR; j++)
+                if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = scaled ? scales[kg + 4 * j - r0] : 1.0f;
+        }
+        if constexpr (kMin) {
+            // Sums of the operand rows over 32 columns on the matrix cores: column j < 4 of the product is sub-block 2 j (the lane quarter kg = j supplies the ones),
+            // column 4 + j sub-block 2 j + 1.  Through LDS they come to the lane that supplies them: (row nn, sub-blocks 2 kg, 2 kg + 1), as two fp16 terms.
+            const uint32_t e0 = nn == kg ? 0x3C003C00u : 0u, e1 = nn == kg + 4 ? 0x3C003C00u : 0u;
+            const half8 ones0 = pack4(e0, e0, e0, e0), ones1 = pack4(e1, e1, e1, e1);
+            ks_float4 S = {0.f, 0.f, 0.f, 0.f}, S1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                S = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][0], ones0, S, 0, 0, 0);
+                S1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][1], ones1, S1, 0, 0, 0);
+            }
+            S += S1;
+            float* const st = (float*)area;
+            __builtin_amdgcn_wave_barrier();
+            if (nn < 8) {
+#pragma unroll
+                for (int r = 0; r < RN; r++) st[(4 * kg + r) * 9 + nn] = S[r];
+            }
+            __builtin_amdgcn_wave_barrier();
+            const float s0 = (nn & 3) < RN ? st[nn * 9 + kg] : 0.0f, s1 = (nn & 3) < RN ? st[nn * 9 + 4 + kg] : 0.0f;
+            const half2v sh = to_half2(s0, s1), sl = to_half2(fmaf((float)sh.x, -1.0f, s0), fmaf((float)sh.y, -1.0f, s1));
+            const uint32_t h = __builtin_bit_cast(uint32_t, sh), l = __builtin_bit_cast(uint32_t, sl);
+            fs = pack4((h & 0xffffu) | (l << 16), h, (l >> 16) | (h & 0xffff0000u), 0u);  // (sh0, sl0), (sh0, sh1), (sl1, sh1)
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the operands are in registers before the next item's load may overwrite the slot
+    };
+    const uint32_t a_lane = 4 * (uint32_t)sizeof(AT) * lane;
+
+    // first group: the lhs, then the first weights, which stay on their way while the lhs is converted.  (Straight-line code: nothing may move a register that such a load has
+    // not filled yet.  A wavefront without a super-block, in the last group, takes the last one and drops it.)
+    int slot = 0;
+    {
+        xraw_t xr[MROWS];
+        const int sb = min(g_first * waves + wave, nblk - 1);
+#pragma unroll
+        for (int j = 0; j < MROWS; j++) hidden_load(xr[j], a_lane, a + (int64_t)min(j, m - 1) * k + sb * 256);
+        issue(sb, 0, 0);
+        wait_vmcnt<I::kLoads>();
+#pragma unroll
+        for (int j = 0; j < MROWS; j++) tie(xr[j]);
+        narrow(xr, ring + I::kSlot);
+    }
+    // (constants of the unpack in vector registers: an and-or in one instruction takes no literal and one scalar at most)
+    uint32_t m_low = ENC == QMM_Q5_K ? 0x01010101u : 0x03030303u, c54 = 0x54545454u;
+    if constexpr (ENC != QMM_Q4_K) asm volatile("" : "+v"(m_low), "+v"(c54));
+    const ks_float4 zero4 = {0.f, 0.f, 0.f, 0.f};
+
+    for (int c0 = 0; c0 < my_items; c0 += chunk) {
+        const int ct = min(chunk, my_items - c0);
+        for (int g = g_first; g < g_end; g++) {
+            const int sb = g * waves + wave;
+            if (sb < nblk) {  // (all wavefronts but for the last group)
+            if (groups > 1 && c0 + g > g_first) {
+                xraw_t xr[MROWS];
+#pragma unroll
+                for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(j, m - 1) * k + sb * 256) + a_lane);
+                narrow(xr, ring + (slot ^ 1) * I::kSlot);
+            }
+            for (int t = 0; t < ct; t++) {
+                // the next item: of the chunk, of the next group, of the next chunk
+                int ng = g, nt = c0 + t + 1;
+                if (t + 1 == ct) {
+                    ng = g + 1, nt = c0;
+                    if (ng == g_end || sb + waves >= nblk) ng = g_first, nt = c0 + ct;
+                }
+                if (nt < my_items) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (what was read from that slot is in registers)
+                    issue(ng * waves + wave, nt, slot ^ 1);
+                    wait_vmcnt<I::kLoads>();
+                } else {
+                    wait_vmcnt<0>();
+                }
+                const uint8_t* const lb = ring + slot * I::kSlot + nn * I::kRow;
+                float v[LR];
+                if constexpr (ENC == QMM_Q6_K) {
+                    const uint32_t* const l32 = (const uint32_t*)lb;
+                    const uint32_t skew = 2u * (((uint32_t)nn * (uint32_t)nblk + (uint32_t)sb) & 1u);  // (16 rows of a tile: n0 is even)
+                    auto rd = [&](int dw) __attribute__((always_inline)) { return __builtin_amdgcn_alignbyte(l32[dw + 1], l32[dw], skew); };
+                    const uint4 s4 = *(const uint4*)(lb + 192);
+                    const uint32_t tail = l32[55];  // bytes 208 .. 211
+                    const uint32_t sd[4] = {__builtin_amdgcn_alignbyte(s4.y, s4.x, skew), __builtin_amdgcn_alignbyte(s4.z, s4.y, skew),
+                                            __builtin_amdgcn_alignbyte(s4.w, s4.z, skew), __builtin_amdgcn_alignbyte(tail, s4.w, skew)};
+                    const float d = h2f((uint16_t)(tail >> (8 * skew)));
+                    const ks_half4 off96 = {(_Float16)96.0f, (_Float16)96.0f, (_Float16)96.0f, (_Float16)96.0f};
+                    float u[2][RN];  // two chains of sums
+#pragma unroll
+                    for (int r = 0; r < RN; r++) u[0][r] = u[1][r] = 0.0f;
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+#pragma unroll
+                        for (int e2 = 0; e2 < 2; e2++) {
+                            if constexpr (RN == 4) __builtin_amdgcn_sched_barrier(0);  // (with more results on their way at once the compiler spills)
+                            const uint32_t QH = rd(32 + 8 * h + 4 * e2 + kg);
+#pragma unroll
+                            for (int c = 0; c < 4; c++) {
+                                const int gr = 8 * h + 2 * c + e2;  // scale group: weights 128 h + 32 c + 16 e2 + (0..15)
+                                const uint32_t QL = rd(16 * h + 8 * (c & 1) + 4 * e2 + kg);
+                                const uint32_t lo = (c >> 1) ? QL & 0xF0F0F0F0u : (QL << 4) & 0xF0F0F0F0u;
+                                const uint32_t hi = ((QH >> (2 * c)) & m_low) | c54;
+                                const uint2 bq = make_uint2(__builtin_amdgcn_perm(hi, lo, 0x05010400u), __builtin_amdgcn_perm(hi, lo, 0x07030602u));
+                                const ks_half4 bw = __builtin_bit_cast(ks_half4, bq) - off96;
+                                const float cs = (float)((int)(sd[gr >> 2] << (24 - 8 * (gr & 3))) >> 24);
+                                const ks_float4 P = __builtin_amdgcn_mfma_f32_16x16x16f16(fq[gr], bw, zero4, 0, 0, 0);
+#pragma unroll
+                                for (int r = 0; r < RN; r++) u[h][r] = fmaf(cs, P[r], u[h][r]);
+                            }
+                        }
+#pragma unroll
+                    for (int j = 0; j < LR; j++) v[j] = d * (PL == 2 ? (u[0][PL * j] + u[1][PL * j]) + (u[0][PL * j + PL - 1] + u[1][PL * j + PL - 1]) : u[0][j] + u[1][j]);
+                } else {
+                    const uint4 hdr = *(const uint4*)lb;
+                    constexpr int kQs = ENC == QMM_Q4_K ? 16 : 48;
+                    const uint4 q0 = *(const uint4*)(lb + kQs + 32 * kg), q1 = *(const uint4*)(lb + kQs + 16 + 32 * kg);
+                    // 6-bit scales and mins of sub-blocks 2 kg, 2 kg + 1 (4 .. 7 use the split encoding)
+                    const int sh = 16 * (kg & 1);
+                    const uint32_t p0 = (hdr.y >> sh) & 0xffffu, p1 = (hdr.z >> sh) & 0xffffu, p2 = (hdr.w >> sh) & 0xffffu;
+                    const uint32_t sc_pair = kg >= 2 ? ((p2 & 0x0F0Fu) | ((p0 >> 2) & 0x3030u)) : (p0 & 0x3F3Fu);
+                    const uint32_t mn_pair = kg >= 2 ? (((p2 >> 4) & 0x0F0Fu) | ((p1 >> 2) & 0x3030u)) : (p1 & 0x3F3Fu);
+                    float d = h2f((uint16_t)(hdr.x & 0xffffu));
+                    // what the codes around their middle leave out: (mid d sc - dmin mn) times the sums of the lhs, both as two fp16 terms, the former times a power of two that
+                    // brings the largest it can be below 2^15
+                    constexpr float kMid = ENC == QMM_Q4_K ? 8.0f : 16.0f;
+                    const float dm = kMid * d, dmin = h2f((uint16_t)(hdr.x >> 16)), e0 = (float)(sc_pair & 0xffu), e1 = (float)(sc_pair >> 8);
+                    const int scale = 15 - __builtin_amdgcn_frexp_expf(63.0f * (fabsf(dm) + fabsf(dmin)));
+                    const float o0 = __builtin_amdgcn_ldexpf(fmaf(dm, e0, -(dmin * (float)(mn_pair & 0xffu))), scale), o1 = __builtin_amdgcn_ldexpf(fmaf(dm, e1, -(dmin * (float)(mn_pair >> 8))), scale);
+                    const half2v oh = to_half2(o0, o1), ol = to_half2(fmaf((float)oh.x, -1.0f, o0), fmaf((float)oh.y, -1.0f, o1));
+                    const uint32_t ohb = __builtin_bit_cast(uint32_t, oh), olb = __builtin_bit_cast(uint32_t, ol);
+                    const half8 offs = pack4(__builtin_amdgcn_perm(ohb, ohb, 0x01000100u), (olb & 0xffffu) | (ohb & 0xffff0000u), (ohb >> 16) | (olb & 0xffff0000u), 0u);
+                    const uint32_t qd[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                    ks_float4 P = zero4, Q = zero4;  // two chains: low and high nibbles
+                    if constexpr (ENC == QMM_Q4_K) {
+                        const uint32_t M1 = 0x000F000Fu, M2 = 0x00F000F0u;
+                        // 64 sc for the low nibbles (q * 2^-24), 4 sc for the high ones (16 q * 2^-24): the operand is sc * (q - 8) * 2^-18 (as sc * q * 2^-24, always a subnormal, the matrix core
+                        // drops low bits of the products)
+                        const uint32_t sp_lo = to_half2_bits(64.0f * e0, 64.0f * e0), sp_hi = to_half2_bits(4.0f * e1, 4.0f * e1);
+                        const uint32_t np_lo = pk_mul(sp_lo, 0x80088008u), np_hi = pk_mul(sp_hi, 0x80808080u);  // -8 * 2^-24, -128 * 2^-24 times it
+                        d *= 262144.0f;
+#pragma unroll
+                        for (int p = 0; p < 4; p++) {
+                            const uint32_t x0 = qd[2 * p], x1 = qd[2 * p + 1], y0 = x0 >> 8, y1 = x1 >> 8;
+                            const half8 blo = pack4(pk_fma(x0 & M1, sp_lo, np_lo), pk_fma(y0 & M1, sp_lo, np_lo), pk_fma(x1 & M1, sp_lo, np_lo), pk_fma(y1 & M1, sp_lo, np_lo));
+                            const half8 bhi = pack4(pk_fma(x0 & M2, sp_hi, np_hi), pk_fma(y0 & M2, sp_hi, np_hi), pk_fma(x1 & M2, sp_hi, np_hi), pk_fma(y1 & M2, sp_hi, np_hi));
+                            P = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][0], blo, P, 0, 0, 0);
+                            Q = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][1], bhi, Q, 0, 0, 0);
+                        }
+                    } else {
+                        const uint4 h0 = *(const uint4*)(lb + 16), h1 = *(const uint4*)(lb + 32);  // fifth bits: bit j of byte i, column i of sub-block j
+                        const uint32_t hd[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+                        const uint32_t s_lo = to_half2_bits(e0, e0), s_hi = to_half2_bits(e1, e1), n_lo = to_half2_bits(-80.0f * e0, -80.0f * e0), n_hi = to_half2_bits(-80.0f * e1, -80.0f * e1);
+#pragma unroll
+                        for (int p = 0; p < 4; p++) {
+                            uint32_t lo[4], hi[4];
+#pragma unroll
+                            for (int i = 0; i < 2; i++) {
+                                const uint32_t x = qd[2 * p + i], f = hd[2 * p + i] >> (2 * kg);
+                                const uint32_t xl = (x << 4) & 0xF0F0F0F0u, xh = x & 0xF0F0F0F0u, fl = (f & m_low) | c54, fh = ((f >> 1) & m_low) | c54;
+                                lo[2 * i] = pk_fma(__builtin_amdgcn_perm(fl, xl, 0x05010400u), s_lo, n_lo);
+                                lo[2 * i + 1] = pk_fma(__builtin_amdgcn_perm(fl, xl, 0x07030602u), s_lo, n_lo);
+                                hi[2 * i] = pk_fma(__builtin_amdgcn_perm(fh, xh, 0x05010400u), s_hi, n_hi);
+                                hi[2 * i + 1] = pk_fma(__builtin_amdgcn_perm(fh, xh, 0x07030602u), s_hi, n_hi);
+                            }
+                            P = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][0], pack4(lo[0], lo[1], lo[2], lo[3]), P, 0, 0, 0);
+                            Q = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[p][1], pack4(hi[0], hi[1], hi[2], hi[3]), Q, 0, 0, 0);
+                        }
+                    }
+                    const ks_float4 O = __builtin_amdgcn_mfma_f32_16x16x32_f16(fs, offs, zero4, 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < LR; j++) {
+                        float sum = P[PL * j] + Q[PL * j], off = O[PL * j];
+                        if constexpr (PL == 2) sum += P[PL * j + PL - 1] + Q[PL * j + PL - 1], off += O[PL * j + PL - 1];
+                        v[j] = fmaf(d, sum, __builtin_amdgcn_ldexpf(off, -scale));
+                    }
+                }
+                float* const mine = accs + ((t * waves + wave) * LR) * 64 + lane;
+#pragma unroll
+                for (int j = 0; j < LR; j++) mine[j * 64] = bs[j] * v[j];
+                slot ^= 1;
+            }
+            }
+            __syncthreads();
+            // the group's result (matrix row 16 tile + nn, lhs row kg + 4 j): dealt to the wavefronts, which add it to that of the groups before
+            const int live = min(waves, nblk - g * waves);
+            constexpr int kEach = MODE == kSmallGated ? 2 : 1;
+            for (int q = wave; q < ct / kEach * LR; q += waves) {
+                const int t = q / LR * kEach, j = q % LR, row = kg + 4 * j;
+                float s[kEach];
+#pragma unroll
+                for (int h = 0; h < kEach; h++) {
+                    const float* const src = accs + (((t + h) * waves) * LR + j) * 64 + lane;
+                    float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    int w = 0;
+                    for (; w + 4 <= live; w += 4)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) c[i] += src[(w + i) * LR * 64];
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+                        if (w + i < live) c[i] += src[(w + i) * LR * 64];
+                    s[h] = (c[0] + c[1]) + (c[2] + c[3]);
+                    if (groups > 1) {
+                        float* const total = totals + ((t + h) * LR + j) * 64 + lane;
+                        if (g > g_first) s[h] = *total + s[h];
+                        if (g + 1 < g_end) *total = s[h];
+                    }
+                }
+                if (g + 1 < g_end) continue;
+                int n0, n;
+                const int mat = matrix_of(c0 + t, n0, n);
+                float r = s[0];
+                if constexpr (MODE == kSmallGated) r = s[0] / (1.0f + expf(-s[0])) * s[kEach - 1];
+                const int64_t at = (int64_t)row * n + n0 + nn;
+                if (row < m && n0 + nn < n) {
+                    if (out_bf16) ((uint16_t*)mats.out[mat])[at] = f2bf(r);
+                    else mats.out[mat][at + (int64_t)blockIdx.y * m * n] = r;
+                }
+            }
+            if (g + 1 < g_end || c0 + chunk < my_items) __syncthreads();
+        }
+    }
+}
+
+template <int ENC, int MROWS, typename AT, int MODE>
+__global__ __launch_bounds__(64 * kSmallWaves) void gemv_kquant_small_mats_kernel(const MmMats mats, const AT* __restrict__ a, int m, int k, const SmallCut cut) {
+    small_body<ENC, MROWS, AT, MODE>(mats, a, m, k, cut);
+}
+
+// The plain call: one matrix [n, k].  Twelve dwords of arguments.
+template <int ENC, int MROWS, typename AT>
+__global__ __launch_bounds__(64 * kSmallWaves) void gemv_kquant_small_kernel(const uint8_t* __restrict__ w, const AT* __restrict__ a, float* __restrict__ out, int n, int m, int k,
+                                                                          int per, int stride, uint32_t packed) {
+    MmMats mats;
+    mats.w[0] = w;
+    mats.out[0] = out;
+    mats.n[0] = n;
+    small_body<ENC, MROWS, AT, kSmallPlain>(mats, a, m, k, SmallCut{per, stride, packed});
+}
+
+namespace {
+
+struct SmallPlan {
+    int waves, groups, grid, parts, per, chunk;
+    size_t lds;
+};
+// Groups of K: of its length only, so that results do not depend on what else a call has.
+int small_groups(int64_t k) {
+    const int groups = (int)((k / 256 + kSmallWaves - 1) / kSmallWaves);
+    return groups == 3 ? 4 : groups;
+}
+// tiles: of 16 weight rows, gated: pairs of them; parts: workgroups that share a tile, one group of K each
+SmallPlan small_plan(int encoding, int64_t m, int64_t tiles, int64_t k, bool gated, bool parts) {
+    SmallPlan p;
+    const int nblk = (int)(k / 256), groups = small_groups(k);
+    p.groups = groups;
+    p.waves = (nblk + groups - 1) / groups;
+    p.parts = parts ? groups : 1;
+    // one workgroup per compute unit (as many as 16 wavefronts allow with few each), all with the same number of tiles or one fewer
+    const int per_cu = std::max(1, kSmallWaves / p.waves);
+    const int64_t most = std::max<int64_t>(1, (int64_t)compute_units() * per_cu / p.parts);
+    p.per = (int)((tiles + most - 1) / most);
+    p.grid = (int)((tiles + p.per - 1) / p.per);
+    const int slot = encoding == QMM_Q4_K ? SmallItem<QMM_Q4_K>::kSlot : encoding == QMM_Q5_K ? SmallItem<QMM_Q5_K>::kSlot : SmallItem<QMM_Q6_K>::kSlot;
+    // (as many items between two barriers as fit: a barrier after each, with two buffers, took Q6_K 28672 x 8192 with 16 rows from 65 to 92 us)
+    const int lr = m <= 4 ? 1 : m <= 8 ? 2 : 4, ring = p.waves * 2 * slot, each = (p.waves + (groups > p.parts ? 1 : 0)) * lr * 256, items = gated ? 2 * p.per : p.per;
+    p.chunk = std::min(std::min(items, 254), (kLdsPerCu / per_cu - ring) / each);
+    if (gated) p.chunk &= ~1;
+    p.lds = (size_t)ring + (size_t)p.chunk * each;
+    return p;
+}
+// A K of several groups: a workgroup per (share of the tiles, group), whose results a launch of their own adds in group order, or all groups in each workgroup?
+// The latter converts the lhs again for every group; both give the same bits.  us, walk / apart: Q4_K 1024 x 14336 4 bf16 rows 13.7 / 7.9, 4096 x 14336 2 bf16 rows
+// 13.7 / 11.8, 8 fp32 rows 23.2 / 14.7; but two groups and many tiles, 28672 x 8192 4 bf16 rows 27.7 / 29.7, 8192 x 8192 11.5 / 12.1.
+bool small_parts(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    const int groups = small_groups(k);
+    if (groups < 2) return false;
+    const double item = encoding == QMM_Q4_K ? 1.4 : encoding == QMM_Q5_K ? 1.75 : 2.1;  // a tile of one group; convert: the lhs of one
+    const double convert = lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
+    const int64_t tiles = (n + 15) / 16;
+    const SmallPlan w = small_plan(encoding, m, tiles, k, false, false), a = small_plan(encoding, m, tiles, k, false, true);
+    const double walk = groups * ((w.per + w.chunk - 1) / w.chunk) * convert + groups * w.per * item;
+    return convert + a.per * item + (a.per - 1) / a.chunk * 1.0 + 2.3 + 1.6e-6 * (4.0 * m * n * groups) < walk;
+}
+
+template <int ENC, int MROWS, typename AT>
+hipError_t run_small(const MmMats& mats, const SmallPlan& p, const AT* a, int m, int k, bool gated, bool out_bf16, hipStream_t s) {
+    const dim3 grid((unsigned)p.grid, (unsigned)p.parts), block((unsigned)(64 * p.waves));
+    const SmallCut cut{p.per, p.grid, (uint32_t)p.waves | (uint32_t)p.chunk << 8 | (uint32_t)out_bf16 << 16 | (uint32_t)(p.parts > 1) << 17 | (uint32_t)p.groups << 18};
+    hipError_t e;
+    if (gated) {
+        if ((e = allow_full_lds<gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallGated>>()) != hipSuccess) return e;
+        gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallGated><<<grid, block, p.lds, s>>>(mats, a, m, k, cut);
+    } else if (mats.count > 1) {
+        if ((e = allow_full_lds<gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallMats>>()) != hipSuccess) return e;
+        gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallMats><<<grid, block, p.lds, s>>>(mats, a, m, k, cut);
+    } else {
+        if ((e = allow_full_lds<gemv_kquant_small_kernel<ENC, MROWS, AT>>()) != hipSuccess) return e;
+        gemv_kquant_small_kernel<ENC, MROWS, AT><<<grid, block, p.lds, s>>>(mats.w[0], a, mats.out[0], mats.n[0], m, k, cut.per, cut.stride, cut.packed);
+    }
+    return hipGetLastError();
+}
+
+template <int ENC>
+hipError_t run_small_rows(const MmMats& mats, const SmallPlan& p, const void* a, int lhs_dtype, int m, int k, bool gated, bool out_bf16, hipStream_t s) {
+    if (lhs_dtype == QMM_F32) {
+        const float* const f = (const float*)a;
+        if (m <= 2) return run_small<ENC, 2>(mats, p, f, m, k, gated, out_bf16, s);
+        if (m <= 4) return run_small<ENC, 4>(mats, p, f, m, k, gated, out_bf16, s);
+        return run_small<ENC, 8>(mats, p, f, m, k, gated, out_bf16, s);
+    }
+    const uint16_t* const b = (const uint16_t*)a;
+    if (m <= 2) return run_small<ENC, 2>(mats, p, b, m, k, gated, out_bf16, s);
+    if (m <= 4) return run_small<ENC, 4>(mats, p, b, m, k, gated, out_bf16, s);
+    if (m <= 8) return run_small<ENC, 8>(mats, p, b, m, k, gated, out_bf16, s);
+    return run_small<ENC, 16>(mats, p, b, m, k, gated, out_bf16, s);
+}
+
+}  // namespace
+
+bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
+    if (encoding != QMM_Q4_K && encoding != QMM_Q5_K && encoding != QMM_Q6_K) return false;
+    // (with the name of an encoding's older small-batch kernel this one goes too)
+    if (kernel_disabled("kquant_small") || kernel_disabled(encoding == QMM_Q4_K ? "q4k_mm" : encoding == QMM_Q5_K ? "q5k_mm" : "q6k_mm")) return false;
+    if (m < 1 || m > (lhs_dtype == QMM_F32 ? 8 : 16) || n < 1 || n > 0x7fffff00 || k < 256 || k % 256 || k > (1 << 20)) return false;
+    if (encoding == QMM_Q4_K || encoding == QMM_Q5_K) return ((uintptr_t)w & 15) == 0;
+    // (loads of four bytes at least: the last block of the matrix has to end at a multiple of four)
+    return ((uintptr_t)w & 3) == 0 && n * (k / 256) % 2 == 0;
+}
+
+// What the parts of K of a plain call with few tiles take (without it a workgroup walks all of K: the same sums).
+int64_t gemv_kquant_small_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    return small_parts(encoding, lhs_dtype, m, n, k) ? small_groups(k) * m * n * 4 : 0;
+}
+
+namespace {
+// out[i] = bf16(part[i] + part[count + i] + ...), in that order
+__global__ __launch_bounds__(256) void small_sum_bf16_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, int64_t count, int parts) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    float v = 0.0f;
+    for (int j = 0; j < parts; j++) v += part[j * count + i];
+    out[i] = f2bf(v);
+}
+}  // namespace
+
+// count matrices [ns[j], k] that share the lhs; gated: two of the same size, gate and up, outs[0] = silu(lhs gate^T) * (lhs up^T).  The caller has asked
+// gemv_kquant_small_supported for each.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (the plain call) gemv_kquant_small_workspace_bytes.
+hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs, int64_t m, int64_t k,
+                                    bool gated, bool out_bf16, void* workspace, hipStream_t s) {
+    if (count < 1 || count > kLanesMaxMats || (gated && (count != 2 || ns[0] != ns[1]))) return hipErrorInvalidValue;
+    MmMats mats;
+    int64_t tiles = 0;
+    for (int j = 0; j < kLanesMaxMats; j++) {
+        const int i = std::min(j, count - 1);
+        if (j < count) tiles += (ns[j] + 15) / 16;
+        mats.w[j] = (const uint8_t*)ws[i];
+        mats.out[j] = outs[gated ? 0 : i];
+        mats.n[j] = (int)ns[i];
+        mats.tile_end[j] = (int)tiles;
+    }
+    mats.count = count;
+    const bool parts = count == 1 && workspace && small_parts(encoding, lhs_dtype, m, ns[0], k);
+    if (parts) mats.out[0] = (float*)workspace;
+    const SmallPlan p = small_plan(encoding, m, gated ? tiles / 2 : tiles, k, gated, parts);
+    const bool store_bf16 = out_bf16 && !parts;
+    hipError_t e = encoding == QMM_Q4_K   ? run_small_rows<QMM_Q4_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
+                   : encoding == QMM_Q5_K ? run_small_rows<QMM_Q5_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
+                                          : run_small_rows<QMM_Q6_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s);
+    if (e != hipSuccess || !parts) return e;
+    const int64_t values = m * ns[0];
+    if (!out_bf16) return launch_sum_shares((const float*)workspace, outs[0], values, p.parts, s);
+    small_sum_bf16_kernel<<<dim3((unsigned)((values + 255) / 256)), dim3(256), 0, s>>>((const float*)workspace, (uint16_t*)outs[0], values, p.parts);
+    return hipGetLastError();
+}
+
+}  // namespace qmm

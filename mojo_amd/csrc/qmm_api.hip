@@ -43,6 +43,24 @@ int hip_status(hipError_t e, const char* what) {
 
 bool aligned(const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 
+// environment variables that send every shape that it takes to one kernel (tests), read once
+bool is_one(const char* name) {
+    const char* e = getenv(name);
+    return e && e[0] == '1';
+}
+bool q4k_lanes_rows_forced() {
+    static const bool set = is_one("QMM_Q4K_LANES_ROWS");
+    return set;
+}
+bool q6k_mm_forced() {
+    static const bool set = is_one("QMM_Q6K_MM");
+    return set;
+}
+bool q5k_mm_forced() {
+    static const bool set = is_one("QMM_Q5K_MM");
+    return set;
+}
+
 // GPTQ with more than 16 lhs rows: do passes of the small-batch kernel (16 rows each, bound by the bytes of the weights)
 // beat the GEMM (128 x 256 output tiles, one workgroup each, bound by K per round of 256 tiles)?  Times in
 // microseconds as measured on 14336 x 4096, 4096 x 14336 and 4096 x 4096 with 64 to 128 rows: a GEMM round costs
@@ -67,11 +85,7 @@ bool q4k_lanes_rows_wins(int64_t n, int64_t k) {
     // per K step and per launch.  Measured, 4 fp32 rows, decode kernel / matrix-core kernel: 512 x 4096 5.1 / 6.7 us,
     // 1024 x 4096 5.2 / 6.7, 2048 x 4096 6.3 / 6.8, 3072 x 4096 7.7 / 6.9, 4096 x 4096 8.9 / 7.0, 14336 x 4096 20.8 / 12.3,
     // 1024 x 8192 9.9 / 10.6, 1024 x 14336 16.2 / 17.5 (bf16 rows: 10.1 / 17.9), 4096 x 14336 42.9 / 18.0.
-    static const bool forced = [] {
-        const char* e = getenv("QMM_Q4K_LANES_ROWS");
-        return e && e[0] == '1';
-    }();
-    return forced || n <= 1024 || n * k <= ((int64_t)8 << 20);
+    return q4k_lanes_rows_forced() || n <= 1024 || n * k <= ((int64_t)8 << 20);
 }
 
 // Q6_K (K a multiple of 2048 up to 32768): the small-batch matrix-core kernel, or passes of the decode kernel (one or two
@@ -82,12 +96,8 @@ bool q6k_mm_wanted(int64_t m, int64_t n, int64_t k) {
     // 4096 rows: 2 10.3 / 9.6, 4 11.7 / 15.2, 8 13.8 / 32.9, 16 36 / 52; 1024 rows: 2 9.8 / 6.1, 4 11.2 / 7.7, 8 13.2 / 21.9,
     // 16 29 / 38; 4096 x 14336 (four rounds over K, side by side): 1 19.2 / 16.1, 2 20.0 / 22.4, 4 22.1 / 47.  (Its fixed cost is
     // the conversion of the lhs in every workgroup and round.)  QMM_Q6K_MM=1 sends every shape there.
-    static const bool forced = [] {
-        const char* e = getenv("QMM_Q6K_MM");
-        return e && e[0] == '1';
-    }();
     // (a K beyond 16384, which the decode kernel with the rows global -> LDS does not take: from one bf16 row on)
-    return forced || m >= 5 || (m >= 3 && n >= 2048) || (m == 2 && (n >= 8192 || (k > 8192 && n >= 2048))) || (k > 16384 && n >= 2048);
+    return q6k_mm_forced() || m >= 5 || (m >= 3 && n >= 2048) || (m == 2 && (n >= 8192 || (k > 8192 && n >= 2048))) || (k > 16384 && n >= 2048);
 }
 
 // Q5_K: the small-batch matrix-core kernel, or passes of the decode kernel (up to four lhs rows each)?
@@ -97,14 +107,10 @@ bool q5k_mm_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     // 4096 x 4096: 4 11.9 / 11.4, 8 14.3 / 22.1; 1024 x 4096: 4 11.6 / 7.8, 8 13.9 / 15.3; 4096 x 14336: 2 34.4 / 33.1, 4 40.4 / 65.4,
     // 8 50.2 / 130; with the rounds of a long K side by side: 2 19.9 / 32.1, 4 21.6 / 65.  QMM_Q5K_MM=1 sends every shape the kernel
     // takes there.
-    static const bool forced = [] {
-        const char* e = getenv("QMM_Q5K_MM");
-        return e && e[0] == '1';
-    }();
     // Other shapes: 5120 x 5120 with 4 rows 21 / 29.8; 32000 x 4096 with 2 rows 28 / 32.2; 8192 x 28672 with one row 50 / 61.
     // (three and four bf16 rows from 16 Mi weights on: 4096 x 4096 8.8 / 9.1 against 10.6 / 10.8)
     const int64_t min3 = lhs_dtype == QMM_BF16 ? ((int64_t)16 << 20) : ((int64_t)32 << 20);
-    return forced || m >= 5 || (m >= 3 && (n * k >= min3 || (k > 4096 && n >= 2048))) ||
+    return q5k_mm_forced() || m >= 5 || (m >= 3 && (n * k >= min3 || (k > 4096 && n >= 2048))) ||
            (m >= 2 && ((k > 8192 && n >= 2048) || n * k >= ((int64_t)96 << 20))) || (k > 16384 && n >= 2048);
 }
 
@@ -334,7 +340,7 @@ static int64_t required_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n,
         return std::max(std::max(a, b), c);
     }
     if (encoding == QMM_Q4_K && m <= 16 && k % 256 == 0) {  // lhs planes from 9 rows on; partial sums of K chunks
-        const int64_t a = qmm::gemv_q4_k_mm_plain_workspace_bytes(lhs_dtype, m, n, k), b = m >= 2 ? qmm::gemv_q4_k_kc_workspace_bytes(m, n, k) : 0;
+        const int64_t a = qmm::gemv_q4_k_mm_workspace_bytes(lhs_dtype, m, k), b = m >= 2 ? qmm::gemv_q4_k_kc_workspace_bytes(m, n, k) : 0;
         const int64_t c = q4k_gemm_from_9_rows(encoding, lhs_dtype, m, n, k) ? qmm::gemm_q4_k_workspace_bytes(lhs_dtype, m, n, k) : 0;
         return std::max(std::max(a, b), c);
     }
@@ -370,6 +376,28 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
     if (encoding == QMM_GPTQ && (!cfg || cfg->desc_act)) return false;
     return workspace && aligned(workspace, 256) && m > 0 && n > 0 && k > 0 && direct_wanted(encoding, cfg, lhs_dtype, m, n, k, w) &&
            workspace_bytes >= qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k);
+}
+
+// K-quants with a few lhs rows: the kernel with a super-block per wavefront, unless one of the others is faster.
+// us, that other / here (weights from memory), over 42 matrices of 256 .. 128256 rows and K of 512 .. 28672 with 2 .. 16 rows:
+// - Q4_K, two to four rows, few long rows (the decode kernel with a sub-block per lane): 1024 x 4096 2 rows 4.0 / 4.7, 4 fp32 rows 5.2 / 5.5 (bf16 4.95 / 4.97), 2048 x 4096 2 rows 4.9 / 5.1,
+//   1024 x 8192 2 rows 4.9 / 7.1, 4 bf16 rows 6.5 / 7.4 (fp32 10.1 / 7.9); but 1024 x 2048 4 rows 4.9 / 4.3, 1024 x 11008 4 rows 13.7 / 6.9.
+// - Q5_K, two fp32 rows on few columns (its decode kernel): 512 x 4096 5.0 / 5.2; 2048 x 4096 5.7 / 5.1.
+// - 9 .. 16 bf16 rows on large matrices with several groups of K, where few results fit LDS next to the ring: Q6_K 28672 x 8192 51 / 66, 4096 x 14336 9 rows 22.2 / 23.3 (16 rows 25.0 / 22.7), Q5_K 8192 x 28672
+//   47 / 51; but Q6_K 8192 x 8192 24 / 21, 5120 x 13824 38 / 24.
+// - Q6_K, five and six fp32 rows, K = 256 or 512: more exact weight by weight (decode_sums_more_exactly), 0.85e-7 against 0.88e-7.
+static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
+    if (m < 2 || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
+    const bool f32 = lhs_dtype == QMM_F32;
+    if (encoding == QMM_Q4_K) {
+        if (m <= 4 && q4k_lanes_rows_forced()) return false;
+        return qmm::kernel_disabled("q4k_lanes_rows") || k <= 2304 || k > 8192 ||
+               !((m == 2 && (n <= 1024 || (k <= 4096 && n * k <= ((int64_t)8 << 20)))) || (m <= 4 && n <= 1024 && f32 == (k <= 4096)));
+    }
+    const bool large = m > 8 && k > 4096;
+    if (encoding == QMM_Q5_K) return !q5k_mm_forced() && !(f32 && m == 2 && n <= 1024 && k > 2304 && k <= 4096) && !(large && n * k >= ((int64_t)190 << 20));
+    if (f32 && (m == 5 || m == 6) && k <= 512) return false;
+    return !q6k_mm_forced() && !(large && (n * k >= ((int64_t)96 << 20) || (m < 12 && k > 8192 && k % 2048 == 0 && n * k >= ((int64_t)54 << 20))));
 }
 
 // Does the kernel that serves this problem store bf16 itself?  (The Q4_K decode kernel does; everything else goes
@@ -424,6 +452,7 @@ static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lh
         return order ? std::max(need, order + ((flags & QMM_FLAG_OUT_BF16) ? up256(m * n * 4) : 0)) : need;
     }
     int64_t ahead = 0;
+    if (!(flags & QMM_FLAG_ACT_Q8K) && small_wanted(encoding, lhs_dtype, m, n, k, nullptr)) return std::max(need, up256(qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, n, k)) + (flags & QMM_FLAG_OUT_BF16 ? up256(m * n * 4) : 0));
     if (flags & QMM_FLAG_ACT_Q8K) {  // (the lhs as fp32 rows in front, where the integer kernels do not serve the call)
         if (q8k_integer_kernel(encoding, m, k) || (flags & QMM_FLAG_OUT_BF16)) return need;
         ahead = up256(m * k * 4);
@@ -475,7 +504,10 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
         if (handled) return QMM_OK;
     }
     if (m <= 0 || n <= 0) return fail(QMM_ERR_INVALID, "qmm_matmul: M=%lld N=%lld must be positive", (long long)m, (long long)n);
-    if (!(inner & QMM_FLAG_ACT_Q8K) && direct_serves(encoding, cfg, lhs_dtype, m, n, k, n_rhs > 0 ? rhs[0] : nullptr, workspace, workspace_bytes))
+    const void* const w = n_rhs > 0 ? rhs[0] : nullptr;
+    const bool small = n_rhs == 1 && w && k > 0 && (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && small_wanted(encoding, lhs_dtype, m, n, k, w) &&
+                       workspace && aligned(workspace, 256) && workspace_bytes >= required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
+    if (!(inner & QMM_FLAG_ACT_Q8K) && (small || direct_serves(encoding, cfg, lhs_dtype, m, n, k, w, workspace, workspace_bytes)))
         return matmul_f32(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, inner, stream, (uint16_t*)out);
     // (the fp32 result sits behind everything the inner call needs, the Q8_K round trip of the lhs included)
     int64_t base = up256(required_bytes_flags(encoding, lhs_dtype, m, n, k, inner));
@@ -629,6 +661,12 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
         if (e != hipSuccess) return hip_status(e, "qmm_matmul(Q8_K round trip)");
         return matmul_f32(encoding, cfg, y, QMM_F32, m, k, rhs, n_rhs, n, out, (char*)workspace + ybytes, workspace_bytes - ybytes, 0, stream);
     }
+    // a few lhs rows
+    if (small_wanted(encoding, lhs_dtype, m, n, k, w)) {
+        const bool parts = workspace && aligned(workspace, 256) && workspace_bytes >= qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, n, k);
+        return hip_status(qmm::launch_gemv_kquant_small(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, m, k, false, out16 != nullptr, parts ? workspace : nullptr, s),
+                          "qmm_matmul(K-quant small batch)");
+    }
     // from a few to a few hundred lhs rows
     if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, w, workspace, workspace_bytes))
         return hip_status(qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, nullptr, nullptr, 0, m, k, out16, workspace, s), "qmm_matmul(direct GEMM)");
@@ -681,30 +719,25 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
 
     // 2..4 lhs rows on a small matrix: the decode kernel with one sub-block per lane (the activations of four rows fit a
     // lane's registers)
-    // (not with 3 or 4 rows where the matrix-core kernel cuts a long K over the grid: 1024 x 14336 with 4 fp32 rows 23.4 -> 10.5 us,
-    // bf16 rows 13.6 -> 10.0)
-    const bool q4k_mm_cuts_k = encoding == QMM_Q4_K && m >= 2 && m <= 8 && !qmm::kernel_disabled("q4k_mm") &&
-                               qmm::gemv_q4_k_mm_plain_workspace_bytes(lhs_dtype, m, n, k) > 0;
-    if (encoding == QMM_Q4_K && m >= 2 && m <= 4 && q4k_lanes_rows_wins(n, k) && !(m >= 3 && q4k_mm_cuts_k)) {
+    if (encoding == QMM_Q4_K && m >= 2 && m <= 4 && q4k_lanes_rows_wins(n, k)) {
         bool handled = false;
         hipError_t e = qmm::launch_gemv_q4_k_lanes_rows(lhs, lhs_dtype, w, (int)m, n, k, out, n, s, &handled);
         if (e != hipSuccess) return hip_status(e, "qmm_matmul(Q4_K decode, 2..4 rows)");
         if (handled) return QMM_OK;
     }
-    // 2..16 lhs rows on few weight rows and long K: the small-batch kernel that cuts K across workgroups (up to 8 rows the
-    // matrix-core kernel below does so itself where its grid then fills the part: 4096 x 14336 with 8 bf16 rows 20.6 -> 15.6 us)
-    if (encoding == QMM_Q4_K && m >= 2 && m <= 16 && q4k_kc_wins(lhs_dtype, m, n, k) && !q4k_mm_cuts_k && qmm::gemv_q4_k_kc_supported(w, k)) {
+    // 2..16 lhs rows on few weight rows and long K: the small-batch kernel that cuts K across workgroups
+    if (encoding == QMM_Q4_K && m >= 2 && m <= 16 && q4k_kc_wins(lhs_dtype, m, n, k) && qmm::gemv_q4_k_kc_supported(w, k)) {
         bool handled = false;
         hipError_t e = qmm::launch_gemv_q4_k_kc(lhs, lhs_dtype, w, (int)m, n, k, out, n, workspace, s, &handled);
         if (e != hipSuccess) return hip_status(e, "qmm_matmul(Q4_K small batch, K chunks)");
         if (handled) return QMM_OK;
     }
-    // 3..16 lhs rows: the small-batch matrix-core kernel; more: the prefill kernel (which also takes 9..16 fp32 rows on a large
+    // 9..16 lhs rows: the small-batch matrix-core kernel over a prepared lhs; more: the prefill kernel (which also takes 9..16 fp32 rows on a large
     // matrix with a long K, where the small-batch kernel works through two planes of a prepared lhs: 28672 x 8192 with 16 rows
     // 70 us against 61 for 32 rows, 8192 x 28672 94 against 76)
     if (q4k_gemm_from_9_rows(encoding, lhs_dtype, m, n, k))
         return hip_status(qmm::launch_gemm_q4_k(lhs, lhs_dtype, w, m, n, k, out, workspace, s), "qmm_matmul(Q4_K GEMM)");
-    if (encoding == QMM_Q4_K && m >= 2 && m <= 16 && !qmm::kernel_disabled("q4k_mm"))
+    if (encoding == QMM_Q4_K && m >= 9 && m <= 16 && !qmm::kernel_disabled("q4k_mm"))
         return hip_status(qmm::launch_gemv_q4_k_mm(lhs, lhs_dtype, w, m, n, k, out, workspace, s), "qmm_matmul(Q4_K small batch)");
     if (encoding == QMM_Q4_K && m > 16)
         return hip_status(qmm::launch_gemm_q4_k(lhs, lhs_dtype, w, m, n, k, out, workspace, s), "qmm_matmul(Q4_K GEMM)");
@@ -978,12 +1011,25 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
         return fail(QMM_ERR_INVALID, "qmm_matmul_grouped: encoding %d is not a GGUF weight encoding", encoding);
     for (int j = 0; j < count; j++)
         if (!rhs[j] || !out[j] || n[j] <= 0) return fail(QMM_ERR_INVALID, "qmm_matmul_grouped: matrix %d: null pointer or N <= 0", j);
-    // Matrices that a call of their own would give to the direct GEMM go there together; the others, if any, then form their own group.
+    // Matrices that a call of their own would give to the small-batch kernel or to the direct GEMM go there together; the others, if any, then form their own group.
     if (m > 0 && m <= INT32_MAX && k > 0 && k <= INT32_MAX && (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && aligned(lhs, 16)) {
         const void *direct_w[64], *rest_w[64];
         int64_t direct_n[64], rest_n[64];
         float *direct_out[64], *rest_out[64];
         int directs = 0, rest = 0;
+        for (int j = 0; j < count; j++) {
+            if (aligned(out[j], 4) && small_wanted(encoding, lhs_dtype, m, n[j], k, rhs[j])) direct_w[directs] = rhs[j], direct_n[directs] = n[j], direct_out[directs++] = out[j];
+            else rest_w[rest] = rhs[j], rest_n[rest] = n[j], rest_out[rest++] = out[j];
+        }
+        for (int j = 0; j < directs; j += qmm::kLanesMaxMats) {
+            const hipError_t e = qmm::launch_gemv_kquant_small(encoding, lhs, lhs_dtype, std::min(qmm::kLanesMaxMats, directs - j), direct_w + j, direct_n + j, direct_out + j, m, k,
+                                                               false, false, nullptr, (hipStream_t)stream);
+            if (e != hipSuccess) return hip_status(e, "qmm_matmul_grouped(K-quant small batch)");
+        }
+        if (directs > 0)
+            return rest == 0 ? QMM_OK
+                             : qmm_matmul_grouped(encoding, lhs, lhs_dtype, m, k, rest, rest_w, rest_n, rest_out, workspace, workspace_bytes, stream);
+        rest = 0;
         for (int j = 0; j < count; j++) {
             if (aligned(rhs[j], 16) && aligned(out[j], 4) && n[j] <= INT32_MAX && direct_serves(encoding, nullptr, lhs_dtype, m, n[j], k, rhs[j], workspace, workspace_bytes))
                 direct_w[directs] = rhs[j], direct_n[directs] = n[j], direct_out[directs++] = out[j];
@@ -1040,8 +1086,8 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
                 return qmm_matmul_grouped(encoding, lhs, lhs_dtype, m, k, rest, rest_w, rest_n, rest_out, workspace, workspace_bytes, stream);
             }
         }
-        if (ok && total <= INT32_MAX && m >= 2 && !qmm::kernel_disabled("q4k_mm")) {
-            // the lhs is narrowed once (in the kernel up to 8 rows, by the separate pass beyond) for all the matrices
+        if (ok && total <= INT32_MAX && m >= 9 && !qmm::kernel_disabled("q4k_mm")) {
+            // the lhs is narrowed once for all the matrices
             const int64_t need = qmm::gemv_q4_k_mm_workspace_bytes(lhs_dtype, m, k);
             if (need > 0 && (!workspace || workspace_bytes < need))
                 return fail(QMM_ERR_WORKSPACE, "qmm_matmul_grouped: workspace of %lld bytes required, %lld given", (long long)need,
@@ -1093,11 +1139,13 @@ int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, i
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul_swiglu: workspace of %lld bytes required, %lld given", (long long)(mm_ws + 2 * plane),
                     (long long)workspace_bytes);
     if (!aligned(workspace, 256)) return fail(QMM_ERR_INVALID, "qmm_matmul_swiglu: workspace must be 256-byte aligned");
-    // Q4_K with 2 .. 8 rows, where the small-batch kernel would serve both products
-    if (encoding == QMM_Q4_K && m >= 2 && m <= 8 && k % 256 == 0 && aligned(gate, 16) && aligned(up, 16) && !(m <= 4 && q4k_lanes_rows_wins(n, k)) &&
-        !qmm::kernel_disabled("q4k_mm") && !qmm::kernel_disabled("q4k_mm_gated") && !direct_serves(encoding, nullptr, lhs_dtype, m, n, k, gate, workspace, mm_ws))
-        return hip_status(qmm::launch_gemv_q4_k_mm_gated(lhs, lhs_dtype, (const uint8_t*)gate, (const uint8_t*)up, m, n, k, out, (hipStream_t)stream),
-                          "qmm_matmul_swiglu(Q4_K small batch)");
+    // where the small-batch kernel would serve both products
+    if (small_wanted(encoding, lhs_dtype, m, n, k, gate) && small_wanted(encoding, lhs_dtype, m, n, k, up)) {
+        const void* const both[2] = {gate, up};
+        const int64_t ns[2] = {n, n};
+        float* const outs[2] = {out, out};
+        return hip_status(qmm::launch_gemv_kquant_small(encoding, lhs, lhs_dtype, 2, both, ns, outs, m, k, true, false, nullptr, (hipStream_t)stream), "qmm_matmul_swiglu(K-quant small batch)");
+    }
     float* g = (float*)((char*)workspace + mm_ws);
     float* u = (float*)((char*)workspace + mm_ws + plane);
     // (one launch for both products where a kernel takes matrices that share their lhs: Q4_K with 2..16 rows)
