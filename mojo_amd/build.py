@@ -38,6 +38,7 @@ FLAGS = [
 PER_FILE_FLAGS = {
     "gemv_q4k_lanes.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_kquant_small.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
+    "gemv_gptq_small.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
     "gemm_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
 }

@@ -28,21 +28,13 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm_lhs.h"
-#include "lds_stream.h"
-#include "qmm_internal.h"
+#include "small_lhs.h"
 
 namespace qmm {
 
 namespace {
 
-typedef _Float16 ks_half4 __attribute__((ext_vector_type(4)));
-typedef float ks_float4 __attribute__((ext_vector_type(4)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float2v __attribute__((ext_vector_type(2)));
-
 constexpr int kSmallWaves = 16;
-constexpr int kSmallPlane = 528;  // an lhs row of a super-block on its way between lanes: 512 bytes + 16 (bank spread)
 
 // The item of a wavefront: 16 rows of one super-block.  kRow: bytes of a row in LDS; Q6_K blocks lie at even addresses, loads to LDS want multiples of
 // four: 212 bytes from the last such address on, the last 16 of them as a piece of their own (which overlaps the one before), and one piece of padding that
@@ -53,20 +45,6 @@ struct SmallItem {
     static constexpr int kRow = ENC == QMM_Q6_K ? 240 : kBpb, kRowPieces = kRow / 16, kPieces = 16 * kRowPieces, kLoads = (kPieces + 63) / 64, kSlot = 16 * kRow;
     static_assert(4 * kSmallPlane + 16 <= kSlot, "four planes of lhs rows and their scales fit a ring slot");
 };
-
-// 16 bytes per lane, non-temporal, global (uniform base + lane offset) -> LDS at lds_base + 16 * lane
-__device__ __forceinline__ void small_stream16(uint32_t lane_offset, const void* uniform_base, uint32_t lds_base) {
-    uint32_t keep;
-    const uint64_t b = (uint64_t)(uintptr_t)uniform_base;
-    const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
-                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep)
-                 : "v"(lane_offset), "s"(sb), "s"(lds_base)
-                 : "memory");
-}
-__device__ __forceinline__ half2v to_half2(float a, float b) { return __builtin_convertvector((float2v{a, b}), half2v); }  // to nearest, one instruction
-__device__ __forceinline__ uint32_t to_half2_bits(float a, float b) { return __builtin_bit_cast(uint32_t, to_half2(a, b)); }
 
 enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
 
@@ -164,50 +142,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
         float* const scales = (float*)(area + 4 * kSmallPlane);
 #pragma unroll
         for (int r0 = 0; r0 < MROWS; r0 += kPass) {
-            float x[kPass][4], mx[kPass], top = 0.0f;
-            bool floor_ok = true;
-#pragma unroll
-            for (int j = 0; j < kPass; j++) {
-                const xraw_t raw = xr[r0 + j];
-                if constexpr (sizeof(AT) == 4) {
-                    x[j][0] = __uint_as_float(raw.x), x[j][1] = __uint_as_float(raw.y), x[j][2] = __uint_as_float(raw.z), x[j][3] = __uint_as_float(raw.w);
-                } else {
-                    x[j][0] = __uint_as_float(raw.x << 16), x[j][1] = __uint_as_float(raw.x & 0xffff0000u);
-                    x[j][2] = __uint_as_float(raw.y << 16), x[j][3] = __uint_as_float(raw.y & 0xffff0000u);
-                }
-                mx[j] = fmaxf(fmaxf(fmaxf(fabsf(x[j][0]), fabsf(x[j][1])), fabsf(x[j][2])), fabsf(x[j][3]));
-                top = fmaxf(top, mx[j]);
-                floor_ok = floor_ok & (__builtin_amdgcn_ballot_w64(mx[j] >= 0.125f) != 0);
-            }
-            // Every row's largest value between 2^-3 and 2^10 (activations of ordinary size): the values go to fp16 as they are, what is below fp16's
-            // normal range (2^-14) is small against the largest, and a sum of 32 is an fp16 number.  Otherwise a power of two per row brings its largest value to [2^9, 2^10) first.
-            const bool scaled = !floor_ok || __builtin_amdgcn_ballot_w64(top >= 1024.0f) != 0;
-            __builtin_amdgcn_wave_barrier();
-            if (scaled) {
-#pragma unroll
-                for (int j = 0; j < kPass; j++) {
-                    // (2^-117: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly; a row with an infinity stays unscaled)
-                    int e = max((int)(wave_max_nonneg_bits(mx[j]) >> 23) - 127, -117);
-                    if (e > 127) e = 9;
-                    const float sc = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
-                    if (lane == 0) scales[j] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) x[j][i] *= sc;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < kPass; j++) {
-                constexpr int i1 = ENC == QMM_Q4_K ? 2 : 1, i2 = ENC == QMM_Q4_K ? 1 : 2;
-                const float xs[4] = {x[j][0], x[j][i1], x[j][i2], x[j][3]};
-                const half2v ha = to_half2(xs[0], xs[1]), hb = to_half2(xs[2], xs[3]);
-                uint8_t* const at = area + (j * PL) * kSmallPlane + 8 * lane;
-                *(uint2*)at = make_uint2(__builtin_bit_cast(uint32_t, ha), __builtin_bit_cast(uint32_t, hb));
-                if constexpr (PL == 2) {  // residual x - hi: exact in fp32
-                    const half2v ra = to_half2(fmaf((float)ha.x, -1.0f, xs[0]), fmaf((float)ha.y, -1.0f, xs[1]));
-                    const half2v rb = to_half2(fmaf((float)hb.x, -1.0f, xs[2]), fmaf((float)hb.y, -1.0f, xs[3]));
-                    *(uint2*)(at + kSmallPlane) = make_uint2(__builtin_bit_cast(uint32_t, ra), __builtin_bit_cast(uint32_t, rb));
-                }
-            }
+            const bool scaled = small_narrow<PL, kPass, ENC == QMM_Q4_K ? kSmallOrderK : kSmallOrderPlain>(xr, r0, area, scales, lane);
             __builtin_amdgcn_wave_barrier();
             if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
                 const uint8_t* const pl = area + ((my_row - r0) * PL + my_part) * kSmallPlane;
@@ -558,7 +493,6 @@ int64_t gemv_kquant_small_workspace_bytes(int encoding, int lhs_dtype, int64_t m
 }
 
 namespace {
-// out[i] = bf16(part[i] + part[count + i] + ...), in that order
 __global__ __launch_bounds__(256) void small_sum_bf16_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, int64_t count, int parts) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
@@ -567,6 +501,11 @@ __global__ __launch_bounds__(256) void small_sum_bf16_kernel(const float* __rest
     out[i] = f2bf(v);
 }
 }  // namespace
+// out[i] = bf16(part[i] + part[count + i] + ...), in that order
+hipError_t launch_sum_shares_bf16(const float* part, uint16_t* out, int64_t count, int shares, hipStream_t s) {
+    small_sum_bf16_kernel<<<dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s>>>(part, out, count, shares);
+    return hipGetLastError();
+}
 
 // count matrices [ns[j], k] that share the lhs; gated: two of the same size, gate and up, outs[0] = silu(lhs gate^T) * (lhs up^T).  The caller has asked
 // gemv_kquant_small_supported for each.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (the plain call) gemv_kquant_small_workspace_bytes.
@@ -594,8 +533,7 @@ hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype
     if (e != hipSuccess || !parts) return e;
     const int64_t values = m * ns[0];
     if (!out_bf16) return launch_sum_shares((const float*)workspace, outs[0], values, p.parts, s);
-    small_sum_bf16_kernel<<<dim3((unsigned)((values + 255) / 256)), dim3(256), 0, s>>>((const float*)workspace, (uint16_t*)outs[0], values, p.parts);
-    return hipGetLastError();
+    return launch_sum_shares_bf16((const float*)workspace, (uint16_t*)outs[0], values, p.parts, s);
 }
 
 }  // namespace qmm

@@ -400,6 +400,13 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
     return !q6k_mm_forced() && !(large && (n * k >= ((int64_t)96 << 20) || (m < 12 && k > 8192 && k % 2048 == 0 && n * k >= ((int64_t)54 << 20))));
 }
 
+// GPTQ with groups in their order, up to 16 lhs rows (fp32: 8).  us, the kernels before (decode, small batch, direct GEMM) / here, weights from memory: one row 4096 x 4096 6.4 / 5.0, 14336 x 4096 9.6 / 8.6,
+// 4096 x 14336 15.3 / 10.9; four bf16 rows 9.4 / 5.5, 12.4 / 9.0, 15.2 / 11.3; eight fp32 rows 13.6 / 7.7, 18.3 / 12.6, 20.9 / 12.9; 16 bf16 rows 11.1 / 8.9, 14.3 / 13.5, 16.8 / 14.6.  Relative error, K = 4096: 4.2e-7 /
+// 0.8e-7 (fp32 rows), 2.2e-7 and 1.2e-7 / 0.65e-7 (one and four bf16 rows).
+static bool gptq_small_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    return encoding == QMM_GPTQ && cfg && !cfg->desc_act && qmm::gemv_gptq_small_supported(lhs_dtype, m, n, k, cfg->group_size);
+}
+
 // Does the kernel that serves this problem store bf16 itself?  (The Q4_K decode kernel does; everything else goes
 // through an fp32 result in the workspace and a narrowing pass.)
 static bool stores_bf16_itself(int encoding, int64_t m, int64_t k, int flags) {
@@ -452,6 +459,7 @@ static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lh
         return order ? std::max(need, order + ((flags & QMM_FLAG_OUT_BF16) ? up256(m * n * 4) : 0)) : need;
     }
     int64_t ahead = 0;
+    if (!(flags & QMM_FLAG_ACT_Q8K) && gptq_small_wanted(encoding, cfg, lhs_dtype, m, n, k)) return std::max(need, up256(qmm::gemv_gptq_small_workspace_bytes(lhs_dtype, m, n, k, cfg->group_size)) + (flags & QMM_FLAG_OUT_BF16 ? up256(m * n * 4) : 0));
     if (!(flags & QMM_FLAG_ACT_Q8K) && small_wanted(encoding, lhs_dtype, m, n, k, nullptr)) return std::max(need, up256(qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, n, k)) + (flags & QMM_FLAG_OUT_BF16 ? up256(m * n * 4) : 0));
     if (flags & QMM_FLAG_ACT_Q8K) {  // (the lhs as fp32 rows in front, where the integer kernels do not serve the call)
         if (q8k_integer_kernel(encoding, m, k) || (flags & QMM_FLAG_OUT_BF16)) return need;
@@ -505,7 +513,9 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
     }
     if (m <= 0 || n <= 0) return fail(QMM_ERR_INVALID, "qmm_matmul: M=%lld N=%lld must be positive", (long long)m, (long long)n);
     const void* const w = n_rhs > 0 ? rhs[0] : nullptr;
-    const bool small = n_rhs == 1 && w && k > 0 && (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && small_wanted(encoding, lhs_dtype, m, n, k, w) &&
+    const bool few = encoding == QMM_GPTQ ? (n_rhs == 3 || n_rhs == 4) && cfg && cfg->group_size > 0 && gptq_small_wanted(encoding, cfg, lhs_dtype, m, n, k)
+                                          : n_rhs == 1 && w && small_wanted(encoding, lhs_dtype, m, n, k, w);
+    const bool small = few && k > 0 && (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) &&
                        workspace && aligned(workspace, 256) && workspace_bytes >= required_bytes_flags(encoding, lhs_dtype, m, n, k, flags);
     if (!(inner & QMM_FLAG_ACT_Q8K) && (small || direct_serves(encoding, cfg, lhs_dtype, m, n, k, w, workspace, workspace_bytes)))
         return matmul_f32(encoding, cfg, lhs, lhs_dtype, m, k, rhs, n_rhs, n, out, workspace, workspace_bytes, inner, stream, (uint16_t*)out);
@@ -574,6 +584,11 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
                                                            (const int32_t*)rhs[3], (int)m, n, k, cfg->group_size, out, n, s, only_if);
             if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order)");
             return QMM_OK;
+        }
+        if (gptq_small_wanted(encoding, cfg, lhs_dtype, m, n, k)) {
+            const bool parts = workspace && aligned(workspace, 256) && workspace_bytes >= qmm::gemv_gptq_small_workspace_bytes(lhs_dtype, m, n, k, cfg->group_size);
+            return hip_status(qmm::launch_gemv_gptq_small(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], m, n, k, cfg->group_size, out,
+                                                          out16 != nullptr, parts ? workspace : nullptr, s), "qmm_matmul(GPTQ, few rows)");
         }
         if (direct_serves(encoding, cfg, lhs_dtype, m, n, k, rhs[0], workspace, workspace_bytes))
             return hip_status(qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],

@@ -35,6 +35,9 @@ SETTINGS = [
     {"QMM_DISABLE": "kquant_mm_rounds_grid"},
     # GPTQ decode on few columns through the kernel with 64 columns per workgroup
     {"QMM_DISABLE": "gptq_cols16"},
+    # the kernels that the one for few rows takes GPTQ calls from, and GPTQ decode on few columns as above
+    {"QMM_DISABLE": "gptq_small"},
+    {"QMM_DISABLE": "gptq_small,gptq_cols16"},
     # the kernels that the direct GEMM takes a few to a few hundred rows from, and those behind them; the direct GEMM without a shared lhs
     {"QMM_DISABLE": "direct"},
     {"QMM_DISABLE": "direct,q4k_mm,q4k_tile,q4_0_small,q4_0_planes,q6k_mm,kquant_planes,gptq_mm"},
