@@ -1,4 +1,4 @@
-// Q4_K, Q5_K and Q6_K with a few lhs rows (2 .. 16 bf16, 2 .. 8 fp32) on the matrix cores, K any multiple of 256: one launch, no workspace.
+// Q4_K, Q5_K and Q6_K with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32) on the matrix cores, K any multiple of 256: one launch, no workspace.
 //
 // Shape of the work.  A workgroup has as many wavefronts, up to 16, as divide the super-blocks of a row evenly into groups: wavefront w owns super-block
 // w + waves g of group g (K = 4096: one group of 16; 14336: four of 14).  It converts the lhs columns of its super-block into matrix-core operands once a
@@ -50,7 +50,7 @@ enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
 
 }  // namespace
 
-// MROWS: lhs rows, 2, 4, 8 or 16 (>= m; rows past m repeat the last one and their results are dropped).
+// MROWS: lhs rows, 1, 2, 4, 8 or 16 (>= m; rows past m repeat the last one and their results are dropped).
 // MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up).
 struct SmallCut {
     int per, stride;  // tiles (gated: pairs) of a workgroup at most, workgroups across the tiles
@@ -464,11 +464,13 @@ template <int ENC>
 hipError_t run_small_rows(const MmMats& mats, const SmallPlan& p, const void* a, int lhs_dtype, int m, int k, bool gated, bool out_bf16, hipStream_t s) {
     if (lhs_dtype == QMM_F32) {
         const float* const f = (const float*)a;
+        if (m == 1) return run_small<ENC, 1>(mats, p, f, m, k, gated, out_bf16, s);
         if (m <= 2) return run_small<ENC, 2>(mats, p, f, m, k, gated, out_bf16, s);
         if (m <= 4) return run_small<ENC, 4>(mats, p, f, m, k, gated, out_bf16, s);
         return run_small<ENC, 8>(mats, p, f, m, k, gated, out_bf16, s);
     }
     const uint16_t* const b = (const uint16_t*)a;
+    if (m == 1) return run_small<ENC, 1>(mats, p, b, m, k, gated, out_bf16, s);
     if (m <= 2) return run_small<ENC, 2>(mats, p, b, m, k, gated, out_bf16, s);
     if (m <= 4) return run_small<ENC, 4>(mats, p, b, m, k, gated, out_bf16, s);
     if (m <= 8) return run_small<ENC, 8>(mats, p, b, m, k, gated, out_bf16, s);

@@ -385,10 +385,20 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 // - Q5_K, two fp32 rows on few columns (its decode kernel): 512 x 4096 5.0 / 5.2; 2048 x 4096 5.7 / 5.1.
 // - 9 .. 16 bf16 rows on large matrices with several groups of K, where few results fit LDS next to the ring: Q6_K 28672 x 8192 51 / 66, 4096 x 14336 9 rows 22.2 / 23.3 (16 rows 25.0 / 22.7), Q5_K 8192 x 28672
 //   47 / 51; but Q6_K 8192 x 8192 24 / 21, 5120 x 13824 38 / 24.
+// - One row (the decode kernels; 72 matrices of 256 .. 128256 rows and K of 512 .. 28672).  They stream a row per wavefront, and a short one leaves their lanes idle; those of Q5_K and Q6_K hold their loads in registers
+//   (Q6_K: unless K is a multiple of 2048).  Q4_K 32000 x 1024 11.9 / 6.4, 14336 x 2048 6.5 / 6.3, but 5632 x 2048 4.4 / 4.9, 14336 x 4096 7.4 / 8.9; Q5_K 4096 x 4096 7.1 / 5.6, 14336 x 4096 12.1 / 10.2, 4096 x 14336 16.7 / 12.4,
+//   but 1024 x 4096 4.3 / 5.0, 2048 x 8192 7.0 / 7.9; Q6_K 4096 x 4096 7.2 / 5.7, 4096 x 11008 16.4 / 11.9, 8192 x 28672 53 / 44, but 1024 x 4096 4.6 / 5.0, 128256 x 4096 77 / 86, 4096 x 14336 13.9 / 14.6.
+//   Relative error, fp32 row, K = 4096: 2.5e-7 / 1.1e-7, 1.9e-7 / 1.2e-7, 3.3e-7 / 1.0e-7.
 // - Q6_K, five and six fp32 rows, K = 256 or 512: more exact weight by weight (decode_sums_more_exactly), 0.85e-7 against 0.88e-7.
 static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
-    if (m < 2 || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
+    if (m < 1 || (m == 1 && encoding == QMM_Q4_K && (k > 2048 || n < 8192)) || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
     const bool f32 = lhs_dtype == QMM_F32;
+    if (m == 1) {
+        if (encoding == QMM_Q4_K) return true;
+        if (encoding == QMM_Q5_K) return !q5k_mm_forced() && (k <= 2048 || k > 8192 || n > 2048);
+        if (q6k_mm_forced()) return false;
+        return n <= 1024 ? k > 8192 : k <= 2048 || k % 2048 != 0 || k > 16384 || (k == 4096 && n > 2048 && n <= 14336);
+    }
     if (encoding == QMM_Q4_K) {
         if (m <= 4 && q4k_lanes_rows_forced()) return false;
         return qmm::kernel_disabled("q4k_lanes_rows") || k <= 2304 || k > 8192 ||
@@ -506,6 +516,10 @@ int qmm_matmul(int encoding, const qmm_gptq_config* cfg, const void* lhs, int lh
     if (m > 0 && n > 0 && k > 0 && m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX && n_rhs == 1 && rhs[0] &&
         (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && aligned(lhs, 16) && aligned(rhs[0], 16) && !(inner & QMM_FLAG_W_BF16) &&
         stores_bf16_itself(encoding, m, k, inner)) {
+        if (small_wanted(encoding, lhs_dtype, m, n, k, rhs[0])) {  // (one group of K: no workspace)
+            const hipError_t e = qmm::launch_gemv_kquant_small(encoding, lhs, lhs_dtype, 1, rhs, &n, &out, m, k, false, true, nullptr, (hipStream_t)stream);
+            return hip_status(e, "qmm_matmul(Q4_K, few columns, bf16 out)");
+        }
         bool handled = false;
         hipError_t e = qmm::launch_gemv_q4_k_lanes(lhs, lhs_dtype, (const uint8_t*)rhs[0], (int)m, n, k, out, n, (hipStream_t)stream, &handled, true);
         if (e != hipSuccess) return hip_status(e, "qmm_matmul(Q4_K decode, bf16 out)");

@@ -37,6 +37,21 @@ def test_against_float64(enc, lhs, m, n, k):
     check(enc, qmatmul(QE[enc], None, a, w, out_dtype=torch.bfloat16), w, a, bits=8)
 
 
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("enc,n,k", [("Q4_K", 8200, 512), ("Q4_K", 9001, 2048), *((e, n, k) for e in ("Q5_K", "Q6_K") for n, k in ((4104, 4096), (2064, 11008), (264, 14336), (2050, 256), (8192, 18944)))])
+def test_one_row(enc, lhs, n, k):
+    """The matrices on which this kernel serves one row."""
+    w, a = packed(enc, n, k), rows(1, k, lhs)
+    check(enc, qmatmul(QE[enc], None, a, w), w, a)
+    check(enc, qmatmul(QE[enc], None, a, w, out_dtype=torch.bfloat16), w, a, bits=8)
+    if enc != "Q4_K":
+        up = packed(enc, n, k, 1)
+        g, u = (qmatmul(QE[enc], None, a, x).double() for x in (w, up))
+        # the same sums but for how a long K is added up (2^-22); exp, the quotient and two products in fp32 (8 units of 2^-24)
+        want = g / (1 + torch.exp(-g)) * u
+        assert ((qmatmul_swiglu(QE[enc], a, w, up).double() - want).norm() / want.norm()).item() <= 2.0**-21
+
+
 @pytest.mark.parametrize("enc", ENCODINGS)
 @pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("scale", [1e-36, 1e-5, 3e4, 1e30])
