@@ -36,10 +36,10 @@ struct WeightTensors {
 
 // How a call is cut: every wavefront takes 32 fm rows x 32 fn columns.  wn = 1: the wk wavefronts of a workgroup take wk parts of K of one tile
 // (gemm_direct.hip).  wn > 1: wn wavefronts side by side share the lhs, wk parts of K (gemm_shared.hip, and with fn = 0, which means one, gemm_staged.hip).  shares:
-// workgroups per tile (1, or 2 that add onto zeros).  centred: gemm_staged.hip, codes of Q4_K and Q5_K around their middle.
+// workgroups per tile (1, or 2 that add onto zeros).  fold, gemm_staged.hip: sums over kStagedFold units are added up in others (staged_folds).  centred: gemm_staged.hip, codes of Q4_K and Q5_K around their middle.
 struct DirectPlan {
     int fm, fn, wk, shares, wn;
-    bool centred = false;
+    bool centred = false, fold = false;
 };
 hipError_t launch_gemm_shared(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
                               int64_t m, int units, hipStream_t s);
@@ -48,6 +48,9 @@ hipError_t launch_gemm_staged(int encoding, bool hilo, const DirectPlan& pl, con
 
 // What gemm_staged.hip has: fp32 rows, small groups and codes around their middle, which all sum a unit of K by itself, leave no registers for 128 rows a wavefront.
 constexpr bool staged_built(int encoding, int flush, int fm, bool hilo, bool centred) { return fm <= 3 || !(hilo || centred || (encoding == QMM_GPTQ && flush == 2)); }
+// What folds its sums there: GPTQ in groups of 128 and more, where there are registers for a second set.
+constexpr int kStagedFold = 4;  // units
+constexpr bool staged_folds(int encoding, int flush, int fm, bool hilo) { return encoding == QMM_GPTQ && flush == 8 && fm <= (hilo ? 2 : 3); }
 
 namespace {
 

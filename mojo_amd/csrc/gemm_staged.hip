@@ -257,7 +257,7 @@ struct StagedLds {
     static constexpr int kW = lhs(kSteps, kBufs), kS = kW + kWeights, kInv = std::max(kS + kSums, kResults), kBytes = kInv + kInvBytes;
 };
 
-template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER>
+template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER, bool FOLD>
 __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
                                                             int shares) {
     using W = StagedOf<ENC, FLUSH, CENTER>;
@@ -289,13 +289,16 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTens
     // off by 2.30e-7 instead of 2.04e-7 after sums of 40 units, Q5_K with bf16 rows by 1.06e-7 instead of 0.99e-7; for codes from 0 the error is that of larger
     // terms.  Never a question of FM: matrices that share a launch share its tile, and keep the bits that calls of their own give.)
     constexpr bool kUnit = unit_sums(ENC, FLUSH, HILO) || (W::kMin && (HILO || CENTER));
-    float16v T[FM], P[FM], M, U[kUnit ? FM : 1];
+    // FOLD: sums over kStagedFold units are added up in others, so that a workgroup that walks all of K is as exact as wavefronts with a part of it each (K = 4096, bf16 rows: 1.03e-7
+    // relative error, folded 0.68e-7, as the direct kernel with four parts).  A fold takes two instructions a value, 1 .. 5 % of a call.
+    float16v T[FM], P[FM], M, U[kUnit ? FM : 1], S[FOLD ? FM : 1];
 #pragma unroll
     for (int a = 0; a < FM; a++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             T[a][r] = 0.0f, P[a][r] = 0.0f;
             if constexpr (kUnit) U[a][r] = 0.0f;
+            if constexpr (FOLD) S[a][r] = 0.0f;
         }
     const float16v zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     const uint32_t l16 = lane * 16;
@@ -399,6 +402,12 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTens
                     }
                     if constexpr (!kUnit || t == 0) asm volatile("" : "+v"(T[a]));
                     else asm volatile("" : "+v"(U[a]));
+                    if constexpr (FOLD && t == 0) {
+                        if (it > 0 && it % kStagedFold == 0) {
+#pragma unroll
+                            for (int r = 0; r < 16; r++) S[a][r] += T[a][r], T[a][r] = 0.0f;
+                        }
+                    }
 #pragma unroll
                     for (int pl = 0; pl < W::kPlanes; pl++)
 #pragma unroll
@@ -444,7 +453,10 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTens
 #pragma unroll
     for (int a = 0; a < FM; a++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) T[a][r] = kUnit ? T[a][r] + fmaf(d, P[a][r], U[a][r]) : fmaf(d, P[a][r], T[a][r]);
+        for (int r = 0; r < 16; r++) {
+            T[a][r] = kUnit ? T[a][r] + fmaf(d, P[a][r], U[a][r]) : fmaf(d, P[a][r], T[a][r]);
+            if constexpr (FOLD) T[a][r] += S[a][r];
+        }
     wait_vmcnt<0>();
     __syncthreads();  // nothing is on its way into the buffers any more, which now take the results
     constexpr int kTile = 64 * result_row(32);
@@ -459,16 +471,16 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTens
     }
 }
 
-template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER>
+template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER, bool FOLD = false>
 hipError_t run_staged(const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units, int shares, hipStream_t s) {
     using L = StagedLds<ENC, FLUSH, FM, WN, WK, HILO, CENTER>;
     static_assert(L::kBytes <= kLdsPerCu, "fits a compute unit");
     const int tiles_m = (int)((m + 32 * FM - 1) / (32 * FM));
     int eights = 0;
     for (int j = 0; j < mats.count; j++) mats.end[j] = eights += (mats.n[j] + 256 * WN - 1) / (256 * WN);
-    hipError_t e = allow_full_lds<gemm_staged_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER>>();
+    hipError_t e = allow_full_lds<gemm_staged_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER, FOLD>>();
     if (e != hipSuccess) return e;
-    gemm_staged_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER><<<dim3(8, (unsigned)tiles_m, (unsigned)(eights * shares)), dim3(64 * WN * WK), L::kBytes, s>>>(wt, mats, p, out16,
+    gemm_staged_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER, FOLD><<<dim3(8, (unsigned)tiles_m, (unsigned)(eights * shares)), dim3(64 * WN * WK), L::kBytes, s>>>(wt, mats, p, out16,
                                                                                                                                (int)m, units, shares);
     return hipGetLastError();
 }
@@ -476,6 +488,8 @@ hipError_t run_staged(const WeightTensors& wt, DirectMats mats, const DirectSpac
 template <int ENC, int FLUSH, bool HILO, bool CENTER = false>
 hipError_t run_staged_plan(const DirectPlan& pl, const WeightTensors& wt, const DirectMats& mats, const DirectSpace& p, uint16_t* out16, int64_t m, int units, hipStream_t s) {
 #define QMM_GS(FM, WN, WK)                       \
+    if constexpr (staged_folds(ENC, FLUSH, FM, HILO)) \
+        if (pl.fold && pl.fm == FM && pl.wn == WN && pl.wk == WK) return run_staged<ENC, FLUSH, FM, WN, WK, HILO, CENTER, true>(wt, mats, p, out16, m, units, pl.shares, s); \
     if constexpr (staged_built(ENC, FLUSH, FM, HILO, CENTER)) \
         if (pl.fm == FM && pl.wn == WN && pl.wk == WK) return run_staged<ENC, FLUSH, FM, WN, WK, HILO, CENTER>(wt, mats, p, out16, m, units, pl.shares, s)
     QMM_GS(2, 2, 4);

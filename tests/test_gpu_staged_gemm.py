@@ -5,7 +5,7 @@ import ctypes as C
 import pytest
 import torch
 
-from mojo_amd import QuantizationEncoding as QE, _lib, qmatmul, qmatmul_grouped
+from mojo_amd import QuantizationEncoding as QE, _lib, dequantize, qmatmul, qmatmul_grouped
 from test_gpu_direct_gemm import check, weights
 
 pytestmark = pytest.mark.gpu
@@ -25,6 +25,17 @@ def test_edges(enc, group, lhs):
         a[m - 1] = 0.0
         check(qmatmul(enc, config, a, *rhs), enc, config, rhs, a)
         check(qmatmul(enc, config, a, *rhs, out_dtype=torch.bfloat16), enc, config, rhs, a)
+
+
+@pytest.mark.parametrize("lhs,m,n,k,limit", [(torch.bfloat16, 160, 11008, 4096, 0.75e-7), (torch.bfloat16, 190, 11008, 2816, 0.76e-7), (torch.float32, 160, 14336, 4096, 1.33e-7),
+                                               (torch.float32, 160, 11008, 5376, 1.37e-7)])
+def test_folded_sums(lhs, m, n, k, limit):
+    """Sums over four units of K that are added up in others (16, 11 and 21 units): a tenth above 0.67e-7, 0.69e-7, 1.21e-7 and 1.25e-7, where one chain over 16 has 1.03e-7
+    (fp32 rows: 1.43e-7)."""
+    config, rhs = weights(QE.GPTQ, 128, n, k)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m + k)).to(lhs)
+    want = a.double() @ dequantize(QE.GPTQ, *rhs, config=config).double().T
+    assert ((qmatmul(QE.GPTQ, config, a, *rhs).double() - want).norm() / want.norm()).item() <= limit
 
 
 @pytest.mark.parametrize("n", [2048 + 1, 14336 - 3])
