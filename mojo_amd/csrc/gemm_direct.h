@@ -48,6 +48,8 @@ hipError_t launch_gemm_staged(int encoding, bool hilo, const DirectPlan& pl, con
 
 // What gemm_staged.hip has: fp32 rows, small groups and codes around their middle, which all sum a unit of K by itself, leave no registers for 128 rows a wavefront.
 constexpr bool staged_built(int encoding, int flush, int fm, bool hilo, bool centred) { return fm <= 3 || !(hilo || centred || (encoding == QMM_GPTQ && flush == 2)); }
+// The last row tile of 32 fm rows as one of 32: where that is all it has, and not the only one (sections: workgroups of a row tile on an XCD; the grid's z has 16 bits).
+inline bool staged_short_last(int fm, int64_t m, int64_t sections) { return m > 32 * fm && (m - 1) % (32 * fm) < 32 && 2 * sections < 65536; }
 // What folds its sums there: GPTQ in groups of 128 and more, where there are registers for a second set.
 constexpr int kStagedFold = 4;  // units
 constexpr bool staged_folds(int encoding, int flush, int fm, bool hilo) { return encoding == QMM_GPTQ && flush == 8 && fm <= (hilo ? 2 : 3); }

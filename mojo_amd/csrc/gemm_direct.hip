@@ -515,6 +515,18 @@ Rounds rounds_of(int64_t wgs, bool pairs) {
     const int64_t cus = compute_units() / 8, deep = (wgs + cus - 1) / cus;
     return pairs ? Rounds{(deep + 1) / 2, deep / 2, deep % 2} : Rounds{deep, deep, 0};
 }
+// When the tiles of a launch of the staged kernel are done: `full` of them and then `last`, which take a and b us, per XCD.
+double staged_tiles_us(int64_t full, int64_t last, double a, double b) {
+    const int64_t cus = compute_units() / 8, busy = full % cus;  // compute units that take one more of the full ones than the others
+    double some = (double)(full / cus) * a, most = busy ? some + a : some, end = most;
+    for (int64_t left = last; left > 0;) {
+        double& free = busy && most < some ? most : some;
+        left -= &free == &most ? busy : cus - busy;
+        free += b;
+        end = std::max(end, free);
+    }
+    return end;
+}
 double direct_us(const DirectCost& c, int plan, int shares, int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const DirectPlan& p = kDirectPlans[plan];
     if (c.unit[plan] == 0.0f) return 1e30;
@@ -578,6 +590,13 @@ int staged_row(int encoding, int group) {
     return encoding == QMM_Q4_K ? 0 : encoding == QMM_Q5_K ? 1 : encoding == QMM_Q6_K ? 2 : encoding == QMM_GPTQ ? (group % 128 == 0 ? 3 : 4) : -1;
 }
 double packed_mb(int encoding, int64_t n, int64_t k) { return (encoding == QMM_Q6_K ? 0.82 : encoding == QMM_Q5_K ? 0.69 : 0.56) * n * k * 1e-6; }
+// The tiles of one plan on `sections` column sections.  A last row tile of up to 32 rows takes 0.8 of the unit of one of 64.
+double staged_tiles_us(const StagedCost& c, int i, int64_t m, int64_t sections, int64_t walk) {
+    const DirectPlan& p = kStagedPlans[i];
+    const bool short_last = staged_short_last(p.fm, m, sections);
+    const int64_t full = short_last ? m / (32 * p.fm) : (m + 32 * p.fm - 1) / (32 * p.fm);
+    return staged_tiles_us(full * sections, short_last ? sections : 0, c.round + walk * c.unit[i], c.round + walk * 0.8 * c.unit[p.wn == 2 ? 0 : p.wn == 4 ? 1 : 2]);
+}
 // What a plan's fp32 sums cost: the square of the relative error of the results (2-norm, against 64 bits) in units of 2^-48 / 6, the mean square of a rounding
 // halved.  An addition counts by the share of K that its sum holds by then: `unit` times half the squares of the parts' lengths, `join` for adding the parts up
 // in order; `first`: additions to zero, which are exact; `length`: what grows with K however it is cut.  Fitted to every plan on 22 K of 256 .. 28672
@@ -643,8 +662,7 @@ double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k,
             p.shares = shares;
             const int64_t parts = p.wk * shares, walk = (direct_units(k) + parts - 1) / parts;
             if (!staged_has(c, i, centred)) continue;
-            const int64_t rounds = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * shares, false).all;
-            const double t = c.base + rounds * (c.round + walk * c.unit[i]) + c.weights * packed_mb(encoding, n, k) + c.lhs * (m * k * 1e-6) +
+            const double t = c.base + staged_tiles_us(c, i, m, (n + 256 * p.wn - 1) / (256 * p.wn) * shares, walk) + c.weights * packed_mb(encoding, n, k) + c.lhs * (m * k * 1e-6) +
                              (c.out + c.share * (shares - 1)) * (m * n * 1e-6);
             if (walk <= longest && t < us && sums_error(e, p, direct_units(k)) <= most) us = t, best = p;
             // (folded sums: 1.03, 14336 x 4096 with 160 bf16 rows 33.3 -> 35.0 us)
@@ -695,7 +713,7 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
             const int i = (int)(&p - kStagedPlans);
             if (!staged_has(c, i, like->centred) || p.wk != like->wk) continue;
             const int64_t walk = (direct_units(k) + p.wk * like->shares - 1) / (p.wk * like->shares);
-            const double t = rounds_of((m + 32 * p.fm - 1) / (32 * p.fm) * ((n + 256 * p.wn - 1) / (256 * p.wn)) * like->shares, false).all * (c.round + walk * c.unit[i]);
+            const double t = staged_tiles_us(c, i, m, (n + 256 * p.wn - 1) / (256 * p.wn) * like->shares, walk);
             if (t < us) us = t, best = p, best.shares = like->shares, best.centred = like->centred;
         }
         return best;
