@@ -1,4 +1,4 @@
-// Q4_K, Q5_K and Q6_K with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32) on the matrix cores, K any multiple of 256: one launch, no workspace.
+// Q4_0, Q4_K, Q5_K and Q6_K with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32) on the matrix cores, K any multiple of 256: one launch, no workspace.
 //
 // Shape of the work.  A workgroup has as many wavefronts, up to 16, as divide the super-blocks of a row evenly into groups: wavefront w owns super-block
 // w + waves g of group g (K = 4096: one group of 16; 14336: four of 14).  It converts the lhs columns of its super-block into matrix-core operands once a
@@ -22,6 +22,7 @@
 //   Q4_K: a masked nibble is the subnormal q * 2^-24 (or 16 q * 2^-24), one packed multiply-add leaves sc * (q - 8) * 2^-18.
 //   Q5_K: a byte permute puts nibble and fifth bit under 0x54: 64 + q; one packed multiply-add, (64 + q) * sc - 80 * sc, leaves sc * (q - 16) (exact: below 2^11).
 //   Q6_K: the same with 96 taken off; sc * q may need 13 bits, so the scale multiplies the results of its 16 weights instead.
+//   Q4_0 (an item is 16 rows x eight blocks): the lhs as Q8_0, quantised as any Q8_0 lhs here, int8 products of 16 (q - 8), whose sums over a block are exact; sum of (sum / 16) * (d_w d_a).
 //   What codes around their middle leave out (Q4_K, Q5_K): mid * d * sc - dmin * mn times the sum of 32 lhs values, both as two fp16 terms, one more matrix product a super-block.
 #include <stdlib.h>
 
@@ -41,7 +42,7 @@ constexpr int kSmallWaves = 16;
 // spreads the rows over the banks.
 template <int ENC>
 struct SmallItem {
-    static constexpr int kBpb = ENC == QMM_Q4_K ? Q4_K_BPB : ENC == QMM_Q5_K ? Q5_K_BPB : Q6_K_BPB;
+    static constexpr int kBpb = ENC == QMM_Q4_0 ? 8 * Q4_0_BPB : ENC == QMM_Q4_K ? Q4_K_BPB : ENC == QMM_Q5_K ? Q5_K_BPB : Q6_K_BPB;  // of 256 columns
     static constexpr int kRow = ENC == QMM_Q6_K ? 240 : kBpb, kRowPieces = kRow / 16, kPieces = 16 * kRowPieces, kLoads = (kPieces + 63) / 64, kSlot = 16 * kRow;
     static_assert(4 * kSmallPlane + 16 <= kSlot, "four planes of lhs rows and their scales fit a ring slot");
 };
@@ -59,12 +60,13 @@ struct SmallCut {
 template <int ENC, int MROWS, typename AT, int MODE>
 __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restrict__ a, int m, int k, const SmallCut& cut) {
     using I = SmallItem<ENC>;
-    constexpr int PL = sizeof(AT) == 4 ? 2 : 1;             // operand rows of an lhs row
+    constexpr bool kQ8 = ENC == QMM_Q4_0;                   // the lhs as Q8_0 codes and block scales
+    constexpr int PL = sizeof(AT) == 4 && !kQ8 ? 2 : 1;     // operand rows of an lhs row
     constexpr int LR = MROWS <= 4 ? 1 : MROWS / 4;          // lhs rows of a lane's results: lane / 16 + 4 j
     constexpr int RN = LR * PL;
     constexpr int kPass = std::min(MROWS, 4 / PL);          // lhs rows that change lanes together
     static_assert(RN <= 4, "operand rows");
-    constexpr bool kMin = ENC != QMM_Q6_K;
+    constexpr bool kMin = ENC == QMM_Q4_K || ENC == QMM_Q5_K;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     // (what follows from the launch comes as arguments: the compiler fetches blockDim and gridDim with a vector load and waits for it)
@@ -123,11 +125,18 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
 
     // ---- lhs operands of the wavefront's super-block.  Operand row nn: lhs row nn / 4 + 4 j, hi part or (fp32) residual, j and part by nn % 4.
     // Q4_K, Q5_K: fragment (p, h) of lane quarter kg holds columns 64 kg + 32 h + 8 p + (0 .. 7; Q4_K in the order 0,2,1,3,4,6,5,7); Q6_K: fragment g holds 16 g + 4 kg + 0 .. 3.
-    half8 fa[ENC == QMM_Q6_K ? 1 : 4][2], fs;
+    // Q4_0: block b of lane quarter kg holds the codes of columns 4 kg .. + 3 and 16 + 4 kg .. + 3; block scales of this lane's results, two fp16 numbers a register.
+    half8 fa[kMin ? 4 : 1][2], fs;
     ks_half4 fq[ENC == QMM_Q6_K ? 16 : 1];
+    u32x2 fc[kQ8 ? 8 : 1];
+    u32x4 fd[kQ8 ? LR : 1];
     float bs[LR];  // inverse lhs scales of this lane's results
 #pragma unroll
-    for (int p = 0; p < (ENC == QMM_Q6_K ? 1 : 4); p++) fa[p][0] = fa[p][1] = pack4(0u, 0u, 0u, 0u);
+    for (int b = 0; b < (kQ8 ? 8 : 1); b++) fc[b] = u32x2{0u, 0u};
+#pragma unroll
+    for (int j = 0; j < (kQ8 ? LR : 1); j++) fd[j] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int p = 0; p < (kMin ? 4 : 1); p++) fa[p][0] = fa[p][1] = pack4(0u, 0u, 0u, 0u);
 #pragma unroll
     for (int g = 0; g < (ENC == QMM_Q6_K ? 16 : 1); g++) fq[g] = ks_half4{0, 0, 0, 0};
     fs = pack4(0u, 0u, 0u, 0u);
@@ -139,27 +148,44 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));  // (what is computed from it here is not kept in registers between the groups)
         const int nn = lane & 15, kg = lane >> 4, my_row = (nn >> 2) + 4 * ((nn & 3) / PL), my_part = (nn & 3) % PL;
-        float* const scales = (float*)(area + 4 * kSmallPlane);
+        if constexpr (kQ8) {
 #pragma unroll
-        for (int r0 = 0; r0 < MROWS; r0 += kPass) {
-            const bool scaled = small_narrow<PL, kPass, ENC == QMM_Q4_K ? kSmallOrderK : kSmallOrderPlain>(xr, r0, area, scales, lane);
-            __builtin_amdgcn_wave_barrier();
-            if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
-                const uint8_t* const pl = area + ((my_row - r0) * PL + my_part) * kSmallPlane;
-                if constexpr (ENC == QMM_Q6_K) {
+            for (int r0 = 0; r0 < MROWS; r0 += kPass) {
+                small_quantize<kPass>(xr, r0, area, lane);
+                asm volatile("" ::: "memory");  // (scales are written as 16-bit numbers and read as vectors: not to be reordered)
+                __builtin_amdgcn_wave_barrier();
+                if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
+                    const uint8_t* const pl = area + (my_row - r0) * kSmallCodes;
 #pragma unroll
-                    for (int g = 0; g < 16; g++) fq[g] = *(const ks_half4*)(pl + 32 * g + 8 * kg);
-                } else {
+                    for (int b = 0; b < 8; b++) fc[b] = *(const u32x2*)(pl + 32 * b + 8 * kg);
+                }
 #pragma unroll
-                    for (int p = 0; p < 4; p++) {
-                        fa[p][0] = *(const half8*)(pl + 128 * kg + 16 * p);
-                        fa[p][1] = *(const half8*)(pl + 128 * kg + 64 + 16 * p);
+                for (int j = 0; j < LR; j++)
+                    if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) fd[j] = *(const u32x4*)(area + (kg + 4 * j - r0) * kSmallCodes + 256);
+            }
+        } else {
+            float* const scales = (float*)(area + 4 * kSmallPlane);
+#pragma unroll
+            for (int r0 = 0; r0 < MROWS; r0 += kPass) {
+                const bool scaled = small_narrow<PL, kPass, ENC == QMM_Q4_K ? kSmallOrderK : kSmallOrderPlain>(xr, r0, area, scales, lane);
+                __builtin_amdgcn_wave_barrier();
+                if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
+                    const uint8_t* const pl = area + ((my_row - r0) * PL + my_part) * kSmallPlane;
+                    if constexpr (ENC == QMM_Q6_K) {
+#pragma unroll
+                        for (int g = 0; g < 16; g++) fq[g] = *(const ks_half4*)(pl + 32 * g + 8 * kg);
+                    } else {
+#pragma unroll
+                        for (int p = 0; p < 4; p++) {
+                            fa[p][0] = *(const half8*)(pl + 128 * kg + 16 * p);
+                            fa[p][1] = *(const half8*)(pl + 128 * kg + 64 + 16 * p);
+                        }
                     }
                 }
-            }
 #pragma unroll
-            for (int j = 0; j < LR; j++)
-                if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = scaled ? scales[kg + 4 * j - r0] : 1.0f;
+                for (int j = 0; j < LR; j++)
+                    if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = scaled ? scales[kg + 4 * j - r0] : 1.0f;
+            }
         }
         if constexpr (kMin) {
             // Sums of the operand rows over 32 columns on the matrix cores: column j < 4 of the product is sub-block 2 j (the lane quarter kg = j supplies the ones),
@@ -205,7 +231,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
     }
     // (constants of the unpack in vector registers: an and-or in one instruction takes no literal and one scalar at most)
     uint32_t m_low = ENC == QMM_Q5_K ? 0x01010101u : 0x03030303u, c54 = 0x54545454u;
-    if constexpr (ENC != QMM_Q4_K) asm volatile("" : "+v"(m_low), "+v"(c54));
+    if constexpr (ENC == QMM_Q5_K || ENC == QMM_Q6_K) asm volatile("" : "+v"(m_low), "+v"(c54));
     const ks_float4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
     for (int c0 = 0; c0 < my_items; c0 += chunk) {
@@ -235,7 +261,32 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
                 }
                 const uint8_t* const lb = ring + slot * I::kSlot + nn * I::kRow;
                 float v[LR];
-                if constexpr (ENC == QMM_Q6_K) {
+                if constexpr (kQ8) {
+                    // codes less 8, times 16, as signed bytes: the dot products of a block come out exact; v = sum of dot / 16 * (d_w d_a), the product of two fp16 numbers exact in fp32
+                    const uint32_t* const l32 = (const uint32_t*)lb;
+                    float u[2][LR];  // two chains of sums
+#pragma unroll
+                    for (int j = 0; j < LR; j++) u[0][j] = u[1][j] = 0.0f;
+#pragma unroll
+                    for (int b = 0; b < 8; b++) {
+                        const int at = (18 * b + 2) >> 2;
+                        uint32_t x;  // the block begins at 0 or 2 mod 4
+                        if ((18 * b + 2) % 4 == 0) x = l32[at + kg];
+                        else x = __builtin_amdgcn_alignbyte(l32[at + kg + 1], l32[at + kg], 2);
+                        const half2v dp = __builtin_bit_cast(half2v, l32[(18 * b) >> 2]);
+                        const _Float16 dw = (18 * b) % 4 ? dp.y : dp.x;
+                        const u32x2 w = {((x << 4) & 0xF0F0F0F0u) ^ 0x80808080u, (x & 0xF0F0F0F0u) ^ 0x80808080u};
+                        const ks_int4 dot = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, fc[b]), __builtin_bit_cast(long, w), ks_int4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < LR; j++) {
+                            const uint32_t pair = fd[j][b >> 1];  // (a bit cast of the element itself takes the first one)
+                            const half2v da2 = __builtin_bit_cast(half2v, pair);
+                            u[b & 1][j] = fmaf((float)dot[j], fmaf((float)dw, (float)(b & 1 ? da2.y : da2.x), 0.0f), u[b & 1][j]);
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < LR; j++) v[j] = 0.0625f * (u[0][j] + u[1][j]);
+                } else if constexpr (ENC == QMM_Q6_K) {
                     const uint32_t* const l32 = (const uint32_t*)lb;
                     const uint32_t skew = 2u * (((uint32_t)nn * (uint32_t)nblk + (uint32_t)sb) & 1u);  // (16 rows of a tile: n0 is even)
                     auto rd = [&](int dw) __attribute__((always_inline)) { return __builtin_amdgcn_alignbyte(l32[dw + 1], l32[dw], skew); };
@@ -336,7 +387,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
                 }
                 float* const mine = accs + ((t * waves + wave) * LR) * 64 + lane;
 #pragma unroll
-                for (int j = 0; j < LR; j++) mine[j * 64] = bs[j] * v[j];
+                for (int j = 0; j < LR; j++) mine[j * 64] = kQ8 ? v[j] : bs[j] * v[j];
                 slot ^= 1;
             }
             }
@@ -420,7 +471,7 @@ SmallPlan small_plan(int encoding, int64_t m, int64_t tiles, int64_t k, bool gat
     const int64_t most = std::max<int64_t>(1, (int64_t)compute_units() * per_cu / p.parts);
     p.per = (int)((tiles + most - 1) / most);
     p.grid = (int)((tiles + p.per - 1) / p.per);
-    const int slot = encoding == QMM_Q4_K ? SmallItem<QMM_Q4_K>::kSlot : encoding == QMM_Q5_K ? SmallItem<QMM_Q5_K>::kSlot : SmallItem<QMM_Q6_K>::kSlot;
+    const int slot = encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? SmallItem<QMM_Q4_K>::kSlot : encoding == QMM_Q5_K ? SmallItem<QMM_Q5_K>::kSlot : SmallItem<QMM_Q6_K>::kSlot;
     // (as many items between two barriers as fit: a barrier after each, with two buffers, took Q6_K 28672 x 8192 with 16 rows from 65 to 92 us)
     const int lr = m <= 4 ? 1 : m <= 8 ? 2 : 4, ring = p.waves * 2 * slot, each = (p.waves + (groups > p.parts ? 1 : 0)) * lr * 256, items = gated ? 2 * p.per : p.per;
     p.chunk = std::min(std::min(items, 254), (kLdsPerCu / per_cu - ring) / each);
@@ -434,8 +485,9 @@ SmallPlan small_plan(int encoding, int64_t m, int64_t tiles, int64_t k, bool gat
 bool small_parts(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const int groups = small_groups(k);
     if (groups < 2) return false;
-    const double item = encoding == QMM_Q4_K ? 1.4 : encoding == QMM_Q5_K ? 1.75 : 2.1;  // a tile of one group; convert: the lhs of one
-    const double convert = lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
+    const double item = encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? 1.4 : encoding == QMM_Q5_K ? 1.75 : 2.1;  // a tile of one group; convert: the lhs of one
+    const double convert = encoding == QMM_Q4_0 ? (m <= 2 ? 1.2 : m <= 4 ? 1.6 : m <= 8 ? 2.6 : 5.0)
+                           : lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
     const int64_t tiles = (n + 15) / 16;
     const SmallPlan w = small_plan(encoding, m, tiles, k, false, false), a = small_plan(encoding, m, tiles, k, false, true);
     const double walk = groups * ((w.per + w.chunk - 1) / w.chunk) * convert + groups * w.per * item;
@@ -480,11 +532,12 @@ hipError_t run_small_rows(const MmMats& mats, const SmallPlan& p, const void* a,
 }  // namespace
 
 bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
-    if (encoding != QMM_Q4_K && encoding != QMM_Q5_K && encoding != QMM_Q6_K) return false;
+    if (encoding != QMM_Q4_0 && encoding != QMM_Q4_K && encoding != QMM_Q5_K && encoding != QMM_Q6_K) return false;
     // (with the name of an encoding's older small-batch kernel this one goes too)
-    if (kernel_disabled("kquant_small") || kernel_disabled(encoding == QMM_Q4_K ? "q4k_mm" : encoding == QMM_Q5_K ? "q5k_mm" : "q6k_mm")) return false;
+    if (kernel_disabled("kquant_small") || kernel_disabled(encoding == QMM_Q4_0 ? "q4_0_small" : encoding == QMM_Q4_K ? "q4k_mm" : encoding == QMM_Q5_K ? "q5k_mm" : "q6k_mm")) return false;
     if (m < 1 || m > (lhs_dtype == QMM_F32 ? 8 : 16) || n < 1 || n > 0x7fffff00 || k < 256 || k % 256 || k > (1 << 20)) return false;
     if (encoding == QMM_Q4_K || encoding == QMM_Q5_K) return ((uintptr_t)w & 15) == 0;
+    if (encoding == QMM_Q4_0) return ((uintptr_t)w & 3) == 0;
     // (loads of four bytes at least: the last block of the matrix has to end at a multiple of four)
     return ((uintptr_t)w & 3) == 0 && n * (k / 256) % 2 == 0;
 }
@@ -529,7 +582,8 @@ hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype
     if (parts) mats.out[0] = (float*)workspace;
     const SmallPlan p = small_plan(encoding, m, gated ? tiles / 2 : tiles, k, gated, parts);
     const bool store_bf16 = out_bf16 && !parts;
-    hipError_t e = encoding == QMM_Q4_K   ? run_small_rows<QMM_Q4_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
+    hipError_t e = encoding == QMM_Q4_0   ? run_small_rows<QMM_Q4_0>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
+                   : encoding == QMM_Q4_K ? run_small_rows<QMM_Q4_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                    : encoding == QMM_Q5_K ? run_small_rows<QMM_Q5_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                                           : run_small_rows<QMM_Q6_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s);
     if (e != hipSuccess || !parts) return e;

@@ -378,7 +378,7 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
            workspace_bytes >= qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k);
 }
 
-// K-quants with a few lhs rows: the kernel with a super-block per wavefront, unless one of the others is faster.
+// Block encodings with a few lhs rows: the kernel with a super-block per wavefront, unless one of the others is faster.
 // us, that other / here (weights from memory), over 42 matrices of 256 .. 128256 rows and K of 512 .. 28672 with 2 .. 16 rows:
 // - Q4_K, two to four rows, few long rows (the decode kernel with a sub-block per lane): 1024 x 4096 2 rows 4.0 / 4.7, 4 fp32 rows 5.2 / 5.5 (bf16 4.95 / 4.97), 2048 x 4096 2 rows 4.9 / 5.1,
 //   1024 x 8192 2 rows 4.9 / 7.1, 4 bf16 rows 6.5 / 7.4 (fp32 10.1 / 7.9); but 1024 x 2048 4 rows 4.9 / 4.3, 1024 x 11008 4 rows 13.7 / 6.9.
@@ -389,13 +389,17 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 //   (Q6_K: unless K is a multiple of 2048).  Q4_K 32000 x 1024 11.9 / 6.4, 14336 x 2048 6.5 / 6.3, but 5632 x 2048 4.4 / 4.9, 14336 x 4096 7.4 / 8.9; Q5_K 4096 x 4096 7.1 / 5.6, 14336 x 4096 12.1 / 10.2, 4096 x 14336 16.7 / 12.4,
 //   but 1024 x 4096 4.3 / 5.0, 2048 x 8192 7.0 / 7.9; Q6_K 4096 x 4096 7.2 / 5.7, 4096 x 11008 16.4 / 11.9, 8192 x 28672 53 / 44, but 1024 x 4096 4.6 / 5.0, 128256 x 4096 77 / 86, 4096 x 14336 13.9 / 14.6.
 //   Relative error, fp32 row, K = 4096: 2.5e-7 / 1.1e-7, 1.9e-7 / 1.2e-7, 3.3e-7 / 1.0e-7.
+// - Q4_0 against its decode kernel (one and two rows; three and four up to K = 4096) and the lhs quantised by a launch of its own (21 matrices): 1 row 8192 x 28672 42 / 31, 32000 x 512 11.6 / 4.6, but 4096 x 4096 4.4 / 4.7; 2 rows
+//   4096 x 4096 5.5 / 4.9, 4096 x 14336 16.7 / 10.9, but 2048 x 5632 6.0 / 7.2, 28672 x 8192 25 / 27; 4 rows 4096 x 4096 7.4 / 5.4, 14336 x 4096 12.7 / 9.5; 8 rows 8.7 / 6.7, 13.4 / 10.4, 4096 x 14336 16.7 / 12.6;
+//   16 bf16 rows 32000 x 512 13.0 / 10.5, 1024 x 14336 14.7 / 12.4, but 4096 x 4096 8.7 / 10.2.
 // - Q6_K, five and six fp32 rows, K = 256 or 512: more exact weight by weight (decode_sums_more_exactly), 0.85e-7 against 0.88e-7.
 static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
-    if (m < 1 || (m == 1 && encoding == QMM_Q4_K && (k > 2048 || n < 8192)) || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
+    if (m < 1 || (m == 1 && (encoding == QMM_Q4_K || encoding == QMM_Q4_0) && k <= 14528 && (k > 2048 || n < 8192)) || (m == 1 && encoding == QMM_Q4_K && k > 2048) || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
     const bool f32 = lhs_dtype == QMM_F32;
     if (m == 1) {
         if (encoding == QMM_Q4_K) return true;
         if (encoding == QMM_Q5_K) return !q5k_mm_forced() && (k <= 2048 || k > 8192 || n > 2048);
+        if (encoding == QMM_Q4_0) return k > 14528 || (k <= 1536 && n >= 8192);
         if (q6k_mm_forced()) return false;
         return n <= 1024 ? k > 8192 : k <= 2048 || k % 2048 != 0 || k > 16384 || (k == 4096 && n > 2048 && n <= 14336);
     }
@@ -404,6 +408,8 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
         return qmm::kernel_disabled("q4k_lanes_rows") || k <= 2304 || k > 8192 ||
                !((m == 2 && (n <= 1024 || (k <= 4096 && n * k <= ((int64_t)8 << 20)))) || (m <= 4 && n <= 1024 && f32 == (k <= 4096)));
     }
+    if (encoding == QMM_Q4_0)
+        return m == 2 ? k > 8192 || ((n > 2048 || k <= 2048) && n * k <= (int64_t)64 << 20) : m <= 8 || k <= 1024 || (n <= 2048 && k <= 2048) || (n <= 1024 && k > 8192);
     const bool large = m > 8 && k > 4096;
     if (encoding == QMM_Q5_K) return !q5k_mm_forced() && !(f32 && m == 2 && n <= 1024 && k > 2304 && k <= 4096) && !(large && n * k >= ((int64_t)190 << 20));
     if (f32 && (m == 5 || m == 6) && k <= 512) return false;

@@ -10,6 +10,7 @@ typedef _Float16 ks_half4 __attribute__((ext_vector_type(4)));
 typedef float ks_float4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float2v __attribute__((ext_vector_type(2)));
+typedef int ks_int4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSmallPlane = 528;  // an lhs row of 256 columns on its way between lanes: 512 bytes + 16 (bank spread)
 
@@ -105,6 +106,51 @@ __device__ __forceinline__ bool small_narrow(const RAW (&xr)[ROWS], int r0, uint
         }
     }
     return scaled;
+}
+
+constexpr int kSmallCodes = 272;  // an lhs row of 256 columns as Q8_0: codes, block by block in the order of small_quantize, then the eight block scales
+
+// Rows r0 .. r0 + PASS - 1 (at most four) as Q8_0 to `area`, kSmallCodes bytes each.  The 32 codes of a block in eight dwords: columns 4 i .. 4 i + 3 and 16 + 4 i .. + 3 lie in dwords 2 i and 2 i + 1.
+// Eight lanes hold a block of every row; the divisions of a block's rule are made once for four rows, by the lane whose number is the row's.
+template <int PASS, typename RAW, int ROWS>
+__device__ __forceinline__ void small_quantize(const RAW (&xr)[ROWS], int r0, uint8_t* area, int lane) {
+    static_assert(PASS <= 4, "a lane of four for each row");
+    float x[PASS][4], amax[PASS];
+#pragma unroll
+    for (int j = 0; j < PASS; j++) {
+        const RAW raw = xr[r0 + j];
+        if constexpr (sizeof(RAW) == 16) {
+            x[j][0] = __uint_as_float(raw.x), x[j][1] = __uint_as_float(raw.y), x[j][2] = __uint_as_float(raw.z), x[j][3] = __uint_as_float(raw.w);
+        } else {
+            x[j][0] = __uint_as_float(raw.x << 16), x[j][1] = __uint_as_float(raw.x & 0xffff0000u);
+            x[j][2] = __uint_as_float(raw.y << 16), x[j][3] = __uint_as_float(raw.y & 0xffff0000u);
+        }
+        float mx = fmaxf(fmaxf(fmaxf(fabsf(x[j][0]), fabsf(x[j][1])), fabsf(x[j][2])), fabsf(x[j][3]));
+        mx = fmaxf(mx, dpp_move<0xB1>(mx));   // lane ^ 1
+        mx = fmaxf(mx, dpp_move<0x4E>(mx));   // lane ^ 2
+        amax[j] = fmaxf(mx, dpp_move<0x141>(mx));  // the other four of the eight (half mirror)
+    }
+    const int mine = lane & 3;
+    float top = amax[0];
+#pragma unroll
+    for (int j = 1; j < PASS; j++) top = mine == j ? amax[j] : top;
+    uint16_t dh;
+    const float id = q8_0_block_rule(top, dh);
+    __builtin_amdgcn_wave_barrier();
+    if ((lane & 4) == 0 && mine < PASS) *(uint16_t*)(area + mine * kSmallCodes + 256 + 2 * (lane >> 3)) = dh;
+#pragma unroll
+    for (int j = 0; j < PASS; j++) {
+        const float inv = j == 0 ? dpp_move<0x00>(id) : j == 1 ? dpp_move<0x55>(id) : j == 2 ? dpp_move<0xAA>(id) : dpp_move<0xFF>(id);  // that of lane j of the four
+        uint32_t c[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            // q8_0_code: rounded with halves away from zero.  Adding the number below 0.5, not 0.5, makes that exact: 0.5 - 2^-25 stays below one, and a half still rounds up.
+            const float t = x[j][i] * inv;
+            c[i] = (uint32_t)(int)(t + __builtin_copysignf(0.49999997f, t));
+        }
+        const uint32_t codes = __builtin_amdgcn_perm(__builtin_amdgcn_perm(c[3], c[2], 0x0C0C0400u), __builtin_amdgcn_perm(c[1], c[0], 0x0C0C0400u), 0x05040100u);
+        *(uint32_t*)(area + j * kSmallCodes + 32 * (lane >> 3) + 8 * (lane & 3) + (lane & 4)) = codes;
+    }
 }
 
 }  // namespace qmm

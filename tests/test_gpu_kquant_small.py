@@ -1,4 +1,4 @@
-"""Q4_K, Q5_K and Q6_K with 2 .. 16 lhs rows: the small-batch kernel at the edges of its tiles (16 weight rows), of its groups of K (up to 16 super-blocks, divided
+"""Q4_0, Q4_K, Q5_K and Q6_K with 1 .. 16 lhs rows: the small-batch kernel at the edges of its tiles (16 weight rows), of its groups of K (up to 16 super-blocks, divided
 evenly) and of its lhs rows (2, 4, 8, 16), against float64 products of the dequantised weights."""
 import pytest
 import torch
@@ -35,6 +35,26 @@ def test_against_float64(enc, lhs, m, n, k):
     w, a = packed(enc, n, k), rows(min(m, 8) if lhs == torch.float32 else m, k, lhs)  # (from nine fp32 rows on other kernels serve the call)
     check(enc, qmatmul(QE[enc], None, a, w), w, a)
     check(enc, qmatmul(QE[enc], None, a, w, out_dtype=torch.bfloat16), w, a, bits=8)
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 8200, 512), (1, 1000, 18944), (2, 18, 256), (2, 4104, 4096), (3, 1000, 768), (4, 17, 14336), (5, 40, 4352), (8, 264, 8192), (7, 4200, 11008), (9, 4112, 1024), (16, 1001, 2048),
+                                   (12, 1000, 14336)])
+def test_q4_0(lhs, m, n, k):
+    """The lhs quantised to Q8_0 by every wavefront for itself: the codes of the package's quantiser, exact sums over blocks."""
+    w, a = packed("Q4_0", n, k), rows(min(m, 8) if lhs == torch.float32 else m, k, lhs)
+    a[0, :32] *= 1e-30
+    a[-1, 32:64] = 0.0
+    a[0, 64:96] = torch.tensor([127.0, *[x + 0.5 for x in range(-15, 16)]], device="cuda").to(lhs)  # halves between codes
+    blocks = quantize(QE.Q8_0, a.float()).view(a.shape[0], -1, 34)
+    x = (blocks[:, :, :2].contiguous().view(torch.float16).double() * blocks[:, :, 2:].contiguous().view(torch.int8).double()).view(a.shape)
+    want = x @ dequantize(QE.Q4_0, w).double().T
+    for got, bits in ((qmatmul(QE.Q4_0, None, a, w), 22), (qmatmul(QE.Q4_0, None, a, w, out_dtype=torch.bfloat16), 8)):
+        assert ((got.double() - want).norm(dim=1) / want.norm(dim=1)).max().item() <= 2.0**-bits
+    ws = [w, packed("Q4_0", n + 16, k, 1)]
+    if m in (4, 8):
+        for got, v in zip(qmatmul_grouped(QE.Q4_0, a, ws), ws):
+            assert torch.equal(got, qmatmul(QE.Q4_0, None, a, v))
 
 
 @pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
