@@ -37,6 +37,18 @@ def test_gguf_edges(enc, n, blocks):
     assert np.array_equal(bits(dequantize(enc, torch.from_numpy(packed).cuda(), dtype=torch.bfloat16)), O.f32_to_bf16(want).view(np.int16))
 
 
+@pytest.mark.parametrize("enc", [QE.Q4_K, QE.Q5_K, QE.Q6_K])
+@pytest.mark.parametrize("scale", [1e-30, 1e-9, 1e-4, 1.0, 1e3, 1e5])
+def test_codes_of_any_magnitude(enc, scale):
+    """Quotients by one reciprocal per sub-block: rounded as divisions are, halves between codes among them, and with scales that are denormal or zero in fp16."""
+    rng = np.random.Generator(np.random.PCG64(11))
+    w = rng.standard_normal((256, 1024), dtype=np.float32)
+    w[::2] = np.round(w[::2] * 6) / np.float32(6) + np.float32(1 / 12)  # few different values, so many quotients of a block that are equal or lie half way
+    w[1::4, ::3] *= np.float32(1e-3)
+    w = (w * np.float32(scale)).astype(np.float32)
+    assert np.array_equal(quantize(enc, torch.from_numpy(w).cuda()).cpu().numpy(), O.quantize(ORACLE[enc], w))
+
+
 @pytest.mark.parametrize("n,k,group", [(8, 32, 32), (72, 96, 96), (64, 512, 128), (56, 640, 160), (200, 1024, 1024), (8, 416, 32)])
 def test_gptq_edges(n, k, group):
     w = weights(n + k, n, k)
