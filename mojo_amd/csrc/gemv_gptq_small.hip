@@ -94,9 +94,11 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
         asm volatile("" : "+v"(lane));  // (what is computed from it here is not kept in registers between the groups)
         const int nn = lane & 15, kg = lane >> 4, my_row = (nn >> 2) + 4 * ((nn & 3) / PL), my_part = (nn & 3) % PL;
         float* const row_scales = (float*)(area + 4 * kSmallPlane);
+        float common = 1.0f;
+        if constexpr (PL == 2) common = small_common_scale<14>(xr);
 #pragma unroll
         for (int r0 = 0; r0 < MROWS; r0 += kPass) {
-            const bool scaled = small_narrow<PL, kPass, kSmallOrderGptq>(xr, r0, area, row_scales, lane);
+            const float inverse = small_narrow<PL, kPass, kSmallOrderGptq, 14>(xr, r0, common, area, row_scales, lane);
             __builtin_amdgcn_wave_barrier();
             if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
                 const uint8_t* const pl = area + ((my_row - r0) * PL + my_part) * kSmallPlane + 16 * kg;
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
             }
 #pragma unroll
             for (int j = 0; j < LR; j++)
-                if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = scaled ? row_scales[kg + 4 * j - r0] : 1.0f;
+                if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = inverse == 0.0f ? row_scales[kg + 4 * j - r0] : inverse;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the operands are in registers before the next item's load may overwrite the slot
     };

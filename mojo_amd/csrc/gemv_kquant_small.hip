@@ -165,9 +165,12 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
             }
         } else {
             float* const scales = (float*)(area + 4 * kSmallPlane);
+            constexpr int kTop = kMin ? 9 : 14;
+            float common = 1.0f;
+            if constexpr (PL == 2) common = small_common_scale<kTop>(xr);
 #pragma unroll
             for (int r0 = 0; r0 < MROWS; r0 += kPass) {
-                const bool scaled = small_narrow<PL, kPass, ENC == QMM_Q4_K ? kSmallOrderK : kSmallOrderPlain>(xr, r0, area, scales, lane);
+                const float inverse = small_narrow<PL, kPass, ENC == QMM_Q4_K ? kSmallOrderK : kSmallOrderPlain, kTop>(xr, r0, common, area, scales, lane);
                 __builtin_amdgcn_wave_barrier();
                 if ((nn & 3) < RN && my_row >= r0 && my_row < r0 + kPass) {
                     const uint8_t* const pl = area + ((my_row - r0) * PL + my_part) * kSmallPlane;
@@ -184,7 +187,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
                 }
 #pragma unroll
                 for (int j = 0; j < LR; j++)
-                    if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = scaled ? scales[kg + 4 * j - r0] : 1.0f;
+                    if (kg + 4 * j >= r0 && kg + 4 * j < r0 + kPass) bs[j] = inverse == 0.0f ? scales[kg + 4 * j - r0] : inverse;
             }
         }
         if constexpr (kMin) {

@@ -38,12 +38,46 @@ __device__ __forceinline__ uint32_t to_half2_bits(float a, float b) { return __b
 // The order in which four (GPTQ: eight) neighbouring columns lie in a plane: 0,1,2,3; 0,2,1,3; 0,4,1,5,2,6,3,7.
 enum { kSmallOrderPlain = 0, kSmallOrderK = 1, kSmallOrderGptq = 2 };
 
+// The lhs is scaled so that what fp16 leaves out of any value is small against its row's largest: by 2^-33 and below where weights have minima (TOP = 9: a sum of 32 values is an fp16 number too), else 2^-39 (TOP = 14), as
+// in the kernels for more rows.
+// fp32 rows (hi part and residual): one power of two for all rows, which brings the largest value to [2^TOP, 2^(TOP + 1)), where every row's largest is at least an eighth of it; the result is that scale, or 0: one for each
+// row.  One search over the wavefront for all of them; one for each row always, and the products, took 8 rows 4096 x 4096 from 8.0 to 8.5 (Q4_K) and 7.8 to 9.3 us (GPTQ).
+template <int TOP, typename RAW, int ROWS>
+__device__ __forceinline__ float small_common_scale(const RAW (&xr)[ROWS]) {
+    float mx[ROWS], top = 0.0f;
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        mx[j] = fmaxf(fmaxf(fmaxf(fabsf(__uint_as_float(xr[j].x)), fabsf(__uint_as_float(xr[j].y))), fabsf(__uint_as_float(xr[j].z))), fabsf(__uint_as_float(xr[j].w)));
+        top = fmaxf(top, mx[j]);
+    }
+    const int e = (int)(wave_max_nonneg_bits(top) >> 23) - 127;
+    if (e < TOP - 126 || e > 126) return 0.0f;
+    const float floor = __uint_as_float((uint32_t)max(127 + e - 3, 0) << 23);
+    bool common = true;
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) common = common & (__builtin_amdgcn_ballot_w64(mx[j] >= floor) != 0);
+    return common ? __uint_as_float((uint32_t)(127 + TOP - e) << 23) : 0.0f;
+}
+
 // Rows r0 .. r0 + PASS - 1 to fp16 planes of kSmallPlane bytes in `area` (fp32 rows, PL = 2: hi part, then residual).  xr[j]: columns 4 lane .. 4 lane + 3 of row j.
-// Where the values are not of ordinary size, each row is scaled by a power of two first, whose inverses go to `scales`, and the result is true.
-template <int PL, int PASS, int ORDER, typename RAW, int ROWS>
-__device__ __forceinline__ bool small_narrow(const RAW (&xr)[ROWS], int r0, uint8_t* area, float* scales, int lane) {
-    float x[PASS][4], mx[PASS], top = 0.0f;
-    bool floor_ok = true;
+// common: what small_common_scale says (fp32 rows).  bf16 rows stay as they are where every value is then an fp16 number (none but zeros below 2^-17, whose last bit is 2^-24) and none is too large.  Otherwise a power of two
+// per row brings its largest value to [2^TOP, 2^(TOP + 1)), and the inverses go to `scales`.  The result is the inverse of the scale of all rows, or 0.
+template <int PL, int PASS, int ORDER, int TOP, typename RAW, int ROWS>
+__device__ __forceinline__ float small_narrow(const RAW (&xr)[ROWS], int r0, float common, uint8_t* area, float* scales, int lane) {
+    float x[PASS][4], sc[PASS];
+    bool each = common == 0.0f;
+    if constexpr (PL == 1) {
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        u16x2 most = {0, 0}, least = {0xffff, 0xffff};
+#pragma unroll
+        for (int j = 0; j < PASS; j++) {
+            const u16x2 v0 = __builtin_bit_cast(u16x2, (uint32_t)xr[r0 + j].x & 0x7fff7fffu), v1 = __builtin_bit_cast(u16x2, (uint32_t)xr[r0 + j].y & 0x7fff7fffu), one = {1, 1};
+            most = __builtin_elementwise_max(most, __builtin_elementwise_max(v0, v1));
+            least = __builtin_elementwise_min(least, __builtin_elementwise_min((u16x2)(v0 - one), (u16x2)(v1 - one)));  // (zeros: the largest number)
+        }
+        const uint16_t m0 = most.x, m1 = most.y, l0 = least.x, l1 = least.y;
+        each = __builtin_amdgcn_ballot_w64(max(m0, m1) >= (127 + TOP + 1) << 7 || min(l0, l1) < ((127 - 17) << 7) - 1) != 0;
+    }
 #pragma unroll
     for (int j = 0; j < PASS; j++) {
         const RAW raw = xr[r0 + j];
@@ -53,29 +87,25 @@ __device__ __forceinline__ bool small_narrow(const RAW (&xr)[ROWS], int r0, uint
             x[j][0] = __uint_as_float(raw.x << 16), x[j][1] = __uint_as_float(raw.x & 0xffff0000u);
             x[j][2] = __uint_as_float(raw.y << 16), x[j][3] = __uint_as_float(raw.y & 0xffff0000u);
         }
-        mx[j] = fmaxf(fmaxf(fmaxf(fabsf(x[j][0]), fabsf(x[j][1])), fabsf(x[j][2])), fabsf(x[j][3]));
-        top = fmaxf(top, mx[j]);
-        floor_ok = floor_ok & (__builtin_amdgcn_ballot_w64(mx[j] >= 0.125f) != 0);
+        sc[j] = common;
     }
-    // Every row's largest value between 2^-3 and 2^10 (activations of ordinary size): the values go to fp16 as they are, what is below fp16's
-    // normal range (2^-14) is small against the largest, and a sum of 32 is an fp16 number.  Otherwise a power of two per row brings its largest value to [2^9, 2^10) first.
-    const bool scaled = !floor_ok || __builtin_amdgcn_ballot_w64(top >= 1024.0f) != 0;
     __builtin_amdgcn_wave_barrier();
-    if (scaled) {
+    if (each) {
 #pragma unroll
         for (int j = 0; j < PASS; j++) {
-            if constexpr (ORDER == kSmallOrderGptq) {  // (of the finite values: an infinity stays one, and the others are held as in any row)
-                mx[j] = 0.0f;
+            float mx = 0.0f;
 #pragma unroll
-                for (int i = 0; i < 4; i++) mx[j] = fmaxf(mx[j], fabsf(x[j][i]) <= 3.402823466e38f ? fabsf(x[j][i]) : 0.0f);
+            for (int i = 0; i < 4; i++)  // (GPTQ: of the finite values: an infinity stays one, and the others are held as in any row)
+                mx = fmaxf(mx, ORDER != kSmallOrderGptq || fabsf(x[j][i]) <= 3.402823466e38f ? fabsf(x[j][i]) : 0.0f);
+            // (the least scale is that whose inverse is 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly; a row with an infinity stays unscaled)
+            int e = max((int)(wave_max_nonneg_bits(mx) >> 23) - 127, TOP - 126);
+            if (e > 127) e = TOP;
+            sc[j] = __uint_as_float((uint32_t)(127 + TOP - e) << 23);
+            if (lane == 0) scales[j] = __uint_as_float((uint32_t)(127 - TOP + e) << 23);
+            if constexpr (PL == 1) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[j][i] *= sc[j];
             }
-            // (2^-117: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly; a row with an infinity stays unscaled)
-            int e = max((int)(wave_max_nonneg_bits(mx[j]) >> 23) - 127, -117);
-            if (e > 127) e = 9;
-            const float sc = __uint_as_float((uint32_t)(127 + 9 - e) << 23);
-            if (lane == 0) scales[j] = __uint_as_float((uint32_t)(127 - 9 + e) << 23);
-#pragma unroll
-            for (int i = 0; i < 4; i++) x[j][i] *= sc;
         }
     }
     // GPTQ: the lane of an even four gives its columns 2, 3 for the next lane's 0, 1 (columns 4, 5 of the eight): (0,4), (1,5) here, (2,6), (3,7) there
@@ -92,20 +122,27 @@ __device__ __forceinline__ bool small_narrow(const RAW (&xr)[ROWS], int r0, uint
     for (int j = 0; j < PASS; j++) {
         constexpr int i1 = ORDER == kSmallOrderK ? 2 : 1, i2 = ORDER == kSmallOrderK ? 1 : 2;
         const float xs[4] = {x[j][0], x[j][i1], x[j][i2], x[j][3]};
-        const half2v ha = to_half2(xs[0], xs[1]), hb = to_half2(xs[2], xs[3]);
         uint8_t* const at = area + (j * PL) * kSmallPlane + 8 * lane;
-        put(at, __builtin_bit_cast(uint32_t, ha), __builtin_bit_cast(uint32_t, hb));
-        if constexpr (PL == 2) {  // residual x - hi: exact in fp32
-            // (GPTQ, whose weights have no minima: an infinity has no residual, so that it gives infinities and not NaN)
-            auto residual = [&](_Float16 h, float v) __attribute__((always_inline)) {
-                return ORDER != kSmallOrderGptq || fabsf((float)h) <= 65504.0f ? fmaf((float)h, -1.0f, v) : 0.0f;
-            };
-            const half2v ra = to_half2(residual(ha.x, xs[0]), residual(ha.y, xs[1]));
-            const half2v rb = to_half2(residual(hb.x, xs[2]), residual(hb.y, xs[3]));
-            put(at + kSmallPlane, __builtin_bit_cast(uint32_t, ra), __builtin_bit_cast(uint32_t, rb));
+        if constexpr (PL == 1) {
+            put(at, to_half2_bits(xs[0], xs[1]), to_half2_bits(xs[2], xs[3]));
+        } else {
+            // (products with a power of two: the rounding to fp16 is the only one, in one instruction with the product)
+            _Float16 h[4], r[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) h[i] = (_Float16)__builtin_fmaf(xs[i], sc[j], 0.0f);
+            // residual x - hi: exact in fp32
+#pragma unroll
+            for (int i = 0; i < 4; i++) r[i] = (_Float16)__builtin_fmaf(xs[i], sc[j], -(float)h[i]);
+            if (ORDER == kSmallOrderGptq && each) {  // (weights without minima: an infinity has no residual, so that it gives infinities and not NaN; rows with one have no common scale)
+#pragma unroll
+                for (int i = 0; i < 4; i++) r[i] = fabsf((float)h[i]) <= 65504.0f ? r[i] : (_Float16)0.0f;
+            }
+            put(at, __builtin_bit_cast(uint32_t, half2v{h[0], h[1]}), __builtin_bit_cast(uint32_t, half2v{h[2], h[3]}));
+            put(at + kSmallPlane, __builtin_bit_cast(uint32_t, half2v{r[0], r[1]}), __builtin_bit_cast(uint32_t, half2v{r[2], r[3]}));
         }
     }
-    return scaled;
+    // (the inverse of a power of two: its exponent, negated)
+    return each ? 0.0f : PL == 1 ? 1.0f : __uint_as_float((254u << 23) - __float_as_uint(common));
 }
 
 constexpr int kSmallCodes = 272;  // an lhs row of 256 columns as Q8_0: codes, block by block in the order of small_quantize, then the eight block scales

@@ -68,6 +68,18 @@ def test_infinities_and_nans_keep_their_kind(lhs):
         assert torch.equal(got[row].nan_to_num(nan=0.0, posinf=1.0, neginf=-1.0), sign * w[:, column].sign())
 
 
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+def test_small_values_next_to_a_few_large_ones(lhs):
+    """Spikes of 0.2 among values of 2^-13: what a row is scaled by decides how much of those fp16 holds."""
+    config, rhs = tensors(264, 4096, 128)
+    a = rows(4, 4096, torch.float32) * 2.0**-13
+    a[:, 5::1024] = 0.2
+    # (roundings of a few large terms do not average out: 2^-21; with the small values held to 2^-25, however large the spikes are, 1.4e-6 and, bf16 with 2^-17, 1.3e-6)
+    check(config, rhs, qmatmul(QE.GPTQ, config, a.to(lhs), *rhs), a.to(lhs), bits=21)
+    a[:, torch.arange(4096, device="cuda") % 1024 != 5] *= 2.0**-4
+    check(config, rhs, qmatmul(QE.GPTQ, config, a.to(lhs), *rhs), a.to(lhs), bits=21)
+
+
 @pytest.mark.parametrize("m", [1, 4, 8])
 def test_a_small_workspace_gives_the_same_sums(m):
     """Groups of K side by side, added by a launch of their own, or, with less than they need, one after the other in each workgroup."""

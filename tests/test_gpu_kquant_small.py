@@ -88,6 +88,18 @@ def test_rows_of_other_magnitudes(enc, lhs, scale):
 
 
 @pytest.mark.parametrize("enc", ENCODINGS)
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+def test_small_values_next_to_a_few_large_ones(enc, lhs):
+    """Spikes of 0.2 among values of 2^-13: what a row is scaled by decides how much of those fp16 holds."""
+    w, a = packed(enc, 264, 4096), rows(8, 4096, torch.float32) * 2.0**-13
+    a[:, 5::1024] = 0.2
+    # (roundings of a few large terms do not average out: 2^-21; with the small values held to 2^-25, however large the spikes are, 1.4e-6 and, bf16 with 2^-17, 1.3e-6)
+    check(enc, qmatmul(QE[enc], None, a.to(lhs), w), w, a.to(lhs), bits=21)
+    a[:, torch.arange(4096, device="cuda") % 1024 != 5] *= 2.0**-4
+    check(enc, qmatmul(QE[enc], None, a.to(lhs), w), w, a.to(lhs), bits=21)
+
+
+@pytest.mark.parametrize("enc", ENCODINGS)
 @pytest.mark.parametrize("m,k", [(4, 4096), (8, 11008), (3, 8448)])
 def test_group_gated_pair_and_parts_of_k_give_the_same_sums(enc, m, k):
     ns = (1032, 520, 40)
