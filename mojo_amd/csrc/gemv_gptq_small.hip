@@ -1,4 +1,4 @@
-// GPTQ with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32) on the matrix cores, K any multiple of 256, groups of 32, 64, 128 or 256: one launch, no workspace needed.
+// GPTQ with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32 a workgroup, up to four times as many side by side) on the matrix cores, K any multiple of 256, groups of 32, 64, 128 or 256: one launch, no workspace needed.
 //
 // Shape of the work: that of gemv_kquant_small.hip.  A workgroup has as many wavefronts, up to 16, as divide the 256-column parts of K evenly into groups; a wavefront keeps the lhs operands
 // of its part in 32 registers and walks the workgroup's tiles of CW output columns with them.  An item, 32 rows of CW words and the scales and zeros over them (2.2 or 4.3 KB), goes
@@ -47,13 +47,19 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
     static_assert(RN <= 4, "operand rows");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nn = lane & 15, kg = lane >> 4;
-    const int waves = (int)(packed & 0xffu), chunk = (int)(packed >> 8) & 0xff, groups = (int)(packed >> 18);
+    const int waves = (int)(packed & 0xffu), chunk = (int)(packed >> 8) & 0xff, groups = (int)(packed >> 18) & 0x1fff;
     const bool apart = (packed >> 16) & 1, bf16 = (packed >> 17) & 1;
     // Neighbouring tiles run on one XCD (ids congruent mod 8), whose L2 then fetches the lines that they share once.
-    const int per_xcd = (stride + 7) >> 3, share = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+    int share, of_k = (int)blockIdx.y, row0 = 0;  // this workgroup's tiles, group of K, first lhs row
+    if (MROWS == small_rows<AT>() && (packed >> 31)) {
+        // several tiles of lhs rows: those that read the same weights side by side (blockIdx.y) on one XCD, every XCD the same number of them
+        row0 = (int)blockIdx.y * MROWS, share = (int)blockIdx.x * ((stride * (apart ? groups : 1) + 7) >> 3) + (int)blockIdx.z, of_k = apart ? share / stride : 0;
+        share -= of_k * stride;
+        if (apart && of_k >= groups) return;
+    } else share = ((int)blockIdx.x & 7) * ((stride + 7) >> 3) + ((int)blockIdx.x >> 3);
     if (share >= stride) return;  // (the whole workgroup)
     const int parts = k >> 8;
-    const int g_first = apart ? (int)blockIdx.y : 0, g_end = apart ? g_first + 1 : groups;
+    const int g_first = apart ? of_k : 0, g_end = apart ? g_first + 1 : groups;
     uint8_t* const ring = smem + wave * (2 * I::kSlot);
     const uint32_t ring_lds = lds_address(ring);
     float* const accs = (float*)(smem + waves * (2 * I::kSlot));  // [chunk][waves][H LR][64]
@@ -118,7 +124,7 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
         xraw_t xr[MROWS];
         const int part = min(g_first * waves + wave, parts - 1);
 #pragma unroll
-        for (int j = 0; j < MROWS; j++) hidden_load(xr[j], a_lane, a + (int64_t)min(j, m - 1) * k + part * 256);
+        for (int j = 0; j < MROWS; j++) hidden_load(xr[j], a_lane, a + (int64_t)min(row0 + j, m - 1) * k + part * 256);
         issue(part, 0, 0);
         wait_vmcnt<I::kLoads>();
 #pragma unroll
@@ -135,7 +141,7 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
                 if (groups > 1 && c0 + g > g_first) {
                     xraw_t xr[MROWS];
 #pragma unroll
-                    for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(j, m - 1) * k + part * 256) + a_lane);
+                    for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(row0 + j, m - 1) * k + part * 256) + a_lane);
                     narrow(xr, ring + (slot ^ 1) * I::kSlot);
                 }
                 for (int t = 0; t < ct; t++) {
@@ -209,7 +215,7 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
             // the group's result (lhs row kg + 4 j, column n0 + H nn + h): dealt to the wavefronts, which add it to that of the groups before
             const int live = min(waves, parts - g * waves);
             for (int q = wave; q < ct * (H * LR); q += waves) {
-                const int t = q / (H * LR), hj = q % (H * LR), h = hj / LR, row = kg + 4 * (hj % LR);
+                const int t = q / (H * LR), hj = q % (H * LR), h = hj / LR, row = row0 + kg + 4 * (hj % LR);
                 const float* const src = accs + ((t * waves) * (H * LR) + hj) * 64 + lane;
                 float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                 int w = 0;
@@ -228,7 +234,7 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
                 if (g + 1 < g_end || row >= m) continue;
                 const int64_t at = (int64_t)row * n + first_column(c0 + t) + H * nn + h;
                 if (bf16) ((uint16_t*)out)[at] = f2bf(r);
-                else out[at + (int64_t)blockIdx.y * m * n] = r;
+                else out[at + (int64_t)of_k * m * n] = r;
             }
             if (g + 1 < g_end || c0 + chunk < my_items) __syncthreads();
         }
@@ -239,7 +245,7 @@ namespace {
 
 struct GptqSmallPlan {
     GptqSmallCut cut;
-    int cw, grid, parts, per_cu;
+    int cw, grid, parts, per_cu, row_tiles;
     size_t lds;
 };
 // Groups of K: of its length only, so that results do not depend on what else a call has.
@@ -252,7 +258,9 @@ int gptq_small_slot(int cw, int group) {
     return cw * 128 + (dwords + 63) / 64 * 256;
 }
 // apart: workgroups that share a tile, one group of K each
-bool gptq_small_cut(int64_t m, int64_t n, int64_t k, int group, bool apart, int cw, GptqSmallPlan& p) {
+bool gptq_small_cut(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool apart, int cw, GptqSmallPlan& p) {
+    p.row_tiles = (int)((m + small_most_rows(lhs_dtype) - 1) / small_most_rows(lhs_dtype));
+    m = std::min(m, small_most_rows(lhs_dtype));
     const int parts = (int)(k / 256), groups = gptq_small_groups(k), lr = m <= 4 ? 1 : m <= 8 ? 2 : 4;
     if (n < cw) return false;
     GptqSmallCut& c = p.cut;
@@ -263,7 +271,7 @@ bool gptq_small_cut(int64_t m, int64_t n, int64_t k, int group, bool apart, int 
     p.parts = apart ? groups : 1;
     const int64_t tiles = (n + cw - 1) / cw;
     p.per_cu = std::max(1, kGsWaves / c.waves);
-    const int64_t most = std::max<int64_t>(1, (int64_t)compute_units() * p.per_cu / p.parts);
+    const int64_t most = std::max<int64_t>(1, small_places(p.per_cu, p.row_tiles) / p.parts);
     c.per = (int)((tiles + most - 1) / most);
     c.stride = (int)((tiles + c.per - 1) / c.per);
     p.grid = (c.stride + 7) / 8 * 8;
@@ -287,14 +295,14 @@ constexpr GptqSmallCost kGptqSmallCost[2][4] = {
     {{0.96f, {1.25f, 1.67f}}, {2.03f, {1.0f, 1.31f}}, {3.3f, {0.5f, 0.8f}}, {}},                        // fp32
 };
 bool gptq_small_plan(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, bool may_part, GptqSmallPlan& best) {
-    const GptqSmallCost& cost = kGptqSmallCost[lhs_dtype == QMM_F32 ? 1 : 0][m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 ? 2 : 3];
+    const GptqSmallCost& cost = kGptqSmallCost[lhs_dtype == QMM_F32 ? 1 : 0][m <= 2 ? 0 : m <= 4 ? 1 : m <= 8 || lhs_dtype == QMM_F32 ? 2 : 3];
     const int groups = gptq_small_groups(k);
     double us = 1e30;
     for (int apart = 0; apart <= (may_part && groups > 1 && n * k < (int64_t)1 << 27 ? 1 : 0); apart++)
-        for (int cw = 16; cw <= (m <= 8 ? 32 : 16); cw += 16) {
+        for (int cw = 16; cw <= (m <= 8 || lhs_dtype == QMM_F32 ? 32 : 16); cw += 16) {
             GptqSmallPlan p;
-            if (!gptq_small_cut(m, n, k, group, apart != 0, cw, p)) continue;
-            const int walk = apart ? 1 : groups, chunks = (p.cut.per + p.cut.chunk - 1) / p.cut.chunk, workgroups = (int)(((int64_t)p.cut.stride * p.parts + compute_units() - 1) / compute_units());
+            if (!gptq_small_cut(lhs_dtype, m, n, k, group, apart != 0, cw, p)) continue;
+            const int walk = apart ? 1 : groups, chunks = (p.cut.per + p.cut.chunk - 1) / p.cut.chunk, workgroups = (int)(((int64_t)p.cut.stride * p.parts * p.row_tiles + compute_units() - 1) / compute_units());
             const double t = cost.convert * ((walk > 1 ? walk * chunks : 1) + 0.3 * (workgroups - 1)) + cost.item[cw / 16 - 1] * p.cut.per * walk * p.cut.waves * p.per_cu / kGsWaves +
                              0.15 * (chunks * walk - 1) + 2.8 * apart;
             if (t < us) us = t, best = p;
@@ -306,7 +314,8 @@ template <int CW, int GS, int MROWS, typename AT>
 hipError_t run_gptq_small(const GptqSmallPlan& p, const uint32_t* qweight, const uint16_t* scales, const uint32_t* qzeros, const AT* a, float* out, int n, int m, int k, hipStream_t s) {
     hipError_t e = allow_full_lds<gemv_gptq_small_kernel<CW, GS, MROWS, AT>>();
     if (e != hipSuccess) return e;
-    gemv_gptq_small_kernel<CW, GS, MROWS, AT><<<dim3((unsigned)p.grid, (unsigned)p.parts), dim3((unsigned)(64 * p.cut.waves)), p.lds, s>>>(qweight, scales, qzeros, a, n, m, k, p.cut.stride, p.cut.per, p.cut.packed(), out);
+    const dim3 grid = p.row_tiles > 1 ? dim3(8, (unsigned)p.row_tiles, (unsigned)((p.cut.stride * p.parts + 7) / 8)) : dim3((unsigned)p.grid, (unsigned)p.parts);
+    gemv_gptq_small_kernel<CW, GS, MROWS, AT><<<grid, dim3((unsigned)(64 * p.cut.waves)), p.lds, s>>>(qweight, scales, qzeros, a, n, m, k, p.cut.stride, p.cut.per, p.cut.packed() | (uint32_t)(p.row_tiles > 1) << 31, out);
     return hipGetLastError();
 }
 
@@ -333,12 +342,12 @@ hipError_t run_gptq_small_rows(const GptqSmallPlan& p, const uint32_t* qweight, 
 bool gemv_gptq_small_supported(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
     // (with the name of the older small-batch kernel this one goes too)
     if (kernel_disabled("gptq_small") || kernel_disabled("gptq_mm") || (group != 32 && group != 64 && group != 128 && group != 256)) return false;
-    if (m < 1 || m > (lhs_dtype == QMM_F32 ? 8 : 16) || n < 16 || n % 8 || n > 1 << 23 || k < 256 || k % 256 || k > 1 << 20) return false;
+    if (m < 1 || m > 4 * small_most_rows(lhs_dtype) || n < 16 || n % 8 || n > 1 << 23 || k < 256 || k % 256 || k > 1 << 20) return false;
     // Nine rows and more, us, older small-batch kernel / this one: two workgroups on a compute unit convert the lhs twice, 5632 x 2048 7.3 / 8.6, 8192 x 1024 5.6 / 6.1; large matrices with several groups of
     // K, few results in LDS at a time, 28672 x 8192 38 / 45; but 2048 x 2048 6.7 / 6.0, 8192 x 8192 17.7 / 16.1.
     // One row, groups of 32, whose scales and zeros leave the larger ring no room: 28672 x 8192 33 .. 36 / 38, but 14336 x 4096 15.2 / 11.5.
     if (m == 1 && group == 32 && k > 4096 && n * k >= (int64_t)1 << 27) return false;
-    return m <= 8 || ((k > 2048 || n <= 16 * compute_units()) && (k <= 4096 || n * k < (int64_t)1 << 27));
+    return m <= 8 || lhs_dtype == QMM_F32 || ((k > 2048 || n <= 16 * compute_units()) && (k <= 4096 || n * k < (int64_t)1 << 27));
 }
 
 // What groups of K side by side take (without it a workgroup walks all of K: the same sums).

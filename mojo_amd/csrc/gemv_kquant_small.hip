@@ -1,4 +1,5 @@
-// Q4_0, Q4_K, Q5_K and Q6_K with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32) on the matrix cores, K any multiple of 256: one launch, no workspace.
+// Q4_0, Q4_K, Q5_K and Q6_K with a few lhs rows (1 .. 16 bf16, 1 .. 8 fp32 a workgroup, up to four times as many side by side) on the matrix cores, K any multiple of 256: one launch, no workspace (groups of K side
+// by side: a second launch and their sums in the workspace).
 //
 // Shape of the work.  A workgroup has as many wavefronts, up to 16, as divide the super-blocks of a row evenly into groups: wavefront w owns super-block
 // w + waves g of group g (K = 4096: one group of 16; 14336: four of 14).  It converts the lhs columns of its super-block into matrix-core operands once a
@@ -17,8 +18,10 @@
 // 4.0e-7 / 1.1e-7, Q5_K 1.7e-7 / 1.2e-7, Q6_K 1.6e-7 / 1.0e-7; bf16 rows 2.5e-7 / 0.8e-7, 1.0e-7 / 0.85e-7, 0.97e-7 / 0.84e-7 (codes around their middle, residuals to nearest, super-blocks added in
 // four chains).
 //
-// Arithmetic.  lhs: a power of two per (row, super-block) where its values are not of ordinary size, then fp16 (bf16 rows: exact down to 2^-26 of the largest; fp32 rows: hi part and residual, 22
-// bits).  Weights: integers sc * (q - mid) (Q4_K, Q5_K) or q (Q6_K) as fp16, so every product is exact and the sums are fp32.
+// More rows than one workgroup takes: each streams all weights, the second one from its XCD's L2, which still beats preparing the lhs with a launch of its own where that launch and the next one's way to its first product
+// are most of the time: 4096 x 4096 Q4_K 16 fp32 rows 11.7 / 9.2 us, 1024 x 14336 23.9 / 11.4 (rule and lines: qmm_api.hip).
+//
+// Arithmetic.  lhs: scaled by powers of two, then fp16 (see small_narrow; bf16 rows: one term; fp32 rows: hi part and residual, 22 bits).  Weights: integers sc * (q - mid) (Q4_K, Q5_K) or q (Q6_K) as fp16, so every product is exact and the sums are fp32.
 //   Q4_K: a masked nibble is the subnormal q * 2^-24 (or 16 q * 2^-24), one packed multiply-add leaves sc * (q - 8) * 2^-18.
 //   Q5_K: a byte permute puts nibble and fifth bit under 0x54: 64 + q; one packed multiply-add, (64 + q) * sc - 80 * sc, leaves sc * (q - 16) (exact: below 2^11).
 //   Q6_K: the same with 96 taken off; sc * q may need 13 bits, so the scale multiplies the results of its 16 weights instead.
@@ -51,11 +54,11 @@ enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
 
 }  // namespace
 
-// MROWS: lhs rows, 1, 2, 4, 8 or 16 (>= m; rows past m repeat the last one and their results are dropped).
+// MROWS: lhs rows of a workgroup, 1, 2, 4, 8 or 16 (rows past m repeat the last one and their results are dropped); more go side by side, in workgroups of their own.
 // MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up).
 struct SmallCut {
     int per, stride;  // tiles (gated: pairs) of a workgroup at most, workgroups across the tiles
-    uint32_t packed;  // wavefronts; << 8: items (tile, matrix) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups
+    uint32_t packed;  // wavefronts; << 8: items (tile, matrix) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups; << 31: several tiles of lhs rows
 };
 template <int ENC, int MROWS, typename AT, int MODE>
 __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restrict__ a, int m, int k, const SmallCut& cut) {
@@ -73,19 +76,26 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = (int)(cut.packed & 0xffu), chunk = (int)(cut.packed >> 8) & 0xff, per = cut.per, stride = cut.stride;
     const bool out_bf16 = (cut.packed >> 16) & 1, apart = (cut.packed >> 17) & 1;
     const int nn = lane & 15, kg = lane >> 4;
-    const int nblk = k >> 8, groups = (int)(cut.packed >> 18);
-    const int g_first = apart ? (int)blockIdx.y : 0, g_end = apart ? g_first + 1 : groups;  // (one group per workgroup, or all of them)
+    const int nblk = k >> 8, groups = (int)(cut.packed >> 18) & 0x1fff;
+    int share = (int)blockIdx.x, part = (int)blockIdx.y, row0 = 0;  // this workgroup's tiles, group of K, first lhs row
+    if (MROWS == small_rows<AT>() && (cut.packed >> 31)) {
+        // several tiles of lhs rows: those that read the same weights side by side (blockIdx.y) on one XCD (ids congruent mod 8), every XCD the same number of them
+        row0 = (int)blockIdx.y * MROWS, share = (int)blockIdx.z * 8 + (int)blockIdx.x, part = apart ? share / stride : 0;
+        share -= part * stride;
+        if (share >= stride || (apart && part >= groups)) return;  // (the whole workgroup)
+    }
+    const int g_first = apart ? part : 0, g_end = apart ? g_first + 1 : groups;  // (one group per workgroup, or all of them)
     const uint32_t row_bytes = (uint32_t)(nblk * I::kBpb);
     uint8_t* const ring = smem + wave * (2 * I::kSlot);
     const uint32_t ring_lds = lds_address(ring);
     float* const accs = (float*)(smem + waves * (2 * I::kSlot));  // [chunk][waves][LR][64]
     float* const totals = accs + chunk * waves * LR * 64;  // [chunk][LR][64], with more than one group
     const int ntiles = MODE == kSmallMats ? mats.tile_end[kLanesMaxMats - 1] : (mats.n[0] + 15) >> 4;
-    const int my_items = (MODE == kSmallGated ? 2 : 1) * ((int)blockIdx.x + (per - 1) * stride < ntiles ? per : per - 1);  // (the grid has no workgroup without a tile)
+    const int my_items = (MODE == kSmallGated ? 2 : 1) * (share + (per - 1) * stride < ntiles ? per : per - 1);  // (the grid has no workgroup without a tile)
 
     // item i of the workgroup: its matrix, and the first row there
     auto matrix_of = [&](int i, int& n0, int& n) __attribute__((always_inline)) {
-        const int tile = (int)blockIdx.x + (MODE == kSmallGated ? i >> 1 : i) * stride;
+        const int tile = share + (MODE == kSmallGated ? i >> 1 : i) * stride;
         int j = 0;
         if constexpr (MODE == kSmallMats) {  // (entries past the last repeat it)
 #pragma unroll
@@ -225,7 +235,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
         xraw_t xr[MROWS];
         const int sb = min(g_first * waves + wave, nblk - 1);
 #pragma unroll
-        for (int j = 0; j < MROWS; j++) hidden_load(xr[j], a_lane, a + (int64_t)min(j, m - 1) * k + sb * 256);
+        for (int j = 0; j < MROWS; j++) hidden_load(xr[j], a_lane, a + (int64_t)min(row0 + j, m - 1) * k + sb * 256);
         issue(sb, 0, 0);
         wait_vmcnt<I::kLoads>();
 #pragma unroll
@@ -245,7 +255,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
             if (groups > 1 && c0 + g > g_first) {
                 xraw_t xr[MROWS];
 #pragma unroll
-                for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(j, m - 1) * k + sb * 256) + a_lane);
+                for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(row0 + j, m - 1) * k + sb * 256) + a_lane);
                 narrow(xr, ring + (slot ^ 1) * I::kSlot);
             }
             for (int t = 0; t < ct; t++) {
@@ -399,7 +409,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
             const int live = min(waves, nblk - g * waves);
             constexpr int kEach = MODE == kSmallGated ? 2 : 1;
             for (int q = wave; q < ct / kEach * LR; q += waves) {
-                const int t = q / LR * kEach, j = q % LR, row = kg + 4 * j;
+                const int t = q / LR * kEach, j = q % LR, row = row0 + kg + 4 * j;
                 float s[kEach];
 #pragma unroll
                 for (int h = 0; h < kEach; h++) {
@@ -427,7 +437,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
                 const int64_t at = (int64_t)row * n + n0 + nn;
                 if (row < m && n0 + nn < n) {
                     if (out_bf16) ((uint16_t*)mats.out[mat])[at] = f2bf(r);
-                    else mats.out[mat][at + (int64_t)blockIdx.y * m * n] = r;
+                    else mats.out[mat][at + (int64_t)part * m * n] = r;
                 }
             }
             if (g + 1 < g_end || c0 + chunk < my_items) __syncthreads();
@@ -454,7 +464,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemv_kquant_small_kernel(con
 namespace {
 
 struct SmallPlan {
-    int waves, groups, grid, parts, per, chunk;
+    int waves, groups, grid, parts, per, chunk, row_tiles;
     size_t lds;
 };
 // Groups of K: of its length only, so that results do not depend on what else a call has.
@@ -463,15 +473,17 @@ int small_groups(int64_t k) {
     return groups == 3 ? 4 : groups;
 }
 // tiles: of 16 weight rows, gated: pairs of them; parts: workgroups that share a tile, one group of K each
-SmallPlan small_plan(int encoding, int64_t m, int64_t tiles, int64_t k, bool gated, bool parts) {
+SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int64_t k, bool gated, bool parts) {
     SmallPlan p;
+    p.row_tiles = (int)((m + small_most_rows(lhs_dtype) - 1) / small_most_rows(lhs_dtype));
+    m = std::min(m, small_most_rows(lhs_dtype));
     const int nblk = (int)(k / 256), groups = small_groups(k);
     p.groups = groups;
     p.waves = (nblk + groups - 1) / groups;
     p.parts = parts ? groups : 1;
     // one workgroup per compute unit (as many as 16 wavefronts allow with few each), all with the same number of tiles or one fewer
     const int per_cu = std::max(1, kSmallWaves / p.waves);
-    const int64_t most = std::max<int64_t>(1, (int64_t)compute_units() * per_cu / p.parts);
+    const int64_t most = std::max<int64_t>(1, small_places(per_cu, p.row_tiles) / p.parts);
     p.per = (int)((tiles + most - 1) / most);
     p.grid = (int)((tiles + p.per - 1) / p.per);
     const int slot = encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? SmallItem<QMM_Q4_K>::kSlot : encoding == QMM_Q5_K ? SmallItem<QMM_Q5_K>::kSlot : SmallItem<QMM_Q6_K>::kSlot;
@@ -492,15 +504,15 @@ bool small_parts(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const double convert = encoding == QMM_Q4_0 ? (m <= 2 ? 1.2 : m <= 4 ? 1.6 : m <= 8 ? 2.6 : 5.0)
                            : lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
     const int64_t tiles = (n + 15) / 16;
-    const SmallPlan w = small_plan(encoding, m, tiles, k, false, false), a = small_plan(encoding, m, tiles, k, false, true);
+    const SmallPlan w = small_plan(encoding, lhs_dtype, m, tiles, k, false, false), a = small_plan(encoding, lhs_dtype, m, tiles, k, false, true);
     const double walk = groups * ((w.per + w.chunk - 1) / w.chunk) * convert + groups * w.per * item;
     return convert + a.per * item + (a.per - 1) / a.chunk * 1.0 + 2.3 + 1.6e-6 * (4.0 * m * n * groups) < walk;
 }
 
 template <int ENC, int MROWS, typename AT>
 hipError_t run_small(const MmMats& mats, const SmallPlan& p, const AT* a, int m, int k, bool gated, bool out_bf16, hipStream_t s) {
-    const dim3 grid((unsigned)p.grid, (unsigned)p.parts), block((unsigned)(64 * p.waves));
-    const SmallCut cut{p.per, p.grid, (uint32_t)p.waves | (uint32_t)p.chunk << 8 | (uint32_t)out_bf16 << 16 | (uint32_t)(p.parts > 1) << 17 | (uint32_t)p.groups << 18};
+    const dim3 grid = p.row_tiles > 1 ? dim3(8, (unsigned)p.row_tiles, (unsigned)((p.grid * p.parts + 7) / 8)) : dim3((unsigned)p.grid, (unsigned)p.parts), block((unsigned)(64 * p.waves));
+    const SmallCut cut{p.per, p.grid, (uint32_t)p.waves | (uint32_t)p.chunk << 8 | (uint32_t)out_bf16 << 16 | (uint32_t)(p.parts > 1) << 17 | (uint32_t)p.groups << 18 | (uint32_t)(p.row_tiles > 1) << 31};
     hipError_t e;
     if (gated) {
         if ((e = allow_full_lds<gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallGated>>()) != hipSuccess) return e;
@@ -538,7 +550,7 @@ bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t
     if (encoding != QMM_Q4_0 && encoding != QMM_Q4_K && encoding != QMM_Q5_K && encoding != QMM_Q6_K) return false;
     // (with the name of an encoding's older small-batch kernel this one goes too)
     if (kernel_disabled("kquant_small") || kernel_disabled(encoding == QMM_Q4_0 ? "q4_0_small" : encoding == QMM_Q4_K ? "q4k_mm" : encoding == QMM_Q5_K ? "q5k_mm" : "q6k_mm")) return false;
-    if (m < 1 || m > (lhs_dtype == QMM_F32 ? 8 : 16) || n < 1 || n > 0x7fffff00 || k < 256 || k % 256 || k > (1 << 20)) return false;
+    if (m < 1 || m > small_most_rows(lhs_dtype) * 4 || n < 1 || n > 0x7fffff00 || k < 256 || k % 256 || k > (1 << 20)) return false;
     if (encoding == QMM_Q4_K || encoding == QMM_Q5_K) return ((uintptr_t)w & 15) == 0;
     if (encoding == QMM_Q4_0) return ((uintptr_t)w & 3) == 0;
     // (loads of four bytes at least: the last block of the matrix has to end at a multiple of four)
@@ -558,6 +570,25 @@ __global__ __launch_bounds__(256) void small_sum_bf16_kernel(const float* __rest
     for (int j = 0; j < parts; j++) v += part[j * count + i];
     out[i] = f2bf(v);
 }
+// The same for matrices that share a launch: matrix j has the values from end[j - 1] to end[j], and their shares at part[j], one after the other.
+struct SmallSums {
+    const float* part[kLanesMaxMats];
+    float* out[kLanesMaxMats];
+    int64_t end[kLanesMaxMats];
+};
+__global__ __launch_bounds__(256) void small_sum_mats_kernel(SmallSums sums, int parts) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= sums.end[kLanesMaxMats - 1]) return;
+    const float* part = sums.part[0];
+    float* out = sums.out[0];
+    int64_t first = 0, end = sums.end[0];
+#pragma unroll
+    for (int j = 1; j < kLanesMaxMats; j++)
+        if (i >= sums.end[j - 1]) part = sums.part[j], out = sums.out[j], first = sums.end[j - 1], end = sums.end[j];
+    float v = 0.0f;
+    for (int j = 0; j < parts; j++) v += part[j * (end - first) + i - first];
+    out[i - first] = v;
+}
 }  // namespace
 // out[i] = bf16(part[i] + part[count + i] + ...), in that order
 hipError_t launch_sum_shares_bf16(const float* part, uint16_t* out, int64_t count, int shares, hipStream_t s) {
@@ -566,7 +597,7 @@ hipError_t launch_sum_shares_bf16(const float* part, uint16_t* out, int64_t coun
 }
 
 // count matrices [ns[j], k] that share the lhs; gated: two of the same size, gate and up, outs[0] = silu(lhs gate^T) * (lhs up^T).  The caller has asked
-// gemv_kquant_small_supported for each.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (the plain call) gemv_kquant_small_workspace_bytes.
+// gemv_kquant_small_supported for each.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (not gated) gemv_kquant_small_workspace_bytes with n = the sum of ns.
 hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs, int64_t m, int64_t k,
                                     bool gated, bool out_bf16, void* workspace, hipStream_t s) {
     if (count < 1 || count > kLanesMaxMats || (gated && (count != 2 || ns[0] != ns[1]))) return hipErrorInvalidValue;
@@ -581,16 +612,29 @@ hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype
         mats.tile_end[j] = (int)tiles;
     }
     mats.count = count;
-    const bool parts = count == 1 && workspace && small_parts(encoding, lhs_dtype, m, ns[0], k);
-    if (parts) mats.out[0] = (float*)workspace;
-    const SmallPlan p = small_plan(encoding, m, gated ? tiles / 2 : tiles, k, gated, parts);
+    int64_t all = 0;
+    for (int j = 0; j < count; j++) all += ns[j];
+    const bool parts = !gated && workspace && small_parts(encoding, lhs_dtype, m, all, k);
+    SmallSums sums;
+    int64_t values = 0;
+    if (parts)
+        for (int j = 0; j < kLanesMaxMats; j++) {
+            sums.part[j] = mats.out[j] = (float*)workspace + values * small_groups(k);
+            sums.out[j] = outs[std::min(j, count - 1)];
+            if (j < count) values += m * ns[j];
+            sums.end[j] = values;
+        }
+    const SmallPlan p = small_plan(encoding, lhs_dtype, m, gated ? tiles / 2 : tiles, k, gated, parts);
     const bool store_bf16 = out_bf16 && !parts;
     hipError_t e = encoding == QMM_Q4_0   ? run_small_rows<QMM_Q4_0>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                    : encoding == QMM_Q4_K ? run_small_rows<QMM_Q4_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                    : encoding == QMM_Q5_K ? run_small_rows<QMM_Q5_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                                           : run_small_rows<QMM_Q6_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s);
     if (e != hipSuccess || !parts) return e;
-    const int64_t values = m * ns[0];
+    if (count > 1) {  // (fp32 results: the callers with several matrices have no others)
+        small_sum_mats_kernel<<<dim3((unsigned)((values + 255) / 256)), dim3(256), 0, s>>>(sums, p.parts);
+        return hipGetLastError();
+    }
     if (!out_bf16) return launch_sum_shares((const float*)workspace, outs[0], values, p.parts, s);
     return launch_sum_shares_bf16((const float*)workspace, (uint16_t*)outs[0], values, p.parts, s);
 }

@@ -253,7 +253,8 @@ PyObject* py_grouped(PyObject*, PyObject* const* a, Py_ssize_t count) {
         if (!packed_matrix(e, t, c.k)) return none();
         rhs[i] = t->data_ptr();
         n[i] = t->size(0);
-        need = std::max(need, qmm_preferred_workspace_bytes(QMM_OP_MATMUL, e->code, nullptr, c.dtype, c.m, n[i], c.k, 0));
+        const int64_t one = qmm_preferred_workspace_bytes(QMM_OP_MATMUL, e->code, nullptr, c.dtype, c.m, n[i], c.k, 0);
+        need = c.m <= 64 ? need + one : std::max(need, one);  // (few rows: matrices that share a launch have their parts of K next to each other)
     }
     for (Py_ssize_t i = 0; i < mats; i++) {
         out[i] = c.result(n[i], at::kFloat);

@@ -393,9 +393,42 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 //   4096 x 4096 5.5 / 4.9, 4096 x 14336 16.7 / 10.9, but 2048 x 5632 6.0 / 7.2, 28672 x 8192 25 / 27; 4 rows 4096 x 4096 7.4 / 5.4, 14336 x 4096 12.7 / 9.5; 8 rows 8.7 / 6.7, 13.4 / 10.4, 4096 x 14336 16.7 / 12.6;
 //   16 bf16 rows 32000 x 512 13.0 / 10.5, 1024 x 14336 14.7 / 12.4, but 4096 x 4096 8.7 / 10.2.
 // - Q6_K, five and six fp32 rows, K = 256 or 512: more exact weight by weight (decode_sums_more_exactly), 0.85e-7 against 0.88e-7.
+// More rows than one workgroup takes (fp32: 8, bf16: 16), GPTQ too: two to four workgroups side by side, each of which streams the weights itself, against the lhs prepared by a launch of its own and the direct, shared or older
+// small-batch GEMM.  us, those / here (45 matrices of 128 .. 38000 rows and K of 512 .. 28672, and groups of two to sixteen; weights from memory):
+// - 9 .. 16 fp32 rows: Q4_K 4096 x 4096 11.7 / 9.2, 14336 x 4096 21.7 / 15.5, 4096 x 14336 25.5 / 19.1, 1024 x 14336 23.9 / 11.4, but 8192 x 28672 61 / 100; GPTQ 4096 x 4096 12.0 / 8.9, but 8192 x 8192 21.7 / 28.8;
+//   Q4_0 5856 x 4096 10.0 / 8.6, 39368 x 512 16.2 / 9.2, but 14336 x 4096 13.5 / 13.7, 3144 x 8192 11.1 / 12.3.
+// - 17 .. 32 fp32 rows: Q4_K 912 x 1024 7.9 / 4.3, 1024 x 14336 24.6 / 13.5; 4096 x 4096 11.9 / 11.4, but 4096, 1024 and 1024 x 4096 in one call 12.9 / 15; GPTQ (never in groups) 4096 x 4096 12.3 / 11.5;
+//   Q4_0 4096, 1024 and 1024 x 4096 15.2 / 11.0.
+// - 17 .. 32 bf16 rows: Q4_K 4096 x 4096 10.5 / 9.8, 14336 x 4096 19.6 / 17.4, 1024 x 14336 19.9 / 11.8, but 32000 x 4096 31 / 34, 8192 x 8192 20.6 / 22, Q5_K 5120 x 5120 17.8 / 15.3, but with two of 1024 x 5120
+//   15.9 / 19.9; Q4_0 600 x 2048 7.9 / 6.9, 21848 x 2560 27 / 20, but 2520 x 2048 20 % longer.
+// - 33 .. 64 bf16 rows: Q4_K 912 x 1024 7.9 / 4.8, 512 x 28672 31 / 15, but two of 1024 x 14336 18.8 / 26; 1520 x 3072 5 % less, 2048 x 5632 12.2 / 13.0; GPTQ 4096 x 4096 12.7 / 11.6.
+// The lines follow K more than the number of weight rows: a call with several matrices sends each where a call of its own would, and two ways for one call cost more than either.
+static bool small_tiles_wanted(int encoding, bool f32, int64_t m, int64_t n, int64_t k) {
+    const int64_t million = (int64_t)1 << 20, weights = n * k;
+    const bool q6 = encoding == QMM_Q6_K;
+    if (encoding == QMM_GPTQ) {
+        if (f32 && m <= 16) return k <= 4096 || weights < (k <= 8192 ? 60 : 80) * million;
+        if (f32) return m <= 32 && weights < (k <= 4096 ? 17 : k <= 8192 ? 24 : 40) * million;
+        if (m <= 32) return weights < (k <= 2048 ? 16 : k <= 4096 ? 80 : k <= 8192 ? 40 : 45) * million;
+        return m <= 64 && weights < (k <= 2048 ? 5 : k <= 4096 ? 20 : k <= 8192 ? 4 : 16) * million;
+    }
+    if (encoding == QMM_Q4_0) {
+        if (f32 && m <= 16) return weights < (k <= 3072 ? 128 : k <= 4096 ? 50 : k <= 8192 ? 24 : 70) * million;
+        if (f32) return m <= 32 && weights < (k <= 4096 ? 45 : k <= 8192 ? 28 : 40) * million;
+        if (k > 8192) return n <= (m <= 32 ? 2048 : m <= 64 ? 512 : 0);
+        if (k <= 2048 && weights < 3 * million) return m <= 64;
+        return m <= 32 && k <= 4096 && weights >= 18 * million && weights < 110 * million;
+    }
+    if (f32 && m <= 16) return weights < (k <= 8192 ? 256 : 128) * million;
+    if (k > 8192) return n <= (f32 ? (m > 32 ? 0 : q6 ? 768 : 1024) : m <= 32 ? (q6 ? 768 : 2048) : m <= 64 ? 512 : 0);
+    if (!f32 && m <= 32) return k <= 4096 && weights < (k <= 2048 ? 16 : 64) * million;
+    return m <= (f32 ? 32 : 64) && k <= 1024 && weights < 5 * million;
+}
+
 static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
     if (m < 1 || (m == 1 && (encoding == QMM_Q4_K || encoding == QMM_Q4_0) && k <= 14528 && (k > 2048 || n < 8192)) || (m == 1 && encoding == QMM_Q4_K && k > 2048) || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
     const bool f32 = lhs_dtype == QMM_F32;
+    if (m > qmm::small_most_rows(lhs_dtype)) return !(encoding == QMM_Q5_K && q5k_mm_forced()) && !(encoding == QMM_Q6_K && q6k_mm_forced()) && small_tiles_wanted(encoding, f32, m, n, k);
     if (m == 1) {
         if (encoding == QMM_Q4_K) return true;
         if (encoding == QMM_Q5_K) return !q5k_mm_forced() && (k <= 2048 || k > 8192 || n > 2048);
@@ -420,7 +453,8 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
 // 4096 x 14336 15.3 / 10.9; four bf16 rows 9.4 / 5.5, 12.4 / 9.0, 15.2 / 11.3; eight fp32 rows 13.6 / 7.7, 18.3 / 12.6, 20.9 / 12.9; 16 bf16 rows 11.1 / 8.9, 14.3 / 13.5, 16.8 / 14.6.  Relative error, K = 4096: 4.2e-7 /
 // 0.8e-7 (fp32 rows), 2.2e-7 and 1.2e-7 / 0.65e-7 (one and four bf16 rows).
 static bool gptq_small_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    return encoding == QMM_GPTQ && cfg && !cfg->desc_act && qmm::gemv_gptq_small_supported(lhs_dtype, m, n, k, cfg->group_size);
+    return encoding == QMM_GPTQ && cfg && !cfg->desc_act && (m <= qmm::small_most_rows(lhs_dtype) || small_tiles_wanted(encoding, lhs_dtype == QMM_F32, m, n, k)) &&
+           qmm::gemv_gptq_small_supported(lhs_dtype, m, n, k, cfg->group_size);
 }
 
 // Does the kernel that serves this problem store bf16 itself?  (The Q4_K decode kernel does; everything else goes
@@ -475,15 +509,22 @@ static int64_t preferred_matmul(int encoding, const qmm_gptq_config* cfg, int lh
         return order ? std::max(need, order + ((flags & QMM_FLAG_OUT_BF16) ? up256(m * n * 4) : 0)) : need;
     }
     int64_t ahead = 0;
-    if (!(flags & QMM_FLAG_ACT_Q8K) && gptq_small_wanted(encoding, cfg, lhs_dtype, m, n, k)) return std::max(need, up256(qmm::gemv_gptq_small_workspace_bytes(lhs_dtype, m, n, k, cfg->group_size)) + (flags & QMM_FLAG_OUT_BF16 ? up256(m * n * 4) : 0));
-    if (!(flags & QMM_FLAG_ACT_Q8K) && small_wanted(encoding, lhs_dtype, m, n, k, nullptr)) return std::max(need, up256(qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, n, k)) + (flags & QMM_FLAG_OUT_BF16 ? up256(m * n * 4) : 0));
+    // the kernels for a few rows; from where others served the call, also what those need (the weights' alignment is not known here)
+    int64_t few = -1;
+    if (!(flags & QMM_FLAG_ACT_Q8K) && gptq_small_wanted(encoding, cfg, lhs_dtype, m, n, k)) few = qmm::gemv_gptq_small_workspace_bytes(lhs_dtype, m, n, k, cfg->group_size);
+    else if (!(flags & QMM_FLAG_ACT_Q8K) && small_wanted(encoding, lhs_dtype, m, n, k, nullptr)) few = qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, n, k);
+    if (few >= 0) {
+        const int64_t direct = m > qmm::small_most_rows(lhs_dtype) && direct_wanted(encoding, cfg, lhs_dtype, m, n, k) ? qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k) : 0;
+        return std::max(std::max(need, direct), up256(few) + (flags & QMM_FLAG_OUT_BF16 ? up256(m * n * 4) : 0));
+    }
     if (flags & QMM_FLAG_ACT_Q8K) {  // (the lhs as fp32 rows in front, where the integer kernels do not serve the call)
         if (q8k_integer_kernel(encoding, m, k) || (flags & QMM_FLAG_OUT_BF16)) return need;
         ahead = up256(m * k * 4);
         lhs_dtype = QMM_F32;
+        if (small_wanted(encoding, lhs_dtype, m, n, k, nullptr)) few = qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, n, k);
     }
-    if (!direct_wanted(encoding, cfg, lhs_dtype, m, n, k)) return need;
-    return std::max(need, ahead + qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k));
+    if (!direct_wanted(encoding, cfg, lhs_dtype, m, n, k)) return few > 0 ? std::max(need, ahead + up256(few)) : need;
+    return std::max(need, ahead + std::max(few > 0 ? up256(few) : 0, qmm::gemm_direct_workspace_bytes(encoding, lhs_dtype, m, k)));
 }
 
 // Where a call takes a workspace at all, the figure holds what the direct GEMM needs too (up to a size that the static buffer also has).
@@ -1056,9 +1097,13 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
             if (aligned(out[j], 4) && small_wanted(encoding, lhs_dtype, m, n[j], k, rhs[j])) direct_w[directs] = rhs[j], direct_n[directs] = n[j], direct_out[directs++] = out[j];
             else rest_w[rest] = rhs[j], rest_n[rest] = n[j], rest_out[rest++] = out[j];
         }
-        for (int j = 0; j < directs; j += qmm::kLanesMaxMats) {
-            const hipError_t e = qmm::launch_gemv_kquant_small(encoding, lhs, lhs_dtype, std::min(qmm::kLanesMaxMats, directs - j), direct_w + j, direct_n + j, direct_out + j, m, k,
-                                                               false, false, nullptr, (hipStream_t)stream);
+        for (int j = 0, take; j < directs; j += take) {
+            take = std::min(qmm::kLanesMaxMats, directs - j);
+            int64_t all = 0;
+            for (int i = 0; i < take; i++) all += direct_n[j + i];
+            const int64_t share = qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, all, k);  // (of groups of K side by side; the same sums without)
+            void* const parts = share > 0 && workspace && aligned(workspace, 256) && workspace_bytes >= share ? workspace : nullptr;
+            const hipError_t e = qmm::launch_gemv_kquant_small(encoding, lhs, lhs_dtype, take, direct_w + j, direct_n + j, direct_out + j, m, k, false, false, parts, (hipStream_t)stream);
             if (e != hipSuccess) return hip_status(e, "qmm_matmul_grouped(K-quant small batch)");
         }
         if (directs > 0)
@@ -1146,6 +1191,11 @@ int64_t qmm_matmul_swiglu_workspace_bytes(int encoding, int lhs_dtype, int64_t m
     return align_up(required_bytes(encoding, lhs_dtype, m, n, k), 256) + 2 * align_up(m * n * 4, 256);
 }
 
+// What gate and up side by side take for their groups of K (0: not so, or one group).
+static int64_t swiglu_share(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    return small_wanted(encoding, lhs_dtype, m, n, k, nullptr) ? qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, 2 * n, k) : 0;
+}
+
 int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, int64_t k, const void* gate, const void* up,
                       int64_t n, float* out, void* workspace, int64_t workspace_bytes, void* stream) {
     if (!lhs || !gate || !up || !out) return fail(QMM_ERR_INVALID, "qmm_matmul_swiglu: null pointer");
@@ -1174,8 +1224,8 @@ int qmm_matmul_swiglu(int encoding, const void* lhs, int lhs_dtype, int64_t m, i
         return fail(QMM_ERR_WORKSPACE, "qmm_matmul_swiglu: workspace of %lld bytes required, %lld given", (long long)(mm_ws + 2 * plane),
                     (long long)workspace_bytes);
     if (!aligned(workspace, 256)) return fail(QMM_ERR_INVALID, "qmm_matmul_swiglu: workspace must be 256-byte aligned");
-    // where the small-batch kernel would serve both products
-    if (small_wanted(encoding, lhs_dtype, m, n, k, gate) && small_wanted(encoding, lhs_dtype, m, n, k, up)) {
+    // where the small-batch kernel would serve both products (but for groups of K side by side: 1024 x 14336 16 bf16 rows 32 us here, 18 as two products)
+    if (small_wanted(encoding, lhs_dtype, m, n, k, gate) && small_wanted(encoding, lhs_dtype, m, n, k, up) && (swiglu_share(encoding, lhs_dtype, m, n, k) == 0 || swiglu_share(encoding, lhs_dtype, m, n, k) > mm_ws)) {
         const void* const both[2] = {gate, up};
         const int64_t ns[2] = {n, n};
         float* const outs[2] = {out, out};
@@ -1207,7 +1257,7 @@ int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_confi
         case QMM_OP_RMSNORM: return up256(m * k * (lhs_dtype == QMM_F32 ? 4 : 2)) + preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, flags);
         case QMM_OP_SWIGLU: {
             const int64_t need = qmm_matmul_swiglu_workspace_bytes(encoding, lhs_dtype, m, n, k);
-            return need ? std::max(need, up256(preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, 0)) + 2 * up256(m * n * 4)) : 0;
+            return need ? std::max(need, std::max(up256(preferred_matmul(encoding, cfg, lhs_dtype, m, n, k, 0)), up256(swiglu_share(encoding, lhs_dtype, m, n, k))) + 2 * up256(m * n * 4)) : 0;
         }
         case QMM_OP_REPACKED: {
             const int64_t need = qmm_matmul_repacked_workspace_bytes(encoding, lhs_dtype, m, n, k);

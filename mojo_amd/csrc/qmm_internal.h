@@ -130,8 +130,10 @@ hipError_t launch_gemv_q4_k_rows(const void* a, int a_dtype, const uint8_t* w, i
                                  float* out, int64_t ldo, hipStream_t s);
 hipError_t launch_gemv_q6_k(const void* a, int a_dtype, const uint8_t* w, int m, int64_t n, int64_t k,
                             float* out, int64_t ldo, hipStream_t s);
-// gemv_kquant_small.hip: Q4_K, Q5_K, Q6_K with up to 16 bf16 or 8 fp32 lhs rows.  gated: two matrices of the same size, gate and
-// up, outs[0] = silu(gate) * up.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (one matrix, fp32 result) what gemv_kquant_small_workspace_bytes says; the same sums.
+// Lhs rows of a workgroup of the kernels for a few rows at most.
+inline int64_t small_most_rows(int lhs_dtype) { return lhs_dtype == QMM_F32 ? 8 : 16; }
+// gemv_kquant_small.hip: Q4_0, Q4_K, Q5_K, Q6_K with up to four times as many lhs rows.  gated: two matrices of the same size, gate and
+// up, outs[0] = silu(gate) * up.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (not gated) what gemv_kquant_small_workspace_bytes says, with n = the sum of ns; the same sums.
 int64_t gemv_kquant_small_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k);
 bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w);
 hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs, int64_t m, int64_t k,

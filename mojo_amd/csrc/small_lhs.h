@@ -12,6 +12,13 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float2v __attribute__((ext_vector_type(2)));
 typedef int ks_int4 __attribute__((ext_vector_type(4)));
 
+// Lhs rows that one workgroup takes at most: a lane holds sums of four operand rows, and an fp32 row is two of them.  More rows go to several workgroups, each of which streams the weights itself.
+template <typename AT>
+constexpr int small_rows() { return sizeof(AT) == 4 ? 8 : 16; }
+static_assert(small_rows<float>() == 8 && small_rows<uint16_t>() == 16, "small_most_rows");
+// Places for workgroups on the part, `tiles` that share weights counted as one; these stay on one XCD, so it is what fits each of the eight.
+inline int64_t small_places(int per_cu, int tiles) { return tiles == 1 ? (int64_t)compute_units() * per_cu : (int64_t)compute_units() * per_cu / 8 / tiles * 8; }
+
 constexpr int kSmallPlane = 528;  // an lhs row of 256 columns on its way between lanes: 512 bytes + 16 (bank spread)
 
 // 16 bytes per lane, global (uniform base + lane offset) -> LDS at lds_base + 16 * lane.  ONCE: non-temporal.

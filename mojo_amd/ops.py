@@ -319,7 +319,8 @@ def qmatmul_grouped(encoding: QuantizationEncoding, lhs: torch.Tensor, rhs: Sequ
     lib = _lib.load()
     lhs_dt = _DTYPES[lhs.dtype]
     outs = [torch.empty((m, w.shape[0]), dtype=torch.float32, device=lhs.device) for w in rhs]
-    need = max(lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, encoding.code, None, lhs_dt, m, w.shape[0], k, 0) for w in rhs)
+    needs = [lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, encoding.code, None, lhs_dt, m, w.shape[0], k, 0) for w in rhs]
+    need = sum(needs) if m <= 64 else max(needs)  # (few rows: matrices that share a launch have their parts of K next to each other)
     ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
     count = len(rhs)
     rhs_p = (C.c_void_p * count)(*[w.data_ptr() for w in rhs])

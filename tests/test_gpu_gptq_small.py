@@ -35,7 +35,7 @@ def check(config, rhs, got, a, bits=22):
 @pytest.mark.parametrize("m,n,k", [(1, 16, 256), (2, 24, 512), (3, 1000, 768), (4, 14344, 4096), (1, 4104, 4352), (8, 264, 8192), (7, 4200, 11008), (16, 1000, 2560), (9, 16, 14336), (12, 8200, 4096), (16, 4112, 5120)])
 def test_against_float64(group, lhs, m, n, k):
     config, rhs = tensors(n, k, group)
-    a = rows(min(m, 8) if lhs == torch.float32 else m, k, lhs)  # (from nine fp32 rows on other kernels serve the call)
+    a = rows(min(m, 8) if lhs == torch.float32 else m, k, lhs)
     check(config, rhs, qmatmul(QE.GPTQ, config, a, *rhs), a)
     check(config, rhs, qmatmul(QE.GPTQ, config, a, *rhs, out_dtype=torch.bfloat16), a, bits=8)
 

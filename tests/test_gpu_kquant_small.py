@@ -1,9 +1,11 @@
-"""Q4_0, Q4_K, Q5_K and Q6_K with 1 .. 16 lhs rows: the small-batch kernel at the edges of its tiles (16 weight rows), of its groups of K (up to 16 super-blocks, divided
+"""Q4_0, Q4_K, Q5_K and Q6_K (and GPTQ, where it has the same rules) with 1 .. 64 lhs rows: the small-batch kernel at the edges of its tiles (16 weight rows), of its groups of K (up to 16 super-blocks, divided
 evenly) and of its lhs rows (2, 4, 8, 16), against float64 products of the dequantised weights."""
+import ctypes
+
 import pytest
 import torch
 
-from mojo_amd import QuantizationEncoding as QE, dequantize, qmatmul, qmatmul_grouped, qmatmul_swiglu, quantize
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, dequantize, qmatmul, qmatmul_grouped, qmatmul_swiglu, quantize
 from mojo_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -32,7 +34,7 @@ def check(enc, got, w, a, bits=22):
 # (18 rows of one block: with 17 the number of Q6_K blocks is odd, which is not this kernel's, see below)
 @pytest.mark.parametrize("m,n,k", [(2, 18, 256), (3, 1000, 768), (4, 4104, 4096), (5, 40, 4352), (8, 264, 8192), (7, 4200, 11008), (16, 1001, 2560), (9, 16, 14336), (12, 8200, 512), (16, 4112, 5120)])
 def test_against_float64(enc, lhs, m, n, k):
-    w, a = packed(enc, n, k), rows(min(m, 8) if lhs == torch.float32 else m, k, lhs)  # (from nine fp32 rows on other kernels serve the call)
+    w, a = packed(enc, n, k), rows(min(m, 8) if lhs == torch.float32 else m, k, lhs)
     check(enc, qmatmul(QE[enc], None, a, w), w, a)
     check(enc, qmatmul(QE[enc], None, a, w, out_dtype=torch.bfloat16), w, a, bits=8)
 
@@ -128,3 +130,55 @@ def test_workspace_is_what_the_parts_of_k_need():
     lib = _lib.load()
     need = lib.qmm_preferred_workspace_bytes(0, 1, None, 0, 4, 4096, 14336, 0)
     assert need >= 4 * 4 * 4096 * 4  # four groups of K, [4, 4096] fp32 each
+
+
+def alone(encoding, config, a, rhs, step):
+    """The rows of `a` in calls of `step` rows, the last of which repeats rows of the one before."""
+    m, out = a.shape[0], []
+    for r in range(0, m, step):
+        first = max(0, min(r, m - step))
+        out.append(qmatmul(encoding, config, a[first : first + step].contiguous(), *rhs)[r - first :])
+    return torch.cat(out)
+
+
+def tile_calls():
+    everywhere = ((16, 256), (1000, 1536), (136, 4608), (264, 14336), (1032, 11008))
+    for enc in ("Q4_0", "GPTQ", *ENCODINGS):
+        for lhs, each in ((torch.float32, 8), (torch.bfloat16, 16)):
+            for tiles in (2, 3, 4):
+                if enc == "GPTQ" or (lhs == torch.float32 and (tiles == 2 or enc == "Q4_0")):
+                    shapes = everywhere
+                elif enc == "Q4_0" or (lhs == torch.bfloat16 and tiles == 2):  # (the others go to other kernels)
+                    shapes = ((16, 256), (1000, 1536), (264, 14336))
+                else:
+                    shapes = ((16, 256), (1000, 768), (264, 14336))
+                for n, k in shapes:
+                    yield enc, lhs, each, n, k, tiles
+
+
+@pytest.mark.parametrize("enc,lhs,rows_each,n,k,tiles", list(tile_calls()))
+def test_tiles_of_lhs_rows(enc, lhs, rows_each, n, k, tiles):
+    """More rows than a workgroup takes: the sums of calls with the rows of one; a last tile of one row and a full one; results in bf16; in a group; with less memory than groups of K need."""
+    config, more = None, ()
+    if enc == "GPTQ":
+        gen = torch.Generator(device="cuda").manual_seed(n + k)
+        words = lambda *shape: torch.randint(-(2**31), 2**31, shape, device="cuda", generator=gen, dtype=torch.int64).to(torch.int32)
+        config, rhs = QuantizationConfig("gptq", 4, 128, False, False), (words(k // 8, n), torch.empty((k // 128, n), device="cuda").uniform_(1e-3, 4e-3, generator=gen).half(), words(k // 128, n // 8))
+    else:
+        rhs, more = (packed(enc, n, k),), (packed(enc, n + 16, k, 1),)
+    encoding, lib = QE[enc], _lib.load()
+    for m in (rows_each * (tiles - 1) + 1, rows_each * tiles):
+        a = rows(m, k, lhs)
+        a[m - 1] *= 3.0 if enc == "Q4_0" else 1e30  # (a row that is scaled on its way to fp16; Q8_0 scales are fp16)
+        want = alone(encoding, config, a, rhs, rows_each)
+        assert torch.equal(qmatmul(encoding, config, a, *rhs), want)
+        assert torch.equal(qmatmul(encoding, config, a, *rhs, out_dtype=torch.bfloat16), want.bfloat16())
+        if more:
+            for got, w in zip(qmatmul_grouped(encoding, a, [*rhs, *more]), (rhs, more)):
+                assert torch.equal(got, alone(encoding, config, a, w, rows_each))
+        out, ptrs = torch.empty((m, n), device="cuda"), (ctypes.c_void_p * len(rhs))(*(t.data_ptr() for t in rhs))
+        cfg = _lib.GptqConfig(4, 128, 0, 0) if config else None
+        kind = _lib.QMM_F32 if lhs == torch.float32 else _lib.QMM_BF16
+        ws = torch.empty(max(256, lib.qmm_matmul_workspace_bytes(encoding.code, kind, m, n, k)), dtype=torch.uint8, device="cuda")
+        assert lib.qmm_matmul(encoding.code, cfg and ctypes.byref(cfg), a.data_ptr(), kind, m, k, ptrs, len(rhs), n, out.data_ptr(), ws.data_ptr(), ws.numel(), 0, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(out, want)
