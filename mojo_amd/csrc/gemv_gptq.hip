@@ -1,4 +1,4 @@
-// GPTQ decode kernel for m <= 4 lhs rows.
+// GPTQ decode kernel for m <= 4 lhs rows, for what gemv_gptq_small.hip declines (K no multiple of 256, other groups).
 //
 // qweight is [K/8, N] int32: a dword holds 8 consecutive k of one output column, and a row of
 // dwords is contiguous in N.  A lane owns one output column; a wavefront's load of one k8 row is

@@ -1,4 +1,4 @@
-// GPTQ small-batch kernel (2..16 lhs rows per pass) on the matrix cores.
+// GPTQ small-batch kernel (2..16 lhs rows per pass) on the matrix cores, for what gemv_gptq_small.hip declines (K no multiple of 256, other groups, the calls named at its rule).
 //
 // A qweight word holds eight consecutive k of one column, which is exactly what a lane supplies of the B
 // operand of v_mfma_f32_16x16x32_f16 (lane l: column l % 16, k = 8 * (l / 16) .. + 7): a lane loads the words of

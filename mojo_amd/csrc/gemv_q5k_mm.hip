@@ -1,4 +1,4 @@
-// Q5_K with up to 16 lhs rows a pass on the matrix cores, K a multiple of 512: the small-batch kernel of Q6_K
+// Q5_K with up to 16 lhs rows a pass on the matrix cores, K a multiple of 512, for what gemv_kquant_small.hip does not take (the rule is in qmm_api.hip): the small-batch kernel of Q6_K
 // (gemv_q6k_mm.hip: persistent workgroups over 16-row tiles, a wavefront owns two super-blocks of every row and keeps the
 // lhs operands of its 512 columns in registers, rows global -> LDS directly into a private ring, partial tiles added
 // through LDS) with Q5_K's arithmetic.

@@ -73,13 +73,6 @@ __device__ __forceinline__ void hidden_load(u32x4& d, const void* g) {
 __device__ __forceinline__ void hidden_load(u32x2& d, const void* g) {
     asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(d) : "v"(g) : "memory");
 }
-// The same from a wave-uniform base and a byte offset per lane.
-__device__ __forceinline__ void hidden_load(u32x4& d, uint32_t lane_offset, const void* uniform_base) {
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(d) : "v"(lane_offset), "s"(uniform_base) : "memory");
-}
-__device__ __forceinline__ void hidden_load(u32x2& d, uint32_t lane_offset, const void* uniform_base) {
-    asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(d) : "v"(lane_offset), "s"(uniform_base) : "memory");
-}
 template <typename T>
 __device__ __forceinline__ void tie(T& d) {
     asm volatile("" : "+v"(d));

@@ -402,6 +402,7 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 // - 17 .. 32 bf16 rows: Q4_K 4096 x 4096 10.5 / 9.8, 14336 x 4096 19.6 / 17.4, 1024 x 14336 19.9 / 11.8, but 32000 x 4096 31 / 34, 8192 x 8192 20.6 / 22, Q5_K 5120 x 5120 17.8 / 15.3, but with two of 1024 x 5120
 //   15.9 / 19.9; Q4_0 600 x 2048 7.9 / 6.9, 21848 x 2560 27 / 20, but 2520 x 2048 20 % longer.
 // - 33 .. 64 bf16 rows: Q4_K 912 x 1024 7.9 / 4.8, 512 x 28672 31 / 15, but two of 1024 x 14336 18.8 / 26; 1520 x 3072 5 % less, 2048 x 5632 12.2 / 13.0; GPTQ 4096 x 4096 12.7 / 11.6.
+// (17 .. 32 bf16 rows with the weights in the last-level cache, which a program's layers do not stay in: Q4_K 4096 x 4096 8.7 / 9.8, Q4_0 14336 x 4096 16.8 / 19.3.)
 // The lines follow K more than the number of weight rows: a call with several matrices sends each where a call of its own would, and two ways for one call cost more than either.
 static bool small_tiles_wanted(int encoding, bool f32, int64_t m, int64_t n, int64_t k) {
     const int64_t million = (int64_t)1 << 20, weights = n * k;

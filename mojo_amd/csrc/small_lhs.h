@@ -21,6 +21,13 @@ inline int64_t small_places(int per_cu, int tiles) { return tiles == 1 ? (int64_
 
 constexpr int kSmallPlane = 528;  // an lhs row of 256 columns on its way between lanes: 512 bytes + 16 (bank spread)
 
+// hidden_load from a wave-uniform base and a byte offset per lane.
+__device__ __forceinline__ void hidden_load(u32x4& d, uint32_t lane_offset, const void* uniform_base) {
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(d) : "v"(lane_offset), "s"(uniform_base) : "memory");
+}
+__device__ __forceinline__ void hidden_load(u32x2& d, uint32_t lane_offset, const void* uniform_base) {
+    asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(d) : "v"(lane_offset), "s"(uniform_base) : "memory");
+}
 // 16 bytes per lane, global (uniform base + lane offset) -> LDS at lds_base + 16 * lane.  ONCE: non-temporal.
 template <bool ONCE = true>
 __device__ __forceinline__ void small_stream16(uint32_t lane_offset, const void* uniform_base, uint32_t lds_base) {
