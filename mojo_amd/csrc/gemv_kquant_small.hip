@@ -252,7 +252,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
         for (int g = g_first; g < g_end; g++) {
             const int sb = g * waves + wave;
             if (sb < nblk) {  // (all wavefronts but for the last group)
-            if (groups > 1 && c0 + g > g_first) {
+            if (g_end - g_first > 1 && c0 + g > g_first) {  // (a group of its own: the operands of the chunk before)
                 xraw_t xr[MROWS];
 #pragma unroll
                 for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(row0 + j, m - 1) * k + sb * 256) + a_lane);

@@ -100,3 +100,11 @@ def test_rmsnorm_in_front():
     a, gamma = rows(3, 2048, torch.float32), 1.0 + 0.1 * torch.randn(2048, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
     normal = a * torch.rsqrt((a.double() ** 2).mean(dim=1, keepdim=True) + 1e-5).float() * gamma
     check(config, rhs, qmatmul_rmsnorm(QE.GPTQ, config, a, gamma, 1e-5, *rhs), normal, bits=21)  # (and the normalisation's rounding)
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 8200, 8192), (24, 2048, 8192)])
+def test_tiles_that_leave_lds_one_by_one(m, n, k):
+    """fp32 rows, groups of K side by side, results of one tile in LDS at a time: the operands of the group serve every tile of the workgroup."""
+    config, rhs = tensors(n, k, 128)
+    a = rows(m, k, torch.float32)
+    check(config, rhs, qmatmul(QE.GPTQ, config, a, *rhs), a)

@@ -132,6 +132,13 @@ def test_workspace_is_what_the_parts_of_k_need():
     assert need >= 4 * 4 * 4096 * 4  # four groups of K, [4, 4096] fp32 each
 
 
+@pytest.mark.parametrize("enc,m,n,k", [("Q6_K", 16, 4104, 14336), ("Q4_K", 16, 28680, 8192)])
+def test_tiles_that_leave_lds_a_few_at_a_time(enc, m, n, k):
+    """Groups of K side by side, results of some of a workgroup's tiles in LDS at a time: the operands of the group serve all of them."""
+    w, a = packed(enc, n, k), rows(m, k, torch.bfloat16)
+    check(enc, qmatmul(QE[enc], None, a, w), w, a)
+
+
 def alone(encoding, config, a, rhs, step):
     """The rows of `a` in calls of `step` rows, the last of which repeats rows of the one before."""
     m, out = a.shape[0], []
