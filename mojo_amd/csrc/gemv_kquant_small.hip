@@ -557,6 +557,13 @@ bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t
     return ((uintptr_t)w & 3) == 0 && n * (k / 256) % 2 == 0;
 }
 
+// What the fullest compute unit gets of a call whose workgroups walk K, a tile being 16 weight rows: small_tiles_wanted.
+SmallLoad small_load(int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    const SmallPlan p = small_plan(QMM_Q4_K, lhs_dtype, m, (n + 15) / 16, k, false, false);
+    const int workgroups = ((int64_t)p.grid * p.row_tiles + compute_units() - 1) / compute_units();
+    return {workgroups, workgroups * p.waves};
+}
+
 // What the parts of K of a plain call with few tiles take (without it a workgroup walks all of K: the same sums).
 int64_t gemv_kquant_small_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     return small_parts(encoding, lhs_dtype, m, n, k) ? small_groups(k) * m * n * 4 : 0;

@@ -402,34 +402,48 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 // - 17 .. 32 bf16 rows: Q4_K 4096 x 4096 10.5 / 9.8, 14336 x 4096 19.6 / 17.4, 1024 x 14336 19.9 / 11.8, but 32000 x 4096 31 / 34, 8192 x 8192 20.6 / 22, Q5_K 5120 x 5120 17.8 / 15.3, but with two of 1024 x 5120
 //   15.9 / 19.9; Q4_0 600 x 2048 7.9 / 6.9, 21848 x 2560 27 / 20, but 2520 x 2048 20 % longer.
 // - 33 .. 64 bf16 rows: Q4_K 912 x 1024 7.9 / 4.8, 512 x 28672 31 / 15, but two of 1024 x 14336 18.8 / 26; 1520 x 3072 5 % less, 2048 x 5632 12.2 / 13.0; GPTQ 4096 x 4096 12.7 / 11.6.
-// (17 .. 32 bf16 rows with the weights in the last-level cache, which a program's layers do not stay in: Q4_K 4096 x 4096 8.7 / 9.8, Q4_0 14336 x 4096 16.8 / 19.3.)
+// - What was slower than those and goes back to them: 17 .. 24 bf16 rows GPTQ 16384 x 4096 18.4 / 19.2, 4096 x 8192 and 4096 x 11008 about equal; Q6_K 15360 x 4096 26.0 / 27.2, 16384 x 2560 19.9 / 20.5; Q4_0
+//   16384 x 2560 17.1 / 16.7 (8192 x 4096 14.9 / 14.3, but weights in the last-level cache 11.8 / 13.8); 16 rows Q4_0 14336 x 1024 9.2 / 9.8, f32 2560 x 8192 10.8 / 11.1, 11008 x 4096 11.9 / 12.2, 4096 x 14336 equal;
+//   32 fp32 rows Q4_0 3584 x 11008 19.3 / 19.5.
+// - Short K: a workgroup has few wavefronts, and what counts is how many the fullest compute unit gets.  33 .. 64 bf16 rows Q4_0 3072 x 768 with 9 of them 7.4 / 8.4, 1536 x 1536 with 12 7.9 / 9.4, 1280 x 2048
+//   with 16 8.2 / 9.7, but 2560 x 1024 with 8 7.5 / 7.0; Q4_K 3584 x 1024 with 16 7.8 / 8.3, 8192 x 512 with 16 7.9 / 8.8, 4096 x 1024 with 12 7.9 / 7.1; 17 rows 6144 x 1280 with 15 8.8 / 10.4, 16384 x 512 with
+//   16 7.9 / 8.8, 12288 x 512 with 12 in six workgroups 7.8 / 8.0, but 6144 x 1024 with 12 7.8 / 7.1.
+// Weights in the last-level cache, which a program's layers do not stay in: the others read them again at little cost, and where the two are close they win.  17 bf16 rows Q4_K 4096 x 4096 8.9 / 9.5, 14336 x 4096
+// 15.3 / 17.2, Q5_K 4096 x 4096 9.3 / 10.4, Q6_K 11008 x 4096 20.6 / 21.5, Q4_0 14336 x 4096 16.9 / 19.2 (from memory 10.3 / 9.9, 19.4 / 17.5, 11.1 / 10.4, 25.2 / 22.1, 21.1 / 19.4).
 // The lines follow K more than the number of weight rows: a call with several matrices sends each where a call of its own would, and two ways for one call cost more than either.
-static bool small_tiles_wanted(int encoding, bool f32, int64_t m, int64_t n, int64_t k) {
+// (Asked once the kernel is known to take the call.)
+static bool small_tiles_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const int64_t million = (int64_t)1 << 20, weights = n * k;
-    const bool q6 = encoding == QMM_Q6_K;
+    const bool f32 = lhs_dtype == QMM_F32, q6 = encoding == QMM_Q6_K;
+    const qmm::SmallLoad load = qmm::small_load(lhs_dtype, m, n, k);
     if (encoding == QMM_GPTQ) {
         if (f32 && m <= 16) return k <= 4096 || weights < (k <= 8192 ? 60 : 80) * million;
-        if (f32) return m <= 32 && weights < (k <= 4096 ? 17 : k <= 8192 ? 24 : 40) * million;
-        if (m <= 32) return weights < (k <= 2048 ? 16 : k <= 4096 ? 80 : k <= 8192 ? 40 : 45) * million;
-        return m <= 64 && weights < (k <= 2048 ? 5 : k <= 4096 ? 20 : k <= 8192 ? 4 : 16) * million;
+        if (f32) return m <= 32 && weights < (k <= 4096 ? 16 : k <= 8192 ? 24 : 40) * million;
+        if (k <= 2048) return m <= 64 && weights < (m <= 32 ? 16 : 5) * million && load.wavefronts <= 12;
+        if (m <= 24 && k <= 4096 && weights >= 54 * million && weights < 68 * million) return false;
+        if (m <= 32) return weights < (k <= 4096 ? 80 : k <= 8192 ? 28 : 40) * million;
+        return m <= 64 && weights < (k <= 4096 ? 20 : k <= 8192 ? 4 : 16) * million;
     }
     if (encoding == QMM_Q4_0) {
-        if (f32 && m <= 16) return weights < (k <= 3072 ? 128 : k <= 4096 ? 50 : k <= 8192 ? 24 : 70) * million;
-        if (f32) return m <= 32 && weights < (k <= 4096 ? 45 : k <= 8192 ? 28 : 40) * million;
+        if (f32 && m <= 16) return weights < (k <= 3072 ? 128 : k <= 4096 ? (m <= 12 ? 50 : 40) : k <= 6144 ? 24 : k <= 8192 ? 18 : k <= 12288 ? 40 : 52) * million;
+        if (f32) return m <= 32 && weights < (k <= 4096 ? 45 : k <= 8192 ? 28 : m <= 24 ? 40 : 34) * million;
         if (k > 8192) return n <= (m <= 32 ? 2048 : m <= 64 ? 512 : 0);
-        if (k <= 2048 && weights < 3 * million) return m <= 64;
-        return m <= 32 && k <= 4096 && weights >= 18 * million && weights < 110 * million;
+        if (k <= 2048 && weights < 3 * million) return m <= 32 || (m <= 64 && load.wavefronts <= 8 && load.workgroups <= (k <= 256 ? 4 : 3));
+        return m <= 32 && k <= 4096 && weights >= 18 * million && weights < 110 * million && (weights < 28 * million || weights >= 42 * million);
     }
     if (f32 && m <= 16) return weights < (k <= 8192 ? 256 : 128) * million;
     if (k > 8192) return n <= (f32 ? (m > 32 ? 0 : q6 ? 768 : 1024) : m <= 32 ? (q6 ? 768 : 2048) : m <= 64 ? 512 : 0);
-    if (!f32 && m <= 32) return k <= 4096 && weights < (k <= 2048 ? 16 : 64) * million;
-    return m <= (f32 ? 32 : 64) && k <= 1024 && weights < 5 * million;
+    if (f32) return m <= 32 && k <= 1024 && weights < 5 * million;
+    const bool spread = load.wavefronts <= 12 && load.workgroups <= 5;
+    if (m <= 32 && k > 2048) return k <= 4096 && weights < (!q6 ? 64 : k <= 3072 ? 40 : 50) * million;
+    if (m <= 32) return weights < 16 * million && (k > 1536 || (k > 1280 ? n <= 4096 : k > 256 ? spread : load.workgroups <= 8));
+    return m <= 64 && k <= 1024 && weights < (q6 && m > 48 ? 4 : 5) * million && (k <= 256 || spread || (m <= 48 && n > 4096 && load.workgroups <= 5));
 }
 
 static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
     if (m < 1 || (m == 1 && (encoding == QMM_Q4_K || encoding == QMM_Q4_0) && k <= 14528 && (k > 2048 || n < 8192)) || (m == 1 && encoding == QMM_Q4_K && k > 2048) || !qmm::gemv_kquant_small_supported(encoding, lhs_dtype, m, n, k, w)) return false;
     const bool f32 = lhs_dtype == QMM_F32;
-    if (m > qmm::small_most_rows(lhs_dtype)) return !(encoding == QMM_Q5_K && q5k_mm_forced()) && !(encoding == QMM_Q6_K && q6k_mm_forced()) && small_tiles_wanted(encoding, f32, m, n, k);
+    if (m > qmm::small_most_rows(lhs_dtype)) return !(encoding == QMM_Q5_K && q5k_mm_forced()) && !(encoding == QMM_Q6_K && q6k_mm_forced()) && small_tiles_wanted(encoding, lhs_dtype, m, n, k);
     if (m == 1) {
         if (encoding == QMM_Q4_K) return true;
         if (encoding == QMM_Q5_K) return !q5k_mm_forced() && (k <= 2048 || k > 8192 || n > 2048);
@@ -443,7 +457,7 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
                !((m == 2 && (n <= 1024 || (k <= 4096 && n * k <= ((int64_t)8 << 20)))) || (m <= 4 && n <= 1024 && f32 == (k <= 4096)));
     }
     if (encoding == QMM_Q4_0)
-        return m == 2 ? k > 8192 || ((n > 2048 || k <= 2048) && n * k <= (int64_t)64 << 20) : m <= 8 || k <= 1024 || (n <= 2048 && k <= 2048) || (n <= 1024 && k > 8192);
+        return m == 2 ? k > 8192 || ((n > 2048 || k <= 2048) && n * k <= (int64_t)64 << 20) : m <= 8 || (k <= 1024 && !(k > 512 && n > 11264 && n <= 16384)) || (n <= 2048 && k <= 2048) || (n <= 1024 && k > 8192);
     const bool large = m > 8 && k > 4096;
     if (encoding == QMM_Q5_K) return !q5k_mm_forced() && !(f32 && m == 2 && n <= 1024 && k > 2304 && k <= 4096) && !(large && n * k >= ((int64_t)190 << 20));
     if (f32 && (m == 5 || m == 6) && k <= 512) return false;
@@ -454,8 +468,8 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
 // 4096 x 14336 15.3 / 10.9; four bf16 rows 9.4 / 5.5, 12.4 / 9.0, 15.2 / 11.3; eight fp32 rows 13.6 / 7.7, 18.3 / 12.6, 20.9 / 12.9; 16 bf16 rows 11.1 / 8.9, 14.3 / 13.5, 16.8 / 14.6.  Relative error, K = 4096: 4.2e-7 /
 // 0.8e-7 (fp32 rows), 2.2e-7 and 1.2e-7 / 0.65e-7 (one and four bf16 rows).
 static bool gptq_small_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    return encoding == QMM_GPTQ && cfg && !cfg->desc_act && (m <= qmm::small_most_rows(lhs_dtype) || small_tiles_wanted(encoding, lhs_dtype == QMM_F32, m, n, k)) &&
-           qmm::gemv_gptq_small_supported(lhs_dtype, m, n, k, cfg->group_size);
+    return encoding == QMM_GPTQ && cfg && !cfg->desc_act && qmm::gemv_gptq_small_supported(lhs_dtype, m, n, k, cfg->group_size) &&
+           (m <= qmm::small_most_rows(lhs_dtype) || small_tiles_wanted(encoding, lhs_dtype, m, n, k));
 }
 
 // Does the kernel that serves this problem store bf16 itself?  (The Q4_K decode kernel does; everything else goes

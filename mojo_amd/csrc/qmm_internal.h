@@ -135,6 +135,10 @@ inline int64_t small_most_rows(int lhs_dtype) { return lhs_dtype == QMM_F32 ? 8 
 // gemv_kquant_small.hip: Q4_0, Q4_K, Q5_K, Q6_K with up to four times as many lhs rows.  gated: two matrices of the same size, gate and
 // up, outs[0] = silu(gate) * up.  out_bf16: the outputs are bf16 arrays.  workspace: null, or (not gated) what gemv_kquant_small_workspace_bytes says, with n = the sum of ns; the same sums.
 int64_t gemv_kquant_small_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k);
+struct SmallLoad {
+    int workgroups, wavefronts;  // on the fullest compute unit
+};
+SmallLoad small_load(int lhs_dtype, int64_t m, int64_t n, int64_t k);  // (k at least 256)
 bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w);
 hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs, int64_t m, int64_t k,
                                     bool gated, bool out_bf16, void* workspace, hipStream_t s);

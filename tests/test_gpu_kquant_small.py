@@ -139,6 +139,17 @@ def test_tiles_that_leave_lds_a_few_at_a_time(enc, m, n, k):
     check(enc, qmatmul(QE[enc], None, a, w), w, a)
 
 
+@pytest.mark.parametrize("enc", ("Q4_0", *ENCODINGS))
+@pytest.mark.parametrize("m,n,k", [(48, 2048, 768), (48, 3072, 768), (64, 2560, 1024), (64, 3584, 1024), (40, 4352, 1024), (17, 6144, 1024), (17, 6144, 1280), (32, 8192, 1280), (32, 6144, 1536), (16, 14336, 768)])
+def test_on_both_sides_of_the_lines_for_a_short_k(enc, m, n, k):
+    """Tiles of lhs rows side by side, or the direct GEMM where a compute unit would get too many of them."""
+    w, a = packed(enc, n, k), rows(m, k, torch.bfloat16)
+    if enc == "Q4_0":
+        blocks = quantize(QE.Q8_0, a.float()).view(m, -1, 34)
+        a = (blocks[:, :, :2].contiguous().view(torch.float16).double() * blocks[:, :, 2:].contiguous().view(torch.int8).double()).view(m, k)
+    check(enc, qmatmul(QE[enc], None, rows(m, k, torch.bfloat16), w), w, a)
+
+
 def alone(encoding, config, a, rhs, step):
     """The rows of `a` in calls of `step` rows, the last of which repeats rows of the one before."""
     m, out = a.shape[0], []
