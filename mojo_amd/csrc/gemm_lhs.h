@@ -64,11 +64,9 @@ __device__ __forceinline__ void rescale_add(float16v& acc, float g, const float1
 //   kLhsOrderQ4K : 32*(f/2) + 16*g + 8*(f%2) + (0,2,1,3,4,6,5,7)[slot]
 //   kLhsOrderGPTQ: 16*f + 8*g + (0,4,1,5,2,6,3,7)[slot], odd columns pre-multiplied by 1/16
 //                  (their codes are used in place in the high nibble position, 16*q)
-//   kLhsOrderQ4K16: 8*(pos/8) + (0,2,1,3,4,6,5,7)[slot]   (natural order, the two middle pairs of every 8 swapped:
-//                  the operand order of the 16x16x32 small-batch kernel)
 //   kLhsOrderTile: 32*g + 8*f + (0,2,1,3,4,6,5,7)[slot]   (slice f pairs 8 columns of the low-nibble sub-block
 //                  with the same 8 of the high-nibble one: what one lane of the tile kernels unpacks from 8 code bytes)
-constexpr int kLhsOrderQ4K = 0, kLhsOrderGPTQ = 1, kLhsOrderQ4K16 = 2, kLhsOrderTile = 3;
+constexpr int kLhsOrderQ4K = 0, kLhsOrderGPTQ = 1, kLhsOrderTile = 2;
 
 // One lhs row by one workgroup of 256 threads.
 // With next > 0 the rows of a16 / a16_lo are lda = k + 256 next halfs long and the sub-block sums go behind the row's k
@@ -130,10 +128,6 @@ __device__ __forceinline__ void prep_lhs_row(int row, const AT* __restrict__ a, 
         } else if constexpr (ORDER == kLhsOrderTile) {
             const int gg = kl >> 5, f = (kl >> 3) & 3;
             const int64_t o = (int64_t)row * lda + (i & ~63) + f * 16 + gg * 8 + (kl & 4);
-            *(uint2*)(a16 + o) = make_uint2(pack_half2(h0, h2), pack_half2(h1, h3));
-            if (a16_lo) *(uint2*)(a16_lo + o) = make_uint2(pack_half2(x0 - h0, x2 - h2), pack_half2(x1 - h1, x3 - h3));
-        } else if constexpr (ORDER == kLhsOrderQ4K16) {
-            const int64_t o = (int64_t)row * lda + i;
             *(uint2*)(a16 + o) = make_uint2(pack_half2(h0, h2), pack_half2(h1, h3));
             if (a16_lo) *(uint2*)(a16_lo + o) = make_uint2(pack_half2(x0 - h0, x2 - h2), pack_half2(x1 - h1, x3 - h3));
         } else {

@@ -452,6 +452,8 @@ int64_t gemm_q4_k_workspace_bytes(int lhs_dtype, int64_t m, int64_t n, int64_t k
     return lhs_planes(nullptr, lhs_dtype, m, k).bytes + (ks > 1 ? (int64_t)ks * m * n * 4 : 0);
 }
 
+int64_t gemm_q4_k_lhs_bytes(int lhs_dtype, int64_t m, int64_t k) { return lhs_planes(nullptr, lhs_dtype, m, k).bytes; }
+
 hipError_t launch_gemm_q4_k(const void* lhs, int lhs_dtype, const uint8_t* w, int64_t m, int64_t n, int64_t k,
                                float* out, void* workspace, hipStream_t s) {
     if (gemm_q4_k_tile_wanted(m, n, k)) return launch_gemm_q4_k_tile(lhs, lhs_dtype, w, m, n, k, out, workspace, s);

@@ -5,7 +5,7 @@
 // wavefront owns whole weight rows (persistent: rows gw, gw + GW, ...).  A row travels as aligned
 // 16-byte pieces straight into a wavefront-private ring of LDS slots (global_load_lds_dwordx4, up
 // to three rows ahead of the one being decoded; the loads are hidden from the compiler and waited
-// for with exact vmcnt counts, see gemv_q4k_mm.hip).  Lane l decodes blocks l, l + 64, ... of the
+// for with exact vmcnt counts, see lds_stream.h).  Lane l decodes blocks l, l + 64, ... of the
 // row: five dwords from LDS joined by v_alignbyte_b32, low / high nibbles masked into two int8x4
 // operands per dword, eight v_dot4_i32_i8 per block.
 //

@@ -1,10 +1,7 @@
-// Q4_K small-batch kernel (2..16 lhs rows) for shapes with few weight rows and long K: every wavefront owns one
-// super-block column, K is cut along blockIdx.y.
+// Q4_K small-batch kernel for shapes with few weight rows and long K (up to 4096 rows, 9 .. 16 fp32 lhs rows, 128 Mi weights and more, where the workspace is too small for the
+// direct GEMM): every wavefront owns one super-block column, K is cut along blockIdx.y.
 //
-// The small-batch kernel in gemv_q4k_mm.hip gives a workgroup whole weight rows, so with N = 4096 a workgroup has a
-// single 16-row tile and prepares the whole lhs (K values per lhs row) for it: on 4096 x 14336 that preparation
-// costs as much as the weights.  Here the work is cut the other way, as in the GPTQ small-batch kernel
-// (gemv_gptq_mm.hip): wavefront w of a workgroup owns super-block b = chunk * waves + w of every weight row, keeps the
+// The work is cut as in the GPTQ small-batch kernel (gemv_gptq_mm.hip): wavefront w of a workgroup owns super-block b = chunk * waves + w of every weight row, keeps the
 // lhs operands of those 256 k (16 rows, fp16 main plane and, for an fp32 lhs, a residual plane with accumulators of
 // its own) in registers, and the workgroup walks over strips of 32 weight rows (two matrix-core tiles of 16).  A lane
 // (row c = l % 16, quarter kq = l / 16) loads the 16-byte header of its row's super-block and, for each of the four

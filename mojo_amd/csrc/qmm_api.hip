@@ -61,16 +61,9 @@ bool q5k_mm_forced() {
     return set;
 }
 
-// GPTQ with more than 16 lhs rows: do passes of the small-batch kernel (16 rows each, bound by the bytes of the weights)
-// beat the GEMM (128 x 256 output tiles, one workgroup each, bound by K per round of 256 tiles)?  Times in
-// microseconds as measured on 14336 x 4096, 4096 x 14336 and 4096 x 4096 with 64 to 128 rows: a GEMM round costs
-// 64 us per 4096 of K (bf16 lhs; 2.1 x that for an fp32 lhs, which runs two launches) whatever N is, so few column tiles
-// (N = 4096: 16 of 256 compute units) and long K favour the passes: 4096 x 14336 with 128 bf16 rows 126 against 209 us.
-// Q4_K with 2..16 lhs rows: the kernel that cuts K across workgroups, or the one that gives a workgroup whole rows?
+// Q4_K with few lhs rows that no kernel before takes (9 .. 16 fp32 rows on 128 Mi weights and more with a workspace too small for the direct GEMM): the kernel that cuts K across
+// workgroups, or the prefill kernel?
 bool q4k_kc_wins(int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    // measured, 4096 x 14336, this kernel against the row kernel: 16 rows 29.5 / 49.9 us (fp32 lhs), 22.2 / 35.0 us (bf16);
-    // 8 rows 27.1 / 26.9 us (fp32), 21.1 / 26.4 us (bf16); 4 rows 26.6 / 18.8 us, 20.9 / 18.7 us.  On 14336 x 4096 and on
-    // K = 4096 the row kernel wins at every row count.
     return m >= (lhs_dtype == QMM_F32 ? 9 : 5) && n <= 4096 && k > 4096;
 }
 
@@ -114,6 +107,11 @@ bool q5k_mm_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k) {
            (m >= 2 && ((k > 8192 && n >= 2048) || n * k >= ((int64_t)96 << 20))) || (k > 16384 && n >= 2048);
 }
 
+// GPTQ with more than 16 lhs rows: do passes of the small-batch kernel (16 rows each, bound by the bytes of the weights)
+// beat the GEMM (128 x 256 output tiles, one workgroup each, bound by K per round of 256 tiles)?  Times in
+// microseconds as measured on 14336 x 4096, 4096 x 14336 and 4096 x 4096 with 64 to 128 rows: a GEMM round costs
+// 64 us per 4096 of K (bf16 lhs; 2.1 x that for an fp32 lhs, which runs two launches) whatever N is, so few column tiles
+// (N = 4096: 16 of 256 compute units) and long K favour the passes: 4096 x 14336 with 128 bf16 rows 126 against 209 us.
 bool gptq_small_batch_wins(int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     // Passes of the small-batch kernel (16 rows each) against the GEMM (128 x 256 tiles, cut into K shares when they are few, an
     // fp32 lhs of up to 256 rows as twice the rows), in microseconds as measured on this part: 4096 x 4096, bf16 / fp32 lhs: a
@@ -339,8 +337,8 @@ static int64_t required_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n,
         const int64_t c = qmm::gemm_q4_0_planes_wanted(m, n, k) ? qmm::gemm_q4_0_planes_workspace_bytes(m, n, k) : 0;
         return std::max(std::max(a, b), c);
     }
-    if (encoding == QMM_Q4_K && m <= 16 && k % 256 == 0) {  // lhs planes from 9 rows on; partial sums of K chunks
-        const int64_t a = qmm::gemv_q4_k_mm_workspace_bytes(lhs_dtype, m, k), b = m >= 2 ? qmm::gemv_q4_k_kc_workspace_bytes(m, n, k) : 0;
+    if (encoding == QMM_Q4_K && m <= 16 && k % 256 == 0) {  // partial sums of K chunks; from 9 rows on the lhs planes of the prefill kernel, whether it serves the call or not
+        const int64_t a = m <= 8 ? 0 : qmm::gemm_q4_k_lhs_bytes(lhs_dtype, m, k), b = m >= 2 ? qmm::gemv_q4_k_kc_workspace_bytes(m, n, k) : 0;
         const int64_t c = q4k_gemm_from_9_rows(encoding, lhs_dtype, m, n, k) ? qmm::gemm_q4_k_workspace_bytes(lhs_dtype, m, n, k) : 0;
         return std::max(std::max(a, b), c);
     }
@@ -395,7 +393,7 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 // - Q6_K, five and six fp32 rows, K = 256 or 512: more exact weight by weight (decode_sums_more_exactly), 0.85e-7 against 0.88e-7.
 // More rows than one workgroup takes (fp32: 8, bf16: 16), GPTQ too: two to four workgroups side by side, each of which streams the weights itself, against the lhs prepared by a launch of its own and the direct, shared or older
 // small-batch GEMM.  us, those / here (45 matrices of 128 .. 38000 rows and K of 512 .. 28672, and groups of two to sixteen; weights from memory):
-// - 9 .. 16 fp32 rows: Q4_K 4096 x 4096 11.7 / 9.2, 14336 x 4096 21.7 / 15.5, 4096 x 14336 25.5 / 19.1, 1024 x 14336 23.9 / 11.4, but 8192 x 28672 61 / 100; GPTQ 4096 x 4096 12.0 / 8.9, but 8192 x 8192 21.7 / 28.8;
+// - 9 .. 16 fp32 rows: Q4_K 4096 x 4096 11.7 / 9.2, 14336 x 4096 21.7 / 15.5, 4096 x 14336 25.5 / 19.1, 1024 x 14336 23.9 / 11.4, 65536 x 4096 68 / 60, 262144 x 1024 75 / 63, but 8192 x 28672 61 / 100; GPTQ 4096 x 4096 12.0 / 8.9, but 8192 x 8192 21.7 / 28.8;
 //   Q4_0 5856 x 4096 10.0 / 8.6, 39368 x 512 16.2 / 9.2, but 14336 x 4096 13.5 / 13.7, 3144 x 8192 11.1 / 12.3.
 // - 17 .. 32 fp32 rows: Q4_K 912 x 1024 7.9 / 4.3, 1024 x 14336 24.6 / 13.5; 4096 x 4096 11.9 / 11.4, but 4096, 1024 and 1024 x 4096 in one call 12.9 / 15; GPTQ (never in groups) 4096 x 4096 12.3 / 11.5;
 //   Q4_0 4096, 1024 and 1024 x 4096 15.2 / 11.0.
@@ -431,7 +429,7 @@ static bool small_tiles_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n
         if (k <= 2048 && weights < 3 * million) return m <= 32 || (m <= 64 && load.wavefronts <= 8 && load.workgroups <= (k <= 256 ? 4 : 3));
         return m <= 32 && k <= 4096 && weights >= 18 * million && weights < 110 * million && (weights < 28 * million || weights >= 42 * million);
     }
-    if (f32 && m <= 16) return weights < (k <= 8192 ? 256 : 128) * million;
+    if (f32 && m <= 16) return (encoding == QMM_Q4_K && k <= 4096) || weights < (k <= 8192 ? 256 : 128) * million;
     if (k > 8192) return n <= (f32 ? (m > 32 ? 0 : q6 ? 768 : 1024) : m <= 32 ? (q6 ? 768 : 2048) : m <= 64 ? 512 : 0);
     if (f32) return m <= 32 && k <= 1024 && weights < 5 * million;
     const bool spread = load.wavefronts <= 12 && load.workgroups <= 5;
@@ -823,13 +821,9 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
         if (e != hipSuccess) return hip_status(e, "qmm_matmul(Q4_K small batch, K chunks)");
         if (handled) return QMM_OK;
     }
-    // 9..16 lhs rows: the small-batch matrix-core kernel over a prepared lhs; more: the prefill kernel (which also takes 9..16 fp32 rows on a large
-    // matrix with a long K, where the small-batch kernel works through two planes of a prepared lhs: 28672 x 8192 with 16 rows
-    // 70 us against 61 for 32 rows, 8192 x 28672 94 against 76)
+    // more than 16 lhs rows, and 9..16 fp32 rows on a large matrix with a long K: the prefill kernel
     if (q4k_gemm_from_9_rows(encoding, lhs_dtype, m, n, k))
         return hip_status(qmm::launch_gemm_q4_k(lhs, lhs_dtype, w, m, n, k, out, workspace, s), "qmm_matmul(Q4_K GEMM)");
-    if (encoding == QMM_Q4_K && m >= 9 && m <= 16 && !qmm::kernel_disabled("q4k_mm"))
-        return hip_status(qmm::launch_gemv_q4_k_mm(lhs, lhs_dtype, w, m, n, k, out, workspace, s), "qmm_matmul(Q4_K small batch)");
     if (encoding == QMM_Q4_K && m > 16)
         return hip_status(qmm::launch_gemm_q4_k(lhs, lhs_dtype, w, m, n, k, out, workspace, s), "qmm_matmul(Q4_K GEMM)");
 
@@ -1139,7 +1133,7 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
             return rest == 0 ? QMM_OK
                              : qmm_matmul_grouped(encoding, lhs, lhs_dtype, m, k, rest, rest_w, rest_n, rest_out, workspace, workspace_bytes, stream);
     }
-    if (encoding == QMM_Q4_K && m >= 1 && m <= 16 && k > 0 && k % 256 == 0 && count <= qmm::kLanesMaxMats &&
+    if (encoding == QMM_Q4_K && m >= 1 && m <= 4 && k > 0 && k % 256 == 0 && count <= qmm::kLanesMaxMats &&
         (lhs_dtype == QMM_F32 || lhs_dtype == QMM_BF16) && aligned(lhs, 16)) {
         bool ok = true;
         int64_t total = 0;
@@ -1157,7 +1151,7 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
         }
         if (ok && total <= INT32_MAX && m >= 2 && m <= 4) {
             // Each matrix goes to the kernel qmm_matmul would give it, so a group and separate calls agree bit for bit:
-            // the small ones as one launch of the decode kernel, the others (below) as one of the matrix-core kernel.
+            // the small ones as one launch of the decode kernel, the others (below) one by one.
             const uint8_t* small_w[qmm::kLanesMaxMats];
             int64_t small_n[qmm::kLanesMaxMats];
             float* small_out[qmm::kLanesMaxMats];
@@ -1180,16 +1174,6 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
                     if (!q4k_lanes_rows_wins(n[j], k)) rest_w[rest] = rhs[j], rest_n[rest] = n[j], rest_out[rest++] = out[j];
                 return qmm_matmul_grouped(encoding, lhs, lhs_dtype, m, k, rest, rest_w, rest_n, rest_out, workspace, workspace_bytes, stream);
             }
-        }
-        if (ok && total <= INT32_MAX && m >= 9 && !qmm::kernel_disabled("q4k_mm")) {
-            // the lhs is narrowed once for all the matrices
-            const int64_t need = qmm::gemv_q4_k_mm_workspace_bytes(lhs_dtype, m, k);
-            if (need > 0 && (!workspace || workspace_bytes < need))
-                return fail(QMM_ERR_WORKSPACE, "qmm_matmul_grouped: workspace of %lld bytes required, %lld given", (long long)need,
-                            (long long)workspace_bytes);
-            if (need > 0 && !aligned(workspace, 256)) return fail(QMM_ERR_INVALID, "qmm_matmul_grouped: workspace must be 256-byte aligned");
-            return hip_status(qmm::launch_gemv_q4_k_mm_grouped(lhs, lhs_dtype, count, ws, n, out, m, k, workspace, (hipStream_t)stream),
-                              "qmm_matmul_grouped(Q4_K small batch)");
         }
     }
     for (int j = 0; j < count; j++) {

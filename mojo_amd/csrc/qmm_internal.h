@@ -110,8 +110,6 @@ struct MmMats {
     int n[kLanesMaxMats];
     int count;
 };
-hipError_t launch_gemv_q4_k_mm_grouped(const void* lhs, int lhs_dtype, int count, const uint8_t* const* ws, const int64_t* ns,
-                                       float* const* outs, int64_t m, int64_t k, void* workspace, hipStream_t s);
 hipError_t launch_gemv_q4_k_lanes_grouped(const void* a, int a_dtype, int count, const uint8_t* const* ws, const int64_t* ns,
                                           float* const* outs, int m, int64_t k, int64_t ldo, hipStream_t s, bool* handled,
                                           bool swiglu = false, bool out_bf16 = false);
@@ -198,9 +196,6 @@ bool gemv_q4_k_kc_supported(const void* w, int64_t k);
 int64_t gemv_q4_k_kc_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemv_q4_k_kc(const void* a, int a_dtype, const uint8_t* w, int m, int64_t n, int64_t k, float* out,
                                int64_t ldo, void* workspace, hipStream_t s, bool* handled);
-int64_t gemv_q4_k_mm_workspace_bytes(int lhs_dtype, int64_t m, int64_t k);
-hipError_t launch_gemv_q4_k_mm(const void* lhs, int lhs_dtype, const uint8_t* w, int64_t m, int64_t n, int64_t k,
-                               float* out, void* workspace, hipStream_t s);
 bool gemm_gptq_supported(int64_t k, int group);
 int64_t gemm_gptq_workspace_bytes(int lhs_dtype, int64_t m, int64_t n, int64_t k);
 bool gemm_gptq_twin(int lhs_dtype, int64_t m);  // an fp32 lhs goes through the GEMM as one lhs of twice the rows
@@ -213,6 +208,7 @@ hipError_t launch_gemv_gptq(const void* a, int a_dtype, const uint32_t* qweight,
                             int64_t ldo, hipStream_t s);
 // Prefill-shape kernels (m > 16).
 int64_t gemm_q4_k_workspace_bytes(int lhs_dtype, int64_t m, int64_t n, int64_t k);
+int64_t gemm_q4_k_lhs_bytes(int lhs_dtype, int64_t m, int64_t k);  // of which the lhs
 hipError_t launch_gemm_q4_k(const void* lhs, int lhs_dtype, const uint8_t* w, int64_t m, int64_t n, int64_t k,
                             float* out, void* workspace, hipStream_t s);
 // The kernel that unpacks each weight tile once per workgroup into LDS (256 x 128 output tiles): taken by

@@ -150,6 +150,15 @@ def test_on_both_sides_of_the_lines_for_a_short_k(enc, m, n, k):
     check(enc, qmatmul(QE[enc], None, rows(m, k, torch.bfloat16), w), w, a)
 
 
+@pytest.mark.parametrize("m", [9, 16])
+def test_no_matrix_is_too_large_for_a_short_k(m):
+    """fp32 rows side by side whatever the number of weights, up to K = 4096."""
+    w, a = packed("Q4_K", 65544, 4096), rows(m, 4096, torch.float32)
+    got = qmatmul(QE.Q4_K, None, a, w)
+    for part in (slice(0, 4112), slice(65544 - 4112, 65544)):
+        check("Q4_K", got[:, part], w[part], a)
+
+
 def alone(encoding, config, a, rhs, step):
     """The rows of `a` in calls of `step` rows, the last of which repeats rows of the one before."""
     m, out = a.shape[0], []
