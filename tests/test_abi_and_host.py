@@ -318,3 +318,17 @@ def test_no_tensors_means_none_is_looked_at():
     assert lib.qmm_matmul_repacked(QE.Q5_K.code, None, at, _lib.QMM_BF16, m, k, end, 0, at, packed, n, at, at, need, 0, None) == -1
     assert lib.qmm_matmul(QE.Q5_K.code, None, at, _lib.QMM_BF16, m, k, end, 0, n, at, at, need, _lib.QMM_FLAG_OUT_BF16, None) == -1
     libc.mprotect(base + page, page, 3)
+
+
+def test_every_switch_that_the_fallback_test_throws_exists():
+    """The library ignores names that it does not know: a setting with one would test nothing."""
+    from test_gpu_fallback_kernels import SETTINGS
+
+    text = ""
+    for name in os.listdir(build.CSRC):
+        with open(os.path.join(build.CSRC, name)) as f:
+            text += f.read()
+    switches = {s for line in text.split("\n") if "kernel_disabled(" in line for s in re.findall(r'"(\w+)"', line)}
+    variables = set(re.findall(r'(?:getenv|is_one)\("(\w+)"\)', text))
+    assert {v for setting in SETTINGS for v in setting} <= variables
+    assert {s for setting in SETTINGS for s in setting.get("QMM_DISABLE", "").split(",") if s} <= switches

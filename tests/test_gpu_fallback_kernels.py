@@ -29,8 +29,11 @@ SETTINGS = [
     {"QMM_DISABLE": "planes_wide,planes_quarters"},
     # ... and Q4_K / GPTQ alone kept off the planes
     {"QMM_DISABLE": "q4k_planes,gptq_planes"},
-    # the plain calls of Q4_K decode and small batch through the kernels that take several matrices
-    {"QMM_DISABLE": "q4k_lanes_plain,q4k_mm_plain"},
+    # the plain calls of Q4_K decode through the kernel that takes several matrices
+    {"QMM_DISABLE": "q4k_lanes_plain"},
+    # the kernels that the one for few rows takes calls of the block encodings from, and those behind the direct GEMM then
+    {"QMM_DISABLE": "kquant_small"},
+    {"QMM_DISABLE": "kquant_small,direct"},
     # the small-batch kernels of Q5_K and Q6_K with the rounds of a long K one after the other in each workgroup
     {"QMM_DISABLE": "kquant_mm_rounds_grid"},
     # GPTQ decode on few columns through the kernel with 64 columns per workgroup
