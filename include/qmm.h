@@ -131,8 +131,8 @@ int64_t qmm_matmul_workspace_bytes_flags(int encoding, int lhs_dtype, int64_t m,
 /*
  * The workspace with which a call runs fastest, never less than the figure that the call requires (qmm_matmul_workspace_bytes and its
  * like): from a few lhs rows on, some kernels keep the narrowed lhs there that others do without.  A call given less than this but
- * enough is served by those others, with results of the same precision.  cfg: GPTQ, else null.  A grouped call: the largest QMM_OP_MATMUL
- * figure of its matrices.
+ * enough is served by those others, with results of the same precision.  cfg: GPTQ, else null.  A grouped call:
+ * qmm_matmul_grouped_workspace_bytes.
  */
 enum qmm_op { QMM_OP_MATMUL = 0, QMM_OP_RMSNORM = 1, QMM_OP_SWIGLU = 2, QMM_OP_REPACKED = 3 };
 int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k, int flags);
@@ -195,13 +195,14 @@ int qmm_matmul_static(int encoding, const qmm_gptq_config* cfg, const void* lhs,
  * Several GGUF weight matrices applied to one lhs, as the callers of ops.qmatmul in a transformer
  * block do (q | k | v, and gate | up, take the same activations):
  *   out[j] fp32[m, n[j]] = lhs[m, k] . dequant(rhs[j])^T,  j < count, all rhs of `encoding` and of row length k.
- * Where a kernel takes the whole group (Q4_K, count <= 4: m = 1 with k <= 16384, or 2 <= m <= 16) this is one
- * launch that numbers the rows of the matrices through (the lhs is staged or narrowed once for all of them), as it is for up to four matrices that the GEMM on packed weights
- * (a few to some hundreds of rows) takes with the same cut of k; otherwise it is one qmm_matmul per matrix, in order.  The results are those of separate calls
- * (workspace: the largest any of them needs).  The reference exposes the per-matrix op only; fusing
- * its calls is its graph compiler's job, for which this is the kernel-side counterpart.
+ * Matrices that one kernel takes share a launch that numbers their rows through, up to four of them (the lhs is staged or narrowed once for all): one row of Q4_K with k <= 16384, what the kernel for
+ * few rows serves (the block encodings, k a multiple of 256), and what the GEMM on packed weights takes with the same cut of k (a few to some hundreds of rows); otherwise it is one qmm_matmul per
+ * matrix, in order.  The results are those of separate calls, whatever the workspace: at least the largest any of them needs (qmm_matmul_workspace_bytes);
+ * qmm_matmul_grouped_workspace_bytes also holds what the fastest route wants.
+ * The reference exposes the per-matrix op only; fusing its calls is its graph compiler's job, for which this is the kernel-side counterpart.
  * rhs, n and out are host arrays.
  */
+int64_t qmm_matmul_grouped_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k, int count, const int64_t* n);
 int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, int64_t k, int count,
                        const void* const* rhs, const int64_t* n, float* const* out, void* workspace,
                        int64_t workspace_bytes, void* stream);

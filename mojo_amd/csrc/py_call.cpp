@@ -246,20 +246,19 @@ PyObject* py_grouped(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (mats < 1 || mats > kMost || !weight_encoding(e) || e->code == QMM_GPTQ || !c.open_lhs(a[1])) return none();
     const void* rhs[kMost];
     void* outs[kMost];
-    int64_t n[kMost], need = 0;
+    int64_t n[kMost];
     at::Tensor out[kMost];
     for (Py_ssize_t i = 0; i < mats; i++) {
         const at::Tensor* t = gpu_tensor(PyList_GET_ITEM(a[2], i), c.device);
         if (!packed_matrix(e, t, c.k)) return none();
         rhs[i] = t->data_ptr();
         n[i] = t->size(0);
-        const int64_t one = qmm_preferred_workspace_bytes(QMM_OP_MATMUL, e->code, nullptr, c.dtype, c.m, n[i], c.k, 0);
-        need = c.m <= 64 ? need + one : std::max(need, one);  // (few rows: matrices that share a launch have their parts of K next to each other)
     }
     for (Py_ssize_t i = 0; i < mats; i++) {
         out[i] = c.result(n[i], at::kFloat);
         outs[i] = out[i].data_ptr();
     }
+    const int64_t need = qmm_matmul_grouped_workspace_bytes(e->code, c.dtype, c.m, c.k, (int)mats, n);
     c10::DataPtr ws = c.workspace(need);
     int rc;
     {

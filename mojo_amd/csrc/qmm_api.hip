@@ -1184,6 +1184,21 @@ int qmm_matmul_grouped(int encoding, const void* lhs, int lhs_dtype, int64_t m, 
     return QMM_OK;
 }
 
+// What separate calls need at most, and what matrices that share a launch of the kernel for few rows need for their groups of K next to each other.
+int64_t qmm_matmul_grouped_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k, int count, const int64_t* n) {
+    if (!n || count < 1 || count > 64) return 0;
+    int64_t need = 0, all = 0;
+    int taken = 0;
+    for (int j = 0; j < count; j++) {
+        need = std::max(need, qmm_preferred_workspace_bytes(QMM_OP_MATMUL, encoding, nullptr, lhs_dtype, m, n[j], k, 0));
+        if (m <= 0 || n[j] <= 0 || k <= 0 || !small_wanted(encoding, lhs_dtype, m, n[j], k, nullptr)) continue;  // (the weights' alignment is not known here)
+        all += n[j];
+        need = std::max(need, qmm::gemv_kquant_small_workspace_bytes(encoding, lhs_dtype, m, all, k));
+        if (++taken % qmm::kLanesMaxMats == 0) all = 0;
+    }
+    return need;
+}
+
 int64_t qmm_matmul_swiglu_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     // one lhs row of Q4_K goes through the decode kernel with the combination as its epilogue: nothing to keep
     if (encoding == QMM_Q4_K && m == 1 && k % 256 == 0 && k <= 16384) return 0;

@@ -319,13 +319,12 @@ def qmatmul_grouped(encoding: QuantizationEncoding, lhs: torch.Tensor, rhs: Sequ
     lib = _lib.load()
     lhs_dt = _DTYPES[lhs.dtype]
     outs = [torch.empty((m, w.shape[0]), dtype=torch.float32, device=lhs.device) for w in rhs]
-    needs = [lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, encoding.code, None, lhs_dt, m, w.shape[0], k, 0) for w in rhs]
-    need = sum(needs) if m <= 64 else max(needs)  # (few rows: matrices that share a launch have their parts of K next to each other)
-    ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
     count = len(rhs)
+    n_p = (C.c_int64 * count)(*[w.shape[0] for w in rhs])
+    need = lib.qmm_matmul_grouped_workspace_bytes(encoding.code, lhs_dt, m, k, count, n_p)
+    ws = torch.empty((need,), dtype=torch.uint8, device=lhs.device) if need > 0 else None
     rhs_p = (C.c_void_p * count)(*[w.data_ptr() for w in rhs])
     out_p = (C.c_void_p * count)(*[o.data_ptr() for o in outs])
-    n_p = (C.c_int64 * count)(*[w.shape[0] for w in rhs])
     rc = lib.qmm_matmul_grouped(encoding.code, _ptr(lhs), lhs_dt, m, k, count, rhs_p, n_p, out_p, _ptr(ws), need, _stream(lhs))
     _lib.check(rc, "qmatmul_grouped")
     return [o.reshape(*lead, o.shape[1]) for o in outs]

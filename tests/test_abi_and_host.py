@@ -332,3 +332,19 @@ def test_every_switch_that_the_fallback_test_throws_exists():
     variables = set(re.findall(r'(?:getenv|is_one)\("(\w+)"\)', text))
     assert {v for setting in SETTINGS for v in setting} <= variables
     assert {s for setting in SETTINGS for s in setting.get("QMM_DISABLE", "").split(",") if s} <= switches
+
+
+def test_grouped_workspace_is_not_what_the_matrices_need_one_after_the_other():
+    """Matrices that share a launch for few rows have their groups of K next to each other; whatever else is kept there, the lhs of the direct GEMM for one, is kept once."""
+    lib = _lib.load()
+
+    def figures(enc, m, k, ns):
+        each = [lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, enc.code, None, _lib.QMM_F32, m, n, k, 0) for n in ns]
+        return lib.qmm_matmul_grouped_workspace_bytes(enc.code, _lib.QMM_F32, m, k, len(ns), (C.c_int64 * len(ns))(*ns)), each
+
+    for enc, m, k, ns in [(QE.Q5_K, 32, 4096, [4096] * 16), (QE.Q6_K, 40, 4096, [1024, 4096]), (QE.Q4_0, 300, 2048, [2048] * 3), (QE.Q4_K, 1, 4096, [4096, 1024])]:
+        got, each = figures(enc, m, k, ns)
+        assert got == max(each), (enc, m, k, ns)
+    assert figures(QE.Q4_K, 4, 14336, [1024, 256, 512])[0] == 4 * 4 * 4 * 1792  # four groups, fp32 [4, 1792]
+    assert figures(QE.Q4_K, 4, 14336, [1024] * 9)[0] == 4 * 4 * 4 * 4096  # four matrices a launch
+    assert lib.qmm_matmul_grouped_workspace_bytes(QE.Q4_K.code, 0, 4, 4096, 0, None) == 0
