@@ -5,7 +5,8 @@
 // w + waves g of group g (K = 4096: one group of 16; 14336: four of 14).  It converts the lhs columns of its super-block into matrix-core operands once a
 // group, keeps them in 32 registers, and walks the workgroup's tiles of 16 weight rows with them.  The super-block of a tile's 16 rows (2.3 .. 3.8 KB) goes global -> LDS
 // directly into a private ring of two slots, one item ahead of the one being multiplied: no wavefront waits for another before the end.  Partial results
-// stay in LDS and are added in wavefront order, so they depend on K and the number of lhs rows only, not on N or on timing.
+// stay in LDS and are added in wavefront order, so their order depends on K only, not on N or on timing
+// (the last bits of a row also on the rows beside it, whose values have a part in how it is scaled: small_lhs.h).
 //
 // Why 16 wavefronts with one super-block each (two before, eight wavefronts): an item is a chain LDS reads -> unpacking -> matrix cores of some 150 vector instructions, and with two
 // wavefronts a SIMD most of it was waiting.  Why the rows of the lhs go where they go (row j to operand row 4 j mod 16, fp32 residuals in the rows between): a

@@ -52,8 +52,9 @@ __device__ __forceinline__ uint32_t to_half2_bits(float a, float b) { return __b
 // The order in which four (GPTQ: eight) neighbouring columns lie in a plane: 0,1,2,3; 0,2,1,3; 0,4,1,5,2,6,3,7.
 enum { kSmallOrderPlain = 0, kSmallOrderK = 1, kSmallOrderGptq = 2 };
 
-// The lhs is scaled so that what fp16 leaves out of any value is small against its row's largest: by 2^-33 and below where weights have minima (TOP = 9: a sum of 32 values is an fp16 number too), else 2^-39 (TOP = 14), as
-// in the kernels for more rows.
+// The lhs is scaled so that what fp16 leaves out of any value, up to 2^-25, is small against its row's largest: with a scale of the row's own 2^-34 of it where weights have minima (TOP = 9: a sum of 32 values is an fp16
+// number too), else 2^-39 (TOP = 14), as in the kernels for more rows; with one scale for all rows 2^-31 and 2^-36 of a row's that is only an eighth of the largest.  Which of the two it is depends on all rows of a
+// workgroup, so the last bits of a row are those of a call with the same rows beside it.
 // fp32 rows (hi part and residual): one power of two for all rows, which brings the largest value to [2^TOP, 2^(TOP + 1)), where every row's largest is at least an eighth of it; the result is that scale, or 0: one for each
 // row.  One search over the wavefront for all of them; one for each row always, and the products, took 8 rows 4096 x 4096 from 8.0 to 8.5 (Q4_K) and 7.8 to 9.3 us (GPTQ).
 template <int TOP, typename RAW, int ROWS>

@@ -78,6 +78,9 @@ def test_small_values_next_to_a_few_large_ones(lhs):
     check(config, rhs, qmatmul(QE.GPTQ, config, a.to(lhs), *rhs), a.to(lhs), bits=21)
     a[:, torch.arange(4096, device="cuda") % 1024 != 5] *= 2.0**-4
     check(config, rhs, qmatmul(QE.GPTQ, config, a.to(lhs), *rhs), a.to(lhs), bits=21)
+    # rows up to 7.9 times smaller than the largest, which fp32 rows share one power of two with: 2^-31 (GPTQ 2^-36) of a row's largest left out of each value, 2^-25 of all
+    a *= torch.linspace(1.0, 1.0 / 7.9, a.shape[0], device="cuda")[:, None]
+    check(config, rhs, qmatmul(QE.GPTQ, config, a.to(lhs), *rhs), a.to(lhs), bits=21)
 
 
 @pytest.mark.parametrize("m", [1, 4, 8])
