@@ -133,12 +133,14 @@ __global__ __launch_bounds__(64 * kGsWaves) void gemv_gptq_small_kernel(const ui
     }
     const ks_float4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
+    int held = g_first;  // the group whose lhs operands are in the registers
     for (int c0 = 0; c0 < my_items; c0 += chunk) {
         const int ct = min(chunk, my_items - c0);
         for (int g = g_first; g < g_end; g++) {
             const int part = g * waves + wave;
             if (part < parts) {  // (all wavefronts but for the last group)
-                if (g_end - g_first > 1 && c0 + g > g_first) {  // (a group of its own: the operands of the chunk before)
+                if (g != held) {
+                    held = g;
                     xraw_t xr[MROWS];
 #pragma unroll
                     for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(row0 + j, m - 1) * k + part * 256) + a_lane);

@@ -59,7 +59,7 @@ enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
 // MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up).
 struct SmallCut {
     int per, stride;  // tiles (gated: pairs) of a workgroup at most, workgroups across the tiles
-    uint32_t packed;  // wavefronts; << 8: items (tile, matrix) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups; << 31: several tiles of lhs rows
+    uint32_t packed;  // wavefronts; << 8: items (tile, matrix) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups of a workgroup; << 31: several tiles of lhs rows
 };
 template <int ENC, int MROWS, typename AT, int MODE>
 __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restrict__ a, int m, int k, const SmallCut& cut) {
@@ -83,9 +83,11 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
         // several tiles of lhs rows: those that read the same weights side by side (blockIdx.y) on one XCD (ids congruent mod 8), every XCD the same number of them
         row0 = (int)blockIdx.y * MROWS, share = (int)blockIdx.z * 8 + (int)blockIdx.x, part = apart ? share / stride : 0;
         share -= part * stride;
-        if (share >= stride || (apart && part >= groups)) return;  // (the whole workgroup)
+        if (share >= stride || (apart && part * waves >= nblk)) return;  // (the whole workgroup)
     }
-    const int g_first = apart ? part : 0, g_end = apart ? g_first + 1 : groups;  // (one group per workgroup, or all of them)
+    // One group per workgroup (then groups is 1, and the operands of the first conversion serve every item), or all of them.  (A flag or a comparison of the group's number instead, as `groups > 1` below, took Q6_K 1184 x 1024
+    // with 33 rows from 4.95 to 5.11 us.)
+    const int g_first = apart ? part : 0, g_end = apart ? g_first + 1 : groups;
     const uint32_t row_bytes = (uint32_t)(nblk * I::kBpb);
     uint8_t* const ring = smem + wave * (2 * I::kSlot);
     const uint32_t ring_lds = lds_address(ring);
@@ -253,7 +255,7 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
         for (int g = g_first; g < g_end; g++) {
             const int sb = g * waves + wave;
             if (sb < nblk) {  // (all wavefronts but for the last group)
-            if (g_end - g_first > 1 && c0 + g > g_first) {  // (a group of its own: the operands of the chunk before)
+            if (groups > 1 && c0 + g > g_first) {
                 xraw_t xr[MROWS];
 #pragma unroll
                 for (int j = 0; j < MROWS; j++) xr[j] = *(const xraw_t*)((const uint8_t*)(a + (int64_t)min(row0 + j, m - 1) * k + sb * 256) + a_lane);
@@ -513,7 +515,7 @@ bool small_parts(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
 template <int ENC, int MROWS, typename AT>
 hipError_t run_small(const MmMats& mats, const SmallPlan& p, const AT* a, int m, int k, bool gated, bool out_bf16, hipStream_t s) {
     const dim3 grid = p.row_tiles > 1 ? dim3(8, (unsigned)p.row_tiles, (unsigned)((p.grid * p.parts + 7) / 8)) : dim3((unsigned)p.grid, (unsigned)p.parts), block((unsigned)(64 * p.waves));
-    const SmallCut cut{p.per, p.grid, (uint32_t)p.waves | (uint32_t)p.chunk << 8 | (uint32_t)out_bf16 << 16 | (uint32_t)(p.parts > 1) << 17 | (uint32_t)p.groups << 18 | (uint32_t)(p.row_tiles > 1) << 31};
+    const SmallCut cut{p.per, p.grid, (uint32_t)p.waves | (uint32_t)p.chunk << 8 | (uint32_t)out_bf16 << 16 | (uint32_t)(p.parts > 1) << 17 | (uint32_t)(p.parts > 1 ? 1 : p.groups) << 18 | (uint32_t)(p.row_tiles > 1) << 31};
     hipError_t e;
     if (gated) {
         if ((e = allow_full_lds<gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallGated>>()) != hipSuccess) return e;
