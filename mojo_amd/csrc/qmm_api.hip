@@ -400,42 +400,38 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 // - 17 .. 32 bf16 rows: Q4_K 4096 x 4096 10.5 / 9.8, 14336 x 4096 19.6 / 17.4, 1024 x 14336 19.9 / 11.8, but 32000 x 4096 31 / 34, 8192 x 8192 20.6 / 22, Q5_K 5120 x 5120 17.8 / 15.3, but with two of 1024 x 5120
 //   15.9 / 19.9; Q4_0 600 x 2048 7.9 / 6.9, 21848 x 2560 27 / 20, but 2520 x 2048 20 % longer.
 // - 33 .. 64 bf16 rows: Q4_K 912 x 1024 7.9 / 4.8, 512 x 28672 31 / 15, but two of 1024 x 14336 18.8 / 26; 1520 x 3072 5 % less, 2048 x 5632 12.2 / 13.0; GPTQ 4096 x 4096 12.7 / 11.6.
-// - What was slower than those and goes back to them: 17 .. 24 bf16 rows GPTQ 16384 x 4096 18.4 / 19.2, 4096 x 8192 and 4096 x 11008 about equal; Q6_K 15360 x 4096 26.0 / 27.2, 16384 x 2560 19.9 / 20.5; Q4_0
-//   16384 x 2560 17.1 / 16.7 (8192 x 4096 14.9 / 14.3, but weights in the last-level cache 11.8 / 13.8); 16 rows Q4_0 14336 x 1024 9.2 / 9.8, f32 2560 x 8192 10.8 / 11.1, 11008 x 4096 11.9 / 12.2, 4096 x 14336 equal;
-//   32 fp32 rows Q4_0 3584 x 11008 19.3 / 19.5.
-// - Short K: a workgroup has few wavefronts, and what counts is how many the fullest compute unit gets.  33 .. 64 bf16 rows Q4_0 3072 x 768 with 9 of them 7.4 / 8.4, 1536 x 1536 with 12 7.9 / 9.4, 1280 x 2048
-//   with 16 8.2 / 9.7, but 2560 x 1024 with 8 7.5 / 7.0; Q4_K 3584 x 1024 with 16 7.8 / 8.3, 8192 x 512 with 16 7.9 / 8.8, 4096 x 1024 with 12 7.9 / 7.1; 17 rows 6144 x 1280 with 15 8.8 / 10.4, 16384 x 512 with
-//   16 7.9 / 8.8, 12288 x 512 with 12 in six workgroups 7.8 / 8.0, but 6144 x 1024 with 12 7.8 / 7.1.
-// Weights in the last-level cache, which a program's layers do not stay in: the others read them again at little cost, and where the two are close they win.  17 bf16 rows Q4_K 4096 x 4096 8.9 / 9.5, 14336 x 4096
-// 15.3 / 17.2, Q5_K 4096 x 4096 9.3 / 10.4, Q6_K 11008 x 4096 20.6 / 21.5, Q4_0 14336 x 4096 16.9 / 19.2 (from memory 10.3 / 9.9, 19.4 / 17.5, 11.1 / 10.4, 25.2 / 22.1, 21.1 / 19.4).
+// - Q4_0, 9 .. 16 fp32 rows: the other kernel has a tile of 16 weight rows a compute unit at a time, and is ahead where they fill its rounds: 11008 x 4096 11.9 / 12.8, 4096 x 14336 17.3 / 18.4, but 4560 x 14336 21.1 / 18.0.
+// - Short K: a workgroup has few wavefronts, and what counts is how many the fullest compute unit gets.  Q4_0 33 .. 64 bf16 rows 3072 x 768 with 9 of them 7.4 / 8.4, 2048 x 1536 with 12 8.7 / 9.6, 1280 x 2048 with 16 8.2 / 9.7,
+//   but 1024 x 1536 with 6 8.0 / 6.8; 9 .. 16 bf16 rows 14336 x 1024 with 16 9.2 / 9.8, but 11976 x 1024 with 12 9.7 / 8.6.  Five wavefronts (K = 1280) do not divide among four SIMDs either: 17 .. 32 bf16 rows with three
+//   workgroups of them Q4_K 5688 x 1280 10.1 / 10.5, Q6_K 5096 x 1280 9.9 / 10.7, 12648 x 1280 14.1 / 18.0, but with two Q4_K 7168 x 1280 10.4 / 9.3.
+// - 17 .. 32 bf16 rows Q6_K 14336 x 4096 24.2 / 24.5, 14528 x 4096 26.3 / 28.7, but 11008 x 4096 23.7 / 22.
+// Over 3000 random calls (128 .. 48000 rows, K of 256 .. 28672, 9 .. 64 rows; the other side forced each time): 0.2 % take more than 4 % longer here than there.  Weights in the last-level cache, which a program's layers do not
+// stay in: the others read them again at little cost, and 4 % take more than 4 % longer here, 17 bf16 rows Q4_K 4096 x 4096 8.9 / 9.5, 14336 x 4096 15.3 / 17.2, Q5_K 4096 x 4096 9.3 / 10.4, Q6_K 11008 x 4096 20.6 / 21.5,
+// Q4_0 14336 x 4096 16.9 / 19.2 (from memory 10.3 / 9.9, 19.4 / 17.5, 11.1 / 10.4, 25.2 / 22.1, 21.1 / 19.4).
 // The lines follow K more than the number of weight rows: a call with several matrices sends each where a call of its own would, and two ways for one call cost more than either.
 // (Asked once the kernel is known to take the call.)
 static bool small_tiles_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const int64_t million = (int64_t)1 << 20, weights = n * k;
     const bool f32 = lhs_dtype == QMM_F32, q6 = encoding == QMM_Q6_K;
     const qmm::SmallLoad load = qmm::small_load(lhs_dtype, m, n, k);
+    const bool five = k > 1024 && k <= 1280 && load.wavefronts > 12;
     if (encoding == QMM_GPTQ) {
         if (f32 && m <= 16) return k <= 4096 || weights < (k <= 8192 ? 60 : 80) * million;
-        if (f32) return m <= 32 && weights < (k <= 4096 ? 16 : k <= 8192 ? 24 : 40) * million;
-        if (k <= 2048) return m <= 64 && weights < (m <= 32 ? 16 : 5) * million && load.wavefronts <= 12;
-        if (m <= 24 && k <= 4096 && weights >= 54 * million && weights < 68 * million) return false;
-        if (m <= 32) return weights < (k <= 4096 ? 80 : k <= 8192 ? 28 : 40) * million;
-        return m <= 64 && weights < (k <= 4096 ? 20 : k <= 8192 ? 4 : 16) * million;
+        if (f32) return m <= 32 && weights < (k <= 4096 ? 17 : k <= 8192 ? 24 : 40) * million;
+        if (m <= 32) return weights < (k <= 2048 ? 16 : k <= 4096 ? 80 : k <= 8192 ? 40 : 45) * million;
+        return m <= 64 && weights < (k <= 2048 ? 5 : k <= 4096 ? 20 : k <= 8192 ? 4 : 16) * million;
     }
     if (encoding == QMM_Q4_0) {
-        if (f32 && m <= 16) return weights < (k <= 3072 ? 128 : k <= 4096 ? (m <= 12 ? 50 : 40) : k <= 6144 ? 24 : k <= 8192 ? 18 : k <= 12288 ? 40 : 52) * million;
-        if (f32) return m <= 32 && weights < (k <= 4096 ? 45 : k <= 8192 ? 28 : m <= 24 ? 40 : 34) * million;
+        if (f32 && m <= 16) return weights < (k <= 3072 ? 128 : k <= 4096 ? 40 : k <= 8192 ? 24 : n > 3584 && n <= 4096 ? 30 : 70) * million;
+        if (f32) return m <= 32 && weights < (k <= 4096 ? 45 : k <= 8192 ? 28 : 40) * million;
         if (k > 8192) return n <= (m <= 32 ? 2048 : m <= 64 ? 512 : 0);
         if (k <= 2048 && weights < 3 * million) return m <= 32 || (m <= 64 && load.wavefronts <= 8 && load.workgroups <= (k <= 256 ? 4 : 3));
-        return m <= 32 && k <= 4096 && weights >= 18 * million && weights < 110 * million && (weights < 28 * million || weights >= 42 * million);
+        return m <= 32 && k <= 4096 && !five && weights >= 18 * million && weights < 110 * million;
     }
     if (f32 && m <= 16) return (encoding == QMM_Q4_K && k <= 4096) || weights < (k <= 8192 ? 256 : 128) * million;
     if (k > 8192) return n <= (f32 ? (m > 32 ? 0 : q6 ? 768 : 1024) : m <= 32 ? (q6 ? 768 : 2048) : m <= 64 ? 512 : 0);
-    if (f32) return m <= 32 && k <= 1024 && weights < 5 * million;
-    const bool spread = load.wavefronts <= 12 && load.workgroups <= 5;
-    if (m <= 32 && k > 2048) return k <= 4096 && weights < (!q6 ? 64 : k <= 3072 ? 40 : 50) * million;
-    if (m <= 32) return weights < 16 * million && (k > 1536 || (k > 1280 ? n <= 4096 : k > 256 ? spread : load.workgroups <= 8));
-    return m <= 64 && k <= 1024 && weights < (q6 && m > 48 ? 4 : 5) * million && (k <= 256 || spread || (m <= 48 && n > 4096 && load.workgroups <= 5));
+    if (!f32 && m <= 32) return k <= 4096 && !five && weights < (k <= 2048 ? 16 : q6 && k > 3072 ? 50 : 64) * million;
+    return m <= (f32 ? 32 : 64) && k <= 1024 && weights < 5 * million;
 }
 
 static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, const void* w) {
@@ -455,7 +451,7 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
                !((m == 2 && (n <= 1024 || (k <= 4096 && n * k <= ((int64_t)8 << 20)))) || (m <= 4 && n <= 1024 && f32 == (k <= 4096)));
     }
     if (encoding == QMM_Q4_0)
-        return m == 2 ? k > 8192 || ((n > 2048 || k <= 2048) && n * k <= (int64_t)64 << 20) : m <= 8 || (k <= 1024 && !(k > 512 && n > 11264 && n <= 16384)) || (n <= 2048 && k <= 2048) || (n <= 1024 && k > 8192);
+        return m == 2 ? k > 8192 || ((n > 2048 || k <= 2048) && n * k <= (int64_t)64 << 20) : m <= 8 || (k <= 1024 && !(k > 512 && n > 12288 && n <= 16384)) || (n <= 2048 && k <= 2048) || (n <= 1024 && k > 8192);
     const bool large = m > 8 && k > 4096;
     if (encoding == QMM_Q5_K) return !q5k_mm_forced() && !(f32 && m == 2 && n <= 1024 && k > 2304 && k <= 4096) && !(large && n * k >= ((int64_t)190 << 20));
     if (f32 && (m == 5 || m == 6) && k <= 512) return false;
