@@ -4,7 +4,8 @@
 // of its part in 32 registers and walks the workgroup's tiles of CW output columns with them.  An item, 32 rows of CW words and the scales and zeros over them (2.2 or 4.3 KB), goes
 // global -> LDS directly into a private ring of two slots, one item ahead of the one being multiplied.
 //
-// What bounds it: the way to the first product (launch, lhs from L2 and its conversion, some 4 us with up to four rows, 6 with sixteen), then memory, 4.5 TB/s at 14336 x 4096.  The tensor lies
+// What bounds it: the way to the first product (launch, lhs from L2 and its conversion, some 4 us with up to four rows, 6 with sixteen), then memory, 4.5 TB/s at 14336 x 4096 (vector
+// instructions issued in half of a wavefront's life, waiting 0.43 .. 0.46 of it).  The tensor lies
 // K row by K row, so a tile is 64 or 128 bytes of every row: 32 columns fill the cache lines, 16 leave it to the L2 of the XCD that neighbouring tiles share.  The kernels before had the loads of
 // one group per wavefront in flight, held in registers, and a workgroup per 64 (one row: 16) columns: figures at the dispatch (qmm_api.hip).
 //

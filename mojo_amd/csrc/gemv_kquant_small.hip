@@ -14,7 +14,8 @@
 // what is done to results (scales, sums, LDS) shrinks to a quarter.
 //
 // What bounds it: the way to the first product (launch, lhs from L2, conversion: some 4 us with four rows, 6 with sixteen), then memory (14336 x 4096, 4 bf16 rows: a tile of 16 rows, 37 .. 54 KB
-// a compute unit, every 1.4 / 1.75 / 2.1 us).  us, the kernels before / this one, 14336 x 4096 4 bf16 rows, weights from memory: Q4_K 11.2 / 9.4, Q5_K 17.8 / 10.8, Q6_K 20.3 / 12.6; 16 bf16 rows
+// a compute unit, every 1.4 / 1.75 / 2.1 us).  Counters: vector instructions are issued in 0.57 .. 0.65 of a wavefront's life (403 of them in the 4.7 us of 4096 x 4096 with 4 fp32 rows, most for the lhs, and a SIMD's
+// four wavefronts do it at the same time), 0.40 .. 0.46 of it is spent waiting, matrix cores are busy 0.09 .. 0.16.  us, the kernels before / this one, 14336 x 4096 4 bf16 rows, weights from memory: Q4_K 11.2 / 9.4, Q5_K 17.8 / 10.8, Q6_K 20.3 / 12.6; 16 bf16 rows
 // 18.6 / 12.7, 17.5 / 13.9, 22.6 / 17.5; 4096 x 14336 4 fp32 rows 13.9 / 12.2, 22.7 / 13.9, 23.1 / 15.7; 2048 x 1024 4 bf16 rows 9.2 / 3.9.  Relative error, K = 4096, before / now: fp32 rows Q4_K
 // 4.0e-7 / 1.1e-7, Q5_K 1.7e-7 / 1.2e-7, Q6_K 1.6e-7 / 1.0e-7; bf16 rows 2.5e-7 / 0.8e-7, 1.0e-7 / 0.85e-7, 0.97e-7 / 0.84e-7 (codes around their middle, residuals to nearest, super-blocks added in
 // four chains).

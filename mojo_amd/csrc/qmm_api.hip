@@ -207,7 +207,7 @@ int static_scratch(void** ws) {
 
 extern "C" {
 
-int qmm_version(void) { return 105; }
+int qmm_version(void) { return 106; }
 
 const char* qmm_last_error(void) { return g_err; }
 
@@ -380,6 +380,7 @@ static bool direct_serves(int encoding, const qmm_gptq_config* cfg, int lhs_dtyp
 // us, that other / here (weights from memory), over 42 matrices of 256 .. 128256 rows and K of 512 .. 28672 with 2 .. 16 rows:
 // - Q4_K, two to four rows, few long rows (the decode kernel with a sub-block per lane): 1024 x 4096 2 rows 4.0 / 4.7, 4 fp32 rows 5.2 / 5.5 (bf16 4.95 / 4.97), 2048 x 4096 2 rows 4.9 / 5.1,
 //   1024 x 8192 2 rows 4.9 / 7.1, 4 bf16 rows 6.5 / 7.4 (fp32 10.1 / 7.9); but 1024 x 2048 4 rows 4.9 / 4.3, 1024 x 11008 4 rows 13.7 / 6.9.
+//   Slower here and left so for the relative error: 2 fp32 rows 1024 x 2048 3.44 / 3.75 (2.6e-7 / 1.1e-7), 4 bf16 rows 1024 x 4096 4.8 / 5.2 (2.6e-7 / 0.8e-7), one fp32 row of Q6_K 14336 x 4096 13.5 / 14.1 (3.3e-7 / 1.0e-7).
 // - Q5_K, two fp32 rows on few columns (its decode kernel): 512 x 4096 5.0 / 5.2; 2048 x 4096 5.7 / 5.1.
 // - 9 .. 16 bf16 rows on large matrices with several groups of K, where few results fit LDS next to the ring: Q6_K 28672 x 8192 51 / 66, 4096 x 14336 9 rows 22.2 / 23.3 (16 rows 25.0 / 22.7), Q5_K 8192 x 28672
 //   47 / 51; but Q6_K 8192 x 8192 24 / 21, 5120 x 13824 38 / 24.
@@ -458,8 +459,8 @@ static bool small_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int6
     return !q6k_mm_forced() && !(large && (n * k >= ((int64_t)96 << 20) || (m < 12 && k > 8192 && k % 2048 == 0 && n * k >= ((int64_t)54 << 20))));
 }
 
-// GPTQ with groups in their order, up to 16 lhs rows (fp32: 8).  us, the kernels before (decode, small batch, direct GEMM) / here, weights from memory: one row 4096 x 4096 6.4 / 5.0, 14336 x 4096 9.6 / 8.6,
-// 4096 x 14336 15.3 / 10.9; four bf16 rows 9.4 / 5.5, 12.4 / 9.0, 15.2 / 11.3; eight fp32 rows 13.6 / 7.7, 18.3 / 12.6, 20.9 / 12.9; 16 bf16 rows 11.1 / 8.9, 14.3 / 13.5, 16.8 / 14.6.  Relative error, K = 4096: 4.2e-7 /
+// GPTQ with groups in their order, up to 16 lhs rows (fp32: 8).  us, the kernels before (decode, small batch, direct GEMM) / here, weights from memory: one bf16 row 4096 x 4096 6.5 / 4.9, 14336 x 4096 10.2 / 8.9,
+// 4096 x 14336 15.6 / 11.6, one fp32 row 6.6 / 5.1, 10.4 / 9.4, 15.7 / 11.4 (weights in the last-level cache 4.5 / 4.8, 7.5 / 8.4, 10.3 / 10.8: the decode kernel has less to do before its first product); four bf16 rows 9.4 / 5.5, 12.4 / 9.0, 15.2 / 11.3; eight fp32 rows 13.6 / 7.7, 18.3 / 12.6, 20.9 / 12.9; 16 bf16 rows 11.1 / 8.9, 14.3 / 13.5, 16.8 / 14.6.  Relative error, K = 4096: 4.2e-7 /
 // 0.8e-7 (fp32 rows), 2.2e-7 and 1.2e-7 / 0.65e-7 (one and four bf16 rows).
 static bool gptq_small_wanted(int encoding, const qmm_gptq_config* cfg, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     return encoding == QMM_GPTQ && cfg && !cfg->desc_act && qmm::gemv_gptq_small_supported(lhs_dtype, m, n, k, cfg->group_size) &&

@@ -11,7 +11,7 @@ namespace qmm {
 
 // Kernel families switched off by the environment variable QMM_DISABLE (a comma-separated list of names, read once
 // per process), for tests and triage: a disabled family reports that it does not take a shape, and the next kernel
-// in the dispatch order serves it.  Names: kquant_small, direct, shared, staged, q4k_lanes, q4k_lanes_rows, q4k_stream, q4k_mm, q4k_kc, q4k_tile, q4k_gemm64, q4k_twin_rows, q4k_rows_v2,
+// in the dispatch order serves it.  Names: kquant_small (q4k_mm: for Q4_K alone), direct, shared, staged, q4k_lanes, q4k_lanes_rows, q4k_stream, q4k_kc, q4k_tile, q4k_gemm64, q4k_twin_rows, q4k_rows_v2,
 // q4_0_stream, q4_0_mfma, q4_0_small, q4_0_small_passes, q4_0_wide, q4_0_planes, q6k_lanes, q6k_slab, q6k_staged, kquant_planes, planes_wide, planes_192, planes_quarters, planes_twin_rows, gptq_twin_rows, gptq_k_shares, gptq_long_k_mm, kquant_mm_rounds_grid, q4k_planes, gptq_planes, gptq_small, gptq_mm, gptq_cols, gptq_cols16, gptq_order.
 // Nothing is disabled by default.
 bool kernel_disabled(const char* family);
