@@ -162,9 +162,10 @@ int64_t qmm_preferred_workspace_bytes(int op, int encoding, const qmm_gptq_confi
  *   Bit 2 (QMM_FLAG_OUT_BF16): `out`
  *   points to bf16[m, n] instead of fp32 (the caller's next op takes bf16 activations): the fp32 result is
  *   rounded to nearest even with NaN mapped to the canonical quiet NaN, the reference's narrowing rule
- *   (stdlib/src/builtin/simd.mojo:3279-3300).  The Q4_K decode kernel (m = 1, K <= 16384) stores bf16 itself;
- *   every other problem computes fp32 into the workspace and narrows in a second launch, which takes
- *   qmm_matmul_workspace_bytes_flags bytes of workspace.
+ *   (stdlib/src/builtin/simd.mojo:3279-3300).  The Q4_K decode kernel (m = 1, K <= 16384), the kernels for a few rows and
+ *   the direct, shared and staged GEMMs store bf16 themselves (the latter two kinds with the workspace that
+ *   qmm_preferred_workspace_bytes names); every other problem computes fp32 into the workspace and narrows in a second
+ *   launch, which takes qmm_matmul_workspace_bytes_flags bytes of workspace.
  * rhs is a host array of device pointers.
  */
 #define QMM_FLAG_W_BF16 1

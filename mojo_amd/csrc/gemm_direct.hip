@@ -791,6 +791,7 @@ bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64
     // this kernel has no such preference), and up to where it crosses that of the GEMMs behind it (direct_range).  Both lines were fitted to
     // timings of 4700 calls, 512 x 512 .. 28672 x 4096 with K of 512 .. 14336 and 1 .. 2048 rows: within 2 % on average of always taking
     // the faster of the two.  E.g. 5120 x 5120, 17 bf16 rows: Q4_0 22 -> 16 us, Q4_K 19.6 -> 14.4, Q5_K 34 -> 15.7, Q6_K 54 -> 17.9.
+    // (Up to 16 rows, and up to 64 on many shapes, the kernels for a few rows are asked first: there `from` counts where those decline, K no multiple of 256 and odd numbers of Q6_K blocks among it.)
     const bool f32 = lhs_dtype == QMM_F32, wide = n >= 6000;
     const double w = (double)n * k / (1 << 20);
     int64_t from = 17;
