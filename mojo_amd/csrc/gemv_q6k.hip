@@ -55,16 +55,19 @@ __device__ __forceinline__ float dot4u(float4 x, uint32_t q) {
 }
 // The same dot with the four bytes spread into fp16 lanes first: a byte value q under a zero byte IS the fp16 subnormal
 // q * 2^-24, and v_fma_mix_f32 multiplies it with an fp32 operand exactly: two byte permutes and four mixed fused
-// multiply-adds instead of four conversions and four multiply-adds.  The result is 2^-24 times dot4u's.
+// multiply-adds instead of four conversions and four multiply-adds.  The dot is 2^-24 times dot4u's and added to u (v).
 typedef _Float16 q6_half2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float dot4h(float4 x, uint32_t q) {
-    const q6_half2 p01 = __builtin_bit_cast(q6_half2, __builtin_amdgcn_perm(q, q, 0x0c010c00u));
-    const q6_half2 p23 = __builtin_bit_cast(q6_half2, __builtin_amdgcn_perm(q, q, 0x0c030c02u));
-    float u = fmaf((float)p01.x, x.x, 0.0f);  // (a fused multiply-add with 0: the mixed instruction has no plain multiply)
-    u = fmaf((float)p01.y, x.y, u);
-    u = fmaf((float)p23.x, x.z, u);
-    return fmaf((float)p23.y, x.w, u);
+// Two dots side by side: an instruction that reads what a mixed one just before it wrote costs a wait state.
+__device__ __forceinline__ void dot4h(float4 x, uint32_t q, float4 y, uint32_t r, float& u, float& v) {
+    const q6_half2 p01 = __builtin_bit_cast(q6_half2, __builtin_amdgcn_perm(q, q, 0x0c010c00u)), r01 = __builtin_bit_cast(q6_half2, __builtin_amdgcn_perm(r, r, 0x0c010c00u));
+    const q6_half2 p23 = __builtin_bit_cast(q6_half2, __builtin_amdgcn_perm(q, q, 0x0c030c02u)), r23 = __builtin_bit_cast(q6_half2, __builtin_amdgcn_perm(r, r, 0x0c030c02u));
+    u = fmaf((float)p01.x, x.x, u), v = fmaf((float)r01.x, y.x, v);
+    u = fmaf((float)p01.y, x.y, u), v = fmaf((float)r01.y, y.y, v);
+    u = fmaf((float)p23.x, x.z, u), v = fmaf((float)r23.x, y.z, v);
+    u = fmaf((float)p23.y, x.w, u), v = fmaf((float)r23.y, y.w, v);
 }
+// the low nibbles of `low`, the high ones of `high`, byte by byte
+__device__ __forceinline__ uint32_t q6_join(uint32_t low, uint32_t high) { return (low & 0x0F0F0F0Fu) | (high & 0xF0F0F0F0u); }
 __device__ __forceinline__ float sbyte(uint32_t x, int shift) { return (float)((int)(x << (24 - shift)) >> 24); }
 
 }  // namespace
@@ -363,6 +366,9 @@ static size_t q6k_rows_lds(int mt, int64_t k) {
 // from the compiler, exact vmcnt waits: lds_stream.h); no registers are spent on staging.
 // L: load instructions per row (64 pieces of 16 bytes each): 4 for 16 super-blocks, 2 for 8.
 // MT: lhs rows (1 or 2; the decode of a weight row is shared, the activations of both rows stay in registers).
+// What bounds it: memory, and close behind it the vector units (128256 x 4096, one fp32 row: 250 instructions a row were issued in 0.75 of the cycles of a launch at 5.65 TB/s, 76 us).  214 of
+// them, 73.3 us: the -32 of the codes through the quartets' own sums, which the chains of a dot begin with, instead of a fifth scale for the sum of 16; scales and d read as bytes and
+// halves where they lie; the nibbles and high bits joined by one bit-field insert; row addresses in scalar registers; two dots side by side (no wait states between mixed instructions).
 template <int MT, int L, typename AT>
 __global__ __launch_bounds__(256) void gemv_q6_k_lanes_kernel(const uint8_t* __restrict__ w, const AT* __restrict__ a,
                                                               float* __restrict__ out, int n, int k, int ring_slots,
@@ -389,17 +395,18 @@ __global__ __launch_bounds__(256) void gemv_q6_k_lanes_kernel(const uint8_t* __r
     const int total_waves = (int)gridDim.x * spw, gw = (int)blockIdx.x * spw + wave / wpr;
     const int my_rows = gw < n ? (n - gw + total_waves - 1) / total_waves : 0;
     const int bq = lane >> 4, t = lane & 15, h = t >> 3, j = t & 7;
-    const int sc_shift = 8 * (j >> 2);
 
     // the first rows are requested before the activations, so that their latencies overlap
     // (the mask follows the slot size, the same for every part, so each of the L instructions has a live lane in
     // every wavefront and the wait counts stay exact; a shorter part repeats its last piece)
+    uint32_t off[L];  // the lane's pieces, from the (wave-uniform) first one of a row part on
+#pragma unroll
+    for (int i = 0; i < L; i++) off[i] = 16u * (uint32_t)min(lane + 64 * i, last_piece);
     auto issue = [&](int ri, int slot) {
         const uint8_t* base = w + (int64_t)(gw + (int64_t)ri * total_waves) * row_bytes + (int64_t)blk0 * Q6_K_BPB - lead;
 #pragma unroll
         for (int i = 0; i < L; i++)
-            if (lane + 64 * i < pieces)
-                load16_to_lds_once(base + 16 * min(lane + 64 * i, last_piece), ring_lds + slot * kSlot + i * 1024);
+            if (lane + 64 * i < pieces) load16_to_lds_once(off[i], base, ring_lds + slot * kSlot + i * 1024);
     };
     int issued = 0, islot = 0, cslot = 0;
     for (; issued < min(ring_slots - 1, my_rows); issued++) {
@@ -407,9 +414,9 @@ __global__ __launch_bounds__(256) void gemv_q6_k_lanes_kernel(const uint8_t* __r
         islot = islot + 1 == ring_slots ? 0 : islot + 1;
     }
     // this lane's activations: per super-block slot `it`, four quartets at columns 128 h + 4 j + {0, 32, 64, 96};
-    // and -32 times the sum of one 16-column group per lane (group t of the super-block)
+    // and -32 times the sum of each, in units of 2^-24 like the dots below (-32 * 2^-24 = -2^-19; the row's sum is scaled back at its end)
     float4 x[MT][4][4];
-    float os[MT][4];
+    float os[MT][4][4];
     bool lv[4];  // the lane's super-block `it` exists in this part
     float keep = 0.0f;
 #pragma unroll
@@ -419,39 +426,22 @@ __global__ __launch_bounds__(256) void gemv_q6_k_lanes_kernel(const uint8_t* __r
         const int blc = min(blk0 + bl, nblk - 1);   // of the row
 #pragma unroll
         for (int mi = 0; mi < MT; mi++) {
-            const AT* ar = a + (int64_t)mi * k + blc * 256;
-            const AT* aq = ar + 128 * h + 4 * j;
-            x[mi][it][0] = load4(aq, 0);
-            x[mi][it][1] = load4(aq, 32);
-            x[mi][it][2] = load4(aq, 64);
-            x[mi][it][3] = load4(aq, 96);
-            // The sum of group t = 8 h + j (columns 128 h + 16 j .. + 15) from the quartets already loaded, not from loads of its
-            // own (a wavefront's lhs loads are half of its start-up: 32 KB through the compute unit's load path for 16 KB of
-            // values): those 16 columns are quartet j / 2 of the four lanes 4 (j % 2) .. + 3 of this half row.  Quartet sums,
-            // added over each aligned group of four lanes; the other group of the eight is a mirror away.
-            float qs[4], qo[4];
+            const AT* aq = a + (int64_t)mi * k + blc * 256 + 128 * h + 4 * j;
 #pragma unroll
-            for (int c4 = 0; c4 < 4; c4++) {
-                const float4 q = x[mi][it][c4];
-                qs[c4] = (q.x + q.y) + (q.z + q.w);
-                qs[c4] += dpp_move<0xB1>(qs[c4]);
-                qs[c4] += dpp_move<0x4E>(qs[c4]);
-                qo[c4] = dpp_move<0x141>(qs[c4]);
+            for (int c = 0; c < 4; c++) {
+                const float4 q = load4(aq, 32 * c);
+                x[mi][it][c] = q;
+                os[mi][it][c] = -0x1p-19f * ((q.x + q.y) + (q.z + q.w));
+                keep += os[mi][it][c];
             }
-            const int cj = j >> 1;
-            const float mine = cj == 0 ? qs[0] : cj == 1 ? qs[1] : cj == 2 ? qs[2] : qs[3];
-            const float othr = cj == 0 ? qo[0] : cj == 1 ? qo[1] : cj == 2 ? qo[2] : qo[3];
-            // (in units of 2^-24 like the dots below: -32 * 2^-24 = -2^-19; the row's sum is scaled back at its end)
-            os[mi][it] = -0x1p-19f * ((j & 1) == (j >> 2) ? mine : othr);
-            keep += os[mi][it];
         }
     }
     // (ordinary loads, younger than the rows requested above: the wait for them also covers those rows, and it
     // is forced here, before the loop, so that no wait of the compiler's lands between the counted ones)
     asm volatile("" : "+v"(keep));
 
-    // dword offsets of this lane's fields inside a super-block
-    const int o_ql = 16 * h + j, o_qh = 32 + 8 * h + j, o_sc = 48 + 2 * h;
+    // dword offsets of this lane's fields inside a super-block, and the byte of its first scale: quartet c has scale 8 h + 2 c + j / 4
+    const int o_ql = 16 * h + j, o_qh = 32 + 8 * h + j, o_sc = 192 + 8 * h + (j >> 2);
     for (int ri = 0; ri < my_rows; ri++) {
         if (issued < my_rows) {
             issue(issued, islot);
@@ -473,26 +463,24 @@ __global__ __launch_bounds__(256) void gemv_q6_k_lanes_kernel(const uint8_t* __r
                 return odd ? __builtin_amdgcn_alignbyte(l32[q0 + dw + 1], l32[q0 + dw], 2u) : l32[q0 + dw];
             };
             const uint32_t A = rd(o_ql), B = rd(o_ql + 8), H = rd(o_qh);
-            const uint32_t s0 = rd(o_sc), s1 = rd(o_sc + 1);
-            const uint32_t dv = odd ? l32[q0 + 52] >> 16 : l32[q0 + 52] & 0xffffu;
-            const float d = h2f((uint16_t)dv);
-            const uint32_t q1 = (A & 0x0F0F0F0Fu) | ((H << 4) & 0x30303030u);
-            const uint32_t q2 = (B & 0x0F0F0F0Fu) | ((H << 2) & 0x30303030u);
-            const uint32_t q3 = ((A >> 4) & 0x0F0F0F0Fu) | (H & 0x30303030u);
-            const uint32_t q4 = ((B >> 4) & 0x0F0F0F0Fu) | ((H >> 2) & 0x30303030u);
-            // the int8 scales of the four quartets and of this lane's 16-column group; d once at the end
-            // (one shift per dword, then sign-extending byte selects: a conversion instruction each)
-            const uint32_t t0 = s0 >> sc_shift, t1 = s1 >> sc_shift, tg = (j < 4 ? s0 : s1) >> (8 * (j & 3));
-            const float c1 = (float)(signed char)(t0 & 0xffu), c2 = (float)(signed char)((t0 >> 16) & 0xffu);
-            const float c3 = (float)(signed char)(t1 & 0xffu), c4 = (float)(signed char)((t1 >> 16) & 0xffu);
-            const float cg = (float)(signed char)(tg & 0xffu);
+            const uint8_t* const block = (const uint8_t*)l32 + Q6_K_BPB * it;
+            const float d = h2f(*(const uint16_t*)(block + 208));
+            // (the high pairs of quartets 0 and 2, 1 and 3 with zeros beside them: then one bit-field insert joins them with the nibbles)
+            const uint32_t H02 = H & 0x33333333u, H13 = (H >> 2) & 0x33333333u;
+            float sc[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) sc[c] = (float)((const signed char*)block)[o_sc + 2 * c];
+            const uint32_t q[4] = {q6_join(A, H02 << 4), q6_join(B, H13 << 4), q6_join(A >> 4, H02), q6_join(B >> 4, H13)};
 #pragma unroll
             for (int mi = 0; mi < MT; mi++) {
-                float u = c1 * dot4h(x[mi][it][0], q1);
-                u = fmaf(c2, dot4h(x[mi][it][1], q2), u);
-                u = fmaf(c3, dot4h(x[mi][it][2], q3), u);
-                u = fmaf(c4, dot4h(x[mi][it][3], q4), u);
-                u = fmaf(cg, os[mi][it], u);
+                float dot[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) dot[c] = os[mi][it][c];
+                dot4h(x[mi][it][0], q[0], x[mi][it][1], q[1], dot[0], dot[1]);
+                dot4h(x[mi][it][2], q[2], x[mi][it][3], q[3], dot[2], dot[3]);
+                float u = sc[0] * dot[0];
+#pragma unroll
+                for (int c = 1; c < 4; c++) u = fmaf(sc[c], dot[c], u);
                 v[mi] = lv[it] ? fmaf(d, u, v[mi]) : v[mi];  // (a select: what a missing super-block's lanes read is arbitrary)
             }
         }
@@ -535,9 +523,9 @@ hipError_t launch_gemv_q6_k_rows(const void* a, int a_dtype, const uint8_t* w, i
     const int wpr = nblk <= 16 ? 1 : nblk <= 32 ? 2 : 4;
     const int64_t need_parts = (int64_t)cus * 4 * 8;  // below 8 row parts per wavefront of a one-workgroup-per-CU grid the row-at-a-time kernel is faster
     if (k % 2048 == 0 && nblk <= 64 && !((uintptr_t)w & 15) && n * wpr >= need_parts && !lanes_off) {
-        // Ring slots and workgroups per compute unit, 128256 x 4096 with one lhs row (us): 3 / 3: 77.9, 2 / 3: 77.8, 2 / 4: 76.9,
-        // 3 / 2: 81.9, 4 / 2: 81.5: the wavefronts per SIMD count (the decode of a row is a chain of LDS reads), a second row
-        // in flight does not.
+        // Ring slots and workgroups per compute unit, 128256 x 4096 with one lhs row (us), with 250 vector instructions a row: 3 / 3: 77.9, 2 / 3: 77.8,
+        // 2 / 4: 76.9, 3 / 2: 81.9, 4 / 2: 81.5; with 214: 2 / 4 73.3, 3 / 4 73.9: the wavefronts per SIMD count (the decode of a row is a chain of
+        // LDS reads), a second row in flight does not.
         const int ring = m == 1 ? 2 : 3, pc = m == 1 ? 4 : 3;
         const int bpw = nblk / wpr;                                  // 8 .. 16, even
         const int pieces = (12 + bpw * Q6_K_BPB + 15) / 16;

@@ -56,6 +56,17 @@ __device__ __forceinline__ void load16_to_lds(uint32_t lane_offset, const void* 
                  : "memory");
 }
 
+__device__ __forceinline__ void load16_to_lds_once(uint32_t lane_offset, const void* uniform_base, uint32_t lds_base) {
+    uint32_t keep;
+    const uint64_t b = (uint64_t)(uintptr_t)uniform_base;
+    const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(lane_offset), "s"(sb), "s"(lds_base)
+                 : "memory");
+}
+
 // 4 bytes per lane, to LDS at lds_base + 4 * lane.
 __device__ __forceinline__ void load4_to_lds(const void* g, uint32_t lds_base) {
     uint32_t keep;
