@@ -66,6 +66,13 @@ __device__ __forceinline__ uint32_t pk_add(uint32_t x, uint32_t y) { return as_u
 template <int J>
 __device__ __forceinline__ uint32_t byte_pair(uint32_t top4, uint32_t v) { return __builtin_amdgcn_perm(top4, v, 0x04000400u | (J << 16) | J); }
 
+// A constant in a vector register that the compiler takes for a variable: (x & mask) | top is one instruction then (v_and_or_b32 has room for one scalar operand and no literal; given two
+// constants the compiler makes two instructions of it).  14 -> 10 of them a step for GPTQ, 16 -> 12 for Q4_0.
+__device__ __forceinline__ uint32_t code_top(uint32_t top) {
+    asm("" : "+v"(top));
+    return top;
+}
+
 // A row is scaled by a power of two so that its largest value lies in [2^kRowTop, 2^(kRowTop + 1)), as high as fp16 goes: an fp32 value is then
 // held to 22 bits down to 2^-17 of the row's largest and to 2^-39 of that below (2^-12 and 2^-34 with a top of 9).  Where sums of 32 values
 // are held in fp16 too (Q4_K, Q5_K), 2^9 leaves them room.
@@ -367,6 +374,7 @@ struct GptqWeights : NoOffsets {
     const uint32_t* qzeros;
     int n, group, col, g, rows, groups;
     uint32_t q[16][FN], s_next[kBlocks], z_next[kBlocks], s_raw[kBlocks], z_raw[kBlocks];
+    uint32_t top0 = code_top(0x64006400u), top1 = code_top(0x54005400u);
 
     __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t*) {
         qw = (const uint32_t*)t.w;
@@ -419,8 +427,7 @@ struct GptqWeights : NoOffsets {
         // exact.  (As fp16 subnormals, codes this small lost bits in the matrix-core sums: 3e-5 relative, against 3e-7.)
         const uint32_t m0 = 0xE400E400u | (z * 0x00010001u), m1 = 0xD400D400u | (z * 0x00100010u);
         const uint32_t x = q[T][f], y = x >> 8;
-        b[0] = pack4(pk_add((x & 0x000F000Fu) | 0x64006400u, m0), pk_add((x & 0x00F000F0u) | 0x54005400u, m1),
-                     pk_add((y & 0x000F000Fu) | 0x64006400u, m0), pk_add((y & 0x00F000F0u) | 0x54005400u, m1));
+        b[0] = pack4(pk_add((x & 0x000F000Fu) | top0, m0), pk_add((x & 0x00F000F0u) | top1, m1), pk_add((y & 0x000F000Fu) | top0, m0), pk_add((y & 0x00F000F0u) | top1, m1));
     }
     template <int T>
     __device__ __forceinline__ void after_step(int next_unit) { load_words(next_unit, T); }
@@ -445,6 +452,7 @@ struct Q40Weights : NoOffsets {
     gd_u4 raw[kLoads];
     uint32_t x[FN][2][3];  // block b in x[f][b & 1]: its eight code bytes in dwords 0, 1 (odd b) or from byte 2 of dword 0 on (even b)
     uint32_t d[FN][8];     // (of lanes g = 0; zero in the others)
+    uint32_t top0 = code_top(0x64006400u), top1 = code_top(0x54005400u);
     struct __attribute__((packed, aligned(2))) Bytes16 {
         gd_u4 v;
     };
@@ -510,11 +518,11 @@ struct Q40Weights : NoOffsets {
         for (int i = 0; i < 2; i++) {
             const uint32_t q = blk & 1 ? x[f][1][i] : __builtin_amdgcn_alignbyte(x[f][0][i + 1], x[f][0][i], 2), y = q >> 8;
             if constexpr (a == 0) {
-                v[2 * i] = pk_add((q & 0x000F000Fu) | 0x64006400u, 0xE408E408u);  // 1024 + q - 1032
-                v[2 * i + 1] = pk_add((y & 0x000F000Fu) | 0x64006400u, 0xE408E408u);
+                v[2 * i] = pk_add((q & 0x000F000Fu) | top0, 0xE408E408u);  // 1024 + q - 1032
+                v[2 * i + 1] = pk_add((y & 0x000F000Fu) | top0, 0xE408E408u);
             } else {
-                v[2 * i] = pk_add((q & 0x00F000F0u) | 0x54005400u, 0xD480D480u);  // 64 + q - 72
-                v[2 * i + 1] = pk_add((y & 0x00F000F0u) | 0x54005400u, 0xD480D480u);
+                v[2 * i] = pk_add((q & 0x00F000F0u) | top1, 0xD480D480u);  // 64 + q - 72
+                v[2 * i + 1] = pk_add((y & 0x00F000F0u) | top1, 0xD480D480u);
             }
         }
         b[0] = pack4(v[0], v[1], v[2], v[3]);

@@ -66,6 +66,7 @@ struct StagedGptq : NoOffsets {
     uint32_t head_stride[kHeads];
     int head_block[kHeads];  // its first column of a unit, in 32s
     uint32_t words[2][2];    // of a block of 32 columns
+    uint32_t top0 = code_top(0x64006400u), top1 = code_top(0x54005400u);
     uint32_t s_raw[kBlocks], z_raw[kBlocks];
 
     __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* at) {
@@ -120,8 +121,7 @@ struct StagedGptq : NoOffsets {
         const uint32_t z = ((z_raw[T / FLUSH] >> zshift) & 0xFu) + 1u;
         const uint32_t m0 = 0xE400E400u | (z * 0x00010001u), m1 = 0xD400D400u | (z * 0x00100010u);
         const uint32_t x = words[(T >> 1) & 1][T & 1], y = x >> 8;
-        b[0] = pack4(pk_add((x & 0x000F000Fu) | 0x64006400u, m0), pk_add((x & 0x00F000F0u) | 0x54005400u, m1),
-                     pk_add((y & 0x000F000Fu) | 0x64006400u, m0), pk_add((y & 0x00F000F0u) | 0x54005400u, m1));
+        b[0] = pack4(pk_add((x & 0x000F000Fu) | top0, m0), pk_add((x & 0x00F000F0u) | top1, m1), pk_add((y & 0x000F000Fu) | top0, m0), pk_add((y & 0x00F000F0u) | top1, m1));
     }
     template <int I>
     __device__ __forceinline__ float scale_at() const { return h2f((uint16_t)s_raw[I]); }
