@@ -651,7 +651,7 @@ double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k,
     const int row = staged_row(encoding, group);
     // (Q6_K: the last block would be read two bytes beyond its end where it begins at a multiple of four, which it does if the blocks before it are even in number)
     if (encoding == QMM_Q6_K && (n * direct_units(k)) % 2 != 0) return 1e30;
-    if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
+    if (row < 0 || k % 256 || k >= 1 << 23 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits; three row tiles of 4 GB)
     const int type = lhs_dtype == QMM_F32 ? 1 : 0;
     const StagedCost& c = kStagedCost[row][type];
     const SumsError& e = kSumsError[row][type][centred ? 3 : 2];

@@ -29,19 +29,23 @@ template <int ENC, bool CENTER>
 struct StagedK : KQuantWeights<ENC, 1, CENTER> {
     using Base = KQuantWeights<ENC, 1, CENTER>;
     using Rows = typename Base::Rows;
-    static constexpr int kLoads = Rows::kLoads;
+    static constexpr int kLoads = Rows::kLoads, kWhole = Rows::kTotal / 64;  // instructions, those of all lanes
     uint32_t stage_lds;
     const uint8_t* stage;
     __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* at) {
         Base::init(t, n0, lane, at);
         stage_lds = lds_address(at);
         stage = this->mine;
+#pragma unroll
+        for (int j = 0; j < kWhole; j++) this->rows.off[j] += load_run_offset(j);
     }
     __device__ __forceinline__ void issue(int unit, int buf) {
         const uint8_t* b = this->rows.w + (int64_t)unit * Rows::kRow;
-#pragma unroll
-        for (int j = 0; j < kLoads; j++)
-            if (j * 64 + 63 < Rows::kTotal || j * 64 + this->lane_ < Rows::kTotal) load16_to_lds(this->rows.off[j], b, stage_lds + buf * Base::kStage + j * 1024);
+        const uint32_t to = stage_lds + buf * Base::kStage;
+        load_run_to_lds<kWhole>(this->rows.off, b, to);
+        if constexpr (kWhole < kLoads) {
+            if (kWhole * 64 + this->lane_ < Rows::kTotal) load16_to_lds(this->rows.off[kWhole], b, to + kWhole * 1024);
+        }
     }
     __device__ __forceinline__ void open(int, int buf) {
         this->mine = stage + buf * Base::kStage;
@@ -59,7 +63,7 @@ struct StagedGptq : NoOffsets {
     const uint8_t* qw;
     const uint8_t* stage;
     const uint8_t* cur;
-    uint32_t stage_lds, off;  // off: of the lane's 16 bytes in the first rows of a unit
+    uint32_t stage_lds, off[4];  // off: of the lane's 16 bytes in the rows 8 j .. 8 j + 7 of a unit
     int n, lane_, zshift;
     float per_group;  // 32 / group
     const uint8_t* head[kHeads];
@@ -79,7 +83,8 @@ struct StagedGptq : NoOffsets {
         per_group = 32.0f / (float)t.group;
         // LDS row p holds word row 4 blk + 2 g + a with p = 4 blk + 2 a + g: the two half wavefronts read other banks
         const int p = lane >> 3, row = (p & 4) + 2 * (p & 1) + ((p >> 1) & 1);
-        off = (uint32_t)row * (uint32_t)n * 4u + (uint32_t)min(n0 + 4 * (lane & 7), n - 4) * 4u;
+#pragma unroll
+        for (int j = 0; j < 4; j++) off[j] = (uint32_t)(row + 8 * j) * (uint32_t)n * 4u + (uint32_t)min(n0 + 4 * (lane & 7), n - 4) * 4u + load_run_offset(j);
 #pragma unroll
         for (int j = 0; j < kHeads; j++) {
             const int i = j * 64 + lane, blk = min(i / kHead, kBlocks - 1), part = i % kHead;
@@ -90,8 +95,7 @@ struct StagedGptq : NoOffsets {
     }
     __device__ __forceinline__ void issue(int unit, int buf) {
         const uint32_t to = stage_lds + buf * kStage;
-#pragma unroll
-        for (int j = 0; j < 4; j++) load16_to_lds(off, qw + (int64_t)(32 * unit + 8 * j) * n * 4, to + j * 1024);
+        load_run_to_lds<4>(off, qw + (int64_t)(32 * unit) * n * 4, to);
 #pragma unroll
         for (int j = 0; j < kHeads; j++) {
             // (a group is a whole number of 32s and K below 2^27: half of one keeps the product off the integers by more than its rounding)
@@ -311,18 +315,21 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const DirectMats& 
     w.init(wt, n0, lane, smem + L::kW + wave * 2 * W::kStage);
     const int64_t row_bytes = (int64_t)units * W::kSteps * 1024 * kPer;
     const int last_tile = (m - 1) >> 5;
-    const uint8_t* src[kLoads];
+    // a wavefront loads kLoads neighbouring operands of a chunk (the last ones some that its neighbour loads too); of one row tile, unless kLoads does not divide what a tile has
+    constexpr bool kOneTile = kPieces % kLoads == 0 && kTotal % kLoads == 0;
+    const int piece0 = min(wn * kLoads, kTotal - kLoads);
+    auto tile_of = [&](int piece) __attribute__((always_inline)) { return min(row0 + piece / kPieces, last_tile); };
+    const uint8_t* const src = (const uint8_t*)p.a16 + tile_of(piece0) * row_bytes + ((int64_t)u0 * W::kSteps * kPer + piece0 % kPieces) * 1024;
+    uint32_t from[kOneTile ? 1 : kLoads];
+    from[0] = l16;
+    if constexpr (!kOneTile) {
 #pragma unroll
-    for (int j = 0; j < kLoads; j++) {
-        const int piece = min(wn + WN * j, kTotal - 1);
-        src[j] = (const uint8_t*)p.a16 + min(row0 + piece / kPieces, last_tile) * row_bytes + ((int64_t)u0 * W::kSteps * kPer + piece % kPieces) * 1024;
+        for (int j = 0; j < kLoads; j++)
+            from[j] = l16 + load_run_offset(j) + (uint32_t)max<int64_t>((tile_of(piece0 + j) - tile_of(piece0)) * row_bytes + 1024 * ((piece0 + j) % kPieces - piece0 % kPieces), 0);  // (0: of no row)
     }
     const int last_chunk = (u1 - u0) * kChunks - 1;
     auto issue_lhs = [&](int chunk, int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < kLoads; j++)
-            load16_to_lds(l16, src[j] + (int64_t)min(chunk, last_chunk) * (kPieces * 1024),
-                          (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + (wk * kBufs + buf) * kBuf + min(wn + WN * j, kTotal - 1) * 1024)));
+        load_run_to_lds<kLoads>(from, src + (int64_t)min(chunk, last_chunk) * (kPieces * 1024), lds0 + (wk * kBufs + buf) * kBuf + piece0 * 1024);
     };
     auto issue_weights = [&](int unit, int buf) __attribute__((always_inline)) {
         w.issue(unit, buf);

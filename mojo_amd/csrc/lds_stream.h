@@ -8,6 +8,8 @@
 // both kinds are issued from inline asm here, and the kernel waits itself with s_waitcnt vmcnt(n),
 // n = the number of load instructions it knows to be younger than the data it needs.
 #pragma once
+#include <type_traits>
+
 #include "qmm_internal.h"
 
 namespace qmm {
@@ -65,6 +67,45 @@ __device__ __forceinline__ void load16_to_lds_once(uint32_t lane_offset, const v
                  : "=&s"(keep)
                  : "v"(lane_offset), "s"(sb), "s"(lds_base)
                  : "memory");
+}
+
+// f(integral_constant<int, 0>), f(4), ... below N
+template <int N, int J = 0, typename F>
+__device__ __forceinline__ void unrolled_runs(F&& f) {
+    if constexpr (J < N) {
+        f(std::integral_constant<int, J>{});
+        unrolled_runs<N, J + 4>(f);
+    }
+}
+// N such loads in a row (load j: 1024 j bytes further in LDS), lane offsets from[j] or, with one entry, from[0] + 1024 j.  The offset of an instruction counts for the address
+// as well as for LDS, so four loads share one write of m0; where each has lane offsets of its own, these are 1024 (j % 4) bytes less (load_run_offset), and 4096 more, which `uniform_base`
+// makes up for.
+constexpr uint32_t load_run_offset(int j) { return 4096u - 1024u * (uint32_t)(j & 3); }
+template <int N, int V>
+__device__ __forceinline__ void load_run_to_lds(const uint32_t (&from)[V], const void* uniform_base, uint32_t lds_base) {
+    static_assert(V == 1 || V >= N, "lane offsets");
+    unrolled_runs<N>([&](auto first) __attribute__((always_inline)) {
+        constexpr int J = decltype(first)::value, kRun = N - J < 4 ? N - J : 4;
+        uint32_t keep;
+        const uint64_t b = (uint64_t)(uintptr_t)uniform_base + (V == 1 ? 1024u * J : 0u) - (V == 1 ? 0u : 4096u);
+        const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
+                            (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+        const uint32_t to = lds_base + 1024u * J, f0 = from[V == 1 ? 0 : J], f1 = from[V == 1 || kRun < 2 ? 0 : J + 1], f2 = from[V == 1 || kRun < 3 ? 0 : J + 2],
+                       f3 = from[V == 1 || kRun < 4 ? 0 : J + 3];
+        if constexpr (kRun == 1)
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(f0), "s"(sb), "s"(to) : "memory");
+        else if constexpr (kRun == 2)
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024\n\ts_mov_b32 m0, %0"
+                         : "=&s"(keep) : "v"(f0), "v"(f1), "s"(sb), "s"(to) : "memory");
+        else if constexpr (kRun == 3)
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\tglobal_load_lds_dwordx4 %2, %4 offset:1024\n\t"
+                         "global_load_lds_dwordx4 %3, %4 offset:2048\n\ts_mov_b32 m0, %0"
+                         : "=&s"(keep) : "v"(f0), "v"(f1), "v"(f2), "s"(sb), "s"(to) : "memory");
+        else
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+                         "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072\n\ts_mov_b32 m0, %0"
+                         : "=&s"(keep) : "v"(f0), "v"(f1), "v"(f2), "v"(f3), "s"(sb), "s"(to) : "memory");
+    });
 }
 
 // 4 bytes per lane, to LDS at lds_base + 4 * lane.
