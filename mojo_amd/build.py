@@ -34,13 +34,16 @@ FLAGS = [
 
 
 # Per-file additions.  Kernel-argument preloading (the first dwords of the argument block arrive in scalar registers
-# with the wavefront instead of through a scalar load) for the decode kernels whose first microsecond decides a launch.
+# with the wavefront instead of through a scalar load) for the kernels whose first microsecond decides a launch.
 PER_FILE_FLAGS = {
     "gemv_q4k_lanes.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_kquant_small.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_gptq_small.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
     "gemm_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
+    "gemm_direct.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
+    "gemm_shared.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
+    "gemm_staged.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
 }
 
 

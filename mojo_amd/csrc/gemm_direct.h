@@ -56,6 +56,29 @@ constexpr bool staged_folds(int encoding, int flush, int fm, bool hilo) { return
 
 namespace {
 
+// Where a workgroup of the direct or the shared kernel is: ids congruent mod 8 run on one XCD; there the row tiles of a column tile follow each other, so that its L2 fetches the
+// weights once.  The shape of the grid, 8 x row tiles x (shares of column sections), spares the divisions; where it does not hold them, one number counts through (tiles_m > 0).
+struct DirectGrid {
+    dim3 grid;
+    int tiles_m;
+};
+inline DirectGrid direct_grid(int tiles_m, int places) {
+    if (tiles_m < 65536 && places < 65536) return {dim3(8, (unsigned)tiles_m, (unsigned)places), 0};
+    return {dim3((unsigned)(8 * tiles_m * places)), tiles_m};
+}
+struct DirectPlace {
+    int tile_m, share, section, eighth;
+};
+__device__ __forceinline__ DirectPlace direct_place(int tiles_m, int shares) {
+    int tile_m = (int)blockIdx.y, place = (int)blockIdx.z, eighth = (int)blockIdx.x;
+    if (tiles_m) {
+        const int i = eighth >> 3;
+        eighth &= 7;
+        place = i / tiles_m, tile_m = i - place * tiles_m;
+    }
+    return {tile_m, place & (shares - 1), place >> (shares - 1), eighth};
+}
+
 typedef uint32_t gd_u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t gd_u2 __attribute__((ext_vector_type(2)));
 

@@ -253,28 +253,33 @@ constexpr int direct_slot(int frags) { return W::kStage > frags * 4096 ? W::kSta
 
 }  // namespace
 
-// Workgroup id -> tile: ids congruent mod 8 run on one XCD; there the row tiles of a column tile follow each other, so that its L2 fetches the
-// weights once.  shares: workgroups per tile (1, or 2 that add onto zeros).
+// shares: workgroups per tile (1, or 2 that add onto zeros).  (The first arguments arrive in scalar registers with the workgroup.)
 template <int ENC, int FLUSH, int FM, int FN, int WK, bool HILO>
-__global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
-                                                                int tiles_m, int shares) {
+__global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(const uint8_t* w0, const void* a16, const float* inv_scales, int rows0, int m, int units, int tiles_m, int shares,
+                                                                 int count, WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16) {
     using W = WeightsOf<ENC, FN, FLUSH, true>;
     constexpr int kSlot = direct_slot<W>(FM * FN);
     extern __shared__ __attribute__((aligned(16))) float red[];  // a slot per wavefront: its packed rows, at the end its results [FM * FN][4][64] float4
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int i = (int)(blockIdx.x >> 3), tile_m = i % tiles_m, rest = i / tiles_m, share = rest % shares;
-    int section = rest / shares, first = 0;
-    wt.w = mats.w[0], wt.n = mats.n[0];
+    const DirectPlace at = direct_place(tiles_m, shares);
+    const int tile_m = at.tile_m, share = at.share;
+    int section = at.section, first = 0;
+    wt.w = w0, wt.n = rows0;
+    if constexpr (ENC != QMM_GPTQ && ENC != QMM_Q4_0) wt.k = units * 256;
     float* __restrict__ out = mats.out[0];
+    if (count > 1) {
 #pragma unroll
-    for (int j = 1; j < kDirectMaxMats; j++)
-        if (j < mats.count && section >= mats.end[j - 1]) wt.w = mats.w[j], wt.n = mats.n[j], out = mats.out[j], first = mats.end[j - 1];
-    const int tile_n = (section - first) * 8 + (int)(blockIdx.x & 7);
+        for (int j = 1; j < kDirectMaxMats; j++)
+            if (j < count && section >= mats.end[j - 1]) wt.w = mats.w[j], wt.n = mats.n[j], out = mats.out[j], first = mats.end[j - 1];
+    }
+    const int tile_n = (section - first) * 8 + at.eighth;
     if (tile_n * 32 * FN >= wt.n) return;
     const int n0 = tile_n * 32 * FN, m0 = tile_m * 32 * FM;
     // this wavefront's units of K
-    const int parts = WK * shares, part = share * WK + wave;
-    const int u0 = (int)((unsigned)units * (unsigned)part / (unsigned)parts), u1 = (int)((unsigned)units * (unsigned)(part + 1) / (unsigned)parts);
+    constexpr int kLogWk = WK == 8 ? 3 : 2;
+    static_assert(WK == 1 << kLogWk, "parts of K");
+    const int log_parts = kLogWk + shares - 1, part = share * WK + wave;
+    const int u0 = (int)((unsigned)units * (unsigned)part >> log_parts), u1 = (int)((unsigned)units * (unsigned)(part + 1) >> log_parts);
 
     constexpr int kParts = FM * FN * 4, kMine = (kParts + WK - 1) / WK;  // parts of the tile (four rows per half wavefront), of which this wavefront stores kMine
     float inv[kMine][4];
@@ -283,7 +288,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int part_e = min(e * WK + wave, kParts - 1), row = m0 + 32 * ((part_e >> 2) / FN) + 8 * (part_e & 3) + 4 * (lane >> 5) + r;
-            inv[e][r] = p.inv[min(row, m - 1)];
+            inv[e][r] = inv_scales[min(row, m - 1)];
         }
     constexpr bool kUnit = ENC == QMM_GPTQ && unit_sums(ENC, W::kFlush, HILO);  // (Q4_0 and Q6_K on two fragments have no registers for them)
     float16v T[FM][FN];
@@ -308,7 +313,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_direct_kernel(WeightTensors w
 #pragma unroll
         for (int a = 0; a < FM; a++) {
             const int tile = min(tile_m * FM + a, (m - 1) >> 5);
-            ap[a] = (const uint8_t*)p.a16 + tile * row_bytes + (int64_t)u0 * W::kSteps * 1024 * kPer;
+            ap[a] = (const uint8_t*)a16 + tile * row_bytes + (int64_t)u0 * W::kSteps * 1024 * kPer;
         }
         const uint32_t l16 = lane * 16;
         half8 af[FM][kAhead][kPer];
@@ -760,8 +765,8 @@ hipError_t run_direct(const WeightTensors& wt, DirectMats mats, const DirectSpac
     constexpr int lds = WK * direct_slot<WeightsOf<ENC, FN, FLUSH, true>>(FM * FN);
     hipError_t e = allow_full_lds<gemm_direct_kernel<ENC, FLUSH, FM, FN, WK, HILO>>();
     if (e != hipSuccess) return e;
-    gemm_direct_kernel<ENC, FLUSH, FM, FN, WK, HILO><<<dim3((unsigned)(8 * eights * tiles_m * shares)), dim3(64 * WK), lds, s>>>(wt, mats, p, out16, (int)m,
-                                                                                                                              units, tiles_m, shares);
+    const DirectGrid g = direct_grid(tiles_m, eights * shares);
+    gemm_direct_kernel<ENC, FLUSH, FM, FN, WK, HILO><<<g.grid, dim3(64 * WK), lds, s>>>(mats.w[0], p.a16, p.inv, mats.n[0], (int)m, units, g.tiles_m, shares, mats.count, wt, mats, p, out16);
     return hipGetLastError();
 }
 

@@ -19,10 +19,10 @@ namespace {
 constexpr int kLhsBuffers = 2;
 constexpr int64_t kFewSharedRows = 64;  // up to which Q5_K and Q6_K take their most exact sums (KQuantWeights, Q6Weights)
 
-// Workgroup id -> tile as in gemm_direct_kernel, with column tiles of 32 WN.
+// Column tiles of 32 WN.  (The first arguments arrive in scalar registers with the workgroup.)
 template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER>
-__global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units,
-                                                            int tiles_m, int shares) {
+__global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(const uint8_t* w0, const void* a16, int rows0, int m, int units, int tiles_m, int shares, int count,
+                                                                      WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16) {
     using W = WeightsOf<ENC, 1, FLUSH, CENTER>;
     constexpr int kPer = HILO ? 2 : 1, kChunk = 8 / kPer, kChunks = W::kSteps / kChunk;
     constexpr int kBuf = FM * kChunk * kPer * 1024, kLoads = FM * kChunk * kPer / WN;
@@ -30,20 +30,24 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];  // [WK][kLhsBuffers][kBuf] lhs, [WN WK] packed rows, the inverse row scales
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wn = wave % WN, wk = wave / WN;
     float* const inv = (float*)(smem + WK * kLhsBuffers * kBuf + WN * WK * W::kStage);
-    const int i = (int)(blockIdx.x >> 3), tile_m = i % tiles_m, rest = i / tiles_m, share = rest % shares;
-    int section = rest / shares, first = 0;
-    wt.w = mats.w[0], wt.n = mats.n[0];
+    const DirectPlace at = direct_place(tiles_m, shares);
+    const int tile_m = at.tile_m, share = at.share;
+    int section = at.section, first = 0;
+    wt.w = w0, wt.n = rows0;
+    if constexpr (ENC != QMM_GPTQ && ENC != QMM_Q4_0) wt.k = units * 256;
     float* __restrict__ out = mats.out[0];
+    if (count > 1) {
 #pragma unroll
-    for (int j = 1; j < kDirectMaxMats; j++)
-        if (j < mats.count && section >= mats.end[j - 1]) wt.w = mats.w[j], wt.n = mats.n[j], out = mats.out[j], first = mats.end[j - 1];
-    const int tile_n = (section - first) * 8 + (int)(blockIdx.x & 7);
+        for (int j = 1; j < kDirectMaxMats; j++)
+            if (j < count && section >= mats.end[j - 1]) wt.w = mats.w[j], wt.n = mats.n[j], out = mats.out[j], first = mats.end[j - 1];
+    }
+    const int tile_n = (section - first) * 8 + at.eighth;
     if (tile_n * 32 * WN >= wt.n) return;
     const int n0 = tile_n * 32 * WN + 32 * wn, m0 = tile_m * 32 * FM;
     // this wavefront's units of K; the workgroup's barriers are those of its longest part
-    const int parts = WK * shares, part = share * WK + wk, walk = (units + parts - 1) / parts;
-    const int u0 = (int)((unsigned)units * (unsigned)part / (unsigned)parts), u1 = (int)((unsigned)units * (unsigned)(part + 1) / (unsigned)parts);
-    if (threadIdx.x < 32 * FM) inv[threadIdx.x] = p.inv[min(m0 + (int)threadIdx.x, m - 1)];
+    constexpr int kLogWk = WK == 2 ? 1 : 0;
+    const int log_parts = kLogWk + shares - 1, part = share * WK + wk, walk = (units + (1 << log_parts) - 1) >> log_parts;
+    const int u0 = (int)((unsigned)units * (unsigned)part >> log_parts), u1 = (int)((unsigned)units * (unsigned)(part + 1) >> log_parts);
 
     constexpr bool kUnit = unit_sums(ENC, W::kFlush, HILO);
     float16v T[FM];
@@ -66,7 +70,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
 #pragma unroll
     for (int j = 0; j < kLoads; j++) {
         const int piece = wn + WN * j;
-        src[j] = (const uint8_t*)p.a16 + min(tile_m * FM + piece / (kChunk * kPer), last_tile) * row_bytes +
+        src[j] = (const uint8_t*)a16 + min(tile_m * FM + piece / (kChunk * kPer), last_tile) * row_bytes +
                  ((int64_t)u0 * W::kSteps * kPer + piece % (kChunk * kPer)) * 1024;
     }
     // chunk c is computed on while c + 1 goes from registers to LDS and c + 2 is on its way
@@ -94,6 +98,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
         store_lhs(0);
         load_lhs(1);
     }
+    if (threadIdx.x < 32 * FM) inv[threadIdx.x] = p.inv[min(m0 + (int)threadIdx.x, m - 1)];
     for (int it = 0; it < walk; it++) {
         const int u = u0 + it;
         if (u >= u1) {  // (a shorter part)
@@ -221,26 +226,26 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_shared_kernel(WeightTens
     }
     const int col = n0 + (lane & 31), g = lane >> 5;
     if (col >= wt.n) return;
+    // (the kind of result chosen once, not at each value)
+    auto each = [&](auto&& store) __attribute__((always_inline)) {
 #pragma unroll
-    for (int a = 0; a < FM; a++) {
-        if (WK == 2 && a / kOwn != wk) continue;
+        for (int a = 0; a < FM; a++) {
+            if (WK == 2 && a / kOwn != wk) continue;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float4 s = *(const float4*)(inv + 32 * a + 8 * j + 4 * g);
-            const float sv[4] = {s.x, s.y, s.z, s.w};
+            for (int j = 0; j < 4; j++) {
+                const float4 s = *(const float4*)(inv + 32 * a + 8 * j + 4 * g);
+                const float sv[4] = {s.x, s.y, s.z, s.w};
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = m0 + 32 * a + 8 * j + 4 * g + r;
-                if (row < m) {
-                    const float x = T[a][4 * j + r] * sv[r];
-                    const int64_t at = (int64_t)row * wt.n + col;
-                    if (shares > 1) unsafeAtomicAdd(out + at, x);
-                    else if (out16) out16[at] = f2bf(x);
-                    else out[at] = x;
+                for (int r = 0; r < 4; r++) {
+                    const int row = m0 + 32 * a + 8 * j + 4 * g + r;
+                    if (row < m) store((int64_t)row * wt.n + col, T[a][4 * j + r] * sv[r]);
                 }
             }
         }
-    }
+    };
+    if (shares > 1) each([&](int64_t at, float x) __attribute__((always_inline)) { unsafeAtomicAdd(out + at, x); });
+    else if (out16) each([&](int64_t at, float x) __attribute__((always_inline)) { out16[at] = f2bf(x); });
+    else each([&](int64_t at, float x) __attribute__((always_inline)) { out[at] = x; });
 }
 
 template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER>
@@ -255,8 +260,8 @@ hipError_t run_shared(const WeightTensors& wt, DirectMats mats, const DirectSpac
     for (int j = 0; j < mats.count; j++) mats.end[j] = eights += (mats.n[j] + 256 * WN - 1) / (256 * WN);
     hipError_t e = allow_full_lds<gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER>>();
     if (e != hipSuccess) return e;
-    gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER><<<dim3((unsigned)(8 * eights * tiles_m * shares)), dim3(64 * WN * WK), lds, s>>>(wt, mats, p, out16, (int)m, units,
-                                                                                                                       tiles_m, shares);
+    const DirectGrid g = direct_grid(tiles_m, eights * shares);
+    gemm_shared_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER><<<g.grid, dim3(64 * WN * WK), lds, s>>>(mats.w[0], p.a16, mats.n[0], (int)m, units, g.tiles_m, shares, mats.count, wt, mats, p, out16);
     return hipGetLastError();
 }
 

@@ -266,9 +266,16 @@ struct StagedGrid {
     int full, sections, shares;
 };
 
-// row0: the first 32 rows of the tile, in 32s; place: which share of which column section
+// What arrives in scalar registers with a workgroup (the rest of the arguments is asked for when it runs).
+struct StagedStart {
+    const void *a16, *sums;
+    int m, units, count;  // count: of the matrices
+};
+
+// wt: of the first matrix; row0: the first 32 rows of the tile, in 32s; place: which share of which column section
 template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER, bool FOLD>
-__device__ __forceinline__ void staged_tile(WeightTensors wt, const DirectMats& mats, const DirectSpace& p, uint16_t* __restrict__ out16, int m, int units, int shares, int row0, int place) {
+__device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart& start, const DirectMats& mats, const DirectSpace& p, uint16_t* __restrict__ out16, int shares, int row0, int place) {
+    const int m = start.m, units = start.units;
     using W = StagedOf<ENC, FLUSH, CENTER>;
     using L = StagedLds<ENC, FLUSH, FM, WN, WK, HILO, CENTER>;
     // a chunk of the lhs: kCS steps, kPieces operands of 1 KB (fp32 rows: hi and residual) for each row tile
@@ -280,11 +287,12 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const DirectMats& 
     float* const inv = (float*)(smem + L::kInv);
     const int share = place & (shares - 1);
     int section = place >> (shares - 1), first = 0;
-    wt.w = mats.w[0], wt.n = mats.n[0];
     float* __restrict__ out = mats.out[0];
+    if (start.count > 1) {
 #pragma unroll
-    for (int j = 1; j < kDirectMaxMats; j++)
-        if (j < mats.count && section >= mats.end[j - 1]) wt.w = mats.w[j], wt.n = mats.n[j], out = mats.out[j], first = mats.end[j - 1];
+        for (int j = 1; j < kDirectMaxMats; j++)
+            if (j < start.count && section >= mats.end[j - 1]) wt.w = mats.w[j], wt.n = mats.n[j], out = mats.out[j], first = mats.end[j - 1];
+    }
     const int tile_n = (section - first) * 8 + (int)blockIdx.x;
     if (tile_n * 32 * WN >= wt.n) return;
     const int n0 = tile_n * 32 * WN + 32 * wn, m0 = row0 * 32;
@@ -319,7 +327,7 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const DirectMats& 
     constexpr bool kOneTile = kPieces % kLoads == 0 && kTotal % kLoads == 0;
     const int piece0 = min(wn * kLoads, kTotal - kLoads);
     auto tile_of = [&](int piece) __attribute__((always_inline)) { return min(row0 + piece / kPieces, last_tile); };
-    const uint8_t* const src = (const uint8_t*)p.a16 + tile_of(piece0) * row_bytes + ((int64_t)u0 * W::kSteps * kPer + piece0 % kPieces) * 1024;
+    const uint8_t* const src = (const uint8_t*)start.a16 + tile_of(piece0) * row_bytes + ((int64_t)u0 * W::kSteps * kPer + piece0 % kPieces) * 1024;
     uint32_t from[kOneTile ? 1 : kLoads];
     from[0] = l16;
     if constexpr (!kOneTile) {
@@ -336,7 +344,7 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const DirectMats& 
 #pragma unroll
         for (int j = 0; j < kSums; j++) {
             const int a = (wn + WN * j) % FM;
-            load16_to_lds(l16, (const uint8_t*)p.sums + ((int64_t)min(row0 + a, last_tile) * units + unit) * 1024,
+            load16_to_lds(l16, (const uint8_t*)start.sums + ((int64_t)min(row0 + a, last_tile) * units + unit) * 1024,
                           (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + L::kS + ((wk * 2 + buf) * FM + a) * 1024)));
         }
     };
@@ -486,18 +494,23 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const DirectMats& 
 // 14336 x 4096 400 bf16 rows (4 x 56 tiles of 96 rows and 56 of 16 on 256 compute units) 95 / 86, Q4_K 4096 x 14336 400 rows 80 / 73, 14336 x 4096 400 fp32 rows 129 / 105, Q5_K 11008 x 4096 260
 // rows 51 / 48, Q6_K 8192 x 8192 400 rows 127 / 114.  Over 1280 problems of 70 .. 1000 rows 0.976 of the time (geometric mean), none more than 4 % slower.
 template <int ENC, int FLUSH, int FM, int WN, int WK, bool HILO, bool CENTER, bool FOLD>
-__global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16, int m, int units, StagedGrid grid) {
+__global__ __launch_bounds__(64 * WN * WK, 2) void gemm_staged_kernel(const uint8_t* w0, const void* a16, const void* sums, int rows0, int m, int units, int full, int sections, int shares, int count,
+                                                                 WeightTensors wt, DirectMats mats, DirectSpace p, uint16_t* __restrict__ out16) {
+    // (the first arguments arrive in scalar registers with the workgroup)
+    const StagedGrid grid{full, sections, shares};
+    const StagedStart start{a16, sums, m, units, count};
+    wt.w = w0, wt.n = rows0, wt.k = units * 256;
     // (the shape of the grid spares the divisions)
     int row_tile = (int)blockIdx.y, place = (int)blockIdx.z;
     if (place < grid.sections) {
         // The last row tile without 32 rows that it has not: 200 rows as 128 + 96.  The same rounds of workgroups, but products of rows that nobody asked for heat the part as others do, and its clock is what
         // the power leaves (1.7 GHz here): 14336 x 4096 200 bf16 rows 43.9 -> 41.0 us.
         if constexpr (FM > 2)
-            if (row_tile == grid.full - 1 && m <= (grid.full * FM - 1) * 32) return staged_tile<ENC, FLUSH, FM - 1, WN, WK, HILO, CENTER, FOLD>(wt, mats, p, out16, m, units, grid.shares, row_tile * FM, place);
-        staged_tile<ENC, FLUSH, FM, WN, WK, HILO, CENTER, FOLD>(wt, mats, p, out16, m, units, grid.shares, row_tile * FM, place);
+            if (row_tile == grid.full - 1 && m <= (grid.full * FM - 1) * 32) return staged_tile<ENC, FLUSH, FM - 1, WN, WK, HILO, CENTER, FOLD>(wt, start, mats, p, out16, grid.shares, row_tile * FM, place);
+        staged_tile<ENC, FLUSH, FM, WN, WK, HILO, CENTER, FOLD>(wt, start, mats, p, out16, grid.shares, row_tile * FM, place);
     } else {
         place = (place - grid.sections) * grid.full + row_tile;
-        if (place < grid.sections) staged_tile<ENC, FLUSH, 1, WN, WK, HILO, CENTER, FOLD>(wt, mats, p, out16, m, units, grid.shares, grid.full * FM, place);
+        if (place < grid.sections) staged_tile<ENC, FLUSH, 1, WN, WK, HILO, CENTER, FOLD>(wt, start, mats, p, out16, grid.shares, grid.full * FM, place);
     }
 }
 
@@ -514,8 +527,8 @@ hipError_t run_staged(const WeightTensors& wt, DirectMats mats, const DirectSpac
     if (e != hipSuccess) return e;
     const bool short_last = staged_short_last(FM, m, (int64_t)eights * shares);
     const int full = (int)(short_last ? m / (32 * FM) : (m + 32 * FM - 1) / (32 * FM)), sections = eights * shares, more = short_last ? (sections + full - 1) / full : 0;
-    gemm_staged_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER, FOLD><<<dim3(8, (unsigned)full, (unsigned)(sections + more)), dim3(64 * WN * WK), lds, s>>>(wt, mats, p, out16, (int)m, units,
-                                                                                                                                        StagedGrid{full, sections, shares});
+    gemm_staged_kernel<ENC, FLUSH, FM, WN, WK, HILO, CENTER, FOLD><<<dim3(8, (unsigned)full, (unsigned)(sections + more)), dim3(64 * WN * WK), lds, s>>>(
+        mats.w[0], p.a16, p.sums, mats.n[0], (int)m, units, full, sections, shares, mats.count, wt, mats, p, out16);
     return hipGetLastError();
 }
 
