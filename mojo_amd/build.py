@@ -39,7 +39,7 @@ PER_FILE_FLAGS = {
     "gemv_q4k_lanes.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_kquant_small.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
     "gemv_gptq_small.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
-    "gemm_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
+    "gemm_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
     "gemv_q4_0.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
     "gemm_direct.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
     "gemm_shared.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],

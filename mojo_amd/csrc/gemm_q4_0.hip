@@ -66,36 +66,54 @@ inline LhsQ8T lhs_q8t(void* ws, int64_t m, int64_t k) {
 
 }  // namespace
 
-// One 32-lane group per (padded lhs row, block); same rounding rule as the Q8_0 quantiser:
+// Eight lanes per (padded lhs row, block), four values each; same rounding rule as the Q8_0 quantiser:
 // d = amax / 127 stored as fp16, codes = round-half-away(x / d) with the fp32 d.
 // WORDS: the K order of gemm_q4_0_small_kernel inside a block: k-group g holds the elements whose weight nibbles share
 // dword g of the block's 16 code bytes (4 g .. 4 g + 3, then 16 + 4 g .. 16 + 4 g + 3) instead of 8 g .. 8 g + 7.
+// What bounds it is its chain of latencies (16 x 4096: 0.3 MB).  With a lane per value it had five exchanges between lanes for the maximum and five for the sum through LDS, a 64-bit division for
+// the row and stores of single bytes.  us, that way / this way, whole calls (with the tiles of a workgroup of the GEMM counted by the host): 4096 x 4096 16 bf16 rows 9.8 / 8.75, 14336 x 4096 16 fp32
+// rows 12.8 / 12.6, 5120 x 5152 20 rows 17.8 / 16.7, 512 x 352 70 rows 9.0 / 7.85.
+// Grid: blocks of a row (32 a workgroup), rows, rows / kQuantizeRows.
+constexpr int kQuantizeRows = 32768;
 template <typename InT, bool WORDS>
-__global__ __launch_bounds__(256) void quantize_q8_0_operand_kernel(const InT* __restrict__ x, int m, int k, int64_t ngroups,
-                                                                    int8_t* __restrict__ codes, float* __restrict__ dscale,
-                                                                    int32_t* __restrict__ csum) {
-    const int64_t grp = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 5;
-    const int l = threadIdx.x & 31;
-    if (grp >= ngroups) return;
-    const int nkb = k >> 5;
-    const int64_t row = grp / nkb;
-    const int kb = (int)(grp - row * nkb);
-    const float v = row < m ? load_f32(x, row * (int64_t)k + kb * 32 + l) : 0.0f;
-    float amax = fabsf(v);
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 32));
+__global__ __launch_bounds__(256) void quantize_q8_0_operand_kernel(const InT* __restrict__ x, int m, int nkb, int8_t* __restrict__ codes,
+                                                                    float* __restrict__ dscale, int32_t* __restrict__ csum) {
+    const int row = (int)blockIdx.z * kQuantizeRows + (int)blockIdx.y;
+    const int kb = (int)blockIdx.x * 32 + (int)(threadIdx.x >> 3), i = threadIdx.x & 7;
+    if (kb >= nkb || row >= (m + 15) / 16 * 16) return;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (row < m) {
+        const InT* const at = x + (int64_t)row * nkb * 32 + kb * 32 + 4 * i;
+        if constexpr (sizeof(InT) == 4) {
+            const float4 f = *(const float4*)at;
+            v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
+        } else {
+            const uint2 h = *(const uint2*)at;
+            v[0] = __uint_as_float(h.x << 16), v[1] = __uint_as_float(h.x & 0xffff0000u), v[2] = __uint_as_float(h.y << 16), v[3] = __uint_as_float(h.y & 0xffff0000u);
+        }
+    }
+    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    amax = fmaxf(amax, dpp_move<0xB1>(amax));
+    amax = fmaxf(amax, dpp_move<0x4E>(amax));
+    amax = fmaxf(amax, dpp_move<0x141>(amax));
     uint16_t dh;
     const float id = q8_0_block_rule(amax, dh);
-    const int q = q8_0_code(v, id);
-    int sum = q;
+    uint32_t word = 0;
+    int sum = 0;
 #pragma unroll
-    for (int off = 16; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 32);
-    const int64_t tile = row >> 4;
-    const int mm = (int)(row & 15);
-    const int g = WORDS ? (l & 15) >> 2 : l >> 3, pos = WORDS ? (l & 3) + 4 * (l >> 4) : l & 7;
-    const int64_t tb = tile * nkb + kb;
-    codes[(tb * 64 + g * 16 + mm) * 8 + pos] = (int8_t)q;
-    if (l == 0) {
+    for (int c = 0; c < 4; c++) {
+        const int q = q8_0_code(v[c], id);
+        sum += q;
+        word |= ((uint32_t)q & 0xffu) << (8 * c);
+    }
+    auto over = [&](auto control) __attribute__((always_inline)) { sum += __builtin_amdgcn_update_dpp(0, sum, decltype(control)::value, 0xf, 0xf, true); };
+    over(std::integral_constant<int, 0xB1>{});
+    over(std::integral_constant<int, 0x4E>{});
+    over(std::integral_constant<int, 0x141>{});
+    const int mm = row & 15, g = WORDS ? i & 3 : i >> 1, half = WORDS ? i >> 2 : i & 1;
+    const int64_t tb = (int64_t)(row >> 4) * nkb + kb;
+    *(uint32_t*)(codes + (tb * 64 + g * 16 + mm) * 8 + 4 * half) = word;
+    if (i == 0) {
         if (WORDS) {
             // one 64-byte record per block: 16 scales as fp16, then 16 times -8 * code sum as int16 (|sum| <= 32 * 127)
             uint16_t* rec = (uint16_t*)dscale + tb * 32;
@@ -286,7 +304,8 @@ __device__ __forceinline__ void q40_wait(int items) {
 __global__ __launch_bounds__(64 * kSWaves) void gemm_q4_0_small_kernel(const uint8_t* __restrict__ w,
                                                                       const int8_t* __restrict__ codes,
                                                                       const float* __restrict__ records,
-                                                                      float* __restrict__ out, int m, int n, int k) {
+                                                                      float* __restrict__ out, int m, int n, int k, int stride, int per) {
+    // (stride: workgroups, per: tiles of one at most; as arguments, not from gridDim, which a vector load would bring, and a division)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -296,7 +315,7 @@ __global__ __launch_bounds__(64 * kSWaves) void gemm_q4_0_small_kernel(const uin
     uint8_t* ring = smem;
     const uint32_t ring_lds = lds_address(ring);
     const int ntiles = (n + 15) >> 4;
-    const int my_tiles = min(kSMaxTiles, (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
+    const int my_tiles = (int)blockIdx.x + (per - 1) * stride < ntiles ? per : per - 1;  // (the grid has no workgroup without a tile)
     const int ngrp = (nkb + kSGroup - 1) / kSGroup;
     const int total = ngrp * my_tiles * kSParts;
     // This wavefront's blocks of group gi, part p: [128 gi + (128 / parts) p + (8 / parts) wave, + 8 / parts) when they
@@ -341,7 +360,7 @@ __global__ __launch_bounds__(64 * kSWaves) void gemm_q4_0_small_kernel(const uin
 
     // this wavefront's row of item (group gi, tile index t, part p) -> ring slot `slot`, row `wave`
     auto issue = [&](int gi, int t, int p, int slot) {
-        const int n0 = ((int)blockIdx.x + t * (int)gridDim.x) * 16;
+        const int n0 = ((int)blockIdx.x + t * stride) * 16;
         const int kb = min(kSGroup * gi + kSItemBlk * p, nkb - 8);  // (a part past the end of K: a valid address, not used)
         const int pieces = min(kSItemBlk, nkb - kb) * Q4_0_BPB / 16;  // 9 per 8 blocks
         const uint8_t* src = w + (int64_t)min(n0 + wave, n - 1) * row_bytes + (int64_t)kb * Q4_0_BPB;
@@ -435,7 +454,7 @@ __global__ __launch_bounds__(64 * kSWaves) void gemm_q4_0_small_kernel(const uin
     __syncthreads();
     {
         const int t = wave >> 2, r = wave & 3;  // 16 (tile, register) pairs, one per wavefront
-        const int col = ((int)blockIdx.x + t * (int)gridDim.x) * 16 + nn, row = 4 * g + r;
+        const int col = ((int)blockIdx.x + t * stride) * 16 + nn, row = 4 * g + r;
         float v = 0.0f;
 #pragma unroll
         for (int ww = 0; ww < kSWaves; ww++) v += sums[((ww * kSMaxTiles + t) * 4 + r) * 64 + lane];
@@ -586,15 +605,15 @@ int64_t gemm_q4_0_workspace_bytes(int64_t m, int64_t k) { return lhs_q8t(nullptr
 hipError_t launch_gemm_q4_0(const void* lhs, int lhs_dtype, const uint8_t* w, int64_t m, int64_t n, int64_t k,
                             float* out, void* workspace, hipStream_t s) {
     const LhsQ8T p = lhs_q8t(workspace, m, k);
-    const int64_t tiles = (m + 15) / 16, ngroups = tiles * 16 * (k / 32);
+    const int64_t tiles = (m + 15) / 16;
     // Up to 16 lhs rows a pass: the weights are read once per pass and the kernel lives on HBM latency (gemm_q4_0_small_kernel).
     // More rows go in passes of 16 (the plane GEMM takes over where it is faster, see gemm_q4_0_planes_wanted): a pass costs 10.6 /
     // 12.8 / 16.0 us on 4096 x 4096 / 14336 x 4096 / 4096 x 14336, the 17..64-row kernel below 20 / 33 / 57 us up to 32 rows
     // and 49 / 56 / 165 up to 64.
     const bool small = k % 256 == 0 && !kernel_disabled("q4_0_small") && (tiles == 1 || !kernel_disabled("q4_0_small_passes"));
-    dim3 qgrid((unsigned)((ngroups * 32 + 255) / 256)), qblock(256);
-#define QMM_Q8_OPERAND(T_, W_)                                                                                        \
-    quantize_q8_0_operand_kernel<T_, W_><<<qgrid, qblock, 0, s>>>((const T_*)lhs, (int)m, (int)k, ngroups, p.codes, p.scale, p.sum)
+    const int64_t rows = tiles * 16;
+    const dim3 qgrid((unsigned)((k / 32 + 31) / 32), (unsigned)std::min<int64_t>(rows, kQuantizeRows), (unsigned)((rows + kQuantizeRows - 1) / kQuantizeRows)), qblock(256);
+#define QMM_Q8_OPERAND(T_, W_) quantize_q8_0_operand_kernel<T_, W_><<<qgrid, qblock, 0, s>>>((const T_*)lhs, (int)m, (int)(k / 32), p.codes, p.scale, p.sum)
     if (lhs_dtype == QMM_F32) {
         if (small) QMM_Q8_OPERAND(float, true);
         else QMM_Q8_OPERAND(float, false);
@@ -626,7 +645,7 @@ hipError_t launch_gemm_q4_0(const void* lhs, int lhs_dtype, const uint8_t* w, in
         for (int64_t t = 0; t < tiles; t++) {  // (codes 512 bytes, records 64 bytes per lhs tile and block)
             gemm_q4_0_small_kernel<<<dim3((unsigned)wgs), dim3(64 * kSWaves), kSLds, s>>>(
                 w, p.codes + t * nkb * 512, (const float*)((const char*)p.scale + t * nkb * 64), out + t * 16 * n,
-                (int)std::min<int64_t>(16, m - 16 * t), (int)n, (int)k);
+                (int)std::min<int64_t>(16, m - 16 * t), (int)n, (int)k, (int)wgs, (int)((ntiles + wgs - 1) / wgs));
         }
         return hipGetLastError();
     }
