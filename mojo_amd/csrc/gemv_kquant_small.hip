@@ -59,8 +59,8 @@ enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
 // MROWS: lhs rows of a workgroup, 1, 2, 4, 8 or 16 (rows past m repeat the last one and their results are dropped); more go side by side, in workgroups of their own.
 // MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up).
 struct SmallCut {
-    int per, stride;  // tiles (gated: pairs) of a workgroup at most, workgroups across the tiles
-    uint32_t packed;  // wavefronts; << 8: items (tile, matrix) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups of a workgroup; << 31: several tiles of lhs rows
+    int per, stride;  // tiles of a workgroup at most, workgroups across the tiles
+    uint32_t packed;  // wavefronts; << 8: tiles of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups of a workgroup; << 31: several tiles of lhs rows
 };
 template <int ENC, int MROWS, typename AT, int MODE>
 __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restrict__ a, int m, int k, const SmallCut& cut) {
@@ -94,19 +94,22 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
     const uint32_t ring_lds = lds_address(ring);
     float* const accs = (float*)(smem + waves * (2 * I::kSlot));  // [chunk][waves][LR][64]
     float* const totals = accs + chunk * waves * LR * 64;  // [chunk][LR][64], with more than one group
-    const int ntiles = MODE == kSmallMats ? mats.tile_end[kLanesMaxMats - 1] : (mats.n[0] + 15) >> 4;
-    const int my_items = (MODE == kSmallGated ? 2 : 1) * (share + (per - 1) * stride < ntiles ? per : per - 1);  // (the grid has no workgroup without a tile)
+    // Weight rows of a matrix in a tile.  Gated: eight of gate and the same eight of up, so that a workgroup has results whole with half as many of them: 14336 x 4096 4 bf16 rows seven such tiles for each
+    // of 256 compute units, where 896 pairs of whole tiles were four (eight tiles) for each of 224, 15.3 -> 13.9 us; Q6_K 13824 x 5120 28.8 -> 26.9, Q4_K 1000 x 4096 3 rows 6.9 -> 5.8, 11008 x 4096
+    // (six tiles either way) 15.0 -> 14.6.  The same sums.
+    constexpr int kTile = MODE == kSmallGated ? 8 : 16;
+    const int ntiles = MODE == kSmallMats ? mats.tile_end[kLanesMaxMats - 1] : (mats.n[0] + kTile - 1) / kTile;
+    const int my_items = share + (per - 1) * stride < ntiles ? per : per - 1;  // (the grid has no workgroup without a tile)
 
     // item i of the workgroup: its matrix, and the first row there
     auto matrix_of = [&](int i, int& n0, int& n) __attribute__((always_inline)) {
-        const int tile = share + (MODE == kSmallGated ? i >> 1 : i) * stride;
+        const int tile = share + i * stride;
         int j = 0;
         if constexpr (MODE == kSmallMats) {  // (entries past the last repeat it)
 #pragma unroll
             for (int i = 0; i + 1 < kLanesMaxMats; i++) j += tile >= mats.tile_end[i] ? 1 : 0;
         }
-        n0 = (MODE == kSmallMats && j ? tile - mats.tile_end[j - 1] : tile) * 16;
-        if constexpr (MODE == kSmallGated) j = i & 1;
+        n0 = (MODE == kSmallMats && j ? tile - mats.tile_end[j - 1] : tile) * kTile;
         n = mats.n[j];
         return j;
     };
@@ -116,24 +119,30 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
 #pragma unroll
     for (int i = 0; i < I::kLoads; i++) {
         const int p = min(lane + 64 * i, I::kPieces - 1), pr = p / I::kRowPieces, pc = p - pr * I::kRowPieces;
-        full[i] = (uint32_t)pr * row_bytes + (ENC == QMM_Q6_K ? 0u : 16u * (uint32_t)pc);
+        full[i] = (uint32_t)(pr % kTile) * row_bytes + (ENC == QMM_Q6_K ? 0u : 16u * (uint32_t)pc);
         if constexpr (ENC == QMM_Q6_K) at_row |= (pc < 13 ? 16u * (uint32_t)pc : 196u) << (8 * i);
     }
     auto issue = [&](int sb, int item, int slot) {
         int n0, n;
         const int j = matrix_of(item, n0, n);
         const uint8_t* const base = mats.w[j] + (int64_t)n0 * row_bytes + (ENC == QMM_Q6_K ? 0 : sb * I::kBpb);
+        const uint8_t* const base2 = MODE == kSmallGated ? mats.w[1] + (base - mats.w[0]) : base;
         const int last = n - 1 - n0;  // rows past the matrix repeat its last row (their results are dropped)
 #pragma unroll
         for (int i = 0; i < I::kLoads; i++) {
             uint32_t off = full[i];
-            if (last < 15) {  // (the last tile of a ragged matrix only)
-                const int pr = min(lane + 64 * i, I::kPieces - 1) / I::kRowPieces;
+            if (last < kTile - 1) {  // (the last tile of a ragged matrix only)
+                const int pr = min(lane + 64 * i, I::kPieces - 1) / I::kRowPieces % kTile;
                 off -= (uint32_t)(pr - min(pr, last)) * row_bytes;
             }
             if constexpr (ENC == QMM_Q6_K) off = ((off + (uint32_t)(sb * Q6_K_BPB)) & ~3u) + ((at_row >> (8 * i)) & 0xffu);
-            if (i < I::kLoads - 1 || I::kPieces % 64 == 0 || lane < I::kPieces - 64 * (I::kLoads - 1))
-                small_stream16(off, base, ring_lds + slot * I::kSlot + i * 1024);
+            if (i < I::kLoads - 1 || I::kPieces % 64 == 0 || lane < I::kPieces - 64 * (I::kLoads - 1)) {
+                const uint32_t to = ring_lds + slot * I::kSlot + i * 1024;
+                constexpr int kGate = 8 * I::kRowPieces;  // pieces of the first of two matrices
+                if (MODE != kSmallGated || 64 * (i + 1) <= kGate) small_stream16(off, base, to);
+                else if (64 * i >= kGate) small_stream16(off, base2, to);
+                else load16_to_lds_once((lane + 64 * i < kGate ? base : base2) + off, to);
+            }
         }
     };
 
@@ -411,35 +420,29 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
             __syncthreads();
             // the group's result (matrix row 16 tile + nn, lhs row kg + 4 j): dealt to the wavefronts, which add it to that of the groups before
             const int live = min(waves, nblk - g * waves);
-            constexpr int kEach = MODE == kSmallGated ? 2 : 1;
-            for (int q = wave; q < ct / kEach * LR; q += waves) {
-                const int t = q / LR * kEach, j = q % LR, row = row0 + kg + 4 * j;
-                float s[kEach];
+            for (int q = wave; q < ct * LR; q += waves) {
+                const int t = q / LR, j = q % LR, row = row0 + kg + 4 * j;
+                const float* const src = accs + ((t * waves) * LR + j) * 64 + lane;
+                float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                int w = 0;
+                for (; w + 4 <= live; w += 4)
 #pragma unroll
-                for (int h = 0; h < kEach; h++) {
-                    const float* const src = accs + (((t + h) * waves) * LR + j) * 64 + lane;
-                    float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                    int w = 0;
-                    for (; w + 4 <= live; w += 4)
+                    for (int i = 0; i < 4; i++) c[i] += src[(w + i) * LR * 64];
 #pragma unroll
-                        for (int i = 0; i < 4; i++) c[i] += src[(w + i) * LR * 64];
-#pragma unroll
-                    for (int i = 0; i < 3; i++)
-                        if (w + i < live) c[i] += src[(w + i) * LR * 64];
-                    s[h] = (c[0] + c[1]) + (c[2] + c[3]);
-                    if (groups > 1) {
-                        float* const total = totals + ((t + h) * LR + j) * 64 + lane;
-                        if (g > g_first) s[h] = *total + s[h];
-                        if (g + 1 < g_end) *total = s[h];
-                    }
+                for (int i = 0; i < 3; i++)
+                    if (w + i < live) c[i] += src[(w + i) * LR * 64];
+                float r = (c[0] + c[1]) + (c[2] + c[3]);
+                if (groups > 1) {
+                    float* const total = totals + (t * LR + j) * 64 + lane;
+                    if (g > g_first) r = *total + r;
+                    if (g + 1 < g_end) *total = r;
                 }
                 if (g + 1 < g_end) continue;
                 int n0, n;
                 const int mat = matrix_of(c0 + t, n0, n);
-                float r = s[0];
-                if constexpr (MODE == kSmallGated) r = s[0] / (1.0f + expf(-s[0])) * s[kEach - 1];
+                if constexpr (MODE == kSmallGated) r = r / (1.0f + expf(-r)) * dpp_move<0x128>(r);  // (lanes nn < 8: gate, times up eight lanes on)
                 const int64_t at = (int64_t)row * n + n0 + nn;
-                if (row < m && n0 + nn < n) {
+                if (row < m && nn < kTile && n0 + nn < n) {
                     if (out_bf16) ((uint16_t*)mats.out[mat])[at] = f2bf(r);
                     else mats.out[mat][at + (int64_t)part * m * n] = r;
                 }
@@ -476,8 +479,8 @@ int small_groups(int64_t k) {
     const int groups = (int)((k / 256 + kSmallWaves - 1) / kSmallWaves);
     return groups == 3 ? 4 : groups;
 }
-// tiles: of 16 weight rows, gated: pairs of them; parts: workgroups that share a tile, one group of K each
-SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int64_t k, bool gated, bool parts) {
+// tiles: of 16 weight rows, gated: of eight of each matrix; parts: workgroups that share a tile, one group of K each
+SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int64_t k, bool parts) {
     SmallPlan p;
     p.row_tiles = (int)((m + small_most_rows(lhs_dtype) - 1) / small_most_rows(lhs_dtype));
     m = std::min(m, small_most_rows(lhs_dtype));
@@ -492,9 +495,8 @@ SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int6
     p.grid = (int)((tiles + p.per - 1) / p.per);
     const int slot = encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? SmallItem<QMM_Q4_K>::kSlot : encoding == QMM_Q5_K ? SmallItem<QMM_Q5_K>::kSlot : SmallItem<QMM_Q6_K>::kSlot;
     // (as many items between two barriers as fit: a barrier after each, with two buffers, took Q6_K 28672 x 8192 with 16 rows from 65 to 92 us)
-    const int lr = m <= 4 ? 1 : m <= 8 ? 2 : 4, ring = p.waves * 2 * slot, each = (p.waves + (groups > p.parts ? 1 : 0)) * lr * 256, items = gated ? 2 * p.per : p.per;
-    p.chunk = std::min(std::min(items, 254), (kLdsPerCu / per_cu - ring) / each);
-    if (gated) p.chunk &= ~1;
+    const int lr = m <= 4 ? 1 : m <= 8 ? 2 : 4, ring = p.waves * 2 * slot, each = (p.waves + (groups > p.parts ? 1 : 0)) * lr * 256;
+    p.chunk = std::min(std::min(p.per, 254), (kLdsPerCu / per_cu - ring) / each);
     p.lds = (size_t)ring + (size_t)p.chunk * each;
     return p;
 }
@@ -508,7 +510,7 @@ bool small_parts(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const double convert = encoding == QMM_Q4_0 ? (m <= 2 ? 1.2 : m <= 4 ? 1.6 : m <= 8 ? 2.6 : 5.0)
                            : lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
     const int64_t tiles = (n + 15) / 16;
-    const SmallPlan w = small_plan(encoding, lhs_dtype, m, tiles, k, false, false), a = small_plan(encoding, lhs_dtype, m, tiles, k, false, true);
+    const SmallPlan w = small_plan(encoding, lhs_dtype, m, tiles, k, false), a = small_plan(encoding, lhs_dtype, m, tiles, k, true);
     const double walk = groups * ((w.per + w.chunk - 1) / w.chunk) * convert + groups * w.per * item;
     return convert + a.per * item + (a.per - 1) / a.chunk * 1.0 + 2.3 + 1.6e-6 * (4.0 * m * n * groups) < walk;
 }
@@ -563,7 +565,7 @@ bool gemv_kquant_small_supported(int encoding, int lhs_dtype, int64_t m, int64_t
 
 // What the fullest compute unit gets of a call whose workgroups walk K, a tile being 16 weight rows: small_tiles_wanted.
 SmallLoad small_load(int lhs_dtype, int64_t m, int64_t n, int64_t k) {
-    const SmallPlan p = small_plan(QMM_Q4_K, lhs_dtype, m, (n + 15) / 16, k, false, false);
+    const SmallPlan p = small_plan(QMM_Q4_K, lhs_dtype, m, (n + 15) / 16, k, false);
     const int workgroups = ((int64_t)p.grid * p.row_tiles + compute_units() - 1) / compute_units();
     return {workgroups, workgroups * p.waves};
 }
@@ -635,7 +637,7 @@ hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype
             if (j < count) values += m * ns[j];
             sums.end[j] = values;
         }
-    const SmallPlan p = small_plan(encoding, lhs_dtype, m, gated ? tiles / 2 : tiles, k, gated, parts);
+    const SmallPlan p = small_plan(encoding, lhs_dtype, m, gated ? (ns[0] + 7) / 8 : tiles, k, parts);
     const bool store_bf16 = out_bf16 && !parts;
     hipError_t e = encoding == QMM_Q4_0   ? run_small_rows<QMM_Q4_0>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                    : encoding == QMM_Q4_K ? run_small_rows<QMM_Q4_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)

@@ -118,6 +118,16 @@ def test_group_gated_pair_and_parts_of_k_give_the_same_sums(enc, m, k):
     assert torch.allclose(qmatmul_swiglu(QE[enc], a, gate, up).double(), g / (1 + torch.exp(-g)) * u, rtol=2.0**-21, atol=1e-30)
 
 
+@pytest.mark.parametrize("enc", ("Q4_0",) + ENCODINGS)
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(2, 1, 512), (4, 7, 512), (1, 8, 8448), (8, 9, 512), (3, 17, 4608), (16, 15, 1024), (4, 2056, 4096), (20, 23, 512), (4, 4099, 512)])
+def test_gated_pair_in_tiles_of_eight_rows_of_each_matrix(enc, lhs, m, n, k):
+    """Eight rows of gate and of up share a tile of the matrix cores: the sums of a call with one matrix, at the edges of such tiles (silu: some 2^-24 for each of its steps)."""
+    gate, up, a = packed(enc, n, k), packed(enc, n, k, 1), rows(m, k, lhs)
+    g, u = qmatmul(QE[enc], None, a, gate).double(), qmatmul(QE[enc], None, a, up).double()
+    assert torch.allclose(qmatmul_swiglu(QE[enc], a, gate, up).double(), g / (1 + torch.exp(-g)) * u, rtol=2.0**-21, atol=1e-30)
+
+
 def test_q6_k_at_every_multiple_of_four_and_an_odd_last_block():
     """Blocks of 210 bytes: rows that begin at 0 and at 2 mod 4 alternate with an odd number of blocks; a matrix of an odd number of them in all is left to the kernels
     that read its last one exactly."""
