@@ -23,29 +23,24 @@ namespace qmm {
 
 namespace {
 
-// The weights of one wavefront: 32 columns, two buffers of a unit of K in LDS that only it writes (issue) and reads (open, before_step).
+// The weights of one wavefront: 32 columns, two buffers of a unit of K in LDS that only it writes (issue, a load at a time) and reads (open, before_step).
 // Q4_K, Q5_K: rows as they lie in memory.
 template <int ENC, bool CENTER>
 struct StagedK : KQuantWeights<ENC, 1, CENTER> {
     using Base = KQuantWeights<ENC, 1, CENTER>;
     using Rows = typename Base::Rows;
-    static constexpr int kLoads = Rows::kLoads, kWhole = Rows::kTotal / 64;  // instructions, those of all lanes
+    static constexpr int kLoads = Rows::kLoads;
     uint32_t stage_lds;
     const uint8_t* stage;
     __device__ __forceinline__ void init(const WeightTensors& t, int n0, int lane, uint8_t* at) {
         Base::init(t, n0, lane, at);
         stage_lds = lds_address(at);
         stage = this->mine;
-#pragma unroll
-        for (int j = 0; j < kWhole; j++) this->rows.off[j] += load_run_offset(j);
     }
+    template <int J>
     __device__ __forceinline__ void issue(int unit, int buf) {
-        const uint8_t* b = this->rows.w + (int64_t)unit * Rows::kRow;
-        const uint32_t to = stage_lds + buf * Base::kStage;
-        load_run_to_lds<kWhole>(this->rows.off, b, to);
-        if constexpr (kWhole < kLoads) {
-            if (kWhole * 64 + this->lane_ < Rows::kTotal) load16_to_lds(this->rows.off[kWhole], b, to + kWhole * 1024);
-        }
+        if (J * 64 + 63 < Rows::kTotal || J * 64 + this->lane_ < Rows::kTotal)
+            load16_to_lds(this->rows.off[J], this->rows.w + (int64_t)unit * Rows::kRow, stage_lds + buf * Base::kStage + J * 1024);
     }
     __device__ __forceinline__ void open(int, int buf) {
         this->mine = stage + buf * Base::kStage;
@@ -84,7 +79,7 @@ struct StagedGptq : NoOffsets {
         // LDS row p holds word row 4 blk + 2 g + a with p = 4 blk + 2 a + g: the two half wavefronts read other banks
         const int p = lane >> 3, row = (p & 4) + 2 * (p & 1) + ((p >> 1) & 1);
 #pragma unroll
-        for (int j = 0; j < 4; j++) off[j] = (uint32_t)(row + 8 * j) * (uint32_t)n * 4u + (uint32_t)min(n0 + 4 * (lane & 7), n - 4) * 4u + load_run_offset(j);
+        for (int j = 0; j < 4; j++) off[j] = (uint32_t)(row + 8 * j) * (uint32_t)n * 4u + (uint32_t)min(n0 + 4 * (lane & 7), n - 4) * 4u;
 #pragma unroll
         for (int j = 0; j < kHeads; j++) {
             const int i = j * 64 + lane, blk = min(i / kHead, kBlocks - 1), part = i % kHead;
@@ -93,14 +88,15 @@ struct StagedGptq : NoOffsets {
             head_stride[j] = part < 16 ? (uint32_t)n * 2u : (uint32_t)(n >> 3) * 4u;
         }
     }
+    template <int J>
     __device__ __forceinline__ void issue(int unit, int buf) {
         const uint32_t to = stage_lds + buf * kStage;
-        load_run_to_lds<4>(off, qw + (int64_t)(32 * unit) * n * 4, to);
-#pragma unroll
-        for (int j = 0; j < kHeads; j++) {
+        if constexpr (J < 4) {
+            load16_to_lds(off[J], qw + (int64_t)(32 * unit) * n * 4, to + J * 1024);
+        } else {
             // (a group is a whole number of 32s and K below 2^27: half of one keeps the product off the integers by more than its rounding)
-            const int group = (int)(((float)(8 * unit + head_block[j]) + 0.5f) * per_group);
-            load4_to_lds(head[j] + (uint64_t)(uint32_t)group * head_stride[j], to + 4096 + j * 256);
+            const int group = (int)(((float)(8 * unit + head_block[J - 4]) + 0.5f) * per_group);
+            load4_to_lds(head[J - 4] + (uint64_t)(uint32_t)group * head_stride[J - 4], to + 4096 + (J - 4) * 256);
         }
     }
     __device__ __forceinline__ void read_words(int blk) {
@@ -162,13 +158,15 @@ struct StagedQ6 : Q6Weights<1, FLUSH> {
         off_tail = row_at(lane & 31) + 208;
         mine_odd = row_at(lane & 31) & 2u;
     }
+    template <int J>
     __device__ __forceinline__ void issue(int unit, int buf) {
         const uint8_t* b = w + (int64_t)unit * Q6_K_BPB;
         const uint32_t o = (unit & 1) ? ~odd : odd, to = stage_lds + buf * kStage;
-#pragma unroll
-        for (int j = 0; j < kWide; j++)
-            if (j * 64 + 63 < kTotal || j * 64 + this->lane_ < kTotal) load16_to_lds(off[j] + 2 - ((o >> j) & 2u), b - 2, to + j * 1024);
-        if (this->lane_ < 32) load4_to_lds(b - 2 + (off_tail + 2 - ((mine_odd ^ (unit << 1)) & 2u)), to + kTail);
+        if constexpr (J < kWide) {
+            if (J * 64 + 63 < kTotal || J * 64 + this->lane_ < kTotal) load16_to_lds(off[J] + 2 - ((o >> J) & 2u), b - 2, to + J * 1024);
+        } else if (this->lane_ < 32) {
+            load4_to_lds(b - 2 + (off_tail + 2 - ((mine_odd ^ (unit << 1)) & 2u)), to + kTail);
+        }
     }
     // 16 bytes at offset `at` of the block
     __device__ __forceinline__ gd_u4 field(int at) const {
@@ -266,6 +264,9 @@ struct StagedGrid {
     int full, sections, shares;
 };
 
+// How many of n loads, spread over the steps before `end` (0: asked for before the first one), are asked for before step t.
+constexpr int spread_before(int n, int end, int t) { return t < 0 ? 0 : t >= end ? n : (t * n + end - 1) / end; }
+
 // What arrives in scalar registers with a workgroup (the rest of the arguments is asked for when it runs).
 struct StagedStart {
     const void *a16, *sums;
@@ -339,14 +340,28 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart&
     auto issue_lhs = [&](int chunk, int buf) __attribute__((always_inline)) {
         load_run_to_lds<kLoads>(from, src + (int64_t)min(chunk, last_chunk) * (kPieces * 1024), lds0 + (wk * kBufs + buf) * kBuf + piece0 * 1024);
     };
-    auto issue_weights = [&](int unit, int buf) __attribute__((always_inline)) {
-        w.issue(unit, buf);
-#pragma unroll
-        for (int j = 0; j < kSums; j++) {
-            const int a = (wn + WN * j) % FM;
-            load16_to_lds(l16, (const uint8_t*)start.sums + ((int64_t)min(row0 + a, last_tile) * units + unit) * 1024,
-                          (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + L::kS + ((wk * 2 + buf) * FM + a) * 1024)));
-        }
+    // bf16 rows: loads are asked for a few at a time; at many at once, 16 cycles of a compute unit's load path for each, the wavefronts stand still.  The chunk that a boundary makes room for in two
+    // halves, the second one a step later; the weights and sums of the next unit over the first steps of this one, early enough to be older than the chunk that the last boundary waits for.
+    // us, all at once / this way: GPTQ 14336 x 4096 400 rows 59.0 / 57.5, Q6_K 8192 x 8192 500 rows 128.8 / 126.3, Q4_K 4096 x 14336 2048 rows 261.7 / 257.8, 4096 x 4096 64 rows 13.2 / 12.5; but fp32 rows, which
+    // have twice the matrix-core instructions to hide loads behind, GPTQ 14336 x 4096 500 rows 116.6 / 119.2, and groups of 32 8192 x 8192 300 bf16 rows 93.2 / 95.0.
+    constexpr bool kFew = !HILO && !(ENC == QMM_GPTQ && FLUSH == 2), kTwice = kFew && kCS >= 4 && kLoads % 2 == 0 && kOneTile;
+    constexpr int kSpread = kFew ? std::min(10, 15 - kCS * (kBufs - 1)) : 0;
+    auto issue_half = [&](int half, int chunk, int buf) __attribute__((always_inline)) {
+        constexpr int kHalf = kLoads / 2;
+        load_run_to_lds<kHalf>(from, src + (int64_t)min(chunk, last_chunk) * (kPieces * 1024) + half * (kHalf * 1024), lds0 + (wk * kBufs + buf) * kBuf + (piece0 + half * kHalf) * 1024);
+    };
+    auto issue_weights = [&](auto first, auto end, int unit, int buf) __attribute__((always_inline)) {  // loads first .. end - 1 of a unit
+        constexpr int kFirst = decltype(first)::value, kEnd = decltype(end)::value;
+        unrolled<kEnd - kFirst>([&](auto i) __attribute__((always_inline)) {
+            constexpr int j = kFirst + decltype(i)::value;
+            if constexpr (j < W::kLoads) {
+                w.template issue<j>(unit, buf);
+            } else {
+                const int a = (wn + WN * (j - W::kLoads)) % FM;
+                load16_to_lds(l16, (const uint8_t*)start.sums + ((int64_t)min(row0 + a, last_tile) * units + unit) * 1024,
+                              (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + L::kS + ((wk * 2 + buf) * FM + a) * 1024)));
+            }
+        });
     };
     half8 af[2][FM][kPer];
     uint32_t at = 0;  // where the lane's operands of the current chunk are
@@ -360,7 +375,7 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart&
     half8 b[2][W::kPlanes];
     float d = 0.0f;
     if (u0 < u1) {
-        issue_weights(u0, 0);
+        issue_weights(std::integral_constant<int, 0>{}, std::integral_constant<int, kWeightLoads>{}, u0, 0);
 #pragma unroll
         for (int c = 0; c < kBufs; c++) issue_lhs(c, c);
     }
@@ -373,7 +388,7 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart&
         read_lhs(0, 0);
         w.template step<0>(0, b[0]);
     }
-    int buf = 0;  // of the current chunk
+    int buf = 0, free_buf = 0;  // of the current chunk, of the one before
     for (int it = 0; it < walk; it++) {
         const int u = u0 + it;
         if (u >= u1) {
@@ -381,21 +396,29 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart&
             for (int c = 0; c < kChunks; c++) __syncthreads();
             continue;
         }
-        issue_weights(min(u + 1, u1 - 1), (it + 1) & 1);
+        const int next = min(u + 1, u1 - 1);
+        if constexpr (kSpread == 0) issue_weights(std::integral_constant<int, 0>{}, std::integral_constant<int, kWeightLoads>{}, next, (it + 1) & 1);
         float dmin = w.min_scale(0), dnext = 0.0f;  // (CENTER: the power of two that the offsets are in units of, made in the first five steps)
         if constexpr (ENC != QMM_GPTQ) dnext = w.scale(0);
         __builtin_amdgcn_sched_barrier(0);
         unrolled<W::kSteps>([&](auto tt) __attribute__((always_inline)) {
             constexpr int t = decltype(tt)::value, chunk = t / kCS, cur = t & 1;
             if constexpr ((t + 1) % kCS == 0) {
-                // Lhs chunk c + 1 has arrived (asked for kBufs - 1 boundaries ago), at the last boundary of a unit also the weights of the next one, and
-                // every wavefront has read chunk c: its buffer takes chunk c + kBufs.
-                static_assert(kChunks >= kBufs, "at the last boundary the weights are older than the chunk that is waited for");
-                wait_vmcnt<(kBufs - 2) * kLoads + (chunk < kBufs - 1 ? kWeightLoads : 0)>();
+                // Lhs chunk c + 1 has arrived (asked for kBufs - 1 boundaries ago, its second half a step later), at the last boundary of a unit also the weights of the next one, and
+                // every wavefront has read chunk c: its buffer takes chunk c + kBufs.  Younger than what is waited for: the chunks asked for since, and the weights of the steps since.
+                constexpr int kSince = t - kCS * (kBufs - 1) + (kTwice ? 1 : 0);
+                static_assert(t + 1 < W::kSteps || kSince >= kSpread, "at the last boundary the weights are older than the chunk that is waited for");
+                static_assert(kSince >= 0 || 16 + kSince >= kSpread, "none of the unit before are younger");
+                wait_vmcnt<(kBufs - 2) * kLoads + spread_before(kWeightLoads, kSpread, t) - spread_before(kWeightLoads, kSpread, kSince)>();
                 __syncthreads();
-                issue_lhs(it * kChunks + chunk + kBufs, buf);
+                if constexpr (kTwice) issue_half(0, it * kChunks + chunk + kBufs, buf);
+                else issue_lhs(it * kChunks + chunk + kBufs, buf);
+                free_buf = buf;
                 buf = buf == kBufs - 1 ? 0 : buf + 1;
                 buffer(buf);
+            }
+            if constexpr (kTwice && t % kCS == 0) {
+                if (t > 0 || it > 0) issue_half(1, it * kChunks + t / kCS - 1 + kBufs, free_buf);
             }
             read_lhs((t + 1) % kCS, cur ^ 1);
             if constexpr (t + 1 == W::kSteps) w.open(u + 1 < u1 ? u + 1 : u, (it + 1) & 1);
@@ -458,6 +481,7 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart&
                     else T[min_a][r] = fmaf(dmin, M[r], T[min_a][r]);
                 }
             }
+            issue_weights(std::integral_constant<int, spread_before(kWeightLoads, kSpread, t)>{}, std::integral_constant<int, spread_before(kWeightLoads, kSpread, t + 1)>{}, next, (it + 1) & 1);
             w.template step<(t + 1) % W::kSteps>(0, b[cur ^ 1]);
             if constexpr (t % W::kFlush != 0) {
                 constexpr int kMfma = FM * kPer * W::kPlanes, kValu = (W::kPlanes == 2 ? 28 : W::kMin ? 12 : 14) + (min_add ? 16 : 0);  // spread evenly
