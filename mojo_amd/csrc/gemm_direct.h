@@ -43,6 +43,9 @@ struct DirectPlan {
 };
 hipError_t launch_gemm_shared(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
                               int64_t m, int units, hipStream_t s);
+// gptq_order.hip: the columns of the weights sorted by group and, unless !lhs_done, those of the lhs in p, with `zero` (up to `zeros` results each) zeroed.
+hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int group, const void* lhs, int lhs_dtype, int64_t m, const DirectSpace& p, const DirectMats& zero,
+                             int64_t zeros, bool& lhs_done, hipStream_t s);
 hipError_t launch_gemm_staged(int encoding, bool hilo, const DirectPlan& pl, const WeightTensors& wt, DirectMats mats, const DirectSpace& p, uint16_t* out16,
                               int64_t m, int units, hipStream_t s);
 
@@ -104,6 +107,76 @@ constexpr int kRowTop = 14, kRowTopWithSums = 9;
 // The operand order of the lhs: step t = 2 blk + a of 16 columns holds, for half wavefront g, the columns
 //   32 blk + 16 g + 8 a + slot order   (kOrderK: slots 0,2,1,3,4,6,5,7; kOrderGptq: 0,4,1,5,2,6,3,7)
 constexpr int kOrderK = 0, kOrderGptq = 1;  // (Q4_0: 32 blk + 16 a + 8 g + the slots of kOrderK)
+
+// Eight columns of a row.
+template <typename AT>
+__device__ __forceinline__ void load8(const AT* p, float (&v)[8]) {
+    if constexpr (sizeof(AT) == 4) {
+        const float4 x = *(const float4*)p, y = *(const float4*)(p + 4);
+        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+        v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+    } else {
+        const uint4 x = *(const uint4*)p;
+        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[2 * i] = __uint_as_float(w[i] << 16);
+            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+        }
+    }
+}
+// Their largest magnitude, of the finite ones.
+__device__ __forceinline__ float largest(float mx, const float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]) <= 3.402823466e38f ? fabsf(v[i]) : 0.0f);
+    return mx;
+}
+// What a row is multiplied by, and its inverse, from the bits of its largest magnitude.
+__device__ __forceinline__ float row_scale(uint32_t largest_bits, int row_top, float& inv) {
+    int e = (int)((largest_bits >> 23) & 0xffu) - 127;
+    e = max(e, row_top - 126);  // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
+    inv = __uint_as_float((uint32_t)(127 - row_top + e) << 23);
+    return __uint_as_float((uint32_t)(127 + row_top - e) << 23);
+}
+// Piece pc (eight columns) of a row, scaled by s (v is left so), as its part of the operands.
+template <typename AT, int ORDER>
+__device__ __forceinline__ void store_piece(_Float16* a16, int steps, int row, int pc, float s, float (&v)[8]) {
+    constexpr bool kF32 = sizeof(AT) == 4;
+    constexpr int perm[2][8] = {{0, 2, 1, 3, 4, 6, 5, 7}, {0, 4, 1, 5, 2, 6, 3, 7}};
+    const int blk = pc >> 2, g = (pc >> 1) & 1, step = 2 * blk + (pc & 1);
+    float h[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] *= s;
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] = h2f(f2h(v[i]));
+    gd_u4 hi;
+#pragma unroll
+    for (int i = 0; i < 4; i++) hi[i] = pack_half2(h[perm[ORDER][2 * i]], h[perm[ORDER][2 * i + 1]]);
+    _Float16* at = a16 + ((int64_t)(row >> 5) * steps + step) * (kF32 ? 1024 : 512) + ((row & 31) + 32 * g) * 8;
+    *(gd_u4*)at = hi;
+    if constexpr (kF32) {
+        gd_u4 lo;
+        float residual[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) residual[i] = fabsf(h[i]) <= 65504.0f ? v[i] - h[i] : 0.0f;  // (an infinity has no residual: inf - inf)
+#pragma unroll
+        for (int i = 0; i < 4; i++) lo[i] = pack_half2(residual[perm[ORDER][2 * i]], residual[perm[ORDER][2 * i + 1]]);
+        *(gd_u4*)(at + 512) = lo;
+    }
+}
+// The e-th of `count` workgroups zeroes its part of the results (m rows).
+__device__ __forceinline__ void zero_out(const DirectMats& z, int m, int e, int count) {
+    const int threads = (int)blockDim.x;
+    for (int j = 0; j < z.count; j++) {
+        float* __restrict__ const out = z.out[j];
+        const int64_t values = (int64_t)m * z.n[j];
+        for (int64_t i = ((int64_t)e * threads + threadIdx.x) * 4; i < values; i += (int64_t)count * threads * 4) {
+            if (i + 3 < values) *(float4*)(out + i) = make_float4(0.f, 0.f, 0.f, 0.f);
+            else
+                for (int64_t q = i; q < values; q++) out[q] = 0.0f;
+        }
+    }
+}
 
 // ---------------------------------------------------------------------------------------------------------------------------
 // the weights of one wavefront: what it holds of a unit of K, how a step's operands come out of it

@@ -46,36 +46,6 @@ DirectSpace direct_space(void* ws, bool f32, bool with_sums, bool with_sums32, i
 // ---------------------------------------------------------------------------------------------------------------------------
 // preparation: one workgroup per lhs row (the first m workgroups), then zeroing of `out` for two workgroups per tile
 // ---------------------------------------------------------------------------------------------------------------------------
-template <typename AT>
-__device__ __forceinline__ void load8(const AT* p, float (&v)[8]) {
-    if constexpr (sizeof(AT) == 4) {
-        const float4 x = *(const float4*)p, y = *(const float4*)(p + 4);
-        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-        v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
-    } else {
-        const uint4 x = *(const uint4*)p;
-        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[2 * i] = __uint_as_float(w[i] << 16);
-            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-        }
-    }
-}
-// the e-th of `count` workgroups zeroes its part of the results (m rows)
-__device__ __forceinline__ void zero_out(const DirectMats& z, int m, int e, int count) {
-    const int threads = (int)blockDim.x;
-    for (int j = 0; j < z.count; j++) {
-        float* __restrict__ const out = z.out[j];
-        const int64_t values = (int64_t)m * z.n[j];
-        for (int64_t i = ((int64_t)e * threads + threadIdx.x) * 4; i < values; i += (int64_t)count * threads * 4) {
-            if (i + 3 < values) *(float4*)(out + i) = make_float4(0.f, 0.f, 0.f, 0.f);
-            else
-                for (int64_t q = i; q < values; q++) out[q] = 0.0f;
-        }
-    }
-}
-
 // With few rows the latency of a row's passes (load, maximum, narrow, store) bounds it: as many threads as leave each one or two pieces of eight
 // columns (200 x 14336 bf16 rows with 256 threads a row 10.1 us, with 1024 7.2); with many, that a row writes 16 bytes of a 128-byte line, the rest
 // of which other workgroups of the XCD fill (500 x 14336: 11.5 us for 28 MB, whatever the number of threads).
@@ -84,7 +54,6 @@ __device__ __forceinline__ void zero_out(const DirectMats& z, int m, int e, int 
 template <typename AT, int ORDER, bool SORTED = false>
 __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict__ a, int m, int k, DirectSpace p, int with_sums, DirectMats zero,
                                                            const int32_t* __restrict__ source) {
-    constexpr bool kF32 = sizeof(AT) == 4;
     extern __shared__ __attribute__((aligned(16))) uint8_t row_lds[];
     __shared__ uint32_t wmax[16];
     const int tid = threadIdx.x, threads = (int)blockDim.x, rows = (m + 63) / 64 * 64;
@@ -111,7 +80,7 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
             const int from[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                if constexpr (kF32) v[i] = ((const float*)row_lds)[from[i]];
+                if constexpr (sizeof(AT) == 4) v[i] = ((const float*)row_lds)[from[i]];
                 else v[i] = __uint_as_float((uint32_t)((const uint16_t*)row_lds)[from[i]] << 16);
             }
         } else {
@@ -119,22 +88,18 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
         }
     };
     float mx = 0.0f;
-    auto top = [&](const float (&v)[8]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]) <= 3.402823466e38f ? fabsf(v[i]) : 0.0f);  // (of the finite values)
-    };
     if (hold) {
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
             if (tid + i * threads < pieces) load(tid + i * threads, held[i]);
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * threads < pieces) top(held[i]);
+            if (tid + i * threads < pieces) mx = largest(mx, held[i]);
     } else {
         for (int pc = tid; pc < pieces; pc += threads) {
             float v[8];
             load(pc, v);
-            top(v);
+            mx = largest(mx, v);
         }
     }
     const uint32_t mb = wave_max_nonneg_bits(mx);
@@ -142,35 +107,15 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     __syncthreads();
     uint32_t mxb = 0;
     for (int i = 0; i < threads >> 6; i++) mxb = max(mxb, wmax[i]);
-    int e = (int)((mxb >> 23) & 0xffu) - 127;
-    const int row_top = with_sums ? kRowTopWithSums : kRowTop;
-    e = max(e, row_top - 126);  // (the smallest inverse scale that is a normal number, 2^-126: the least fp32 value, 2^-149, becomes 2^-23 and is held exactly)
-    const float s = __uint_as_float((uint32_t)(127 + row_top - e) << 23);
-    if (tid == 0) p.inv[row] = __uint_as_float((uint32_t)(127 - row_top + e) << 23);
+    float inv;
+    const float s = row_scale(mxb, with_sums ? kRowTopWithSums : kRowTop, inv);
+    if (tid == 0) p.inv[row] = inv;
     const int tile = row >> 5, lane = row & 31;
     auto emit = [&](int pc, float (&v)[8]) __attribute__((always_inline)) {
-        constexpr int perm[2][8] = {{0, 2, 1, 3, 4, 6, 5, 7}, {0, 4, 1, 5, 2, 6, 3, 7}};
-        const int blk = pc >> 2, g = (pc >> 1) & 1, step = 2 * blk + (pc & 1);
-        float h[8], sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] *= s;
-#pragma unroll
-        for (int i = 0; i < 8; i++) h[i] = h2f(f2h(v[i]));
-        gd_u4 hi;
-#pragma unroll
-        for (int i = 0; i < 4; i++) hi[i] = pack_half2(h[perm[ORDER][2 * i]], h[perm[ORDER][2 * i + 1]]);
-        _Float16* at = p.a16 + ((int64_t)tile * steps + step) * (kF32 ? 1024 : 512) + (lane + 32 * g) * 8;
-        *(gd_u4*)at = hi;
-        if constexpr (kF32) {
-            gd_u4 lo;
-            float residual[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) residual[i] = fabsf(h[i]) <= 65504.0f ? v[i] - h[i] : 0.0f;  // (an infinity has no residual: inf - inf)
-#pragma unroll
-            for (int i = 0; i < 4; i++) lo[i] = pack_half2(residual[perm[ORDER][2 * i]], residual[perm[ORDER][2 * i + 1]]);
-            *(gd_u4*)(at + 512) = lo;
-        }
+        store_piece<AT, ORDER>(p.a16, steps, row, pc, s, v);
         if (with_sums) {
+            const int blk = pc >> 2;
+            float sum = 0.0f;
 #pragma unroll
             for (int i = 0; i < 8; i += 2) sum += v[i] + v[i + 1];
             sum += dpp_move<0xB1>(sum);
@@ -853,7 +798,7 @@ int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int6
 // call of its own; the tile is the one that suits them together).  q | k | v of 4096 | 1024 | 1024 x 4096 with 16 rows: one launch for three.
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
                               const uint16_t* scales, const uint32_t* qzeros, int group, int64_t m, int64_t k, uint16_t* out16, void* workspace,
-                              hipStream_t s, bool any_rows, const int32_t* source) {
+                              hipStream_t s, bool any_rows, const GptqOrder* order) {
     const bool q40 = encoding == QMM_Q4_0, f32 = lhs_dtype == QMM_F32, sums = encoding == QMM_Q4_K || encoding == QMM_Q5_K || q40;
     if (count < 1 || count > kDirectMaxMats) return hipErrorInvalidValue;
     const DirectSpace p = direct_space(workspace, f32 && !q40, sums, sums && !q40, m, k);
@@ -869,12 +814,17 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
     if (q40) {
         if (f32) direct_prep_q8_kernel<float><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, zero);
         else direct_prep_q8_kernel<uint16_t><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, zero);
-    } else if (source) {  // (the rest of the path takes it up to K = 32768, fp32 rows of 128 KB)
+    } else if (order) {  // (the rest of the path takes it up to K = 32768, fp32 rows of 128 KB)
         if (encoding != QMM_GPTQ || k % 32 || k > 32768) return hipErrorInvalidValue;
-        hipError_t e = f32 ? allow_full_lds<direct_prep_kernel<float, kOrderGptq, true>, 64>() : allow_full_lds<direct_prep_kernel<uint16_t, kOrderGptq, true>, 64>();
+        bool lhs_done;
+        hipError_t e = launch_gptq_order(*order, ns[0], k, group, lhs, lhs_dtype, m, p, zero, zeros, lhs_done, s);
+        if (e == hipSuccess && !lhs_done)
+            e = f32 ? allow_full_lds<direct_prep_kernel<float, kOrderGptq, true>, 64>() : allow_full_lds<direct_prep_kernel<uint16_t, kOrderGptq, true>, 64>();
         if (e != hipSuccess) return e;
         const size_t row = (size_t)k * (f32 ? 4 : 2);
-        if (f32) direct_prep_kernel<float, kOrderGptq, true><<<dim3(grid), dim3(threads), row, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero, source);
+        const int32_t* const source = order->space.source;
+        if (lhs_done) {
+        } else if (f32) direct_prep_kernel<float, kOrderGptq, true><<<dim3(grid), dim3(threads), row, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero, source);
         else direct_prep_kernel<uint16_t, kOrderGptq, true><<<dim3(grid), dim3(threads), row, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, sums, zero, source);
     } else if (encoding == QMM_GPTQ) {
         if (f32) direct_prep_kernel<float, kOrderGptq><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, sums, zero, nullptr);

@@ -2,20 +2,23 @@
 // groups serve the call.
 //
 // The kernel that looks the group of every k up (gemv_gptq.hip) passes over the weights once per four rows and multiplies on the vector
-// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 99 us.  Sorting costs one launch and one pass over the packed weights: a workgroup holds some
+// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 77 us.  Sorting costs one launch and one pass over the packed weights: a workgroup holds some
 // columns of the output in LDS (all of K), sorts the columns of K by group while those are on their way, and takes the eight nibbles of every word of the sorted
-// matrix from there.  The preparation of the lhs in the direct GEMM reads its rows in the same order.
+// matrix from there.  Workgroups of the same launch hold rows of the lhs there instead and leave the operands of the direct GEMM in the same order; where the launch has no room for them,
+// that GEMM's own preparation does.
 // What bounds the pass, at 14336 x 4096 (2 x 29 MB, 22 us with nothing in the caches, 2.6 TB/s): loads, sort (hidden behind them but for its start),
 // nibbles (two vector instructions each, about 6 us) and stores one after the other, since all workgroups run at once.
 // us of the whole call with the sort as a launch of its own and a sorted copy of the lhs / this way, nothing in the caches: 14336 x 4096 400 rows 127 / 122, 8 rows 50 / 44;
 // 4096 x 14336 64 rows 76 / 63; 4096 x 4096 64 rows 37 / 30; 8192 x 8192 300 rows 130 / 123; 1024 x 4096 20 rows 29 / 22; 8192 x 28672 20 rows 184 / 174;
-// 3584 x 18944 33 rows 90 / 90.
+// 3584 x 18944 33 rows 90 / 90.  With the lhs as a launch of its own / in the same one: 14336 x 4096 400 rows 81.5 / 77.6, 8 rows 36.5 / 32.9, 100 fp32 rows 56.7 / 52.0; 4096 x 4096
+// 64 rows 25.0 / 24.3; 1024 x 4096 20 rows 17.4 / 14.6; 3584 x 18944 33 rows 68.4 / 63.9; 2560 x 9088 9 fp32 rows 38.4 / 33.3; 28672 x 8192 40 rows 108.7 / 107.0.
 //
 // A sorted column list is a plain-group matrix only if every group has exactly group_size columns, which is so in any checkpoint that was
 // quantised group by group.  The device finds out: where it is not so, the sort leaves a mark, the order as it was (the products are then
 // meaningless) and the look-up kernel, launched behind them, replaces the whole result; otherwise that launch returns at once.
 #include <algorithm>
 
+#include "gemm_direct.h"
 #include "lds_stream.h"
 #include "qmm_internal.h"
 
@@ -27,6 +30,44 @@ typedef uint32_t go_u4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 16, kThreads = 64 * kWaves;
 
+// The lhs: its rows (the first workgroups of the grid), where their operands and inverse scales go, and the results that are added to (the next ones zero them).
+struct OrderLhs {
+    const void* a;
+    _Float16* a16;
+    float* inv;
+    int m, workgroups, zeroing;  // multiples of 8
+    DirectMats zero;
+};
+constexpr int lhs_rows(int cols, int size) { return cols / (size == 4 ? 8 : 4); }  // of a workgroup: as many bytes as its words of the weights
+
+// The bits of a row's largest magnitude, of the finite ones, by one wavefront: every wavefront of a row for itself (LDS is full of words and order), on the bits of the values,
+// two vector instructions a dword.
+template <typename AT>
+__device__ __forceinline__ uint32_t wave_largest(const AT* x, int k, int lane) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    constexpr int kPer = 16 / sizeof(AT);
+    uint32_t top = 0;
+    for (int i = lane * kPer; i < k; i += 64 * kPer) {
+        const go_u4 y = *(const go_u4*)(x + i);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if constexpr (sizeof(AT) == 4) top = max(top, y[j] & 0x7fffffffu);
+            else top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top), __builtin_bit_cast(u16x2, y[j] & 0x7fff7fffu)));
+        }
+    }
+    if constexpr (sizeof(AT) == 2) top = max(top & 0xffff0000u, top << 16);
+    float mx = __uint_as_float(top);
+    if (__any(top >= 0x7f800000u)) {
+        mx = 0.0f;
+        for (int pc = lane; pc < k >> 3; pc += 64) {
+            float v[8];
+            load8(x + pc * 8, v);
+            mx = largest(mx, v);
+        }
+    }
+    return wave_max_nonneg_bits(mx);
+}
+
 // Workgroup: COLS columns of the weights, neighbours on one XCD (they share cache lines).  It sorts for itself while its words are on their way to LDS: where the
 // sort was a launch of one workgroup it took 6.6 us at K = 4096 and 18 at 14336.
 // Stable sort (within a group the columns keep their order), wavefront w takes a sixteenth of K, TURNS times 64 columns; group indices outside [0, groups) are
@@ -34,15 +75,24 @@ constexpr int kWaves = 16, kThreads = 64 * kWaves;
 // LDS: [k / 8][COLS] words, uint16 [k] order, uint16 [kWaves][groups] counts.
 // Where that is more than a compute unit has (K beyond 26208, less with groups of 32 or 64), or leaves room for one workgroup and there are several for each compute unit: a launch of
 // one workgroup without words (qweight null) that only sorts, then TURNS = 0, which takes the order from memory.
-template <int COLS, int TURNS>
-__global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_permute_kernel(const uint32_t* __restrict__ qweight, const int32_t* __restrict__ g_idx, int n,
-                                                                                          int k, int group, int bits, int per_xcd, int32_t* __restrict__ source,
-                                                                                          int32_t* __restrict__ uneven, uint32_t* __restrict__ sorted_w) {
+template <typename AT, int COLS, int TURNS>
+__global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kernel(const uint32_t* __restrict__ qweight, const int32_t* __restrict__ g_idx, int n, int k, int group, int bits,
+                                                                                  int per_xcd, int32_t* __restrict__ source, int32_t* __restrict__ uneven,
+                                                                                  uint32_t* __restrict__ sorted_w, OrderLhs lhs) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = (int)blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int kPieces = COLS / 4, kRows = kThreads / kPieces;  // rows of words per turn
-    const int slab = ((b & 7) * per_xcd + (b >> 3)) * COLS;
-    if (slab >= n) return;
+    constexpr int kLhsRows = lhs_rows(COLS, sizeof(AT)), kRowWaves = kWaves / kLhsRows;
+    const int b = (int)blockIdx.x - lhs.workgroups - lhs.zeroing, slab = ((b & 7) * per_xcd + (b >> 3)) * COLS;
+    if (b >= 0 && slab >= n) return;
+    if (b < 0 && b >= -lhs.zeroing) {
+        zero_out(lhs.zero, lhs.m, b + lhs.zeroing, lhs.zeroing);
+        return;
+    }
+    // (rows of one group of eight on one XCD: a 128-byte line of an operand holds eight rows)
+    const bool of_lhs = b < 0;
+    const int turn = (int)blockIdx.x >> 3, row0 = (turn / (8 / kLhsRows) * 8 + ((int)blockIdx.x & 7)) * 8 + turn % (8 / kLhsRows) * kLhsRows;
+    if (of_lhs && row0 >= lhs.m) return;
     const int col = slab + 4 * (tid & (kPieces - 1)), rows = qweight ? k >> 3 : 0, r0 = tid / kPieces, groups = k / group;
     const bool in_n = col < n;  // (N is a multiple of 8)
     uint16_t* const order = (uint16_t*)(smem + (size_t)rows * COLS * 4);
@@ -52,6 +102,13 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_permu
 
     auto load_words = [&]() __attribute__((always_inline)) {
         const uint32_t to = lds_address(smem) + wave * 1024;
+        if (of_lhs) {
+            const uint8_t* const from = (const uint8_t*)lhs.a + (int64_t)row0 * k * sizeof(AT);
+            const int bytes = min(kLhsRows, lhs.m - row0) * k * (int)sizeof(AT);
+            for (int i = 0; i * (kThreads * 16) < bytes; i++)
+                if (i * (kThreads * 16) + tid * 16 < bytes) load16_to_lds(from + i * (kThreads * 16) + tid * 16, to + i * (kThreads * 16));
+            return;
+        }
         const uint32_t* const from = qweight + (in_n ? col : 0);
         for (int i = 0; i * kRows < rows; i++)
             if (i * kRows + r0 < rows) load16_to_lds(from + (int64_t)(i * kRows + r0) * n, to + i * (kThreads * 16));
@@ -127,20 +184,46 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_permu
         __syncthreads();
         if (b == 0) {
             if (tid == 0) *uneven = as_is;
-            for (int i = tid; i < k; i += kThreads) source[i] = order[i];
+            if (source)
+                for (int i = tid; i < k; i += kThreads) source[i] = order[i];
         }
+    }
+    auto sources = [&](int r) __attribute__((always_inline)) {  // of sorted columns 8 r .. 8 r + 7
+        if constexpr (TURNS == 0) {
+            const go_u4 s0 = *(const go_u4*)(source + 8 * r), s1 = *(const go_u4*)(source + 8 * r + 4);
+            return go_u4{s0.x | s0.y << 16, s0.z | s0.w << 16, s1.x | s1.y << 16, s1.z | s1.w << 16};
+        } else {
+            return *(const go_u4*)(order + 8 * r);
+        }
+    };
+    if (of_lhs) {
+        const int row = row0 + wave / kRowWaves, pieces = k >> 3, steps = (k + 255) / 256 * 16;
+        if (row >= lhs.m) return;
+        const AT* const x = (const AT*)smem + wave / kRowWaves * k;
+        float v[8], inv;
+        const float scale = row_scale(wave_largest(x, k, lane), kRowTop, inv);
+        if (wave % kRowWaves == 0 && lane == 0) lhs.inv[row] = inv;
+        for (int pc = wave % kRowWaves * 64 + lane; pc < 2 * steps; pc += 64 * kRowWaves) {  // (zeros up to a whole unit)
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = 0.0f;
+            if (pc < pieces) {
+                const go_u4 s = sources(pc);
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const AT y = x[(j & 1) ? s[j >> 1] >> 16 : s[j >> 1] & 0xffffu];
+                    if constexpr (sizeof(AT) == 4) v[j] = y;
+                    else v[j] = __uint_as_float((uint32_t)y << 16);
+                }
+            }
+            store_piece<AT, kOrderGptq>(lhs.a16, steps, row, pc, scale, v);
+        }
+        return;
     }
     if (!in_n) return;
     const uint8_t* const words = smem + 16 * (tid & (kPieces - 1));
 #pragma unroll 2
     for (int r = r0; r < rows; r += kRows) {
-        go_u4 s;
-        if constexpr (TURNS == 0) {
-            const go_u4 s0 = *(const go_u4*)(source + 8 * r), s1 = *(const go_u4*)(source + 8 * r + 4);
-            s = go_u4{s0.x | s0.y << 16, s0.z | s0.w << 16, s1.x | s1.y << 16, s1.z | s1.w << 16};
-        } else {
-            s = *(const go_u4*)(order + 8 * r);
-        }
+        const go_u4 s = sources(r);
         go_u4 o = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -189,7 +272,8 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     return look_up > std::min(11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w, 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0));
 }
 
-hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int64_t n, int64_t k, int group, const GptqOrderSpace& p, hipStream_t s) {
+hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int group, const void* a, int lhs_dtype, int64_t m, const DirectSpace& p, const DirectMats& zero,
+                             int64_t zeros, bool& lhs_done, hipStream_t s) {
     const int groups = (int)(k / group);
     int bits = 0;
     while ((1 << bits) < groups) bits++;
@@ -207,19 +291,37 @@ hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int6
                             (2 * (words(cols) + sort_lds) > kLdsPerCu && n > (int64_t)(cols == 32 ? 48 : cols) * compute_units());
     if (sort_apart) cols = k <= 5120 ? 32 : k <= 20480 ? 16 : 8;  // (32 up to where two fit, 28672 x 5120 32 / 16 columns 78.5 / 80.4; 16 up to where one does, 14336 x 20480 16 / 8 165 / 175)
     const unsigned per_xcd = (unsigned)((n + 8 * cols - 1) / (8 * cols));
+    // The lhs in the same launch where none of its workgroups sorts or the slabs' last round has room for them; otherwise the caller's preparation reads its rows in the order left in memory.
+    // us, that way / in the same launch nevertheless: 4096 x 14336 400 rows (one workgroup a compute unit) 97 / 105, 4096 x 4096 2000 rows 86.2 / 86.5, 4000 157.5 / 158.5.
+    const bool f32 = lhs_dtype == QMM_F32;
+    const OrderLhs none{};
+    const OrderLhs lhs{a, p.a16, p.inv, (int)m, (int)((m + 63) / 64 * 64 / lhs_rows(cols, f32 ? 4 : 2)), (int)(std::min<int64_t>(1024, (zeros + 4095) / 4096) + 7) / 8 * 8, zero};
+    const int64_t at_once = compute_units() * (k <= 8192 && 2 * (words(cols) + sort_lds) <= kLdsPerCu ? 2 : 1), slabs = (n + cols - 1) / cols;
+    lhs_done = sort_apart || (slabs + lhs.workgroups + at_once - 1) / at_once == (slabs + at_once - 1) / at_once;
+    int32_t* const source = sort_apart || !lhs_done ? order.space.source : nullptr;
     hipError_t e;
-#define QMM_GO(COLS, TURNS, WORDS, GRID, LDS)                                                                                                       \
-    do {                                                                                                                                            \
-        if ((e = allow_full_lds<gptq_order_permute_kernel<COLS, TURNS>>()) != hipSuccess) return e;                                                 \
-        gptq_order_permute_kernel<COLS, TURNS><<<dim3(GRID), dim3(kThreads), LDS, s>>>(WORDS, g_idx, (int)n, (int)k, group, bits, (int)per_xcd,     \
-                                                                                       p.source, p.uneven, p.qweight);                              \
+#define QMM_GO(AT, COLS, TURNS, WORDS, GRID, LDS, LHS)                                                                                                                  \
+    do {                                                                                                                                                                \
+        if ((e = allow_full_lds<gptq_order_kernel<AT, COLS, TURNS>>()) != hipSuccess) return e;                                                                         \
+        gptq_order_kernel<AT, COLS, TURNS><<<dim3(GRID), dim3(kThreads), LDS, s>>>(WORDS, order.g_idx, (int)n, (int)k, group, bits, (int)per_xcd, source,               \
+                                                                                   order.space.uneven, order.space.qweight, LHS);                                       \
     } while (0)
-#define QMM_GO_WORDS(COLS, TURNS) QMM_GO(COLS, TURNS, qweight, 8 * per_xcd, words(COLS) + sort_lds)
+#define QMM_GO_LHS(COLS, TURNS, LDS)                                                                                                 \
+    do {                                                                                                                                    \
+        const unsigned grid = 8 * per_xcd + (unsigned)(lhs.workgroups + lhs.zeroing);                                                             \
+        if (f32) QMM_GO(float, COLS, TURNS, order.qweight, grid, LDS, lhs);                                                                 \
+        else QMM_GO(uint16_t, COLS, TURNS, order.qweight, grid, LDS, lhs);                                                                  \
+    } while (0)
+#define QMM_GO_WORDS(COLS, TURNS)                                                                            \
+    do {                                                                                                     \
+        if (lhs_done) QMM_GO_LHS(COLS, TURNS, words(COLS) + sort_lds);                                       \
+        else QMM_GO(uint16_t, COLS, TURNS, order.qweight, 8 * per_xcd, words(COLS) + sort_lds, none);        \
+    } while (0)
     if (sort_apart) {
-        QMM_GO(8, 32, nullptr, 1, sort_lds);
-        if (cols == 32) QMM_GO(32, 0, qweight, 8 * per_xcd, words(32));
-        else if (cols == 16) QMM_GO(16, 0, qweight, 8 * per_xcd, words(16));
-        else QMM_GO(8, 0, qweight, 8 * per_xcd, words(8));
+        QMM_GO(uint16_t, 8, 32, nullptr, 1, sort_lds, none);
+        if (cols == 32) QMM_GO_LHS(32, 0, words(32));
+        else if (cols == 16) QMM_GO_LHS(16, 0, words(16));
+        else QMM_GO_LHS(8, 0, words(8));
     } else if (cols == 32) {  // (fits up to K = 9100)
         if (k <= 4096) QMM_GO_WORDS(32, 4);
         else if (k <= 8192) QMM_GO_WORDS(32, 8);
@@ -235,6 +337,7 @@ hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int6
         else QMM_GO_WORDS(8, 32);
     }
 #undef QMM_GO_WORDS
+#undef QMM_GO_LHS
 #undef QMM_GO
     return hipGetLastError();
 }

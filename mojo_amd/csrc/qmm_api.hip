@@ -642,14 +642,12 @@ static int matmul_f32(int encoding, const qmm_gptq_config* cfg, const void* lhs,
                 return fail(QMM_ERR_INVALID, "qmm_matmul: GPTQ desc_act=True needs rhs[3] = g_idx int32[K]");
             const int32_t* only_if = nullptr;
             if (order_serves(cfg, lhs_dtype, m, n, k, flags, workspace, workspace_bytes)) {
-                const qmm::GptqOrderSpace p = qmm::gptq_order_space(workspace, n, k);
-                hipError_t e = qmm::launch_gptq_order((const uint32_t*)rhs[0], (const int32_t*)rhs[3], n, k, cfg->group_size, p, s);
-                if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, sort)");
-                const void* sorted[1] = {p.qweight};
-                e = qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, sorted, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], cfg->group_size, m, k,
-                                            nullptr, (char*)workspace + p.bytes, s, true, p.source);
+                const qmm::GptqOrder order{(const uint32_t*)rhs[0], (const int32_t*)rhs[3], qmm::gptq_order_space(workspace, n, k)};
+                const void* sorted[1] = {order.space.qweight};
+                const hipError_t e = qmm::launch_gemm_direct(encoding, lhs, lhs_dtype, 1, sorted, &n, &out, (const uint16_t*)rhs[1], (const uint32_t*)rhs[2], cfg->group_size, m, k,
+                                                             nullptr, (char*)workspace + order.space.bytes, s, true, &order);
                 if (e != hipSuccess) return hip_status(e, "qmm_matmul(GPTQ act-order, direct GEMM)");
-                only_if = p.uneven;
+                only_if = order.space.uneven;
             }
             hipError_t e = qmm::launch_gemv_gptq_act_order(lhs, lhs_dtype, (const uint32_t*)rhs[0], (const uint16_t*)rhs[1], (const uint32_t*)rhs[2],
                                                            (const int32_t*)rhs[3], (int)m, n, k, cfg->group_size, out, n, s, only_if);

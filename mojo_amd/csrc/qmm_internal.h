@@ -22,17 +22,31 @@ bool twin_rows_allowed();
 // compute units of the current device (asked for once; 256 where there is none)
 int compute_units();
 
+// gptq_order.hip: the columns of an act-order matrix and of the lhs sorted by group into the workspace.  `uneven` is set where the groups are not of
+// group_size columns each: the sorted forms are then of no use, and the look-up kernel above (only_if = uneven) has to follow the product.
+struct GptqOrderSpace {
+    int32_t* uneven;
+    int32_t* source;
+    uint32_t* qweight;
+    int64_t bytes;
+};
+struct GptqOrder {
+    const uint32_t* qweight;
+    const int32_t* g_idx;
+    GptqOrderSpace space;
+};
+
 // gemm_direct.hip: a few to a few hundred lhs rows, more where the staged kernel pays, every encoding; out16 != null: bf16 results (out is then unused).
 // w: the weights, where they are known: beyond some rows the answer rests on the staged kernel, which does not take every alignment (null: any).
 // any_rows: called with more rows than gemm_direct_wanted says, held to the error of the direct and shared kernels all the same.
-// source (GPTQ, K a multiple of 32): column p of the weights is column source[p] of the lhs.
+// order (GPTQ, K a multiple of 32, one matrix): the weights are those of order->space, made here from an act-order matrix.
 bool gemm_direct_wanted(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group, const void* w);
 bool gemm_direct_takes_staged(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);  // which of its kernels a call that it serves goes to
 int64_t gemm_direct_workspace_bytes(int encoding, int lhs_dtype, int64_t m, int64_t k);
 constexpr int kDirectMaxMats = 4;  // count: matrices that share the lhs (out16: one)
 hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int count, const void* const* ws, const int64_t* ns, float* const* outs,
                               const uint16_t* scales, const uint32_t* qzeros, int group, int64_t m, int64_t k, uint16_t* out16, void* workspace,
-                              hipStream_t s, bool any_rows = false, const int32_t* source = nullptr);
+                              hipStream_t s, bool any_rows = false, const GptqOrder* order = nullptr);
 
 hipError_t launch_read_probe(const void* buf, int64_t bytes, hipStream_t s);
 // register-resident matrix-core loop (probes.hip): `workgroups` workgroups of 8 wavefronts, out fp32 [workgroups * 512]
@@ -180,18 +194,9 @@ hipError_t launch_gemv_gptq_act_order(const void* a, int a_dtype, const uint32_t
                                       const uint32_t* qzeros, const int32_t* g_idx, int m, int64_t n, int64_t k, int group,
                                       float* out, int64_t ldo, hipStream_t s, const int32_t* only_if = nullptr);
 
-// gptq_order.hip: the columns of an act-order matrix and of the lhs sorted by group into the workspace.  `uneven` is set where the groups are not of
-// group_size columns each: the sorted forms are then of no use, and the look-up kernel above (only_if = uneven) has to follow the product.
-struct GptqOrderSpace {
-    int32_t* uneven;
-    int32_t* source;
-    uint32_t* qweight;
-    int64_t bytes;
-};
 GptqOrderSpace gptq_order_space(void* workspace, int64_t n, int64_t k);
 bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group);
 bool gptq_act_order_table_fits(int64_t m, int64_t k, int group);  // the look-up kernel's scales in LDS
-hipError_t launch_gptq_order(const uint32_t* qweight, const int32_t* g_idx, int64_t n, int64_t k, int group, const GptqOrderSpace& p, hipStream_t s);
 bool gemv_q4_k_kc_supported(const void* w, int64_t k);
 int64_t gemv_q4_k_kc_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemv_q4_k_kc(const void* a, int a_dtype, const uint8_t* w, int m, int64_t n, int64_t k, float* out,

@@ -161,3 +161,29 @@ def test_qweight_at_any_multiple_of_four(n, k, words):
     got = qmatmul(QE.GPTQ, config, a, moved, *rhs[1:])
     check(got, config, rhs, a, sorted_columns=True)
     assert torch.equal(got, qmatmul(QE.GPTQ, config, a, *rhs))
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(33, 8200, 4096), (41, 8200, 4128),  # slabs of 32 columns: 8 bf16 rows of the lhs a workgroup, 4 of fp32
+                                   (23, 4104, 4096), (21, 4104, 14336),  # of 16: 4 and 2
+                                   (35, 40, 4096), (22, 40, 26112),  # of 8: 2 and 1
+                                   (21, 2056, 20480), (23, 2056, 20608), (25, 12296, 4608),  # the sort as a launch of its own
+                                   (600, 1032, 2048), (300, 4104, 4128)])  # more rows than the last round of the slabs has room for: a preparation of their own
+def test_rows_of_the_lhs_beside_the_slabs(m, n, k, lhs):
+    """Rows whose largest value is anywhere, an infinity, none at all (zeros), tiny, and what is left of a workgroup's rows."""
+    config, rhs = act_order(n, k, 32, m)
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    a = torch.randn((m, k), device="cuda", generator=gen)
+    a[torch.arange(m), torch.randint(0, k, (m,), device="cuda", generator=gen)] = 300.0
+    a[2] = 0.0
+    a[3] *= 2.0**-100
+    a[m - 1, k - 1] = -1000.0
+    a = a.to(lhs)
+    broken = a.clone()
+    broken[5, 0], broken[6, k - 1], broken[11, k // 2] = float("inf"), float("-inf"), float("nan")
+    got = qmatmul(QE.GPTQ, config, broken, *rhs)
+    rows = [r for r in range(m) if r not in (5, 6, 11)]
+    check(got[rows], config, rhs, a[rows])
+    assert not torch.isfinite(got[[5, 6, 11]]).any()
+    assert torch.equal(got[2], torch.zeros_like(got[2]))
+    assert torch.equal(got[rows], qmatmul(QE.GPTQ, config, a, *rhs)[rows])
