@@ -2,12 +2,12 @@
 // groups serve the call.
 //
 // The kernel that looks the group of every k up (gemv_gptq.hip) passes over the weights once per four rows and multiplies on the vector
-// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 77 us.  Sorting costs one launch and one pass over the packed weights: a workgroup holds some
+// units: 14336 x 4096 with 400 bf16 rows took 2.4 ms, this way 75 us.  Sorting costs one launch and one pass over the packed weights: a workgroup holds some
 // columns of the output in LDS (all of K), sorts the columns of K by group while those are on their way, and takes the eight nibbles of every word of the sorted
 // matrix from there.  Workgroups of the same launch hold rows of the lhs there instead and leave the operands of the direct GEMM in the same order; where the launch has no room for them,
 // that GEMM's own preparation does.
-// What bounds the pass, at 14336 x 4096 (2 x 29 MB, 22 us with nothing in the caches, 2.6 TB/s): loads, sort (hidden behind them but for its start),
-// nibbles (two vector instructions each, about 6 us) and stores one after the other, since all workgroups run at once.
+// What bounds the pass, at 14336 x 4096 (2 x 29 MB and 400 rows of the lhs, 18 us in a trace with nothing in the caches, 3.6 TB/s): loads (the sort hides behind them but for its start), nibbles (about 2 us) and stores one
+// after the other, since all workgroups run at once.
 // us of the whole call with the sort as a launch of its own and a sorted copy of the lhs / this way, nothing in the caches: 14336 x 4096 400 rows 127 / 122, 8 rows 50 / 44;
 // 4096 x 14336 64 rows 76 / 63; 4096 x 4096 64 rows 37 / 30; 8192 x 8192 300 rows 130 / 123; 1024 x 4096 20 rows 29 / 22; 8192 x 28672 20 rows 184 / 174;
 // 3584 x 18944 33 rows 90 / 90.  With the lhs as a launch of its own / in the same one: 14336 x 4096 400 rows 81.5 / 77.6, 8 rows 36.5 / 32.9, 100 fp32 rows 56.7 / 52.0; 4096 x 4096
@@ -37,6 +37,9 @@ struct OrderLhs {
     float* inv;
     int m, workgroups, zeroing;  // multiples of 8
     DirectMats zero;
+};
+struct __attribute__((packed, aligned(4))) OrderWords {  // (qweight begins at any multiple of four)
+    go_u4 v;
 };
 constexpr int lhs_rows(int cols, int size) { return cols / (size == 4 ? 8 : 4); }  // of a workgroup: as many bytes as its words of the weights
 
@@ -68,11 +71,44 @@ __device__ __forceinline__ uint32_t wave_largest(const AT* x, int k, int lane) {
     return wave_max_nonneg_bits(mx);
 }
 
+// Eight words of eight nibbles: nibble j of word i and nibble i of word j change places.
+__device__ __forceinline__ void transpose_nibbles(uint32_t (&a)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t lo = a[i], hi = a[i + 4];
+        a[i] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        a[i + 4] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+    }
+#pragma unroll
+    for (int i = 0; i < 6; i += i == 1 ? 3 : 1) {
+        const uint32_t lo = a[i], hi = a[i + 2];
+        a[i] = __builtin_amdgcn_perm(hi, lo, 0x06020400u);
+        a[i + 2] = __builtin_amdgcn_perm(hi, lo, 0x07030501u);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const uint32_t lo = a[i], hi = a[i + 1];
+        a[i] = (lo & 0x0f0f0f0fu) | ((hi << 4) & 0xf0f0f0f0u);
+        a[i + 1] = ((lo >> 4) & 0x0f0f0f0fu) | (hi & 0xf0f0f0f0u);
+    }
+}
+// LDS holds, for every column of K, the nibbles of the slab's columns of N side by side.  Where column k lies, in such rows: the eight of a word are exchanged, so that the
+// wavefronts that write them use all banks.  Its own inverse.
+template <int COLS>
+__device__ __forceinline__ uint32_t place_of(uint32_t k) { return k ^ ((k >> (COLS == 32 ? 4 : COLS == 16 ? 5 : 6)) & 7u); }
+
+// How the nibbles are taken.  Turned: the words go through registers on their way to LDS and are transposed there, eight columns of K by eight of N; a word of the sorted matrix is then eight
+// dwords transposed back: 1.4 vector instructions a nibble, 3 where every nibble is shifted out of a word as it came (loads go straight to LDS then).  Against that, us of the whole call, as
+// they come / turned: 14336 x 4096 400 rows 77.6 / 74.6, 8 rows 32.9 / 31.1, 100 fp32 rows 52.0 / 48.0; 4096 x 4096 64 rows 24.3 / 23.6; 28672 x 8192 40 rows 107.0 / 100.9; 5120 x 20480 64
+// rows 90.6 / 87.9; 8192 x 8192 500 rows (32 columns, 128 registers) 96.9 / 92.7.  Not for slabs of 8 columns, whose loads would be 16 bytes a row and instruction (1024 x 4096 2000 rows 45.1 / 45.9,
+// 8192 x 28672 300 rows 271 / 280), and not with eight turns and two workgroups a compute unit: 64 registers do not hold the words beside the groups (8192 x 8192 with spills 98 / 104).
+constexpr bool order_turned(int cols, int turns) { return cols > 8 && turns != 8; }
+
 // Workgroup: COLS columns of the weights, neighbours on one XCD (they share cache lines).  It sorts for itself while its words are on their way to LDS: where the
 // sort was a launch of one workgroup it took 6.6 us at K = 4096 and 18 at 14336.
 // Stable sort (within a group the columns keep their order), wavefront w takes a sixteenth of K, TURNS times 64 columns; group indices outside [0, groups) are
 // clamped, as in the look-up kernel.  The first workgroup leaves the order (source[p]: the column of K at sorted position p) and the mark in memory.
-// LDS: [k / 8][COLS] words, uint16 [k] order, uint16 [kWaves][groups] counts.
+// LDS: [k / 8][COLS] words (turned: [k][COLS / 8], see place_of), uint16 [k] order, uint16 [kWaves][groups] counts.
 // Where that is more than a compute unit has (K beyond 26208, less with groups of 32 or 64), or leaves room for one workgroup and there are several for each compute unit: a launch of
 // one workgroup without words (qweight null) that only sorts, then TURNS = 0, which takes the order from memory.
 template <typename AT, int COLS, int TURNS>
@@ -81,7 +117,9 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
                                                                                   uint32_t* __restrict__ sorted_w, OrderLhs lhs) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int kPieces = COLS / 4, kRows = kThreads / kPieces;  // rows of words per turn
+    constexpr bool kTurned = order_turned(COLS, TURNS);
+    constexpr int kPieces = COLS / (kTurned ? 8 : 4), kRows = kThreads / kPieces;  // threads to a row of words, rows a turn
+    constexpr int kHeld = TURNS == 0 ? 2 : COLS == 32 && TURNS == 16 ? 5 : (TURNS * COLS + 63) / 64;  // turns of words in registers while the sort runs
     constexpr int kLhsRows = lhs_rows(COLS, sizeof(AT)), kRowWaves = kWaves / kLhsRows;
     const int b = (int)blockIdx.x - lhs.workgroups - lhs.zeroing, slab = ((b & 7) * per_xcd + (b >> 3)) * COLS;
     if (b >= 0 && slab >= n) return;
@@ -93,29 +131,62 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
     const bool of_lhs = b < 0;
     const int turn = (int)blockIdx.x >> 3, row0 = (turn / (8 / kLhsRows) * 8 + ((int)blockIdx.x & 7)) * 8 + turn % (8 / kLhsRows) * kLhsRows;
     if (of_lhs && row0 >= lhs.m) return;
-    const int col = slab + 4 * (tid & (kPieces - 1)), rows = qweight ? k >> 3 : 0, r0 = tid / kPieces, groups = k / group;
+    const int col = slab + (kTurned ? 8 : 4) * (tid & (kPieces - 1)), rows = qweight ? k >> 3 : 0, r0 = tid / kPieces, groups = k / group;
     const bool in_n = col < n;  // (N is a multiple of 8)
     uint16_t* const order = (uint16_t*)(smem + (size_t)rows * COLS * 4);
     uint16_t* const counts = order + k;
     uint32_t* const pairs = (uint32_t*)counts;  // (k is even)
     uint32_t* const bad = (uint32_t*)order;     // until the order is written
 
-    auto load_words = [&]() __attribute__((always_inline)) {
-        const uint32_t to = lds_address(smem) + wave * 1024;
-        if (of_lhs) {
-            const uint8_t* const from = (const uint8_t*)lhs.a + (int64_t)row0 * k * sizeof(AT);
-            const int bytes = min(kLhsRows, lhs.m - row0) * k * (int)sizeof(AT);
-            for (int i = 0; i * (kThreads * 16) < bytes; i++)
-                if (i * (kThreads * 16) + tid * 16 < bytes) load16_to_lds(from + i * (kThreads * 16) + tid * 16, to + i * (kThreads * 16));
-            return;
+    auto place = [&](uint32_t src) __attribute__((always_inline)) { return kTurned && !of_lhs ? place_of<COLS>(src) : src; };
+    uint32_t* const nibbles = (uint32_t*)smem + (tid & (kPieces - 1));
+    OrderWords held[kHeld][2];
+    auto load_words = [&](int turn0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++) {
+            const uint32_t* const from = qweight + (int64_t)min((turn0 + i) * kRows + r0, rows - 1) * n + min(col, n - 8);
+            held[i][0] = *(const OrderWords*)from;
+            held[i][1] = *(const OrderWords*)(from + 4);
         }
-        const uint32_t* const from = qweight + (in_n ? col : 0);
-        for (int i = 0; i * kRows < rows; i++)
-            if (i * kRows + r0 < rows) load16_to_lds(from + (int64_t)(i * kRows + r0) * n, to + i * (kThreads * 16));
+    };
+    auto spread_words = [&](int turn0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++) {
+            const int r = (turn0 + i) * kRows + r0;
+            if (r < rows) {
+                uint32_t a[8];
+#pragma unroll
+                for (int c = 0; c < 4; c++) a[c] = held[i][0].v[c], a[4 + c] = held[i][1].v[c];
+                transpose_nibbles(a);
+                const uint32_t mixed = place_of<COLS>(8 * r) & 7u;
+#pragma unroll
+                for (int c = 0; c < 8; c++) nibbles[(8 * r + (c ^ mixed)) * kPieces] = a[c];
+            }
+        }
+    };
+    auto load_16s = [&](const uint8_t* from, int bytes) __attribute__((always_inline)) {  // (of the lhs)
+        for (int i = 0; i * (kThreads * 16) < bytes; i++)
+            if (i * (kThreads * 16) + tid * 16 < bytes) load16_to_lds(from + i * (kThreads * 16) + tid * 16, lds_address(smem) + wave * 1024 + i * (kThreads * 16));
+    };
+    auto load_lds = [&]() __attribute__((always_inline)) {
+        if (of_lhs) {
+            load_16s((const uint8_t*)lhs.a + (int64_t)row0 * k * sizeof(AT), min(kLhsRows, lhs.m - row0) * k * (int)sizeof(AT));
+        } else if constexpr (!kTurned) {
+            const uint32_t* const from = qweight + (in_n ? col : 0);
+            for (int i = 0; i * kRows < rows; i++)
+                if (i * kRows + r0 < rows) load16_to_lds(from + (int64_t)(i * kRows + r0) * n, lds_address(smem) + wave * 1024 + i * (kThreads * 16));
+        }
     };
     if constexpr (TURNS == 0) {
-        load_words();
-        wait_vmcnt<0>();
+        if (of_lhs || !kTurned) {
+            load_lds();
+            wait_vmcnt<0>();
+        } else {
+            for (int turn = 0; turn * kRows < rows; turn += kHeld) {
+                load_words(turn);
+                spread_words(turn);
+            }
+        }
         __syncthreads();
     } else {
         // (asked for before the words: a wait for these would be one for everything asked for earlier)
@@ -130,7 +201,8 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
             g[t] = min(max(g[t], 0), groups - 1);
             tie(g[t]);
         }
-        load_words();
+        if (of_lhs || !kTurned) load_lds();
+        else load_words(0);
 
         const int turns = min(per, max(0, k - lo));  // columns of this wavefront
         __syncthreads();
@@ -156,7 +228,7 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
         const bool as_is = *bad != 0;
         __syncthreads();
         if (as_is) {
-            for (int i = tid; i < k; i += kThreads) order[i] = (uint16_t)i;
+            for (int i = tid; i < k; i += kThreads) order[i] = (uint16_t)place(i);
         } else {
             uint16_t* const mine = counts + wave * groups;
     #pragma unroll
@@ -172,7 +244,7 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
                 const int rank = __popcll(same & ((1ull << lane) - 1)), count = __popcll(same);
                 if (live) {
                     const uint32_t at = mine[g[t]];
-                    order[g[t] * group + (int)at + rank] = (uint16_t)(lo + 64 * t + lane);
+                    order[g[t] * group + (int)at + rank] = (uint16_t)place(lo + 64 * t + lane);
                     if (rank == count - 1) mine[g[t]] = (uint16_t)(at + (uint32_t)count);
                 }
                 // (the next turn of this wavefront reads what its lanes wrote: LDS operations of a wavefront are performed in order)
@@ -180,12 +252,13 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
                 __builtin_amdgcn_wave_barrier();
             }
         }
-        wait_vmcnt<0>();
+        if (of_lhs || !kTurned) wait_vmcnt<0>();
+        else spread_words(0);
         __syncthreads();
         if (b == 0) {
             if (tid == 0) *uneven = as_is;
             if (source)
-                for (int i = tid; i < k; i += kThreads) source[i] = order[i];
+                for (int i = tid; i < k; i += kThreads) source[i] = (int32_t)place(order[i]);
         }
     }
     auto sources = [&](int r) __attribute__((always_inline)) {  // of sorted columns 8 r .. 8 r + 7
@@ -220,19 +293,31 @@ __global__ __launch_bounds__(kThreads, TURNS <= 8 ? 8 : 4) void gptq_order_kerne
         return;
     }
     if (!in_n) return;
-    const uint8_t* const words = smem + 16 * (tid & (kPieces - 1));
 #pragma unroll 2
     for (int r = r0; r < rows; r += kRows) {
         const go_u4 s = sources(r);
-        go_u4 o = {0u, 0u, 0u, 0u};
+        go_u4* const to = (go_u4*)(sorted_w + (int64_t)r * n + col);
+        if constexpr (kTurned) {
+            uint32_t a[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const uint32_t src = (j & 1) ? s[j >> 1] >> 16 : s[j >> 1] & 0xffffu;
-            const go_u4 x = *(const go_u4*)(words + (src >> 3) * (COLS * 4));
+            for (int j = 0; j < 8; j++) {
+                const uint32_t src = (j & 1) ? s[j >> 1] >> 16 : s[j >> 1] & 0xffffu;
+                a[j] = nibbles[(TURNS == 0 ? place(src) : src) * kPieces];
+            }
+            transpose_nibbles(a);
+            to[0] = go_u4{a[0], a[1], a[2], a[3]};
+            to[1] = go_u4{a[4], a[5], a[6], a[7]};
+        } else {
+            go_u4 o = {0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_alignbit(x[c] >> ((src << 2) & 31u), o[c], 4);
+            for (int j = 0; j < 8; j++) {
+                const uint32_t src = (j & 1) ? s[j >> 1] >> 16 : s[j >> 1] & 0xffffu;
+                const go_u4 x = *(const go_u4*)(smem + 16 * (tid & (kPieces - 1)) + (src >> 3) * (COLS * 4));
+#pragma unroll
+                for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_alignbit(x[c] >> ((src << 2) & 31u), o[c], 4);
+            }
+            to[0] = o;
         }
-        *(go_u4*)(sorted_w + (int64_t)r * n + col) = o;
     }
 }
 
@@ -324,7 +409,7 @@ hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int g
         else QMM_GO_LHS(8, 0, words(8));
     } else if (cols == 32) {  // (fits up to K = 9100)
         if (k <= 4096) QMM_GO_WORDS(32, 4);
-        else if (k <= 8192) QMM_GO_WORDS(32, 8);
+        else if (2 * (words(32) + sort_lds) <= kLdsPerCu) QMM_GO_WORDS(32, 8);
         else QMM_GO_WORDS(32, 16);
     } else if (cols == 16) {  // (up to K = 16380)
         if (k <= 4096) QMM_GO_WORDS(16, 4);

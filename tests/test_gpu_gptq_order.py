@@ -167,6 +167,7 @@ def test_qweight_at_any_multiple_of_four(n, k, words):
 @pytest.mark.parametrize("m,n,k", [(33, 8200, 4096), (41, 8200, 4128),  # slabs of 32 columns: 8 bf16 rows of the lhs a workgroup, 4 of fp32
                                    (23, 4104, 4096), (21, 4104, 14336),  # of 16: 4 and 2
                                    (35, 40, 4096), (22, 40, 26112),  # of 8: 2 and 1
+                                   (33, 8200, 160), (23, 4104, 2080), (21, 4104, 4512),  # rows of words that fill part of a turn
                                    (21, 2056, 20480), (23, 2056, 20608), (25, 12296, 4608),  # the sort as a launch of its own
                                    (600, 1032, 2048), (300, 4104, 4128)])  # more rows than the last round of the slabs has room for: a preparation of their own
 def test_rows_of_the_lhs_beside_the_slabs(m, n, k, lhs):
