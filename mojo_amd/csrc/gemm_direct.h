@@ -108,29 +108,51 @@ constexpr int kRowTop = 14, kRowTopWithSums = 9;
 //   32 blk + 16 g + 8 a + slot order   (kOrderK: slots 0,2,1,3,4,6,5,7; kOrderGptq: 0,4,1,5,2,6,3,7)
 constexpr int kOrderK = 0, kOrderGptq = 1;  // (Q4_0: 32 blk + 16 a + 8 g + the slots of kOrderK)
 
-// Eight columns of a row.
+// Eight columns of a row as they lie in memory.
 template <typename AT>
-__device__ __forceinline__ void load8(const AT* p, float (&v)[8]) {
-    if constexpr (sizeof(AT) == 4) {
-        const float4 x = *(const float4*)p, y = *(const float4*)(p + 4);
-        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-        v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
-    } else {
-        const uint4 x = *(const uint4*)p;
-        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+struct LhsPiece {
+    gd_u4 raw[sizeof(AT) / 2];
+};
+template <typename AT>
+__device__ __forceinline__ LhsPiece<AT> load_piece(const AT* p) {
+    LhsPiece<AT> x;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[2 * i] = __uint_as_float(w[i] << 16);
-            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-        }
+    for (int i = 0; i < (int)sizeof(AT) / 2; i++) x.raw[i] = ((const gd_u4*)p)[i];
+    return x;
+}
+template <typename AT>
+__device__ __forceinline__ void unpack_piece(const LhsPiece<AT>& x, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        if constexpr (sizeof(AT) == 4) v[i] = __uint_as_float(x.raw[i >> 2][i & 3]);
+        else v[i] = __uint_as_float((i & 1) ? x.raw[0][i >> 1] & 0xffff0000u : x.raw[0][i >> 1] << 16);
     }
 }
-// Their largest magnitude, of the finite ones.
-__device__ __forceinline__ float largest(float mx, const float (&v)[8]) {
+// Their largest magnitude, on the bits: two vector instructions a dword, where a comparison that leaves out what is not finite takes five.  (bf16: the low and the high halves apart, until largest_of.)
+template <typename AT>
+__device__ __forceinline__ uint32_t largest_bits(uint32_t top, const LhsPiece<AT>& x) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(AT) / 2; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if constexpr (sizeof(AT) == 4) top = max(top, x.raw[i][j] & 0x7fffffffu);
+            else top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top), __builtin_bit_cast(u16x2, x.raw[i][j] & 0x7fff7fffu)));
+        }
+    return top;
+}
+template <typename AT>
+__device__ __forceinline__ float largest_of(uint32_t top) { return __uint_as_float(sizeof(AT) == 4 ? top : max(top & 0xffff0000u, top << 16)); }
+// Of the finite ones: for wavefronts in which largest_of is none.
+template <typename AT>
+__device__ __forceinline__ float largest_finite(float mx, const LhsPiece<AT>& x) {
+    float v[8];
+    unpack_piece(x, v);
 #pragma unroll
     for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]) <= 3.402823466e38f ? fabsf(v[i]) : 0.0f);
     return mx;
 }
+__device__ __forceinline__ bool any_not_finite(float mx) { return __any(__float_as_uint(mx) >= 0x7f800000u); }
 // What a row is multiplied by, and its inverse, from the bits of its largest magnitude.
 __device__ __forceinline__ float row_scale(uint32_t largest_bits, int row_top, float& inv) {
     int e = (int)((largest_bits >> 23) & 0xffu) - 127;
@@ -138,30 +160,36 @@ __device__ __forceinline__ float row_scale(uint32_t largest_bits, int row_top, f
     inv = __uint_as_float((uint32_t)(127 - row_top + e) << 23);
     return __uint_as_float((uint32_t)(127 + row_top - e) << 23);
 }
+// Two values as fp16, one instruction.
+__device__ __forceinline__ uint32_t narrow2(float x, float y) {
+    typedef float float2v __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v{x, y}), half2v));
+}
 // Piece pc (eight columns) of a row, scaled by s (v is left so), as its part of the operands.
 template <typename AT, int ORDER>
 __device__ __forceinline__ void store_piece(_Float16* a16, int steps, int row, int pc, float s, float (&v)[8]) {
     constexpr bool kF32 = sizeof(AT) == 4;
     constexpr int perm[2][8] = {{0, 2, 1, 3, 4, 6, 5, 7}, {0, 4, 1, 5, 2, 6, 3, 7}};
     const int blk = pc >> 2, g = (pc >> 1) & 1, step = 2 * blk + (pc & 1);
-    float h[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] *= s;
+    HalfPack hi;
 #pragma unroll
-    for (int i = 0; i < 8; i++) h[i] = h2f(f2h(v[i]));
-    gd_u4 hi;
-#pragma unroll
-    for (int i = 0; i < 4; i++) hi[i] = pack_half2(h[perm[ORDER][2 * i]], h[perm[ORDER][2 * i + 1]]);
-    _Float16* at = a16 + ((int64_t)(row >> 5) * steps + step) * (kF32 ? 1024 : 512) + ((row & 31) + 32 * g) * 8;
-    *(gd_u4*)at = hi;
+    for (int i = 0; i < 4; i++) hi.u[i] = narrow2(v[perm[ORDER][2 * i]], v[perm[ORDER][2 * i + 1]]);
+    const uint32_t at = (uint32_t)step * (kF32 ? 2048u : 1024u) + (uint32_t)((row & 31) + 32 * g) * 16u;  // (below 2^23)
+    uint8_t* const tile = (uint8_t*)a16 + (int64_t)(row >> 5) * steps * (kF32 ? 2048 : 1024);
+    *(half8*)(tile + at) = hi.h;
     if constexpr (kF32) {
-        gd_u4 lo;
+        HalfPack lo;
         float residual[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) residual[i] = fabsf(h[i]) <= 65504.0f ? v[i] - h[i] : 0.0f;  // (an infinity has no residual: inf - inf)
+        for (int i = 0; i < 8; i++) {
+            const float h = (float)hi.h[i], x = v[perm[ORDER][i]];
+            residual[i] = fabsf(h) <= 65504.0f ? x - h : 0.0f;  // (an infinity has no residual: inf - inf)
+        }
 #pragma unroll
-        for (int i = 0; i < 4; i++) lo[i] = pack_half2(residual[perm[ORDER][2 * i]], residual[perm[ORDER][2 * i + 1]]);
-        *(gd_u4*)(at + 512) = lo;
+        for (int i = 0; i < 4; i++) lo.u[i] = narrow2(residual[2 * i], residual[2 * i + 1]);
+        *(half8*)(tile + at + 1024) = lo.h;
     }
 }
 // The e-th of `count` workgroups zeroes its part of the results (m rows).

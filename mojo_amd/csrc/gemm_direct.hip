@@ -47,8 +47,9 @@ DirectSpace direct_space(void* ws, bool f32, bool with_sums, bool with_sums32, i
 // preparation: one workgroup per lhs row (the first m workgroups), then zeroing of `out` for two workgroups per tile
 // ---------------------------------------------------------------------------------------------------------------------------
 // With few rows the latency of a row's passes (load, maximum, narrow, store) bounds it: as many threads as leave each one or two pieces of eight
-// columns (200 x 14336 bf16 rows with 256 threads a row 10.1 us, with 1024 7.2); with many, that a row writes 16 bytes of a 128-byte line, the rest
-// of which other workgroups of the XCD fill (500 x 14336: 11.5 us for 28 MB, whatever the number of threads).
+// columns (200 x 14336 bf16 rows with 256 threads a row 10.1 us, with 1024 7.2), all of which are asked for before the first is looked at; with many, that a row writes 16 bytes of a
+// 128-byte line, the rest of which other workgroups of the XCD fill.  us in a trace, the pieces widened to fp32 as they arrive (a wait after each) and compared as such / kept as they are:
+// 500 x 14336 bf16 rows 13.8 / 11.7 (28 MB), 200 x 14336 7.6 / 7.1; of calls, Q4_K 4096 x 14336 200 rows 47.0 / 46.4, 4096 x 28672 40 fp32 rows 57.3 / 56.3, 512 x 2048 24 fp32 rows 9.7 / 8.6.
 // Rows of one group of eight go to workgroups of one XCD (ids congruent mod 8): a 128-byte line of an operand holds eight rows.
 // SORTED: column p of the operands is column source[p] of the row, which lies in LDS (k values) meanwhile.
 template <typename AT, int ORDER, bool SORTED = false>
@@ -67,46 +68,49 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
     const int pieces = k >> 3;  // of eight columns, one per thread and turn
     const int steps = (k + 255) / 256 * 16;
     constexpr int kHeld = 4;    // rows of up to 32768 columns (1024 threads) stay in registers between the search for the maximum and the narrowing
-    float held[kHeld][8];
-    const bool hold = pieces <= kHeld * threads;
+    LhsPiece<AT> held[kHeld];   // (as they came: a conversion after each load would wait for it before the next is asked for)
+    const int turns = (pieces + threads - 1) / threads;
     if constexpr (SORTED) {
         constexpr int kPer = 16 / sizeof(AT);
         for (int i = tid * kPer; i < k; i += threads * kPer) *(gd_u4*)((AT*)row_lds + i) = *(const gd_u4*)(ar + i);
         __syncthreads();
     }
-    auto load = [&](int pc, float (&v)[8]) __attribute__((always_inline)) {
+    auto load = [&](int pc) __attribute__((always_inline)) {
         if constexpr (SORTED) {
             const int4 s0 = *(const int4*)(source + 8 * pc), s1 = *(const int4*)(source + 8 * pc + 4);
             const int from[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+            LhsPiece<AT> x;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                if constexpr (sizeof(AT) == 4) v[i] = ((const float*)row_lds)[from[i]];
-                else v[i] = __uint_as_float((uint32_t)((const uint16_t*)row_lds)[from[i]] << 16);
+                if constexpr (sizeof(AT) == 4) x.raw[i >> 2][i & 3] = ((const uint32_t*)row_lds)[from[i]];
+                else if (i & 1) x.raw[0][i >> 1] |= (uint32_t)((const uint16_t*)row_lds)[from[i]] << 16;
+                else x.raw[0][i >> 1] = ((const uint16_t*)row_lds)[from[i]];
             }
+            return x;
         } else {
-            load8(ar + pc * 8, v);
+            return load_piece(ar + pc * 8);
         }
     };
-    float mx = 0.0f;
-    if (hold) {
+    uint32_t top = 0;
+    if (turns <= kHeld) {
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * threads < pieces) load(tid + i * threads, held[i]);
+            if (i < turns) held[i] = load(min(tid + i * threads, pieces - 1));
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * threads < pieces) mx = largest(mx, held[i]);
+            if (i < turns) top = largest_bits(top, held[i]);
     } else {
-        for (int pc = tid; pc < pieces; pc += threads) {
-            float v[8];
-            load(pc, v);
-            mx = largest(mx, v);
-        }
+        for (int pc = tid; pc < pieces; pc += threads) top = largest_bits(top, load(pc));
+    }
+    float mx = largest_of<AT>(top);
+    if (any_not_finite(mx)) {
+        mx = 0.0f;
+        for (int pc = tid; pc < pieces; pc += threads) mx = largest_finite(mx, load(pc));
     }
     const uint32_t mb = wave_max_nonneg_bits(mx);
     if ((tid & 63) == 0) wmax[tid >> 6] = mb;
     __syncthreads();
-    uint32_t mxb = 0;
-    for (int i = 0; i < threads >> 6; i++) mxb = max(mxb, wmax[i]);
+    const uint32_t mxb = wave_max_nonneg_bits(__uint_as_float((tid & 63) < threads >> 6 ? wmax[tid & 63] : 0u));
     float inv;
     const float s = row_scale(mxb, with_sums ? kRowTopWithSums : kRowTop, inv);
     if (tid == 0) p.inv[row] = inv;
@@ -133,16 +137,17 @@ __global__ __launch_bounds__(1024) void direct_prep_kernel(const AT* __restrict_
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         emit(pc, v);
     }
-    if (hold) {
+    auto emit_piece = [&](int pc, const LhsPiece<AT>& x) __attribute__((always_inline)) {
+        float v[8];
+        unpack_piece(x, v);
+        emit(pc, v);
+    };
+    if (turns <= kHeld) {
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (tid + i * threads < pieces) emit(tid + i * threads, held[i]);
+            if (tid + i * threads < pieces) emit_piece(tid + i * threads, held[i]);
     } else {
-        for (int pc = tid; pc < pieces; pc += threads) {
-            float v[8];
-            load(pc, v);
-            emit(pc, v);
-        }
+        for (int pc = tid; pc < pieces; pc += threads) emit_piece(pc, load(pc));
     }
 }
 
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(1024) void direct_prep_q8_kernel(const AT* __restri
     for (int pc = tid; pc < units * 32; pc += threads) {
         const int blk = pc >> 2, sub = pc & 3, g = sub & 1, step = 2 * blk + (sub >> 1);
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (pc < pieces) load8(ar + pc * 8, v);
+        if (pc < pieces) unpack_piece(load_piece(ar + pc * 8), v);
         float mx = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]));

@@ -43,30 +43,15 @@ struct __attribute__((packed, aligned(4))) OrderWords {  // (qweight begins at a
 };
 constexpr int lhs_rows(int cols, int size) { return cols / (size == 4 ? 8 : 4); }  // of a workgroup: as many bytes as its words of the weights
 
-// The bits of a row's largest magnitude, of the finite ones, by one wavefront: every wavefront of a row for itself (LDS is full of words and order), on the bits of the values,
-// two vector instructions a dword.
+// The bits of a row's largest magnitude, of the finite ones, by one wavefront: every wavefront of a row for itself (LDS is full of words and order).
 template <typename AT>
 __device__ __forceinline__ uint32_t wave_largest(const AT* x, int k, int lane) {
-    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-    constexpr int kPer = 16 / sizeof(AT);
     uint32_t top = 0;
-    for (int i = lane * kPer; i < k; i += 64 * kPer) {
-        const go_u4 y = *(const go_u4*)(x + i);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if constexpr (sizeof(AT) == 4) top = max(top, y[j] & 0x7fffffffu);
-            else top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top), __builtin_bit_cast(u16x2, y[j] & 0x7fff7fffu)));
-        }
-    }
-    if constexpr (sizeof(AT) == 2) top = max(top & 0xffff0000u, top << 16);
-    float mx = __uint_as_float(top);
-    if (__any(top >= 0x7f800000u)) {
+    for (int pc = lane; pc < k >> 3; pc += 64) top = largest_bits(top, load_piece(x + pc * 8));
+    float mx = largest_of<AT>(top);
+    if (any_not_finite(mx)) {
         mx = 0.0f;
-        for (int pc = lane; pc < k >> 3; pc += 64) {
-            float v[8];
-            load8(x + pc * 8, v);
-            mx = largest(mx, v);
-        }
+        for (int pc = lane; pc < k >> 3; pc += 64) mx = largest_finite(mx, load_piece(x + pc * 8));
     }
     return wave_max_nonneg_bits(mx);
 }
