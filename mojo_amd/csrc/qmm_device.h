@@ -27,12 +27,18 @@ __device__ __forceinline__ uint16_t f2h(float f) {
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 // Round-to-nearest-even with canonical NaN, the rule of the reference's
 // software bf16 narrowing (stdlib/src/builtin/simd.mojo:3279-3300).
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t x = __float_as_uint(f);
-    if ((x & 0x7fffffffu) > 0x7f800000u) return (uint16_t)(((x >> 16) & 0x8000u) | 0x7fc0u);
-    x += 0x7fffu + ((x >> 16) & 1u);
-    return (uint16_t)(x >> 16);
+// The instruction rounds so; it keeps the payload of a NaN, which is looked for once for all lanes.
+__device__ __forceinline__ uint32_t f2bf2(float x, float y) {
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+    uint32_t r = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2v{x, y}), b2v));
+    if (__any(x != x || y != y)) {
+        if (x != x) r = (r & 0xffff0000u) | (__float_as_uint(x) >> 16 & 0x8000u) | 0x7fc0u;
+        if (y != y) r = (r & 0xffffu) | (__float_as_uint(y) & 0x80000000u) | 0x7fc00000u;
+    }
+    return r;
 }
+__device__ __forceinline__ uint16_t f2bf(float x) { return (uint16_t)f2bf2(x, 0.0f); }
 
 // lhs element i as fp32; InT is float or a bf16 bit pattern (uint16_t).
 template <typename InT>

@@ -14,7 +14,9 @@ namespace qmm {
 // A lane owns V consecutive elements (8 of a bf16 output, 4 of an fp32 one: 16 bytes), so that a wavefront stores 1 KB in one
 // instruction, and always the same place of a block: the field offsets and shifts are set once per lane, and the lanes of a
 // block read its header and codes from the same cache lines.  (One element per lane, byte loads and 2-byte stores: 14336 x 4096
-// Q4_K to bf16 took 130 us.)
+// Q4_K to bf16 took 130 us.)  What four steps load is asked for before the first of them is used, behind no branch, and bf16 pairs are made by one instruction.  us, a wait behind each load and
+// a branch for the NaN of each value / this way, 14336 x 4096 to fp32 and bf16: Q4_0 53.9 / 50.7 and 31.0 / 27.5, Q4_K 64.7 / 50.4 and 40.7 / 28.1, Q5_K 67.1 / 52.1 and 41.8 / 30.3, Q6_K 54.4 / 51.9 and
+// 35.4 / 32.1; with the output where the last call left it, Q4_K to bf16 26.0 / 22.7 (6.6 TB/s).
 
 typedef uint32_t dq_u4 __attribute__((ext_vector_type(4)));
 typedef float dq_f4 __attribute__((ext_vector_type(4)));
@@ -27,57 +29,71 @@ struct Codes {
 };
 __device__ __forceinline__ float code_f32(const uint32_t* w, int i) { return (float)byte_of(w[i >> 2], i & 3); }
 
-__device__ __forceinline__ uint32_t bf16_pair(float x, float y) { return (uint32_t)f2bf(x) | ((uint32_t)f2bf(y) << 16); }
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) { return f2bf2(x, y); }
 
 __device__ __forceinline__ void store_elems(float* out, const float (&v)[4]) { __builtin_nontemporal_store(dq_f4{v[0], v[1], v[2], v[3]}, (dq_f4*)out); }
 __device__ __forceinline__ void store_elems(uint16_t* out, const float (&v)[8]) {
     __builtin_nontemporal_store(dq_u4{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]), bf16_pair(v[4], v[5]), bf16_pair(v[6], v[7])}, (dq_u4*)out);
 }
 
-// elements pos .. pos + V - 1 of the block at b
+// Elements pos .. pos + V - 1 of the block at b: what is loaded for them, and what it means.
 template <int ENC, int V>
-__device__ __forceinline__ void dequant_elems(const uint8_t* b, int pos, float (&v)[V]) {
-    if constexpr (ENC == QMM_Q4_0) {
-        uint16_t dh;
-        __builtin_memcpy(&dh, b, 2);
-        const float d = h2f(dh);
-        Codes<V> c(b + 2 + (pos & 15));
+struct Elems {  // Q4_K, Q5_K (blocks are 16-byte aligned)
+    dq_u4 hdr;
+    Codes<V> c, fifth;
+    __device__ __forceinline__ Elems(const uint8_t* b, int pos)
+        : hdr(*(const dq_u4*)b), c(b + (ENC == QMM_Q4_K ? 16 : 48) + 32 * (pos >> 6) + (pos & 31)), fifth(b + (ENC == QMM_Q5_K ? 16 : 0) + (pos & 31)) {}
+    __device__ __forceinline__ void values(int pos, float (&v)[V]) const {
+        const int j = pos >> 5, shift = 8 * (j & 3);
+        const uint32_t late = (uint32_t)((3 - j) >> 31);
+        // (q4k_scale_min without a branch: half of a block's lanes are on either side of it)
+        const uint32_t s0 = (hdr.y >> shift) & 255u, s1 = (hdr.z >> shift) & 255u, s2 = (hdr.w >> shift) & 255u;
+        const uint32_t sc = (s0 & 63u & ~late) | (((s2 & 15u) | ((s0 >> 6) << 4)) & late),
+                       mn = (s1 & 63u & ~late) | (((s2 >> 4) | ((s1 >> 6) << 4)) & late);
+        const float ds = h2f((uint16_t)(hdr.x & 0xffffu)) * (float)sc, dm = h2f((uint16_t)(hdr.x >> 16)) * (float)mn;
 #pragma unroll
-        for (int i = 0; i < V / 4; i++) c.w[i] = (c.w[i] >> (pos & 16 ? 4 : 0)) & 0x0f0f0f0fu;
+        for (int i = 0; i < V / 4; i++) {
+            uint32_t w[1] = {(c.w[i] >> (j & 1 ? 4 : 0)) & 0x0f0f0f0fu};
+            if constexpr (ENC == QMM_Q5_K) w[0] |= ((fifth.w[i] >> j) & 0x01010101u) << 4;
 #pragma unroll
-        for (int i = 0; i < V; i++) v[i] = (code_f32(c.w, i) - 8.0f) * d;
-    } else if constexpr (ENC == QMM_Q6_K) {
-        const int h = pos >> 7, quarter = (pos >> 5) & 3, l = pos & 31;
-        uint16_t dh;
-        __builtin_memcpy(&dh, b + 208, 2);
-        const float ds = h2f(dh) * (float)((const int8_t*)b)[192 + 8 * h + (l >> 4) + 2 * quarter];
-        const Codes<V> lo(b + 64 * h + 32 * (quarter & 1) + l), hi(b + 128 + 32 * h + l);
-        uint32_t w[V / 4];
-#pragma unroll
-        for (int i = 0; i < V / 4; i++)
-            w[i] = ((lo.w[i] >> (quarter & 2 ? 4 : 0)) & 0x0f0f0f0fu) | (((hi.w[i] >> (2 * quarter)) & 0x03030303u) << 4);
-#pragma unroll
-        for (int i = 0; i < V; i++) v[i] = ds * (code_f32(w, i) - 32.0f);
-    } else {  // Q4_K, Q5_K (blocks are 16-byte aligned)
-        const dq_u4 hdr = *(const dq_u4*)b;
-        const float d = h2f((uint16_t)(hdr.x & 0xffffu)), dmin = h2f((uint16_t)(hdr.x >> 16));
-        const uint32_t s[3] = {hdr.y, hdr.z, hdr.w};
-        const int j = pos >> 5, l = pos & 31;
-        uint32_t sc, mn;
-        q4k_scale_min(j, s, sc, mn);
-        const float ds = d * (float)sc, dm = dmin * (float)mn;
-        Codes<V> c(b + (ENC == QMM_Q4_K ? 16 : 48) + 32 * (pos >> 6) + l);
-#pragma unroll
-        for (int i = 0; i < V / 4; i++) c.w[i] = (c.w[i] >> (j & 1 ? 4 : 0)) & 0x0f0f0f0fu;
-        if constexpr (ENC == QMM_Q5_K) {
-            const Codes<V> fifth(b + 16 + l);
-#pragma unroll
-            for (int i = 0; i < V / 4; i++) c.w[i] |= ((fifth.w[i] >> j) & 0x01010101u) << 4;
+            for (int e = 0; e < 4; e++) v[4 * i + e] = ds * code_f32(w, e) - dm;
         }
-#pragma unroll
-        for (int i = 0; i < V; i++) v[i] = ds * code_f32(c.w, i) - dm;
     }
-}
+};
+
+template <int V>
+struct Elems<QMM_Q4_0, V> {
+    uint16_t d;
+    Codes<V> c;
+    __device__ __forceinline__ Elems(const uint8_t* b, int pos) : c(b + 2 + (pos & 15)) { __builtin_memcpy(&d, b, 2); }
+    __device__ __forceinline__ void values(int pos, float (&v)[V]) const {
+        const float df = h2f(d);
+        const uint32_t shift = pos & 16 ? 4 : 0;
+#pragma unroll
+        for (int i = 0; i < V; i++) v[i] = ((float)((c.w[i >> 2] >> (shift + 8 * (i & 3))) & 15u) - 8.0f) * df;
+    }
+};
+
+template <int V>
+struct Elems<QMM_Q6_K, V> {
+    uint16_t d;
+    int8_t scale;
+    Codes<V> lo, hi;
+    __device__ __forceinline__ Elems(const uint8_t* b, int pos)
+        : scale(((const int8_t*)b)[192 + (pos >> 4)]), lo(b + 64 * (pos >> 7) + 32 * ((pos >> 5) & 1) + (pos & 31)), hi(b + 128 + 32 * (pos >> 7) + (pos & 31)) {
+        __builtin_memcpy(&d, b + 208, 2);
+    }
+    __device__ __forceinline__ void values(int pos, float (&v)[V]) const {
+        const int quarter = (pos >> 5) & 3;
+        const float ds = h2f(d) * (float)scale;
+#pragma unroll
+        for (int i = 0; i < V / 4; i++) {
+            const uint32_t w[1] = {((lo.w[i] >> (quarter & 2 ? 4 : 0)) & 0x0f0f0f0fu) | (((hi.w[i] >> (2 * quarter)) & 0x03030303u) << 4)};
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[4 * i + j] = ds * (code_f32(w, j) - 32.0f);
+        }
+    }
+};
 
 template <int ENC, typename OutT>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w, int64_t total, OutT* __restrict__ out) {
@@ -86,14 +102,22 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
     constexpr int V = 16 / sizeof(OutT), kStep = 256 * V, kAhead = 4;  // (a workgroup walks kAhead steps: their loads are in flight together)
     const int pos = (int)(threadIdx.x * V) % EPB;
     const int64_t first = (int64_t)blockIdx.x * (kStep * kAhead) + threadIdx.x * V;
-#pragma unroll
-    for (int u = 0; u < kAhead; u++) {
-        const int64_t e = first + u * kStep;
-        if (e < total) {
-            float v[V];
-            dequant_elems<ENC, V>(w + e / EPB * BPB, pos, v);
-            store_elems(out + e, v);
-        }
+    auto convert = [&](const Elems<ENC, V>& x, int64_t e) __attribute__((always_inline)) {
+        float v[V];
+        x.values(pos, v);
+        store_elems(out + e, v);
+    };
+    if ((int64_t)(blockIdx.x + 1) * (kStep * kAhead) <= total) {
+        const uint8_t* const b = w + first / EPB * BPB;
+        constexpr int kBytes = kStep / EPB * BPB;
+        const Elems<ENC, V> x0(b, pos), x1(b + kBytes, pos), x2(b + 2 * kBytes, pos), x3(b + 3 * kBytes, pos);
+        __builtin_amdgcn_sched_barrier(0);
+        convert(x0, first);
+        convert(x1, first + kStep);
+        convert(x2, first + 2 * kStep);
+        convert(x3, first + 3 * kStep);
+    } else {
+        for (int64_t e = first; e < total; e += kStep) convert(Elems<ENC, V>(w + e / EPB * BPB, pos), e);
     }
 }
 

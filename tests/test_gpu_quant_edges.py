@@ -65,3 +65,22 @@ def test_gptq_edges(n, k, group):
         plain = O.dequantize_gptq(qw, sc, qz, group, g_idx)
         assert np.array_equal(bits(dequantize(QE.GPTQ, *rhs, config=config)), plain.view(np.int32))
         assert np.array_equal(bits(dequantize(QE.GPTQ, *rhs, config=config, dtype=torch.bfloat16)), O.f32_to_bf16(plain).view(np.int16))
+
+
+@pytest.mark.parametrize("enc", list(ORACLE))
+@pytest.mark.parametrize("n", [4, 15, 16, 17, 31, 32, 33, 65])  # a workgroup's 4096 (fp32) or 8192 (bf16) elements, with and without a rest
+def test_dequantised_workgroups_with_and_without_a_rest(enc, n):
+    """Block scales that are infinite or no number beside finite ones: a bf16 NaN is 0x7fc0, with either sign."""
+    k = 256
+    packed = O.quantize(ORACLE[enc], weights(n, n, k))
+    blocks = packed.reshape(-1, O.BLOCK[ORACLE[enc]][1])
+    at = 208 if enc == QE.Q6_K else 0
+    for block, scale in ((1, 0x7C00), (2, 0x7E01), (len(blocks) - 1, 0xFC00)):
+        blocks[block, at : at + 2] = [scale & 255, scale >> 8]
+    want = O.dequantize(ORACLE[enc], packed, k)
+    got = dequantize(enc, torch.from_numpy(packed).cuda())
+    assert np.array_equal(np.isnan(want), got.isnan().cpu().numpy()) and np.isnan(want).any()
+    assert np.array_equal(bits(got)[~np.isnan(want)], want.view(np.int32)[~np.isnan(want)])
+    got = bits(dequantize(enc, torch.from_numpy(packed).cuda(), dtype=torch.bfloat16))
+    assert np.array_equal(got[~np.isnan(want)], O.f32_to_bf16(want).view(np.int16)[~np.isnan(want)])
+    assert (got[np.isnan(want)] & 0x7FFF == 0x7FC0).all()
