@@ -4,9 +4,9 @@
 // instructions), but brings everything through registers, which leaves room for 64 rows a wavefront: 8.5 vector instructions a matrix-core instruction, where
 // a wavefront of those hides four (32 cycles against 12 + 4 each), and 2.3 us a unit of 256 columns for 64 x 256 results.  Here loads go from
 // memory to LDS directly (load16_to_lds) and hold no registers while they are on their way, so that a wavefront takes up to 128 rows: 5 vector instructions
-// a matrix-core instruction, 2.5 .. 3.0 us a unit for 128 x 256 results.  What bounds a unit now: the matrix cores (2.2 us of it), then a
-// barrier every four or eight steps.  By the counters (profiles/staged_gemm__counters.txt) the matrix cores of the compute units in use are busy 0.42 .. 0.59 of a launch of
-// 45 us and more (0.27 of one of 20), a wavefront waits 0.27 .. 0.39 of its time, 0.02 .. 0.04 for LDS, which is active 0.19 .. 0.32 of it.  What bounds a call of a few units: 14 us
+// a matrix-core instruction, 2.4 .. 2.9 us a unit for 128 x 256 results.  What bounds a unit now: the matrix cores (2.2 us of it, at the 1.7 GHz that the power leaves them) and the loads to
+// LDS, 16 cycles of a compute unit a KB (reads from LDS take 4), which overlap less than they might; then a barrier every four or eight steps.  By the counters (profiles/staged_gemm__counters.txt) the matrix cores of the compute units in use are busy 0.41 .. 0.61 of a launch of
+// 40 us and more (0.26 of one of 20), a wavefront waits 0.26 .. 0.39 of its time, 0.02 .. 0.03 for LDS, which is active 0.19 .. 0.32 of it.  What bounds a call of a few units: 14 us
 // around them (the preparation 2.6, the boundary between the launches 2.4, the way to the first unit 3, the results 3 .. 4).
 //
 // us, without this kernel / with it, weights from memory (profiles/staged_gemm__plans.txt): Q4_K 14336 x 4096 200 bf16 rows 53 / 44, 320 85 / 60, 4096 x 4096 200 rows 25 / 22,
@@ -15,7 +15,8 @@
 // shared kernels served, 0.80 .. 0.85 and 0.65 .. 0.71 beyond.
 //
 // Tried without gain: 64 x 64 results a wavefront with one wavefront a SIMD (nothing hides its waits: 2.1 us for 64 x 256); wavefronts that load only weights or
-// only lhs, with the weights two units ahead; the loads spread over the steps; chunks of the lhs half as long and twice as many.
+// only lhs, with the weights two units ahead; chunks of the lhs half as long and twice as many or of two steps with up to six buffers (14336 x 4096 200 rows 38.2 / 39.9 us, 4096 x 14336 54.5 / 65.4);
+// one buffer for the packed weights of Q6_K and chunks twice as long (4096 x 14336 500 rows 113.8 / 113.2).
 #include "gemm_direct.h"
 #include "lds_stream.h"
 
