@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import oracle as O
-from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, dequantize, quantize, quantize_gptq
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, dequantize, qmatmul_rmsnorm, quantize, quantize_gptq
 
 pytestmark = pytest.mark.gpu
 ORACLE = {QE.Q4_0: O.Q4_0, QE.Q4_K: O.Q4_K, QE.Q5_K: O.Q5_K, QE.Q6_K: O.Q6_K}
@@ -84,3 +84,20 @@ def test_dequantised_workgroups_with_and_without_a_rest(enc, n):
     got = bits(dequantize(enc, torch.from_numpy(packed).cuda(), dtype=torch.bfloat16))
     assert np.array_equal(got[~np.isnan(want)], O.f32_to_bf16(want).view(np.int16)[~np.isnan(want)])
     assert (got[np.isnan(want)] & 0x7FFF == 0x7FC0).all()
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [32, 256, 288, 4096, 4128, 8192, 8224, 16384, 16416, 33056])  # a thread's 16, 32 and 64 values, and rows longer than those
+def test_rms_normalised_rows_of_every_length(k, lhs):
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    config = QuantizationConfig("gptq", 4, 32, False, True)
+    rhs = quantize_gptq(torch.randn((40, k), device="cuda", generator=gen) * 0.02, config)[:3]
+    x = (torch.randn((3, k), device="cuda", generator=gen) * torch.tensor([[1.0], [1e-3], [300.0]], device="cuda")).to(lhs)
+    gamma = torch.rand(k, device="cuda", generator=gen) + 0.5
+    y = x.double() / (x.double().square().mean(dim=1, keepdim=True) + 1e-5).sqrt() * gamma.double()
+    w = dequantize(QE.GPTQ, *rhs, config=config).double()
+    want, size = y @ w.T, y.abs() @ w.abs().T
+    # The sum of squares: K / 256 additions one after the other and ten more, half of their error behind the square root, five roundings; bf16 rows are rounded once more.  The product: K / 16 additions and 32 on
+    # products of up to sixteen times their size.
+    bound = ((k / 512 + 10) * 2.0**-24 + (2.0**-8 if lhs == torch.bfloat16 else 0.0) + (k / 16 + 32) * 2.0**-24 * 16) * size
+    assert ((qmatmul_rmsnorm(QE.GPTQ, config, x, gamma, 1e-5, *rhs).double() - want).abs() <= bound).all()
