@@ -1,10 +1,12 @@
 """Quantisers and dequantisers at the edges of their tiles, byte for byte against the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import oracle as O
-from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, dequantize, qmatmul_rmsnorm, quantize, quantize_gptq
+from mojo_amd import QuantizationConfig, QuantizationEncoding as QE, _lib, dequantize, qmatmul_rmsnorm, quantize, quantize_gptq
 
 pytestmark = pytest.mark.gpu
 ORACLE = {QE.Q4_0: O.Q4_0, QE.Q4_K: O.Q4_K, QE.Q5_K: O.Q5_K, QE.Q6_K: O.Q6_K}
@@ -101,3 +103,20 @@ def test_rms_normalised_rows_of_every_length(k, lhs):
     # products of up to sixteen times their size.
     bound = ((k / 512 + 10) * 2.0**-24 + (2.0**-8 if lhs == torch.bfloat16 else 0.0) + (k / 16 + 32) * 2.0**-24 * 16) * size
     assert ((qmatmul_rmsnorm(QE.GPTQ, config, x, gamma, 1e-5, *rhs).double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 33, 256), (301, 65, 512), (300, 8, 256), (67, 3, 288)])
+@pytest.mark.parametrize("offset", [0, 1, 4, 8])  # of the results, in values: 16-byte aligned or not
+def test_bf16_results_anywhere(m, n, k, offset):
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    packed = quantize(QE.Q4_0, torch.randn((n, k), device="cuda", generator=gen))
+    a = torch.randn((m, k), device="cuda", generator=gen)
+    lib = _lib.load()
+    need = max(lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.Q4_0.code, None, _lib.QMM_F32, m, n, k, flags) for flags in (0, _lib.QMM_FLAG_OUT_BF16))
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device="cuda")
+    want, got = torch.empty((m, n), device="cuda"), torch.zeros(m * n + 16, dtype=torch.bfloat16, device="cuda")
+    for out, flags in ((want, 0), (got[offset:], _lib.QMM_FLAG_OUT_BF16)):
+        assert lib.qmm_matmul(QE.Q4_0.code, None, a.data_ptr(), _lib.QMM_F32, m, k, (C.c_void_p * 1)(packed.data_ptr()), 1, n, out.data_ptr(), ws.data_ptr(), ws.numel(), flags,
+                              torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(got[offset : offset + m * n].view(m, n), want.bfloat16())
+    assert not got[:offset].any() and not got[offset + m * n :].any()
