@@ -165,6 +165,9 @@ __device__ __forceinline__ uint32_t narrow2(float x, float y) {
     typedef float float2v __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v{x, y}), half2v));
 }
+// Where the eight values of lane (row of the tile, half g of a step's 16 columns) lie among the operands of a row tile, in bytes; per: terms of a value (bf16 1, fp32 2).  A row tile takes 64 K per
+// bytes: more than 32 bits from K = 2^25 on.
+constexpr int64_t operand_offset(int step, int row, int g, int per) { return (int64_t)step * (1024 * per) + (row + 32 * g) * 16; }
 // Piece pc (eight columns) of a row, scaled by s (v is left so), as its part of the operands.
 template <typename AT, int ORDER>
 __device__ __forceinline__ void store_piece(_Float16* a16, int steps, int row, int pc, float s, float (&v)[8]) {
@@ -176,9 +179,8 @@ __device__ __forceinline__ void store_piece(_Float16* a16, int steps, int row, i
     HalfPack hi;
 #pragma unroll
     for (int i = 0; i < 4; i++) hi.u[i] = narrow2(v[perm[ORDER][2 * i]], v[perm[ORDER][2 * i + 1]]);
-    const uint32_t at = (uint32_t)step * (kF32 ? 2048u : 1024u) + (uint32_t)((row & 31) + 32 * g) * 16u;  // (below 2^23)
-    uint8_t* const tile = (uint8_t*)a16 + (int64_t)(row >> 5) * steps * (kF32 ? 2048 : 1024);
-    *(half8*)(tile + at) = hi.h;
+    uint8_t* const at = (uint8_t*)a16 + (int64_t)(row >> 5) * operand_offset(steps, 0, 0, kF32 ? 2 : 1) + operand_offset(step, row & 31, g, kF32 ? 2 : 1);
+    *(half8*)at = hi.h;
     if constexpr (kF32) {
         HalfPack lo;
         float residual[8];
@@ -189,7 +191,7 @@ __device__ __forceinline__ void store_piece(_Float16* a16, int steps, int row, i
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) lo.u[i] = narrow2(residual[2 * i], residual[2 * i + 1]);
-        *(half8*)(tile + at + 1024) = lo.h;
+        *(half8*)(at + 1024) = lo.h;
     }
 }
 // The e-th of `count` workgroups zeroes its part of the results (m rows).

@@ -302,6 +302,18 @@ def test_q6_k_that_ends_between_multiples_of_four_is_not_served_beyond_the_direc
         assert wanted(QE.Q6_K, m, n, k + 256, 0x10000)
 
 
+def test_operands_of_long_rows_do_not_overlap(tmp_path):
+    """The places of a row tile's operands, as the preparation of the lhs works them out, against 64-bit arithmetic: with K = 2^25 (fp32) and 2^26 (bf16) they pass 32 bits."""
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("needs hipcc")
+    checks = "\n".join(f"static_assert(qmm::operand_offset({k // 16 - 1}, {row}, {g}, {per}) == {(k // 16 - 1) * 1024 * per + (row + 32 * g) * 16}LL);"
+                       for per, k in ((1, 256), (2, 256), (1, 2**26 + 256), (2, 2**25 + 256), (1, 2**31 - 256), (2, 2**31 - 256)) for row, g in ((0, 0), (31, 1)))
+    source = tmp_path / "places.hip"
+    source.write_text('#include "gemm_direct.h"\n' + checks + "\n")
+    proc = subprocess.run([build.HIPCC, "-std=c++17", "--offload-arch=gfx950", "--cuda-host-only", "-fsyntax-only", f"-I{build.CSRC}", str(source)], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr[-3000:]
+
+
 def test_no_tensors_means_none_is_looked_at():
     """n_rhs = 0 with an array all the same (here one that ends where memory does): an error, not a read of its first entry."""
     import mmap

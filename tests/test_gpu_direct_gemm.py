@@ -154,6 +154,25 @@ def test_values_far_below_the_largest_of_their_row(group, lhs, spike):
     assert worst <= 1.0, worst
 
 
+@pytest.mark.parametrize("enc,lhs,k", [(QE.Q4_K, torch.float32, 2**25 + 256), (QE.Q6_K, torch.float32, 2**25 + 256), (QE.Q4_K, torch.bfloat16, 2**26 + 256)])
+def test_rows_whose_operands_take_more_than_32_bits_of_address(enc, lhs, k):
+    """17 rows of 2^25 (fp32) or 2^26 (bf16) columns and some: a row tile's operands pass 4 GB.  The first and the last 256 columns hold most of the product, so that it is wrong by as much as it is
+    large where one takes the other's place."""
+    m, n = 17, 8
+    assert _lib.load().qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, enc.code, None, _lib.QMM_F32 if lhs == torch.float32 else _lib.QMM_BF16, m, n, k, 0) > 2**32  # (the direct GEMM's)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    w = quantize(enc, torch.empty((n, k), device="cuda").normal_(0.0, 0.02, generator=gen))
+    a = torch.empty((m, k), device="cuda").normal_(generator=gen)
+    a[:, :256] *= 2.0**12
+    a[:, -256:] *= 2.0**12
+    a = a.to(lhs)
+    plain = dequantize(enc, w, k=k)
+    want = sum(x.double() @ y.double().T for x, y in zip(a.split(2**22, 1), plain.split(2**22, 1)))
+    got = qmatmul(enc, None, a, w)
+    # (up to 2^15 sums of a unit one after the other: 2^-24 of what is summed up each, as a random walk below 2^-15)
+    assert ((got.double() - want).norm() / want.norm()).item() < 2.0**-15
+
+
 # Relative error (2-norm over all results, against float64) of quantised N(0, 0.02) weights and N(0, 1) rows.  The bounds lie a tenth above what the chains of
 # rounded sums give (measured, in the comment, with what longer chains and codes around another mean gave); leaving the residual of fp32 rows out would give 1.4e-4.
 PRECISION = [
