@@ -597,8 +597,12 @@ double sums_error(const SumsError& e, const DirectPlan& p, int64_t units, int64_
     }
     return e.base + e.length * (double)units + (e.unit * 0.5 * squares + e.join * join + e.first * held_parts) / (double)units;
 }
-// Codes around their middle: unit sums, and no plan with 128 rows a wavefront, which has no registers for them.
-bool staged_has(const StagedCost& c, int plan, bool centred) { return c.unit[plan] != 0.0f && !(centred && kStagedPlans[plan].fm == 4); }
+// Codes around their middle: unit sums, and no plan with 128 rows a wavefront, which has no registers for them.  Row tiles of 96 (the last one of 128 may be one) have wavefronts whose loads cross from one
+// 32 rows' operands to another's, with offsets of 32 bits; those 32 rows take 128 K bytes: not from K = 2^23 on.
+constexpr int64_t kStagedLongRows = 1 << 23;
+bool staged_has(const StagedCost& c, int plan, bool centred, int64_t k) {
+    return c.unit[plan] != 0.0f && !(centred && kStagedPlans[plan].fm == 4) && (k < kStagedLongRows || kStagedPlans[plan].fm == 2);
+}
 // What loads to LDS want.  Scales and zeros of GPTQ lie so; only a Q6_K tensor may begin elsewhere.
 bool staged_takes(const void* w) { return ((uintptr_t)w & 3) == 0; }
 // The best of its plans whose parts of K are at most `longest` units and whose sums are off by no more than `most` (sums_error); returns its time (1e30: there is none).
@@ -606,7 +610,7 @@ double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k,
     const int row = staged_row(encoding, group);
     // (Q6_K: the last block would be read two bytes beyond its end where it begins at a multiple of four, which it does if the blocks before it are even in number)
     if (encoding == QMM_Q6_K && (n * direct_units(k)) % 2 != 0) return 1e30;
-    if (row < 0 || k % 256 || k >= 1 << 23 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits; three row tiles of 4 GB)
+    if (row < 0 || k % 256 || k >= 1 << 27 || m > 1 << 21 || n > 1 << 23 || kernel_disabled("staged")) return 1e30;  // (the grid's y and z have 16 bits)
     const int type = lhs_dtype == QMM_F32 ? 1 : 0;
     const StagedCost& c = kStagedCost[row][type];
     const SumsError& e = kSumsError[row][type][centred ? 3 : 2];
@@ -616,7 +620,7 @@ double staged_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k,
             DirectPlan p = kStagedPlans[i];
             p.shares = shares;
             const int64_t parts = p.wk * shares, walk = (direct_units(k) + parts - 1) / parts;
-            if (!staged_has(c, i, centred)) continue;
+            if (!staged_has(c, i, centred, k)) continue;
             const double t = c.base + staged_tiles_us(c, i, m, (n + 256 * p.wn - 1) / (256 * p.wn) * shares, walk) + c.weights * packed_mb(encoding, n, k) + c.lhs * (m * k * 1e-6) +
                              (c.out + c.share * (shares - 1)) * (m * n * 1e-6);
             if (walk <= longest && t < us && sums_error(e, p, direct_units(k)) <= most) us = t, best = p;
@@ -666,7 +670,7 @@ DirectPlan direct_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_
         for (const DirectPlan& p : kStagedPlans) {
             const StagedCost& c = kStagedCost[staged_row(encoding, group)][type];
             const int i = (int)(&p - kStagedPlans);
-            if (!staged_has(c, i, like->centred) || p.wk != like->wk) continue;
+            if (!staged_has(c, i, like->centred, k) || p.wk != like->wk) continue;
             const int64_t walk = (direct_units(k) + p.wk * like->shares - 1) / (p.wk * like->shares);
             const double t = staged_tiles_us(c, i, m, (n + 256 * p.wn - 1) / (256 * p.wn) * like->shares, walk);
             if (t < us) us = t, best = p, best.shares = like->shares, best.centred = like->centred;

@@ -327,6 +327,7 @@ __device__ __forceinline__ void staged_tile(WeightTensors wt, const StagedStart&
     const int last_tile = (m - 1) >> 5;
     // a wavefront loads kLoads neighbouring operands of a chunk (the last ones some that its neighbour loads too); of one row tile, unless kLoads does not divide what a tile has
     constexpr bool kOneTile = kPieces % kLoads == 0 && kTotal % kLoads == 0;
+    static_assert(kOneTile || FM == 3, "the plans with 64 rows a tile take rows of any length (kStagedLongRows)");
     const int piece0 = min(wn * kLoads, kTotal - kLoads);
     auto tile_of = [&](int piece) __attribute__((always_inline)) { return min(row0 + piece / kPieces, last_tile); };
     const uint8_t* const src = (const uint8_t*)start.a16 + tile_of(piece0) * row_bytes + ((int64_t)u0 * W::kSteps * kPer + piece0 % kPieces) * 1024;

@@ -302,6 +302,14 @@ def test_q6_k_that_ends_between_multiples_of_four_is_not_served_beyond_the_direc
         assert wanted(QE.Q6_K, m, n, k + 256, 0x10000)
 
 
+def test_long_rows_go_to_the_staged_gemm():
+    """K of 2^23 and more, below 2^27: by row tiles of 64, whose loads need no offsets from one 32 rows' operands to another's."""
+    call = getattr(C.CDLL(_lib.LIB_PATH), "_ZN3qmm24gemm_direct_takes_stagedEiillli")
+    call.argtypes, call.restype = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int], C.c_bool
+    for enc, lhs, m, n, group in ((QE.GPTQ, _lib.QMM_BF16, 600, 8, 128), (QE.GPTQ, _lib.QMM_F32, 800, 64, 128), (QE.Q4_K, _lib.QMM_F32, 1000, 64, 0), (QE.Q5_K, _lib.QMM_BF16, 1600, 8, 0)):
+        assert all(call(enc.code, lhs, m, n, k, group) for k in (2**23 - 256, 2**23, 2**23 + 256, 2**25))
+
+
 def test_operands_of_long_rows_do_not_overlap(tmp_path):
     """The places of a row tile's operands, as the preparation of the lhs works them out, against 64-bit arithmetic: with K = 2^25 (fp32) and 2^26 (bf16) they pass 32 bits."""
     if not os.path.exists(build.HIPCC):

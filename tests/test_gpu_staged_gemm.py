@@ -143,3 +143,18 @@ def test_precision(enc, group, m, n, k, lhs, most):
     (QE.Q5_K, 0, 193, 5120, 4096, torch.bfloat16, 1.0544e-7), (QE.Q4_K, 0, 200, 4096, 4096, torch.bfloat16, 1.9066e-7), (QE.Q5_K, 0, 481, 7104, 512, torch.bfloat16, 2.0712e-7)])
 def test_no_less_exact_than_the_kernel_before(enc, group, m, n, k, lhs, most):
     test_precision(enc, group, m, n, k, lhs, 1.003 * most)
+
+
+def test_rows_of_more_than_2_to_the_23_columns():
+    """Row tiles whose operands lie half a gigabyte apart, eight of them and one row: bf16 rows of 2^23 + 256 columns.  The first and the last 256 columns hold most of the product."""
+    m, n, k = 513, 8, 2**23 + 256
+    config, rhs = weights(QE.GPTQ, 128, n, k)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    a = torch.empty((m, k), dtype=torch.bfloat16, device="cuda").normal_(generator=gen)
+    a[:, :256] *= 2.0**12
+    a[:, -256:] *= 2.0**12
+    plain = dequantize(QE.GPTQ, *rhs, config=config)
+    want = sum(x.double() @ y.double().T for x, y in zip(a.split(2**19, 1), plain.split(2**19, 1)))
+    got = qmatmul(QE.GPTQ, config, a, *rhs)
+    # (2^14 sums of a unit one after the other and their parts: 2^-24 of what is summed up each, as a random walk below 2^-15)
+    assert ((got.double() - want).norm() / want.norm()).item() < 2.0**-15
