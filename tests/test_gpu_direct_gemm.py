@@ -127,6 +127,42 @@ def test_gptq_infinities_and_nans_keep_their_kind(group, order, m, n, k, lhs):
     check(got[rest], QE.GPTQ, config, rhs, a[rest])
 
 
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("enc", [QE.Q4_K, QE.Q5_K, QE.Q6_K])
+@pytest.mark.parametrize("m,n,k", [(17, 264, 512), (33, 2056, 1024), (200, 4104, 512), (40, 264, 33024)])  # (the last one: more pieces of a row than its threads hold)
+def test_k_quant_rows_with_infinities_and_nans(enc, m, n, k, lhs):
+    """A row with an infinity or a NaN has no finite result; what is finite in it (1e30) scales it, and rows beside it are what they are."""
+    _, rhs = weights(enc, 0, n, k)
+    a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(4)).to(lhs)
+    a[1, 7], a[3, k - 1], a[4, 5], a[5, 100], a[5, 101] = float("inf"), -float("inf"), float("nan"), float("inf"), 1e30
+    a[6] = float("inf")
+    a[8] = float("nan")
+    special = [1, 3, 4, 5, 6, 8]
+    got = qmatmul(enc, None, a, *rhs)
+    assert not got[special].isfinite().any() and got[[4, 8]].isnan().all()
+    rest = [i for i in range(m) if i not in special]
+    check(got[rest], enc, None, rhs, a[rest])
+
+
+@pytest.mark.parametrize("enc,group,lhs,m,n,k", [(QE.GPTQ, 32, torch.bfloat16, 2**23 + 40, 8, 32), (QE.Q4_K, 0, torch.float32, 6000000, 1, 256)])
+def test_more_row_tiles_than_a_grid_counts_apart(enc, group, lhs, m, n, k):
+    """65536 row tiles and more, which are numbered through."""
+    config, rhs = weights(enc, group, n, k)
+    a = torch.empty((m, k), dtype=lhs, device="cuda").normal_(generator=torch.Generator(device="cuda").manual_seed(5))
+    got = qmatmul(enc, config, a, *rhs)
+    for x, y in zip(got.split(2**20), a.split(2**20)):
+        check(x, enc, config, rhs, y)
+
+
+def test_more_q4_0_rows_than_one_slice_of_the_quantiser():
+    """32768 rows and some: the grid of the lhs quantiser has a second slice (K no multiple of 256 and more results than the direct GEMM serves)."""
+    m, n, k = 32768 + 41, 208, 96
+    _, rhs = weights(QE.Q4_0, 0, n, k)
+    for lhs in (torch.float32, torch.bfloat16):
+        a = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(6)).to(lhs)
+        check(qmatmul(QE.Q4_0, None, a, *rhs), QE.Q4_0, None, rhs, a)
+
+
 @pytest.mark.parametrize("lhs,spike", [(torch.float32, 2.0**20), (torch.bfloat16, 2.0**28)])
 @pytest.mark.parametrize("group", [128, 32])
 def test_values_far_below_the_largest_of_their_row(group, lhs, spike):

@@ -120,3 +120,71 @@ def test_bf16_results_anywhere(m, n, k, offset):
                               torch.cuda.current_stream().cuda_stream) == 0
     assert torch.equal(got[offset : offset + m * n].view(m, n), want.bfloat16())
     assert not got[:offset].any() and not got[offset + m * n :].any()
+
+
+@pytest.mark.parametrize("n", [1, 7, 9, 33, 2047, 4101])
+@pytest.mark.parametrize("offset", [0, 1, 2, 5, 8])  # of the results, in values
+def test_results_narrowed_by_a_launch_of_their_own(n, offset):
+    """One row of Q6_K with an odd number of blocks in all, which no kernel that stores bf16 itself serves: the decode kernel's fp32 results and the launch behind it, whose eights leave n mod 8 values."""
+    k = 768
+    packed = quantize(QE.Q6_K, torch.randn((n, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n)))
+    a = torch.randn((1, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(k))
+    lib = _lib.load()
+    need = [lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.Q6_K.code, None, _lib.QMM_F32, 1, n, k, flags) for flags in (0, _lib.QMM_FLAG_OUT_BF16)]
+    assert need[1] >= need[0] + 4 * n  # (the fp32 results lie there)
+    ws = torch.empty(need[1], dtype=torch.uint8, device="cuda")
+    want, got = torch.empty(n, device="cuda"), torch.zeros(n + 16, dtype=torch.bfloat16, device="cuda")
+    for out, flags in ((want, 0), (got[offset:], _lib.QMM_FLAG_OUT_BF16)):
+        assert lib.qmm_matmul(QE.Q6_K.code, None, a.data_ptr(), _lib.QMM_F32, 1, k, (C.c_void_p * 1)(packed.data_ptr()), 1, n, out.data_ptr(), ws.data_ptr(), ws.numel(), flags,
+                              torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(got[offset : offset + n], want.bfloat16())
+    assert not got[:offset].any() and not got[offset + n :].any()
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+def test_narrowed_values_of_every_exponent(offset):
+    """Ties and their neighbours at every exponent of fp32, subnormal numbers, the largest, infinities and NaNs: one value a row, times one, through the act-order look-up kernel (whose products and
+    sums are exact here) and the launch that narrows, over more results than its grid has lanes."""
+    k, n = 32, 1464
+    high, low = torch.tensor([0, 1, 0x7E, 0x7F]) << 16, torch.tensor([0, 1, 0x7FFF, 0x8000, 0x8001, 0xFFFF])
+    values = ((torch.arange(255) << 23)[:, None, None] + high[:, None] + low).flatten()
+    values = torch.cat([values, torch.tensor([0x7F800000, 0x7F800001, 0x7FC00000, 0x7FFFFFFF])])
+    values = torch.cat([values[values > 0], -0x80000000 + values[values > 0]]).int().view(torch.float32).cuda()
+    m = len(values)
+    assert m * n > 8 * 256 * 8192
+    a = torch.zeros((m, k), device="cuda")
+    a[torch.arange(m), torch.arange(m) % k] = values
+    rhs = (torch.full((k // 8, n), 0x22222222, dtype=torch.int32, device="cuda"), torch.ones((1, n), dtype=torch.float16, device="cuda"), torch.zeros((1, n // 8), dtype=torch.int32, device="cuda"),
+           torch.zeros(k, dtype=torch.int32, device="cuda"))  # codes 2, zero point 1
+    lib, cfg = _lib.load(), _lib.GptqConfig(4, 32, 1, 1)
+    need = lib.qmm_matmul_workspace_bytes_flags(QE.GPTQ.code, _lib.QMM_F32, m, n, k, _lib.QMM_FLAG_OUT_BF16)
+    assert 4 * m * n <= need < lib.qmm_preferred_workspace_bytes(_lib.QMM_OP_MATMUL, QE.GPTQ.code, C.byref(cfg), _lib.QMM_F32, m, n, k, _lib.QMM_FLAG_OUT_BF16)  # (no room for sorted columns)
+    ws, got = torch.empty(need, dtype=torch.uint8, device="cuda"), torch.zeros(m * n + offset, dtype=torch.bfloat16, device="cuda")
+    assert lib.qmm_matmul(QE.GPTQ.code, C.byref(cfg), a.data_ptr(), _lib.QMM_F32, m, k, (C.c_void_p * 4)(*[t.data_ptr() for t in rhs]), 4, n, got[offset:].data_ptr(), ws.data_ptr(), need,
+                          _lib.QMM_FLAG_OUT_BF16, torch.cuda.current_stream().cuda_stream) == 0
+    got = got[offset:].view(m, n).view(torch.int16)
+    assert torch.equal(got, got[:, :1].expand(m, n))
+    got, want, x = got[:, 0].cpu().numpy(), O.f32_to_bf16(values.cpu().numpy()).view(np.int16), values.cpu().numpy()
+    assert np.array_equal(got[~np.isnan(x)], want[~np.isnan(x)])
+    assert (got[np.isnan(x)] & 0x7FFF == 0x7FC0).all()
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [32, 256, 288, 1024, 1056, 4096, 4128, 8192, 8224, 16384, 16416, 33056])
+@pytest.mark.parametrize("place", [0, 1, 2])  # the first values of a row, some in its middle, the last
+def test_rms_of_rows_that_32_values_decide(k, place, lhs):
+    """Nearly all of a row's squares in 32 values: a sum that leaves them out is wrong by a large factor, at whichever of a thread's values they are."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    config = QuantizationConfig("gptq", 4, 32, False, True)
+    rhs = quantize_gptq(torch.randn((40, k), device="cuda", generator=gen) * 0.02, config)[:3]
+    first = (0, k // 64 * 32, k - 32)[place]
+    x = torch.randn((3, k), device="cuda", generator=gen)
+    x[:, first : first + 32] *= 1024
+    x = x.to(lhs)
+    gamma = torch.rand(k, device="cuda", generator=gen) + 0.5
+    y = x.double() / (x.double().square().mean(dim=1, keepdim=True) + 1e-5).sqrt() * gamma.double()
+    w = dequantize(QE.GPTQ, *rhs, config=config).double()
+    want, size = y @ w.T, y.abs() @ w.abs().T
+    # as above; a sum without those values would make the results larger by sqrt(32 * 2^20 / k), 31 times at the longest
+    bound = ((k / 512 + 10) * 2.0**-24 + (2.0**-8 if lhs == torch.bfloat16 else 0.0) + (k / 16 + 32) * 2.0**-24 * 16) * size
+    assert ((qmatmul_rmsnorm(QE.GPTQ, config, x, gamma, 1e-5, *rhs).double() - want).abs() <= bound).all()
