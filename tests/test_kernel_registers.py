@@ -64,3 +64,10 @@ def test_staged_gemm_keeps_its_sums_in_registers(kernels):
     found = {name: spilled for name, (_, spilled) in kernels.items() if name.startswith("gemm_staged_kernel<")}
     assert len(found) > 50
     assert {name: spilled for name, spilled in found.items() if spilled} == {}
+
+
+def test_lhs_preparation_leaves_room_for_a_second_row(kernels):
+    """Workgroups of 1024 threads: with more than 64 registers a compute unit holds one of them, 66 made thousands of long fp32 rows slower."""
+    found = {name: c for name, c in kernels.items() if name.startswith("direct_prep_kernel<")}
+    assert len(found) == 6
+    assert {name: c for name, c in found.items() if c[0] > 64 or c[1]} == {}
