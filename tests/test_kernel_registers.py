@@ -71,3 +71,9 @@ def test_lhs_preparation_leaves_room_for_a_second_row(kernels):
     found = {name: c for name, c in kernels.items() if name.startswith("direct_prep_kernel<")}
     assert len(found) == 6
     assert {name: c for name, c in found.items() if c[0] > 64 or c[1]} == {}
+
+
+def test_direct_gemm_of_gptq_runs_three_wavefronts_a_simd(kernels):
+    """Two fragments of columns side by side, bf16 rows: up to 168 registers.  With 170 two wavefronts fit, and 10512 x 2304 with 349 rows took 44.8 us instead of 40.8."""
+    (registers, spilled), = [c for name, c in kernels.items() if name == "gemm_direct_kernel<3, 8, 1, 2, 4, false>"]
+    assert registers <= 168 and spilled == 0
