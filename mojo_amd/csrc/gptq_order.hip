@@ -342,6 +342,20 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     return look_up > std::min(11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w, 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0));
 }
 
+// How many workgroups zero results beside those of the lhs, in the launch of `slabs` workgroups that the part takes `at_once` of; -1: the lhs has a launch of its own.  zeros: results of the largest matrix
+// that is added to.
+// A workgroup of the lhs, or one that zeroes, takes a place like a slab's.  One more than there are places costs the time of a slab: 7400 x 8832 29 bf16 rows (232 slabs, 8 of the lhs, 256 places) with 56
+// that zero 57, with 8 42, the lhs as a launch of its own 46 us; 7560 x 8064 13 rows 49 / 35.6 / 40, 4056 x 18176 13 rows (254 slabs) 70 / - / 63.  The launch of its own costs 4 .. 7 us: 5120 x 20480 64 rows 88 / 95,
+// 14336 x 4096 400 rows 69 / 74, but 4096 x 14336 400 rows (one workgroup a compute unit) 101 / 93.  Where the sort is apart and the slabs fill three rounds or more, they end at different times, and a tenth
+// of them more is still cheaper: 24440 x 8192 42 rows 100 / 104, 5128 x 25856 66 fp32 rows 141 / 151; but thousands of rows 6984 x 25088 2283 rows 1013 / 919.  (1117 calls with the sort apart: 0.2 % off the faster of
+// both on average, always in the same launch 0.4 %, 28 of them slower than with the rows behind it.)
+int order_lhs_room(int64_t slabs, int64_t at_once, int64_t workgroups, int64_t zeros, bool sort_apart) {
+    const int64_t rounds = (slabs + at_once - 1) / at_once, room = rounds * at_once - slabs - workgroups, wanted = (std::min<int64_t>(1024, (zeros + 4095) / 4096) + 7) / 8 * 8;
+    const int64_t zeroing = std::min(wanted, std::max<int64_t>(room, 0) / 8 * 8);
+    if (room >= 0 && zeros <= zeroing << 18) return (int)zeroing;
+    return sort_apart && rounds >= 3 && 10 * (std::min<int64_t>(wanted, 8) - room) <= slabs ? (int)wanted : -1;
+}
+
 hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int group, const void* a, int lhs_dtype, int64_t m, const DirectSpace& p, const DirectMats& zero,
                              int64_t zeros, bool& lhs_done, hipStream_t s) {
     const int groups = (int)(k / group);
@@ -361,13 +375,14 @@ hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int g
                             (2 * (words(cols) + sort_lds) > kLdsPerCu && n > (int64_t)(cols == 32 ? 48 : cols) * compute_units());
     if (sort_apart) cols = k <= 5120 ? 32 : k <= 20480 ? 16 : 8;  // (32 up to where two fit, 28672 x 5120 32 / 16 columns 78.5 / 80.4; 16 up to where one does, 14336 x 20480 16 / 8 165 / 175)
     const unsigned per_xcd = (unsigned)((n + 8 * cols - 1) / (8 * cols));
-    // The lhs in the same launch where none of its workgroups sorts or the slabs' last round has room for them; otherwise the caller's preparation reads its rows in the order left in memory.
-    // us, that way / in the same launch nevertheless: 4096 x 14336 400 rows (one workgroup a compute unit) 97 / 105, 4096 x 4096 2000 rows 86.2 / 86.5, 4000 157.5 / 158.5.
+    // The lhs in the same launch where the slabs' last round has room for its workgroups and for some that zero results (order_lhs_room); otherwise the caller's preparation reads its rows in the order
+    // left in memory.
     const bool f32 = lhs_dtype == QMM_F32;
+    const int64_t lds = words(cols) + (sort_apart ? 0 : sort_lds), at_once = compute_units() * (2 * lds <= kLdsPerCu && (sort_apart || k <= 8192) ? 2 : 1);
+    const int workgroups = (int)((m + 63) / 64 * 64 / lhs_rows(cols, f32 ? 4 : 2)), zeroing = order_lhs_room((n + cols - 1) / cols, at_once, workgroups, zeros, sort_apart);
+    lhs_done = zeroing >= 0;
     const OrderLhs none{};
-    const OrderLhs lhs{a, p.a16, p.inv, (int)m, (int)((m + 63) / 64 * 64 / lhs_rows(cols, f32 ? 4 : 2)), (int)(std::min<int64_t>(1024, (zeros + 4095) / 4096) + 7) / 8 * 8, zero};
-    const int64_t at_once = compute_units() * (k <= 8192 && 2 * (words(cols) + sort_lds) <= kLdsPerCu ? 2 : 1), slabs = (n + cols - 1) / cols;
-    lhs_done = sort_apart || (slabs + lhs.workgroups + at_once - 1) / at_once == (slabs + at_once - 1) / at_once;
+    const OrderLhs lhs{a, p.a16, p.inv, (int)m, workgroups, std::max(zeroing, 0), zero};
     int32_t* const source = sort_apart || !lhs_done ? order.space.source : nullptr;
     hipError_t e;
 #define QMM_GO(AT, COLS, TURNS, WORDS, GRID, LDS, LHS)                                                                                                                  \
@@ -376,22 +391,18 @@ hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int g
         gptq_order_kernel<AT, COLS, TURNS><<<dim3(GRID), dim3(kThreads), LDS, s>>>(WORDS, order.g_idx, (int)n, (int)k, group, bits, (int)per_xcd, source,               \
                                                                                    order.space.uneven, order.space.qweight, LHS);                                       \
     } while (0)
-#define QMM_GO_LHS(COLS, TURNS, LDS)                                                                                                 \
-    do {                                                                                                                                    \
-        const unsigned grid = 8 * per_xcd + (unsigned)(lhs.workgroups + lhs.zeroing);                                                             \
-        if (f32) QMM_GO(float, COLS, TURNS, order.qweight, grid, LDS, lhs);                                                                 \
-        else QMM_GO(uint16_t, COLS, TURNS, order.qweight, grid, LDS, lhs);                                                                  \
-    } while (0)
-#define QMM_GO_WORDS(COLS, TURNS)                                                                            \
-    do {                                                                                                     \
-        if (lhs_done) QMM_GO_LHS(COLS, TURNS, words(COLS) + sort_lds);                                       \
-        else QMM_GO(uint16_t, COLS, TURNS, order.qweight, 8 * per_xcd, words(COLS) + sort_lds, none);        \
+#define QMM_GO_WORDS(COLS, TURNS)                                                                                                          \
+    do {                                                                                                                                   \
+        const unsigned grid = 8 * per_xcd + (lhs_done ? (unsigned)(lhs.workgroups + lhs.zeroing) : 0u);                                    \
+        if (!lhs_done) QMM_GO(uint16_t, COLS, TURNS, order.qweight, grid, lds, none);                                                      \
+        else if (f32) QMM_GO(float, COLS, TURNS, order.qweight, grid, lds, lhs);                                                           \
+        else QMM_GO(uint16_t, COLS, TURNS, order.qweight, grid, lds, lhs);                                                                 \
     } while (0)
     if (sort_apart) {
         QMM_GO(uint16_t, 8, 32, nullptr, 1, sort_lds, none);
-        if (cols == 32) QMM_GO_LHS(32, 0, words(32));
-        else if (cols == 16) QMM_GO_LHS(16, 0, words(16));
-        else QMM_GO_LHS(8, 0, words(8));
+        if (cols == 32) QMM_GO_WORDS(32, 0);
+        else if (cols == 16) QMM_GO_WORDS(16, 0);
+        else QMM_GO_WORDS(8, 0);
     } else if (cols == 32) {  // (fits up to K = 9100)
         if (k <= 4096) QMM_GO_WORDS(32, 4);
         else if (2 * (words(32) + sort_lds) <= kLdsPerCu) QMM_GO_WORDS(32, 8);
@@ -407,7 +418,6 @@ hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int g
         else QMM_GO_WORDS(8, 32);
     }
 #undef QMM_GO_WORDS
-#undef QMM_GO_LHS
 #undef QMM_GO
     return hipGetLastError();
 }

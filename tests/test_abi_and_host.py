@@ -310,6 +310,25 @@ def test_long_rows_go_to_the_staged_gemm():
         assert all(call(enc.code, lhs, m, n, k, group) for k in (2**23 - 256, 2**23, 2**23 + 256, 2**25))
 
 
+def test_workgroups_beside_the_slabs_find_a_place():
+    """Act-order: rows of the lhs and the zeroing of results share the launch that sorts the weights only where no slab has to wait for them (a few, where slabs of several rounds end at different times)."""
+    room = getattr(C.CDLL(_lib.LIB_PATH), "_ZN3qmm14order_lhs_roomEllllb")
+    room.argtypes, room.restype = [C.c_int64] * 4 + [C.c_bool], C.c_int
+    shared = 0
+    for slabs in (1, 232, 240, 248, 255, 256, 257, 480, 512, 700, 768, 1016):
+        for workgroups in (8, 16, 32, 256, 1152):
+            for zeros in (0, 1, 13 * 7560, 29 * 7400, 1 << 21, 1 << 24):
+                for apart in (False, True):
+                    rounds, zeroing = -(-slabs // 256), room(slabs, 256, workgroups, zeros, apart)
+                    if zeroing < 0:
+                        continue
+                    shared += 1
+                    assert zeroing % 8 == 0 and (zeroing > 0) == (zeros > 0)
+                    assert slabs + workgroups + zeroing <= 256 * rounds or (apart and rounds >= 3 and slabs + workgroups + min(zeroing, 8) <= 256 * rounds + slabs // 10)
+    assert shared > 100
+    assert room(237, 256, 8, 13 * 7560, False) == 8 and room(254, 256, 16, 0, True) == -1 and room(873, 256, 1152, 0, True) == -1
+
+
 def test_operands_of_long_rows_do_not_overlap(tmp_path):
     """The places of a row tile's operands, as the preparation of the lhs works them out, against 64-bit arithmetic: with K = 2^25 (fp32) and 2^26 (bf16) they pass 32 bits."""
     if not os.path.exists(build.HIPCC):

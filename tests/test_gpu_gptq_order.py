@@ -188,3 +188,12 @@ def test_rows_of_the_lhs_beside_the_slabs(m, n, k, lhs):
     assert not torch.isfinite(got[[5, 6, 11]]).any()
     assert torch.equal(got[2], torch.zeros_like(got[2]))
     assert torch.equal(got[rows], qmatmul(QE.GPTQ, config, a, *rhs)[rows])
+
+
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(13, 4056, 18176),  # the sort apart, no place left for the rows: a preparation behind it
+                                   (13, 7400, 8064),  # room for a few workgroups that zero, not for as many as there could be
+                                   (42, 24440, 8192),  # rounds of slabs, and a few places more than the last one has
+                                   (2500, 2056, 20480)])  # thousands of rows, the sort apart
+def test_rows_of_the_lhs_and_places_beside_the_slabs(m, n, k, lhs):
+    test_rows_of_the_lhs_beside_the_slabs(m, n, k, lhs)
