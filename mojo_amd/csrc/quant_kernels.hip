@@ -243,68 +243,89 @@ hipError_t launch_f32_to_bf16(const float* x, uint16_t* out, int64_t count, hipS
 }
 
 // RMS normalisation of one row per workgroup: y = (x * rsqrt(mean(x^2) + eps)) * gamma in fp32, stored in the dtype of x.
-// A thread holds every 256th value of the row, HELD of them at a time, all asked for (gamma's too, where the row is no longer than that) before the first is used; a load at a time, each pass
-// was a chain of K / 256 latencies.  us, a load at a time / this way, normalisation and product: Q4_K 4096 x 4096 one fp32 row 9.6 / 7.6, 200 bf16 rows 30.1 / 25.2, 2000 97.1 / 94.2;
-// 4096 x 14336 one bf16 row 25.8 / 16.1 (with 32 values held 16.9), 500 fp32 rows 174.5 / 158.0; GPTQ 4096 x 11008 4 rows 24.3 / 17.6; Q4_0 4096 x 32768 8 fp32 rows 52.4 / 35.0.  The sums are the same.
-template <typename T, int HELD>
+// A thread holds every 256th value of the row, HELD of them at a time, all asked for (ONCE, a row no longer than that: gamma's too, and nothing is read twice) before the first is used; a load at a time, each
+// pass was a chain of K / 256 latencies.  Few rows are bound by those, many by memory, and by the loads that a compute unit has in flight: buffer loads, whose addresses take one register where a
+// pointer for each load took two and left room for one to three wavefronts a SIMD (16 / 32 / 64 values: 136 / 236 / 400 registers, now 40 / 72 / 136 with fp32 rows).  us, normalisation and a product with
+// Q4_0 32 x K, a load at a time / pointers / this way: K = 14336 one bf16 row 23.0 / 13.2 / 10.2, 400 rows 56.0 / 41.3 / 34.4, 2000 121.5 / 131.9 / 99.3; 12288 2000 bf16 rows 105 / 119 / 88; 8448 2000 bf16 rows
+// 78.8 / 98.6 / 69.9; 4096 400 bf16 rows 23.9 / 18.4 / 17.6; 2048 5000 bf16 rows 56.8 / 56.0 / 47.6; 1024 5000 fp32 rows 36.0 / 38.8 / 31.9.  The sums are the same.
+template <typename T, int HELD, bool ONCE>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const T* __restrict__ x, const float* __restrict__ gamma, float eps, uint32_t k, T* __restrict__ y) {
     __shared__ float red[4];
-    const T* xr = x + (int64_t)blockIdx.x * k;
-    T* yr = y + (int64_t)blockIdx.x * k;
-    const uint32_t tid = threadIdx.x;
-    const bool once = k <= HELD * 256;
+    const T* const xr = x + (int64_t)blockIdx.x * k;
+    T* const yr = y + (int64_t)blockIdx.x * k;
+    // Values first .. first + 256 HELD - 1 of an array as a buffer: an offset beyond the row reads zero and stores nothing.
+    auto part = [&](const auto* row, uint32_t first) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(row + first), 0, (int)(min(k - first, HELD * 256u) * (uint32_t)sizeof(*row)), 0x00020000);
+    };
+    // (made where it is used: with the offsets of every load in registers from one pass to the next, 16 values and their gammas took 81)
+    auto mine = [&](uint32_t size) __attribute__((always_inline)) {
+        uint32_t at = threadIdx.x * size;
+        asm volatile("" : "+v"(at));
+        return at;
+    };
     T v[HELD];
     float g[HELD], ss = 0.0f;
     auto load = [&](uint32_t first) __attribute__((always_inline)) {
+        const auto from = part(xr, first);
+        const uint32_t at = mine(sizeof(T));
 #pragma unroll
-        for (int j = 0; j < HELD; j++) v[j] = xr[min(first + j * 256, k - 1)];
+        for (int j = 0; j < HELD; j++) {
+            if constexpr (sizeof(T) == 4) v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at + 1024u * j, 0, 0));
+            else v[j] = __builtin_amdgcn_raw_buffer_load_b16(from, at + 512u * j, 0, 0);
+        }
     };
     auto load_gamma = [&](uint32_t first) __attribute__((always_inline)) {
+        const auto from = part(gamma, first);
+        const uint32_t at = mine(4);
 #pragma unroll
-        for (int j = 0; j < HELD; j++) g[j] = gamma[min(first + j * 256, k - 1)];
+        for (int j = 0; j < HELD; j++) g[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at + 1024u * j, 0, 0));
     };
-    for (uint32_t first = tid; first < k; first += HELD * 256) {
+    for (uint32_t first = 0; first < (ONCE ? 1 : k); first += HELD * 256) {
         load(first);
-        if (once) load_gamma(first);
+        if constexpr (ONCE) load_gamma(first);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < HELD; j++) {
             const float z = load_f32(v, j);
-            ss = first + j * 256 < k ? fmaf(z, z, ss) : ss;
+            ss = fmaf(z, z, ss);  // (beyond the row: plus zero)
         }
     }
     ss = wave_sum_dpp(ss);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float rs = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)k + eps);
-    for (uint32_t first = tid; first < k; first += HELD * 256) {
-        if (!once) {
+    for (uint32_t first = 0; first < (ONCE ? 1 : k); first += HELD * 256) {
+        if constexpr (!ONCE) {
             load(first);
             load_gamma(first);
             __builtin_amdgcn_sched_barrier(0);
         }
+        const auto to = part(yr, first);
+        const uint32_t at = mine(sizeof(T));
 #pragma unroll
         for (int j = 0; j < HELD; j++) {
-            const uint32_t i = first + j * 256;
             const float z = (load_f32(v, j) * rs) * g[j];
-            if (i < k) {
-                if constexpr (sizeof(T) == 4) yr[i] = z;
-                else yr[i] = f2bf(z);
-            }
+            if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, z), to, at + 1024u * j, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b16(f2bf(z), to, at + 512u * j, 0, 0);
         }
     }
 }
 
 hipError_t launch_rmsnorm(const void* x, int x_dtype, const float* gamma, float eps, int64_t rows, int64_t k, void* y, hipStream_t s) {
     const dim3 grid((unsigned)rows), block(256);
-#define QMM_RMS(HELD)                                                                                                                                \
-    do {                                                                                                                                             \
-        if (x_dtype == QMM_F32) rmsnorm_kernel<float, HELD><<<grid, block, 0, s>>>((const float*)x, gamma, eps, (uint32_t)k, (float*)y);                  \
-        else rmsnorm_kernel<uint16_t, HELD><<<grid, block, 0, s>>>((const uint16_t*)x, gamma, eps, (uint32_t)k, (uint16_t*)y);                            \
+#define QMM_RMS(HELD, ONCE)                                                                                                                               \
+    do {                                                                                                                                                  \
+        if (x_dtype == QMM_F32) rmsnorm_kernel<float, HELD, ONCE><<<grid, block, 0, s>>>((const float*)x, gamma, eps, (uint32_t)k, (float*)y);            \
+        else rmsnorm_kernel<uint16_t, HELD, ONCE><<<grid, block, 0, s>>>((const uint16_t*)x, gamma, eps, (uint32_t)k, (uint16_t*)y);                      \
     } while (0)
-    if (k <= 4096) QMM_RMS(16);
-    else if (k <= 8192 || k > 16384) QMM_RMS(32);
-    else QMM_RMS(64);
+    // (no more loads than the row has values for: K = 512 5000 bf16 rows with 4 / 16 a thread 25.5 / 34.0 us.  Longer rows than 64 hold are read twice, with 32: 20480 one fp32 row 32 / 64 values 10.6 / 11.5,
+    // 5000 bf16 rows 456 / 471; 28672 and 32768 within 2 % either way.)
+    if (k <= 1024) QMM_RMS(4, true);
+    else if (k <= 2048) QMM_RMS(8, true);
+    else if (k <= 4096) QMM_RMS(16, true);
+    else if (k <= 8192) QMM_RMS(32, true);
+    else if (k <= 16384) QMM_RMS(64, true);
+    else QMM_RMS(32, false);
 #undef QMM_RMS
     return hipGetLastError();
 }

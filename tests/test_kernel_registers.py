@@ -77,3 +77,12 @@ def test_direct_gemm_of_gptq_runs_three_wavefronts_a_simd(kernels):
     """Two fragments of columns side by side, bf16 rows: up to 168 registers.  With 170 two wavefronts fit, and 10512 x 2304 with 349 rows took 44.8 us instead of 40.8."""
     (registers, spilled), = [c for name, c in kernels.items() if name == "gemm_direct_kernel<3, 8, 1, 2, 4, false>"]
     assert registers <= 168 and spilled == 0
+
+
+def test_rms_normalisation_holds_values_not_addresses(kernels):
+    """A value and its gamma for each of a thread's places in the row, and one offset: pointers for every load took 136, 236 and 400 registers for 16, 32 and 64 places."""
+    found = {name: c for name, c in kernels.items() if name.startswith("rmsnorm_kernel<")}
+    assert len(found) == 12
+    for name, (registers, spilled) in found.items():
+        held = int(re.search(r", (\d+), (?:true|false)>", name).group(1))
+        assert registers <= 2 * held + 40 and spilled == 0, name
