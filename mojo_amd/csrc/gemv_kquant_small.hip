@@ -52,15 +52,15 @@ struct SmallItem {
     static_assert(4 * kSmallPlane + 16 <= kSlot, "four planes of lhs rows and their scales fit a ring slot");
 };
 
-enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2 };
+enum { kSmallPlain = 0, kSmallMats = 1, kSmallGated = 2, kSmallPairs = 3 };
 
 }  // namespace
 
 // MROWS: lhs rows of a workgroup, 1, 2, 4, 8 or 16 (rows past m repeat the last one and their results are dropped); more go side by side, in workgroups of their own.
-// MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up).
+// MODE: one matrix; several that share the lhs (their tiles numbered through); gate and up (result silu(gate) * up), eight rows of each in a tile, or a tile of gate and one of up after the other.
 struct SmallCut {
-    int per, stride;  // tiles of a workgroup at most, workgroups across the tiles
-    uint32_t packed;  // wavefronts; << 8: tiles of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups of a workgroup; << 31: several tiles of lhs rows
+    int per, stride;  // tiles (pairs of them) of a workgroup at most, workgroups across the tiles
+    uint32_t packed;  // wavefronts; << 8: items (tile of a matrix, or of both) of a workgroup whose partial results fit LDS together; << 16: bf16 results; << 17: a group of K per workgroup; << 18: groups of a workgroup; << 31: several tiles of lhs rows
 };
 template <int ENC, int MROWS, typename AT, int MODE>
 __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restrict__ a, int m, int k, const SmallCut& cut) {
@@ -94,22 +94,23 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
     const uint32_t ring_lds = lds_address(ring);
     float* const accs = (float*)(smem + waves * (2 * I::kSlot));  // [chunk][waves][LR][64]
     float* const totals = accs + chunk * waves * LR * 64;  // [chunk][LR][64], with more than one group
-    // Weight rows of a matrix in a tile.  Gated: eight of gate and the same eight of up, so that a workgroup has results whole with half as many of them: 14336 x 4096 4 bf16 rows seven such tiles for each
-    // of 256 compute units, where 896 pairs of whole tiles were four (eight tiles) for each of 224, 15.3 -> 13.9 us; Q6_K 13824 x 5120 28.8 -> 26.9, Q4_K 1000 x 4096 3 rows 6.9 -> 5.8, 11008 x 4096
-    // (six tiles either way) 15.0 -> 14.6.  The same sums.
-    constexpr int kTile = MODE == kSmallGated ? 8 : 16;
+    // Weight rows of a matrix in a tile.  Gated, eight of gate and the same eight of up: a workgroup has results whole with half as many of them.  14336 x 4096 4 bf16 rows: seven such tiles for each
+    // of 256 compute units, where 896 pairs of whole tiles were four (eight tiles) for each of 224, 15.3 -> 13.9 us; Q6_K 13824 x 5120 28.8 -> 26.9, Q4_K 1000 x 4096 3 rows 6.9 -> 5.8.  The same sums.
+    // Pairs of whole tiles are left to small_gated_plan's choice.
+    constexpr int kTile = MODE == kSmallGated ? 8 : 16, kEach = MODE == kSmallPairs ? 2 : 1;  // kEach: items that make a result
     const int ntiles = MODE == kSmallMats ? mats.tile_end[kLanesMaxMats - 1] : (mats.n[0] + kTile - 1) / kTile;
-    const int my_items = share + (per - 1) * stride < ntiles ? per : per - 1;  // (the grid has no workgroup without a tile)
+    const int my_items = kEach * (share + (per - 1) * stride < ntiles ? per : per - 1);  // (the grid has no workgroup without a tile)
 
     // item i of the workgroup: its matrix, and the first row there
     auto matrix_of = [&](int i, int& n0, int& n) __attribute__((always_inline)) {
-        const int tile = share + i * stride;
+        const int tile = share + i / kEach * stride;
         int j = 0;
         if constexpr (MODE == kSmallMats) {  // (entries past the last repeat it)
 #pragma unroll
             for (int i = 0; i + 1 < kLanesMaxMats; i++) j += tile >= mats.tile_end[i] ? 1 : 0;
         }
         n0 = (MODE == kSmallMats && j ? tile - mats.tile_end[j - 1] : tile) * kTile;
+        if constexpr (MODE == kSmallPairs) j = i & 1;
         n = mats.n[j];
         return j;
     };
@@ -420,27 +421,33 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
             __syncthreads();
             // the group's result (matrix row 16 tile + nn, lhs row kg + 4 j): dealt to the wavefronts, which add it to that of the groups before
             const int live = min(waves, nblk - g * waves);
-            for (int q = wave; q < ct * LR; q += waves) {
-                const int t = q / LR, j = q % LR, row = row0 + kg + 4 * j;
-                const float* const src = accs + ((t * waves) * LR + j) * 64 + lane;
-                float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                int w = 0;
-                for (; w + 4 <= live; w += 4)
+            for (int q = wave; q < ct / kEach * LR; q += waves) {
+                const int t = q / LR * kEach, j = q % LR, row = row0 + kg + 4 * j;
+                float s[kEach];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) c[i] += src[(w + i) * LR * 64];
+                for (int h = 0; h < kEach; h++) {
+                    const float* const src = accs + (((t + h) * waves) * LR + j) * 64 + lane;
+                    float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    int w = 0;
+                    for (; w + 4 <= live; w += 4)
 #pragma unroll
-                for (int i = 0; i < 3; i++)
-                    if (w + i < live) c[i] += src[(w + i) * LR * 64];
-                float r = (c[0] + c[1]) + (c[2] + c[3]);
-                if (groups > 1) {
-                    float* const total = totals + (t * LR + j) * 64 + lane;
-                    if (g > g_first) r = *total + r;
-                    if (g + 1 < g_end) *total = r;
+                        for (int i = 0; i < 4; i++) c[i] += src[(w + i) * LR * 64];
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+                        if (w + i < live) c[i] += src[(w + i) * LR * 64];
+                    s[h] = (c[0] + c[1]) + (c[2] + c[3]);
+                    if (groups > 1) {
+                        float* const total = totals + ((t + h) * LR + j) * 64 + lane;
+                        if (g > g_first) s[h] = *total + s[h];
+                        if (g + 1 < g_end) *total = s[h];
+                    }
                 }
                 if (g + 1 < g_end) continue;
                 int n0, n;
                 const int mat = matrix_of(c0 + t, n0, n);
+                float r = s[0];
                 if constexpr (MODE == kSmallGated) r = r / (1.0f + expf(-r)) * dpp_move<0x128>(r);  // (lanes nn < 8: gate, times up eight lanes on)
+                if constexpr (MODE == kSmallPairs) r = r / (1.0f + expf(-r)) * s[kEach - 1];
                 const int64_t at = (int64_t)row * n + n0 + nn;
                 if (row < m && nn < kTile && n0 + nn < n) {
                     if (out_bf16) ((uint16_t*)mats.out[mat])[at] = f2bf(r);
@@ -472,6 +479,7 @@ namespace {
 
 struct SmallPlan {
     int waves, groups, grid, parts, per, chunk, row_tiles;
+    bool pairs;
     size_t lds;
 };
 // Groups of K: of its length only, so that results do not depend on what else a call has.
@@ -479,8 +487,8 @@ int small_groups(int64_t k) {
     const int groups = (int)((k / 256 + kSmallWaves - 1) / kSmallWaves);
     return groups == 3 ? 4 : groups;
 }
-// tiles: of 16 weight rows, gated: of eight of each matrix; parts: workgroups that share a tile, one group of K each
-SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int64_t k, bool parts) {
+// tiles: of 16 weight rows, gated: of eight of each matrix, or pairs of them (each = 2 items); parts: workgroups that share a tile, one group of K each; per: tiles of a workgroup, 0: as few as there are places for
+SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int64_t k, bool parts, int each = 1, int per = 0) {
     SmallPlan p;
     p.row_tiles = (int)((m + small_most_rows(lhs_dtype) - 1) / small_most_rows(lhs_dtype));
     m = std::min(m, small_most_rows(lhs_dtype));
@@ -491,14 +499,36 @@ SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int6
     // one workgroup per compute unit (as many as 16 wavefronts allow with few each), all with the same number of tiles or one fewer
     const int per_cu = std::max(1, kSmallWaves / p.waves);
     const int64_t most = std::max<int64_t>(1, small_places(per_cu, p.row_tiles) / p.parts);
-    p.per = (int)((tiles + most - 1) / most);
+    p.per = per ? per : (int)((tiles + most - 1) / most);
     p.grid = (int)((tiles + p.per - 1) / p.per);
     const int slot = encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? SmallItem<QMM_Q4_K>::kSlot : encoding == QMM_Q5_K ? SmallItem<QMM_Q5_K>::kSlot : SmallItem<QMM_Q6_K>::kSlot;
     // (as many items between two barriers as fit: a barrier after each, with two buffers, took Q6_K 28672 x 8192 with 16 rows from 65 to 92 us)
-    const int lr = m <= 4 ? 1 : m <= 8 ? 2 : 4, ring = p.waves * 2 * slot, each = (p.waves + (groups > p.parts ? 1 : 0)) * lr * 256;
-    p.chunk = std::min(std::min(p.per, 254), (kLdsPerCu / per_cu - ring) / each);
-    p.lds = (size_t)ring + (size_t)p.chunk * each;
+    const int lr = m <= 4 ? 1 : m <= 8 ? 2 : 4, ring = p.waves * 2 * slot, bytes = (p.waves + (groups > p.parts ? 1 : 0)) * lr * 256;
+    p.chunk = std::min(std::min(each * p.per, 254), (kLdsPerCu / per_cu - ring) / bytes) / each * each;
+    p.lds = (size_t)ring + (size_t)p.chunk * bytes;
+    p.pairs = each == 2;
     return p;
+}
+// us: a tile of one group of K, the lhs of one
+double small_item_us(int encoding) { return encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? 1.4 : encoding == QMM_Q5_K ? 1.75 : 2.1; }
+double small_convert_us(int encoding, int lhs_dtype, int64_t m) {
+    return encoding == QMM_Q4_0 ? (m <= 2 ? 1.2 : m <= 4 ? 1.6 : m <= 8 ? 2.6 : 5.0)
+           : lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
+}
+// A gated pair: tiles with eight rows of each matrix, or pairs of whole ones?  By what the fullest compute unit gets, its workgroups' lhs and items one after the other.  The former may leave it an item less, but
+// where several workgroups fit a compute unit they are more workgroups, and each converts the lhs: Q4_K 2816 x 1024 16 fp32 rows 6.5 / 7.3 us, Q4_0 4864 x 1024 8 fp32 rows 5.8 / 6.4 in pairs / halves.
+// With more than four lhs rows a workgroup, pairs also where nothing is gained: half as many results to a wavefront's store is 2 .. 8 % there (9728 x 2560 16 fp32 rows Q4_0 13.6 / 14.4, 18944 x 3584
+// 16 bf16 rows Q4_K 23.4 / 24.3); up to four rows, halves dealt like pairs (Q5_K 2816 x 1024 4 rows in pairs, halves, so dealt 4.5 / 4.3 / 4.15).  Over 460 calls, 1 .. 24 rows, 1.00 of the time of pairs at
+// worst, 0.95 on average; always halves 0.96, up to 1.15.
+SmallPlan small_gated_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
+    const SmallPlan halves = small_plan(encoding, lhs_dtype, m, (n + 7) / 8, k, false), pairs = small_plan(encoding, lhs_dtype, m, (n + 15) / 16, k, false, 2);
+    const int64_t rows = std::min(m, small_most_rows(lhs_dtype));
+    auto us = [&](const SmallPlan& p, int items) {
+        const int64_t workgroups = ((int64_t)p.grid * p.row_tiles + compute_units() - 1) / compute_units();
+        return workgroups * (small_convert_us(encoding, lhs_dtype, rows) + items * p.per * small_item_us(encoding));
+    };
+    if (rows > 4) return us(halves, 1) < 0.99 * us(pairs, 2) ? halves : pairs;
+    return us(halves, 1) <= us(pairs, 2) ? halves : small_plan(encoding, lhs_dtype, m, (n + 7) / 8, k, false, 1, 2 * pairs.per);
 }
 // A K of several groups: a workgroup per (share of the tiles, group), whose results a launch of their own adds in group order, or all groups in each workgroup?
 // The latter converts the lhs again for every group; both give the same bits.  us, walk / apart: Q4_K 1024 x 14336 4 bf16 rows 13.7 / 7.9, 4096 x 14336 2 bf16 rows
@@ -506,9 +536,7 @@ SmallPlan small_plan(int encoding, int lhs_dtype, int64_t m, int64_t tiles, int6
 bool small_parts(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const int groups = small_groups(k);
     if (groups < 2) return false;
-    const double item = encoding == QMM_Q4_0 || encoding == QMM_Q4_K ? 1.4 : encoding == QMM_Q5_K ? 1.75 : 2.1;  // a tile of one group; convert: the lhs of one
-    const double convert = encoding == QMM_Q4_0 ? (m <= 2 ? 1.2 : m <= 4 ? 1.6 : m <= 8 ? 2.6 : 5.0)
-                           : lhs_dtype == QMM_F32 ? (m <= 2 ? 1.7 : m <= 4 ? 2.2 : 3.7) : (m <= 2 ? 1.5 : m <= 4 ? 1.7 : m <= 8 ? 3.0 : encoding == QMM_Q6_K ? 3.6 : 4.4);
+    const double item = small_item_us(encoding), convert = small_convert_us(encoding, lhs_dtype, m);
     const int64_t tiles = (n + 15) / 16;
     const SmallPlan w = small_plan(encoding, lhs_dtype, m, tiles, k, false), a = small_plan(encoding, lhs_dtype, m, tiles, k, true);
     const double walk = groups * ((w.per + w.chunk - 1) / w.chunk) * convert + groups * w.per * item;
@@ -520,7 +548,14 @@ hipError_t run_small(const MmMats& mats, const SmallPlan& p, const AT* a, int m,
     const dim3 grid = p.row_tiles > 1 ? dim3(8, (unsigned)p.row_tiles, (unsigned)((p.grid * p.parts + 7) / 8)) : dim3((unsigned)p.grid, (unsigned)p.parts), block((unsigned)(64 * p.waves));
     const SmallCut cut{p.per, p.grid, (uint32_t)p.waves | (uint32_t)p.chunk << 8 | (uint32_t)out_bf16 << 16 | (uint32_t)(p.parts > 1) << 17 | (uint32_t)(p.parts > 1 ? 1 : p.groups) << 18 | (uint32_t)(p.row_tiles > 1) << 31};
     hipError_t e;
-    if (gated) {
+    if (gated && p.pairs) {
+        if constexpr (MROWS > 4) {
+            if ((e = allow_full_lds<gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallPairs>>()) != hipSuccess) return e;
+            gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallPairs><<<grid, block, p.lds, s>>>(mats, a, m, k, cut);
+        } else {
+            return hipErrorInvalidValue;
+        }
+    } else if (gated) {
         if ((e = allow_full_lds<gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallGated>>()) != hipSuccess) return e;
         gemv_kquant_small_mats_kernel<ENC, MROWS, AT, kSmallGated><<<grid, block, p.lds, s>>>(mats, a, m, k, cut);
     } else if (mats.count > 1) {
@@ -637,7 +672,7 @@ hipError_t launch_gemv_kquant_small(int encoding, const void* lhs, int lhs_dtype
             if (j < count) values += m * ns[j];
             sums.end[j] = values;
         }
-    const SmallPlan p = small_plan(encoding, lhs_dtype, m, gated ? (ns[0] + 7) / 8 : tiles, k, parts);
+    const SmallPlan p = gated ? small_gated_plan(encoding, lhs_dtype, m, ns[0], k) : small_plan(encoding, lhs_dtype, m, tiles, k, parts);
     const bool store_bf16 = out_bf16 && !parts;
     hipError_t e = encoding == QMM_Q4_0   ? run_small_rows<QMM_Q4_0>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)
                    : encoding == QMM_Q4_K ? run_small_rows<QMM_Q4_K>(mats, p, lhs, lhs_dtype, (int)m, (int)k, gated, store_bf16, s)

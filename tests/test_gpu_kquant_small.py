@@ -128,6 +128,17 @@ def test_gated_pair_in_tiles_of_eight_rows_of_each_matrix(enc, lhs, m, n, k):
     assert torch.allclose(qmatmul_swiglu(QE[enc], a, gate, up).double(), g / (1 + torch.exp(-g)) * u, rtol=2.0**-21, atol=1e-30)
 
 
+@pytest.mark.parametrize("enc", ("Q4_0",) + ENCODINGS)
+@pytest.mark.parametrize("lhs", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(8, 2816, 1024), (16, 2815, 1024), (12, 9721, 2560), (20, 4850, 1024), (16, 6130, 4608), (8, 11007, 512),  # pairs of whole tiles: more than four rows
+                                   (4, 2816, 1024), (2, 4862, 1024), (3, 2801, 512)])  # eight rows of each matrix, as many a workgroup as in pairs
+def test_gated_pair_dealt_in_pairs_of_tiles(enc, lhs, m, n, k):
+    """A workgroup with two items for a result, or twice as many tiles as there are places for: the sums of a call with one matrix, with a last tile that is ragged or has no second half."""
+    gate, up, a = packed(enc, n, k), packed(enc, n, k, 1), rows(m, k, lhs)
+    g, u = qmatmul(QE[enc], None, a, gate).double(), qmatmul(QE[enc], None, a, up).double()
+    assert torch.allclose(qmatmul_swiglu(QE[enc], a, gate, up).double(), g / (1 + torch.exp(-g)) * u, rtol=2.0**-21, atol=1e-30)
+
+
 def test_q6_k_at_every_multiple_of_four_and_an_odd_last_block():
     """Blocks of 210 bytes: rows that begin at 0 and at 2 mod 4 alternate with an odd number of blocks; a matrix of an odd number of them in all is left to the kernels
     that read its last one exactly."""
