@@ -342,18 +342,25 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     return look_up > std::min(11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w, 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0));
 }
 
-// How many workgroups zero results beside those of the lhs, in the launch of `slabs` workgroups that the part takes `at_once` of; -1: the lhs has a launch of its own.  zeros: results of the largest matrix
-// that is added to.
-// A workgroup of the lhs, or one that zeroes, takes a place like a slab's.  One more than there are places costs the time of a slab: 7400 x 8832 29 bf16 rows (232 slabs, 8 of the lhs, 256 places) with 56
-// that zero 57, with 8 42, the lhs as a launch of its own 46 us; 7560 x 8064 13 rows 49 / 35.6 / 40, 4056 x 18176 13 rows (254 slabs) 70 / - / 63.  The launch of its own costs 4 .. 7 us: 5120 x 20480 64 rows 88 / 95,
-// 14336 x 4096 400 rows 69 / 74, but 4096 x 14336 400 rows (one workgroup a compute unit) 101 / 93.  Where the sort is apart and the slabs fill three rounds or more, they end at different times, and a tenth
-// of them more is still cheaper: 24440 x 8192 42 rows 100 / 104, 5128 x 25856 66 fp32 rows 141 / 151; but thousands of rows 6984 x 25088 2283 rows 1013 / 919.  (1117 calls with the sort apart: 0.2 % off the faster of
-// both on average, always in the same launch 0.4 %, 28 of them slower than with the rows behind it.)
-int order_lhs_room(int64_t slabs, int64_t at_once, int64_t workgroups, int64_t zeros, bool sort_apart) {
-    const int64_t rounds = (slabs + at_once - 1) / at_once, room = rounds * at_once - slabs - workgroups, wanted = (std::min<int64_t>(1024, (zeros + 4095) / 4096) + 7) / 8 * 8;
-    const int64_t zeroing = std::min(wanted, std::max<int64_t>(room, 0) / 8 * 8);
-    if (room >= 0 && zeros <= zeroing << 18) return (int)zeroing;
-    return sort_apart && rounds >= 3 && 10 * (std::min<int64_t>(wanted, 8) - room) <= slabs ? (int)wanted : -1;
+// How many workgroups zero results beside those of the lhs (`rows` rows each) and `slabs` others, in a launch of which the part takes `at_once`; -1: the lhs has a launch of its own.  zeros: results of the
+// largest matrix that is added to.
+// Workgroups go to the eight XCDs in turn, and there to four groups of compute units in turn, whichever of those is free: one long workgroup more than a group has places for costs the time of a slab.  Those
+// that zero, and those of the lhs beyond its rows, end at once, but count in turn; so their number decides where the others go, and a few with nothing to do may help.  us by that number: 7840 x 5504 18 bf16 rows (31 slabs and a workgroup of
+// the lhs for the 32 places of an XCD) 8 / 16 / 32 / 40 36.1 / 36.0 / 29.3 / 35.9, 7400 x 8832 29 rows 8 / 16 / 32 / 56 41.7 / 41.8 / 41.9 / 57, 7560 x 8064 13 rows 8 / 16 / 24 35.6 / 48.9 / 48.8.  Of 5048 ways to launch 210
+// calls 5022 are faster or slower than with a launch for the lhs as this has them.  That launch costs 4 .. 7 us (14336 x 4096 400 rows 69 / 74, 5120 x 20480 64 rows 88 / 95), less than a slab (4096 x 14336 400
+// rows 101 / 93, 4056 x 18176 13 rows 70 / 63, 6984 x 25088 2283 rows 1013 / 919); two to a compute unit and in several rounds they end at different times, and one more costs less (24440 x 8192 42 rows 100 / 104,
+// 30688 x 5120 1126 rows 388 / 397; of 60 such calls none took longer so).
+int order_lhs_room(int64_t slabs, int64_t at_once, int64_t m, int64_t rows, int64_t zeros) {
+    // of the first XCD, which has as many as any
+    const int64_t own = (slabs + 7) / 8, places = at_once / 32, turns = (m + 63) / 64 * (8 / rows), live = m / 64 * (8 / rows) + (std::min<int64_t>(m % 64, 8) + rows - 1) / rows;
+    const int64_t wanted = (std::min<int64_t>(1024, (zeros + 4095) / 4096) + 7) / 8 * 8, alone = ((own + 3) / 4 + places - 1) / places;
+    if (alone > 1 && at_once > compute_units()) return (int)wanted;
+    for (int64_t zeroing = wanted; zeroing < wanted + 32; zeroing += 8) {
+        int64_t most = 0;
+        for (int64_t e = 0; e < 4; e++) most = std::max(most, (live - e + 3) / 4 + (own - ((e - turns - zeroing / 8) & 3) + 3) / 4);
+        if ((most + places - 1) / places == alone) return (int)zeroing;
+    }
+    return -1;
 }
 
 hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int group, const void* a, int lhs_dtype, int64_t m, const DirectSpace& p, const DirectMats& zero,
@@ -375,14 +382,13 @@ hipError_t launch_gptq_order(const GptqOrder& order, int64_t n, int64_t k, int g
                             (2 * (words(cols) + sort_lds) > kLdsPerCu && n > (int64_t)(cols == 32 ? 48 : cols) * compute_units());
     if (sort_apart) cols = k <= 5120 ? 32 : k <= 20480 ? 16 : 8;  // (32 up to where two fit, 28672 x 5120 32 / 16 columns 78.5 / 80.4; 16 up to where one does, 14336 x 20480 16 / 8 165 / 175)
     const unsigned per_xcd = (unsigned)((n + 8 * cols - 1) / (8 * cols));
-    // The lhs in the same launch where the slabs' last round has room for its workgroups and for some that zero results (order_lhs_room); otherwise the caller's preparation reads its rows in the order
-    // left in memory.
+    // The lhs in the same launch where that takes no longer (order_lhs_room); otherwise the caller's preparation reads its rows in the order left in memory.
     const bool f32 = lhs_dtype == QMM_F32;
     const int64_t lds = words(cols) + (sort_apart ? 0 : sort_lds), at_once = compute_units() * (2 * lds <= kLdsPerCu && (sort_apart || k <= 8192) ? 2 : 1);
-    const int workgroups = (int)((m + 63) / 64 * 64 / lhs_rows(cols, f32 ? 4 : 2)), zeroing = order_lhs_room((n + cols - 1) / cols, at_once, workgroups, zeros, sort_apart);
+    const int rows = lhs_rows(cols, f32 ? 4 : 2), zeroing = order_lhs_room((n + cols - 1) / cols, at_once, m, rows, zeros);
     lhs_done = zeroing >= 0;
     const OrderLhs none{};
-    const OrderLhs lhs{a, p.a16, p.inv, (int)m, workgroups, std::max(zeroing, 0), zero};
+    const OrderLhs lhs{a, p.a16, p.inv, (int)m, (int)((m + 63) / 64 * 64 / rows), std::max(zeroing, 0), zero};
     int32_t* const source = sort_apart || !lhs_done ? order.space.source : nullptr;
     hipError_t e;
 #define QMM_GO(AT, COLS, TURNS, WORDS, GRID, LDS, LHS)                                                                                                                  \

@@ -311,22 +311,41 @@ def test_long_rows_go_to_the_staged_gemm():
 
 
 def test_workgroups_beside_the_slabs_find_a_place():
-    """Act-order: rows of the lhs and the zeroing of results share the launch that sorts the weights only where no slab has to wait for them (a few, where slabs of several rounds end at different times)."""
-    room = getattr(C.CDLL(_lib.LIB_PATH), "_ZN3qmm14order_lhs_roomEllllb")
-    room.argtypes, room.restype = [C.c_int64] * 4 + [C.c_bool], C.c_int
-    shared = 0
-    for slabs in (1, 232, 240, 248, 255, 256, 257, 480, 512, 700, 768, 1016):
-        for workgroups in (8, 16, 32, 256, 1152):
-            for zeros in (0, 1, 13 * 7560, 29 * 7400, 1 << 21, 1 << 24):
-                for apart in (False, True):
-                    rounds, zeroing = -(-slabs // 256), room(slabs, 256, workgroups, zeros, apart)
-                    if zeroing < 0:
+    """Act-order: rows of the lhs and the zeroing of results share the launch that sorts the weights where no group of compute units, of four in each XCD that take workgroups in turn, gets more rounds of
+    long ones than the weights alone would have: counted out here one by one."""
+    room = getattr(C.CDLL(_lib.LIB_PATH), "_ZN3qmm14order_lhs_roomElllll")
+    room.argtypes, room.restype = [C.c_int64] * 5, C.c_int
+
+    def rounds(slabs, at_once, m, rows, zeroing):
+        worst = 0
+        for xcd in range(8):
+            per, each, long = -(-slabs // 8), 8 // rows, [0] * 4
+            for turn in range(-(-m // 64) * each):  # (gptq_order_kernel's rows of a workgroup)
+                if (turn // each * 8 + xcd) * 8 + turn % each * rows < m:
+                    long[turn % 4] += 1
+            first = -(-m // 64) * each + zeroing // 8
+            for i in range(max(0, min(per, slabs - xcd * per))):
+                long[(first + i) % 4] += 1
+            worst = max(worst, *long)
+        return -(-worst // (at_once // 32))
+
+    shared = apart = 0
+    for slabs in (1, 8, 129, 232, 237, 245, 254, 256, 257, 480, 512, 700, 1016):
+        for at_once, rows in ((256, 1), (256, 4), (512, 2), (256, 8)):
+            alone = -(-(-(-slabs // 8)) // 4)
+            alone = -(-alone // (at_once // 32))
+            for m in (1, 8, 13, 29, 64, 66, 300, 1000):
+                for zeros in (0, 1, 13 * 7560, 29 * 7400, 1 << 21):
+                    got, most = room(slabs, at_once, m, rows, zeros), -(-min(1024, -(-zeros // 4096)) // 8) * 8
+                    if got < 0:
+                        apart += 1
+                        assert all(rounds(slabs, at_once, m, rows, most + 8 * i) > alone for i in range(4))
                         continue
                     shared += 1
-                    assert zeroing % 8 == 0 and (zeroing > 0) == (zeros > 0)
-                    assert slabs + workgroups + zeroing <= 256 * rounds or (apart and rounds >= 3 and slabs + workgroups + min(zeroing, 8) <= 256 * rounds + slabs // 10)
-    assert shared > 100
-    assert room(237, 256, 8, 13 * 7560, False) == 8 and room(254, 256, 16, 0, True) == -1 and room(873, 256, 1152, 0, True) == -1
+                    assert got % 8 == 0 and most <= got < most + 32
+                    if at_once == 256 or alone == 1:  # (two a compute unit, several rounds: always)
+                        assert rounds(slabs, at_once, m, rows, got) == alone
+    assert shared > 300 and apart > 300
 
 
 def test_operands_of_long_rows_do_not_overlap(tmp_path):
