@@ -50,8 +50,7 @@ DirectSpace direct_space(void* ws, bool f32, bool with_sums, bool with_sums32, i
 // columns (200 x 14336 bf16 rows with 256 threads a row 10.1 us, with 1024 7.2), all of which are asked for before the first is looked at; with many, that a row writes 16 bytes of a
 // 128-byte line, the rest of which other workgroups of the XCD fill.  us in a trace, the pieces widened to fp32 as they arrive (a wait after each) and compared as such / kept as they are:
 // 500 x 14336 bf16 rows 13.8 / 11.7 (28 MB), 200 x 14336 7.6 / 7.1; of calls, Q4_K 4096 x 14336 200 rows 47.0 / 46.4, 4096 x 28672 40 fp32 rows 57.3 / 56.3, 512 x 2048 24 fp32 rows 9.7 / 8.6.
-// Two workgroups of 1024 threads to a compute unit, 64 registers: with 66 one, GPTQ 696 x 7936 327 fp32 rows 33.9 / 34.9 us, Q4_K 616 x 6400 416 rows 33.65 / 34.15.  A sorted row's turns without the wavefronts that
-// have no piece in them: act-order 1232 x 3712 2507 bf16 rows 92.1 / 95.7, 888 x 4352 1610 fp32 rows 63.5 / 67.2.
+// Two workgroups of 1024 threads to a compute unit, 64 registers: with 66 one, GPTQ 696 x 7936 327 fp32 rows 33.9 / 34.9 us, Q4_K 616 x 6400 416 rows 33.65 / 34.15.
 // Rows of one group of eight go to workgroups of one XCD (ids congruent mod 8): a 128-byte line of an operand holds eight rows.
 // SORTED: column p of the operands is column source[p] of the row, which lies in LDS (k values) meanwhile.
 template <typename AT, int ORDER, bool SORTED = false>
@@ -94,15 +93,13 @@ __global__ __launch_bounds__(1024, 8) void direct_prep_kernel(const AT* __restri
         }
     };
     uint32_t top = 0;
-    // (SORTED: none for a wavefront without a piece, which would take its values from LDS for nothing.  A branch on what all lanes share, so that no wait comes with it.)
-    const int wave0 = SORTED ? __builtin_amdgcn_readfirstlane(tid & ~63) : 0;
     if (turns <= kHeld) {
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (wave0 + i * threads < pieces) held[i] = load(min(tid + i * threads, pieces - 1));
+            if (i < turns) held[i] = load(min(tid + i * threads, pieces - 1));
 #pragma unroll
         for (int i = 0; i < kHeld; i++)
-            if (wave0 + i * threads < pieces) top = largest_bits(top, held[i]);
+            if (i < turns) top = largest_bits(top, held[i]);
     } else {
         for (int pc = tid; pc < pieces; pc += threads) top = largest_bits(top, load(pc));
     }
@@ -195,6 +192,12 @@ __global__ __launch_bounds__(1024) void direct_prep_q8_kernel(const AT* __restri
 }
 
 int prep_threads(int64_t k) { return k <= 2048 ? 256 : k <= 4096 ? 512 : 1024; }
+// For a sorted row, whose values come from LDS: as many turns, with as few threads as they need.  us, act-order calls, 512 or 1024 threads in every turn / branches around what a wavefront has no piece of, with
+// a wait at each / this way: 1232 x 3712 2507 bf16 rows 95.6 / 92.6 / 91.5, 2208 x 2688 1940 rows 88.0 / 83.3 / 82.2, 888 x 4352 1610 fp32 rows 66.6 / 63.2 / 62.9.
+int sorted_prep_threads(int64_t k) {
+    const int64_t pieces = k / 8, turns = (pieces + prep_threads(k) - 1) / prep_threads(k);
+    return (int)((pieces + turns * 64 - 1) / (turns * 64) * 64);
+}
 
 constexpr int direct_ahead(int enc, int fm, int fn, bool hilo, int flush) {
     if (fm * fn == 2) return hilo ? 4 : 8;
@@ -826,7 +829,7 @@ hipError_t launch_gemm_direct(int encoding, const void* lhs, int lhs_dtype, int 
         if (plans[j].shares > 1) zero.out[zero.count] = outs[j], zero.n[zero.count++] = (int)ns[j], zeros = std::max(zeros, m * ns[j]);
     }
     const unsigned grid = (unsigned)((m + 63) / 64 * 64 + std::min<int64_t>(1024, (zeros + 4095) / 4096));
-    const int threads = prep_threads(k);
+    const int threads = order ? sorted_prep_threads(k) : prep_threads(k);
     if (q40) {
         if (f32) direct_prep_q8_kernel<float><<<dim3(grid), dim3(threads), 0, s>>>((const float*)lhs, (int)m, (int)k, p, zero);
         else direct_prep_q8_kernel<uint16_t><<<dim3(grid), dim3(threads), 0, s>>>((const uint16_t*)lhs, (int)m, (int)k, p, zero);
