@@ -528,7 +528,7 @@ double shared_us(const SharedCost& c, int plan, int shares, int64_t m, int64_t n
 }
 // The same for the kernel whose lhs and weights go to LDS by themselves (gemm_staged.hip).  On 1215 problems that it was not fitted to (512 x 512 .. 28672 x 8192, K up to
 // 18944, 33 .. 4096 rows, weights from memory; profiles/staged_gemm__plans.txt): 4 .. 6 % off on average by encoding and lhs type, what it has first takes 1 .. 2 % longer than
-// the best plan.
+// the best plan.  (Fitted before bf16 rows' loads were spread over the steps and before a last tile of 96 or 128 rows without its last 32 left these out: such plans cost up to 7 % less than it says.)
 // other: what the GEMMs behind this file (planes, tiles) take, from 200 rows on, in us: a fixed part, per MB of weights, per million lhs values, per million
 // results, per 10^9 products with the rows in 256s (8 .. 12 % off beyond direct_range, where it is asked for, and what is picked there by it takes 0.9 % longer on average than the
 // faster of both; none for groups that are no multiple of 128, which have no such GEMM).

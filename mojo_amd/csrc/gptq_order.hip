@@ -324,10 +324,11 @@ GptqOrderSpace gptq_order_space(void* workspace, int64_t n, int64_t k) {
 
 // The look-up kernel or the sort and the direct GEMM: the predicted time of both in microseconds.  The look-up kernel walks K with one workgroup per 64
 // columns, in passes of up to four rows; where its table of scales does not fit LDS (small groups on a long K), every weight reads its
-// scale from memory.  The sorted way is four launches and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
+// scale from memory.  The sorted way is three launches (up to five where the lhs or the sort has one of its own) and one pass over the weights, whatever the number of rows up to 32.  Fitted to timings of
 // 15 matrices (512 x 512 .. 28672 x 8192, groups of 32 and 128, weights from memory) with 1 .. 12 rows; what is taken, the second line included, takes 0.14 % longer on
-// average than the faster of the two (profiles/gptq_act_order__look_up_against_sorted.txt, 576 calls).  us, look-up / sorted: 14336 x 4096 4 bf16 rows 34 / 38, 5 rows 47 / 38, fp32 6 rows
-// 40.2 / 40.2; 4096 x 4096 2 / 3 bf16 rows 27 / 22, 32 / 22; 8192 x 8192 4 rows 62 / 42; 512 x 512 8 / 12 fp32 rows 9 / 12, 13.6 / 12.4; 1024 x 14336 one bf16 row 43 / 41, one fp32 row 42 / 46.
+// average than the faster of the two (profiles/gptq_act_order__look_up_against_sorted.txt, 576 calls, from when the lhs had a launch of its own and nibbles were sorted one by one: the sorted way has become 4 .. 8 us
+// cheaper, and up to a fifth is lost near the line).  us, look-up / sorted, now: 14336 x 4096 4 bf16 rows 29.9 / 30.2, 5 rows 42.9 / 29.9, fp32 4 rows 21.1 / 32.0, 6 rows 39.2 / 32.2; 11008 x 4096 4 bf16 rows
+// 27.9 / 28.5; 4096 x 4096 2 / 3 bf16 rows 21.9 / 17.7, 26.6 / 17.9; 8192 x 8192 4 rows 57.8 / 39.2; 512 x 512 8 / 12 fp32 rows 9.7 / 10.0, 14.8 / 10.0; 1024 x 14336 one bf16 row 40 / 32.5, one fp32 row 41.9 / 37.1.
 bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group) {
     if (k > 32768 || n % 8 || k % 32 || kernel_disabled("gptq_order")) return false;
     const bool f32 = lhs_dtype == QMM_F32;
@@ -337,8 +338,8 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
     if (!gptq_act_order_table_fits(m, k, group)) one *= f32 ? 1.9 : 3.0;
     const double look_up = one * ((m / 4) * rows[3] + rows[std::min<int64_t>(m % 4, 3)]);
     // Beyond some 60 M weights that line finds the look-up kernel ahead with one row more or two, but there it is two to four times further off: the second line, from when
-    // the sort was a launch of its own.  Relative error, us, look-up / sorted: 5504 x 18944 4 fp32 rows 5.7e-7 / 1.3e-7, 100 / 92; 18944 x 4096 6 rows 2.8e-7 / 1.2e-7,
-    // 71 / 56; groups of 32, 11648 x 12032 2 rows 4.7e-7 / 1.5e-7, 84 / 100; 32000 x 28672 4 bf16 rows 6.1e-7 / 1.4e-7, 420 / 483.
+    // the sort was a launch of its own.  Relative error, us, look-up / sorted: 5504 x 18944 4 fp32 rows 5.7e-7 / 1.3e-7, 99 / 79; 18944 x 4096 6 rows 2.8e-7 / 1.2e-7,
+    // 69 / 48; groups of 32, 11648 x 12032 2 rows 4.7e-7 / 1.5e-7, 83 / 87; 32000 x 28672 4 bf16 rows 6.1e-7 / 1.4e-7, 419 / 479.
     return look_up > std::min(11.0 + (f32 ? 1.8 : 1.5) * kk + (f32 ? 0.40 : 0.35) * w, 13.0 + 2.1 * kk + 0.31 * w + 0.12 * (n / 1024.0));
 }
 
