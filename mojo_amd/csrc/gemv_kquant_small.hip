@@ -459,8 +459,11 @@ __device__ __forceinline__ void small_body(const MmMats& mats, const AT* __restr
     }
 }
 
+// Wavefronts a SIMD that the compiler may aim at.  A launch has four, but for six it packs one and two bf16 rows of Q6_K into 80 registers where 90 keep an item's unpacking in flight: 4096 | 1024 | 1024
+// x 4096 2 rows 8.4 / 7.8 us, 3664 | 3664 | 3664 x 1024 one row 5.3 / 4.95.
+constexpr int small_simd_waves(int enc, int rows, int size, int mode) { return enc == QMM_Q6_K && rows <= 2 && size == 2 && mode == kSmallMats ? 5 : 8; }
 template <int ENC, int MROWS, typename AT, int MODE>
-__global__ __launch_bounds__(64 * kSmallWaves) void gemv_kquant_small_mats_kernel(const MmMats mats, const AT* __restrict__ a, int m, int k, const SmallCut cut) {
+__global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_eu(4, small_simd_waves(ENC, MROWS, sizeof(AT), MODE)))) void gemv_kquant_small_mats_kernel(const MmMats mats, const AT* __restrict__ a, int m, int k, const SmallCut cut) {
     small_body<ENC, MROWS, AT, MODE>(mats, a, m, k, cut);
 }
 
