@@ -353,7 +353,7 @@ bool gptq_order_wanted(int lhs_dtype, int64_t m, int64_t n, int64_t k, int group
 // 30688 x 5120 1126 rows 388 / 397; of 60 such calls none took longer so).
 int order_lhs_room(int64_t slabs, int64_t at_once, int64_t m, int64_t rows, int64_t zeros) {
     // of the first XCD, which has as many as any
-    const int64_t own = (slabs + 7) / 8, places = at_once / 32, turns = (m + 63) / 64 * (8 / rows), live = m / 64 * (8 / rows) + (std::min<int64_t>(m % 64, 8) + rows - 1) / rows;
+    const int64_t own = (slabs + 7) / 8, places = std::max<int64_t>(1, at_once / 32), turns = (m + 63) / 64 * (8 / rows), live = m / 64 * (8 / rows) + (std::min<int64_t>(m % 64, 8) + rows - 1) / rows;
     const int64_t wanted = (std::min<int64_t>(1024, (zeros + 4095) / 4096) + 7) / 8 * 8, alone = ((own + 3) / 4 + places - 1) / places;
     if (alone > 1 && at_once > compute_units()) return (int)wanted;
     for (int64_t zeroing = wanted; zeroing < wanted + 32; zeroing += 8) {
