@@ -521,7 +521,7 @@ double small_convert_us(int encoding, int lhs_dtype, int64_t m) {
 // A gated pair: tiles with eight rows of each matrix, or pairs of whole ones?  By what the fullest compute unit gets, its workgroups' lhs and items one after the other.  The former may leave it an item less, but
 // where several workgroups fit a compute unit they are more workgroups, and each converts the lhs: Q4_K 2816 x 1024 16 fp32 rows 6.5 / 7.3 us, Q4_0 4864 x 1024 8 fp32 rows 5.8 / 6.4 in pairs / halves.
 // With more than four lhs rows a workgroup, pairs also where nothing is gained: half as many results to a wavefront's store is 2 .. 8 % there (9728 x 2560 16 fp32 rows Q4_0 13.6 / 14.4, 18944 x 3584
-// 16 bf16 rows Q4_K 23.4 / 24.3); up to four rows, halves dealt like pairs (Q5_K 2816 x 1024 4 rows in pairs, halves, so dealt 4.5 / 4.3 / 4.15).  Over 460 calls, 1 .. 24 rows, 1.00 of the time of pairs at
+// 16 bf16 rows Q4_K 23.4 / 24.3); up to four rows, halves dealt like pairs (Q5_K 2816 x 1024 4 rows in pairs, halves, so dealt 4.5 / 4.3 / 4.15).  Over 460 calls, 1 .. 24 rows, 1.02 of the time of pairs at
 // worst, 0.95 on average; always halves 0.96, up to 1.15.
 SmallPlan small_gated_plan(int encoding, int lhs_dtype, int64_t m, int64_t n, int64_t k) {
     const SmallPlan halves = small_plan(encoding, lhs_dtype, m, (n + 7) / 8, k, false), pairs = small_plan(encoding, lhs_dtype, m, (n + 15) / 16, k, false, 2);
